@@ -65,7 +65,7 @@ typedef unsigned int store_u32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned int store_u32x2 __attribute__((ext_vector_type(2)));
 static __constant__ int g_dev_store_through = 1;
 #define TR_DEFINE_STORE_THROUGH_SETTER(name)                                                          \
-    int name(int on) { return (int)hipMemcpyToSymbol(HIP_SYMBOL(g_dev_store_through), &on, sizeof(int)); }
+    int name(int on) { return (int)hipMemcpyToSymbol(HIP_SYMBOL(::tnn_rocm::g_dev_store_through), &on, sizeof(int)); }
 
 __device__ __forceinline__ void store_out16(void *p, store_u32x4 v) {
     if (g_dev_store_through)

@@ -190,18 +190,21 @@ int tnn_rocm_event_record(void *event, void *stream) {
 
 // every translation unit holds its own copy of the switch (common.h); they are set together (weak: a stand-alone
 // program may link this file with only some of the kernels)
-__attribute__((weak)) int gemm_set_store_through(int on);
+__attribute__((weak)) int gemm_f32_set_store_through(int on);
+__attribute__((weak)) int gemm_f16_set_store_through(int on);
+__attribute__((weak)) int gemm_f16_ln_set_store_through(int on);
+__attribute__((weak)) int gemm_bf16_set_store_through(int on);
+__attribute__((weak)) int gemm_bf16_ln_set_store_through(int on);
+__attribute__((weak)) int gemm_i8_set_store_through(int on);
 __attribute__((weak)) int attention_set_store_through(int on);
 __attribute__((weak)) int rowwise_set_store_through(int on);
 __attribute__((visibility("default"))) int tnn_rocm_debug_set_store_through(int on) {
     on = on ? 1 : 0;
     TR_CHECK_HIP(hipDeviceSynchronize());
-    if (gemm_set_store_through)
-        TR_CHECK_HIP((hipError_t)gemm_set_store_through(on));
-    if (attention_set_store_through)
-        TR_CHECK_HIP((hipError_t)attention_set_store_through(on));
-    if (rowwise_set_store_through)
-        TR_CHECK_HIP((hipError_t)rowwise_set_store_through(on));
+    int (*const setters[])(int) = {gemm_f32_set_store_through, gemm_f16_set_store_through, gemm_f16_ln_set_store_through, gemm_bf16_set_store_through, gemm_bf16_ln_set_store_through, gemm_i8_set_store_through, attention_set_store_through, rowwise_set_store_through};
+    for (auto set : setters)
+        if (set)
+            TR_CHECK_HIP((hipError_t)set(on));
     return 0;
 }
 
