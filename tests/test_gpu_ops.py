@@ -538,6 +538,60 @@ def test_gemm_every_tile_configuration(code):
         lib.tnn_rocm_debug_set_gemm_config(0)
 
 
+@pytest.mark.parametrize("code", [9111141, 9121141, 3112221, 3112222, 3212221, 4221141])
+@pytest.mark.parametrize("M,N,K", [(1, 8, 256), (33, 776, 256), (130, 136, 3072)])
+def test_gemm_small_product_shapes(code, M, N, K):
+    """The tile shapes of the small products, forced where they can go wrong: one row, a remainder of one row or of eight
+    columns behind whole tiles, fewer slabs than a ring or a wave count has places, many slabs.  fp16 epilogues (the
+    folded LayerNorm with its statistics and the row sums handed on among them), fp32 where the shape serves it, int8
+    bit-exact."""
+    from tnn_amd import capi
+    lib = capi.load()
+    say("tile configuration %d, M=%d N=%d K=%d" % (code, M, N, K))
+    rng = np.random.default_rng(code + M)
+    r32 = lambda *s: rng.standard_normal(s).astype(np.float32)
+    a, w = torch.from_numpy(r32(M, K) + 0.5), torch.from_numpy(r32(N, K) * 0.03)
+    res, bias = torch.from_numpy(r32(M, N)), r32(N) * 0.1
+    ah, wh, rh = a.half(), w.half(), res.half()
+    af, wf, rf = (t.float().numpy() for t in (ah, wh, rh))
+    g, be = 1 + 0.2 * r32(K), 0.3 * r32(K)
+    go, beo = dev(1 + 0.2 * r32(N)), dev(0.3 * r32(N))
+    a8, w8 = rng.integers(-128, 128, (M, K), dtype=np.int8), rng.integers(-127, 128, (N, K), dtype=np.int8)
+    b8 = rng.integers(-20000, 20000, N).astype(np.int32)
+    scale = orc.fc_int8_scale((rng.uniform(0.5, 1.5, N) * 1e-3).astype(np.float32), np.float32(0.37), N)
+    ref_q, ref_acc = orc.fc_int8(a8, w8, b8, scale)
+    w1f, cs, b1f = _fold_ln_weights(w.numpy(), bias, g, be, torch.float16)
+    o = ops()
+    lib.tnn_rocm_debug_set_gemm_config(code)
+    try:
+        got = host(o.gemm(ah.cuda(), wh.cuda(), True, bias=dev(bias), gelu=True))
+        assert rel_err(got, orc.gelu(orc.inner_product(af, wf, bias))) <= FP16_TOL
+        got = host(o.gemm(ah.cuda(), wh.cuda(), True, bias=dev(bias), residual=rh.cuda()))
+        assert rel_err(got, orc.inner_product(af, wf, bias) + rf) <= FP16_TOL
+        h, st = o.gemm_ln(ah.cuda(), w1f.cuda(), dev(b1f), dev(cs), 1e-5, want_stats=True)
+        assert rel_err(host(h), orc.inner_product(orc.layernorm(af, g, be, 1e-5), w.numpy(), bias)) <= FP16_TOL
+        a64 = af.astype(np.float64)
+        assert np.abs(host(st)[:, 0] * np.sqrt(a64.var(1) + 1e-5) - 1).max() <= 1e-5
+        out_st = dev(np.stack([1 / np.sqrt(rf.var(1) + 1e-5), rf.mean(1)], 1).astype(np.float32))
+        plain = o.gemm_residual_ln(ah.cuda(), wh.cuda(), rh.cuda(), out_st, go, beo, bias=dev(bias))
+        assert rel_err(host(plain), orc.inner_product(af, wf, bias) + orc.layernorm(rf, host(go), host(beo), 1e-5)) <= FP16_TOL
+        c, (sums, blocks) = o.gemm_residual_ln(ah.cuda(), wh.cuda(), rh.cuda(), out_st, go, beo, bias=dev(bias), want_row_sums=True)
+        assert torch.equal(c, plain) and blocks <= o.MAX_ROW_SUM_BLOCKS
+        if blocks:
+            cf = host(c).astype(np.float64)
+            got_s = host(sums)[:blocks].astype(np.float64).sum(0)
+            assert np.abs(got_s[:, 0] - cf.sum(1)).max() <= 1e-5 * np.abs(cf).sum(1).max()
+            assert np.abs(got_s[:, 1] / (cf ** 2).sum(1) - 1).max() <= 1e-5
+        q, acc, _ = o.gemm_i8(dev(a8), dev(w8), dev(b8), dev(scale), want_acc=True)
+        assert np.array_equal(host(acc), ref_acc)
+        assert np.array_equal(host(q), ref_q)
+        if code in (9111141, 9121141, 4221141):
+            got = host(o.gemm(a.cuda(), w.cuda(), True, bias=dev(bias), residual=res.cuda()))
+            assert rel_err(got, orc.inner_product(a.numpy(), w.numpy(), bias) + res.numpy()) <= 1e-5
+    finally:
+        lib.tnn_rocm_debug_set_gemm_config(0)
+
+
 # ---- int8 GEMM: bit-exact accumulators and outputs -----------------------------------------------
 @pytest.mark.parametrize("M,N,K", [(1, 1, 1), (2, 4, 9), (2, 16, 19), (7, 32, 16), (128, 3072, 768), (128, 768, 3072),
                                    (300, 768, 768), (65, 100, 200)])

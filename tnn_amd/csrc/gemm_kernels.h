@@ -901,12 +901,16 @@ __global__ void __launch_bounds__(WM *WN * 64)
 // NSTAGE = 2 or 3: slabs travel global -> LDS directly (global_load_lds_dwordx4: no staging registers and no LDS
 //     store instructions), into NSTAGE un-padded buffers whose 16-byte chunks are XOR-swizzled per row so that the
 //     fragment reads stay free of bank conflicts; loads run NSTAGE-1 slabs ahead of the MFMAs.
-template <int TM_, int TN_, int WGM_, int WGN_, int WGK_, int SLAB_, int NSTAGE_ = 0> struct TileCfg {
+// OWN (with WGM = WGN = 1): every k-wave has a ring of NSTAGE slabs of its own and walks a contiguous part of K by itself.
+//     A slab is then SLAB bytes of k of ALL rows of the tile for ONE wave, and nothing in the main loop concerns another
+//     wave: no barrier, each wave waits for its own loads only.
+template <int TM_, int TN_, int WGM_, int WGN_, int WGK_, int SLAB_, int NSTAGE_ = 0, bool OWN_ = false> struct TileCfg {
     static constexpr int TM = TM_, TN = TN_, WGM = WGM_, WGN = WGN_, WGK = WGK_, SLAB = SLAB_, NSTAGE = NSTAGE_;
+    static constexpr bool OWN = OWN_;
     static constexpr int BM = 32 * TM * WGM, BN = 32 * TN * WGN;
     static constexpr int STRIDE = NSTAGE_ ? SLAB : SLAB + 16;
     static constexpr int SSTR   = 32 * TN + 4;  // staged row stride in 32-bit words
-    static constexpr size_t slab_bytes  = (size_t)(NSTAGE_ ? NSTAGE_ : 2) * (BM + BN) * STRIDE;
+    static constexpr size_t slab_bytes  = (size_t)(NSTAGE_ ? NSTAGE_ : 2) * (BM + BN) * STRIDE * (OWN_ ? WGK_ : 1);
     static constexpr size_t stage_bytes = (size_t)WGM_ * WGN_ * WGK_ * 32 * SSTR * 4;
     static constexpr size_t lds_bytes   = slab_bytes > stage_bytes ? slab_bytes : stage_bytes;
     // where an epilogue that leaves row sums keeps its BM x BN / 8 pairs: in the part of the slab area the staging does
@@ -915,9 +919,10 @@ template <int TM_, int TN_, int WGM_, int WGN_, int WGK_, int SLAB_, int NSTAGE_
     static constexpr size_t sums_offset = (slab_bytes >= stage_bytes + sums_bytes) ? stage_bytes : lds_bytes;
     static constexpr int NW = WGM * WGN * WGK, NT = 64 * NW;  // waves and threads per workgroup
     static_assert(NW == 4 || NW == 8, "four or eight waves per workgroup");
-    static_assert((SLAB / 32) % WGK == 0, "k-steps of a slab must split evenly over the k-waves");
-    static_assert((BM * (SLAB / 16)) % NT == 0 && (BN * (SLAB / 16)) % NT == 0, "slab must divide over the workgroup");
-    static_assert(NSTAGE_ == 0 || NSTAGE_ == 2 || NSTAGE_ == 3, "register-staged, or two / three direct-to-LDS stages");
+    static_assert(OWN_ || (SLAB / 32) % WGK == 0, "k-steps of a slab must split evenly over the k-waves");
+    static_assert(OWN_ || ((BM * (SLAB / 16)) % NT == 0 && (BN * (SLAB / 16)) % NT == 0), "slab must divide over the workgroup");
+    static_assert(!OWN_ || (WGM_ == 1 && WGN_ == 1 && NSTAGE_ >= 2 && NSTAGE_ <= 4), "rings of two to four slabs, k-waves only");
+    static_assert(OWN_ || NSTAGE_ == 0 || (NSTAGE_ >= 2 && NSTAGE_ <= 5), "register-staged, or two to five direct-to-LDS stages");
 };
 
 // Dynamic LDS of one (tile shape, epilogue) pair, for the kernel and its launcher alike: the slab / staging area, what
@@ -925,7 +930,7 @@ template <int TM_, int TN_, int WGM_, int WGN_, int WGK_, int SLAB_, int NSTAGE_
 // its per-row pairs.
 template <typename CFG, typename Epi> struct EpiLds {
     static constexpr size_t lut_need   = CFG::stage_bytes + 256;  // Int8Epilogue's table behind the staging area
-    static constexpr size_t stats_need = CFG::stage_bytes + (size_t)CFG::BM * 8 * (1 + 2 * CFG::WGK * CFG::WGN);
+    static constexpr size_t stats_need = CFG::stage_bytes + (size_t)CFG::BM * (8 + 16 * CFG::WGK * CFG::WGN);
     static constexpr size_t base0 = std::is_same<Epi, Int8Epilogue>::value && lut_need > CFG::lds_bytes ? lut_need : CFG::lds_bytes;
     // row statistics and the partial-sum buffer sit behind the staging area; handed-over sums park {rstd, mean} per row
     // behind the slabs before the main loop
@@ -1002,13 +1007,118 @@ __global__ void __launch_bounds__(CFG::NT)
     const int frag_off = (lane >> 5) * 16;
     const int nk       = K / KB;
 
-    // LayerNorm-folding epilogues: this lane's share of sum / sum of squares of A row (wm * TM + i) * 32 + frag_row
-    float ln_s1[TM], ln_s2[TM];
+    // LayerNorm-folding epilogues: this lane's share of sum / sum of squares of A row (wm * TM + i) * 32 + frag_row.  The
+    // eight values of a fragment are added up in fp32, the fragments in double: every tile shape deals the fragments out to
+    // its waves in another way, and the statistics should not depend on that.
+    double ln_s1[TM], ln_s2[TM];
 #pragma unroll
     for (int i = 0; i < TM; ++i)
-        ln_s1[i] = ln_s2[i] = 0.f;
+        ln_s1[i] = ln_s2[i] = 0.0;
+    auto ln_take = [&](const uint4 &frag, int i) __attribute__((always_inline)) {
+        float s1 = 0.f, s2 = 0.f;
+        ln_accumulate<DT>(frag, s1, s2);
+        ln_s1[i] += (double)s1;
+        ln_s2[i] += (double)s2;
+    };
 
-    if constexpr (CFG::NSTAGE > 0) {
+    if constexpr (CFG::OWN) {
+        // Every wave streams its own part of K: both panels' rows of one 64-byte k-slab per stage, through a ring that
+        // only this wave fills and reads.  Row swizzle as in the shared pipeline below.
+        static_assert(!TakesRowSums<Epi>::value, "own-ring shapes take the row statistics from their A fragments");
+        constexpr int NS   = CFG::NSTAGE;
+        constexpr int RPL  = 1024 / SLAB;  // slab rows per load instruction
+        constexpr int R256 = 256 / SLAB;
+        constexpr int A_LD = BM / RPL, B_LD = BN / RPL, LPW = A_LD + B_LD;
+        constexpr int STAGE = (BM + BN) * SLAB;
+        static_assert(SLAB <= 256 && BM % RPL == 0 && BN % RPL == 0 && (NS - 1) * LPW < 64, "ring shape");
+        uint32_t a_off[A_LD], b_off[B_LD];
+        const int lrow = lane / VPR, lpos = lane % VPR;
+#pragma unroll
+        for (int i = 0; i < A_LD; ++i) {
+            const int r = i * RPL + lrow;
+            int row     = m0 + r;
+            row         = row < M ? row : M - 1;
+            a_off[i]    = ((uint32_t)row * (uint32_t)lda + (uint32_t)((lpos ^ ((r / R256) % VPR)) * VEC)) * (uint32_t)sizeof(T);
+        }
+#pragma unroll
+        for (int i = 0; i < B_LD; ++i) {
+            const int r = i * RPL + lrow;
+            int row     = n0 + r;
+            row         = row < N ? row : N - 1;
+            b_off[i]    = ((uint32_t)row * (uint32_t)ldb + (uint32_t)((lpos ^ ((r / R256) % VPR)) * VEC)) * (uint32_t)sizeof(T);
+        }
+        const int uwave         = __builtin_amdgcn_readfirstlane(wave);
+        const uint32_t ring_dst = (uint32_t)(uintptr_t)lds_dyn + (uint32_t)(uwave * NS * STAGE);
+        const unsigned char *const ring = lds_dyn + uwave * NS * STAGE;
+        // spelled as assembly for the reason given at the shared pipeline's load
+        auto load16 = [](const T *base, uint32_t byte_off, uint32_t lds_addr) {
+            asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+                         :
+                         : "v"(byte_off), "s"(base), "s"(lds_addr)
+                         : "memory", "m0");
+        };
+        auto issue = [&](int slab, int stage) __attribute__((always_inline)) {
+            const uint32_t dst = ring_dst + (uint32_t)(stage * STAGE);
+            const T *ga = A + (size_t)slab * KB, *gb = B + (size_t)slab * KB;
+#pragma unroll
+            for (int i = 0; i < B_LD; ++i)  // the weights first: they come from further away
+                load16(gb, b_off[i], dst + BM * SLAB + i * 1024);
+#pragma unroll
+            for (int i = 0; i < A_LD; ++i)
+                load16(ga, a_off[i], dst + i * 1024);
+        };
+        const int fswz = (frag_row / R256) % VPR;
+        const int frow = frag_row * SLAB;
+        const int k_lo = nk * uwave / CFG::WGK, k_hi = nk * (uwave + 1) / CFG::WGK;
+#pragma unroll
+        for (int p = 0; p < NS; ++p)
+            if (k_lo + p < k_hi)
+                issue(k_lo + p, p);
+        int stage = 0;
+        for (int kt = k_lo; kt < k_hi; ++kt) {
+            // slab kt is complete once at most the loads of the slabs requested after it are outstanding
+            const int behind = k_hi - 1 - kt;
+            if (NS > 3 && behind >= 3)
+                TR_WAIT_VMCNT(NS > 3 ? 3 * LPW : 0);
+            else if (NS > 2 && behind >= 2)
+                TR_WAIT_VMCNT(NS > 2 ? 2 * LPW : 0);
+            else if (behind >= 1)
+                TR_WAIT_VMCNT(LPW);
+            else
+                TR_WAIT_VMCNT(0);
+            asm volatile("" ::: "memory");
+            const unsigned char *sa = ring + stage * STAGE, *sb = sa + BM * SLAB;
+            uint4 fa[SLAB / 32][TM], fb[SLAB / 32][TN];
+#pragma unroll
+            for (int kk = 0; kk < SLAB / 32; ++kk) {
+                const int chunk = ((kk * 2 + (lane >> 5)) ^ fswz) * 16;
+#pragma unroll
+                for (int i = 0; i < TM; ++i)
+                    fa[kk][i] = *reinterpret_cast<const uint4 *>(sa + i * 32 * SLAB + frow + chunk);
+#pragma unroll
+                for (int j = 0; j < TN; ++j)
+                    fb[kk][j] = *reinterpret_cast<const uint4 *>(sb + j * 32 * SLAB + frow + chunk);
+            }
+            // the fragments are in registers before the slab's place is given to the next load
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            if (kt + NS < k_hi)
+                issue(kt + NS, stage);
+#pragma unroll
+            for (int kk = 0; kk < SLAB / 32; ++kk) {
+                if constexpr (Epi::kRowStats) {
+#pragma unroll
+                    for (int i = 0; i < TM; ++i)
+                        ln_take(fa[kk][i], i);
+                }
+#pragma unroll
+                for (int i = 0; i < TM; ++i)
+#pragma unroll
+                    for (int j = 0; j < TN; ++j)
+                        GemmTraits<DT>::mma(fb[kk][j], fa[kk][i], acc[i][j]);
+            }
+            stage = stage + 1 == NS ? 0 : stage + 1;
+        }
+    } else if constexpr (CFG::NSTAGE > 0) {
         // Direct-to-LDS pipeline.  One load instruction of a wave fills 1024 contiguous LDS bytes (lane L writes
         // bytes 16L..16L+15), i.e. RPL whole slab rows; the lane picks WHICH 16 global bytes land there, so the
         // swizzle is applied on the global side: physical chunk p of LDS row r holds logical chunk p ^ f(r),
@@ -1064,30 +1174,46 @@ __global__ void __launch_bounds__(CFG::NT)
         // byte offset of this lane's fragment chunk inside a slab row, per k-step of the slab
         const int fswz = (frag_row / R256) % VPR;
         const int frow = frag_row * SLAB;
-        auto compute = [&](int stage) {
+        // One slab: this wave's fragments of it, then `between` (the requests for the slab that goes into the stage freed
+        // last), then the MFMAs.  READ_AHEAD reads all of the slab's fragments before the requests, so that the LDS
+        // latency runs while the requests are issued; it needs the registers for them.
+        constexpr int KSTEPS      = SLAB / 32 / WGK;
+        constexpr bool READ_AHEAD = NS >= 4 && (TM + TN) * KSTEPS <= 8;
+        auto compute = [&](int stage, auto between) __attribute__((always_inline)) {
             const unsigned char *sa = lds_dyn + stage * STAGE, *sb = sa + BM * SLAB;
-#pragma unroll
-            for (int kk = wk; kk < SLAB / 32; kk += WGK) {
-                const int chunk = ((kk * 2 + (lane >> 5)) ^ fswz) * 16;
-                uint4 fa[TM], fb[TN];
+            uint4 fa[READ_AHEAD ? KSTEPS : 1][TM], fb[READ_AHEAD ? KSTEPS : 1][TN];
+            auto read = [&](int ks, int slot) __attribute__((always_inline)) {
+                const int chunk = (((wk + ks * WGK) * 2 + (lane >> 5)) ^ fswz) * 16;
 #pragma unroll
                 for (int i = 0; i < TM; ++i)
-                    fa[i] = *reinterpret_cast<const uint4 *>(sa + (wm * TM + i) * 32 * SLAB + frow + chunk);
+                    fa[slot][i] = *reinterpret_cast<const uint4 *>(sa + (wm * TM + i) * 32 * SLAB + frow + chunk);
 #pragma unroll
                 for (int j = 0; j < TN; ++j)
-                    fb[j] = *reinterpret_cast<const uint4 *>(sb + (wn * TN + j) * 32 * SLAB + frow + chunk);
+                    fb[slot][j] = *reinterpret_cast<const uint4 *>(sb + (wn * TN + j) * 32 * SLAB + frow + chunk);
+            };
+            if constexpr (READ_AHEAD) {
+#pragma unroll
+                for (int ks = 0; ks < KSTEPS; ++ks)
+                    read(ks, ks);
+            }
+            between();
+#pragma unroll
+            for (int ks = 0; ks < KSTEPS; ++ks) {
+                const int slot = READ_AHEAD ? ks : 0;
+                if constexpr (!READ_AHEAD)
+                    read(ks, 0);
                 if constexpr (Epi::kRowStats && !TakesRowSums<Epi>::value) {
                     // the WGN waves that hold the same A rows take turns over the row groups and k-steps
 #pragma unroll
                     for (int i = 0; i < TM; ++i)
-                        if ((i + kk / WGK) % WGN == wn)
-                            ln_accumulate<DT>(fa[i], ln_s1[i], ln_s2[i]);
+                        if ((i + ks) % WGN == wn)
+                            ln_take(fa[slot][i], i);
                 }
 #pragma unroll
                 for (int i = 0; i < TM; ++i)
 #pragma unroll
                     for (int j = 0; j < TN; ++j)
-                        GemmTraits<DT>::mma(fb[j], fa[i], acc[i][j]);
+                        GemmTraits<DT>::mma(fb[slot][j], fa[slot][i], acc[i][j]);
             }
         };
         constexpr int LPW = A_LD + B_LD;
@@ -1186,8 +1312,13 @@ __global__ void __launch_bounds__(CFG::NT)
         // one slab; with_sums (the last slab in the late form) also requests the row sums
         auto step = [&](int kt, auto with_sums) __attribute__((always_inline)) {
             // slab kt has landed once at most the loads of the slabs issued after it are outstanding
-            if (NS == 3 && kt + 1 < nk)
-                TR_WAIT_VMCNT(LPW);
+            const int behind = nk - 1 - kt;
+            if (NS > 4 && behind >= 3)
+                TR_WAIT_VMCNT(NS > 4 ? 3 * LPW : 0);
+            else if (NS > 3 && behind >= 2)
+                TR_WAIT_VMCNT(NS > 3 ? 2 * LPW : 0);
+            else if (NS > 2 && behind >= 1)
+                TR_WAIT_VMCNT(NS > 2 ? LPW : 0);
             else
                 TR_WAIT_VMCNT(0);
             // everyone's part of slab kt is in LDS, and everyone is done reading slab kt - 1 (its fragments were
@@ -1197,11 +1328,12 @@ __global__ void __launch_bounds__(CFG::NT)
             if (kt == 0)
                 TR_TL(1);  // first slab landed
             asm volatile("" ::: "memory");  // no LDS access may be moved across the barrier by the compiler
-            if (kt + NS - 1 < nk)
-                issue(kt + NS - 1, fill);
-            if constexpr (decltype(with_sums)::value)
-                request_sums();
-            compute(stage);
+            compute(stage, [&]() __attribute__((always_inline)) {
+                if (kt + NS - 1 < nk)
+                    issue(kt + NS - 1, fill);
+                if constexpr (decltype(with_sums)::value)
+                    request_sums();
+            });
             stage = stage + 1 == NS ? 0 : stage + 1;
             fill  = fill + 1 == NS ? 0 : fill + 1;
         };
@@ -1321,7 +1453,7 @@ __global__ void __launch_bounds__(CFG::NT)
     // LayerNorm-folding epilogues: reduce the lanes' partial row sums over the two k-halves of a fragment and the WGK
     // k-waves (fixed order), giving {rstd, mean} per tile row; both arrays sit behind the staging area
     float2 *const row_st   = reinterpret_cast<float2 *>(lds_dyn + (TakesRowSums<Epi>::value ? CFG::lds_bytes : CFG::stage_bytes));  // [BM]
-    float2 *const row_part = row_st + BM;                                             // [WGK * WGN * 2][BM]
+    double2 *const row_part = reinterpret_cast<double2 *>(row_st + BM);               // [WGK * WGN][BM]
     int8_t *const lut_lds = reinterpret_cast<int8_t *>(lds_dyn + CFG::stage_bytes);  // Int8Epilogue's table, 256 bytes
     if constexpr (std::is_same<Epi, Int8Epilogue>::value) {
         if (epi.lut && tid < 64)
@@ -1354,15 +1486,18 @@ __global__ void __launch_bounds__(CFG::NT)
     if constexpr (Epi::kRowStats && !TakesRowSums<Epi>::value) {
         static_assert(CFG::NSTAGE > 0, "LayerNorm-folding epilogues run on the direct-to-LDS pipeline");
 #pragma unroll
-        for (int i = 0; i < TM; ++i)
-            row_part[((wk * WGN + wn) * 2 + (lane >> 5)) * BM + (wm * TM + i) * 32 + frag_row] = make_float2(ln_s1[i], ln_s2[i]);
+        for (int i = 0; i < TM; ++i) {
+            const double s1 = ln_s1[i] + __shfl_xor(ln_s1[i], 32, 64), s2 = ln_s2[i] + __shfl_xor(ln_s2[i], 32, 64);
+            if (lane < 32)
+                row_part[(wk * WGN + wn) * BM + (wm * TM + i) * 32 + frag_row] = make_double2(s1, s2);
+        }
         __syncthreads();
         if (tid < BM) {
             double s1 = 0.0, s2 = 0.0;
-            for (int q = 0; q < WGK * WGN * 2; ++q) {
-                float2 v = row_part[q * BM + tid];
-                s1 += (double)v.x;
-                s2 += (double)v.y;
+            for (int q = 0; q < WGK * WGN; ++q) {
+                const double2 v = row_part[q * BM + tid];
+                s1 += v.x;
+                s2 += v.y;
             }
             const double mean = s1 * (double)epi.ln.inv_cols;
             const double var  = s2 * (double)epi.ln.inv_cols - mean * mean;
@@ -1531,8 +1666,9 @@ __global__ void __launch_bounds__(CFG::NT)
     TR_TL(4);  // kernel end
 }
 
-// internal: the chosen tile shape leaves no LDS for the row-sum side output; the caller launches the plain form
-constexpr int kTileTooLargeForSums = -12345;
+// internal: the chosen tile shape does not leave row sums (no LDS, too many tile columns) or does not take them; the
+// caller launches the form without
+constexpr int kNotWithRowSums = -12345;
 thread_local int t_last_tiles_n = 0;  // tile columns of this thread's last tiled launch (the row-sum block count)
 
 template <int DT, typename CFG, typename Epi>
@@ -1541,12 +1677,14 @@ int launch_tiled(hipStream_t s, const void *A, const void *B, int M, int N, int 
     int tiles_m = (M + CFG::BM - 1) / CFG::BM, tiles_n = (N + CFG::BN - 1) / CFG::BN;
     typedef EpiLds<CFG, Epi> L;
     const size_t lds = L::total;
+    if (EmitsRowSums<Epi>::value && tiles_n > kMaxRowSumBlocks)
+        return kNotWithRowSums;
     if (EmitsRowSums<Epi>::value) {
         // the row sums are not taken at the price of a workgroup per CU (the plain form runs instead)
         const size_t without = L::plain + L::side_bytes + 16;
         const long cu = 160 * 1024;
         if (lds > (size_t)cu || cu / (long)(lds + 1024) < (cu / (long)(without + 1024) > 4 ? 4 : cu / (long)(without + 1024)))
-            return kTileTooLargeForSums;
+            return kNotWithRowSums;
     }
     auto kern   = gemm_nk_tiled_kernel<DT, CFG, Epi>;
     if (lds > 64 * 1024) {
@@ -1582,44 +1720,81 @@ int launch_tiled(hipStream_t s, const void *A, const void *B, int M, int N, int 
     return 0;
 }
 
-// Configuration codes: TM TN WGM WGN WGK S (one decimal digit each; slab bytes = 64 << S).
-//   112210 / 112211   64 x  64, 4 waves                 222210  128 x 128, 4 waves
-//   222221           128 x 128, 8 waves (two k-waves)   224211  256 x 128, 8 waves
-//   332221           192 x 192, 8 waves (two k-waves)   331182   96 x  96, 8 k-waves, 256-byte slabs
-//   111182            32 x  32, 8 k-waves, 256-byte slabs (fp32 only: small products)
+// Configuration codes: [P] TM TN WGM WGN WGK S (one decimal digit each; slab bytes = 64 << S; P = number of
+// direct-to-LDS stages, 9 = rings of the waves' own, absent = slabs staged through registers).
+//   9111141   32 x  32, 4 k-waves with rings of their own     9121141   32 x  64, likewise
+//   3112221   64 x  64, 8 waves (two k-waves), 3 stages       3112222   64 x  64, 8 waves, 256-byte slabs
+//   4221141   64 x  64, 4 k-waves, 4 stages                   3212221  128 x  64, 8 waves
+//   2112211   64 x  64, 4 waves, 2 stages                     2222221  128 x 128, 8 waves (two k-waves)
+//   3332221  192 x 192, 8 waves (two k-waves)                 3331182   96 x  96, 8 k-waves, 256-byte slabs
+//   112210    64 x  64 and 222210 128 x 128, 4 waves: rows that are no multiple of 128 bytes
 // Eight-wave workgroups put two waves on every SIMD inside one tile: while one waits for its LDS fragments the
 // other issues MFMAs, and a larger tile per CU moves fewer bytes through LDS and L2 per flop.  Four-wave tiles
 // larger than 128 x 128 (one wave per SIMD) were measured and never won with compiler-scheduled code.
 constexpr int kNumCU = 256;
 
-// Shape heuristic, from measurements on MI355X (fp16; M in {1024, 3072, 4096, 16384}, N and K in
-// {768, 1024, 2304, 3072, 4096}; times in us, best alternative in parentheses):
-//   * default 128x128 with eight waves: M=4096 N=3072 K=1024 37 (4 waves 43), M=4096 N=1024 K=4096 45 (54),
-//     M=16384 N=3072 K=768 122 (135), M=16384 N=768 K=3072 95 (106);
-//   * small launches (at most ~0.6 tiles of 128x128 per CU): 64x64 tiles keep every CU busy
-//     (M=3072 N=768 K=768 12.4 vs 12.9; M=1024 shapes 9.5-19 vs 13-35);
-//   * a narrow N with a long K and about one 96x96 tile per CU: eight k-waves on one 96x96 tile
-//     (M=3072 N=768 K=3072 25.6 vs 30.7);
-//   * between one and two 128x128 tiles per CU: 256x128 when that is a single round (M=3072 N=2304 19.7 vs 20.6);
-//   * slightly more than one round of 128x128 at two workgroups per CU, but a single round of 192x192
-//     (M=3072 N=3072: 576 tiles for 512 slots): 192x192 (28.8 vs 31.9).
-inline int pick_tile_config(long M, long N, size_t kbytes) {
-    auto tiles = [&](int bm, int bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
-    const long t128 = tiles(128, 128), slots = 2 * kNumCU;
-    if (kbytes % 128 != 0)
-        return t128 > kNumCU ? 222210 : 112210;
-    if (kbytes >= 4096 && kbytes % 256 == 0) {
-        const long t96 = tiles(96, 96);
-        if (t96 <= kNumCU && t96 > kNumCU / 2 && t128 <= kNumCU)
-            return 331182;
+// What a launch takes on this chip with each tile shape.  The busiest CU works through n = ceil(tiles / 256) tiles, up to
+// `slots` of them side by side (what its LDS and registers hold): full sets of `slots`, then the rest.  A set costs its
+// number of 128-byte k-slabs times slab[its tiles - 1], every set after the first also `round` (ramp and epilogue that
+// nothing covers), and the launch `fixed`; microseconds.  The figures are a least-squares fit to 800 launches (fp16 and int8:
+// M from 16 to 8192, the four projections of hidden sizes 768 and 1024 with their fused epilogues; fp32: M from 16 to
+// 3072), taken over twelve weight sets in turn so that weights come from the memory-side cache as they do inside a
+// network.  The shape it picks is on average 1.4 % (fp16), 0.6 % (int8), 2.7 % (fp32) behind the best of the shapes for the
+// same launch; the rules it replaced, made for M >= 1024, were 51 %, 34 % and 77 % behind over that range:
+//   M=  32 N= 768 K=3072 fp16  23.1 -> 7.3 us   (64x64 tiles: 12 CUs, one two-stage slab after another)
+//   M= 256 N= 768 K=3072 fp16  23.7 -> 7.2      M= 256 N=2304 K=768 fp16  8.7 -> 6.2
+//   M=1000 N= 768 K=3072 fp16  24.3 -> 12.4     M=1000 N= 768 K=768 fp16  8.7 -> 5.5
+struct TileCost {
+    int code, bm, bn, slots;
+    float fixed, round, slab[4];
+};
+constexpr TileCost kTilesHalf[] = {
+    {9111141, 32, 32, 2, 3.47f, 2.09f, {0.067f, 0.147f}},
+    {9121141, 32, 64, 1, 3.46f, 2.56f, {0.121f}},
+    {3112221, 64, 64, 3, 3.72f, 3.06f, {0.205f, 0.377f, 0.654f}},
+    {3112222, 64, 64, 1, 3.45f, 3.09f, {0.179f}},
+    {3212221, 128, 64, 2, 4.60f, 5.12f, {0.287f, 0.607f}},
+    {4221141, 64, 64, 2, 4.34f, 3.22f, {0.158f, 0.351f}},
+    {2112211, 64, 64, 4, 2.96f, 1.83f, {0.411f, 0.493f, 0.607f, 0.877f}},
+    {2222221, 128, 128, 2, 4.84f, 5.77f, {0.561f, 1.044f}},
+    {3332221, 192, 192, 1, 10.15f, 13.25f, {0.767f}},
+    {3331182, 96, 96, 1, 6.94f, 7.10f, {0.264f}},
+};
+constexpr TileCost kTilesI8[] = {
+    {9111141, 32, 32, 2, 2.98f, 1.93f, {0.078f, 0.151f}},
+    {9121141, 32, 64, 1, 3.25f, 2.21f, {0.130f}},
+    {3112221, 64, 64, 3, 3.40f, 2.05f, {0.218f, 0.398f, 0.701f}},
+    {3112222, 64, 64, 1, 3.09f, 2.21f, {0.196f}},
+    {3212221, 128, 64, 2, 4.05f, 3.04f, {0.313f, 0.644f}},
+    {4221141, 64, 64, 2, 4.06f, 2.67f, {0.174f, 0.389f}},
+    {2112211, 64, 64, 4, 3.00f, 1.56f, {0.424f, 0.558f, 0.687f, 0.944f}},
+    {2222221, 128, 128, 2, 5.15f, 3.79f, {0.640f, 1.156f}},
+    {3332221, 192, 192, 1, 9.89f, 9.10f, {0.860f}},
+    {3331182, 96, 96, 1, 6.72f, 5.80f, {0.314f}},
+};
+// fp32 MFMAs take 16 times the matrix-pipe time of half ones: the pipe is the bound and what counts is an even spread
+constexpr TileCost kTilesF32[] = {
+    {9111141, 32, 32, 2, 3.80f, 3.25f, {0.141f, 0.275f}},
+    {9121141, 32, 64, 1, 4.24f, 3.76f, {0.257f}},
+    {2112211, 64, 64, 4, 4.37f, 3.17f, {0.548f, 1.019f, 1.490f, 2.032f}},
+    {4221141, 64, 64, 2, 4.94f, 4.95f, {0.500f, 0.995f}},
+};
+
+template <int COUNT> inline int pick_tile_config(const TileCost (&shapes)[COUNT], long M, long N, size_t kbytes) {
+    int best        = 0;
+    float best_cost = 0.f;
+    const float slabs = (float)(kbytes / 128);
+    for (const TileCost &t : shapes) {
+        if (kbytes % (64u << (t.code % 10)) != 0)
+            continue;
+        const long tiles = ((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn), n = (tiles + kNumCU - 1) / kNumCU;
+        const long sets = n / t.slots, rest = n % t.slots;
+        float cost = t.fixed + slabs * ((float)sets * t.slab[t.slots - 1] + (rest ? t.slab[rest - 1] : 0.f)) +
+                     t.round * (float)(sets + (rest ? 1 : 0) - 1);
+        if (best == 0 || cost < best_cost)
+            best = t.code, best_cost = cost;
     }
-    if (t128 * 10 <= kNumCU * 6)
-        return 112211;
-    if (t128 > kNumCU && t128 <= slots && tiles(256, 128) <= kNumCU)
-        return 224211;
-    if (t128 > slots && t128 < slots + slots / 4 && tiles(192, 192) <= kNumCU)
-        return 332221;
-    return 222221;
+    return best;
 }
 
 template <int DT, typename Epi>
@@ -1629,40 +1804,25 @@ int launch_gemm_fast(hipStream_t s, const void *A, const void *B, int M, int N, 
     const int forced = g_gemm_force_cfg;
     int cfg       = forced > 0 ? forced : tune_override(N, K, nullptr);
     size_t kbytes = (size_t)K * sizeof(T);
+    // direct-to-LDS loads address a panel with a 32-bit byte offset
+    const bool wide = (size_t)M * lda * sizeof(T) >= (1ull << 32) || (size_t)N * ldb * sizeof(T) >= (1ull << 32);
     if (cfg == 0) {
-        // slabs that are whole 128-byte multiples go global -> LDS directly; average kernel durations inside a
-        // 12-layer forward at M=3072 on MI355X (fp16, us, register-staged in parentheses): 192x192 three stages
-        // N=3072 K=768 26.7 (28.7); 96x96 k-split three stages N=768 K=3072 25.9 (28.0); 64x64 two stages
-        // N=768 K=768 11.4 (12.3); 128x128 two stages N=2304 K=768 19.1 (256x128 register-staged 20.5)
-        int code = pick_tile_config(M, N, kbytes);
-        if (DT == TNN_ROCM_I8 && kbytes % 128 == 0) {
-            // int8 tiles finish their K loop in half the slabs, so the fixed cost per tile weighs more and small tiles
-            // that fill every CU win earlier than for fp16.  Inside the 12-layer int8 encoder at M=4096 (forward
-            // 1.258 ms): 64x64 for N=768 (192 tiles of 128x128, K=768 and K=3072) and for N=2304 (576 tiles of
-            // 128x128 for 512 slots, a second round for an eighth of the work) -> 1.216 ms.
-            const long t128 = (((long)M + 127) / 128) * (((long)N + 127) / 128), slots = 2 * kNumCU;
-            if (t128 < kNumCU || (code == 222221 && t128 > slots && t128 * 4 <= slots * 5))
-                code = 112211;
-        }
-        switch (code) {
-            case 112211: cfg = 2112211; break;
-            case 222221: cfg = 2222221; break;
-            case 224211: cfg = 2222221; break;  // two 128x128 workgroups per CU beat one 256x128 (19.1 vs 20.3)
-            case 332221: cfg = 3332221; break;
-            case 331182: cfg = 3331182; break;
-            default: cfg = code; break;
-        }
+        if (kbytes % 128 != 0 || wide)
+            cfg = (((long)M + 127) / 128) * (((long)N + 127) / 128) > kNumCU ? 222210 : 112210;
+        else if (DT == TNN_ROCM_F32)
+            cfg = pick_tile_config(kTilesF32, M, N, kbytes);
+        else if (DT == TNN_ROCM_I8)
+            cfg = pick_tile_config(kTilesI8, M, N, kbytes);
+        else
+            cfg = pick_tile_config(kTilesHalf, M, N, kbytes);
     }
-    if (DT == TNN_ROCM_F32 && (cfg % 1000000 == 224211 || cfg % 1000000 == 332221 || cfg % 1000000 == 331182))
-        cfg = 222221;
-    if (DT == TNN_ROCM_F32)
-        cfg %= 1000000;  // the fp32 instantiations are register-staged only
-    if (DT == TNN_ROCM_F32 && forced <= 0 && cfg == 112211 && kbytes % 256 == 0 && kbytes >= 2048 &&
-        (((long)M + 63) / 64) * (((long)N + 63) / 64) * 2 <= kNumCU) {
-        // A small fp32 product (one attention layer at 128 tokens: 24 tiles of 64x64) leaves nine CUs in ten idle,
-        // and the fp32 matrix pipe is 16 times slower than the fp16 one: 32x32 tiles with the K range dealt to
-        // eight waves put four times as many CUs to work on each a quarter of the MFMAs.
-        cfg = 111182;
+    switch (cfg) {  // a code of 128-byte or larger slabs without its stage digit
+        case 112211: cfg = 2112211; break;
+        case 222221:
+        case 224211: cfg = 2222221; break;
+        case 332221: cfg = 3332221; break;
+        case 331182: cfg = 3331182; break;
+        default: break;
     }
     if (kbytes % (64u << (cfg % 10)) != 0) {
         set_error("gemm: K=%d is not a whole number of slabs for tuning configuration %d", K, cfg);
@@ -1672,46 +1832,42 @@ int launch_gemm_fast(hipStream_t s, const void *A, const void *B, int M, int N, 
     return launch_tiled<DT, TileCfg<TMv, TNv, WGMv, WGNv, WGKv, SLABv>, Epi>(s, A, B, M, N, K, lda, ldb, epi)
 #define TR_FAST_DL(TMv, TNv, WGMv, WGNv, WGKv, SLABv, NSv)                                                            \
     return launch_tiled<DT, TileCfg<TMv, TNv, WGMv, WGNv, WGKv, SLABv, NSv>, Epi>(s, A, B, M, N, K, lda, ldb, epi)
-    if constexpr (Epi::kRowStats) {
-        // the LayerNorm-folding epilogues exist for the direct-to-LDS pipeline only (half types, 128-byte slabs)
-        switch (cfg % 1000000) {
-            case 112211: TR_FAST_DL(1, 1, 2, 2, 1, 128, 2);
-            case 222221:
-            case 224211: TR_FAST_DL(2, 2, 2, 2, 2, 128, 2);
-            case 332221: TR_FAST_DL(3, 3, 2, 2, 2, 128, 3);
-            case 331182: TR_FAST_DL(3, 3, 1, 1, 8, 256, 3);
+#define TR_FAST_OWN(TMv, TNv, WGKv, SLABv, NSv)                                                                       \
+    return launch_tiled<DT, TileCfg<TMv, TNv, 1, 1, WGKv, SLABv, NSv, true>, Epi>(s, A, B, M, N, K, lda, ldb, epi)
+    if constexpr (TakesRowSums<Epi>::value) {
+        if (cfg >= 9000000)
+            return kNotWithRowSums;
+    } else {
+        switch (cfg) {
+            case 9111141: TR_FAST_OWN(1, 1, 4, 128, 2);
+            case 9121141: TR_FAST_OWN(1, 2, 4, 128, 2);
             default: break;
         }
-        set_error("gemm: tuning configuration %d has no LayerNorm-folding form", cfg);
-        return TNN_ROCM_EINVAL;
-    } else {
-    switch (cfg) {
-        case 112210: TR_FAST(1, 1, 2, 2, 1, 64);
-        case 112211: TR_FAST(1, 1, 2, 2, 1, 128);
-        case 222210: TR_FAST(2, 2, 2, 2, 1, 64);
-        case 222221: TR_FAST(2, 2, 2, 2, 2, 128);
-        default: break;
     }
-    if constexpr (DT == TNN_ROCM_F32) {
-        if (cfg == 111182)
-            TR_FAST(1, 1, 1, 1, 8, 256);
+    switch (cfg) {
+        case 2112211: TR_FAST_DL(1, 1, 2, 2, 1, 128, 2);
+        case 4221141: TR_FAST_DL(2, 2, 1, 1, 4, 128, 4);
+        default: break;
     }
     if constexpr (DT != TNN_ROCM_F32) {
         switch (cfg) {
-            case 2112211: TR_FAST_DL(1, 1, 2, 2, 1, 128, 2);
+            case 3112221: TR_FAST_DL(1, 1, 2, 2, 2, 128, 3);
+            case 3112222: TR_FAST_DL(1, 1, 2, 2, 2, 256, 3);
+            case 3212221: TR_FAST_DL(2, 1, 2, 2, 2, 128, 3);
             case 2222221: TR_FAST_DL(2, 2, 2, 2, 2, 128, 2);
             case 3332221: TR_FAST_DL(3, 3, 2, 2, 2, 128, 3);
             case 3331182: TR_FAST_DL(3, 3, 1, 1, 8, 256, 3);
             default: break;
         }
+    }
+    if constexpr (!Epi::kRowStats) {  // the LayerNorm-folding epilogues exist for the direct-to-LDS pipelines only
         switch (cfg) {
-            case 224211: TR_FAST(2, 2, 4, 2, 1, 128);
-            case 332221: TR_FAST(3, 3, 2, 2, 2, 128);
-            case 331182: TR_FAST(3, 3, 1, 1, 8, 256);
+            case 112210: TR_FAST(1, 1, 2, 2, 1, 64);
+            case 222210: TR_FAST(2, 2, 2, 2, 1, 64);
             default: break;
         }
     }
-    }
+#undef TR_FAST_OWN
 #undef TR_FAST
 #undef TR_FAST_DL
     set_error("gemm: unknown tuning configuration %d", cfg);
@@ -1820,11 +1976,12 @@ int GemmTyped<DT>::ln(hipStream_t s, const void *t, const void *w_folded, const 
                       const float *row_sums, int row_sum_blocks, int M, int N, int K, int flags, const void *residual) {
     const LnFold ln{1.0f / (float)K, eps, colsum, gamma, beta, y, g_ln_y_ahead.load(), (float2 *)row_stats,
                     (const float2 *)row_sums, row_sum_blocks};
+    int rc = kNotWithRowSums;  // a tile shape that takes the statistics from its own tiles declines handed-over sums
     if (row_sums && row_sum_blocks <= 12)
-        return launch_ln<DT, 12>(s, t, w_folded, bias_folded, C, ln, M, N, K, flags, residual);
-    if (row_sums)
-        return launch_ln<DT, kMaxRowSumBlocks>(s, t, w_folded, bias_folded, C, ln, M, N, K, flags, residual);
-    return launch_ln<DT, 0>(s, t, w_folded, bias_folded, C, ln, M, N, K, flags, residual);
+        rc = launch_ln<DT, 12>(s, t, w_folded, bias_folded, C, ln, M, N, K, flags, residual);
+    else if (row_sums)
+        rc = launch_ln<DT, kMaxRowSumBlocks>(s, t, w_folded, bias_folded, C, ln, M, N, K, flags, residual);
+    return rc == kNotWithRowSums ? launch_ln<DT, 0>(s, t, w_folded, bias_folded, C, ln, M, N, K, flags, residual) : rc;
 }
 
 template <int DT, int SUMS>
@@ -1850,10 +2007,13 @@ int GemmTyped<DT>::qkv_split_ln(hipStream_t s, const void *t, const void *wqkv_f
                                 int K, int vt_key_order) {
     const LnFold ln{1.0f / (float)K, eps, colsum, gamma, beta, y, g_ln_y_ahead.load(), (float2 *)row_stats,
                     (const float2 *)row_sums, row_sum_blocks};
+    int rc = kNotWithRowSums;
     if (row_sums && row_sum_blocks <= 12)
-        return launch_qkv_split_ln<DT, 12>(s, t, wqkv_folded, bqkv_folded, qk, vt, ln, B, S, heads, K, vt_key_order);
-    if (row_sums)
-        return launch_qkv_split_ln<DT, kMaxRowSumBlocks>(s, t, wqkv_folded, bqkv_folded, qk, vt, ln, B, S, heads, K, vt_key_order);
+        rc = launch_qkv_split_ln<DT, 12>(s, t, wqkv_folded, bqkv_folded, qk, vt, ln, B, S, heads, K, vt_key_order);
+    else if (row_sums)
+        rc = launch_qkv_split_ln<DT, kMaxRowSumBlocks>(s, t, wqkv_folded, bqkv_folded, qk, vt, ln, B, S, heads, K, vt_key_order);
+    if (rc != kNotWithRowSums)
+        return rc;
     return launch_qkv_split_ln<DT, 0>(s, t, wqkv_folded, bqkv_folded, qk, vt, ln, B, S, heads, K, vt_key_order);
 }
 
@@ -1885,7 +2045,7 @@ int GemmTyped<DT>::residual_ln(hipStream_t s, const void *x, const void *w, cons
         const int rc = launch_residual_ln<DT, true>(s, x, w, bias, C, t, row_stats, gamma, beta, M, N, K, flags, row_sums);
         if (rc == 0)
             *row_sum_blocks = t_last_tiles_n;
-        if (rc != kTileTooLargeForSums)
+        if (rc != kNotWithRowSums)
             return rc;
     }
     return launch_residual_ln<DT, false>(s, x, w, bias, C, t, row_stats, gamma, beta, M, N, K, flags, nullptr);
