@@ -64,6 +64,10 @@ TNN_ROCM_API int tnn_rocm_memset(void *ptr, int value, size_t bytes, void *strea
 TNN_ROCM_API int tnn_rocm_memcpy_h2d(void *dst, const void *host_src, size_t bytes, void *stream);
 TNN_ROCM_API int tnn_rocm_memcpy_d2h(void *host_dst, const void *src, size_t bytes, void *stream);
 TNN_ROCM_API int tnn_rocm_memcpy_d2d(void *dst, const void *src, size_t bytes, void *stream);
+/* Copy by a kernel on the stream, returning when it is enqueued: dst and src are device memory or memory of
+ * tnn_rocm_malloc_host (which the device reads and writes in place).  For the small transfers of a request: the runtime's
+ * own copies of pageable memory wait for the stream, and cost several launches' time of host work. */
+TNN_ROCM_API int tnn_rocm_copy_mapped(void *dst, const void *src, size_t bytes, void *stream);
 TNN_ROCM_API int tnn_rocm_stream_create(void **stream);
 TNN_ROCM_API int tnn_rocm_stream_destroy(void *stream);
 TNN_ROCM_API int tnn_rocm_stream_sync(void *stream);

@@ -68,7 +68,9 @@ int tnn_host_share_command_queue(void *handle, void *other);
 int tnn_host_set_cpu_num_threads(void *handle, int num_threads);
 /* Instance::GetCommandQueue (instance.h:71): the hipStream_t the instance launches on */
 void *tnn_host_stream(void *handle);
-/* Instance::GetOutputMat (instance.h:128) converted to fp32 NCHW on the host.  dims must hold 8 ints. */
+/* The current dims of an output blob, so that a caller can allocate what the calls below fill.  dims must hold 8 ints. */
+int tnn_host_output_dims(void *handle, const char *name, int *dims, int *ndims);
+/* Instance::GetOutputMat (instance.h:128) converted to fp32 NCHW on the host, straight into out.  dims must hold 8 ints. */
 int tnn_host_get_output(void *handle, const char *name, float *out, size_t capacity, int *dims, int *ndims);
 /* The same through a Mat of the caller's choice (mat_type as for tnn_host_set_input; RESERVED_INT8_TEST hands out an int8
  * blob's values as they are, blob_converter_default.cc:347-350); capacity in bytes. */

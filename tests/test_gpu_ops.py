@@ -1371,3 +1371,29 @@ def test_gemm_i8_with_gelu_table_bit_exact(M, N, K):
     ref = orc.quantize_x86(orc.gelu(orc.dequantize(ref_q, s_mid)), s_out)
     assert np.array_equal(fused, ref)
     assert len(np.unique(host(q))) > 100                    # the requantised values span the int8 range
+
+
+@pytest.mark.parametrize("bytes_,offset", [(1, 0), (15, 0), (16, 0), (4099, 0), (4099, 4), (5 << 20, 0)])
+def test_copy_mapped_both_ways(bytes_, offset):
+    """The kernel copy between page-locked host memory and device memory: single bytes, a tail behind whole vectors,
+    pointers that are not 16-byte aligned, more vectors than the grid has lanes."""
+    import ctypes
+    from tnn_amd import capi
+    lib = capi.load()
+    say("copy_mapped %d bytes, offset %d" % (bytes_, offset))
+    src = np.random.default_rng(bytes_).integers(0, 256, bytes_ + offset, dtype=np.uint8)
+    pinned = ctypes.c_void_p()
+    assert lib.tnn_rocm_malloc_host(ctypes.byref(pinned), bytes_ + offset + 16) == 0
+    try:
+        view = np.ctypeslib.as_array(ctypes.cast(pinned, ctypes.POINTER(ctypes.c_uint8)), (bytes_ + offset + 16,))
+        view[:bytes_ + offset] = src
+        on_device = torch.zeros(bytes_ + 16, dtype=torch.uint8, device="cuda")
+        capi.call("tnn_rocm_copy_mapped", on_device.data_ptr(), pinned.value + offset, bytes_, None)
+        torch.cuda.synchronize()
+        assert np.array_equal(host(on_device)[:bytes_], src[offset:]) and not host(on_device)[bytes_:].any()
+        view[:] = 0
+        capi.call("tnn_rocm_copy_mapped", pinned.value + offset, on_device.data_ptr(), bytes_, None)
+        torch.cuda.synchronize()
+        assert np.array_equal(view[offset:bytes_ + offset], src[offset:]) and not view[bytes_ + offset:].any()
+    finally:
+        lib.tnn_rocm_free_host(pinned)

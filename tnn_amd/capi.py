@@ -28,6 +28,7 @@ SIGNATURES = {
     "tnn_rocm_memcpy_h2d": [_vp, _vp, _sz, _vp],
     "tnn_rocm_memcpy_d2h": [_vp, _vp, _sz, _vp],
     "tnn_rocm_memcpy_d2d": [_vp, _vp, _sz, _vp],
+    "tnn_rocm_copy_mapped": [_vp, _vp, _sz, _vp],
     "tnn_rocm_stream_create": [C.POINTER(_vp)],
     "tnn_rocm_stream_destroy": [_vp],
     "tnn_rocm_stream_sync": [_vp],

@@ -1,6 +1,7 @@
 """ctypes front-end of the C++ host (tnn_amd/lib/libtnn_rocm_host.so): an engine Instance on DEVICE_ROCM created
 from .tnnproto text + .tnnmodel bytes.  No fallback: a missing library or a failed call raises."""
 import ctypes as C
+import math
 import os
 
 import numpy as np
@@ -37,6 +38,7 @@ SIGNATURES = {
     "tnn_host_forward_with_callback": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p]),
     "tnn_host_share_command_queue": (C.c_int, [C.c_void_p, C.c_void_p]),
     "tnn_host_set_cpu_num_threads": (C.c_int, [C.c_void_p, C.c_int]),
+    "tnn_host_output_dims": (C.c_int, [C.c_void_p, C.c_char_p, C.POINTER(C.c_int), C.POINTER(C.c_int)]),
     "tnn_host_get_output": (C.c_int, [C.c_void_p, C.c_char_p, C.c_void_p, C.c_size_t, C.POINTER(C.c_int),
                                       C.POINTER(C.c_int)]),
     "tnn_host_get_output_as": (C.c_int, [C.c_void_p, C.c_char_p, C.c_int, C.c_void_p, C.c_size_t, C.POINTER(C.c_int),
@@ -248,25 +250,22 @@ class RocmInstance:
         return load().tnn_host_stream(self._h)
 
     def output(self, name="", max_elems=1 << 25):
-        buf = np.empty(max_elems, np.float32)
-        dims = (C.c_int * 8)()
-        nd = C.c_int(0)
-        self._check(load().tnn_host_get_output(self._h, name.encode(), buf.ctypes.data_as(C.c_void_p), max_elems, dims,
-                                               C.byref(nd)), "GetOutputMat")
-        shape = [dims[i] for i in range(nd.value)]
-        return buf[:int(np.prod(shape, dtype=np.int64))].reshape(shape).copy()
+        return self.output_as(name, np.float32, max_elems)
 
     def output_as(self, name, dtype, max_elems=1 << 25):
         """the output through a Mat of the given numpy type: float32, int32, int8 (an int8 blob's values as they are),
         float16, or uint16 (bfloat16 bit patterns)"""
-        dtype = np.dtype(dtype)
-        buf = np.empty(max_elems, dtype)
+        lib, dtype = load(), np.dtype(dtype)
         dims = (C.c_int * 8)()
         nd = C.c_int(0)
-        self._check(load().tnn_host_get_output_as(self._h, name.encode(), _MAT_CODE[dtype], buf.ctypes.data_as(C.c_void_p),
-                                                  buf.nbytes, dims, C.byref(nd)), "GetOutputMat")
-        shape = [dims[i] for i in range(nd.value)]
-        return buf[:int(np.prod(shape, dtype=np.int64))].reshape(shape).copy()
+        self._check(lib.tnn_host_output_dims(self._h, name.encode(), dims, C.byref(nd)), "GetOutputMat")
+        shape = dims[:nd.value]
+        # an array of exactly the output's size: the allocator hands the memory of the last one out again, where a fresh
+        # mapping costs a page fault for every 4 KB
+        out = np.empty(shape if math.prod(shape) <= max_elems else 0, dtype)
+        self._check(lib.tnn_host_get_output_as(self._h, name.encode(), _MAT_CODE[dtype], out.ctypes.data, out.nbytes, dims,
+                                               C.byref(nd)), "GetOutputMat")
+        return out
 
     def time_loop(self, warmup, iters, out_name):
         """the engine benchmark tool's loop (SetInputMat for every input set so far + Forward + GetOutputMat per

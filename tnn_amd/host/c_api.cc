@@ -153,10 +153,11 @@ HOST_API int tnn_host_set_input(void *hp, const char *name, const void *data, in
     Status st = h->inst->SetInputMat(mat, MatConvertParam(), name ? name : "");
     if (st != TNN_OK)
         return fail(h, st);
-    auto keep = std::make_shared<Mat>(DEVICE_NAIVE, mat->GetMatType(), d);  // owns its memory
+    auto &keep = h->inputs[name ? name : ""];
+    if (!keep || keep->GetMatType() != mat->GetMatType() || keep->GetDims() != d)
+        keep = std::make_shared<Mat>(DEVICE_NAIVE, mat->GetMatType(), d);  // owns its memory
     if (keep->GetData() && data)
         memcpy(keep->GetData(), data, (size_t)DimsVectorUtils::Count(d) * MatElemBytes(mat_type));
-    h->inputs[name ? name : ""] = keep;
     return 0;
 }
 
@@ -375,48 +376,44 @@ HOST_API void *tnn_host_stream(void *hp) {
     return q;
 }
 
-HOST_API int tnn_host_get_output(void *hp, const char *name, float *out, size_t capacity, int *dims, int *ndims) {
-    auto h = static_cast<Handle *>(hp);
-    std::shared_ptr<Mat> mat;
-    Status st = h->inst->GetOutputMat(mat, MatConvertParam(), name ? name : "", DEVICE_NAIVE, NCHW_FLOAT);
+// the dims of an output, and whether its elements fit the caller's buffer
+static int OutputDims(Handle *h, const char *name, size_t capacity_elems, DimsVector *d, int *dims, int *ndims) {
+    Status st = h->inst->GetOutputDims(*d, name ? name : "");
     if (st != TNN_OK)
         return fail(h, st);
-    DimsVector d = mat->GetDims();
-    size_t count = (size_t)DimsVectorUtils::Count(d);
     if (ndims)
-        *ndims = (int)d.size();
+        *ndims = (int)d->size();
     if (dims)
-        for (size_t i = 0; i < d.size() && i < 8; ++i)
-            dims[i] = d[i];
-    if (count > capacity) {
+        for (size_t i = 0; i < d->size() && i < 8; ++i)
+            dims[i] = (*d)[i];
+    if ((size_t)DimsVectorUtils::Count(*d) > capacity_elems) {
         h->err = "output buffer too small";
         return -2;
     }
-    memcpy(out, mat->GetData(), count * sizeof(float));
     return 0;
 }
 
-// GetOutputMat through a Mat of the caller's choice (codes of tnn_host_set_input); capacity in bytes
+HOST_API int tnn_host_output_dims(void *hp, const char *name, int *dims, int *ndims) {
+    DimsVector d;
+    return OutputDims(static_cast<Handle *>(hp), name, (size_t)-1, &d, dims, ndims);
+}
+
+// GetOutputMat through a Mat of the caller's choice (codes of tnn_host_set_input) over the caller's own buffer: the
+// conversion writes there, no Mat of the instance's lies in between; capacity in bytes
 HOST_API int tnn_host_get_output_as(void *hp, const char *name, int mat_type, void *out, size_t capacity_bytes, int *dims,
                                     int *ndims) {
     auto h = static_cast<Handle *>(hp);
-    std::shared_ptr<Mat> mat;
-    Status st = h->inst->GetOutputMat(mat, MatConvertParam(), name ? name : "", DEVICE_NAIVE, MatTypeOf(mat_type));
-    if (st != TNN_OK)
-        return fail(h, st);
-    DimsVector d = mat->GetDims();
-    size_t bytes = (size_t)DimsVectorUtils::Count(d) * MatElemBytes(mat_type);
-    if (ndims)
-        *ndims = (int)d.size();
-    if (dims)
-        for (size_t i = 0; i < d.size() && i < 8; ++i)
-            dims[i] = d[i];
-    if (bytes > capacity_bytes) {
-        h->err = "output buffer too small";
-        return -2;
-    }
-    memcpy(out, mat->GetData(), bytes);
-    return 0;
+    DimsVector d;
+    int rc = OutputDims(h, name, capacity_bytes / MatElemBytes(mat_type), &d, dims, ndims);
+    if (rc != 0)
+        return rc;
+    Mat mat(DEVICE_NAIVE, MatTypeOf(mat_type), d, out);
+    Status st = h->inst->ConvertOutput(mat, MatConvertParam(), name ? name : "");
+    return st == TNN_OK ? 0 : fail(h, st);
+}
+
+HOST_API int tnn_host_get_output(void *hp, const char *name, float *out, size_t capacity, int *dims, int *ndims) {
+    return tnn_host_get_output_as(hp, name, 0, out, capacity * sizeof(float), dims, ndims);
 }
 
 HOST_API int tnn_host_layer_count(void *hp) { return static_cast<Handle *>(hp)->inst->GetNetwork()->LayerCount(); }

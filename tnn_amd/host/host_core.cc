@@ -1694,22 +1694,42 @@ Status Instance::SetInputMat(std::shared_ptr<Mat> mat, MatConvertParam param, st
     return conv.second->ConvertFromMatAsync(*mat, param, q);  // instance.cc:241: the forward that follows is on the same queue
 }
 
-Status Instance::GetOutputMat(std::shared_ptr<Mat> &mat, MatConvertParam param, std::string output_name,
-                              DeviceType device, MatType mat_type) {
+Status Instance::FindOutput(std::string *output_name, Blob **blob) {
     BlobMap outs;
     network_->GetAllOutputBlobs(outs);
     if (outs.empty())
         return Status(TNNERR_COMMON_ERROR, "instance.GetAllOutputBlobs Error");
+    auto it = output_name->empty() ? outs.begin() : outs.find(*output_name);
+    if (it == outs.end())
+        return Status(TNNERR_MODEL_ERR, "instance dont have the output with name: " + *output_name);
+    *output_name = it->first;
+    *blob        = it->second;
+    return TNN_OK;
+}
+
+Status Instance::GetOutputDims(DimsVector &dims, const std::string &output_name) {
+    std::string name = output_name;
+    Blob *blob       = nullptr;
+    RETURN_ON_NEQ(FindOutput(&name, &blob), TNN_OK);
+    dims = blob->GetBlobDesc().dims;
+    return TNN_OK;
+}
+
+Status Instance::ConvertOutput(Mat &mat, MatConvertParam param, std::string output_name) {
     Blob *blob = nullptr;
-    if (output_name.empty()) {
-        blob        = outs.begin()->second;
-        output_name = outs.begin()->first;
-    } else {
-        auto it = outs.find(output_name);
-        if (it == outs.end())
-            return Status(TNNERR_MODEL_ERR, "instance dont have the output with name: " + output_name);
-        blob = it->second;
-    }
+    RETURN_ON_NEQ(FindOutput(&output_name, &blob), TNN_OK);
+    void *q = nullptr;
+    network_->GetCommandQueue(&q);
+    auto &conv = output_converters_[output_name];  // instance.cc:298-305
+    if (!conv.second || conv.first != blob)
+        conv = {blob, std::make_shared<BlobConverter>(blob)};
+    return conv.second->ConvertToMat(mat, param, q);
+}
+
+Status Instance::GetOutputMat(std::shared_ptr<Mat> &mat, MatConvertParam param, std::string output_name,
+                              DeviceType device, MatType mat_type) {
+    Blob *blob = nullptr;
+    RETURN_ON_NEQ(FindOutput(&output_name, &blob), TNN_OK);
     auto &cached = output_mats_[output_name];
     if (!cached || cached->GetMatType() != mat_type || cached->GetDeviceType() != device ||
         cached->GetDims() != blob->GetBlobDesc().dims) {
@@ -1719,12 +1739,7 @@ Status Instance::GetOutputMat(std::shared_ptr<Mat> &mat, MatConvertParam param, 
             return Status(TNNERR_OUTOFMEMORY, "no memory for the output mat on the device asked for");
         }
     }
-    void *q = nullptr;
-    network_->GetCommandQueue(&q);
-    auto &conv = output_converters_[output_name];  // instance.cc:298-305
-    if (!conv.second || conv.first != blob)
-        conv = {blob, std::make_shared<BlobConverter>(blob)};
-    RETURN_ON_NEQ(conv.second->ConvertToMat(*cached, param, q), TNN_OK);
+    RETURN_ON_NEQ(ConvertOutput(*cached, param, output_name), TNN_OK);
     mat = cached;
     return TNN_OK;
 }

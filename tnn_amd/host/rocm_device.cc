@@ -337,6 +337,7 @@ public:
         tnn_rocm_free(staging_);
         tnn_rocm_free(params_);
         tnn_rocm_free_host(bounce_);
+        tnn_rocm_free_host(stage_);
     }
 
     Status ConvertFromMat(Mat &mat, MatConvertParam param, void *q) override {
@@ -364,14 +365,12 @@ public:
         if (mat.GetMatType() == NC_INT32) {
             if (desc.data_type != DATA_TYPE_INT32)
                 return Status(TNNERR_PARAM_ERR, "NC_INT32 mat needs an int32 blob");
-            ROCM_CALL(tnn_rocm_memcpy_h2d(dst, mat.GetData(), count * 4, q));
-            return TNN_OK;
+            return FromHost(dst, mat.GetData(), count * 4, q);
         }
         if (mat.GetMatType() == RESERVED_INT8_TEST) {
             if (desc.data_type != DATA_TYPE_INT8)
                 return Status(TNNERR_PARAM_ERR, "int8 mat needs an int8 blob");
-            ROCM_CALL(tnn_rocm_memcpy_h2d(dst, mat.GetData(), count, q));
-            return TNN_OK;
+            return FromHost(dst, mat.GetData(), count, q);
         }
         if (mat.GetMatType() == RESERVED_BFP16_TEST || mat.GetMatType() == RESERVED_FP16_TEST) {
             // host values that are bfloat16 / half already (how the engine's layer test feeds a half-precision blob:
@@ -380,13 +379,11 @@ public:
             const DataType mt = mat.GetMatType() == RESERVED_BFP16_TEST ? DATA_TYPE_BFP16 : DATA_TYPE_HALF;
             if (desc.data_type != DATA_TYPE_FLOAT && desc.data_type != DATA_TYPE_HALF && desc.data_type != DATA_TYPE_BFP16)
                 return Status(TNNERR_PARAM_ERR, "a half or bfloat16 mat needs a float blob");
-            if (desc.data_type == mt) {
-                ROCM_CALL(tnn_rocm_memcpy_h2d(dst, mat.GetData(), count * 2, q));
-                return TNN_OK;
-            }
-            RETURN_ON_NEQ(Staging(count * 2), TNN_OK);
-            ROCM_CALL(tnn_rocm_memcpy_h2d(staging_, mat.GetData(), count * 2, q));
-            ROCM_CALL(tnn_rocm_cast(q, (int)mt, staging_, (int)desc.data_type, dst, count));
+            if (desc.data_type == mt)
+                return FromHost(dst, mat.GetData(), count * 2, q);
+            const void *seen = nullptr;
+            RETURN_ON_NEQ(ShowDevice(mat.GetData(), count * 2, q, &seen), TNN_OK);
+            ROCM_CALL(tnn_rocm_cast(q, (int)mt, seen, (int)desc.data_type, dst, count));
             return TNN_OK;
         }
         if (mat.GetMatType() != NCHW_FLOAT)
@@ -398,14 +395,12 @@ public:
             ApplyScaleBias(src, scaled.data(), desc.dims, param);
             src = scaled.data();
         }
-        if (desc.data_type == DATA_TYPE_FLOAT) {
-            ROCM_CALL(tnn_rocm_memcpy_h2d(dst, src, count * 4, q));
-            return TNN_OK;
-        }
-        RETURN_ON_NEQ(Staging(count * 4), TNN_OK);
-        ROCM_CALL(tnn_rocm_memcpy_h2d(staging_, src, count * 4, q));
+        if (desc.data_type == DATA_TYPE_FLOAT)
+            return FromHost(dst, src, count * 4, q);
         if (desc.data_type == DATA_TYPE_HALF || desc.data_type == DATA_TYPE_BFP16) {
-            ROCM_CALL(tnn_rocm_cast(q, TNN_ROCM_F32, staging_, (int)desc.data_type, dst, count));
+            const void *seen = nullptr;
+            RETURN_ON_NEQ(ShowDevice(src, count * 4, q, &seen), TNN_OK);
+            ROCM_CALL(tnn_rocm_cast(q, TNN_ROCM_F32, seen, (int)desc.data_type, dst, count));
         } else if (desc.data_type == DATA_TYPE_INT8) {
             // float mat into an int8 blob goes through the blob's scale (blob_converter_default.cc:396-403),
             // with the reciprocal-multiply quantiser of the x86 path
@@ -436,7 +431,9 @@ public:
             }
             float s   = sc[0];
             float inv = (float)(1.0 / s);
-            ROCM_CALL(tnn_rocm_quantize(q, TNN_ROCM_F32, staging_, inv, (int8_t *)dst, count));
+            const void *seen = nullptr;
+            RETURN_ON_NEQ(ShowDevice(src, count * 4, q, &seen), TNN_OK);
+            ROCM_CALL(tnn_rocm_quantize(q, TNN_ROCM_F32, seen, inv, (int8_t *)dst, count));
         } else {
             return Status(TNNERR_PARAM_ERR, "RocmBlobConverter: unsupported blob data type");
         }
@@ -456,12 +453,10 @@ public:
         if (mat.GetDeviceType() != DEVICE_NAIVE)
             return Status(TNNERR_PARAM_ERR, "RocmBlobConverter: the mat lives on another device");
         if (mat.GetMatType() == NC_INT32 && desc.data_type == DATA_TYPE_INT32) {
-            ROCM_CALL(tnn_rocm_memcpy_d2h(mat.GetData(), src, count * 4, q));
-            return TNN_OK;
+            return ToHost(mat.GetData(), src, count * 4, q);
         }
         if (mat.GetMatType() == RESERVED_INT8_TEST && desc.data_type == DATA_TYPE_INT8) {
-            ROCM_CALL(tnn_rocm_memcpy_d2h(mat.GetData(), src, count, q));
-            return TNN_OK;
+            return ToHost(mat.GetData(), src, count, q);
         }
         if (mat.GetMatType() == RESERVED_BFP16_TEST || mat.GetMatType() == RESERVED_FP16_TEST) {
             // the blob's values as bfloat16 / half on the host (blob_converter_default.cc:205-208, 245-249): copied from a
@@ -471,9 +466,10 @@ public:
                 return Status(TNNERR_PARAM_ERR, "a half or bfloat16 mat needs a float blob");
             if (desc.data_type == mt)
                 return ToHost(mat.GetData(), src, count * 2, q);
-            RETURN_ON_NEQ(Staging(count * 2), TNN_OK);
-            ROCM_CALL(tnn_rocm_cast(q, (int)desc.data_type, src, (int)mt, staging_, count));
-            return ToHost(mat.GetData(), staging_, count * 2, q);
+            void *made = nullptr;
+            RETURN_ON_NEQ(MakeForHost(count * 2, &made), TNN_OK);
+            ROCM_CALL(tnn_rocm_cast(q, (int)desc.data_type, src, (int)mt, made, count));
+            return ToHost(mat.GetData(), made, count * 2, q);
         }
         if (mat.GetMatType() != NCHW_FLOAT)
             return Status(TNNERR_PARAM_ERR, "RocmBlobConverter: unsupported mat type");
@@ -487,14 +483,16 @@ public:
                 out[i] = (float)iv[i];
         } else if (desc.data_type == DATA_TYPE_FLOAT) {
             RETURN_ON_NEQ(ToHost(mat.GetData(), src, count * 4, q), TNN_OK);
-        } else if (desc.data_type == DATA_TYPE_HALF && count * 2 >= kBounceMinBytes && CpuWidensHalf()) {
+        } else if ((desc.data_type == DATA_TYPE_HALF || desc.data_type == DATA_TYPE_BFP16) && count * 4 > kMappedMaxBytes &&
+                   CpuWidensHalf()) {
             // a large half-precision blob crosses the bus as it is (half the bytes of its fp32 form) and is widened on
             // the way from the page-locked buffer into the Mat, which replaces the plain copy of that step
-            RETURN_ON_NEQ(HalfToHostFloat((float *)mat.GetData(), src, count, q), TNN_OK);
+            RETURN_ON_NEQ(HalfToHostFloat((float *)mat.GetData(), src, count, desc.data_type == DATA_TYPE_HALF, q), TNN_OK);
         } else {
-            RETURN_ON_NEQ(Staging(count * 4), TNN_OK);
+            void *made = nullptr;
             if (desc.data_type == DATA_TYPE_HALF || desc.data_type == DATA_TYPE_BFP16) {
-                ROCM_CALL(tnn_rocm_cast(q, (int)desc.data_type, src, TNN_ROCM_F32, staging_, count));
+                RETURN_ON_NEQ(MakeForHost(count * 4, &made), TNN_OK);
+                ROCM_CALL(tnn_rocm_cast(q, (int)desc.data_type, src, TNN_ROCM_F32, made, count));
             } else if (desc.data_type == DATA_TYPE_INT8) {
                 auto bi = dynamic_cast<BlobInt8 *>(blob_);
                 if (!bi || !bi->GetIntResource() || bi->GetIntResource()->scale_handle.GetDataCount() < 1)
@@ -519,11 +517,12 @@ public:
                     return TNN_OK;
                 }
                 float s = sc[0];
-                ROCM_CALL(tnn_rocm_dequantize(q, (const int8_t *)src, s, TNN_ROCM_F32, staging_, count));
+                RETURN_ON_NEQ(MakeForHost(count * 4, &made), TNN_OK);
+                ROCM_CALL(tnn_rocm_dequantize(q, (const int8_t *)src, s, TNN_ROCM_F32, made, count));
             } else {
                 return Status(TNNERR_PARAM_ERR, "RocmBlobConverter: unsupported blob data type");
             }
-            RETURN_ON_NEQ(ToHost(mat.GetData(), staging_, count * 4, q), TNN_OK);
+            RETURN_ON_NEQ(ToHost(mat.GetData(), made, count * 4, q), TNN_OK);
         }
         if (NeedsScaleBias(param, desc.dims)) {
             std::vector<float> tmp(count);
@@ -710,7 +709,7 @@ private:
         return TNN_OK;
     }
     static bool CpuWidensHalf() {
-        static const bool yes = __builtin_cpu_supports("f16c") && __builtin_cpu_supports("avx");
+        static const bool yes = __builtin_cpu_supports("f16c") && __builtin_cpu_supports("avx2");
         return yes;
     }
     // IEEE half -> float (exact) with the CPU's conversion instruction, eight at a time; without it the blob is widened on
@@ -722,23 +721,90 @@ private:
         for (; i < n; ++i)
             d[i] = _cvtsh_ss(s[i]);
     }
-    Status HalfToHostFloat(float *host_dst, const void *dev_src, size_t count, void *q) {
+    // bfloat16 -> float (exact): the bits are the upper half of the float's
+    __attribute__((target("avx2"))) static void WidenBf16(const uint16_t *s, float *d, size_t n) {
+        size_t i = 0;
+        for (; i + 8 <= n; i += 8)
+            _mm256_storeu_ps(d + i, _mm256_castsi256_ps(_mm256_slli_epi32(
+                                        _mm256_cvtepu16_epi32(_mm_loadu_si128((const __m128i *)(s + i))), 16)));
+        for (; i < n; ++i) {
+            const uint32_t u = (uint32_t)s[i] << 16;
+            memcpy(d + i, &u, 4);
+        }
+    }
+    Status HalfToHostFloat(float *host_dst, const void *dev_src, size_t count, bool ieee, void *q) {
         RETURN_ON_NEQ(Bounce(count * 2), TNN_OK);
         ROCM_CALL(tnn_rocm_memcpy_d2h(bounce_, dev_src, count * 2, q));
         const int parts = 4;
 #pragma omp parallel for num_threads(parts) schedule(static)
         for (int i = 0; i < parts; ++i) {
             size_t lo = (count / parts * i) & ~(size_t)31, hi = i + 1 == parts ? count : (count / parts * (i + 1)) & ~(size_t)31;
-            WidenF16C((const uint16_t *)bounce_ + lo, host_dst + lo, hi - lo);
+            (ieee ? WidenF16C : WidenBf16)((const uint16_t *)bounce_ + lo, host_dst + lo, hi - lo);
         }
         return TNN_OK;
     }
-    // Device to host.  A Mat's memory is pageable, and a copy into pageable memory is staged by the runtime in small
-    // pieces on one thread (about 8 GB/s: 1.1 ms for the 9.4 MB fp32 output of a batch-8 encoder).  Large outputs
-    // therefore go by DMA into a page-locked buffer the converter keeps, and from there into the Mat on a few threads.
+    // ---- the small transfers of a request ----
+    // Up to kMappedMaxBytes the device reads and writes page-locked host memory in place, by kernels on the stream: an
+    // input is copied into the converter's buffer and fetched by a kernel, with no wait for the stream (15 us per input
+    // when it was a copy of pageable memory, 3 us so); an output is converted straight into the page-locked buffer.
+    // A place of an input's buffer is written again only when the stream has passed the kernel that read it.
+    Status ShowDevice(const void *host_src, size_t bytes, void *q, const void **seen) {
+        if (bytes > kMappedMaxBytes) {
+            RETURN_ON_NEQ(Staging(bytes), TNN_OK);
+            ROCM_CALL(tnn_rocm_memcpy_h2d(staging_, host_src, bytes, q));
+            *seen = staging_;
+            return TNN_OK;
+        }
+        // slots of equal size, so that several requests pass before one is written again
+        const size_t slot = (bytes + 255) & ~(size_t)255;
+        if (slot > stage_slot_ || stage_next_ == stage_slots_) {
+            if (stage_)
+                ROCM_CALL(tnn_rocm_stream_sync(q));
+            stage_next_ = 0;
+        }
+        if (slot > stage_slot_) {
+            tnn_rocm_free_host(stage_);
+            stage_              = nullptr;
+            stage_slot_         = 0;
+            const size_t slots  = std::max<size_t>(2, std::min<size_t>(16, kMappedMaxBytes / slot));
+            int rc              = tnn_rocm_malloc_host(&stage_, slots * slot);
+            if (rc != 0)
+                return RocmStatus(rc, TNNERR_OUTOFMEMORY, "converter page-locked buffer");
+            stage_slot_  = slot;
+            stage_slots_ = slots;
+        }
+        void *mine = (char *)stage_ + stage_next_++ * stage_slot_;
+        memcpy(mine, host_src, bytes);
+        *seen = mine;
+        return TNN_OK;
+    }
+    Status FromHost(void *dev_dst, const void *host_src, size_t bytes, void *q) {
+        if (bytes > kMappedMaxBytes) {
+            ROCM_CALL(tnn_rocm_memcpy_h2d(dev_dst, host_src, bytes, q));
+            return TNN_OK;
+        }
+        const void *seen = nullptr;
+        RETURN_ON_NEQ(ShowDevice(host_src, bytes, q, &seen), TNN_OK);
+        ROCM_CALL(tnn_rocm_copy_mapped(dev_dst, seen, bytes, q));
+        return TNN_OK;
+    }
+    // where a conversion for ToHost should leave its result
+    Status MakeForHost(size_t bytes, void **made) {
+        RETURN_ON_NEQ(bytes > kMappedMaxBytes ? Staging(bytes) : Bounce(bytes), TNN_OK);
+        *made = bytes > kMappedMaxBytes ? staging_ : bounce_;
+        return TNN_OK;
+    }
+    // Device (or the page-locked buffer, from MakeForHost) to host.  A Mat's memory is pageable, and a copy into pageable
+    // memory is staged by the runtime in small pieces on one thread (about 8 GB/s: 1.1 ms for the 9.4 MB fp32 output of a
+    // batch-8 encoder).  Outputs therefore go into a page-locked buffer the converter keeps, small ones by a kernel, large
+    // ones by DMA, and from there into the Mat, large ones on a few threads.
     Status ToHost(void *host_dst, const void *dev_src, size_t bytes, void *q) {
-        if (bytes < kBounceMinBytes) {
-            ROCM_CALL(tnn_rocm_memcpy_d2h(host_dst, dev_src, bytes, q));
+        if (bytes <= kMappedMaxBytes) {
+            RETURN_ON_NEQ(Bounce(bytes), TNN_OK);
+            if (dev_src != bounce_)
+                ROCM_CALL(tnn_rocm_copy_mapped(bounce_, dev_src, bytes, q));
+            ROCM_CALL(tnn_rocm_stream_sync(q));
+            memcpy(host_dst, bounce_, bytes);
             return TNN_OK;
         }
         RETURN_ON_NEQ(Bounce(bytes), TNN_OK);
@@ -751,7 +817,11 @@ private:
         }
         return TNN_OK;
     }
-    static constexpr size_t kBounceMinBytes = 1u << 20;
+    static constexpr size_t kMappedMaxBytes = 512u << 10;
+    void *stage_        = nullptr;  // page-locked input slots
+    size_t stage_slot_  = 0;        // bytes per slot
+    size_t stage_slots_ = 0;
+    size_t stage_next_  = 0;
     void *staging_     = nullptr;
     size_t staging_sz_ = 0;
     void *bounce_      = nullptr;

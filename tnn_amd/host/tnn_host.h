@@ -832,9 +832,13 @@ public:
     Status SetInputMat(std::shared_ptr<Mat> mat, MatConvertParam param, std::string input_name = "");
     Status GetOutputMat(std::shared_ptr<Mat> &mat, MatConvertParam param = MatConvertParam(),
                         std::string output_name = "", DeviceType device = DEVICE_NAIVE, MatType mat_type = NCHW_FLOAT);
+    // GetOutputMat into a Mat of the caller's (same element count), without the instance's own Mat in between
+    Status ConvertOutput(Mat &mat, MatConvertParam param = MatConvertParam(), std::string output_name = "");
+    Status GetOutputDims(DimsVector &dims, const std::string &output_name = "");
     DefaultNetwork *GetNetwork() { return network_.get(); }
 
 private:
+    Status FindOutput(std::string *output_name, Blob **blob);
     NetworkConfig net_config_;
     ModelConfig model_config_;
     std::shared_ptr<ModelInterpreter> interpreter_;

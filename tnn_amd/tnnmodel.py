@@ -218,14 +218,14 @@ class Graph:
 
     def model(self):
         magic = MAGIC_V2 if _version == 2 else MAGIC_V1
-        out = _u32(magic) + _i32(len(self.resources))
+        parts = [_u32(magic), _i32(len(self.resources))]
         for name, type_str, payload in self.resources:
-            out += _i32(_LAYER_TYPE_NUM.get(type_str, 0)) + _str(type_str) + _str(name) + payload
+            parts += [_i32(_LAYER_TYPE_NUM.get(type_str, 0)), _str(type_str), _str(name), payload]
         if self.constants:
-            out += _u32(magic) + _i32(len(self.constants))
+            parts += [_u32(magic), _i32(len(self.constants))]
             for key in sorted(self.constants):
-                out += _str(key) + raw_buffer(self.constants[key])
-        return out
+                parts += [_str(key), raw_buffer(self.constants[key])]
+        return b"".join(parts)  # one copy: appending record by record copies the whole file for each
 
 
 # ---------------------------------------------------------------------------------------------------
