@@ -129,7 +129,8 @@ TNN_ROCM_API int tnn_rocm_gemm_i8(void *stream, const int8_t *A, const int8_t *W
  * of cpu_mat_mul_layer_acc.cc:64-117, compute_elewise.cc:37-65, cpu_softmax_layer_acc.cc:30-97,
  * without materialising the [B*h,S,S] scores.  fp32 accumulation, online softmax.
  * Element (b, head, s, e) of Q is at q[b*q_sb + head*q_sh + s*q_ss + e] (e contiguous); same for
- * K, V (kv strides) and out.  head_dim must be 64.  dtype F16 or BF16.
+ * K, V (kv strides) and out.  head_dim must be 64.  dtype F16, BF16 or F32 (fp32 throughout; the softmax as the layers form
+ * it: scores * scale + mask, exp of the difference to the row's maximum).
  *   mask   : optional additive fp32 [B, S] (broadcast over heads and query rows), e.g. 0 / -10000
  *   kv_len : optional int32 [B]; keys j >= kv_len[b] are excluded exactly (−inf) and their tiles
  *            skipped.  kv_len[b] = 0 (the mask routines below never produce it: a row that masks every key keeps all

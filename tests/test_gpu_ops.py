@@ -585,11 +585,40 @@ def test_gemm_small_product_shapes(code, M, N, K):
         q, acc, _ = o.gemm_i8(dev(a8), dev(w8), dev(b8), dev(scale), want_acc=True)
         assert np.array_equal(host(acc), ref_acc)
         assert np.array_equal(host(q), ref_q)
-        if code in (9111141, 9121141, 4221141):
+        if code in (9111141, 9121141):
             got = host(o.gemm(a.cuda(), w.cuda(), True, bias=dev(bias), residual=res.cuda()))
             assert rel_err(got, orc.inner_product(a.numpy(), w.numpy(), bias) + res.numpy()) <= 1e-5
     finally:
         lib.tnn_rocm_debug_set_gemm_config(0)
+
+
+@pytest.mark.parametrize("code", [9111141, 9121141, 9111181, 9221141, 9321140, 3231142, 2331142, 3222121, 2222221])
+@pytest.mark.parametrize("M,N,K", [(1, 8, 128), (97, 104, 192), (130, 136, 3072)])
+def test_gemm_fp32_split_shapes(code, M, N, K):
+    """fp32 products on three bf16 planes, every tile shape: no further from float64 than an fp32 sum is, over magnitudes
+    from 1e-30 to 1e30; an infinity, a NaN and values next to the largest one come out as in plain fp32 arithmetic."""
+    from tnn_amd import capi
+    lib = capi.load()
+    if K * 4 % (64 << (code % 10)):
+        K += 64
+    rng = np.random.default_rng(code + M)
+    a = rng.standard_normal((M, K)).astype(np.float32) * np.float32(10.0) ** rng.integers(-30, 31, (M, 1)).astype(np.float32)
+    w = rng.standard_normal((N, K)).astype(np.float32)
+    a[0, 3], w[2, 5], w[3, 7] = np.inf, np.nan, 3.4e38
+    a[M - 1, 7] = 1e-3 if M > 1 else a[0, 7]
+    lib.tnn_rocm_debug_set_gemm_config(code)
+    try:
+        got = host(ops().gemm(dev(a), dev(w), True))
+    finally:
+        lib.tnn_rocm_debug_set_gemm_config(0)
+    with np.errstate(all="ignore"):
+        exact = a.astype(np.float64) @ w.astype(np.float64).T
+        size = np.abs(a.astype(np.float64)) @ np.abs(w.astype(np.float64)).T
+    fine = np.isfinite(exact) & (size < 1e38)
+    assert np.array_equal(np.isnan(got[0]), np.isnan(exact[0])) and np.array_equal(np.isinf(got[0]), np.isinf(exact[0]))
+    assert np.isnan(got[:, 2]).all() and fine[1:].sum() >= (M - 1) * (N - 2)
+    # K roundings of half a unit of the sum's magnitude at most, far fewer in fact
+    assert (np.abs(got[fine] - exact[fine]) <= 2.0 ** -24 * 4 * np.sqrt(K) * size[fine]).all()
 
 
 # ---- int8 GEMM: bit-exact accumulators and outputs -----------------------------------------------
@@ -807,6 +836,26 @@ def test_attention_bf16():
     say("attention bf16")
     got, ref = _attn_case(2, 4, 192, [192, 77], seed=5, dtype=torch.bfloat16)
     assert rel_err(got, ref) <= 3e-2
+
+
+@pytest.mark.parametrize("B,h,S", [(1, 1, 1), (2, 3, 31), (1, 2, 32), (2, 2, 33), (3, 4, 128), (1, 2, 161), (2, 1, 500)])
+@pytest.mark.parametrize("masked", ["none", "lengths", "additive"])
+def test_attention_fp32(B, h, S, masked):
+    """The fp32 kernel around its blocks of 32 queries and keys and its four key waves: against the checker at fp32 accuracy"""
+    say("attention fp32 B=%d h=%d S=%d %s" % (B, h, S, masked))
+    rng = np.random.default_rng(S * 7 + B)
+    q, k, v = (rng.standard_normal((B, h, S, 64)).astype(np.float32) for _ in range(3))
+    q *= 3
+    mask, kv = None, None
+    if masked == "lengths":
+        lens = rng.integers(1, S + 1, B).astype(np.int32)
+        kv, mask = dev(lens), np.where(np.arange(S)[None, :] < lens[:, None], 0.0, -10000.0).astype(np.float32)
+    elif masked == "additive":
+        mask = rng.standard_normal((B, S)).astype(np.float32) * 4
+        mask[:, S // 2:] -= 10000.0 * (rng.random((B, S - S // 2)) < 0.5)
+    got = host(ops().attention(dev(q), dev(k), dev(v), 0.125, mask=dev(mask) if masked == "additive" else None, kv_len=kv))
+    ref = orc.attention_core(q, k, v, 0.125, mask)
+    assert got.dtype == np.float32 and rel_err(got, ref) <= 3e-6
 
 
 def test_attention_packed_qkv_layout():

@@ -10,7 +10,7 @@ CSRC = os.path.join(HERE, "csrc")
 LIB_DIR = os.path.join(HERE, "lib")
 LIB_PATH = os.path.join(LIB_DIR, "libtnn_rocm.so")
 
-HIP_SOURCES = ["runtime.hip", "elementwise.hip", "rowwise.hip", "attention.hip", "gemm.hip",
+HIP_SOURCES = ["runtime.hip", "elementwise.hip", "rowwise.hip", "attention.hip", "attention_f32.hip", "gemm.hip",
                "gemm_f32.hip", "gemm_f16.hip", "gemm_f16_ln.hip", "gemm_bf16.hip", "gemm_bf16_ln.hip", "gemm_i8.hip"]
 
 HIPCC_FLAGS = [

@@ -23,6 +23,12 @@
 
 using namespace tnn_rocm;
 
+namespace tnn_rocm {
+int launch_attention_f32(hipStream_t s, const float *q, const float *k, const float *v, float *out, int B, int heads, int S,
+                         long q_sb, long q_sh, long q_ss, long kv_sb, long kv_sh, long kv_ss, long o_sb, long o_sh, long o_ss,
+                         float scale, const float *mask, const int32_t *kv_len);
+}
+
 namespace {
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
@@ -1114,8 +1120,8 @@ int tnn_rocm_attention(void *stream, int dtype, const void *q, const void *k, co
         return 0;
     TR_REQUIRE(q && k && v && out, TNN_ROCM_EINVAL, "attention: null pointer");
     TR_REQUIRE(head_dim == kD, TNN_ROCM_ESHAPE, "attention: head_dim %d unsupported (64 only)", head_dim);
-    TR_REQUIRE(dtype == TNN_ROCM_F16 || dtype == TNN_ROCM_BF16, TNN_ROCM_EDTYPE,
-               "attention: dtype %d unsupported (F16 or BF16)", dtype);
+    TR_REQUIRE(dtype == TNN_ROCM_F16 || dtype == TNN_ROCM_BF16 || dtype == TNN_ROCM_F32, TNN_ROCM_EDTYPE,
+               "attention: dtype %d unsupported (F16, BF16 or F32)", dtype);
     TR_REQUIRE(B <= 65535 && heads <= 65535, TNN_ROCM_ESHAPE, "attention: batch/heads exceed the grid limit");
     auto ok = [](const void *ptr, long a, long b2, long c) {
         return ((((uintptr_t)ptr) & 15u) == 0) && a % 8 == 0 && b2 % 8 == 0 && c % 8 == 0;
@@ -1125,6 +1131,9 @@ int tnn_rocm_attention(void *stream, int dtype, const void *q, const void *k, co
                TNN_ROCM_EALIGN, "attention: pointers must be 16-byte aligned and strides multiples of 8 elements");
     TR_REQUIRE(q_ss >= kD && kv_ss >= kD && o_ss >= kD, TNN_ROCM_ESHAPE, "attention: row stride below head_dim");
     TR_REQUIRE((long)S * kv_ss < (1l << 31), TNN_ROCM_ESHAPE, "attention: S * row stride exceeds 32-bit tile offsets");
+    if (dtype == TNN_ROCM_F32)
+        return launch_attention_f32((hipStream_t)stream, (const float *)q, (const float *)k, (const float *)v, (float *)out, B,
+                                    heads, S, q_sb, q_sh, q_ss, kv_sb, kv_sh, kv_ss, o_sb, o_sh, o_ss, scale, mask, kv_len);
     AttnParams p;
     p.q = (const uint16_t *)q;
     p.k = (const uint16_t *)k;

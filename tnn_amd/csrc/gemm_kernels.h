@@ -10,7 +10,8 @@
 //   fp16 : v_mfma_f32_32x32x16_f16   (8 halfs per lane per operand)
 //   bf16 : v_mfma_f32_32x32x16_bf16
 //   int8 : v_mfma_i32_32x32x32_i8    (16 bytes per lane per operand), exact int32 accumulation
-//   fp32 : 4 x v_mfma_f32_32x32x2f32 per 16-byte operand read
+//   fp32 : 4 x v_mfma_f32_32x32x2f32 per 16-byte operand read (general kernel and slabs staged through registers); the
+//          direct-to-LDS kernels split every value into three bf16 planes, see split_f32.h
 //
 // The contraction index inside one MFMA is symmetric between the two operands, so any fixed
 // assignment of k-values to (lane half, vector element) gives the same sum; both panels use the
@@ -24,6 +25,7 @@
 #include <type_traits>
 
 #include "gemm_typed.h"
+#include "split_f32.h"
 
 // Hook for scratch builds that include this file to time the tiled kernel from inside: TR_TL(i) marks point i of a
 // workgroup's life (0 entry, 5 first slabs requested, 6 row sums added up, 1 first slab landed, 2 main loop done,
@@ -45,8 +47,10 @@ typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 constexpr int kSlabBytes  = 64;               // bytes of k per row per LDS slab
 constexpr int kLdsStride  = kSlabBytes + 16;  // padded row stride in bytes (bank spread for b128 reads)
 
+// FRAGS: 16-byte LDS reads per operand and step of the tiled kernel
 template <int DT> struct GemmTraits;
 template <> struct GemmTraits<TNN_ROCM_F16> {
+    static constexpr int FRAGS = 1;
     typedef half_t elem;
     typedef f32x16 acc;
     static __device__ __forceinline__ void mma(const uint4 &a, const uint4 &b, acc &c) {
@@ -55,6 +59,7 @@ template <> struct GemmTraits<TNN_ROCM_F16> {
     }
 };
 template <> struct GemmTraits<TNN_ROCM_BF16> {
+    static constexpr int FRAGS = 1;
     typedef bf16_bits elem;
     typedef f32x16 acc;
     static __device__ __forceinline__ void mma(const uint4 &a, const uint4 &b, acc &c) {
@@ -63,6 +68,7 @@ template <> struct GemmTraits<TNN_ROCM_BF16> {
     }
 };
 template <> struct GemmTraits<TNN_ROCM_I8> {
+    static constexpr int FRAGS = 1;
     typedef int8_t elem;
     typedef i32x16 acc;
     static __device__ __forceinline__ void mma(const uint4 &a, const uint4 &b, acc &c) {
@@ -73,6 +79,14 @@ template <> struct GemmTraits<TNN_ROCM_I8> {
 template <> struct GemmTraits<TNN_ROCM_F32> {
     typedef float elem;
     typedef f32x16 acc;
+    // the tiled kernel: two reads make one 16-wide step of three bf16 planes (split_f32.h)
+    static constexpr int FRAGS = 2;
+    static __device__ __forceinline__ Split3 prepare(const uint4 (&f)[2], const SplitConst &c) {
+        const float x[8] = {__uint_as_float(f[0].x), __uint_as_float(f[0].y), __uint_as_float(f[0].z), __uint_as_float(f[0].w),
+                            __uint_as_float(f[1].x), __uint_as_float(f[1].y), __uint_as_float(f[1].z), __uint_as_float(f[1].w)};
+        return split3(x, c);
+    }
+    // the general kernel: fp32 matrix instructions
     static __device__ __forceinline__ void mma(const uint4 &a, const uint4 &b, acc &c) {
         c = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(a.x), __uint_as_float(b.x), c, 0, 0, 0);
         c = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(a.y), __uint_as_float(b.y), c, 0, 0, 0);
@@ -80,7 +94,82 @@ template <> struct GemmTraits<TNN_ROCM_F32> {
         c = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(a.w), __uint_as_float(b.w), c, 0, 0, 0);
     }
 };
+// fp32, pipelined: the planes of the operands of the STEPS steps that a wave takes from one slab.  turn() multiplies one
+// slab's planes while it makes the next one's from their LDS reads: a matrix instruction leaves the vector ALU free for 7 of
+// its 8 issue slots, and the conversion (28 vector instructions per operand and step) goes into them a piece at a time.
+// The order is pinned: left to itself the compiler issues the two kinds one after the other, with the wait states that a
+// dot product's result needs standing empty (64x64 tile, K=3072: 43 us; pinned: 41 us).
+template <int TM, int TN, int STEPS> struct SplitSlab {
+    static constexpr int OPS    = TM + TN;
+    static constexpr int MFMAS  = STEPS * kSplitProducts * TM * TN;
+    static constexpr int PIECES = STEPS * OPS * 6;  // per operand and step two groups of four values, three pieces each
+    Split3 op[STEPS][OPS];                          // A's operands, then B's
+    struct Reads {
+        uint4 f[STEPS][OPS][2];
+    };
 
+    __device__ __forceinline__ void convert(const Reads &rd, const SplitConst &sc) {
+#pragma unroll
+        for (int ks = 0; ks < STEPS; ++ks)
+#pragma unroll
+            for (int o = 0; o < OPS; ++o)
+                op[ks][o] = GemmTraits<TNN_ROCM_F32>::prepare(rd.f[ks][o], sc);
+    }
+    __device__ __forceinline__ void mfma(int q, f32x16 (&acc)[TM][TN]) const {
+        const int ks = q / (kSplitProducts * TM * TN), r = q % (kSplitProducts * TM * TN);
+        const int product = r / (TM * TN), i = r % (TM * TN) / TN, j = r % TN;
+        split_mma(op[ks][TM + j], op[ks][i], product, acc[i][j]);
+    }
+    __device__ __forceinline__ void multiply(f32x16 (&acc)[TM][TN]) const {
+#pragma unroll
+        for (int q = 0; q < MFMAS; ++q)
+            mfma(q, acc);
+    }
+    // piece k of a conversion: for group k % 2 of operand k / 6, one plane and what is left of the values
+    static __device__ __forceinline__ void piece(int k, SplitSlab &next, float (&rest)[STEPS][OPS][8], const SplitConst &sc) {
+        const int ks = k / (OPS * 6), o = k / 6 % OPS, plane = k % 6 / 2, g = k % 2;
+        float *x = rest[ks][o] + g * 4;
+        uint32_t *p = next.op[ks][o].p[plane] + g * 2;
+        p[0] = split_pack(x[0], x[1]);
+        p[1] = split_pack(x[2], x[3]);
+        if (plane < 2) {
+            x[0] = split_rest(p[0], sc.lo, x[0]);
+            x[1] = split_rest(p[0], sc.hi, x[1]);
+            x[2] = split_rest(p[1], sc.lo, x[2]);
+            x[3] = split_rest(p[1], sc.hi, x[3]);
+        }
+    }
+    __device__ __forceinline__ void turn(const Reads &rd, SplitSlab &next, f32x16 (&acc)[TM][TN], const SplitConst &sc) const {
+        // the first matrix instructions alone: the LDS reads arrive meanwhile
+        constexpr int LEAD = MFMAS >= 24 ? 4 : 2, SLOTS = MFMAS - LEAD;
+        float rest[STEPS][OPS][8];
+#pragma unroll
+        for (int q = 0; q < MFMAS; ++q) {
+            mfma(q, acc);
+            __builtin_amdgcn_sched_barrier(0);
+            if (q == LEAD - 1) {
+#pragma unroll
+                for (int ks = 0; ks < STEPS; ++ks)
+#pragma unroll
+                    for (int o = 0; o < OPS; ++o)
+#pragma unroll
+                        for (int h = 0; h < 2; ++h) {
+                            rest[ks][o][h * 4 + 0] = __uint_as_float(rd.f[ks][o][h].x);
+                            rest[ks][o][h * 4 + 1] = __uint_as_float(rd.f[ks][o][h].y);
+                            rest[ks][o][h * 4 + 2] = __uint_as_float(rd.f[ks][o][h].z);
+                            rest[ks][o][h * 4 + 3] = __uint_as_float(rd.f[ks][o][h].w);
+                        }
+            }
+            if (q >= LEAD) {
+                const int upto = PIECES * (q - LEAD + 1) / SLOTS;
+#pragma unroll
+                for (int k = PIECES * (q - LEAD) / SLOTS; k < upto; ++k)
+                    piece(k, next, rest, sc);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+    }
+};
 
 // ---- epilogues ----------------------------------------------------------------------------------
 // Optional abilities of an epilogue type, false where the type does not name them:
@@ -152,7 +241,7 @@ template <int DT> struct FloatEpilogue {
         if (flags & TNN_ROCM_EPI_GELU) {
 #pragma unroll
             for (int t = 0; t < 8; ++t)
-                v[t] = (DT == TNN_ROCM_F32) ? gelu_erf(v[t]) : gelu_erf_fast(v[t]);
+                v[t] = (DT == TNN_ROCM_F32) ? gelu_erf_wide(v[t]) : gelu_erf_fast(v[t]);
         }
         constexpr int NV = 8 * sizeof(T) / 16;  // 16-byte vectors per eight elements
         u32x4 packed[NV];
@@ -919,7 +1008,6 @@ template <int TM_, int TN_, int WGM_, int WGN_, int WGK_, int SLAB_, int NSTAGE_
     static constexpr size_t sums_offset = (slab_bytes >= stage_bytes + sums_bytes) ? stage_bytes : lds_bytes;
     static constexpr int NW = WGM * WGN * WGK, NT = 64 * NW;  // waves and threads per workgroup
     static_assert(NW == 4 || NW == 8, "four or eight waves per workgroup");
-    static_assert(OWN_ || (SLAB / 32) % WGK == 0, "k-steps of a slab must split evenly over the k-waves");
     static_assert(OWN_ || ((BM * (SLAB / 16)) % NT == 0 && (BN * (SLAB / 16)) % NT == 0), "slab must divide over the workgroup");
     static_assert(!OWN_ || (WGM_ == 1 && WGN_ == 1 && NSTAGE_ >= 2 && NSTAGE_ <= 4), "rings of two to four slabs, k-waves only");
     static_assert(OWN_ || NSTAGE_ == 0 || (NSTAGE_ >= 2 && NSTAGE_ <= 5), "register-staged, or two to five direct-to-LDS stages");
@@ -949,6 +1037,13 @@ template <typename CFG, typename Epi> struct EpiLds {
 // s_waitcnt that waits only for the vector-memory counter to drop to n (gfx9 encoding: vmcnt in bits 3:0 and
 // 15:14, expcnt 6:4 and lgkmcnt 11:8 left at their maxima)
 #define TR_WAIT_VMCNT(n) __builtin_amdgcn_s_waitcnt((((n)&0xF) | ((((n) >> 4) & 3) << 14) | (0x7 << 4) | (0xF << 8)))
+
+__device__ __forceinline__ float plain_dot(const float *a, const float *b, int k) {
+    float sum = 0.f;
+    for (int i = 0; i < k; ++i)
+        sum = fmaf(a[i], b[i], sum);
+    return sum;
+}
 
 template <int DT, typename CFG, typename Epi>
 __global__ void __launch_bounds__(CFG::NT)
@@ -1006,6 +1101,8 @@ __global__ void __launch_bounds__(CFG::NT)
     const int frag_row = lane & 31;
     const int frag_off = (lane >> 5) * 16;
     const int nk       = K / KB;
+    constexpr int FRAGS = GemmTraits<DT>::FRAGS, KSTEP = 32 * FRAGS;  // bytes of k per row that one step multiplies
+    const SplitConst split_const;
 
     // LayerNorm-folding epilogues: this lane's share of sum / sum of squares of A row (wm * TM + i) * 32 + frag_row.  The
     // eight values of a fragment are added up in fp32, the fragments in double: every tile shape deals the fragments out to
@@ -1075,7 +1172,8 @@ __global__ void __launch_bounds__(CFG::NT)
             if (k_lo + p < k_hi)
                 issue(k_lo + p, p);
         int stage = 0;
-        for (int kt = k_lo; kt < k_hi; ++kt) {
+        // this wave's fragments of slab kt, and the request for the slab that takes its place
+        auto fetch = [&](int kt, uint4 (&f)[SLAB / KSTEP][TM + TN][FRAGS]) __attribute__((always_inline)) {
             // slab kt is complete once at most the loads of the slabs requested after it are outstanding
             const int behind = k_hi - 1 - kt;
             if (NS > 3 && behind >= 3)
@@ -1088,35 +1186,66 @@ __global__ void __launch_bounds__(CFG::NT)
                 TR_WAIT_VMCNT(0);
             asm volatile("" ::: "memory");
             const unsigned char *sa = ring + stage * STAGE, *sb = sa + BM * SLAB;
-            uint4 fa[SLAB / 32][TM], fb[SLAB / 32][TN];
 #pragma unroll
-            for (int kk = 0; kk < SLAB / 32; ++kk) {
-                const int chunk = ((kk * 2 + (lane >> 5)) ^ fswz) * 16;
+            for (int kf = 0; kf < SLAB / 32; ++kf) {
+                const int chunk = ((kf * 2 + (lane >> 5)) ^ fswz) * 16;
 #pragma unroll
                 for (int i = 0; i < TM; ++i)
-                    fa[kk][i] = *reinterpret_cast<const uint4 *>(sa + i * 32 * SLAB + frow + chunk);
+                    f[kf / FRAGS][i][kf % FRAGS] = *reinterpret_cast<const uint4 *>(sa + i * 32 * SLAB + frow + chunk);
 #pragma unroll
                 for (int j = 0; j < TN; ++j)
-                    fb[kk][j] = *reinterpret_cast<const uint4 *>(sb + j * 32 * SLAB + frow + chunk);
+                    f[kf / FRAGS][TM + j][kf % FRAGS] = *reinterpret_cast<const uint4 *>(sb + j * 32 * SLAB + frow + chunk);
             }
             // the fragments are in registers before the slab's place is given to the next load
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
             if (kt + NS < k_hi)
                 issue(kt + NS, stage);
+            stage = stage + 1 == NS ? 0 : stage + 1;
+        };
+        if constexpr (DT == TNN_ROCM_F32) {
+            if (k_lo < k_hi) {
+                typedef SplitSlab<TM, TN, SLAB / KSTEP> Planes;
+                Planes p, q;
+                auto half = [&](int kt, const Planes &now, Planes &next) __attribute__((always_inline)) {
+                    typename Planes::Reads rd;
+                    fetch(kt, rd.f);
+                    now.turn(rd, next, acc, split_const);
+                };
+                {
+                    typename Planes::Reads rd;
+                    fetch(k_lo, rd.f);
+                    p.convert(rd, split_const);
+                }
+                int kt = k_lo + 1;
+                for (; kt + 1 < k_hi; kt += 2) {
+                    half(kt, p, q);
+                    half(kt + 1, q, p);
+                }
+                if (kt < k_hi) {
+                    half(kt, p, q);
+                    q.multiply(acc);
+                } else {
+                    p.multiply(acc);
+                }
+            }
+        } else {
+            for (int kt = k_lo; kt < k_hi; ++kt) {
+                uint4 f[SLAB / KSTEP][TM + TN][FRAGS];
+                fetch(kt, f);
 #pragma unroll
-            for (int kk = 0; kk < SLAB / 32; ++kk) {
-                if constexpr (Epi::kRowStats) {
+                for (int kk = 0; kk < SLAB / KSTEP; ++kk) {
+                    if constexpr (Epi::kRowStats) {
+#pragma unroll
+                        for (int i = 0; i < TM; ++i)
+                            ln_take(f[kk][i][0], i);
+                    }
 #pragma unroll
                     for (int i = 0; i < TM; ++i)
-                        ln_take(fa[kk][i], i);
+#pragma unroll
+                        for (int j = 0; j < TN; ++j)
+                            GemmTraits<DT>::mma(f[kk][TM + j][0], f[kk][i][0], acc[i][j]);
                 }
-#pragma unroll
-                for (int i = 0; i < TM; ++i)
-#pragma unroll
-                    for (int j = 0; j < TN; ++j)
-                        GemmTraits<DT>::mma(fb[kk][j], fa[kk][i], acc[i][j]);
             }
-            stage = stage + 1 == NS ? 0 : stage + 1;
         }
     } else if constexpr (CFG::NSTAGE > 0) {
         // Direct-to-LDS pipeline.  One load instruction of a wave fills 1024 contiguous LDS bytes (lane L writes
@@ -1177,19 +1306,23 @@ __global__ void __launch_bounds__(CFG::NT)
         // One slab: this wave's fragments of it, then `between` (the requests for the slab that goes into the stage freed
         // last), then the MFMAs.  READ_AHEAD reads all of the slab's fragments before the requests, so that the LDS
         // latency runs while the requests are issued; it needs the registers for them.
-        constexpr int KSTEPS      = SLAB / 32 / WGK;
+        constexpr int KSTEPS      = SLAB / KSTEP / WGK;
+        static_assert((SLAB / KSTEP) % WGK == 0, "k-steps of a slab must split evenly over the k-waves");
         constexpr bool READ_AHEAD = NS >= 4 && (TM + TN) * KSTEPS <= 8;
         auto compute = [&](int stage, auto between) __attribute__((always_inline)) {
             const unsigned char *sa = lds_dyn + stage * STAGE, *sb = sa + BM * SLAB;
-            uint4 fa[READ_AHEAD ? KSTEPS : 1][TM], fb[READ_AHEAD ? KSTEPS : 1][TN];
+            uint4 fa[READ_AHEAD ? KSTEPS : 1][TM][FRAGS], fb[READ_AHEAD ? KSTEPS : 1][TN][FRAGS];
             auto read = [&](int ks, int slot) __attribute__((always_inline)) {
-                const int chunk = (((wk + ks * WGK) * 2 + (lane >> 5)) ^ fswz) * 16;
 #pragma unroll
-                for (int i = 0; i < TM; ++i)
-                    fa[slot][i] = *reinterpret_cast<const uint4 *>(sa + (wm * TM + i) * 32 * SLAB + frow + chunk);
+                for (int f = 0; f < FRAGS; ++f) {
+                    const int chunk = ((((wk + ks * WGK) * FRAGS + f) * 2 + (lane >> 5)) ^ fswz) * 16;
 #pragma unroll
-                for (int j = 0; j < TN; ++j)
-                    fb[slot][j] = *reinterpret_cast<const uint4 *>(sb + (wn * TN + j) * 32 * SLAB + frow + chunk);
+                    for (int i = 0; i < TM; ++i)
+                        fa[slot][i][f] = *reinterpret_cast<const uint4 *>(sa + (wm * TM + i) * 32 * SLAB + frow + chunk);
+#pragma unroll
+                    for (int j = 0; j < TN; ++j)
+                        fb[slot][j][f] = *reinterpret_cast<const uint4 *>(sb + (wn * TN + j) * 32 * SLAB + frow + chunk);
+                }
             };
             if constexpr (READ_AHEAD) {
 #pragma unroll
@@ -1207,13 +1340,13 @@ __global__ void __launch_bounds__(CFG::NT)
 #pragma unroll
                     for (int i = 0; i < TM; ++i)
                         if ((i + ks) % WGN == wn)
-                            ln_take(fa[slot][i], i);
+                            ln_take(fa[slot][i][0], i);
                 }
 #pragma unroll
                 for (int i = 0; i < TM; ++i)
 #pragma unroll
                     for (int j = 0; j < TN; ++j)
-                        GemmTraits<DT>::mma(fb[slot][j], fa[slot][i], acc[i][j]);
+                        GemmTraits<DT>::mma(fb[slot][j][0], fa[slot][i][0], acc[i][j]);
             }
         };
         constexpr int LPW = A_LD + B_LD;
@@ -1344,6 +1477,59 @@ __global__ void __launch_bounds__(CFG::NT)
             step(nk - 1, std::true_type());
             finish_sums(0);
             TR_TL(6);  // handed-over row sums added up
+        } else if constexpr (DT == TNN_ROCM_F32) {
+            typedef SplitSlab<TM, TN, KSTEPS> Planes;
+            Planes p, q;
+            auto fetch = [&](int kt, uint4 (&f)[KSTEPS][TM + TN][FRAGS]) __attribute__((always_inline)) {
+                // slab kt - 1 is in this wave's registers, see the barrier below
+                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+                const int behind = nk - 1 - kt;
+                if (NS > 2 && behind >= 1)
+                    TR_WAIT_VMCNT(NS > 2 ? LPW : 0);
+                else
+                    TR_WAIT_VMCNT(0);
+                __builtin_amdgcn_s_barrier();
+                asm volatile("" ::: "memory");
+                const unsigned char *sa = lds_dyn + stage * STAGE, *sb = sa + BM * SLAB;
+#pragma unroll
+                for (int ks = 0; ks < KSTEPS; ++ks)
+#pragma unroll
+                    for (int h = 0; h < FRAGS; ++h) {
+                        const int chunk = ((((wk + ks * WGK) * FRAGS + h) * 2 + (lane >> 5)) ^ fswz) * 16;
+#pragma unroll
+                        for (int i = 0; i < TM; ++i)
+                            f[ks][i][h] = *reinterpret_cast<const uint4 *>(sa + (wm * TM + i) * 32 * SLAB + frow + chunk);
+#pragma unroll
+                        for (int j = 0; j < TN; ++j)
+                            f[ks][TM + j][h] = *reinterpret_cast<const uint4 *>(sb + (wn * TN + j) * 32 * SLAB + frow + chunk);
+                    }
+                if (kt + NS - 1 < nk)
+                    issue(kt + NS - 1, fill);
+                stage = stage + 1 == NS ? 0 : stage + 1;
+                fill  = fill + 1 == NS ? 0 : fill + 1;
+            };
+            static_assert(NS <= 3, "waits written for up to three stages");
+            auto half = [&](int kt, const Planes &now, Planes &next) __attribute__((always_inline)) {
+                typename Planes::Reads rd;
+                fetch(kt, rd.f);
+                now.turn(rd, next, acc, split_const);
+            };
+            {
+                typename Planes::Reads rd;
+                fetch(0, rd.f);
+                p.convert(rd, split_const);
+            }
+            int kt = 1;
+            for (; kt + 1 < nk; kt += 2) {
+                half(kt, p, q);
+                half(kt + 1, q, p);
+            }
+            if (kt < nk) {
+                half(kt, p, q);
+                q.multiply(acc);
+            } else {
+                p.multiply(acc);
+            }
         } else {
             for (int kt = 0; kt < nk; ++kt)
                 step(kt, std::false_type());
@@ -1576,6 +1762,21 @@ __global__ void __launch_bounds__(CFG::NT)
             }
             const int m = m0 + ((pos / WGN) * TM + i) * 32 + row;
             const int n = n0 + (pos % WGN) * CW + c8;
+            if constexpr (DT == TNN_ROCM_F32 && CFG::NSTAGE > 0) {
+                // an infinity in an operand has no planes (inf - inf is no number): such a sum is formed again from the
+                // operands themselves
+#pragma unroll
+                for (int t = 0; t < 8; ++t) {
+                    const float v = t < 4 ? lo[t] : hi[t - 4];
+                    if (!(__builtin_fabsf(v) < INFINITY) && m < M && n + t < N) {
+                        const float f = plain_dot(A + (size_t)m * lda, B + (size_t)(n + t) * ldb, K);
+                        if (t < 4)
+                            lo[t & 3] = f;
+                        else
+                            hi[t & 3] = f;
+                    }
+                }
+            }
             const int nl = (pos % WGN) * CW + c8;  // column inside the tile
             if constexpr (Epi::kRowStats) {
                 if (m < M && n + 7 < N) {  // N is a multiple of 8 for these epilogues (checked at launch)
@@ -1726,6 +1927,8 @@ int launch_tiled(hipStream_t s, const void *A, const void *B, int M, int N, int 
 //   3112221   64 x  64, 8 waves (two k-waves), 3 stages       3112222   64 x  64, 8 waves, 256-byte slabs
 //   4221141   64 x  64, 4 k-waves, 4 stages                   3212221  128 x  64, 8 waves
 //   2112211   64 x  64, 4 waves, 2 stages                     2222221  128 x 128, 8 waves (two k-waves)
+//   fp32 only: 9111181 32 x 32, 8 k-waves; 9221141, 9321140 64 x 64 and 96 x 64, 4 k-waves with rings of their own;
+//   3231142, 2331142 64 x 96 and 96 x 96, 4 k-waves; 3222121 128 x 64, 4 waves (two k-waves)
 //   3332221  192 x 192, 8 waves (two k-waves)                 3331182   96 x  96, 8 k-waves, 256-byte slabs
 //   112210    64 x  64 and 222210 128 x 128, 4 waves: rows that are no multiple of 128 bytes
 // Eight-wave workgroups put two waves on every SIMD inside one tile: while one waits for its LDS fragments the
@@ -1772,12 +1975,23 @@ constexpr TileCost kTilesI8[] = {
     {3332221, 192, 192, 1, 9.89f, 9.10f, {0.860f}},
     {3331182, 96, 96, 1, 6.72f, 5.80f, {0.314f}},
 };
-// fp32 MFMAs take 16 times the matrix-pipe time of half ones: the pipe is the bound and what counts is an even spread
+// fp32 on three bf16 planes: six matrix instructions per operand pair and the conversion between them, so a step costs five
+// times a half one.  Large wave tiles convert less per product, K is split over the waves of a CU wherever tiles are few.
+// Fit and sweep as above (M from 16 to 3072, hidden size 768; the pick is 0.2 % behind the best shape on average).
+// us, v_mfma_f32 kernels before -> now:  M=1536: N=768 K=768 27 -> 18, N=3072 K=768 74 -> 52, N=768 K=3072 83 -> 55
+//   M=128: N=768 K=768 7.6 -> 7.0, N=3072 K=768 15.2 -> 10.0, N=768 K=3072 17.6 -> 15.5   (3072 x 768 x 3072: 168 TFLOP/s)
+// Error against float64 (2-norm over 2-norm; 300 x 760 x 768 / 129 x 264 x 3072): 1.5e-7 .. 3e-7 / 3e-7 .. 6e-7 by shape,
+// v_mfma_f32_32x32x2_f32: 5.0e-7 / 9.9e-7.
 constexpr TileCost kTilesF32[] = {
-    {9111141, 32, 32, 2, 3.80f, 3.25f, {0.141f, 0.275f}},
-    {9121141, 32, 64, 1, 4.24f, 3.76f, {0.257f}},
-    {2112211, 64, 64, 4, 4.37f, 3.17f, {0.548f, 1.019f, 1.490f, 2.032f}},
-    {4221141, 64, 64, 2, 4.94f, 4.95f, {0.500f, 0.995f}},
+    {9111141, 32, 32, 2, 3.63f, 1.18f, {0.135f, 0.276f}},
+    {9121141, 32, 64, 1, 4.33f, 3.30f, {0.214f}},
+    {9111181, 32, 32, 1, 3.96f, 2.69f, {0.125f}},
+    {9221141, 64, 64, 1, 5.66f, 5.47f, {0.319f}},
+    {9321140, 96, 64, 1, 6.16f, 7.00f, {0.483f}},
+    {3231142, 64, 96, 1, 6.12f, 5.36f, {0.546f}},
+    {2331142, 96, 96, 1, 7.61f, 7.87f, {0.725f}},
+    {3222121, 128, 64, 2, 5.62f, 5.02f, {0.723f, 1.280f}},
+    {2222221, 128, 128, 1, 6.89f, 10.92f, {1.175f}},
 };
 
 template <int COUNT> inline int pick_tile_config(const TileCost (&shapes)[COUNT], long M, long N, size_t kbytes) {
@@ -1844,13 +2058,21 @@ int launch_gemm_fast(hipStream_t s, const void *A, const void *B, int M, int N, 
             default: break;
         }
     }
-    switch (cfg) {
-        case 2112211: TR_FAST_DL(1, 1, 2, 2, 1, 128, 2);
-        case 4221141: TR_FAST_DL(2, 2, 1, 1, 4, 128, 4);
-        default: break;
-    }
-    if constexpr (DT != TNN_ROCM_F32) {
+    if constexpr (DT == TNN_ROCM_F32) {
         switch (cfg) {
+            case 9111181: TR_FAST_OWN(1, 1, 8, 128, 2);
+            case 9221141: TR_FAST_OWN(2, 2, 4, 128, 2);
+            case 9321140: TR_FAST_OWN(3, 2, 4, 64, 3);
+            case 3231142: TR_FAST_DL(2, 3, 1, 1, 4, 256, 3);
+            case 2331142: TR_FAST_DL(3, 3, 1, 1, 4, 256, 2);
+            case 3222121: TR_FAST_DL(2, 2, 2, 1, 2, 128, 3);
+            case 2222221: TR_FAST_DL(2, 2, 2, 2, 2, 128, 2);
+            default: break;
+        }
+    } else {
+        switch (cfg) {
+            case 2112211: TR_FAST_DL(1, 1, 2, 2, 1, 128, 2);
+            case 4221141: TR_FAST_DL(2, 2, 1, 1, 4, 128, 4);
             case 3112221: TR_FAST_DL(1, 1, 2, 2, 2, 128, 3);
             case 3112222: TR_FAST_DL(1, 1, 2, 2, 2, 256, 3);
             case 3212221: TR_FAST_DL(2, 1, 2, 2, 2, 128, 3);
