@@ -675,6 +675,32 @@ def test_instance_reshape_matches_fresh_instances():
     inst.close()
 
 
+@pytest.mark.parametrize("B,S", [(1, 2), (2, 33), (3, 128), (1, 200)])
+def test_fp32_attention_group_equals_its_layers(B, S):
+    """A plain fp32 forward runs every attention core as one group; ForwardWithCallback runs the same instance's layers one
+    by one.  Same answer at fp32 accuracy, before and after Instance::Reshape, and against the checker."""
+    host, tnnmodel, EncoderConfig, make_weights, make_inputs = _mods()
+    say("host: fp32 attention group, B=%d S=%d" % (B, S))
+    cfg = EncoderConfig(2, 128, 2, 256)
+    w = make_weights(cfg, seed=31, bias_std=0.05)
+    inst = host.RocmInstance.from_graph(tnnmodel.encoder_graph(cfg, w, 2, 200, dynamic=True), "fp32")
+    for b, s in ((2, 200), (B, S)):
+        if (b, s) != (2, 200):
+            inst.reshape({"input_ids": [b, s], "token_type_ids": [b, s], "attention_bias": [b, 1, 1, s]})
+        ids, seg, lens, mask = make_inputs(cfg, b, s, max(1, s // 3), s, seed=50 + s)
+        for n, v in (("input_ids", ids), ("token_type_ids", seg), ("attention_bias", mask.reshape(b, 1, 1, s))):
+            inst.set_input(n, v)
+        inst.forward()
+        got = inst.output("last_hidden").reshape(b * s, -1).copy()
+        seen = []
+        inst.forward_with_callback(after=lambda name, typ, blobs: seen.append(typ))
+        assert seen.count("Softmax") == 2
+        alone = inst.output("last_hidden").reshape(b * s, -1)
+        ref = encoder_ref.encoder(w, cfg, encoder_ref.embed(w, ids, seg, cfg.eps), b, s, mask)
+        assert rel_err(got, alone) <= 3e-6 and rel_err(got, ref) <= FP32_ASSERT
+    inst.close()
+
+
 def test_instance_reshape_fp32_batch_only_with_static_head_split():
     """A graph whose head split names B and S cannot change them (the element count check of reshape_layer.cc:41-63
     fails, as in the engine); the error names the layer.  The un-fused fp32 path reshapes through the dynamic graph."""

@@ -16,8 +16,10 @@
 #include <cmath>
 #include <cstdlib>
 #include <functional>
+#include <set>
 
 #include "rocm_device.h"
+#include "rocm_network.h"
 
 namespace TNN_NS {
 
@@ -435,7 +437,7 @@ public:
         FoldGelu();
         FoldResidual();
         if (half_)
-            FuseAttention();  // the attention kernel computes in fp16; fp32 nets keep the decomposed core
+            FuseAttention();  // fp32 nets keep the core's layers, and run them as a group (RocmFindAttentionGroups)
         const char *fold = getenv("TNN_ROCM_FOLD_LN");
         if (half_ && !(fold && fold[0] == '0'))
             FoldLayerNorm();
@@ -447,6 +449,35 @@ public:
                 HandOverRowSums();
         }
         return TNN_OK;
+    }
+
+    // The attention cores of a graph that keeps them as layers, see RocmFindAttentionGroups
+    std::vector<RocmLayerGroup> FindAttention(NetStructure *s, NetResource *r) {
+        structure_ = s;
+        resource_  = r;
+        std::vector<RocmLayerGroup> found;
+        auto &L = structure_->layers;
+        GraphIndex g(L);
+        for (int si = 0; si < (int)L.size(); ++si) {
+            if (!L[si] || L[si]->type != LAYER_SOFTMAX)
+                continue;
+            AttentionCore m;
+            AttentionMatcher matcher(structure_, resource_,
+                                     [this](const GraphIndex &gi, const std::string &blob, const std::vector<int> &o4,
+                                            const std::vector<int> &o3, std::vector<int> *chain, DimsVector *shape) {
+                                         return HeadSplitSource(gi, blob, o4, o3, chain, shape);
+                                     });
+            RocmLayerGroup group;
+            if (!matcher.Match(g, si, &m) || !MakeAttention(m, L[si]->name, &group.layer, &group.resource))
+                continue;
+            group.first = *std::min_element(m.chain.begin(), m.chain.end());
+            group.last  = *std::max_element(m.chain.begin(), m.chain.end());
+            // The memory plan is that of the single layers: nothing else may run between the first and the last of them,
+            // or it could write where the group still reads or reads after the group has written.
+            if ((int)std::set<int>(m.chain.begin(), m.chain.end()).size() == group.last - group.first + 1)
+                found.push_back(group);
+        }
+        return found;
     }
 
 private:
@@ -732,6 +763,67 @@ private:
         return li;
     }
 
+    // the fused layer and its resource (three projections side by side) for a matched attention core; false where the fused
+    // kernels do not serve the core's sizes
+    bool MakeAttention(const AttentionCore &m, const std::string &name, std::shared_ptr<LayerInfo> *layer,
+                       std::shared_ptr<LayerResource> *resource) {
+        auto &L = structure_->layers;
+        const std::string &mask = m.mask;
+        const float scale = m.scale;
+        const int lq = m.lq, lk = m.lk, lv = m.lv, rs = m.rs;
+        const DimsVector &shape_q = m.split_shape;
+        // ---- the three projections are plain linears of equal width
+        auto rq = ResOf<RocmFusedLinearResource>(L[lq]->name), rk = ResOf<RocmFusedLinearResource>(L[lk]->name),
+             rv = ResOf<RocmFusedLinearResource>(L[lv]->name);
+        if (!rq || !rk || !rv)
+            return false;
+        auto dq = rq->weight_nk.GetBufferDims();
+        if (dq != rk->weight_nk.GetBufferDims() || dq != rv->weight_nk.GetBufferDims())
+            return false;
+        int H = dq[0], K = dq[1];
+        int heads    = shape_q[shape_q.size() - 2];
+        int head_dim = shape_q.back();
+        int seq      = shape_q[shape_q.size() - 3];
+        // seq 0 / -1: the split copies (or infers) the sequence length, i.e. the model is meant for
+        // Instance::Reshape; the acc then reads S from its input blob [B,S,H] at every reshape
+        if (heads * head_dim != H || K != H || head_dim != 64 || seq < -1)
+            return false;
+        // ---- build the fused layer
+        auto fl      = std::make_shared<LayerInfo>();
+        fl->type     = LAYER_ROCM_FUSED_ATTENTION;
+        fl->type_str = "RocmFusedAttention";
+        fl->name     = name + "_fused_attention";
+        fl->inputs   = {L[lq]->inputs[0]};
+        if (!mask.empty())
+            fl->inputs.push_back(mask);
+        fl->outputs  = {L[rs]->outputs[0]};
+        auto fp      = std::make_shared<RocmFusedAttentionParam>();
+        fp->type     = fl->type_str;
+        fp->name     = fl->name;
+        fp->heads    = heads;
+        fp->head_dim = head_dim;
+        fp->scale    = scale;
+        fp->has_mask = mask.empty() ? 0 : 1;
+        fp->split_rank  = (int)shape_q.size();
+        fp->merge_shape = ParamOf<ReshapeLayerParam>(L[rs])->shape;
+        fl->param    = fp;
+        fp->seq_len  = seq > 0 ? seq : 0;
+        auto fr       = std::make_shared<RocmFusedLinearResource>();
+        fr->name      = fl->name;
+        fr->weight_nk = RawBuffer(3 * H * K * 4, {3 * H, K});
+        fr->bias      = RawBuffer(3 * H * 4, {3 * H});
+        RocmFusedLinearResource *src[3] = {rq, rk, rv};
+        for (int t = 0; t < 3; ++t) {
+            memcpy(fr->weight_nk.force_to<float *>() + (size_t)t * H * K, src[t]->weight_nk.force_to<float *>(),
+                   (size_t)H * K * 4);
+            if (src[t]->bias.GetDataCount() == H)
+                memcpy(fr->bias.force_to<float *>() + (size_t)t * H, src[t]->bias.force_to<float *>(), (size_t)H * 4);
+        }
+        *layer    = fl;
+        *resource = fr;
+        return true;
+    }
+
     void FuseAttention() {
         auto &L = structure_->layers;
         bool changed = true;
@@ -750,61 +842,13 @@ private:
                                          });
                 if (!matcher.Match(g, si, &m))
                     continue;
-                const std::vector<int> &chain = m.chain;
-                const std::string &mask = m.mask;
-                const float scale = m.scale;
-                const int lq = m.lq, lk = m.lk, lv = m.lv, rs = m.rs;
-                const DimsVector &shape_q = m.split_shape;
-                // ---- the three projections are plain linears of equal width
-                auto rq = ResOf<RocmFusedLinearResource>(L[lq]->name), rk = ResOf<RocmFusedLinearResource>(L[lk]->name),
-                     rv = ResOf<RocmFusedLinearResource>(L[lv]->name);
-                if (!rq || !rk || !rv)
+                std::shared_ptr<LayerInfo> fl;
+                std::shared_ptr<LayerResource> fr;
+                if (!MakeAttention(m, sm->name, &fl, &fr))
                     continue;
-                auto dq = rq->weight_nk.GetBufferDims();
-                if (dq != rk->weight_nk.GetBufferDims() || dq != rv->weight_nk.GetBufferDims())
-                    continue;
-                int H = dq[0], K = dq[1];
-                int heads    = shape_q[shape_q.size() - 2];
-                int head_dim = shape_q.back();
-                int seq      = shape_q[shape_q.size() - 3];
-                // seq 0 / -1: the split copies (or infers) the sequence length, i.e. the model is meant for
-                // Instance::Reshape; the acc then reads S from its input blob [B,S,H] at every reshape
-                if (heads * head_dim != H || K != H || head_dim != 64 || seq < -1)
-                    continue;
-                int first = *std::min_element(chain.begin(), chain.end());
-                // ---- build the fused layer
-                auto fl      = std::make_shared<LayerInfo>();
-                fl->type     = LAYER_ROCM_FUSED_ATTENTION;
-                fl->type_str = "RocmFusedAttention";
-                fl->name     = sm->name + "_fused_attention";
-                fl->inputs   = {L[lq]->inputs[0]};
-                if (!mask.empty())
-                    fl->inputs.push_back(mask);
-                fl->outputs  = {L[rs]->outputs[0]};
-                auto fp      = std::make_shared<RocmFusedAttentionParam>();
-                fp->type     = fl->type_str;
-                fp->name     = fl->name;
-                fp->heads    = heads;
-                fp->head_dim = head_dim;
-                fp->scale    = scale;
-                fp->has_mask = mask.empty() ? 0 : 1;
-                fp->split_rank  = (int)shape_q.size();
-                fp->merge_shape = ParamOf<ReshapeLayerParam>(L[rs])->shape;
-                fl->param    = fp;
-                fp->seq_len  = seq > 0 ? seq : 0;
-                auto fr       = std::make_shared<RocmFusedLinearResource>();
-                fr->name      = fl->name;
-                fr->weight_nk = RawBuffer(3 * H * K * 4, {3 * H, K});
-                fr->bias      = RawBuffer(3 * H * 4, {3 * H});
-                RocmFusedLinearResource *src[3] = {rq, rk, rv};
-                for (int t = 0; t < 3; ++t) {
-                    memcpy(fr->weight_nk.force_to<float *>() + (size_t)t * H * K, src[t]->weight_nk.force_to<float *>(),
-                           (size_t)H * K * 4);
-                    if (src[t]->bias.GetDataCount() == H)
-                        memcpy(fr->bias.force_to<float *>() + (size_t)t * H, src[t]->bias.force_to<float *>(), (size_t)H * 4);
-                }
+                const int first = *std::min_element(m.chain.begin(), m.chain.end());
                 resource_->resource_map[fl->name] = fr;
-                for (int idx : chain)
+                for (int idx : m.chain)
                     L[idx] = nullptr;
                 L[first] = fl;
                 changed  = true;
@@ -1457,7 +1501,12 @@ optimizer::NetOptimizerRegister<RocmFusionPass> g_net_optimizer_rocm_fuse_encode
 optimizer::NetOptimizerRegister<RocmInsertInt8Reformat> g_net_optimizer_rocm_insert_int8_reformat(optimizer::P2);
 optimizer::NetOptimizerRegister<RocmInt8FusionPass> g_net_optimizer_rocm_fuse_int8(optimizer::PLAST);
 
+
 }  // namespace
+
+std::vector<RocmLayerGroup> RocmFindAttentionGroups(NetStructure *structure, NetResource *resource) {
+    return RocmFusionPass().FindAttention(structure, resource);
+}
 
 // ---- LayerNorm folded into a projection: weight preparation ---------------------------------------------------
 // value of f after rounding to the activation type (round to nearest even, as the device conversion does)
@@ -1644,8 +1693,9 @@ public:
         auto in = inputs[0]->GetBlobDesc().dims;
         H_      = p->heads * p->head_dim;
         DataType dt = outputs[0]->GetBlobDesc().data_type;
-        if (dt != DATA_TYPE_HALF && dt != DATA_TYPE_BFP16)
-            return Status(TNNERR_LAYER_ERR, "fused attention runs in fp16/bf16 only");
+        const bool full = dt == DATA_TYPE_FLOAT && !p->quant && !p->ln_fold && !p->out_quant;
+        if (dt != DATA_TYPE_HALF && dt != DATA_TYPE_BFP16 && !full)
+            return Status(TNNERR_LAYER_ERR, "fused attention runs in fp16/bf16, with float projections and output also in fp32");
         if (p->quant) {
             auto wd = res8->weight.GetBufferDims();
             if (in.empty() || wd.size() != 2 || wd[0] != 3 * H_ || in.back() != wd[1] ||
@@ -1758,7 +1808,7 @@ public:
                                                (long)seq_ * H_, d, (long)H_, p->scale, mask, kv, vt_order));
             return TNN_OK;
         }
-        if (seq_ % 8 == 0 && H_ % 64 == 0) {
+        if (dt != DATA_TYPE_FLOAT && seq_ % 8 == 0 && H_ % 64 == 0) {
             // projection writes Q|K row-major and V already transposed per head: the attention kernel then stages
             // V tiles with 16-byte copies
             char *vt = (char *)qkv + (size_t)T_ * 2 * H_ * es;
@@ -1777,8 +1827,7 @@ public:
                                                (long)seq_ * H_, d, (long)H_, p->scale, mask, kv, vt_order));
             return TNN_OK;
         }
-        // sequence lengths that are not a multiple of 8 (only reachable by Instance::Reshape when a fold was decided
-        // at another length): packed Q|K|V rows and the kernel that reads V row-major
+        // fp32, and sequence lengths that are not a multiple of 8: packed Q|K|V rows and the kernel that reads V row-major
         if (p->out_quant)
             return Status(TNNERR_PARAM_ERR, "fused attention: the quantised output needs a sequence length that is a multiple of 8");
         if (p->ln_fold)

@@ -58,6 +58,84 @@ void RocmNetwork::Signature(std::vector<uint64_t> *sig) {
     }
 }
 
+#ifndef TNN_ROCM_ENGINE_TREE
+Status RocmNetwork::Init(NetworkConfig &net_config, ModelInterpreter *interpreter, const InputShapesMap &max_inputs_shape) {
+    RETURN_ON_NEQ(DefaultNetwork::Init(net_config, interpreter, max_inputs_shape), TNN_OK);
+    if (config_.precision != PRECISION_HIGH)
+        return TNN_OK;
+    for (auto &found : RocmFindAttentionGroups(&structure_, &resource_)) {
+        Group g;
+        g.first = found.first, g.last = found.last;
+        g.layer = found.layer, g.resource = found.resource;
+        for (auto &name : g.layer->inputs)
+            g.inputs.push_back(GetBlob(name));
+        for (auto &name : g.layer->outputs)
+            g.outputs.push_back(GetBlob(name));
+        bool known = true;
+        for (auto blobs : {&g.inputs, &g.outputs})
+            for (Blob *b : *blobs)
+                known &= b != nullptr && b->GetBlobDesc().data_type == DATA_TYPE_FLOAT;
+        if (!known)
+            continue;
+        g.acc.reset(device_->CreateLayerAcc(g.layer->type));
+        if (!g.acc)
+            continue;
+        g.acc->SetConstantResource(&resource_.constant_map);
+        RETURN_ON_NEQ(g.acc->Init(context_, g.layer->param.get(), g.resource.get(), g.inputs, g.outputs), TNN_OK);
+        groups_.push_back(std::move(g));
+    }
+    return ReshapeGroups();
+}
+
+Status RocmNetwork::Reshape(const InputShapesMap &inputs) {
+    RETURN_ON_NEQ(DefaultNetwork::Reshape(inputs), TNN_OK);
+    return ReshapeGroups();
+}
+
+Status RocmNetwork::ReshapeGroups() {
+    auto range = [](Blob *b) {
+        const char *at = (const char *)b->GetHandle().base + b->GetHandle().bytes_offset;
+        return std::make_pair(at, at + (size_t)DimsVectorUtils::Count(b->GetBlobDesc().dims) * sizeof(float));
+    };
+    for (auto &g : groups_) {
+        // the projections read all of the input before the attention kernel writes, but the mask is read while it does
+        g.active       = true;
+        const auto out = range(g.outputs[0]);
+        for (size_t i = 1; i < g.inputs.size(); ++i) {
+            const auto in = range(g.inputs[i]);
+            g.active &= g.inputs[i]->IsConstant() || in.second <= out.first || out.second <= in.first;
+        }
+        if (!g.active)
+            continue;
+        RETURN_ON_NEQ(g.acc->ReloadConstantBlobs(g.inputs, true), TNN_OK);
+        // shapes that the kernels do not take are the layers' business
+        g.active = g.acc->Reshape(g.inputs, g.outputs) == TNN_OK;
+    }
+    return TNN_OK;
+}
+
+Status RocmNetwork::RunLayers(void *prof_stream) {
+    if (groups_.empty() || profiling_)
+        return DefaultNetwork::RunLayers(prof_stream);
+    size_t next = 0;
+    for (int i = 0; i < (int)layers_.size(); ++i) {
+        while (next < groups_.size() && groups_[next].first < i)
+            ++next;
+        if (next < groups_.size() && groups_[next].first == i && groups_[next].active) {
+            Status st = groups_[next].acc->Forward(groups_[next].inputs, groups_[next].outputs);
+            if (st != TNN_OK)
+                return Status((int)st, "Forward error of layers " + layers_[i]->GetLayerName() + " and on: " + st.description());
+            i = groups_[next].last;
+            continue;
+        }
+        Status st = layers_[i]->Forward();
+        if (st != TNN_OK)
+            return Status((int)st, "Forward error of layer " + layers_[i]->GetLayerName() + ": " + st.description());
+    }
+    return TNN_OK;
+}
+#endif
+
 #ifdef TNN_ROCM_ENGINE_TREE
 Status RocmNetwork::InitLayers(NetStructure *net_structure, NetResource *net_resource) {
     // float blobs follow the network precision (PRECISION_HIGH: fp32; PRECISION_LOW: bfloat16; otherwise fp16), the

@@ -19,6 +19,16 @@
 
 namespace TNN_NS {
 
+// Layers first .. last of a net that one acc computes in their place.  The graph, its blobs and the memory plan stay those of
+// the single layers; what lies between the group's inputs and its output is simply not written.
+struct RocmLayerGroup {
+    int first = 0, last = 0;
+    std::shared_ptr<LayerInfo> layer;  // type, inputs, output and parameters of the acc that stands for the group
+    std::shared_ptr<LayerResource> resource;
+};
+// the attention cores (projections included) that an fp32 net keeps as layers
+std::vector<RocmLayerGroup> RocmFindAttentionGroups(NetStructure *structure, NetResource *resource);
+
 class RocmNetwork : public DefaultNetwork {
 public:
     RocmNetwork();
@@ -26,6 +36,17 @@ public:
     Status Forward() override;
     Status ForwardAsync(Callback call_back) override;
 
+#ifndef TNN_ROCM_ENGINE_TREE
+    Status Init(NetworkConfig &net_config, ModelInterpreter *interpreter, const InputShapesMap &max_inputs_shape = InputShapesMap()) override;
+    Status Reshape(const InputShapesMap &inputs) override;
+
+protected:
+    // The layer loop of a plain forward.  An fp32 net keeps its attention as layers (every intermediate blob is there for
+    // ForwardWithCallback, profiling and whoever names one as a model output), and those ways of running it take them one
+    // by one; a plain forward runs each core as a group: one projection for Q, K and V and one attention kernel instead of
+    // sixteen launches that pass the [B*h, S, S] scores through memory six times.
+    Status RunLayers(void *prof_stream) override;
+#endif
 #ifdef TNN_ROCM_ENGINE_TREE
 protected:
     // The engine settles every blob's data type in UpdateBlobPrecision (default_network.cc:362-440), which returns
@@ -38,6 +59,18 @@ protected:
 #endif
 
 private:
+#ifndef TNN_ROCM_ENGINE_TREE
+    struct Group {
+        int first = 0, last = 0;
+        bool active = false;  // false: the shapes or the memory plan at hand do not allow it, its layers run one by one
+        std::shared_ptr<LayerInfo> layer;
+        std::shared_ptr<LayerResource> resource;
+        std::unique_ptr<AbstractLayerAcc> acc;
+        std::vector<Blob *> inputs, outputs;
+    };
+    Status ReshapeGroups();
+    std::vector<Group> groups_;
+#endif
     // Everything a recording depends on: dims and device address of every blob the layers touch, and the context's
     // scratch allocation count.  A recording is replayed only under the signature it was made with, so a Reshape, a
     // re-planned blob pool or a grown workspace lead back to eager passes and a new recording by themselves.

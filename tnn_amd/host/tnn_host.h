@@ -779,16 +779,16 @@ protected:
     std::vector<BaseLayer *> layers_;
     NetworkConfig config_;
     bool profiling_ = false;
+    NetStructure structure_;  // per-instance copy: optimizer rewrites never touch the interpreter
+    NetResource resource_;
+    virtual Status RunLayers(void *prof_stream);  // the layer loop inside Forward / ForwardAsync
 
 private:
     std::map<Blob *, int64_t> blob_capacity_;  // bytes behind each planned blob
-    NetStructure structure_;  // per-instance copy: optimizer rewrites never touch the interpreter
-    NetResource resource_;
     std::map<std::string, Blob *> blobs_;
     std::vector<void *> allocations_;
     BlobMap inputs_, outputs_;
     std::vector<char> prof_on_;
-    Status RunLayers(void *prof_stream);
     std::vector<std::pair<void *, void *>> prof_events_;
     std::vector<LayerProfile> prof_;
 };
