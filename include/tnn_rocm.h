@@ -371,7 +371,9 @@ TNN_ROCM_API int tnn_rocm_gelu_i8(void *stream, const int8_t *q_in, float in_sca
  *   gemm_tune     : "MxNxK:code,..." overrides of the heuristic for single shapes (also TNN_ROCM_GEMM_TUNE at first use)
  *   gemm_group_m  : tiles per group of the XCD-aware tile order (0 = default)
  *   ln_y_ahead    : 1 (default) = the LayerNorm-folding GEMMs request the source vectors of their y output early
- *   attention_dma : 1 (default) = V^T attention stages K / V^T tiles global -> LDS directly, 0 = through registers
+ *   attention_dma : 1 (default) = by size: the kernel for few query blocks, or K / V^T tiles staged global -> LDS directly
+ *                   (row-major V: through registers); 0 = always through registers; 2 = always the kernel for few query
+ *                   blocks; 3 = never that one
  *   store_through : 1 (default) = GEMM and attention results are stored through the L2 at device scope, so that no
  *                   dirty lines wait for the write-back at the end of the kernel; 0 = ordinary write-back stores.
  *                   Read by the kernels when they run (recorded graphs follow it too); waits for the device first. */

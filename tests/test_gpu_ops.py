@@ -838,6 +838,40 @@ def test_attention_bf16():
     assert rel_err(got, ref) <= 3e-2
 
 
+@pytest.mark.parametrize("tdt,tol", [(torch.float16, FP16_TOL), (torch.bfloat16, 1.5e-2)])
+@pytest.mark.parametrize("B,h,S", [(1, 1, 1), (2, 3, 31), (1, 2, 32), (2, 2, 33), (1, 2, 129), (2, 1, 200), (1, 2, 8), (2, 2, 40),
+                                   (1, 3, 48), (2, 1, 520)])
+def test_attention_few_query_blocks(B, h, S, tdt, tol):
+    """The kernel for few query blocks, forced, around its blocks of 32 queries and keys and its four key waves: row-major V,
+    V^T in both key orders, lengths, an additive mask, the quantised second output"""
+    from tnn_amd import capi
+    say("attention, few query blocks, B=%d h=%d S=%d %s" % (B, h, S, tdt))
+    rng = np.random.default_rng(S * 3 + B)
+    H = 64 * h
+    qkv = torch.from_numpy(rng.standard_normal((B * S, 3 * H)).astype(np.float32)).to(tdt)
+    q, k, v = (x.float().numpy().reshape(B, S, h, 64).transpose(0, 2, 1, 3) for x in qkv.split(H, 1))
+    lens = rng.integers(1, S + 1, B).astype(np.int32)
+    cut = np.where(np.arange(S)[None, :] < lens[:, None], 0.0, -10000.0).astype(np.float32)
+    add = (rng.standard_normal((B, S)) * 3).astype(np.float32)
+    ref = {n: orc.attention_core(q, k, v, 0.125, m).transpose(0, 2, 1, 3).reshape(B * S, H) for n, m in (("len", cut), ("add", add))}
+    o, lib = ops(), capi.load()
+    lib.tnn_rocm_debug_set_attention_dma(2)
+    try:
+        assert rel_err(host(o.attention_packed(qkv.cuda(), B, S, h, 0.125, kv_len=dev(lens))), ref["len"]) <= tol
+        assert rel_err(host(o.attention_packed(qkv.cuda(), B, S, h, 0.125, mask=dev(add))), ref["add"]) <= tol
+        if S % 8 == 0:
+            qk = qkv[:, :2 * H].contiguous().cuda()
+            vt = qkv[:, 2 * H:].reshape(B, S, h, 64).permute(0, 2, 3, 1).contiguous()
+            nat = o.attention_qk_vt(qk, vt.cuda(), B, S, h, 0.125, kv_len=dev(lens), q8_inv_scale=np.float32(40.0))
+            assert rel_err(host(nat[0]), ref["len"]) <= tol
+            assert np.array_equal(host(nat[1]), orc.quantize_x86(host(nat[0]).astype(np.float32), np.float32(1 / 40.0)))
+            if S % 16 == 0:
+                per = host(o.attention_qk_vt(qk, o.permute_keys(vt).cuda(), B, S, h, 0.125, kv_len=dev(lens), vt_key_order=1))
+                assert np.array_equal(per, host(nat[0]))
+    finally:
+        lib.tnn_rocm_debug_set_attention_dma(1)
+
+
 @pytest.mark.parametrize("B,h,S", [(1, 1, 1), (2, 3, 31), (1, 2, 32), (2, 2, 33), (3, 4, 128), (1, 2, 161), (2, 1, 500)])
 @pytest.mark.parametrize("masked", ["none", "lengths", "additive"])
 def test_attention_fp32(B, h, S, masked):

@@ -100,27 +100,28 @@ template <> struct AttnT<TNN_ROCM_BF16> {
     }
     static __device__ __forceinline__ float to_float(uint16_t bits) { return __uint_as_float((uint32_t)bits << 16); }
     static __device__ __forceinline__ uint32_t pack2(float lo, float hi) {
-        return (uint32_t)float_to_bf16(lo) | ((uint32_t)float_to_bf16(hi) << 16);
+        return floats_to_bf16_pair(lo, hi);
     }
     static __device__ __forceinline__ uint32_t pack_only(float lo, float hi) {
-        return (uint32_t)float_to_bf16(lo) | ((uint32_t)float_to_bf16(hi) << 16);
+        return floats_to_bf16_pair(lo, hi);
     }
     static __device__ __forceinline__ void add_packed(uint32_t pk, float &sum) {
         sum += __uint_as_float(pk << 16) + __uint_as_float(pk & 0xffff0000u);
     }
     static __device__ __forceinline__ uint32_t pack_prob(float lo, float hi, float &sum) {
-        uint32_t l = float_to_bf16(lo), h = float_to_bf16(hi);
-        sum += __uint_as_float(l << 16) + __uint_as_float(h << 16);  // the rounded values, as in the fp16 path
-        return l | (h << 16);
+        const uint32_t pk = floats_to_bf16_pair(lo, hi);
+        add_packed(pk, sum);  // the rounded values, as in the fp16 path
+        return pk;
     }
 };
 
-struct AttnParams {
+struct AttnParams : StoreThrough {
     const uint16_t *q, *k, *v;
     uint16_t *o;
     long q_sb, q_sh, q_ss, kv_sb, kv_sh, kv_ss, o_sb, o_sh, o_ss;
     long vt_sb, vt_sh, vt_sd;  // V^T layout (VT kernels): element (b, head, d, s) at v[b*vt_sb + head*vt_sh + d*vt_sd + s]
     int S, B, heads;
+    FixedDivisor by_blocks, by_heads;  // query blocks of a head (set by the launch, which knows the block size); heads
     float scale_log2e;  // scale * log2(e)
     const float *mask;  // [B,S] additive or null
     const int32_t *kv_len;
@@ -167,6 +168,7 @@ __global__ void __launch_bounds__(NW * 64, (NW == 4 && DT == TNN_ROCM_F16) ? 3 :
     unsigned char *const lds_k1 = lds_all + 2 * kTileBytes, *const lds_vt1 = lds_all + 3 * kTileBytes;
     static_assert(BQ * kRowBytes <= 2 * kTileBytes, "Q / O staging must fit half of the tile buffers");
 
+    touch_kernel_args<sizeof(AttnParams)>();
     const int tid  = threadIdx.x;
     const int lane = tid & 63;
     const int wave = tid >> 6;
@@ -182,8 +184,8 @@ __global__ void __launch_bounds__(NW * 64, (NW == 4 && DT == TNN_ROCM_F16) ? 3 :
     const int vid   = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
     if (vid >= total)
         return;  // the grid is padded to a multiple of 8; whole workgroups leave before any barrier
-    const int bh   = vid / n_q;
-    const int b    = bh / p.heads;
+    const int bh   = p.by_blocks.quotient(vid);
+    const int b    = p.by_heads.quotient(bh);
     const int head = bh - b * p.heads;
     const int q0   = (vid - bh * n_q) * BQ + wave * 32;
 
@@ -445,7 +447,7 @@ __global__ void __launch_bounds__(NW * 64, (NW == 4 && DT == TNN_ROCM_F16) ? 3 :
             const int qrow = q0 + r;
             if (qrow < S) {
                 const u32x4 v = *reinterpret_cast<const u32x4 *>(stage + r * kRowBytes + (lane & 7) * 16);
-                store_out16(ob + (size_t)qrow * p.o_ss + (lane & 7) * 8, v);
+                store_out16(p.through, ob + (size_t)qrow * p.o_ss + (lane & 7) * 8, v);
                 if (p.oq) {
                     // the Reformat layer that follows in a quantised net (x86 form: multiply by 1/scale, round half
                     // away from zero, saturate), applied to the values as stored
@@ -462,7 +464,7 @@ __global__ void __launch_bounds__(NW * 64, (NW == 4 && DT == TNN_ROCM_F16) ? 3 :
                         q8[w] = packed;
                     }
                     int8_t *oqb = p.oq + (size_t)b * p.o_sb + (size_t)head * p.o_sh;
-                    store_out8(oqb + (size_t)qrow * p.o_ss + (lane & 7) * 8, q8);
+                    store_out8(p.through, oqb + (size_t)qrow * p.o_ss + (lane & 7) * 8, q8);
                 }
             }
         }
@@ -490,6 +492,7 @@ __global__ void __launch_bounds__(NW * 64, (NW == 4 && DT == TNN_ROCM_F16) ? 3 :
     __shared__ __attribute__((aligned(16))) unsigned char lds_all[3 * kStage];
     __shared__ __attribute__((aligned(16))) float lds_bias[3][kTileKV];
 
+    touch_kernel_args<sizeof(AttnParams)>();
     const int tid  = threadIdx.x;
     const int lane = tid & 63;
     const int wave = tid >> 6;
@@ -502,8 +505,8 @@ __global__ void __launch_bounds__(NW * 64, (NW == 4 && DT == TNN_ROCM_F16) ? 3 :
     const int vid   = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
     if (vid >= total)
         return;
-    const int bh   = vid / n_q;
-    const int b    = bh / p.heads;
+    const int bh   = p.by_blocks.quotient(vid);
+    const int b    = p.by_heads.quotient(bh);
     const int head = bh - b * p.heads;
     const int q0   = (vid - bh * n_q) * BQ + wave * 32;
 
@@ -988,7 +991,7 @@ __global__ void __launch_bounds__(NW * 64, (NW == 4 && DT == TNN_ROCM_F16) ? 3 :
             const int qrow = q0 + r;
             if (qrow < S) {
                 const u32x4 v = *reinterpret_cast<const u32x4 *>(stg + r * kRowBytes + (lane & 7) * 16);
-                store_out16(ob + (size_t)qrow * p.o_ss + (lane & 7) * 8, v);
+                store_out16(p.through, ob + (size_t)qrow * p.o_ss + (lane & 7) * 8, v);
                 if (p.oq) {
                     u32x2 q8;
 #pragma unroll
@@ -1003,7 +1006,7 @@ __global__ void __launch_bounds__(NW * 64, (NW == 4 && DT == TNN_ROCM_F16) ? 3 :
                         q8[w] = packed;
                     }
                     int8_t *oqb = p.oq + (size_t)b * p.o_sb + (size_t)head * p.o_sh;
-                    store_out8(oqb + (size_t)qrow * p.o_ss + (lane & 7) * 8, q8);
+                    store_out8(p.through, oqb + (size_t)qrow * p.o_ss + (lane & 7) * 8, q8);
                 }
             }
         }
@@ -1062,47 +1065,310 @@ __global__ void mask_to_kv_len_kernel(const typename Elem<DT>::type *__restrict_
 }
 
 // 128-row query blocks when that already gives >= 2 workgroups per CU, else 64-row blocks
-std::atomic<int> g_attention_dma{1};  // experiment hook: 0 keeps the register-staged kernel for the V^T layout as well
+// experiment hook: 1 = by size; 0 keeps the register-staged kernel for everything; 2 = the kernel for few query blocks for
+// everything; 3 = never that one
+std::atomic<int> g_attention_dma{1};
 
-template <bool VT> int launch_attention(hipStream_t s, int dtype, const AttnParams &p, int B, int heads, int S) {
-    long blocks128 = (long)((S + 127) / 128) * heads * B;
-    auto padded = [&](long n_q) { return dim3((unsigned)(((n_q * heads * B + 7) / 8) * 8)); };
-    if (VT && g_attention_dma) {
+// ---- few query blocks -----------------------------------------------------------------------------------------------
+// The same core for launches that leave most of the chip idle in the forms above (one sequence of 32 to 512 tokens, 12
+// heads: 12 to 96 workgroups).  A workgroup takes 32 queries; its four waves take every fourth block of 32 keys each, with a
+// running maximum and sum of their own, and are merged through LDS at the end, so the chain from the first load to the last
+// product is a quarter as long.  Nothing is shared between the waves: Q, K and V go from memory straight into the fragment
+// registers (K and V^T 16 bytes per lane and row; row-major V two neighbouring columns per lane and key, which the packing of
+// two keys into one register then sorts out), so there is no staging, no barrier before the merge, and any sequence length
+// serves.  What bounds it is latency: arguments, then Q, K and V at once, then the products.
+// Measured at the rule in front of launch_attention.
+template <int DT, bool VT> __global__ void __launch_bounds__(256, 2) attention_short_kernel(AttnParams p) {
+    constexpr int NW = 4, BQ = 32, BK = 32, ROW = kD + 4;
+    __shared__ __attribute__((aligned(16))) float stage[NW][BQ * ROW];
+    __shared__ float stat_m[NW][BQ], stat_l[NW][BQ];
+    touch_kernel_args<sizeof(AttnParams)>();
+    const int tid  = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int g    = lane >> 5;
+    const int lq   = lane & 31;
+    const int S    = p.S;
+    const int n_q   = (S + BQ - 1) / BQ;
+    const int total = n_q * p.heads * p.B;
+    const int per   = (total + 7) >> 3;
+    const int vid   = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
+    if (vid >= total)
+        return;  // the grid is padded to a multiple of 8; whole workgroups leave before any barrier
+    const int bh   = p.by_blocks.quotient(vid);
+    const int b    = p.by_heads.quotient(bh);
+    const int head = bh - b * p.heads;
+    const int q0   = (vid - bh * n_q) * BQ;
+    const uint16_t *qb = p.q + (size_t)b * p.q_sb + (size_t)head * p.q_sh;
+    const uint16_t *kb = p.k + (size_t)b * p.kv_sb + (size_t)head * p.kv_sh;
+    const uint16_t *vb = VT ? p.v + (size_t)b * p.vt_sb + (size_t)head * p.vt_sh : p.v + (size_t)b * p.kv_sb + (size_t)head * p.kv_sh;
+    const uint32_t ss = (uint32_t)p.kv_ss, vd = (uint32_t)p.vt_sd;
+
+    // rows past the end are clamped to the last one: such keys get the score -inf, such queries are never stored
+    u32x4 qf[4], kf[4];
+    uint32_t vr[VT ? 1 : 16];
+    u32x4 vf_t[VT ? 4 : 1];
+    auto load_k = [&](int t) __attribute__((always_inline)) {
+        const int row = t * BK + lq < S ? t * BK + lq : S - 1;
+        const uint16_t *src = kb + ((uint32_t)row * ss + 8u * g);
+#pragma unroll
+        for (int kk = 0; kk < 4; ++kk)
+            kf[kk] = *reinterpret_cast<const u32x4 *>(src + kk * 16);
+    };
+    auto load_v = [&](int t) __attribute__((always_inline)) {
+        if constexpr (VT) {
+            // row d = 32*dt + lq of V^T, the eight keys of lane half g in step st: contiguous in the accumulators' key
+            // order, two groups of four in the natural one
+#pragma unroll
+            for (int dt = 0; dt < 2; ++dt)
+#pragma unroll
+                for (int st = 0; st < 2; ++st) {
+                    const uint16_t *row = vb + (uint32_t)(dt * 32 + lq) * vd;
+                    const int k0        = t * BK + st * 16;
+                    if (p.vt_perm) {
+                        vf_t[dt * 2 + st] = *reinterpret_cast<const u32x4 *>(row + (k0 < S ? k0 + 8 * g : 8 * g));
+                    } else {
+                        const int a = k0 + 4 * g < S ? k0 + 4 * g : S - 4, c = k0 + 8 + 4 * g < S ? k0 + 8 + 4 * g : S - 4;
+                        const u32x2 lo = *reinterpret_cast<const u32x2 *>(row + a), hi = *reinterpret_cast<const u32x2 *>(row + c);
+                        vf_t[dt * 2 + st] = u32x4{lo[0], lo[1], hi[0], hi[1]};
+                    }
+                }
+        } else {
+            // slot e of step st and lane half g: key 16*st + 4*g + e (e < 4), 16*st + 8 + 4*g + e-4; columns 2*lq, 2*lq + 1
+#pragma unroll
+            for (int st = 0; st < 2; ++st)
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const int key = t * BK + 16 * st + 4 * g + (e & 3) + (e & 4) * 2;
+                    vr[st * 8 + e] = *reinterpret_cast<const uint32_t *>(vb + ((uint32_t)(key < S ? key : S - 1) * ss + 2u * lq));
+                }
+        }
+    };
+    {
+        const int row = q0 + lq < S ? q0 + lq : S - 1;
+        const uint16_t *src = qb + (size_t)row * p.q_ss + 8 * g;
+#pragma unroll
+        for (int kk = 0; kk < 4; ++kk)
+            qf[kk] = *reinterpret_cast<const u32x4 *>(src + kk * 16);
+    }
+    if (wave * BK < S) {  // before the sequence's length is known
+        load_k(wave);
+        load_v(wave);
+    }
+    int kv_end        = S;
+    bool mask_is_zero = false;
+    if (p.kv_len) {
+        int l        = p.kv_len[b];
+        mask_is_zero = l >= 0 && (l & kKvLenMaskZero) != 0;
+        l            = l >= 0 ? (l & ~kKvLenMaskZero) : l;
+        kv_end       = l < 0 ? 0 : (l < S ? l : S);
+    }
+    const float *mb   = p.mask && !mask_is_zero ? p.mask + (size_t)b * S : nullptr;
+    const int n_tiles = (kv_end + BK - 1) / BK;
+
+    f32x16 oacc[2];
+#pragma unroll
+    for (int dt = 0; dt < 2; ++dt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+            oacc[dt][r] = 0.f;
+    float m_i = -INFINITY, l_i = 0.f;
+    for (int t = wave; t < n_tiles; t += NW) {
+        f32x16 s;
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+            s[r] = 0.f;
+#pragma unroll
+        for (int kk = 0; kk < 4; ++kk)
+            AttnT<DT>::mma(kf[kk], qf[kk], s);
+        u32x4 vf[4];  // [dt][st], out of the way of the next block's loads
+        if constexpr (VT) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                vf[q] = vf_t[q];
+        } else {
+#pragma unroll
+            for (int st = 0; st < 2; ++st)
+#pragma unroll
+                for (int h = 0; h < 4; ++h) {
+                    const uint32_t x = vr[st * 8 + 2 * h], y = vr[st * 8 + 2 * h + 1];
+                    vf[st][h]     = __builtin_amdgcn_perm(y, x, 0x05040100u);
+                    vf[2 + st][h] = __builtin_amdgcn_perm(y, x, 0x07060302u);
+                }
+        }
+        if (t + NW < n_tiles) {
+            load_k(t + NW);
+            load_v(t + NW);
+        }
+        // softmax in the exp2 domain; register r is key 8*(r/4) + 4*g + r%4 of the block
+        float mx = -INFINITY;
+        const bool biased = mb != nullptr || (t + 1) * BK > kv_end;  // uniform
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            float v = s[r] * p.scale_log2e;
+            if (biased) {
+                const int key = t * BK + 8 * (r >> 2) + 4 * g + (r & 3);
+                if (mb)
+                    v = fmaf(mb[key < S ? key : S - 1], kLog2e, v);
+                v = key < kv_end ? v : -INFINITY;
+            }
+            s[r] = v;
+            mx   = fmaxf(mx, v);
+        }
+        mx                = half_swap_max(mx);
+        const float m_new = fmaxf(m_i, mx);
+        const float m_use = m_new == -INFINITY ? 0.f : m_new;
+        const float alpha = __builtin_amdgcn_exp2f(m_i - m_use);
+        float rs = 0.f;
+        u32x4 pf[2];
+#pragma unroll
+        for (int st = 0; st < 2; ++st)
+#pragma unroll
+            for (int h = 0; h < 4; ++h)
+                pf[st][h] = AttnT<DT>::pack_prob(__builtin_amdgcn_exp2f(s[8 * st + 2 * h] - m_use),
+                                                 __builtin_amdgcn_exp2f(s[8 * st + 2 * h + 1] - m_use), rs);
+        if (!__all(m_new == m_i)) {
+#pragma unroll
+            for (int dt = 0; dt < 2; ++dt)
+#pragma unroll
+                for (int r = 0; r < 16; ++r)
+                    oacc[dt][r] *= alpha;
+        }
+        m_i = m_new;
+#pragma unroll
+        for (int st = 0; st < 2; ++st)
+#pragma unroll
+            for (int dt = 0; dt < 2; ++dt)
+                AttnT<DT>::mma(vf[dt * 2 + st], pf[st], oacc[dt]);
+        l_i = fmaf(l_i, alpha, half_swap_sum(rs));
+    }
+
+    // ---- merge: every wave leaves its sums, scaled to its own maximum; a thread then adds up eight columns of a row
+    {
+        float *row = stage[wave] + lq * ROW;
+#pragma unroll
+        for (int r4 = 0; r4 < 4; ++r4) {
+            const int i0 = 8 * r4 + 4 * g;  // accumulator rows i0 .. i0+3
+            typedef float f32x4 __attribute__((ext_vector_type(4)));
+            if constexpr (VT) {  // column 32*dt + i
+#pragma unroll
+                for (int dt = 0; dt < 2; ++dt)
+                    *reinterpret_cast<f32x4 *>(row + dt * 32 + i0) =
+                        f32x4{oacc[dt][r4 * 4], oacc[dt][r4 * 4 + 1], oacc[dt][r4 * 4 + 2], oacc[dt][r4 * 4 + 3]};
+            } else {  // column 2*i + dt
+                *reinterpret_cast<f32x4 *>(row + 2 * i0)     = f32x4{oacc[0][r4 * 4], oacc[1][r4 * 4], oacc[0][r4 * 4 + 1], oacc[1][r4 * 4 + 1]};
+                *reinterpret_cast<f32x4 *>(row + 2 * i0 + 4) = f32x4{oacc[0][r4 * 4 + 2], oacc[1][r4 * 4 + 2], oacc[0][r4 * 4 + 3], oacc[1][r4 * 4 + 3]};
+            }
+        }
+        if (lane < 32) {
+            stat_m[wave][lq] = m_i;
+            stat_l[wave][lq] = l_i;
+        }
+    }
+    __syncthreads();
+    const int row = tid >> 3, c = (tid & 7) * 8;
+    if (q0 + row >= S)
+        return;
+    float top = stat_m[0][row];
+#pragma unroll
+    for (int w = 1; w < NW; ++w)
+        top = fmaxf(top, stat_m[w][row]);
+    top = top == -INFINITY ? 0.f : top;
+    float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, sum = 0.f;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+        const float f = __builtin_amdgcn_exp2f(stat_m[w][row] - top);
+        sum           = fmaf(stat_l[w][row], f, sum);
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+            acc[e] = fmaf(stage[w][row * ROW + c + e], f, acc[e]);
+    }
+    const float inv = sum > 0.f ? 1.0f / sum : 0.f;
+    u32x4 out;
+#pragma unroll
+    for (int h = 0; h < 4; ++h)
+        out[h] = AttnT<DT>::pack2(acc[2 * h] * inv, acc[2 * h + 1] * inv);
+    const size_t at = (size_t)b * p.o_sb + (size_t)head * p.o_sh + (size_t)(q0 + row) * p.o_ss + c;
+    store_out16(p.through, p.o + at, out);
+    if (p.oq) {  // the values as stored, quantised (see attention_kernel)
+        u32x2 q8;
+#pragma unroll
+        for (int w = 0; w < 2; ++w) {
+            uint32_t packed = 0;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const uint32_t word = out[w * 2 + (e >> 1)];
+                const float f       = AttnT<DT>::to_float((uint16_t)(e & 1 ? word >> 16 : word & 0xffffu));
+                packed |= (uint32_t)(uint8_t)float2int8_ref(__fmul_rn(f, p.q_inv)) << (8 * e);
+            }
+            q8[w] = packed;
+        }
+        store_out8(p.through, p.oq + at, q8);
+    }
+}
+
+// The kernel for few query blocks is the faster one as long as its blocks of 32 queries are about as many as the chip has CUs
+// (V^T layout: the LDS-staged kernel reads every K and V tile once per 64 or 128 queries and wins from there on), several times
+// as many where V comes row-major (its transposition through LDS is what the other kernel waits for), and always where one
+// block holds the whole sequence (the other kernels' 64 queries are then half empty).  us, fp16, 12 heads, before -> now:
+//   V^T        B1 S32 5.0 -> 4.0   B1 S128 6.0 -> 4.8   B1 S256 6.8 -> 5.5   B1 S512 9.1 -> 6.9   B2 S512 9.7 (this one: 10.3)
+//   row-major  B1 S197 8.2 -> 5.5   B5 S197 9.7 -> 7.1   B8 S384 18.3 -> 17.2   B16 S256 14.3 (this one: 15.9)
+// A launch with the quantised second output stays with the other kernels: the two forms round differently (within the type's
+// own rounding), and an int8 step that falls the other way is a 127th of the range for every layer behind it.
+constexpr long kShortBlocksVT = 256, kShortBlocksRows = 1200;
+
+template <bool VT> int launch_attention(hipStream_t s, int dtype, AttnParams p, int B, int heads, int S) {
+    const long blocks128 = (long)((S + 127) / 128) * heads * B, blocks32 = (long)((S + 31) / 32) * heads * B;
+    const int mode = g_attention_dma;
+    const bool few = !p.oq && (S <= 32 || blocks32 <= (VT ? kShortBlocksVT : kShortBlocksRows));
+    p.by_heads     = FixedDivisor::of((uint32_t)heads);
+    // grid of the launch with BQ queries per block
+    auto blocks_of = [&](int bq) {
+        const long n_q = (S + bq - 1) / bq;
+        p.by_blocks    = FixedDivisor::of((uint32_t)n_q);
+        return dim3((unsigned)(((n_q * heads * B + 7) / 8) * 8));
+    };
+#define TR_LAUNCH(KERNEL, THREADS) hipLaunchKernelGGL(KERNEL, grid, dim3(THREADS), 0, s, p)
+    if (mode == 2 || (mode == 1 && few)) {
+        const dim3 grid = blocks_of(32);
+        if (dtype == TNN_ROCM_F16)
+            TR_LAUNCH((attention_short_kernel<TNN_ROCM_F16, VT>), 256);
+        else
+            TR_LAUNCH((attention_short_kernel<TNN_ROCM_BF16, VT>), 256);
+    } else if (VT && mode) {
 #define TR_LAUNCH_DMA(NWv, THREADS)                                                                                   \
     do {                                                                                                              \
         if (dtype == TNN_ROCM_F16 && p.vt_perm)                                                                       \
-            hipLaunchKernelGGL((attention_dma_kernel<TNN_ROCM_F16, NWv, true>), grid, dim3(THREADS), 0, s, p);        \
+            TR_LAUNCH((attention_dma_kernel<TNN_ROCM_F16, NWv, true>), THREADS);                                      \
         else if (dtype == TNN_ROCM_F16)                                                                               \
-            hipLaunchKernelGGL((attention_dma_kernel<TNN_ROCM_F16, NWv, false>), grid, dim3(THREADS), 0, s, p);       \
+            TR_LAUNCH((attention_dma_kernel<TNN_ROCM_F16, NWv, false>), THREADS);                                     \
         else if (p.vt_perm)                                                                                           \
-            hipLaunchKernelGGL((attention_dma_kernel<TNN_ROCM_BF16, NWv, true>), grid, dim3(THREADS), 0, s, p);       \
+            TR_LAUNCH((attention_dma_kernel<TNN_ROCM_BF16, NWv, true>), THREADS);                                     \
         else                                                                                                          \
-            hipLaunchKernelGGL((attention_dma_kernel<TNN_ROCM_BF16, NWv, false>), grid, dim3(THREADS), 0, s, p);      \
+            TR_LAUNCH((attention_dma_kernel<TNN_ROCM_BF16, NWv, false>), THREADS);                                    \
     } while (0)
         if (blocks128 >= 512) {
-            dim3 grid = padded((S + 127) / 128);
+            const dim3 grid = blocks_of(128);
             TR_LAUNCH_DMA(4, 256);
         } else {
-            dim3 grid = padded((S + 63) / 64);
+            const dim3 grid = blocks_of(64);
             TR_LAUNCH_DMA(2, 128);
         }
 #undef TR_LAUNCH_DMA
-        TR_CHECK_LAUNCH();
-        return 0;
-    }
-    if (blocks128 >= 512) {
-        dim3 grid = padded((S + 127) / 128);
+    } else if (blocks128 >= 512) {
+        const dim3 grid = blocks_of(128);
         if (dtype == TNN_ROCM_F16)
-            hipLaunchKernelGGL((attention_kernel<TNN_ROCM_F16, 4, VT>), grid, dim3(256), 0, s, p);
+            TR_LAUNCH((attention_kernel<TNN_ROCM_F16, 4, VT>), 256);
         else
-            hipLaunchKernelGGL((attention_kernel<TNN_ROCM_BF16, 4, VT>), grid, dim3(256), 0, s, p);
+            TR_LAUNCH((attention_kernel<TNN_ROCM_BF16, 4, VT>), 256);
     } else {
-        dim3 grid = padded((S + 63) / 64);
+        const dim3 grid = blocks_of(64);
         if (dtype == TNN_ROCM_F16)
-            hipLaunchKernelGGL((attention_kernel<TNN_ROCM_F16, 2, VT>), grid, dim3(128), 0, s, p);
+            TR_LAUNCH((attention_kernel<TNN_ROCM_F16, 2, VT>), 128);
         else
-            hipLaunchKernelGGL((attention_kernel<TNN_ROCM_BF16, 2, VT>), grid, dim3(128), 0, s, p);
+            TR_LAUNCH((attention_kernel<TNN_ROCM_BF16, 2, VT>), 128);
     }
+#undef TR_LAUNCH
     TR_CHECK_LAUNCH();
     return 0;
 }
@@ -1210,7 +1476,6 @@ int tnn_rocm_attention_vt_q8(void *stream, int dtype, const void *q, const void 
     return launch_attention<true>((hipStream_t)stream, dtype, p, B, heads, S);
 }
 
-TR_DEFINE_STORE_THROUGH_SETTER(attention_set_store_through)
 __attribute__((visibility("default"))) int tnn_rocm_debug_set_attention_dma(int on) {
     g_attention_dma = on;
     return 0;

@@ -34,11 +34,12 @@ constexpr int kBlockK        = 32;
 constexpr int kKvLenMaskZero = 1 << 30;  // flag bit of a kv_len entry, see tnn_rocm_mask_to_kv_len_flagged
 constexpr int kStageRow      = kD + 4;   // floats; the pad spreads the rows over the banks
 
-struct AttnF32Params {
+struct AttnF32Params : StoreThrough {
     const float *q, *k, *v;
     float *o;
     long q_sb, q_sh, q_ss, kv_sb, kv_sh, kv_ss, o_sb, o_sh, o_ss;
     int S, B, heads;
+    FixedDivisor by_blocks, by_heads;
     float scale;
     const float *mask;  // [B,S] additive or null
     const int32_t *kv_len;
@@ -53,6 +54,7 @@ template <int NW> __global__ void __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) at
     __shared__ __attribute__((aligned(16))) float stage[NW][kBlockQ * kStageRow];
     __shared__ float stat_m[NW][kBlockQ], stat_l[NW][kBlockQ];
 
+    touch_kernel_args<sizeof(AttnF32Params)>();
     const int tid  = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -66,8 +68,8 @@ template <int NW> __global__ void __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) at
     const int vid   = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
     if (vid >= total)
         return;  // the grid is padded to a multiple of 8; whole workgroups leave before any barrier
-    const int bh   = vid / n_q;
-    const int b    = bh / p.heads;
+    const int bh   = p.by_blocks.quotient(vid);
+    const int b    = p.by_heads.quotient(bh);
     const int head = bh - b * p.heads;
     const int q0   = (vid - bh * n_q) * kBlockQ;
 
@@ -245,7 +247,7 @@ template <int NW> __global__ void __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) at
 #pragma unroll
         for (int e = 0; e < 4; ++e)
             acc[e] *= inv;
-        store_out16(p.o + (size_t)b * p.o_sb + (size_t)head * p.o_sh + (size_t)(q0 + row) * p.o_ss + c,
+        store_out16(p.through, p.o + (size_t)b * p.o_sb + (size_t)head * p.o_sh + (size_t)(q0 + row) * p.o_ss + c,
                     __builtin_bit_cast(store_u32x4, acc));
     }
 }
@@ -264,6 +266,8 @@ int launch_attention_f32(hipStream_t s, const float *q, const float *k, const fl
     p.kv_sb = kv_sb, p.kv_sh = kv_sh, p.kv_ss = kv_ss;
     p.o_sb = o_sb, p.o_sh = o_sh, p.o_ss = o_ss;
     p.S = S, p.B = B, p.heads = heads;
+    p.by_blocks = FixedDivisor::of((uint32_t)((S + kBlockQ - 1) / kBlockQ));
+    p.by_heads  = FixedDivisor::of((uint32_t)heads);
     p.scale  = scale;
     p.mask   = mask;
     p.kv_len = kv_len;
@@ -280,7 +284,3 @@ int launch_attention_f32(hipStream_t s, const float *q, const float *k, const fl
 }
 
 }  // namespace tnn_rocm
-
-extern "C" {
-TR_DEFINE_STORE_THROUGH_SETTER(attention_f32_set_store_through)
-}

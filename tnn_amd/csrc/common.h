@@ -6,6 +6,8 @@
 #include <stdint.h>
 #include <stdio.h>
 
+#include <atomic>
+
 #include "tnn_rocm.h"
 
 namespace tnn_rocm {
@@ -41,12 +43,12 @@ typedef uint16_t bf16_bits;
 __device__ __forceinline__ float bf16_to_float(bf16_bits v) {
     return __uint_as_float(((uint32_t)v) << 16);
 }
-__device__ __forceinline__ bf16_bits float_to_bf16(float f) {
-    uint32_t u = __float_as_uint(f);
-    if ((u & 0x7fffffffu) > 0x7f800000u)
-        return (bf16_bits)((u >> 16) | 0x40);  // quiet NaN
-    u += 0x7fffu + ((u >> 16) & 1u);           // round to nearest even
-    return (bf16_bits)(u >> 16);
+// round to nearest even, a NaN stays a (quiet) NaN: v_cvt_pk_bf16_f32, where the integer sequence for it takes six instructions
+__device__ __forceinline__ bf16_bits float_to_bf16(float f) { return __builtin_bit_cast(bf16_bits, (__bf16)f); }
+__device__ __forceinline__ uint32_t floats_to_bf16_pair(float lo, float hi) {
+    typedef float f2 __attribute__((ext_vector_type(2)));
+    typedef __bf16 b2 __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector((f2{lo, hi}), b2));
 }
 
 // Element load/store as float for the three floating dtypes.
@@ -60,36 +62,38 @@ __device__ __forceinline__ bf16_bits float_to_bf16(float f) {
 // The compiler has no spelling for a 16-byte store at device scope, hence the assembly; a store of more than 8 bytes
 // needs two wait states before its data registers may be overwritten, which the hazard recognizer cannot see through
 // an asm statement, so they are part of it.  No memory clobber: nothing in these kernels reads what they store.
-// The switch (one copy per translation unit, set together by tnn_rocm_debug_set_store_through) is there for A/B runs.
+// Whether they do is a kernel argument (StoreThrough, set by tnn_rocm_debug_set_store_through for A/B runs): as a variable in
+// device memory the switch cost every kernel two dependent scalar loads of cold lines in front of its first store, 0.2 us.
 typedef unsigned int store_u32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned int store_u32x2 __attribute__((ext_vector_type(2)));
-static __constant__ int g_dev_store_through = 1;
-#define TR_DEFINE_STORE_THROUGH_SETTER(name)                                                          \
-    int name(int on) { return (int)hipMemcpyToSymbol(HIP_SYMBOL(::tnn_rocm::g_dev_store_through), &on, sizeof(int)); }
+inline std::atomic<int> g_store_through{1};
+struct StoreThrough {
+    int through = g_store_through.load(std::memory_order_relaxed);
+};
 
-__device__ __forceinline__ void store_out16(void *p, store_u32x4 v) {
-    if (g_dev_store_through)
+__device__ __forceinline__ void store_out16(int through, void *p, store_u32x4 v) {
+    if (through)
         asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" ::"v"(p), "v"(v));
     else
         *reinterpret_cast<store_u32x4 *>(p) = v;
 }
-__device__ __forceinline__ void store_out8(void *p, store_u32x2 v) {
-    if (g_dev_store_through)
+__device__ __forceinline__ void store_out8(int through, void *p, store_u32x2 v) {
+    if (through)
         asm volatile("global_store_dwordx2 %0, %1, off sc1" ::"v"(p), "v"(v));
     else
         *reinterpret_cast<store_u32x2 *>(p) = v;
 }
-__device__ __forceinline__ void store_out8(float2 *p, float2 v) {
-    store_out8((void *)p, store_u32x2{__float_as_uint(v.x), __float_as_uint(v.y)});
+__device__ __forceinline__ void store_out8(int through, float2 *p, float2 v) {
+    store_out8(through, (void *)p, store_u32x2{__float_as_uint(v.x), __float_as_uint(v.y)});
 }
-__device__ __forceinline__ void store_out4(void *p, uint32_t v) {
-    if (g_dev_store_through)
+__device__ __forceinline__ void store_out4(int through, void *p, uint32_t v) {
+    if (through)
         asm volatile("global_store_dword %0, %1, off sc1" ::"v"(p), "v"(v));
     else
         *reinterpret_cast<uint32_t *>(p) = v;
 }
-__device__ __forceinline__ void store_out2(void *p, uint16_t v) {
-    if (g_dev_store_through)
+__device__ __forceinline__ void store_out2(int through, void *p, uint16_t v) {
+    if (through)
         asm volatile("global_store_short %0, %1, off sc1" ::"v"(p), "v"((uint32_t)v));
     else
         *reinterpret_cast<uint16_t *>(p) = v;
@@ -100,22 +104,22 @@ template <> struct Elem<TNN_ROCM_F32> {
     typedef float type;
     static __device__ __forceinline__ float ld(const float *p) { return *p; }
     static __device__ __forceinline__ void st(float *p, float v) { *p = v; }
-    static __device__ __forceinline__ void st_out(float *p, float v) { store_out4(p, __float_as_uint(v)); }
+    static __device__ __forceinline__ void st_out(int through, float *p, float v) { store_out4(through, p, __float_as_uint(v)); }
 };
 template <> struct Elem<TNN_ROCM_F16> {
     typedef half_t type;
     static __device__ __forceinline__ float ld(const half_t *p) { return (float)*p; }
     static __device__ __forceinline__ void st(half_t *p, float v) { *p = (half_t)v; }
-    static __device__ __forceinline__ void st_out(half_t *p, float v) {
+    static __device__ __forceinline__ void st_out(int through, half_t *p, float v) {
         const half_t h = (half_t)v;
-        store_out2(p, *reinterpret_cast<const uint16_t *>(&h));
+        store_out2(through, p, *reinterpret_cast<const uint16_t *>(&h));
     }
 };
 template <> struct Elem<TNN_ROCM_BF16> {
     typedef bf16_bits type;
     static __device__ __forceinline__ float ld(const bf16_bits *p) { return bf16_to_float(*p); }
     static __device__ __forceinline__ void st(bf16_bits *p, float v) { *p = float_to_bf16(v); }
-    static __device__ __forceinline__ void st_out(bf16_bits *p, float v) { store_out2(p, float_to_bf16(v)); }
+    static __device__ __forceinline__ void st_out(int through, bf16_bits *p, float v) { store_out2(through, p, float_to_bf16(v)); }
 };
 
 // Round half away from zero exactly as the reference's float2int8: add +-0.5f in fp32 (one
@@ -224,6 +228,32 @@ __device__ __forceinline__ float wave_max(float v) {
     return v;
 }
 
+// A kernel's arguments lie in cache lines that nothing on the chip has read yet.  The compiler loads them as it comes to them,
+// one miss after the other (1700 clocks to a GEMM's first slab request, with five lines); touched together they cost one.
+template <size_t BYTES> __device__ __forceinline__ void touch_kernel_args() {
+    typedef const __attribute__((address_space(4))) uint32_t *KernArg;
+    const KernArg args = (KernArg)__builtin_amdgcn_kernarg_segment_ptr();
+    uint32_t touched   = 0;
+#pragma unroll
+    for (int w = 0; w < (int)(BYTES / 4); w += 16)
+        touched |= args[w];
+    asm volatile("" ::"s"(touched));
+}
+
+// Division by a number the host knows, as a product: three scalar instructions where the compiler's sequence for an unknown
+// divisor takes some forty dependent ones, in front of everything else a workgroup does.  With s = ceil(log2 d) and
+// magic = ceil(2^(31+s) / d) the quotient is exact for every n below 2^31.
+struct FixedDivisor {
+    uint32_t magic, shift;
+    __device__ __forceinline__ int quotient(int n) const { return (int)(((uint64_t)(uint32_t)n * magic) >> shift); }
+    static FixedDivisor of(uint32_t d) {
+        uint32_t s = 0;
+        d          = d < 1 ? 1 : d;
+        while ((1ull << s) < d)
+            ++s;
+        return {(uint32_t)(((1ull << (31 + s)) + d - 1) / d), 31 + s};
+    }
+};
 static inline bool is_float_dtype(int dt) {
     return dt == TNN_ROCM_F32 || dt == TNN_ROCM_F16 || dt == TNN_ROCM_BF16;
 }

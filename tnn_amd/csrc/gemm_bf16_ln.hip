@@ -8,7 +8,3 @@ template int GemmTyped<TNN_ROCM_BF16>::qkv_split_ln(hipStream_t, const void *, c
     *, const float *, const float *, float, void *, void *, void *, float *, const float *, int, int, int, int, int,
     int);
 }  // namespace tnn_rocm
-
-extern "C" {
-TR_DEFINE_STORE_THROUGH_SETTER(gemm_bf16_ln_set_store_through)
-}

@@ -9,7 +9,3 @@ template int GemmTyped<TNN_ROCM_F16>::qkv_split(hipStream_t, const void *, const
 template int GemmTyped<TNN_ROCM_F16>::residual_ln(hipStream_t, const void *, const void *, const float *, void *, const
     void *, const float *, const float *, const float *, int, int, int, int, float *, int *);
 }  // namespace tnn_rocm
-
-extern "C" {
-TR_DEFINE_STORE_THROUGH_SETTER(gemm_f16_set_store_through)
-}

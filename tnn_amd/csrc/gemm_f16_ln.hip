@@ -8,7 +8,3 @@ template int GemmTyped<TNN_ROCM_F16>::qkv_split_ln(hipStream_t, const void *, co
     *, const float *, const float *, float, void *, void *, void *, float *, const float *, int, int, int, int, int,
     int);
 }  // namespace tnn_rocm
-
-extern "C" {
-TR_DEFINE_STORE_THROUGH_SETTER(gemm_f16_ln_set_store_through)
-}

@@ -5,7 +5,3 @@ namespace tnn_rocm {
 template int GemmTyped<TNN_ROCM_F32>::plain(hipStream_t, bool, const void *, const void *, void *, int, int, int, int,
     int, int, int, int, int, int, const float *, const void *, int);
 }  // namespace tnn_rocm
-
-extern "C" {
-TR_DEFINE_STORE_THROUGH_SETTER(gemm_f32_set_store_through)
-}

@@ -49,7 +49,3 @@ template int GemmI8::qkv_split<TNN_ROCM_BF16>(hipStream_t, const int8_t *, const
     const float *, void *, void *, int, int, int, int, int);
 
 }  // namespace tnn_rocm
-
-extern "C" {
-TR_DEFINE_STORE_THROUGH_SETTER(gemm_i8_set_store_through)
-}

@@ -190,11 +190,15 @@ template <typename E, typename = void> struct ColArrays : std::integral_constant
 template <typename E> struct ColArrays<E, typename std::enable_if<(E::kColArrays > 0)>::type> : std::integral_constant<int, E::kColArrays> {};
 template <typename E, typename = void> struct RowIn : std::false_type {};
 template <typename E> struct RowIn<E, typename std::enable_if<E::kRowIn>::type> : std::true_type {};
+//   kAheadVecs     the epilogue reads that many 16-byte vectors of another matrix (a residual) per item: ahead_src(m, n) is
+//                  where they are, or null.  A shape whose threads have one item each requests them before its first slab
+template <typename E, typename = void> struct AheadVecs : std::integral_constant<int, 0> {};
+template <typename E> struct AheadVecs<E, typename std::enable_if<(E::kAheadVecs > 0)>::type> : std::integral_constant<int, E::kAheadVecs> {};
 template <typename E, typename = void> struct SumBlocks : std::integral_constant<int, 1> {};
 template <typename E> struct SumBlocks<E, typename std::enable_if<E::kTakesRowSums>::type> : std::integral_constant<int, E::kSumBlocks> {};  // tile columns of a producer a consumer can add up (768 columns of 32)
 
 
-template <int DT> struct FloatEpilogue {
+template <int DT> struct FloatEpilogue : StoreThrough {
     typedef typename Elem<DT>::type T;
     static constexpr bool kRowStats = false;
     int flags;
@@ -227,8 +231,12 @@ template <int DT> struct FloatEpilogue {
     // (half) / 32-byte (fp32) pieces, so that the lanes of one row together write full cache lines
     static constexpr int kColArrays = 1;  // bias
     __device__ __forceinline__ float col_src(int, int n) const { return (flags & TNN_ROCM_EPI_BIAS) ? bias[n] : 0.f; }
-    // cl = the item's eight columns of the bias in LDS
-    __device__ __forceinline__ void store8(int m, int n, const float (&acc)[8], const float *cl, int) const {
+    static constexpr int kAheadVecs = 8 * sizeof(T) / 16;
+    __device__ __forceinline__ const void *ahead_src(int m, int n) const {
+        return (flags & TNN_ROCM_EPI_RESIDUAL) ? residual + (size_t)m * ldr + n : nullptr;
+    }
+    // cl = the item's eight columns of the bias in LDS; ahead = the residual's vectors where they have been requested already
+    __device__ __forceinline__ void store8(int m, int n, const float (&acc)[8], const float *cl, int, const u32x4 *ahead) const {
         float v[8];
 #pragma unroll
         for (int t = 0; t < 8; ++t)
@@ -250,7 +258,7 @@ template <int DT> struct FloatEpilogue {
             const u32x4 *rp = reinterpret_cast<const u32x4 *>(residual + (size_t)m * ldr + n);
 #pragma unroll
             for (int q = 0; q < NV; ++q)
-                packed[q] = rp[q];
+                packed[q] = ahead ? ahead[q] : rp[q];
 #pragma unroll
             for (int t = 0; t < 8; ++t)
                 v[t] += Elem<DT>::ld(&pe[t]);
@@ -261,7 +269,7 @@ template <int DT> struct FloatEpilogue {
         u32x4 *cp = reinterpret_cast<u32x4 *>(C + (size_t)m * ldc + n);
 #pragma unroll
         for (int q = 0; q < NV; ++q)
-            store_out16(&cp[q], packed[q]);
+            store_out16(through, &cp[q], packed[q]);
     }
 };
 
@@ -271,7 +279,7 @@ template <int DT> struct FloatEpilogue {
 __device__ __forceinline__ int key_slot(int s, int sh) { return (s & ~12) | ((s & 4) << sh) | ((s & 8) >> sh); }
 
 // QKV projection epilogue: columns [0,2H) -> qk[T,2H]; columns [2H,3H) -> V^T[b][head][d][s]
-template <int DT> struct QkvSplitEpilogue {
+template <int DT> struct QkvSplitEpilogue : StoreThrough {
     typedef typename Elem<DT>::type T;
     static constexpr bool kRowStats = false;
     const float *bias;
@@ -294,7 +302,7 @@ template <int DT> struct QkvSplitEpilogue {
     __device__ __forceinline__ bool direct(int n0) const { return n0 >= 2 * H; }
     static constexpr int kColArrays = 1;  // bias
     __device__ __forceinline__ float col_src(int, int n) const { return bias ? bias[n] : 0.f; }
-    __device__ __forceinline__ void store8(int m, int n, const float (&acc)[8], const float *cl, int) const {
+    __device__ __forceinline__ void store8(int m, int n, const float (&acc)[8], const float *cl, int, const u32x4 *) const {
         float v[8];
 #pragma unroll
         for (int t = 0; t < 8; ++t)
@@ -314,13 +322,13 @@ template <int DT> struct QkvSplitEpilogue {
             u32x4 *cp = reinterpret_cast<u32x4 *>(qk + (size_t)m * 2 * H + n);
 #pragma unroll
             for (int q = 0; q < NV; ++q)
-                store_out16(&cp[q], packed[q]);
+                store_out16(through, &cp[q], packed[q]);
         } else {
             int c = n - 2 * H, b = m / S, s_ = key_slot(m - b * S, vt_sh);
             T *dst = vt + (((size_t)b * heads + (c >> 6)) * 64 + (c & 63)) * S + s_;
 #pragma unroll
             for (int t = 0; t < 8; ++t)
-                Elem<DT>::st_out(dst + (size_t)t * S, v[t]);
+                Elem<DT>::st_out(through, dst + (size_t)t * S, v[t]);
         }
     }
 };
@@ -376,7 +384,7 @@ __device__ __forceinline__ unsigned elem_offset24(int m, unsigned ld, int n) {
 
 // SUMS: 0 = the statistics come from the A fragments; else the most row-sum blocks the kernel is handed (12 or 24: that
 // many register pairs hold them while they are in flight)
-template <int DT, int SUMS = 0> struct LnFloatEpilogue {
+template <int DT, int SUMS = 0> struct LnFloatEpilogue : StoreThrough {
     typedef typename Elem<DT>::type T;
     static constexpr bool kRowStats = true;
     static constexpr bool kTakesRowSums = SUMS > 0;
@@ -393,8 +401,13 @@ template <int DT, int SUMS = 0> struct LnFloatEpilogue {
     __device__ __forceinline__ bool direct(int) const { return false; }
     static constexpr int kColArrays = 2;  // colsum, b'
     __device__ __forceinline__ float col_src(int k, int n) const { return k == 0 ? ln.colsum[n] : bias[n]; }
-    // st = {rstd, mean} of row m; cl = the item's eight columns of the two arrays in LDS, cs apart
-    __device__ __forceinline__ void store8(int m, int n, const float (&acc)[8], float2 st, const float *cl, int cs) const {
+    static constexpr int kAheadVecs = 8 * sizeof(T) / 16;
+    __device__ __forceinline__ const void *ahead_src(int m, int n) const {
+        return (flags & TNN_ROCM_EPI_RESIDUAL) ? residual + elem_offset24(m, (unsigned)ldc, n) : nullptr;
+    }
+    // st = {rstd, mean} of row m; cl = the item's eight columns of the two arrays in LDS, cs apart; ahead as in FloatEpilogue
+    __device__ __forceinline__ void store8(int m, int n, const float (&acc)[8], float2 st, const float *cl, int cs,
+                                           const u32x4 *ahead) const {
         float4 g0 = *reinterpret_cast<const float4 *>(cl), g1 = *reinterpret_cast<const float4 *>(cl + 4);
         float4 b0 = *reinterpret_cast<const float4 *>(cl + cs), b1 = *reinterpret_cast<const float4 *>(cl + cs + 4);
         const float g[8] = {g0.x, g0.y, g0.z, g0.w, g1.x, g1.y, g1.z, g1.w};
@@ -417,7 +430,7 @@ template <int DT, int SUMS = 0> struct LnFloatEpilogue {
             const u32x4 *rp = reinterpret_cast<const u32x4 *>(residual + elem_offset24(m, (unsigned)ldc, n));
 #pragma unroll
             for (int q = 0; q < NV; ++q)
-                packed[q] = rp[q];
+                packed[q] = ahead ? ahead[q] : rp[q];
             float w[8];
 #pragma unroll
             for (int t = 0; t < 8; ++t)
@@ -437,12 +450,12 @@ template <int DT, int SUMS = 0> struct LnFloatEpilogue {
         u32x4 *cp = reinterpret_cast<u32x4 *>(C + elem_offset24(m, (unsigned)ldc, n));
 #pragma unroll
         for (int q = 0; q < NV; ++q)
-            store_out16(&cp[q], packed[q]);
+            store_out16(through, &cp[q], packed[q]);
     }
 };
 
 // QKV projection of LayerNorm(t): QkvSplitEpilogue's layout with the folded-LayerNorm correction on the accumulators
-template <int DT, int SUMS = 0> struct LnQkvSplitEpilogue {
+template <int DT, int SUMS = 0> struct LnQkvSplitEpilogue : StoreThrough {
     typedef typename Elem<DT>::type T;
     static constexpr bool kRowStats = true;
     static constexpr bool kTakesRowSums = SUMS > 0;
@@ -459,7 +472,8 @@ template <int DT, int SUMS = 0> struct LnQkvSplitEpilogue {
     __device__ __forceinline__ bool direct(int n0) const { return n0 >= 2 * H; }
     static constexpr int kColArrays = 2;  // colsum, b'
     __device__ __forceinline__ float col_src(int k, int n) const { return k == 0 ? ln.colsum[n] : bias[n]; }
-    __device__ __forceinline__ void store8(int m, int n, const float (&acc)[8], float2 st, const float *cl, int cs) const {
+    __device__ __forceinline__ void store8(int m, int n, const float (&acc)[8], float2 st, const float *cl, int cs,
+                                           const u32x4 *) const {
         float4 g0 = *reinterpret_cast<const float4 *>(cl), g1 = *reinterpret_cast<const float4 *>(cl + 4);
         float4 b0 = *reinterpret_cast<const float4 *>(cl + cs), b1 = *reinterpret_cast<const float4 *>(cl + cs + 4);
         const float g[8] = {g0.x, g0.y, g0.z, g0.w, g1.x, g1.y, g1.z, g1.w};
@@ -478,14 +492,14 @@ template <int DT, int SUMS = 0> struct LnQkvSplitEpilogue {
             u32x4 *cp = reinterpret_cast<u32x4 *>(qk + elem_offset24(m, 2u * (unsigned)H, n));
 #pragma unroll
             for (int q = 0; q < NV; ++q)
-                store_out16(&cp[q], packed[q]);
+                store_out16(through, &cp[q], packed[q]);
         } else {
             // B * S * 3H < 2^31 is checked at launch: 32-bit offsets throughout
             int c = n - 2 * H, bb = m / S, s_ = key_slot(m - bb * S, vt_sh);
             T *dst = vt + (unsigned)(((bb * heads + (c >> 6)) * 64 + (c & 63)) * S + s_);
 #pragma unroll
             for (int t = 0; t < 8; ++t)
-                Elem<DT>::st_out(dst + (unsigned)(t * S), v[t]);
+                Elem<DT>::st_out(through, dst + (unsigned)(t * S), v[t]);
         }
     }
 };
@@ -494,7 +508,7 @@ template <int DT, int SUMS = 0> struct LnQkvSplitEpilogue {
 // (LnFold::stats): C = act(x W^T + b) + ((t - mean) * rstd * gamma + beta).  The normalised tensor is rebuilt from t in
 // registers, in the LayerNorm kernel's half-precision form x * rstd * gamma + (beta - mean * rstd * gamma), and never
 // stored.  N is the normalised width.
-template <int DT, bool SUMS = false> struct LnResidualEpilogue {
+template <int DT, bool SUMS = false> struct LnResidualEpilogue : StoreThrough {
     typedef typename Elem<DT>::type T;
     static constexpr bool kRowStats = false;
     static constexpr bool kEmitsRowSums = SUMS;
@@ -526,11 +540,14 @@ template <int DT, bool SUMS = false> struct LnResidualEpilogue {
         return k == 0 ? ((flags & TNN_ROCM_EPI_BIAS) ? bias[n] : 0.f) : k == 1 ? gamma[n] : beta[n];
     }
     __device__ __forceinline__ float2 row_src(int m) const { return st[m]; }
-    // cl = the item's eight columns of the three arrays in LDS, cs apart; s = {rstd, mean} of row m
-    __device__ __forceinline__ float2 store8(int m, int n, const float (&acc)[8], const float *cl, int cs, float2 s) const {
+    static constexpr int kAheadVecs = 1;
+    __device__ __forceinline__ const void *ahead_src(int m, int n) const { return t + elem_offset24(m, (unsigned)ldc, n); }
+    // cl = the item's eight columns of the three arrays in LDS, cs apart; s = {rstd, mean} of row m; ahead as in FloatEpilogue
+    __device__ __forceinline__ float2 store8(int m, int n, const float (&acc)[8], const float *cl, int cs, float2 s,
+                                             const u32x4 *ahead) const {
         static_assert(sizeof(T) == 2, "half-precision blobs only");
         const unsigned off = elem_offset24(m, (unsigned)ldc, n);
-        u32x4 packed = *reinterpret_cast<const u32x4 *>(t + off);
+        u32x4 packed = ahead ? *ahead : *reinterpret_cast<const u32x4 *>(t + off);
         float v[8];
         {
             float4 b0 = *reinterpret_cast<const float4 *>(cl), b1 = *reinterpret_cast<const float4 *>(cl + 4);
@@ -554,7 +571,7 @@ template <int DT, bool SUMS = false> struct LnResidualEpilogue {
 #pragma unroll
         for (int q = 0; q < 8; ++q)
             Elem<DT>::st(&pe[q], v[q]);
-        store_out16(C + off, packed);
+        store_out16(through, C + off, packed);
         float2 sums = make_float2(0.f, 0.f);
         if constexpr (SUMS) {  // of the values as stored (rounded to the blob type): what the next GEMM reads
             ln_accumulate<DT>(__builtin_bit_cast(uint4, packed), sums.x, sums.y);
@@ -563,7 +580,7 @@ template <int DT, bool SUMS = false> struct LnResidualEpilogue {
     }
 };
 
-struct Int8Epilogue {
+struct Int8Epilogue : StoreThrough {
     static constexpr bool kRowStats = false;
     // optional 256-entry table applied to the requantised value (index q + 128): an int8 -> int8 function that
     // followed the layer (dequantise, GELU, quantise) folded into this epilogue.  The tiled kernel keeps a copy in LDS.
@@ -621,8 +638,13 @@ struct Int8Epilogue {
     __device__ __forceinline__ float col_src(int k, int n) const {
         return k == 0 ? (bias ? __int_as_float(bias[n]) : 0.f) : (scale ? scale[n] : 0.f);
     }
-    // cl = the item's eight columns of the two arrays in LDS, cs apart
-    __device__ __forceinline__ void store8(int m, int n, const int (&acc)[8], const int8_t *lut_lds, const float *cl, int cs) const {
+    static constexpr int kAheadVecs = 1;  // a half residual; an fp32 one is read in its place
+    __device__ __forceinline__ const void *ahead_src(int m, int n) const {
+        return out_f && residual && out_f_dtype != TNN_ROCM_F32 ? (const half_t *)residual + (size_t)m * ldo + n : nullptr;
+    }
+    // cl = the item's eight columns of the two arrays in LDS, cs apart; ahead as in FloatEpilogue
+    __device__ __forceinline__ void store8(int m, int n, const int (&acc)[8], const int8_t *lut_lds, const float *cl, int cs,
+                                           const u32x4 *ahead) const {
         int a[8];
 #pragma unroll
         for (int t = 0; t < 8; ++t)
@@ -655,7 +677,7 @@ struct Int8Epilogue {
                     q[t] = lut_lds[(int)q[t] + 128];
             }
             if (out)
-                store_out8(out + o, *reinterpret_cast<const store_u32x2 *>(q));
+                store_out8(through, out + o, *reinterpret_cast<const store_u32x2 *>(q));
             if (out_f) {
                 float d[8];
 #pragma unroll
@@ -670,14 +692,14 @@ struct Int8Epilogue {
                         d[6] = __fadd_rn(d[6], r1.z), d[7] = __fadd_rn(d[7], r1.w);
                     }
                     float4 *fp = reinterpret_cast<float4 *>((float *)out_f + o);
-                    store_out16(fp, store_u32x4{__float_as_uint(d[0]), __float_as_uint(d[1]), __float_as_uint(d[2]),
+                    store_out16(through, fp, store_u32x4{__float_as_uint(d[0]), __float_as_uint(d[1]), __float_as_uint(d[2]),
                                                 __float_as_uint(d[3])});
-                    store_out16(fp + 1, store_u32x4{__float_as_uint(d[4]), __float_as_uint(d[5]), __float_as_uint(d[6]),
+                    store_out16(through, fp + 1, store_u32x4{__float_as_uint(d[4]), __float_as_uint(d[5]), __float_as_uint(d[6]),
                                                     __float_as_uint(d[7])});
                 } else {
                     half_t h[8];
                     if (residual) {
-                        *reinterpret_cast<u32x4 *>(h) = *reinterpret_cast<const u32x4 *>((const half_t *)residual + o);
+                        *reinterpret_cast<u32x4 *>(h) = ahead ? *ahead : *reinterpret_cast<const u32x4 *>((const half_t *)residual + o);
 #pragma unroll
                         for (int t = 0; t < 8; ++t)
                             d[t] = __fadd_rn(d[t], (float)h[t]);
@@ -685,7 +707,7 @@ struct Int8Epilogue {
 #pragma unroll
                     for (int t = 0; t < 8; ++t)
                         h[t] = (half_t)d[t];
-                    store_out16((half_t *)out_f + o, *reinterpret_cast<const u32x4 *>(h));
+                    store_out16(through, (half_t *)out_f + o, *reinterpret_cast<const u32x4 *>(h));
                 }
             }
         }
@@ -696,7 +718,7 @@ struct Int8Epilogue {
 // formed in registers (requantisation with scale[n] = w_scale[n] / o_scale of the column's section) and written
 // already dequantised (q * dequant[n], the value the following Reformat layer produces) in the layout of
 // QkvSplitEpilogue: columns [0,2H) -> qk[T,2H]; columns [2H,3H) -> V^T[b][head][d][s].
-template <int DT> struct Int8QkvSplitEpilogue {
+template <int DT> struct Int8QkvSplitEpilogue : StoreThrough {
     typedef typename Elem<DT>::type T;
     static constexpr bool kRowStats = false;
     const int32_t *bias;
@@ -733,7 +755,7 @@ template <int DT> struct Int8QkvSplitEpilogue {
     __device__ __forceinline__ float col_src(int k, int n) const {
         return k == 0 ? (bias ? __int_as_float(bias[n]) : 0.f) : k == 1 ? scale[n] : dequant[n];
     }
-    __device__ __forceinline__ void store8(int m, int n, const int (&acc)[8], const float *cl, int cs) const {
+    __device__ __forceinline__ void store8(int m, int n, const int (&acc)[8], const float *cl, int cs, const u32x4 *) const {
         // the item's eight columns of the three arrays, from LDS
         const i32x4 b0 = *reinterpret_cast<const i32x4 *>(cl), b1 = *reinterpret_cast<const i32x4 *>(cl + 4);
         const float4 s0 = *reinterpret_cast<const float4 *>(cl + cs), s1 = *reinterpret_cast<const float4 *>(cl + cs + 4);
@@ -757,13 +779,13 @@ template <int DT> struct Int8QkvSplitEpilogue {
             u32x4 *cp = reinterpret_cast<u32x4 *>(qk + (size_t)m * 2 * H + n);
 #pragma unroll
             for (int q = 0; q < NV; ++q)
-                store_out16(&cp[q], packed[q]);
+                store_out16(through, &cp[q], packed[q]);
         } else {
             int c = n - 2 * H, b = m / S, s_ = key_slot(m - b * S, vt_sh);
             T *dst = vt + (((size_t)b * heads + (c >> 6)) * 64 + (c & 63)) * S + s_;
 #pragma unroll
             for (int t = 0; t < 8; ++t)
-                Elem<DT>::st_out(dst + (size_t)t * S, v[t]);
+                Elem<DT>::st_out(through, dst + (size_t)t * S, v[t]);
         }
     }
 };
@@ -1038,6 +1060,11 @@ template <typename CFG, typename Epi> struct EpiLds {
 // 15:14, expcnt 6:4 and lgkmcnt 11:8 left at their maxima)
 #define TR_WAIT_VMCNT(n) __builtin_amdgcn_s_waitcnt((((n)&0xF) | ((((n) >> 4) & 3) << 14) | (0x7 << 4) | (0xF << 8)))
 
+struct TileOrder {
+    int group_m;
+    FixedDivisor group, rows, last_rows;  // tiles of a group; tile rows of a group; tile rows of the last, smaller group
+};
+
 __device__ __forceinline__ float plain_dot(const float *a, const float *b, int k) {
     float sum = 0.f;
     for (int i = 0; i < k; ++i)
@@ -1049,7 +1076,7 @@ template <int DT, typename CFG, typename Epi>
 __global__ void __launch_bounds__(CFG::NT)
     gemm_nk_tiled_kernel(const typename GemmTraits<DT>::elem *__restrict__ A,
                          const typename GemmTraits<DT>::elem *__restrict__ B, int M, int N, int K, long lda, long ldb,
-                         int tiles_m, int tiles_n, int group_m, Epi epi) {
+                         int tiles_m, int tiles_n, TileOrder order, Epi epi) {
     typedef typename GemmTraits<DT>::elem T;
     typedef typename GemmTraits<DT>::acc Acc;
     constexpr int TM = CFG::TM, TN = CFG::TN, WGN = CFG::WGN, WGK = CFG::WGK, SLAB = CFG::SLAB;
@@ -1076,18 +1103,71 @@ __global__ void __launch_bounds__(CFG::NT)
     // compact block of the tile grid: their A and W panels fit that L2 and are fetched from HBM once, instead of
     // the whole W panel streaming through every L2 once per tile row.
     TR_TL(0);  // entry
+    touch_kernel_args<64 + sizeof(TileOrder) + sizeof(Epi)>();
     const int n_tiles = tiles_m * tiles_n;
     const int per_xcd = (n_tiles + 7) >> 3;
     const int vid     = (int)(blockIdx.x & 7) * per_xcd + (int)(blockIdx.x >> 3);
+    const int grp      = order.group.quotient(vid);
+    const int first_m  = grp * order.group_m;
+    const bool last_g  = tiles_m - first_m < order.group_m;
+    const int rows_g   = last_g ? tiles_m - first_m : order.group_m;
+    const int in_grp   = vid - grp * order.group_m * tiles_n;
+    const int col_g    = last_g ? order.last_rows.quotient(in_grp) : order.rows.quotient(in_grp);
+    const int m0       = (first_m + in_grp - col_g * rows_g) * BM;
+    const int n0       = col_g * BN;
     if (vid >= n_tiles)
         return;  // the grid is padded to a multiple of 8; whole workgroups leave before any barrier
-    const int group_sz = group_m * tiles_n;
-    const int grp      = vid / group_sz;
-    const int first_m  = grp * group_m;
-    const int rows_g   = tiles_m - first_m < group_m ? tiles_m - first_m : group_m;
-    const int in_grp   = vid - grp * group_sz;
-    const int m0       = (first_m + in_grp % rows_g) * BM;
-    const int n0       = (in_grp / rows_g) * BN;
+
+    // ---- what the epilogue reads, requested before the first slab where a thread has one item and registers to spare: behind
+    // the main loop the same loads are two latencies one after the other (columns and row pairs, then the residual), 0.4 us
+    // of a launch of 4
+    constexpr int CW    = TN * 32;       // columns per wave
+    constexpr int CPR   = CW / 8;        // 8-column pieces per staged row
+    constexpr int POS   = CFG::NW / WGK;  // wave positions (wm, wn) in the tile
+    constexpr int ITEMS = POS * 32 * CPR;
+    constexpr bool EARLY = TM == 1 && ITEMS <= NT && CFG::NSTAGE > 0;
+    const bool by_rows   = epi.direct(n0);
+    // row and first column (inside the tile) of an item of the first 32-row group of every wave position
+    auto item_at = [&](int item, int *row, int *col) __attribute__((always_inline)) {
+        const int c8  = by_rows ? ((item >> 5) % CPR) * 8 : (item % CPR) * 8;
+        const int r   = by_rows ? (item & 31) : (item / CPR) % 32;
+        const int pos = item / (CPR * 32);
+        *row          = (pos / WGN) * TM * 32 + r;
+        *col          = (pos % WGN) * CW + c8;
+    };
+    constexpr int COLQ = (ColArrays<Epi>::value * BN + NT - 1) / NT;
+    float early_col[COLQ > 0 ? COLQ : 1];
+    float2 early_row = make_float2(0.f, 0.f);
+    constexpr int AHEAD = EARLY ? AheadVecs<Epi>::value : 0;
+    u32x4 ahead_vec[AHEAD > 0 ? AHEAD : 1];
+    auto request_columns = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int q = 0; q < COLQ; ++q) {
+            // clamped, not guarded: what lies outside is never used, and a branch costs more than the load
+            constexpr int LAST = ColArrays<Epi>::value * BN - 1;
+            const int e  = q * NT + tid < LAST ? q * NT + tid : LAST, n = n0 + e % BN;
+            early_col[q] = epi.col_src(e / BN, n < N ? n : N - 1);
+        }
+        if constexpr (RowIn<Epi>::value)
+            early_row = epi.row_src(m0 + tid % BM < M ? m0 + tid % BM : M - 1);
+    };
+    if constexpr (EARLY) {
+        if constexpr (ColArrays<Epi>::value > 0)
+            request_columns();
+        if constexpr (AHEAD > 0) {
+            int row = 0, col = 0;
+            item_at(tid % ITEMS, &row, &col);
+            const int m = m0 + row < M ? m0 + row : M - 1, n = n0 + col + 8 <= N ? n0 + col : N - 8;
+            if (N >= 8) {
+                const u32x4 *src = reinterpret_cast<const u32x4 *>(epi.ahead_src(m, n));
+                if (src) {
+#pragma unroll
+                    for (int q = 0; q < AHEAD; ++q)
+                        ahead_vec[q] = src[q];
+                }
+            }
+        }
+    }
 
     Acc acc[TM][TN];
 #pragma unroll
@@ -1624,15 +1704,10 @@ __global__ void __launch_bounds__(CFG::NT)
     // buffers are free after the main loop); the workgroup then walks the staged rows with eight columns per
     // thread, adds the WGK partial sums and applies the epilogue, so a store instruction covers whole lines of C
     // and bias/residual are read in the same coalesced shape.
-    constexpr int CW   = TN * 32;       // columns per wave
     constexpr int SSTR = CFG::SSTR;     // staged row stride in 32-bit words (16-byte pad spreads the b128 banks)
-    constexpr int CPR  = CW / 8;        // 8-column pieces per staged row
-    constexpr int POS  = CFG::NW / WGK;  // wave positions (wm, wn) in the tile
-    constexpr int ITEMS = POS * 32 * CPR;
     typedef AccT acc4 __attribute__((ext_vector_type(4)));
     AccT *const stage_all = reinterpret_cast<AccT *>(lds_dyn);
     AccT *const stage_me  = stage_all + wave * (32 * SSTR);  // wave = (wm*WGN + wn)*WGK + wk
-    const bool by_rows = epi.direct(n0);
     const int tid_piece = tid % CPR, tid_rowpos = tid / CPR;
     __syncthreads();  // every wave is done reading the slabs
     TR_TL(2);         // main loop done
@@ -1650,24 +1725,21 @@ __global__ void __launch_bounds__(CFG::NT)
     float *const col_lds        = reinterpret_cast<float *>(lds_dyn + EpiLds<CFG, Epi>::col_offset);
     const float2 *const row_lds = reinterpret_cast<const float2 *>(lds_dyn + EpiLds<CFG, Epi>::row_offset);
     if constexpr (ColArrays<Epi>::value > 0) {
+        if constexpr (!EARLY)
+            request_columns();
 #pragma unroll
-        for (int q = 0; q < (ColArrays<Epi>::value * BN + NT - 1) / NT; ++q) {
-            const int e = q * NT + tid;
-            if (e < ColArrays<Epi>::value * BN) {
-                const int c = e % BN;
-                col_lds[e]  = n0 + c < N ? epi.col_src(e / BN, n0 + c) : 0.f;
-            }
-        }
+        for (int q = 0; q < COLQ; ++q)
+            if (q * NT + tid < ColArrays<Epi>::value * BN)
+                col_lds[q * NT + tid] = early_col[q];
     }
     if constexpr (RowIn<Epi>::value) {
         if (tid < BM)
-            reinterpret_cast<float2 *>(lds_dyn + EpiLds<CFG, Epi>::row_offset)[tid] =
-                m0 + tid < M ? epi.row_src(m0 + tid) : make_float2(0.f, 0.f);
+            reinterpret_cast<float2 *>(lds_dyn + EpiLds<CFG, Epi>::row_offset)[tid] = early_row;
     }
     if constexpr (Epi::kRowStats && TakesRowSums<Epi>::value) {
         // {rstd, mean} were parked in LDS before the main loop (the barrier above orders that write); hand them on
         if (epi.ln.stats && n0 == 0 && tid < BM && m0 + tid < M)
-            store_out8(&epi.ln.stats[m0 + tid], row_st[tid]);
+            store_out8(epi.through, &epi.ln.stats[m0 + tid], row_st[tid]);
     }
     if constexpr (Epi::kRowStats && !TakesRowSums<Epi>::value) {
         static_assert(CFG::NSTAGE > 0, "LayerNorm-folding epilogues run on the direct-to-LDS pipeline");
@@ -1690,7 +1762,7 @@ __global__ void __launch_bounds__(CFG::NT)
             const float2 st   = make_float2((float)(1.0 / sqrt(var + (double)epi.ln.eps)), (float)mean);
             row_st[tid]       = st;
             if (epi.ln.stats && n0 == 0 && m0 + tid < M)  // every tile column holds them; the first one hands them on
-                store_out8(&epi.ln.stats[m0 + tid], st);
+                store_out8(epi.through, &epi.ln.stats[m0 + tid], st);
         }
         // row_st is read after the first staging barrier below
     }
@@ -1778,10 +1850,11 @@ __global__ void __launch_bounds__(CFG::NT)
                 }
             }
             const int nl = (pos % WGN) * CW + c8;  // column inside the tile
+            const u32x4 *const ahead = AHEAD > 0 ? ahead_vec : nullptr;
             if constexpr (Epi::kRowStats) {
                 if (m < M && n + 7 < N) {  // N is a multiple of 8 for these epilogues (checked at launch)
                     AccT v[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-                    epi.store8(m, n, v, row_st[m - m0], col_lds + nl, BN);
+                    epi.store8(m, n, v, row_st[m - m0], col_lds + nl, BN, ahead);
                 }
             } else if constexpr (EmitsRowSums<Epi>::value) {
                 // N is a multiple of 8 for these epilogues (checked at launch); every item leaves its eight columns'
@@ -1789,7 +1862,7 @@ __global__ void __launch_bounds__(CFG::NT)
                 float2 sm = make_float2(0.f, 0.f);
                 if (m < M && n + 7 < N) {
                     AccT v[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-                    sm = epi.store8(m, n, v, col_lds + nl, BN, row_lds[m - m0]);
+                    sm = epi.store8(m, n, v, col_lds + nl, BN, row_lds[m - m0], ahead);
                 }
                 reinterpret_cast<float2 *>(lds_dyn + CFG::sums_offset)[(((pos / WGN) * TM + i) * 32 + row) * (BN / 8) +
                                                                      ((pos % WGN) * CW + c8) / 8] = sm;
@@ -1797,11 +1870,11 @@ __global__ void __launch_bounds__(CFG::NT)
                 AccT v[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
                 if (n + 7 < N) {
                     if constexpr (std::is_same<Epi, Int8Epilogue>::value)
-                        epi.store8(m, n, v, epi.lut ? lut_lds : nullptr, col_lds + nl, BN);
+                        epi.store8(m, n, v, epi.lut ? lut_lds : nullptr, col_lds + nl, BN, ahead);
                     else if constexpr (RowIn<Epi>::value)
-                        (void)epi.store8(m, n, v, col_lds + nl, BN, row_lds[m - m0]);
+                        (void)epi.store8(m, n, v, col_lds + nl, BN, row_lds[m - m0], ahead);
                     else if constexpr (ColArrays<Epi>::value > 0)
-                        epi.store8(m, n, v, col_lds + nl, BN);
+                        epi.store8(m, n, v, col_lds + nl, BN, ahead);
                     else
                         epi.store8(m, n, v);
                 } else {
@@ -1826,7 +1899,7 @@ __global__ void __launch_bounds__(CFG::NT)
 #pragma unroll
             for (int q = 0; q < BN / 8; ++q)
                 s1 += part[q].x, s2 += part[q].y;
-            store_out8(&epi.row_sums[(size_t)(n0 / BN) * M + m0 + tid], make_float2(s1, s2));
+            store_out8(epi.through, &epi.row_sums[(size_t)(n0 / BN) * M + m0 + tid], make_float2(s1, s2));
         }
     }
     if constexpr (Epi::kRowStats) {
@@ -1913,10 +1986,15 @@ int launch_tiled(hipStream_t s, const void *A, const void *B, int M, int N, int 
         while ((long)(group_m + 1) * (group_m + 1) <= resident)
             ++group_m;
     group_m = group_m > tiles_m ? tiles_m : group_m;
+    TileOrder order;
+    order.group_m   = group_m;
+    order.group     = FixedDivisor::of((uint32_t)(group_m * tiles_n));
+    order.rows      = FixedDivisor::of((uint32_t)group_m);
+    order.last_rows = FixedDivisor::of((uint32_t)(tiles_m % group_m));
     unsigned grid = (unsigned)(((tiles_m * tiles_n + 7) / 8) * 8);
     t_last_tiles_n = tiles_n;
     hipLaunchKernelGGL(kern, dim3(grid), dim3(CFG::NT), lds, s, (const T *)A, (const T *)B, M, N, K, lda, ldb, tiles_m, tiles_n,
-                       group_m, epi);
+                       order, epi);
     TR_CHECK_LAUNCH();
     return 0;
 }

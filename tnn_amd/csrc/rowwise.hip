@@ -56,7 +56,7 @@ __global__ void __launch_bounds__(kBlock) layernorm_kernel(const typename Elem<D
                                                            const float *__restrict__ beta,
                                                            typename Elem<DT>::type *__restrict__ y, int rows, int cols,
                                                            float eps, int8_t *__restrict__ out_q, float q_inv,
-                                                           EmbedRows emb) {
+                                                           EmbedRows emb, StoreThrough mode) {
     typedef typename Elem<DT>::type T;
     constexpr int VEC = VECTOR ? (int)(16 / sizeof(T)) : 1;
     const int lane    = threadIdx.x & (LPR - 1);
@@ -170,7 +170,7 @@ __global__ void __launch_bounds__(kBlock) layernorm_kernel(const typename Elem<D
 #pragma unroll
                 for (int t = 0; t < VEC; ++t)
                     Elem<DT>::st(&e[t], o[t]);
-                store_out16(reinterpret_cast<uint4 *>(py) + vi, store_u32x4{raw.x, raw.y, raw.z, raw.w});
+                store_out16(mode.through, reinterpret_cast<uint4 *>(py) + vi, store_u32x4{raw.x, raw.y, raw.z, raw.w});
                 if (pq) {  // the VEC (4 or 8) quantised values of this lane leave as one 4- or 8-byte store
                     uint32_t w[2] = {0u, 0u};
 #pragma unroll
@@ -179,9 +179,9 @@ __global__ void __launch_bounds__(kBlock) layernorm_kernel(const typename Elem<D
                         w[t >> 2] |= (uint32_t)(uint8_t)q << (8 * (t & 3));
                     }
                     if (VEC == 8)
-                        store_out8(pq + (size_t)vi * VEC, store_u32x2{w[0], w[1]});
+                        store_out8(mode.through, pq + (size_t)vi * VEC, store_u32x2{w[0], w[1]});
                     else
-                        store_out4(pq + (size_t)vi * VEC, w[0]);
+                        store_out4(mode.through, pq + (size_t)vi * VEC, w[0]);
                 }
             } else {
                 T tmp;
@@ -265,7 +265,8 @@ int launch_layernorm(hipStream_t s, const void *x, const void *res, const float 
 #define TR_LN(LPR, NV)                                                                                                \
     hipLaunchKernelGGL((layernorm_kernel<DT, true, LPR, NV>),                                                         \
                        dim3((rows + kRowsPerBlk * (kWave / LPR) - 1) / (kRowsPerBlk * (kWave / LPR))), block, 0, s,   \
-                       (const T *)x, (const T *)res, gamma, beta, (T *)y, rows, cols, eps, out_q, q_inv, emb)
+                       (const T *)x, (const T *)res, gamma, beta, (T *)y, rows, cols, eps, out_q, q_inv, emb,     \
+                       StoreThrough())
         if (nv <= 64)
             TR_LN(32, 2);
         else if (nv <= 128)
@@ -277,7 +278,7 @@ int launch_layernorm(hipStream_t s, const void *x, const void *res, const float 
 #undef TR_LN
     } else if (cols <= kWave * kMaxVecPerLn) {
         hipLaunchKernelGGL((layernorm_kernel<DT, false, kWave, kMaxVecPerLn>), grid, block, 0, s, (const T *)x,
-                           (const T *)res, gamma, beta, (T *)y, rows, cols, eps, out_q, q_inv, emb);
+                           (const T *)res, gamma, beta, (T *)y, rows, cols, eps, out_q, q_inv, emb, StoreThrough());
     } else {
         hipLaunchKernelGGL((layernorm_long_kernel<DT>), grid, block, 0, s, (const T *)x, (const T *)res, gamma, beta,
                            (T *)y, rows, cols, eps, out_q, q_inv);
@@ -385,8 +386,6 @@ int launch_softmax(hipStream_t s, const void *x, void *y, int outer, int channel
 }  // namespace
 
 extern "C" {
-TR_DEFINE_STORE_THROUGH_SETTER(rowwise_set_store_through)
-
 int tnn_rocm_layernorm(void *stream, int dtype, const void *x, const void *residual, const float *gamma,
                        const float *beta, void *y, int rows, int cols, float eps, int8_t *out_q, float q_inv_scale) {
     TR_REQUIRE(rows >= 0 && cols >= 0, TNN_ROCM_ESHAPE, "layernorm: negative size");

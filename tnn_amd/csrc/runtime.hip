@@ -188,24 +188,8 @@ int tnn_rocm_event_record(void *event, void *stream) {
     return 0;
 }
 
-// every translation unit holds its own copy of the switch (common.h); they are set together (weak: a stand-alone
-// program may link this file with only some of the kernels)
-__attribute__((weak)) int gemm_f32_set_store_through(int on);
-__attribute__((weak)) int gemm_f16_set_store_through(int on);
-__attribute__((weak)) int gemm_f16_ln_set_store_through(int on);
-__attribute__((weak)) int gemm_bf16_set_store_through(int on);
-__attribute__((weak)) int gemm_bf16_ln_set_store_through(int on);
-__attribute__((weak)) int gemm_i8_set_store_through(int on);
-__attribute__((weak)) int attention_set_store_through(int on);
-__attribute__((weak)) int attention_f32_set_store_through(int on);
-__attribute__((weak)) int rowwise_set_store_through(int on);
 __attribute__((visibility("default"))) int tnn_rocm_debug_set_store_through(int on) {
-    on = on ? 1 : 0;
-    TR_CHECK_HIP(hipDeviceSynchronize());
-    int (*const setters[])(int) = {gemm_f32_set_store_through, gemm_f16_set_store_through, gemm_f16_ln_set_store_through, gemm_bf16_set_store_through, gemm_bf16_ln_set_store_through, gemm_i8_set_store_through, attention_set_store_through, attention_f32_set_store_through, rowwise_set_store_through};
-    for (auto set : setters)
-        if (set)
-            TR_CHECK_HIP((hipError_t)set(on));
+    g_store_through = on ? 1 : 0;
     return 0;
 }
 
