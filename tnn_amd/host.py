@@ -1,6 +1,7 @@
 """ctypes front-end of the C++ host (tnn_amd/lib/libtnn_rocm_host.so): an engine Instance on DEVICE_ROCM created
 from .tnnproto text + .tnnmodel bytes.  No fallback: a missing library or a failed call raises."""
 import ctypes as C
+import functools
 import math
 import os
 
@@ -74,6 +75,12 @@ _MAT_CODE = {np.dtype(np.float32): 0, np.dtype(np.int32): 1, np.dtype(np.int8): 
 
 class HostError(RuntimeError):
     pass
+
+
+@functools.lru_cache(maxsize=256)
+def _dims_array(shape):
+    """the C array of a shape: building one takes longer than the rest of an input's way through this module"""
+    return (C.c_int * max(len(shape), 1))(*shape)
 
 
 def _shape_args(input_shapes):
@@ -176,16 +183,17 @@ class RocmInstance:
         if a.dtype not in _MAT_CODE:
             raise TypeError("inputs are fp32 (NCHW_FLOAT), int32 (NC_INT32), int8 (RESERVED_INT8_TEST), float16 "
                             "(RESERVED_FP16_TEST) or uint16 holding bfloat16 bits (RESERVED_BFP16_TEST) host arrays")
-        dims = (C.c_int * max(a.ndim, 1))(*a.shape)
-        self._check(load().tnn_host_set_input(self._h, name.encode(), a.ctypes.data_as(C.c_void_p),
-                                              _MAT_CODE[a.dtype], dims, a.ndim), "SetInputMat")
+        rc = _lib.tnn_host_set_input(self._h, name.encode(), a.ctypes.data, _MAT_CODE[a.dtype], _dims_array(a.shape), a.ndim)
+        if rc != 0:
+            self._check(rc, "SetInputMat")
 
     def set_input_device(self, name, data_ptr, np_dtype, shape):
         """SetInputMat with a Mat in device memory (data_ptr: a device address holding `shape` elements of np_dtype, e.g. a
         torch tensor's data_ptr()); the memory must stay unchanged until the instance's stream has passed the copy"""
-        dims = (C.c_int * max(len(shape), 1))(*shape)
-        self._check(load().tnn_host_set_input_device(self._h, name.encode(), C.c_void_p(data_ptr), _MAT_CODE[np.dtype(np_dtype)],
-                                                     dims, len(shape)), "SetInputMat (device mat)")
+        rc = _lib.tnn_host_set_input_device(self._h, name.encode(), data_ptr, _MAT_CODE[np.dtype(np_dtype)], _dims_array(tuple(shape)),
+                                            len(shape))
+        if rc != 0:
+            self._check(rc, "SetInputMat (device mat)")
 
     def output_device(self, name, np_dtype):
         """GetOutputMat as a Mat in device memory the instance owns -> (device address, shape)"""
