@@ -1028,6 +1028,10 @@ template <int TM_, int TN_, int WGM_, int WGN_, int WGK_, int SLAB_, int NSTAGE_
     // not reach when that is large enough (dead by then), else behind everything
     static constexpr size_t sums_bytes  = (size_t)BM * BN;
     static constexpr size_t sums_offset = (slab_bytes >= stage_bytes + sums_bytes) ? stage_bytes : lds_bytes;
+    // ... unless there is no such part and a row of a wave's columns lies in eight neighbouring lanes: the lanes then add up
+    // the sums of each wave's columns among themselves (128 x 128: 16 KB of LDS would cost the CU's second workgroup)
+    static constexpr bool sums_by_lanes = TN_ == 2 && !(slab_bytes >= stage_bytes + sums_bytes);
+    static constexpr int sum_cols       = sums_by_lanes ? 32 * TN_ : BN;  // columns behind one pair of row sums
     static constexpr int NW = WGM * WGN * WGK, NT = 64 * NW;  // waves and threads per workgroup
     static_assert(NW == 4 || NW == 8, "four or eight waves per workgroup");
     static_assert(OWN_ || ((BM * (SLAB / 16)) % NT == 0 && (BN * (SLAB / 16)) % NT == 0), "slab must divide over the workgroup");
@@ -1049,7 +1053,7 @@ template <typename CFG, typename Epi> struct EpiLds {
     // without / with the row-sum side output (eight bytes per eight columns and row)
     static constexpr size_t plain     = base1;
     static constexpr size_t with_sums = CFG::sums_offset + CFG::sums_bytes > base1 ? CFG::sums_offset + CFG::sums_bytes : base1;
-    static constexpr size_t front      = EmitsRowSums<Epi>::value ? with_sums : plain;
+    static constexpr size_t front      = EmitsRowSums<Epi>::value && !CFG::sums_by_lanes ? with_sums : plain;
     static constexpr size_t col_offset = (front + 15) & ~(size_t)15;
     static constexpr size_t row_offset = col_offset + (size_t)ColArrays<Epi>::value * CFG::BN * 4;
     static constexpr size_t side_bytes = (size_t)ColArrays<Epi>::value * CFG::BN * 4 + (RowIn<Epi>::value ? (size_t)CFG::BM * 8 : 0);
@@ -1864,8 +1868,19 @@ __global__ void __launch_bounds__(CFG::NT)
                     AccT v[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
                     sm = epi.store8(m, n, v, col_lds + nl, BN, row_lds[m - m0], ahead);
                 }
-                reinterpret_cast<float2 *>(lds_dyn + CFG::sums_offset)[(((pos / WGN) * TM + i) * 32 + row) * (BN / 8) +
-                                                                     ((pos % WGN) * CW + c8) / 8] = sm;
+                if constexpr (CFG::sums_by_lanes) {
+                    static_assert(CPR == 8 && ITEMS % NT == 0, "eight lanes hold a row, and every lane has an item");
+#pragma unroll
+                    for (int o = 1; o < 8; o <<= 1) {
+                        sm.x += __shfl_xor(sm.x, o, 64);
+                        sm.y += __shfl_xor(sm.y, o, 64);
+                    }
+                    if (piece == 0 && m < M && n < N)
+                        store_out8(epi.through, &epi.row_sums[(size_t)(n / CFG::sum_cols) * M + m], sm);
+                } else {
+                    reinterpret_cast<float2 *>(lds_dyn + CFG::sums_offset)[(((pos / WGN) * TM + i) * 32 + row) * (BN / 8) +
+                                                                         ((pos % WGN) * CW + c8) / 8] = sm;
+                }
             } else if (m < M) {
                 AccT v[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
                 if (n + 7 < N) {
@@ -1889,7 +1904,7 @@ __global__ void __launch_bounds__(CFG::NT)
             __syncthreads();
     }
     TR_TL(3);  // C stored
-    if constexpr (EmitsRowSums<Epi>::value) {
+    if constexpr (EmitsRowSums<Epi>::value && !CFG::sums_by_lanes) {
         // this tile's share of every row's sum and sum of squares, added up in a fixed order, for the folding GEMM
         // that reads C next
         __syncthreads();
@@ -1943,7 +1958,7 @@ __global__ void __launch_bounds__(CFG::NT)
 // internal: the chosen tile shape does not leave row sums (no LDS, too many tile columns) or does not take them; the
 // caller launches the form without
 constexpr int kNotWithRowSums = -12345;
-thread_local int t_last_tiles_n = 0;  // tile columns of this thread's last tiled launch (the row-sum block count)
+thread_local int t_last_sum_blocks = 0;  // row-sum blocks of this thread's last tiled launch
 
 template <int DT, typename CFG, typename Epi>
 int launch_tiled(hipStream_t s, const void *A, const void *B, int M, int N, int K, long lda, long ldb, const Epi &epi) {
@@ -1951,9 +1966,10 @@ int launch_tiled(hipStream_t s, const void *A, const void *B, int M, int N, int 
     int tiles_m = (M + CFG::BM - 1) / CFG::BM, tiles_n = (N + CFG::BN - 1) / CFG::BN;
     typedef EpiLds<CFG, Epi> L;
     const size_t lds = L::total;
-    if (EmitsRowSums<Epi>::value && tiles_n > kMaxRowSumBlocks)
+    const int sum_blocks = (N + CFG::sum_cols - 1) / CFG::sum_cols;
+    if (EmitsRowSums<Epi>::value && sum_blocks > kMaxRowSumBlocks)
         return kNotWithRowSums;
-    if (EmitsRowSums<Epi>::value) {
+    if (EmitsRowSums<Epi>::value && !CFG::sums_by_lanes) {
         // the row sums are not taken at the price of a workgroup per CU (the plain form runs instead)
         const size_t without = L::plain + L::side_bytes + 16;
         const long cu = 160 * 1024;
@@ -1992,7 +2008,7 @@ int launch_tiled(hipStream_t s, const void *A, const void *B, int M, int N, int 
     order.rows      = FixedDivisor::of((uint32_t)group_m);
     order.last_rows = FixedDivisor::of((uint32_t)(tiles_m % group_m));
     unsigned grid = (unsigned)(((tiles_m * tiles_n + 7) / 8) * 8);
-    t_last_tiles_n = tiles_n;
+    t_last_sum_blocks = sum_blocks;
     hipLaunchKernelGGL(kern, dim3(grid), dim3(CFG::NT), lds, s, (const T *)A, (const T *)B, M, N, K, lda, ldb, tiles_m, tiles_n,
                        order, epi);
     TR_CHECK_LAUNCH();
@@ -2344,7 +2360,7 @@ int GemmTyped<DT>::residual_ln(hipStream_t s, const void *x, const void *w, cons
     if (row_sums && N <= 64 * kMaxRowSumBlocks) {
         const int rc = launch_residual_ln<DT, true>(s, x, w, bias, C, t, row_stats, gamma, beta, M, N, K, flags, row_sums);
         if (rc == 0)
-            *row_sum_blocks = t_last_tiles_n;
+            *row_sum_blocks = t_last_sum_blocks;
         if (rc != kNotWithRowSums)
             return rc;
     }
