@@ -162,6 +162,14 @@ TNN_ROCM_API int tnn_rocm_attention_vt_q8(void *stream, int dtype, const void *q
                                           long q_sb, long q_sh, long q_ss, long k_sb, long k_sh, long k_ss, long vt_sb,
                                           long vt_sh, long vt_sd, long o_sb, long o_sh, long o_ss, float scale,
                                           const float *mask, const int32_t *kv_len, int vt_key_order);
+/* The same through the kernels that stage K and V^T in LDS, whatever the size (the form above takes another kernel for few
+ * query blocks, which rounds its operands in another place).  For quantised nets: an int8 step of the context that falls the
+ * other way is a 127th of its range for every layer behind it, so their attention keeps one form at every size. */
+TNN_ROCM_API int tnn_rocm_attention_vt_q8_staged(void *stream, int dtype, const void *q, const void *k, const void *vt, void *out,
+                                          int8_t *out_q, float out_q_inv_scale, int B, int heads, int S, int head_dim,
+                                          long q_sb, long q_sh, long q_ss, long k_sb, long k_sh, long k_ss, long vt_sb,
+                                          long vt_sh, long vt_sd, long o_sb, long o_sh, long o_ss, float scale,
+                                          const float *mask, const int32_t *kv_len, int vt_key_order);
 
 /* The int8 GEMM above with a float consumer folded in: out_f = (float)q * dequant_scale (+ residual), where q is
  * the requantised int8 value of tnn_rocm_gemm_i8 (never written).  This is QuantizedInnerProduct -> Reformat

@@ -1313,14 +1313,12 @@ template <int DT, bool VT> __global__ void __launch_bounds__(256, 2) attention_s
 // block holds the whole sequence (the other kernels' 64 queries are then half empty).  us, fp16, 12 heads, before -> now:
 //   V^T        B1 S32 5.0 -> 4.0   B1 S128 6.0 -> 4.8   B1 S256 6.8 -> 5.5   B1 S512 9.1 -> 6.9   B2 S512 9.7 (this one: 10.3)
 //   row-major  B1 S197 8.2 -> 5.5   B5 S197 9.7 -> 7.1   B8 S384 18.3 -> 17.2   B16 S256 14.3 (this one: 15.9)
-// A launch with the quantised second output stays with the other kernels: the two forms round differently (within the type's
-// own rounding), and an int8 step that falls the other way is a 127th of the range for every layer behind it.
 constexpr long kShortBlocksVT = 256, kShortBlocksRows = 1200;
 
-template <bool VT> int launch_attention(hipStream_t s, int dtype, AttnParams p, int B, int heads, int S) {
+template <bool VT> int launch_attention(hipStream_t s, int dtype, AttnParams p, int B, int heads, int S, bool by_size = true) {
     const long blocks128 = (long)((S + 127) / 128) * heads * B, blocks32 = (long)((S + 31) / 32) * heads * B;
     const int mode = g_attention_dma;
-    const bool few = !p.oq && (S <= 32 || blocks32 <= (VT ? kShortBlocksVT : kShortBlocksRows));
+    const bool few = by_size && (S <= 32 || blocks32 <= (VT ? kShortBlocksVT : kShortBlocksRows));
     p.by_heads     = FixedDivisor::of((uint32_t)heads);
     // grid of the launch with BQ queries per block
     auto blocks_of = [&](int bq) {
@@ -1429,7 +1427,7 @@ int tnn_rocm_attention_vt(void *stream, int dtype, const void *q, const void *k,
                                     k_sh, k_ss, vt_sb, vt_sh, vt_sd, o_sb, o_sh, o_ss, scale, mask, kv_len, 0);
 }
 
-int tnn_rocm_attention_vt_q8(void *stream, int dtype, const void *q, const void *k, const void *vt, void *out,
+static int attention_vt(bool by_size, void *stream, int dtype, const void *q, const void *k, const void *vt, void *out,
                              int8_t *out_q, float out_q_inv_scale, int B, int heads, int S, int head_dim, long q_sb,
                              long q_sh, long q_ss, long k_sb, long k_sh, long k_ss, long vt_sb, long vt_sh, long vt_sd,
                              long o_sb, long o_sh, long o_ss, float scale, const float *mask, const int32_t *kv_len,
@@ -1473,7 +1471,27 @@ int tnn_rocm_attention_vt_q8(void *stream, int dtype, const void *q, const void 
     p.oq      = out_q;
     p.q_inv   = out_q_inv_scale;
     p.vt_perm = vt_key_order;
-    return launch_attention<true>((hipStream_t)stream, dtype, p, B, heads, S);
+    return launch_attention<true>((hipStream_t)stream, dtype, p, B, heads, S, by_size);
+}
+
+int tnn_rocm_attention_vt_q8(void *stream, int dtype, const void *q, const void *k, const void *vt, void *out,
+                             int8_t *out_q, float out_q_inv_scale, int B, int heads, int S, int head_dim, long q_sb,
+                             long q_sh, long q_ss, long k_sb, long k_sh, long k_ss, long vt_sb, long vt_sh, long vt_sd,
+                             long o_sb, long o_sh, long o_ss, float scale, const float *mask, const int32_t *kv_len,
+                             int vt_key_order) {
+    return attention_vt(true, stream, dtype, q, k, vt, out, out_q, out_q_inv_scale, B, heads, S, head_dim, q_sb, q_sh,
+                        q_ss, k_sb, k_sh, k_ss, vt_sb, vt_sh, vt_sd, o_sb, o_sh, o_ss, scale, mask, kv_len,
+                        vt_key_order);
+}
+
+int tnn_rocm_attention_vt_q8_staged(void *stream, int dtype, const void *q, const void *k, const void *vt, void *out,
+                             int8_t *out_q, float out_q_inv_scale, int B, int heads, int S, int head_dim, long q_sb,
+                             long q_sh, long q_ss, long k_sb, long k_sh, long k_ss, long vt_sb, long vt_sh, long vt_sd,
+                             long o_sb, long o_sh, long o_ss, float scale, const float *mask, const int32_t *kv_len,
+                             int vt_key_order) {
+    return attention_vt(false, stream, dtype, q, k, vt, out, out_q, out_q_inv_scale, B, heads, S, head_dim, q_sb,
+                        q_sh, q_ss, k_sb, k_sh, k_ss, vt_sb, vt_sh, vt_sd, o_sb, o_sh, o_ss, scale, mask, kv_len,
+                        vt_key_order);
 }
 
 __attribute__((visibility("default"))) int tnn_rocm_debug_set_attention_dma(int on) {

@@ -1802,7 +1802,7 @@ public:
                                                  (const int32_t *)bias_, (const float *)scale_, (const float *)dequant_, qkv,
                                                  vt, B_, seq_, p->heads, K_, vt_order));
             const long row = 2L * H_;
-            ROCM_CALL(tnn_rocm_attention_vt_q8(Stream(), (int)dt, base, base + (size_t)H_ * es, vt, Ptr(outputs[0]), out_q,
+            ROCM_CALL(tnn_rocm_attention_vt_q8_staged(Stream(), (int)dt, base, base + (size_t)H_ * es, vt, Ptr(outputs[0]), out_q,
                                                out_q_inv, B_, p->heads, seq_, p->head_dim, (long)seq_ * row, d, row,
                                                (long)seq_ * row, d, row, (long)p->heads * 64 * seq_, 64L * seq_, (long)seq_,
                                                (long)seq_ * H_, d, (long)H_, p->scale, mask, kv, vt_order));
