@@ -5,7 +5,7 @@ import pytest
 
 import encoder_ref
 import orc
-from test_gpu_ops import rel_err, say, FP16_TOL, FP32_TOL, FP32_ASSERT
+from test_gpu_ops import rel_err, say, BF16_TOL, FP16_TOL, FP32_TOL, FP32_ASSERT
 
 torch = pytest.importorskip("torch")
 pytestmark = pytest.mark.gpu
@@ -698,6 +698,60 @@ def test_fp32_attention_group_equals_its_layers(B, S):
         alone = inst.output("last_hidden").reshape(b * s, -1)
         ref = encoder_ref.encoder(w, cfg, encoder_ref.embed(w, ids, seg, cfg.eps), b, s, mask)
         assert rel_err(got, alone) <= 3e-6 and rel_err(got, ref) <= FP32_ASSERT
+    inst.close()
+
+
+@pytest.mark.parametrize("precision", ["fp32", "fp16", "bf16"])
+def test_two_attention_masks_in_one_net(precision):
+    """Two layers, each with a padding mask of its own, made in the graph as Sub(1 - m) -> Mul(-10000) right in front of the
+    layer: the memory plan gives the second mask the buffer of the first one, whose last reader has passed by then.  Each
+    layer has to see its own mask: in Forward, layer by layer (ForwardWithCallback), and against the checker."""
+    host, tnnmodel, EncoderConfig, make_weights, _ = _mods()
+    say("host: two attention masks, " + precision)
+    cfg = EncoderConfig(2, 128, 2, 256)
+    B, S = 2, 48
+    w = make_weights(cfg, seed=61, bias_std=0.05, with_embeddings=False)
+    for lw in w["layers"]:  # an attention output that weighs as much as the residual beside it
+        lw["wv"], lw["wo"] = lw["wv"] * 4, lw["wo"] * 8
+    g = tnnmodel.encoder_graph(cfg, w, B, S, with_embeddings=False)
+    g.inputs = [i for i in g.inputs if i[0] != "attention_bias"]
+    layers = []
+    for t, n, i, o, pr in g.layers:
+        if n in ("l0_q_mm", "l1_q_mm"):
+            mk = "m" + n[1]
+            g.add_input(mk, [B, 1, 1, S])
+            g.res_eltwise(mk + "_inv", "Sub", np.array([1.0], np.float32))      # constant first: 1 - m
+            g.res_eltwise(mk + "_scale", "Mul", np.array([-10000.0], np.float32))
+            for b in ("_pad", "_bias"):
+                g._blob(mk + b)
+            layers += [("Sub", mk + "_inv", [mk], [mk + "_pad"], ["0"]), ("Mul", mk + "_scale", [mk + "_pad"], [mk + "_bias"], ["1"])]
+        layers.append((t, n, ["m" + n[1] + "_bias" if b == "attention_bias" else b for b in i], o, pr))
+    g.layers = layers
+    rng = np.random.default_rng(62)
+    x = rng.standard_normal((B, S, cfg.hidden)).astype(np.float32)
+    lens = [np.array([40, 9]), np.array([17, 48])]
+    keep = [(np.arange(S)[None, :] < n[:, None]).astype(np.float32) for n in lens]
+    inst = host.RocmInstance.from_graph(g, precision)
+    inst.set_input("hidden", x)
+    for k in (0, 1):
+        inst.set_input("m%d" % k, keep[k].reshape(B, 1, 1, S))
+    inst.forward()
+    got = inst.output("last_hidden").reshape(B * S, -1).copy()
+    inst.forward_with_callback(after=lambda name, typ, blobs: None)
+    alone = inst.output("last_hidden").reshape(B * S, -1)
+
+    def checker(masks):
+        y = x.reshape(B * S, -1)
+        for lw, m in zip(w["layers"], masks):
+            y = encoder_ref.encoder_layer(y, lw, B, S, cfg.heads, (1 - m) * np.float32(-10000.0), cfg.eps)
+        return y
+
+    ref = checker(keep)
+    tol = {"fp32": FP32_ASSERT, "fp16": FP16_TOL, "bf16": BF16_TOL}[precision]
+    err, err_alone = rel_err(got, ref), rel_err(got, alone)
+    say("  to the checker %.3g, to the layers one by one %.3g" % (err, err_alone))
+    assert rel_err(checker([keep[0], keep[0]]), ref) > 4 * tol  # the first mask twice would be seen
+    assert err <= tol and err_alone <= (3e-6 if precision == "fp32" else 0)
     inst.close()
 
 

@@ -77,8 +77,8 @@ Status RocmContext::OnInstanceForwardBegin() {
     return TNN_OK;
 }
 
-Status RocmContext::AttentionMask(const void *mask_blob, int mask_dtype, int B, int S, bool one_row, const float **mask_f32,
-                                  const int32_t **kv_len) {
+Status RocmContext::AttentionMask(const std::string &name, const void *mask_blob, int mask_dtype, int B, int S, bool one_row,
+                                  const float **mask_f32, const int32_t **kv_len) {
     auto &c = mask_cache_;
     if ((size_t)B * S > c.cap_mask || (size_t)B > c.cap_len || !c.kv_len) {
         ROCM_CALL(tnn_rocm_stream_sync(stream_));
@@ -97,13 +97,14 @@ Status RocmContext::AttentionMask(const void *mask_blob, int mask_dtype, int B, 
     // a dense fp32 mask is read where it lies; any other (half precision, or one row for all sequences) from the copy
     const bool in_place = mask_dtype == TNN_ROCM_F32 && !one_row;
     const float *m      = in_place ? (const float *)mask_blob : (const float *)c.mask_f32;
-    if (c.src != mask_blob || c.epoch != forward_epoch_) {
+    if (c.src != mask_blob || c.name != name || c.epoch != forward_epoch_) {
         // Keys after the last one whose additive mask lies within 1000 of the row's largest value contribute
         // exp(-1000 + score difference) == 0 in fp32 and are cut (a plain 0 / -10000 padding mask is flagged: the
         // attention kernel then works from the lengths alone); one launch, which also makes the fp32 copy.
         ROCM_CALL(tnn_rocm_mask_prepare_strided(stream_, mask_dtype, mask_blob, one_row ? 0L : (long)S,
                                                 in_place ? nullptr : (float *)c.mask_f32, (int32_t *)c.kv_len, B, S, -1000.0f));
         c.src   = mask_blob;
+        c.name  = name;
         c.epoch = forward_epoch_;
     }
     *mask_f32 = m;

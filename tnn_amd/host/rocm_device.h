@@ -73,10 +73,13 @@ public:
     // page-locked word kernels raise on a data error (e.g. Gather index out of range)
     int32_t *ErrorFlag() { return error_flag_; }
     // The padding mask is one blob shared by every attention layer of a forward pass: the first layer that asks
-    // derives its fp32 copy and the per-sequence key counts, later layers of the same forward reuse them.
-    // one_row: the blob holds S values that serve every sequence (an additive mask [1,1,1,S])
-    Status AttentionMask(const void *mask_blob, int mask_dtype, int B, int S, bool one_row, const float **mask_f32,
-                         const int32_t **kv_len);
+    // derives its fp32 copy and the per-sequence key counts, later layers of the same forward that read the same blob reuse
+    // them.  The blob is known by its name, which stands for one value per forward (the rewrites take an attention core only
+    // if nothing writes its mask after the core has begun); the address alone is not enough, since a second mask may lie
+    // where the first one lay, once that has had its last reader.  one_row: the blob holds S values that serve every sequence
+    // (an additive mask [1,1,1,S])
+    Status AttentionMask(const std::string &name, const void *mask_blob, int mask_dtype, int B, int S, bool one_row,
+                         const float **mask_f32, const int32_t **kv_len);
 
 private:
     int device_id_       = 0;
@@ -88,6 +91,7 @@ private:
     uint64_t forward_epoch_ = 0;
     uint64_t memory_epoch_  = 0;
     struct MaskEntry {
+        std::string name;
         const void *src = nullptr;
         uint64_t epoch  = 0;
         int B = 0, S = 0;

@@ -1777,8 +1777,8 @@ public:
         const int32_t *kv = nullptr;
         if (p->has_mask) {
             Blob *mb = In(inputs[1]);
-            RETURN_ON_NEQ(context_->AttentionMask(Ptr(mb), (int)mb->GetBlobDesc().data_type, B_, seq_, mask_one_row_, &mask, &kv),
-                          TNN_OK);
+            RETURN_ON_NEQ(context_->AttentionMask(mb->GetBlobDesc().name, Ptr(mb), (int)mb->GetBlobDesc().data_type, B_, seq_,
+                                                  mask_one_row_, &mask, &kv), TNN_OK);
         }
         const char *base = (const char *)qkv;
         const long d     = p->head_dim;
