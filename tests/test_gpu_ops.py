@@ -621,6 +621,38 @@ def test_gemm_fp32_split_shapes(code, M, N, K):
     assert (np.abs(got[fine] - exact[fine]) <= 2.0 ** -24 * 4 * np.sqrt(K) * size[fine]).all()
 
 
+@pytest.mark.parametrize("code", [0, 9111181, 9321140, 2331142, 2222221])
+def test_gemm_fp32_not_finite_costs_a_few_launches(code):
+    """An overflow upstream makes whole rows, or all, of an activation NaN: the product says so, and does not take orders of
+    magnitude longer for it (three to five times as long; the bound leaves room for a busy device)."""
+    from tnn_amd import capi
+    lib = capi.load()
+    say("gemm fp32 not finite, code %d" % code)
+    M, N, K = 384, 768, 3072
+    rng = np.random.default_rng(5)
+    fine = rng.standard_normal((M, K)).astype(np.float32)
+    w = dev(rng.standard_normal((N, K)).astype(np.float32))
+    rows, every = fine.copy(), np.full((M, K), np.nan, np.float32)
+    rows[7, 100], rows[200, 9] = np.nan, np.inf
+    took = []
+    lib.tnn_rocm_debug_set_gemm_config(code)
+    try:
+        for a, bad in ((fine, []), (rows, [7, 200]), (every, range(M))):
+            a = dev(a)
+            got = np.isfinite(host(ops().gemm(a, w, True)))
+            assert got.all(1).sum() == M - len(bad) and not got[list(bad)].any()
+            ev = [torch.cuda.Event(enable_timing=True) for _ in range(11)]
+            for e in ev:
+                e.record()
+                ops().gemm(a, w, True)
+            torch.cuda.synchronize()
+            took.append(min(ev[i].elapsed_time(ev[i + 1]) for i in range(10)))
+    finally:
+        lib.tnn_rocm_debug_set_gemm_config(0)
+    say("  us: finite %.1f, two rows not finite %.1f, all NaN %.1f" % tuple(1e3 * t for t in took))
+    assert max(took) <= 20 * took[0]
+
+
 # ---- int8 GEMM: bit-exact accumulators and outputs -----------------------------------------------
 @pytest.mark.parametrize("M,N,K", [(1, 1, 1), (2, 4, 9), (2, 16, 19), (7, 32, 16), (128, 3072, 768), (128, 768, 3072),
                                    (300, 768, 768), (65, 100, 200)])

@@ -1069,11 +1069,27 @@ struct TileOrder {
     FixedDivisor group, rows, last_rows;  // tiles of a group; tile rows of a group; tile rows of the last, smaller group
 };
 
-__device__ __forceinline__ float plain_dot(const float *a, const float *b, int k) {
-    float sum = 0.f;
-    for (int i = 0; i < k; ++i)
-        sum = fmaf(a[i], b[i], sum);
-    return sum;
+// An infinity, a NaN or a value that rounds to infinity in bfloat16 has no planes (inf - inf is no number), and turns every sum
+// it enters into something that is not finite.  A wave that finds such a sum in one of its 32 x 32 blocks multiplies that block
+// again, its own part of K, with the fp32 matrix instruction and operands straight from memory, and takes those sums in the
+// place of the ones that are not finite.  pa, pb = this lane's row of A and of B, eight values into the step for the upper
+// lanes; steps of 16 k from `first` to `end`, `stride` apart.
+// Nothing overlaps here, so a block costs several times what it did: [384,3072] x [3072,768] takes 28 us, with two rows that
+// are not finite 74, with every value NaN 91 (one thread per sum: 1.6 ms and 1.9 ms; 96 x 96 tiles 78 -> 350, were 13 ms).
+__device__ __forceinline__ void multiply_again(const float *pa, const float *pb, int first, int end, int stride, f32x16 &acc) {
+    f32x16 sum;
+#pragma unroll
+    for (int r = 0; r < 16; ++r)
+        sum[r] = 0.f;
+#pragma unroll 1
+    for (int t = first; t < end; t += stride) {
+        const uint4 *a = reinterpret_cast<const uint4 *>(pa + (size_t)t * 16), *b = reinterpret_cast<const uint4 *>(pb + (size_t)t * 16);
+        GemmTraits<TNN_ROCM_F32>::mma(b[0], a[0], sum);
+        GemmTraits<TNN_ROCM_F32>::mma(b[1], a[1], sum);
+    }
+#pragma unroll
+    for (int r = 0; r < 16; ++r)
+        acc[r] = split_finite(__builtin_fabsf(acc[r])) ? acc[r] : sum[r];
 }
 
 template <int DT, typename CFG, typename Epi>
@@ -1701,6 +1717,29 @@ __global__ void __launch_bounds__(CFG::NT)
 #undef TR_CLAMPK
     }
 
+    if constexpr (DT == TNN_ROCM_F32 && CFG::NSTAGE > 0) {
+        constexpr int STEPS = SLAB / KSTEP;  // 16-wide steps per slab
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j) {
+                float size = 0.f;
+#pragma unroll
+                for (int r = 0; r < 16; ++r)
+                    size += __builtin_fabsf(acc[i][j][r]);
+                if (__all(split_finite(size)))
+                    continue;
+                // clamped as the slabs' rows are
+                const int ra = m0 + (wm * TM + i) * 32 + frag_row, rb = n0 + (wn * TN + j) * 32 + frag_row;
+                const T *pa = A + (size_t)(ra < M ? ra : M - 1) * lda + 8 * (lane >> 5);
+                const T *pb = B + (size_t)(rb < N ? rb : N - 1) * ldb + 8 * (lane >> 5);
+                if constexpr (CFG::OWN)
+                    multiply_again(pa, pb, nk * wk / WGK * STEPS, nk * (wk + 1) / WGK * STEPS, 1, acc[i][j]);
+                else
+                    multiply_again(pa, pb, wk, nk * STEPS, WGK, acc[i][j]);
+            }
+    }
+
     typedef typename std::remove_reference<decltype(acc[0][0][0])>::type AccT;
     // Row-contiguous epilogue.  In the accumulator layout one store instruction touches 32 rows with 16 bytes
     // each, i.e. 32 partial cache lines; the L2 then sees eight times as many write requests as there are lines.
@@ -1838,21 +1877,6 @@ __global__ void __launch_bounds__(CFG::NT)
             }
             const int m = m0 + ((pos / WGN) * TM + i) * 32 + row;
             const int n = n0 + (pos % WGN) * CW + c8;
-            if constexpr (DT == TNN_ROCM_F32 && CFG::NSTAGE > 0) {
-                // an infinity in an operand has no planes (inf - inf is no number): such a sum is formed again from the
-                // operands themselves
-#pragma unroll
-                for (int t = 0; t < 8; ++t) {
-                    const float v = t < 4 ? lo[t] : hi[t - 4];
-                    if (!(__builtin_fabsf(v) < INFINITY) && m < M && n + t < N) {
-                        const float f = plain_dot(A + (size_t)m * lda, B + (size_t)(n + t) * ldb, K);
-                        if (t < 4)
-                            lo[t & 3] = f;
-                        else
-                            hi[t & 3] = f;
-                    }
-                }
-            }
             const int nl = (pos % WGN) * CW + c8;  // column inside the tile
             const u32x4 *const ahead = AHEAD > 0 ? ahead_vec : nullptr;
             if constexpr (Epi::kRowStats) {

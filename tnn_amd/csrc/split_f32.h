@@ -73,5 +73,9 @@ __device__ __forceinline__ void split_mma(const Split3 &a, const Split3 &b, int 
                                                 0, 0, 0);
 }
 
+// is x, a value without sign, neither infinite nor a NaN?  On the bits: of a sum of magnitudes "< INFINITY" the compiler makes
+// "!= INFINITY", which a NaN passes.
+__device__ __forceinline__ bool split_finite(float x) { return (__float_as_uint(x) & 0x7fffffffu) < 0x7f800000u; }
+
 }  // namespace tnn_rocm
 #endif
