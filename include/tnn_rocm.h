@@ -135,6 +135,7 @@ TNN_ROCM_API int tnn_rocm_gemm_i8(void *stream, const int8_t *A, const int8_t *W
  *   kv_len : optional int32 [B]; keys j >= kv_len[b] are excluded exactly (−inf) and their tiles
  *            skipped.  kv_len[b] = 0 (the mask routines below never produce it: a row that masks every key keeps all
  *            of them, as the reference's softmax does) writes the sequence's output rows as zeros.
+ *            A row whose every score is -inf comes out as NaN in F32, as from the softmax layer, and as zeros in F16 / BF16.
  *            (bit 30 of an entry may be set by tnn_rocm_mask_to_kv_len_flagged: mask row b is then not read). */
 TNN_ROCM_API int tnn_rocm_attention(void *stream, int dtype, const void *q, const void *k, const void *v, void *out,
                                     int B, int heads, int S, int head_dim, long q_sb, long q_sh, long q_ss, long kv_sb,

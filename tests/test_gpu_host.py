@@ -701,6 +701,27 @@ def test_fp32_attention_group_equals_its_layers(B, S):
     inst.close()
 
 
+def test_fp32_attention_group_equals_its_layers_where_a_mask_hides_every_key():
+    """An additive mask of -inf throughout leaves a sequence without an answer: NaN from the softmax layer, and from the group;
+    the other sequence is not concerned."""
+    host, tnnmodel, EncoderConfig, make_weights, make_inputs = _mods()
+    say("host: fp32 attention group, a mask of -inf")
+    cfg, B, S = EncoderConfig(2, 128, 2, 256), 2, 40
+    w = make_weights(cfg, seed=31, bias_std=0.05)
+    inst = host.RocmInstance.from_graph(tnnmodel.encoder_graph(cfg, w, B, S), "fp32")
+    ids, seg, lens, mask = make_inputs(cfg, B, S, 20, S, seed=51)
+    mask[1] = -np.inf
+    for n, v in (("input_ids", ids), ("token_type_ids", seg), ("attention_bias", mask.reshape(B, 1, 1, S))):
+        inst.set_input(n, v)
+    inst.forward()
+    got = inst.output("last_hidden").reshape(B, S, -1).copy()
+    inst.forward_with_callback(after=lambda name, typ, blobs: None)
+    alone = inst.output("last_hidden").reshape(B, S, -1)
+    assert np.isnan(alone[1]).all() and np.isnan(got[1]).all()
+    assert rel_err(got[0], alone[0]) <= 3e-6
+    inst.close()
+
+
 @pytest.mark.parametrize("precision", ["fp32", "fp16", "bf16"])
 def test_two_attention_masks_in_one_net(precision):
     """Two layers, each with a padding mask of its own, made in the graph as Sub(1 - m) -> Mul(-10000) right in front of the

@@ -924,6 +924,64 @@ def test_attention_fp32(B, h, S, masked):
     assert got.dtype == np.float32 and rel_err(got, ref) <= 3e-6
 
 
+def _attention_layers(q, k, v, scale, mask):
+    """the decomposed layers in float64, scores and probabilities as they are: infinities and NaN take their course"""
+    q, k, v = (t.astype(np.float64) for t in (q, k, v))
+    s = (q[..., :, None, :] * k[..., None, :, :]).sum(-1) * scale + (0 if mask is None else mask.astype(np.float64)[:, None, None, :])
+    p = np.exp(s - s.max(-1, keepdims=True))
+    p /= p.sum(-1, keepdims=True)
+    return (p[..., None] * v[..., None, :, :]).sum(-2)
+
+
+@pytest.mark.parametrize("S", [7, 32, 70, 200])
+@pytest.mark.parametrize("what", ["k -inf", "k +inf", "k nan", "q nan", "q inf", "v inf", "v nan", "v near the largest", "k near the largest",
+                                  "v all the largest", "row of -inf", "scores beyond the largest"])
+def test_attention_fp32_special_values(S, what):
+    """Values without bf16 planes (infinities, NaN, finite ones that round to infinity in bfloat16) give what the layers make
+    of them in plain arithmetic: a key whose score is -inf has probability 0, a huge V stays finite, a query whose scores
+    are all -inf has no answer, and nothing spreads to rows, columns and heads that it does not concern."""
+    say("attention fp32 S=%d, %s" % (S, what))
+    rng = np.random.default_rng(S)
+    B, h = 2, 2
+    q, k, v = (rng.standard_normal((B, h, S, 64)).astype(np.float32) for _ in range(3))
+    q[..., 5] = np.abs(q[..., 5]) + np.float32(0.5)
+    at, mask = S // 2, None
+    if what in ("k -inf", "k +inf", "k nan"):
+        k[1, 0, at, 5] = {"k -inf": -np.inf, "k +inf": np.inf, "k nan": np.nan}[what]
+    elif what in ("q nan", "q inf"):
+        q[0, 1, at, 9] = np.nan if what == "q nan" else np.inf
+        k[0, 1, :, 9] = -np.abs(k[0, 1, :, 9])
+        k[0, 1, 0, 9] = 1  # one key scores +inf for that query
+    elif what in ("v inf", "v nan"):
+        v[0, 0, at, 17] = np.inf if what == "v inf" else np.nan
+    elif what == "v near the largest":
+        v[1, 1, at, 3], v[1, 1, 0, 60] = 3.4e38, -3.4e38
+    elif what == "v all the largest":
+        v[0, 1, :, 8] = 3.4e38
+    elif what == "k near the largest":
+        q[..., 9], k[..., 9], k[1, 1, at, 9] = 1e-38, 0, 3.4e38
+    elif what == "row of -inf":
+        mask = rng.standard_normal((B, S)).astype(np.float32)
+        mask[1], mask[0, at] = -np.inf, -np.inf
+    else:
+        q[0, 0, at], k[0, 0, 1], k[0, 0, 2] = 2e19, 3e19, -3e19  # +3.8e40: infinite in fp32, and so the row has no answer
+    got = host(ops().attention(dev(q), dev(k), dev(v), 0.125, mask=None if mask is None else dev(mask)))
+    with np.errstate(all="ignore"):
+        ref = _attention_layers(q, k, v, 0.125, mask)
+        if what == "scores beyond the largest":
+            ref[0, 0, at] = np.nan
+    assert np.array_equal(np.isnan(got), np.isnan(ref))
+    assert np.array_equal(np.isposinf(got), np.isposinf(ref)) and np.array_equal(np.isneginf(got), np.isneginf(ref))
+    fine = np.isfinite(ref)
+    assert fine.any()
+    for b in range(B):  # by head: one holds values of 1e38
+        for i in range(h):
+            f = fine[b, i]
+            for d in (range(64) if "largest" in what else [slice(None)]):
+                if f[:, d].any():
+                    assert rel_err(got[b, i][:, d][f[:, d]], ref[b, i][:, d][f[:, d]]) <= 3e-6
+
+
 def test_attention_packed_qkv_layout():
     say("attention packed [T,3H]")
     B, S, h = 2, 96, 12

@@ -14,6 +14,11 @@
 // is key 8*(r/4) + 4*g + r%4), and the probabilities are in the register order that the second product O^T = V^T P^T wants,
 // given V rows in that order.  Row i of block dt of O^T is column d = 2*i + dt of the head.
 //
+// An infinity, a NaN or a value that rounds to infinity in bfloat16 has no planes and makes every sum it enters something that is
+// not finite.  A workgroup that finds such a sum, or a sum of probabilities times values that ran over, does its block again
+// with the fp32 matrix instruction, operands straight from memory (`exact` below): the answer is then that of the layers in
+// fp32 arithmetic.  The check is 33 instructions a wave.
+//
 // What bounds it: the vector ALU (conversion of K, V and P: 28 instructions per operand and 16-wide step, and the
 // exponentials) and the matrix pipe, about equal.  us, the decomposed launches -> this kernel, 12 heads:
 //   1 x 128 tokens 45 -> 7.6, 4 x 384 136 -> 29 (K and V read once per block of 32 queries: 113 MB from L2), 8 x 128 11, 1 x 512 16
@@ -53,6 +58,7 @@ __device__ __forceinline__ float other_half(float v) {
 template <int NW> __global__ void __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) attention_f32_kernel(AttnF32Params p) {
     __shared__ __attribute__((aligned(16))) float stage[NW][kBlockQ * kStageRow];
     __shared__ float stat_m[NW][kBlockQ], stat_l[NW][kBlockQ];
+    __shared__ int again[NW];
 
     touch_kernel_args<sizeof(AttnF32Params)>();
     const int tid  = threadIdx.x;
@@ -85,49 +91,38 @@ template <int NW> __global__ void __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) at
     const float *kb = p.k + (size_t)b * p.kv_sb + (size_t)head * p.kv_sh;
     const float *vb = p.v + (size_t)b * p.kv_sb + (size_t)head * p.kv_sh;
     const float *mb = p.mask && !mask_is_zero ? p.mask + (size_t)b * S : nullptr;
-    const SplitConst sc;
-
-    // Rows past the end are clamped to the last one: keys at or beyond kv_end get the score -inf, queries past S are never
-    // stored.  Per-head extents fit 32 bits (checked by the launcher).
-    Split3 qf[4];
-    {
-        int row = q0 + lq;
-        row     = row < S ? row : S - 1;
-        const float *src = qb + (size_t)row * p.q_ss + 8 * g;
-#pragma unroll
-        for (int kk = 0; kk < 4; ++kk) {
-            const f32x4 lo = *reinterpret_cast<const f32x4 *>(src + kk * 16), hi = *reinterpret_cast<const f32x4 *>(src + kk * 16 + 4);
-            const float x[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-            qf[kk]           = split3(x, sc);
-        }
-    }
-
-    f32x16 oacc[2];
-#pragma unroll
-    for (int dt = 0; dt < 2; ++dt)
-#pragma unroll
-        for (int r = 0; r < 16; ++r)
-            oacc[dt][r] = 0.f;
-    float m_i = -INFINITY, l_i = 0.f;
-
     const uint32_t ss   = (uint32_t)p.kv_ss;
     const int n_tiles   = (kv_end + kBlockK - 1) / kBlockK;
-    f32x4 kraw[8];
-    auto load_k = [&](int t) __attribute__((always_inline)) {
-        int row = t * kBlockK + lq;
-        row     = row < S ? row : S - 1;
-        const float *src = kb + ((uint32_t)row * ss + 8u * g);
+    f32x16 oacc[2];
+    float m_i, l_i, low;
+    // Rows past the end are clamped to the last one: keys at or beyond kv_end get the score -inf, queries past S are never
+    // stored.  Per-head extents fit 32 bits (checked by the launcher).
+    // this lane's row of Q, or of K in block t: eight values of every 16-wide step
+    auto load_row = [&](const float *src, f32x4 (&raw)[8]) __attribute__((always_inline)) {
 #pragma unroll
         for (int kk = 0; kk < 4; ++kk) {
-            kraw[2 * kk]     = *reinterpret_cast<const f32x4 *>(src + kk * 16);
-            kraw[2 * kk + 1] = *reinterpret_cast<const f32x4 *>(src + kk * 16 + 4);
+            raw[2 * kk]     = *reinterpret_cast<const f32x4 *>(src + kk * 16);
+            raw[2 * kk + 1] = *reinterpret_cast<const f32x4 *>(src + kk * 16 + 4);
         }
     };
-    if (wave < n_tiles)
-        load_k(wave);
-    for (int t = wave; t < n_tiles; t += NW) {
-        // V of this block: slot e of step st and lane half g is key 16*st + 4*g + e (e < 4), 16*st + 8 + 4*g + e-4
-        f32x2 vraw[16];
+    auto load_q = [&](f32x4 (&raw)[8]) __attribute__((always_inline)) {
+        const int row = q0 + lq < S ? q0 + lq : S - 1;
+        load_row(qb + (size_t)row * p.q_ss + 8 * g, raw);
+    };
+    auto load_k = [&](int t, f32x4 (&raw)[8]) __attribute__((always_inline)) {
+        const int row = t * kBlockK + lq < S ? t * kBlockK + lq : S - 1;
+        load_row(kb + ((uint32_t)row * ss + 8u * g), raw);
+    };
+    auto begin = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int dt = 0; dt < 2; ++dt)
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+                oacc[dt][r] = 0.f;
+        m_i = -INFINITY, l_i = 0.f, low = 0.f;
+    };
+    // V of block t: slot e of step st and lane half g is key 16*st + 4*g + e (e < 4), 16*st + 8 + 4*g + e-4
+    auto load_v = [&](int t, f32x2 (&vraw)[16]) __attribute__((always_inline)) {
 #pragma unroll
         for (int st = 0; st < 2; ++st)
 #pragma unroll
@@ -136,29 +131,16 @@ template <int NW> __global__ void __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) at
                 row     = row < S ? row : S - 1;
                 vraw[st * 8 + e] = *reinterpret_cast<const f32x2 *>(vb + ((uint32_t)row * ss + 2u * lq));
             }
-        // ---- S^T = K Q^T
-        f32x16 s;
-#pragma unroll
-        for (int r = 0; r < 16; ++r)
-            s[r] = 0.f;
-#pragma unroll
-        for (int kk = 0; kk < 4; ++kk) {
-            const f32x4 lo = kraw[2 * kk], hi = kraw[2 * kk + 1];
-            const float x[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-            const Split3 kf  = split3(x, sc);
-#pragma unroll
-            for (int pr = 0; pr < kSplitProducts; ++pr)
-                split_mma(kf, qf[kk], pr, s);
-        }
-        if (t + NW < n_tiles)
-            load_k(t + NW);
-        // ---- softmax over this block's keys: scores * scale + mask, as the decomposed layers form them
+    };
+    // softmax over block t's keys: scores * scale + mask, as the decomposed layers form them
+    auto softmax = [&](int t, f32x16 &s) __attribute__((always_inline)) {
         float mx = -INFINITY;
 #pragma unroll
         for (int r4 = 0; r4 < 4; ++r4) {
             const int key0 = t * kBlockK + 8 * r4 + 4 * g;
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
+                low     = fminf(low, s[r4 * 4 + e]);
                 float v = __fmul_rn(s[r4 * 4 + e], p.scale);
                 if (mb)
                     v = __fadd_rn(v, mb[key0 + e < S ? key0 + e : S - 1]);
@@ -186,29 +168,9 @@ template <int NW> __global__ void __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) at
                     oacc[dt][r] *= alpha;
         }
         m_i = m_new;
-        // ---- O^T += V^T P^T
-#pragma unroll
-        for (int st = 0; st < 2; ++st) {
-            const float x[8] = {s[8 * st + 0], s[8 * st + 1], s[8 * st + 2], s[8 * st + 3],
-                                s[8 * st + 4], s[8 * st + 5], s[8 * st + 6], s[8 * st + 7]};
-            const Split3 pf  = split3(x, sc);
-            Split3 vf[2];
-#pragma unroll
-            for (int dt = 0; dt < 2; ++dt) {
-                const f32x2 *vr  = vraw + st * 8;
-                const float y[8] = {vr[0][dt], vr[1][dt], vr[2][dt], vr[3][dt], vr[4][dt], vr[5][dt], vr[6][dt], vr[7][dt]};
-                vf[dt]           = split3(y, sc);
-            }
-#pragma unroll
-            for (int pr = 0; pr < kSplitProducts; ++pr)
-#pragma unroll
-                for (int dt = 0; dt < 2; ++dt)
-                    split_mma(vf[dt], pf, pr, oacc[dt]);
-        }
-    }
-
-    // ---- merge the waves: every wave leaves its sums, scaled to its own maximum
-    {
+    };
+    // every wave leaves its sums, scaled to its own maximum
+    auto leave = [&]() __attribute__((always_inline)) {
         float *row = stage[wave] + lq * kStageRow;
 #pragma unroll
         for (int r4 = 0; r4 < 4; ++r4) {
@@ -220,8 +182,117 @@ template <int NW> __global__ void __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) at
             stat_m[wave][lq] = m_i;
             stat_l[wave][lq] = l_i;
         }
+    };
+
+    {
+        const SplitConst sc;
+        Split3 qf[4];
+        f32x4 kraw[8];
+        load_q(kraw);
+#pragma unroll
+        for (int kk = 0; kk < 4; ++kk) {
+            const f32x4 lo = kraw[2 * kk], hi = kraw[2 * kk + 1];
+            const float x[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+            qf[kk]           = split3(x, sc);
+        }
+        begin();
+        if (wave < n_tiles)
+            load_k(wave, kraw);
+        for (int t = wave; t < n_tiles; t += NW) {
+            f32x2 vraw[16];
+            load_v(t, vraw);
+            // ---- S^T = K Q^T
+            f32x16 s;
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+                s[r] = 0.f;
+#pragma unroll
+            for (int kk = 0; kk < 4; ++kk) {
+                const f32x4 lo = kraw[2 * kk], hi = kraw[2 * kk + 1];
+                const float x[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+                const Split3 kf  = split3(x, sc);
+#pragma unroll
+                for (int pr = 0; pr < kSplitProducts; ++pr)
+                    split_mma(kf, qf[kk], pr, s);
+            }
+            if (t + NW < n_tiles)
+                load_k(t + NW, kraw);
+            softmax(t, s);
+            // ---- O^T += V^T P^T
+#pragma unroll
+            for (int st = 0; st < 2; ++st) {
+                const float x[8] = {s[8 * st + 0], s[8 * st + 1], s[8 * st + 2], s[8 * st + 3],
+                                    s[8 * st + 4], s[8 * st + 5], s[8 * st + 6], s[8 * st + 7]};
+                const Split3 pf  = split3(x, sc);
+                Split3 vf[2];
+#pragma unroll
+                for (int dt = 0; dt < 2; ++dt) {
+                    const f32x2 *vr  = vraw + st * 8;
+                    const float y[8] = {vr[0][dt], vr[1][dt], vr[2][dt], vr[3][dt], vr[4][dt], vr[5][dt], vr[6][dt], vr[7][dt]};
+                    vf[dt]           = split3(y, sc);
+                }
+#pragma unroll
+                for (int pr = 0; pr < kSplitProducts; ++pr)
+#pragma unroll
+                    for (int dt = 0; dt < 2; ++dt)
+                        split_mma(vf[dt], pf, pr, oacc[dt]);
+            }
+        }
+    }
+    leave();
+    {
+        // a score of -inf may be one that has no planes, or one that is; anything else that is not finite is in the sums
+        float size = l_i;
+#pragma unroll
+        for (int dt = 0; dt < 2; ++dt)
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+                size += __builtin_fabsf(oacc[dt][r]);
+        const int bad = __any(!split_finite(size) || !split_finite(low));
+        if (lane == 0)
+            again[wave] = bad;
     }
     __syncthreads();
+    int any_bad = 0;
+#pragma unroll
+    for (int w = 0; w < NW; ++w)
+        any_bad |= again[w];
+    const bool exact = __builtin_amdgcn_readfirstlane(any_bad) != 0;
+    // probabilities are taken down by a power of two of at least S, so that no partial sum runs over before the division
+    const int down = 32 - __builtin_clz((unsigned)S);
+    if (exact) {
+        __syncthreads();  // everyone has read the flags
+        const float pscale = __uint_as_float((uint32_t)(127 - down) << 23);
+        begin();
+#pragma unroll 1
+        for (int t = wave; t < n_tiles; t += NW) {
+            f32x16 s;
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+                s[r] = 0.f;
+            f32x4 kraw[8], qraw[8];
+            load_k(t, kraw);
+            load_q(qraw);
+#pragma unroll
+            for (int kk = 0; kk < 8; ++kk)
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    s = __builtin_amdgcn_mfma_f32_32x32x2f32(kraw[kk][e], qraw[kk][e], s, 0, 0, 0);
+            softmax(t, s);
+            f32x2 vraw[16];
+            load_v(t, vraw);
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+#pragma unroll
+                for (int dt = 0; dt < 2; ++dt)
+                    oacc[dt] = __builtin_amdgcn_mfma_f32_32x32x2f32(vraw[r][dt], s[r] * pscale, oacc[dt], 0, 0, 0);
+        }
+        leave();
+        __syncthreads();
+    }
+    const float up = exact ? __uint_as_float((uint32_t)(127 + down) << 23) : 1.f;
+
+    // ---- merge the waves
 #pragma unroll
     for (int it = 0; it < kBlockQ * kD / 4 / (NW * 64); ++it) {
         const int item = it * NW * 64 + tid, row = item / (kD / 4), c = item % (kD / 4) * 4;
@@ -243,10 +314,11 @@ template <int NW> __global__ void __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) at
             for (int e = 0; e < 4; ++e)
                 acc[e] = fmaf(x[e], f, acc[e]);
         }
-        const float inv = total_l > 0.f ? 1.0f / total_l : 0.f;
+        // no key at all: zeros; a row whose every score is -inf: no number, as the softmax layer makes of it
+        const float inv = total_l > 0.f ? 1.0f / total_l : kv_end > 0 ? NAN : 0.f;
 #pragma unroll
         for (int e = 0; e < 4; ++e)
-            acc[e] *= inv;
+            acc[e] = acc[e] * inv * up;
         store_out16(p.through, p.o + (size_t)b * p.o_sb + (size_t)head * p.o_sh + (size_t)(q0 + row) * p.o_ss + c,
                     __builtin_bit_cast(store_u32x4, acc));
     }
