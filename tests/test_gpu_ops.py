@@ -621,6 +621,30 @@ def test_gemm_fp32_split_shapes(code, M, N, K):
     assert (np.abs(got[fine] - exact[fine]) <= 2.0 ** -24 * 4 * np.sqrt(K) * size[fine]).all()
 
 
+@pytest.mark.parametrize("code", [9111141, 9121141, 9111181, 9221141, 9321140, 3231142, 2331142, 3222121, 2222221])
+@pytest.mark.parametrize("ea,ew", [(-118, 0), (-126, 30), (-140, 60), (0, -118), (-100, -20), (110, -60), (60, 25)])
+def test_gemm_fp32_split_small_and_large(code, ea, ew):
+    """Operands at the ends of the fp32 range (values below the normal ones among them) keep their 24 bits through the three
+    planes, and sums that run over on the way are formed again: no further from float64 than an fp32 sum is, plus half of the
+    smallest step for a result below the normal range."""
+    from tnn_amd import capi
+    lib = capi.load()
+    M, N, K = 97, 104, 256
+    rng = np.random.default_rng(code % 1000 + 200 + ea)
+    a = (rng.standard_normal((M, K)) * 2.0 ** ea).astype(np.float32)
+    w = (rng.standard_normal((N, K)) * 2.0 ** ew).astype(np.float32)
+    a[5] = 0
+    lib.tnn_rocm_debug_set_gemm_config(code)
+    try:
+        got = host(ops().gemm(dev(a), dev(w), True)).astype(np.float64)
+    finally:
+        lib.tnn_rocm_debug_set_gemm_config(0)
+    exact = a.astype(np.float64) @ w.astype(np.float64).T
+    size = np.abs(a.astype(np.float64)) @ np.abs(w.astype(np.float64)).T
+    assert (got[5] == 0).all() and np.isfinite(got).all()
+    assert (np.abs(got - exact) <= 2.0 ** -24 * 4 * size + 2.0 ** -149).all()
+
+
 @pytest.mark.parametrize("code", [0, 9111181, 9321140, 2331142, 2222221])
 def test_gemm_fp32_not_finite_costs_a_few_launches(code):
     """An overflow upstream makes whole rows, or all, of an activation NaN: the product says so, and does not take orders of
@@ -980,6 +1004,20 @@ def test_attention_fp32_special_values(S, what):
             for d in (range(64) if "largest" in what else [slice(None)]):
                 if f[:, d].any():
                     assert rel_err(got[b, i][:, d][f[:, d]], ref[b, i][:, d][f[:, d]]) <= 3e-6
+
+
+@pytest.mark.parametrize("eq,ek,ev,scale", [(-118, 118, 0, 0.125), (40, -120, 0, 2.0 ** 77), (0, 0, -118, 0.125), (0, 0, -138, 0.125),
+                                            (50, 50, 0, 2.0 ** -103), (0, 0, 110, 0.125), (0, 0, 80, 0.125)])
+@pytest.mark.parametrize("S", [20, 150])
+def test_attention_fp32_small_and_large(S, eq, ek, ev, scale):
+    """Q, K and V at the ends of the fp32 range keep their 24 bits; a product of the scale with a power of two that cancels it
+    is exact, so the answer is that of the ordinary sizes, shifted."""
+    say("attention fp32 S=%d, 2^%d 2^%d 2^%d" % (S, eq, ek, ev))
+    rng = np.random.default_rng(S + 200 + ev)
+    q, k, v = ((rng.standard_normal((1, 2, S, 64)) * 2.0 ** e).astype(np.float32) for e in (eq, ek, ev))
+    got = host(ops().attention(dev(q), dev(k), dev(v), scale)).astype(np.float64)
+    ref = _attention_layers(q, k, v, float(np.float32(scale)), None)
+    assert np.abs(got - ref).max() <= 3e-6 * np.abs(ref).max() + 2.0 ** -149
 
 
 def test_attention_packed_qkv_layout():

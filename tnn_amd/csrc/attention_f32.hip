@@ -14,12 +14,12 @@
 // is key 8*(r/4) + 4*g + r%4), and the probabilities are in the register order that the second product O^T = V^T P^T wants,
 // given V rows in that order.  Row i of block dt of O^T is column d = 2*i + dt of the head.
 //
-// An infinity, a NaN or a value that rounds to infinity in bfloat16 has no planes and makes every sum it enters something that is
-// not finite.  A workgroup that finds such a sum, or a sum of probabilities times values that ran over, does its block again
+// An infinity, a NaN or a finite value from 2^104 on has no planes (split_f32.h) and makes every sum it enters something that is
+// not finite, as a sum beyond 2^80 becomes by itself.  A workgroup that finds such a sum does its block again
 // with the fp32 matrix instruction, operands straight from memory (`exact` below): the answer is then that of the layers in
 // fp32 arithmetic.  The check is 33 instructions a wave.
 //
-// What bounds it: the vector ALU (conversion of K, V and P: 28 instructions per operand and 16-wide step, and the
+// What bounds it: the vector ALU (conversion of K, V and P: 36 instructions per operand and 16-wide step, and the
 // exponentials) and the matrix pipe, about equal.  us, the decomposed launches -> this kernel, 12 heads:
 //   1 x 128 tokens 45 -> 7.6, 4 x 384 136 -> 29 (K and V read once per block of 32 queries: 113 MB from L2), 8 x 128 11, 1 x 512 16
 #include "common.h"
@@ -45,7 +45,8 @@ struct AttnF32Params : StoreThrough {
     long q_sb, q_sh, q_ss, kv_sb, kv_sh, kv_ss, o_sb, o_sh, o_ss;
     int S, B, heads;
     FixedDivisor by_blocks, by_heads;
-    float scale;
+    float scale, split_scale;  // of a score, of a score made from planes
+    int planes;                // 0: the scale is too small for split_scale, the block is done with the fp32 instruction
     const float *mask;  // [B,S] additive or null
     const int32_t *kv_len;
 };
@@ -133,7 +134,7 @@ template <int NW> __global__ void __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) at
             }
     };
     // softmax over block t's keys: scores * scale + mask, as the decomposed layers form them
-    auto softmax = [&](int t, f32x16 &s) __attribute__((always_inline)) {
+    auto softmax = [&](int t, float scale, f32x16 &s) __attribute__((always_inline)) {
         float mx = -INFINITY;
 #pragma unroll
         for (int r4 = 0; r4 < 4; ++r4) {
@@ -141,7 +142,7 @@ template <int NW> __global__ void __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) at
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 low     = fminf(low, s[r4 * 4 + e]);
-                float v = __fmul_rn(s[r4 * 4 + e], p.scale);
+                float v = __fmul_rn(s[r4 * 4 + e], scale);
                 if (mb)
                     v = __fadd_rn(v, mb[key0 + e < S ? key0 + e : S - 1]);
                 v             = key0 + e < kv_end ? v : -INFINITY;
@@ -217,7 +218,7 @@ template <int NW> __global__ void __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) at
             }
             if (t + NW < n_tiles)
                 load_k(t + NW, kraw);
-            softmax(t, s);
+            softmax(t, p.split_scale, s);
             // ---- O^T += V^T P^T
 #pragma unroll
             for (int st = 0; st < 2; ++st) {
@@ -248,7 +249,8 @@ template <int NW> __global__ void __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) at
 #pragma unroll
             for (int r = 0; r < 16; ++r)
                 size += __builtin_fabsf(oacc[dt][r]);
-        const int bad = __any(!split_finite(size) || !split_finite(low));
+        // the sums of up to four waves are added up below
+        const int bad = !p.planes || __any(!split_finite(size * 4.f) || !split_finite(low));
         if (lane == 0)
             again[wave] = bad;
     }
@@ -278,7 +280,7 @@ template <int NW> __global__ void __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) at
 #pragma unroll
                 for (int e = 0; e < 4; ++e)
                     s = __builtin_amdgcn_mfma_f32_32x32x2f32(kraw[kk][e], qraw[kk][e], s, 0, 0, 0);
-            softmax(t, s);
+            softmax(t, p.scale, s);
             f32x2 vraw[16];
             load_v(t, vraw);
 #pragma unroll
@@ -290,7 +292,7 @@ template <int NW> __global__ void __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) at
         leave();
         __syncthreads();
     }
-    const float up = exact ? __uint_as_float((uint32_t)(127 + down) << 23) : 1.f;
+    const float up = exact ? __uint_as_float((uint32_t)(127 + down) << 23) : kSplitUnscale;
 
     // ---- merge the waves
 #pragma unroll
@@ -340,7 +342,9 @@ int launch_attention_f32(hipStream_t s, const float *q, const float *k, const fl
     p.S = S, p.B = B, p.heads = heads;
     p.by_blocks = FixedDivisor::of((uint32_t)((S + kBlockQ - 1) / kBlockQ));
     p.by_heads  = FixedDivisor::of((uint32_t)heads);
-    p.scale  = scale;
+    p.scale       = scale;
+    p.split_scale = scale * kSplitUnscale;
+    p.planes      = !(scale > -1e-20f && scale < 1e-20f);  // no bit of split_scale is lost from 2^-78 on
     p.mask   = mask;
     p.kv_len = kv_len;
     const long total = (long)((S + kBlockQ - 1) / kBlockQ) * heads * B;

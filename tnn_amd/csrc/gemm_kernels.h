@@ -96,7 +96,7 @@ template <> struct GemmTraits<TNN_ROCM_F32> {
 };
 // fp32, pipelined: the planes of the operands of the STEPS steps that a wave takes from one slab.  turn() multiplies one
 // slab's planes while it makes the next one's from their LDS reads: a matrix instruction leaves the vector ALU free for 7 of
-// its 8 issue slots, and the conversion (28 vector instructions per operand and step) goes into them a piece at a time.
+// its 8 issue slots, and the conversion (36 vector instructions per operand and step) goes into them a piece at a time.
 // The order is pinned: left to itself the compiler issues the two kinds one after the other, with the wait states that a
 // dot product's result needs standing empty (64x64 tile, K=3072: 43 us; pinned: 41 us).
 template <int TM, int TN, int STEPS> struct SplitSlab {
@@ -130,6 +130,8 @@ template <int TM, int TN, int STEPS> struct SplitSlab {
         const int ks = k / (OPS * 6), o = k / 6 % OPS, plane = k % 6 / 2, g = k % 2;
         float *x = rest[ks][o] + g * 4;
         uint32_t *p = next.op[ks][o].p[plane] + g * 2;
+        if (plane == 0)
+            x[0] *= kSplitScale, x[1] *= kSplitScale, x[2] *= kSplitScale, x[3] *= kSplitScale;
         p[0] = split_pack(x[0], x[1]);
         p[1] = split_pack(x[2], x[3]);
         if (plane < 2) {
@@ -1069,8 +1071,8 @@ struct TileOrder {
     FixedDivisor group, rows, last_rows;  // tiles of a group; tile rows of a group; tile rows of the last, smaller group
 };
 
-// An infinity, a NaN or a value that rounds to infinity in bfloat16 has no planes (inf - inf is no number), and turns every sum
-// it enters into something that is not finite.  A wave that finds such a sum in one of its 32 x 32 blocks multiplies that block
+// An infinity, a NaN or a finite value from 2^104 on has no planes (split_f32.h), and turns every sum it enters into something
+// that is not finite, as a sum beyond 2^80 becomes by itself.  A wave that finds such a sum in one of its 32 x 32 blocks multiplies that block
 // again, its own part of K, with the fp32 matrix instruction and operands straight from memory, and takes those sums in the
 // place of the ones that are not finite.  pa, pb = this lane's row of A and of B, eight values into the step for the upper
 // lanes; steps of 16 k from `first` to `end`, `stride` apart.
@@ -1727,6 +1729,9 @@ __global__ void __launch_bounds__(CFG::NT)
 #pragma unroll
                 for (int r = 0; r < 16; ++r)
                     size += __builtin_fabsf(acc[i][j][r]);
+#pragma unroll
+                for (int r = 0; r < 16; ++r)
+                    acc[i][j][r] *= kSplitUnscale;
                 if (__all(split_finite(size)))
                     continue;
                 // clamped as the slabs' rows are

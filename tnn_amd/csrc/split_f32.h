@@ -2,9 +2,15 @@
 //
 // An fp32 value has 24 significant bits, a bfloat16 eight of its own and the same exponent range, so a value is exactly the
 // sum of three of them: x = x1 + x2 + x3 with x1 = bf16(x), x2 = bf16(x - x1), x3 = bf16(x - x1 - x2), each rounded to
-// nearest (both differences are exact in fp32).  A product is then the sum of nine bf16 products, each exact in the fp32
-// accumulator; the six down to x1*y3 / x2*y2 / x3*y1 are formed.  The three left out are below 2^-26 |x y| together, a
-// quarter of the rounding error that an fp32 product itself carries.  (The scheme is that of Henry, Tang and Heinecke,
+// nearest (both differences are exact in fp32), as long as x3's last place is one that bfloat16 has.  Below 2^-109 it has not
+// (its smallest step is 2^-133), so the planes are those of 2^24 x: exact for every x down to the smallest there is, and a
+// sum of products comes out 2^48 times too large, which its reader takes back.  What the factor costs at the other end shows:
+// x from 2^104 on, or a sum from 2^80 on, gives an infinity or a NaN, as an operand that is infinite or NaN does; the readers
+// look for those and form such a sum again with the fp32 matrix instruction.  The multiplication makes 4.5 instructions per
+// value of 3.5; most go into issue slots that the matrix instructions leave (fp32 request of 4 x 384 tokens, 2887 us without,
+// 2901 with).  A product is then the sum of nine bf16 products, each exact in the fp32 accumulator; the six down to x1*y3 /
+// x2*y2 / x3*y1 are formed.  The three left out are below 2^-26 |x y| together, a quarter of the rounding error that an fp32
+// product itself carries.  (The scheme is that of Henry, Tang and Heinecke,
 // "Leveraging the bfloat16 Artificial Intelligence Datatype For Higher-Precision Computations", ARITH 2019.)
 //
 // Why: the fp32 matrix instruction does 256 operations per CU and clock, the bf16 one 4096, i.e. 683 after six products.
@@ -23,6 +29,9 @@ typedef __bf16 split_bf16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 split_bf16x8 __attribute__((ext_vector_type(8)));
 typedef float split_f32x2 __attribute__((ext_vector_type(2)));
 typedef float split_f32x16 __attribute__((ext_vector_type(16)));
+
+constexpr float kSplitScale   = 16777216.0f;                 // 2^24, of every operand
+constexpr float kSplitUnscale = 1.0f / 281474976710656.0f;   // 2^-48, of every sum of products
 
 // eight values of k of one row or column: one operand of v_mfma_f32_32x32x16_bf16 per plane
 struct Split3 {
@@ -52,7 +61,7 @@ __device__ __forceinline__ Split3 split3(const float (&x)[8], const SplitConst &
     Split3 s;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        const float a = x[2 * i], b = x[2 * i + 1];
+        const float a = x[2 * i] * kSplitScale, b = x[2 * i + 1] * kSplitScale;
         s.p[0][i]      = split_pack(a, b);
         const float ra = split_rest(s.p[0][i], c.lo, a), rb = split_rest(s.p[0][i], c.hi, b);
         s.p[1][i]      = split_pack(ra, rb);
