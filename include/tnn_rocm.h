@@ -71,6 +71,8 @@ TNN_ROCM_API int tnn_rocm_copy_mapped(void *dst, const void *src, size_t bytes, 
 TNN_ROCM_API int tnn_rocm_stream_create(void **stream);
 TNN_ROCM_API int tnn_rocm_stream_destroy(void *stream);
 TNN_ROCM_API int tnn_rocm_stream_sync(void *stream);
+/* waits for everything launched on the stream's device (NULL: the current device), on any stream */
+TNN_ROCM_API int tnn_rocm_device_sync(void *stream);
 /* hipEvent timing on a stream, for the profiler hook of Context (source/tnn/core/context.cc:84-100) */
 TNN_ROCM_API int tnn_rocm_event_create(void **event);
 TNN_ROCM_API int tnn_rocm_event_destroy(void *event);

@@ -32,6 +32,7 @@ SIGNATURES = {
     "tnn_rocm_stream_create": [C.POINTER(_vp)],
     "tnn_rocm_stream_destroy": [_vp],
     "tnn_rocm_stream_sync": [_vp],
+    "tnn_rocm_device_sync": [_vp],
     "tnn_rocm_graph_begin_capture": [_vp],
     "tnn_rocm_graph_end_capture": [_vp, C.POINTER(_vp)],
     "tnn_rocm_graph_launch": [_vp, _vp],

@@ -134,6 +134,21 @@ int tnn_rocm_stream_sync(void *stream) {
     return 0;
 }
 
+int tnn_rocm_device_sync(void *stream) {
+    int current = 0, device = 0;
+    TR_CHECK_HIP(hipGetDevice(&current));
+    device = current;
+    if (stream)
+        TR_CHECK_HIP(hipStreamGetDevice((hipStream_t)stream, &device));
+    if (device != current)
+        TR_CHECK_HIP(hipSetDevice(device));
+    const hipError_t e = hipDeviceSynchronize();
+    if (device != current)
+        TR_CHECK_HIP(hipSetDevice(current));
+    TR_CHECK_HIP(e);
+    return 0;
+}
+
 int tnn_rocm_graph_begin_capture(void *stream) {
     TR_REQUIRE(stream, TNN_ROCM_EINVAL, "graph capture needs a non-default stream");
     TR_CHECK_HIP(hipStreamBeginCapture((hipStream_t)stream, hipStreamCaptureModeThreadLocal));

@@ -352,6 +352,7 @@ public:
     }
 
     Status ConvertFromMatAsync(Mat &mat, MatConvertParam param, void *q) override {
+        RETURN_ON_NEQ(OnQueue(q), TNN_OK);
         auto &desc   = blob_->GetBlobDesc();
         size_t count = (size_t)DimsVectorUtils::Count(desc.dims);
         if (mat.GetDeviceType() != DEVICE_NAIVE && mat.GetDeviceType() != DEVICE_ROCM)
@@ -442,6 +443,7 @@ public:
     }
 
     Status ConvertToMatAsync(Mat &mat, MatConvertParam param, void *q) override {
+        RETURN_ON_NEQ(OnQueue(q), TNN_OK);
         auto &desc   = blob_->GetBlobDesc();
         size_t count = (size_t)DimsVectorUtils::Count(desc.dims);
         if ((size_t)DimsVectorUtils::Count(mat.GetDims()) != count)
@@ -534,6 +536,15 @@ public:
     }
 
 private:
+    // The buffers of this converter are ordered by the queue it works on.  A caller may come with another queue, while what it
+    // gave to the first one has yet to read them: the device is waited for (not the first queue, which may be gone by now).
+    // A program that keeps to one queue, as an Instance does, never pays for this.
+    Status OnQueue(void *q) {
+        if (q != queue_ && (stage_ || staging_ || bounce_ || params_))
+            ROCM_CALL(tnn_rocm_device_sync(q));
+        queue_ = q;
+        return TNN_OK;
+    }
     // ---- Mats whose memory is on this device (role of the DEVICE_CUDA branches of cuda_blob_converter.cc:62-81, 141-161):
     // nothing crosses the bus and nothing waits for the stream except the few bytes of scale and bias ----
     static bool IsFloatBlob(DataType t) { return t == DATA_TYPE_FLOAT || t == DATA_TYPE_HALF || t == DATA_TYPE_BFP16; }
@@ -819,6 +830,7 @@ private:
         return TNN_OK;
     }
     static constexpr size_t kMappedMaxBytes = 512u << 10;
+    void *queue_        = nullptr;  // the queue that the buffers below were last used on
     void *stage_        = nullptr;  // page-locked input slots
     size_t stage_slot_  = 0;        // bytes per slot
     size_t stage_slots_ = 0;
