@@ -92,7 +92,8 @@ TNN_ROCM_API int tnn_rocm_graph_destroy(void *graph_exec);
 enum {
     TNN_ROCM_EPI_NONE     = 0,
     TNN_ROCM_EPI_BIAS     = 1, /* + bias[N] (fp32 vector)                                     */
-    TNN_ROCM_EPI_GELU     = 2, /* erf GELU: 0.5*x*(erf(x*0.70710679)+1)  (cpu_gelu_layer_acc.cc:42-45) */
+    TNN_ROCM_EPI_GELU     = 2, /* erf GELU: 0.5*x*(erf(x*0.70710679)+1)  (cpu_gelu_layer_acc.cc:42-45); on fp32 sums within
+                                  an ulp of the exact function for |x| < 6, where the expression itself is 45 ulp away */
     TNN_ROCM_EPI_RESIDUAL = 4  /* + residual[M,N] (same dtype as C)                            */
 };
 

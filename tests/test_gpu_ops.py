@@ -83,6 +83,47 @@ def test_gelu_fp32(n):
     assert got[0] == 0 and got[1] == 0 and got[2] == np.inf and got[3] == 0 and got[4] == 40.0
 
 
+def test_gelu_of_fp32_products():
+    """The GELU of a product over its whole range, through one-hot weights (a sum is then one operand, exactly): within an ulp
+    of the exact function for |x| < 6, and the same bits in whole groups of eight columns, in the columns behind the last
+    group, on every tile shape and in the general kernel."""
+    from tnn_amd import capi
+    lib = capi.load()
+    say("gelu of fp32 products")
+    M, K = 4096, 64
+    x = np.concatenate([np.linspace(-9.5, 9.5, M * K - 4096), 10.0 ** np.linspace(-38, 0, 2048), -10.0 ** np.linspace(-38, 0, 2048)])
+    x = x.astype(np.float32).reshape(M, K)
+    x[0, :6] = 40, -40, 3e38, -3e38, 0, -0.0
+    eye = np.eye(K, dtype=np.float32)
+    o = ops()
+    got = host(o.gemm(dev(x), dev(eye), True, gelu=True))
+    for code in (-1, 9111141, 9111181, 3222121, 2222221):
+        lib.tnn_rocm_debug_set_gemm_config(code)
+        try:
+            assert np.array_equal(host(o.gemm(dev(x), dev(eye), True, gelu=True)), got), code
+            assert np.array_equal(host(o.gemm(dev(x), dev(eye[:60]), True, gelu=True)), got[:, :60]), code
+        finally:
+            lib.tnn_rocm_debug_set_gemm_config(0)
+    # K no multiple of four: the general kernel
+    assert np.array_equal(host(o.gemm(dev(x[:, :63]), dev(eye[:63, :63]), True, gelu=True)), got[:, :63])
+    half = x[:, :64].astype(np.float16)
+    a = host(o.gemm(dev(half), dev(eye.astype(np.float16)), True, gelu=True))
+    assert np.array_equal(host(o.gemm(dev(half), dev(eye[:60].astype(np.float16)), True, gelu=True)), a[:, :60], equal_nan=True)
+    x64 = x.astype(np.float64)
+    exact = 0.5 * x64 * torch.special.erfc(torch.from_numpy(-x64 / np.sqrt(2.0))).numpy()
+    near = np.abs(x64) < 6
+    ulp = np.spacing(np.abs(exact).astype(np.float32)).astype(np.float64)
+    worst = (np.abs(got - exact) / ulp)[near].max()
+    tail = (x64 <= -6) & (x64 > -9)
+    far = (np.abs(got - exact) / np.abs(exact))[tail].max()
+    say("  |x| < 6: %.3f ulp; -9 .. -6: %.3g relative" % (worst, far))
+    assert worst <= 1.0
+    assert (np.abs(got - exact) <= ulp)[x64 >= 6].all()
+    # half an ulp of the rounding, and a polynomial that is 2e-9 * a^2 / 16 off beyond a = 4
+    assert far <= 2.0 ** -24 + 2e-9 * 81 / 16
+    assert (np.abs(got - exact) <= 1.1e-18)[x64 <= -9].all()
+
+
 def test_tanh():
     say("tanh")
     x = np.concatenate([np.linspace(-12, 12, 4001), [0.0, 1e-8, -1e-8, 50.0, -50.0]]).astype(np.float32)

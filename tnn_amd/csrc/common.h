@@ -152,9 +152,9 @@ __device__ __forceinline__ float gelu_erf(float x) {
 // 1e-18 and a is clamped so the polynomial stays inside its fitted range).  Six fused multiply-adds, one clamp, one
 // exp2, one max and the final multiply-add: 13 issue slots against 19 for the rational form 7.1.26 of Abramowitz &
 // Stegun used before and ~40 for erff.  Against the correctly rounded fp16 result 0.4 % of the values differ, by one
-// ulp (2.8 % for the rational form).  fp32 outputs keep gelu_erf.
-// max(x, 0) is formed as x/2 + |x/2|: exact for every finite x (halving and the sum of equal or opposite halves do not
-// round), and unlike the maximum instruction, which returns its other operand for a NaN, it hands a NaN through, as the
+// ulp (2.8 % for the rational form).  fp32 products take gelu_erf_wide below, the fp32 layer gelu_erf above.
+// max(x, 0) is formed as x/2 + |x/2|: exact for every finite x above twice the smallest normal value (halving and the sum of
+// equal or opposite halves do not round there), and unlike the maximum instruction, which returns its other operand for a NaN, it hands a NaN through, as the
 // reference's GELU does (and gives NaN for -inf, where the reference's 0.5 x (erf + 1) is -inf times 0).  An overflow
 // upstream therefore stays visible in the output instead of turning into zeros.
 __device__ __forceinline__ float max_with_zero(float x) {
@@ -179,10 +179,10 @@ __device__ __forceinline__ float gelu_erf_fast(float x) {
 
 // The same function for fp32 results, without the double erf's branches and range reductions: Phi(-a) = 2^-q(a) as above, q as a
 // polynomial of degree 16 in a/4.5 - 1 (minimax fit on [0, 9], 2e-9 relative in Phi up to a = 4, growing as a^2 / 16 beyond,
-// where an ulp of x moves Phi by more), 2^f on [-1/2, 1/2] of degree 7 (4e-11), all in double: within 0.93 ulp of
-// the exact value for |x| < 6 (gelu_erf: 45 ulp, its x * 0.7071f is rounded to fp32).  31 instructions and no branch; in the
-// GEMM epilogue of [1536,768] x [768,3072] GELU took 30 of 82 us with gelu_erf and takes 5 with this.  Quantisers that must meet the
-// reference's bits keep gelu_erf.
+// where an ulp of x moves Phi by more), 2^f on [-1/2, 1/2] of degree 7 (4e-11), all in double: within 0.57 ulp of
+// the exact value for |x| < 6 (260 000 points) (gelu_erf: 45 ulp, its x * 0.7071f is rounded to fp32).  31 instructions and no branch; in the
+// GEMM epilogue of [1536,768] x [768,3072] GELU took 30 of 82 us with gelu_erf and takes 5 with this.  The stand-alone layer and
+// the int8 tables keep gelu_erf: what they write may go into a quantiser that has to meet the reference's bits.
 __device__ __forceinline__ float gelu_erf_wide(float x) {
     const float a  = __builtin_amdgcn_fmed3f(fabsf(x), 0.f, 9.0f);
     const double u = fma((double)a, 1.0 / 4.5, -1.0);
@@ -212,7 +212,8 @@ __device__ __forceinline__ float gelu_erf_wide(float x) {
     e             = fma(e, f, 0.24022651198159448);
     e             = fma(e, f, 0.6931471807284522);
     e             = fma(e, f, 0.9999999999616818);
-    return (float)fma(-(double)a, ldexp(e, -(int)n), (double)max_with_zero(x));
+    const double h = 0.5 * (double)x;  // max(x, 0) as above, in double: there half of the smallest floats is exact too
+    return (float)fma(-(double)a, ldexp(e, -(int)n), h + fabs(h));
 }
 
 __device__ __forceinline__ float wave_sum(float v) {

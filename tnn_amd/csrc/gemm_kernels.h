@@ -200,6 +200,11 @@ template <typename E, typename = void> struct SumBlocks : std::integral_constant
 template <typename E> struct SumBlocks<E, typename std::enable_if<E::kTakesRowSums>::type> : std::integral_constant<int, E::kSumBlocks> {};  // tile columns of a producer a consumer can add up (768 columns of 32)
 
 
+// GELU of a product, in every kernel and at every column the same function of the sum
+template <int DT> __device__ __forceinline__ float gelu_of_product(float v) {
+    return DT == TNN_ROCM_F32 ? gelu_erf_wide(v) : gelu_erf_fast(v);
+}
+
 template <int DT> struct FloatEpilogue : StoreThrough {
     typedef typename Elem<DT>::type T;
     static constexpr bool kRowStats = false;
@@ -222,7 +227,7 @@ template <int DT> struct FloatEpilogue : StoreThrough {
         if (flags & TNN_ROCM_EPI_BIAS)
             v = v + bias_n;
         if (flags & TNN_ROCM_EPI_GELU)
-            v = gelu_erf(v);
+            v = gelu_of_product<DT>(v);
         if (flags & TNN_ROCM_EPI_RESIDUAL)
             v = v + Elem<DT>::ld(&residual[(size_t)m * ldr + n]);
         Elem<DT>::st(&C[(size_t)m * ldc + n], v);
@@ -251,7 +256,7 @@ template <int DT> struct FloatEpilogue : StoreThrough {
         if (flags & TNN_ROCM_EPI_GELU) {
 #pragma unroll
             for (int t = 0; t < 8; ++t)
-                v[t] = (DT == TNN_ROCM_F32) ? gelu_erf_wide(v[t]) : gelu_erf_fast(v[t]);
+                v[t] = gelu_of_product<DT>(v[t]);
         }
         constexpr int NV = 8 * sizeof(T) / 16;  // 16-byte vectors per eight elements
         u32x4 packed[NV];
@@ -421,7 +426,7 @@ template <int DT, int SUMS = 0> struct LnFloatEpilogue : StoreThrough {
         if (flags & TNN_ROCM_EPI_GELU) {
 #pragma unroll
             for (int t = 0; t < 8; ++t)
-                v[t] = gelu_erf_fast(v[t]);
+                v[t] = gelu_of_product<DT>(v[t]);
         }
         // the two forms each end in their own conversion and store: joined behind the branch, the form without a
         // residual pays eight register copies per item for the join
@@ -529,7 +534,7 @@ template <int DT, bool SUMS = false> struct LnResidualEpilogue : StoreThrough {
         if (flags & TNN_ROCM_EPI_BIAS)
             v = v + bias_n;
         if (flags & TNN_ROCM_EPI_GELU)
-            v = gelu_erf(v);
+            v = gelu_of_product<DT>(v);
         const float2 s = st[m];
         const float mrs = s.y * s.x;
         v = v + (Elem<DT>::ld(&t[(size_t)m * ldc + n]) * s.x * gamma[n] + (beta[n] - mrs * gamma[n]));
@@ -559,7 +564,7 @@ template <int DT, bool SUMS = false> struct LnResidualEpilogue : StoreThrough {
         if (flags & TNN_ROCM_EPI_GELU) {
 #pragma unroll
             for (int q = 0; q < 8; ++q)
-                v[q] = gelu_erf_fast(v[q]);
+                v[q] = gelu_of_product<DT>(v[q]);
         }
         T *pe = reinterpret_cast<T *>(&packed);
         const float mrs = s.y * s.x;
@@ -1922,10 +1927,16 @@ __global__ void __launch_bounds__(CFG::NT)
                     else
                         epi.store8(m, n, v);
                 } else {
-#pragma unroll
+                    // the last columns one at a time, from LDS again: eight copies of the epilogue were a third of the library
+#pragma unroll 1
                     for (int t = 0; t < 8; ++t)
-                        if (n + t < N)
-                            epi.store(m, n + t, v[t], epi.col_const(n + t));
+                        if (n + t < N) {
+                            AccT x = src[t];
+#pragma unroll
+                            for (int q = 1; q < WGK; ++q)
+                                x += src[q * (32 * SSTR) + t];
+                            epi.store(m, n + t, x, epi.col_const(n + t));
+                        }
                 }
             }
         }
