@@ -388,13 +388,15 @@ TNN_ROCM_API int tnn_rocm_gelu_i8(void *stream, const int8_t *q_in, float in_sca
  *                   blocks; 3 = never that one
  *   store_through : 1 (default) = GEMM and attention results are stored through the L2 at device scope, so that no
  *                   dirty lines wait for the write-back at the end of the kernel; 0 = ordinary write-back stores.
- *                   Read by the kernels when they run (recorded graphs follow it too); waits for the device first. */
+ *                   Goes into a launch when it is made: a graph recorded through tnn_rocm_graph_* keeps the form it was
+ *                   recorded with, an Instance records again.  The call waits for the device first. */
 TNN_ROCM_API int tnn_rocm_debug_set_gemm_config(int cfg);
 TNN_ROCM_API int tnn_rocm_debug_set_gemm_tune(const char *spec);
 TNN_ROCM_API int tnn_rocm_debug_set_gemm_group_m(int group_m);
 TNN_ROCM_API int tnn_rocm_debug_set_ln_y_ahead(int on);
 TNN_ROCM_API int tnn_rocm_debug_set_attention_dma(int on);
 TNN_ROCM_API int tnn_rocm_debug_set_store_through(int on);
+TNN_ROCM_API int tnn_rocm_debug_store_through(void); /* the switch as it stands */
 
 #ifdef __cplusplus
 }

@@ -239,6 +239,37 @@ def test_graph_replay_matches_eager_on_every_replay(monkeypatch):
     default.close()
 
 
+def test_recorded_forwards_follow_the_store_switch(monkeypatch, capfd):
+    """The form of the result stores is an argument of every launch: an instance that replays recorded forwards records again
+    when the switch is set, and finds its recording when it is set back."""
+    host, tnnmodel, EncoderConfig, make_weights, make_inputs = _mods()
+    from tnn_amd import capi
+    lib = capi.load()
+    say("host: store switch and graph replay")
+    cfg, B, S = EncoderConfig.bert_base(1), 1, 64
+    g = tnnmodel.encoder_graph(cfg, make_weights(cfg, seed=13, bias_std=0.02), B, S)
+    monkeypatch.setenv("TNN_ROCM_GRAPH", "1")
+    monkeypatch.setenv("TNN_ROCM_VERBOSE", "1")
+    inst = host.RocmInstance.from_graph(g, "fp16")
+    ids, seg, lens, mask = make_inputs(cfg, B, S, 20, S, seed=100)
+    for n, v in (("input_ids", ids), ("token_type_ids", seg), ("attention_bias", mask.reshape(B, 1, 1, S))):
+        inst.set_input(n, v)
+    capfd.readouterr()
+    outs, recorded = [], []
+    try:
+        for through in (1, 0, 1, 0):
+            assert lib.tnn_rocm_debug_set_store_through(through) == 0
+            for _ in range(4):
+                inst.forward()
+            outs.append(inst.output("last_hidden").copy())
+            recorded.append(capfd.readouterr().err.count("forward recorded"))
+    finally:
+        lib.tnn_rocm_debug_set_store_through(1)
+    assert recorded == [1, 1, 0, 0]
+    assert all(np.array_equal(o, outs[0]) for o in outs)
+    inst.close()
+
+
 def test_two_instances_on_two_threads_match_their_sequential_results():
     """One Context per Instance, instances used from different threads at the same time (the engine's threading
     contract, source/tnn/core/instance.cc and default_network.cc:632-633: all work of an instance on its own stream,

@@ -1254,7 +1254,11 @@ def test_store_through_switch_changes_no_result():
         return out
 
     try:
-        assert lib.tnn_rocm_debug_set_store_through(0) == 0
+        big = torch.randn(8192, 8192, device="cuda")
+        for _ in range(4):
+            big = torch.tanh(big @ big)
+        assert lib.tnn_rocm_debug_set_store_through(0) == 0 and lib.tnn_rocm_debug_store_through() == 0
+        assert torch.cuda.current_stream().query()  # the call has waited for what was running
         back = run()
     finally:
         assert lib.tnn_rocm_debug_set_store_through(1) == 0

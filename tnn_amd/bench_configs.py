@@ -9,7 +9,8 @@
 
   stores  the headline forward (12-layer BERT-base fp16, B8 S384) with the results of the GEMM / attention / LayerNorm
           kernels stored through the L2 at device scope (the default) against ordinary write-back stores: one instance,
-          one recorded graph, the switch (tnn_rocm_debug_set_store_through) flipped between timing rounds
+          the switch (tnn_rocm_debug_set_store_through) flipped between timing rounds; with TNN_ROCM_GRAPH=1 one recorded
+          graph per form
 
 Every configuration runs Instance::Forward on DEVICE_ROCM from .tnnproto/.tnnmodel bytes built in memory (synthetic
 weights and inputs, seeded), prints one JSON line and needs the built libraries; nothing falls back to the CPU."""

@@ -203,10 +203,16 @@ int tnn_rocm_event_record(void *event, void *stream) {
     return 0;
 }
 
-__attribute__((visibility("default"))) int tnn_rocm_debug_set_store_through(int on) {
+int tnn_rocm_debug_set_store_through(int on) {
+    int devices = 0;
+    tnn_rocm_device_count(&devices);
+    if (devices > 0)
+        TR_CHECK_HIP(hipDeviceSynchronize());
     g_store_through = on ? 1 : 0;
     return 0;
 }
+
+int tnn_rocm_debug_store_through(void) { return g_store_through; }
 
 int tnn_rocm_event_elapsed_ms(void *start, void *stop, float *ms) {
     TR_REQUIRE(start && stop && ms, TNN_ROCM_EINVAL, "event_elapsed_ms: null argument");

@@ -1,5 +1,6 @@
 #include "rocm_network.h"
 
+#include <cstdio>
 #include <cstdlib>
 
 namespace TNN_NS {
@@ -38,6 +39,7 @@ void RocmNetwork::Signature(std::vector<uint64_t> *sig) {
     sig->clear();
     auto rocm = dynamic_cast<RocmContext *>(context_);
     sig->push_back(rocm ? rocm->MemoryEpoch() : 0);
+    sig->push_back((uint64_t)tnn_rocm_debug_store_through());  // an argument of the recorded launches
     for (auto layer : layers_) {
         const std::vector<Blob *> ins = layer->GetInputBlobs(), outs = layer->GetOutputBlobs();
         for (auto blobs : {&ins, &outs})
@@ -291,6 +293,8 @@ Status RocmNetwork::ForwardAsync(Callback call_back) {
     r.signature = sig;
     r.exec      = exec;
     recordings_.push_back(r);
+    if (getenv("TNN_ROCM_VERBOSE"))
+        fprintf(stderr, "tnn-rocm: forward recorded, %zu kept\n", recordings_.size());
     if (tnn_rocm_graph_launch(exec, stream) != 0)
         return Status(TNNERR_CUDA_KERNEL_LAUNCH_ERROR, std::string("graph launch failed: ") + tnn_rocm_last_error());
     return TNN_OK;

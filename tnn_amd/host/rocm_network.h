@@ -71,8 +71,8 @@ private:
     Status ReshapeGroups();
     std::vector<Group> groups_;
 #endif
-    // Everything a recording depends on: dims and device address of every blob the layers touch, and the context's
-    // scratch allocation count.  A recording is replayed only under the signature it was made with, so a Reshape, a
+    // Everything a recording depends on: dims and device address of every blob the layers touch, the context's scratch
+    // allocation count and the form of the result stores.  A recording is replayed only under the signature it was made with, so a Reshape, a
     // re-planned blob pool or a grown workspace lead back to eager passes and a new recording by themselves.
     void Signature(std::vector<uint64_t> *sig);
     void DropGraphs();
