@@ -1108,6 +1108,33 @@ def test_instances_come_and_go_without_leaving_memory_behind(precision):
     assert host1 - host0 <= 4 << 20, (host0, host1)   # one instance of this model holds far more than that
 
 
+def test_an_fp32_net_holds_its_weights_once():
+    """The attention groups of an fp32 net and the layers they stand for (which ForwardWithCallback still runs) share one set of
+    projection weights on the device; projections without a bias among them."""
+    host, tnnmodel, EncoderConfig, make_weights, _ = _mods()
+    say("host: device memory of an fp32 net")
+    cfg = EncoderConfig(4, 1024, 16, 1024)
+    w = make_weights(cfg, seed=11, with_embeddings=False)
+    g = tnnmodel.encoder_graph(cfg, w, 1, 32, with_embeddings=False)
+    weights = sum(a.nbytes for lw in w["layers"] for a in lw.values())
+    host.RocmInstance.from_graph(g, "fp32").close()  # what the runtime keeps for itself
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    inst = host.RocmInstance.from_graph(g, "fp32")
+    held = free - torch.cuda.mem_get_info()[0]
+    say("  weights %.1f MiB, instance %.1f MiB" % (weights / 2 ** 20, held / 2 ** 20))
+    # twice the Q, K and V weights would be half as much again; blobs of 32 tokens are small, and every matrix is whole 2 MiB pieces
+    assert weights <= held <= 1.25 * weights
+    x = np.random.default_rng(3).standard_normal((1, 32, 1024)).astype(np.float32)
+    inst.set_input("hidden", x)
+    inst.set_input("attention_bias", np.zeros((1, 1, 1, 32), np.float32))
+    inst.forward()
+    got = inst.output("last_hidden").copy()
+    inst.forward_with_callback(after=lambda name, typ, blobs: None)
+    assert rel_err(got, inst.output("last_hidden")) <= 3e-6
+    inst.close()
+
+
 def _bf16_bits(x32):
     """float32 -> bfloat16 bit patterns, round to nearest even (finite values)"""
     u = np.ascontiguousarray(x32, np.float32).view(np.uint32).astype(np.uint64)

@@ -2,6 +2,7 @@
 #include "rocm_device.h"
 #include <immintrin.h>
 
+#include <algorithm>
 #include <cstdint>
 #include <cstdio>
 
@@ -252,6 +253,14 @@ static TypeDeviceRegister<RocmDevice> g_rocm_device_register(DEVICE_ROCM);
 RocmLayerAcc::~RocmLayerAcc() {
     for (void *p : owned_device_)
         tnn_rocm_free(p);
+}
+Status RocmLayerAcc::ReleaseOwned(void *ptr) {
+    auto it = std::find(owned_device_.begin(), owned_device_.end(), ptr);
+    if (ptr && it != owned_device_.end()) {
+        owned_device_.erase(it);
+        ROCM_CALL(tnn_rocm_free(ptr));
+    }
+    return TNN_OK;
 }
 Status RocmLayerAcc::Init(Context *context, LayerParam *param, LayerResource *resource,
                           const std::vector<Blob *> &inputs, const std::vector<Blob *> &outputs) {

@@ -148,6 +148,8 @@ protected:
     virtual DataType ConstantBlobDataType(const std::vector<Blob *> &inputs, int index);
     // device copy of host data converted from src_type to dst_type (fp32 -> fp16/bf16 on device); owned by the acc
     Status UploadConverted(const void *host, size_t count, DataType src_type, DataType dst_type, void **out);
+    // frees a device buffer this acc owns; one it does not own is left alone
+    Status ReleaseOwned(void *ptr);
     void *Stream() { return context_->Stream(); }
     // the blob an input resolves to: this acc's device copy for constants, the blob itself otherwise
     Blob *In(Blob *b) {

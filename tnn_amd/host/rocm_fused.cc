@@ -468,8 +468,9 @@ public:
                                          return HeadSplitSource(gi, blob, o4, o3, chain, shape);
                                      });
             RocmLayerGroup group;
-            if (!matcher.Match(g, si, &m) || !MakeAttention(m, L[si]->name, &group.layer, &group.resource))
+            if (!matcher.Match(g, si, &m) || !MakeAttention(m, L[si]->name, false, &group.layer, &group.resource))
                 continue;
+            group.projections[0] = m.lq, group.projections[1] = m.lk, group.projections[2] = m.lv;
             group.first = *std::min_element(m.chain.begin(), m.chain.end());
             group.last  = *std::max_element(m.chain.begin(), m.chain.end());
             // The memory plan is that of the single layers: nothing else may run between the first and the last of them,
@@ -765,7 +766,9 @@ private:
 
     // the fused layer and its resource (three projections side by side) for a matched attention core; false where the fused
     // kernels do not serve the core's sizes
-    bool MakeAttention(const AttentionCore &m, const std::string &name, std::shared_ptr<LayerInfo> *layer,
+    // pack: the resource holds the three projections' weights one behind the other; else only their dims, and the acc gets
+    // the weights from the projections' accs (RocmShareProjections)
+    bool MakeAttention(const AttentionCore &m, const std::string &name, bool pack, std::shared_ptr<LayerInfo> *layer,
                        std::shared_ptr<LayerResource> *resource) {
         auto &L = structure_->layers;
         const std::string &mask = m.mask;
@@ -810,10 +813,10 @@ private:
         fp->seq_len  = seq > 0 ? seq : 0;
         auto fr       = std::make_shared<RocmFusedLinearResource>();
         fr->name      = fl->name;
-        fr->weight_nk = RawBuffer(3 * H * K * 4, {3 * H, K});
-        fr->bias      = RawBuffer(3 * H * 4, {3 * H});
+        fr->weight_nk = RawBuffer(pack ? 3 * H * K * 4 : 0, {3 * H, K});
+        fr->bias      = RawBuffer(pack ? 3 * H * 4 : 0, {3 * H});
         RocmFusedLinearResource *src[3] = {rq, rk, rv};
-        for (int t = 0; t < 3; ++t) {
+        for (int t = 0; t < 3 && pack; ++t) {
             memcpy(fr->weight_nk.force_to<float *>() + (size_t)t * H * K, src[t]->weight_nk.force_to<float *>(),
                    (size_t)H * K * 4);
             if (src[t]->bias.GetDataCount() == H)
@@ -844,7 +847,7 @@ private:
                     continue;
                 std::shared_ptr<LayerInfo> fl;
                 std::shared_ptr<LayerResource> fr;
-                if (!MakeAttention(m, sm->name, &fl, &fr))
+                if (!MakeAttention(m, sm->name, true, &fl, &fr))
                     continue;
                 const int first = *std::min_element(m.chain.begin(), m.chain.end());
                 resource_->resource_map[fl->name] = fr;
@@ -1670,6 +1673,19 @@ public:
         return TNN_OK;
     }
 
+    const void *Weight() const { return weight_; }
+    const void *Bias() const { return bias_; }
+    // weight and bias lie in memory of another acc from now on
+    Status LieIn(void *weight, void *bias) {
+        RETURN_ON_NEQ(ReleaseOwned(weight_), TNN_OK);
+        weight_ = weight;
+        if (!bias_)
+            return TNN_OK;
+        RETURN_ON_NEQ(ReleaseOwned(bias_), TNN_OK);
+        bias_ = bias;
+        return TNN_OK;
+    }
+
 private:
     void *weight_ = nullptr, *bias_ = nullptr, *colsum_ = nullptr, *gamma_ = nullptr, *beta_ = nullptr, *res_gamma_ = nullptr,
          *res_beta_ = nullptr;
@@ -1845,6 +1861,26 @@ public:
         return TNN_OK;
     }
 
+    // Q, K and V weights of fp32 projections that exist already: packed here, and shared with them
+    Status TakeProjections(RocmFusedLinearLayerAcc *const (&from)[3]) {
+        auto p         = dynamic_cast<RocmFusedAttentionParam *>(param_);
+        const size_t h = (size_t)p->heads * p->head_dim, wb = h * h * sizeof(float), bb = h * sizeof(float);
+        for (void **to : {&weight_, &bias_}) {
+            ROCM_CALL(tnn_rocm_malloc(to, 3 * (to == &weight_ ? wb : bb)));
+            owned_device_.push_back(*to);
+        }
+        ROCM_CALL(tnn_rocm_memset(bias_, 0, 3 * bb, Stream()));
+        for (int t = 0; t < 3; ++t) {
+            ROCM_CALL(tnn_rocm_memcpy_d2d((char *)weight_ + t * wb, from[t]->Weight(), wb, Stream()));
+            if (from[t]->Bias())
+                ROCM_CALL(tnn_rocm_memcpy_d2d((char *)bias_ + t * bb, from[t]->Bias(), bb, Stream()));
+        }
+        ROCM_CALL(tnn_rocm_stream_sync(Stream()));
+        for (int t = 0; t < 3; ++t)
+            RETURN_ON_NEQ(from[t]->LieIn((char *)weight_ + t * wb, (char *)bias_ + t * bb), TNN_OK);
+        return TNN_OK;
+    }
+
 private:
     void *weight_ = nullptr, *bias_ = nullptr, *scale_ = nullptr, *dequant_ = nullptr, *colsum_ = nullptr, *gamma_ = nullptr,
          *beta_ = nullptr;
@@ -1852,6 +1888,17 @@ private:
     bool mask_one_row_ = false;
 };
 REGISTER_ROCM_ACC(RocmFusedAttentionLayerAcc, LAYER_ROCM_FUSED_ATTENTION);
+
+Status RocmShareProjections(AbstractLayerAcc *attention, AbstractLayerAcc *const projections[3]) {
+    auto att = dynamic_cast<RocmFusedAttentionLayerAcc *>(attention);
+    RocmFusedLinearLayerAcc *from[3];
+    for (int t = 0; t < 3; ++t) {
+        from[t] = dynamic_cast<RocmFusedLinearLayerAcc *>(projections[t]);
+        if (!att || !from[t] || !from[t]->Weight())
+            return Status(TNNERR_NULL_PARAM, "attention group: a projection without weights");
+    }
+    return att->TakeProjections(from);
+}
 
 // ---- RocmFusedEmbedding ----------------------------------------------------------------------------------------
 class RocmFusedEmbeddingLayerAcc : public RocmLayerAcc {

@@ -84,6 +84,10 @@ Status RocmNetwork::Init(NetworkConfig &net_config, ModelInterpreter *interprete
             continue;
         g.acc->SetConstantResource(&resource_.constant_map);
         RETURN_ON_NEQ(g.acc->Init(context_, g.layer->param.get(), g.resource.get(), g.inputs, g.outputs), TNN_OK);
+        AbstractLayerAcc *projections[3];
+        for (int t = 0; t < 3; ++t)
+            projections[t] = layers_[found.projections[t]]->layer_acc_;
+        RETURN_ON_NEQ(RocmShareProjections(g.acc.get(), projections), TNN_OK);
         groups_.push_back(std::move(g));
     }
     return ReshapeGroups();

@@ -23,11 +23,15 @@ namespace TNN_NS {
 // the single layers; what lies between the group's inputs and its output is simply not written.
 struct RocmLayerGroup {
     int first = 0, last = 0;
+    int projections[3] = {0, 0, 0};    // the layers that make Q, K and V
     std::shared_ptr<LayerInfo> layer;  // type, inputs, output and parameters of the acc that stands for the group
     std::shared_ptr<LayerResource> resource;
 };
 // the attention cores (projections included) that an fp32 net keeps as layers
 std::vector<RocmLayerGroup> RocmFindAttentionGroups(NetStructure *structure, NetResource *resource);
+// One set of weights for a group and its layers: the attention acc packs the device weights of the three projections, and
+// the projections' accs go on with the packed ones.  The attention acc must outlive any Forward of theirs.
+Status RocmShareProjections(AbstractLayerAcc *attention, AbstractLayerAcc *const projections[3]);
 
 class RocmNetwork : public DefaultNetwork {
 public:

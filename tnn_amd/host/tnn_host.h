@@ -666,6 +666,7 @@ public:
 
 protected:
     friend class DefaultNetwork;  // this host's Reshape infers every shape before it touches blob memory
+    friend class RocmNetwork;     // gives layers that it runs as a group one set of weights
     // base_layer.h:101-105
     virtual Status InferOutputShape(bool ignore_error = false);
     virtual Status InferOutputDataType();
