@@ -12,6 +12,10 @@
           the switch (tnn_rocm_debug_set_store_through) flipped between timing rounds; with TNN_ROCM_GRAPH=1 one recorded
           graph per form
 
+  tiles   every tile shape of the GEMM kernel in the place of the one the library picks, one projection of the encoder at a
+          time, inside the forward: --precision fp16 | bf16 | fp32 | int8, --batch, --seq, --layers, --large; "us" is what a
+          launch of that projection gains (-) or loses, median over rounds that alternate with the library's own choice
+
 Every configuration runs Instance::Forward on DEVICE_ROCM from .tnnproto/.tnnmodel bytes built in memory (synthetic
 weights and inputs, seeded), prints one JSON line and needs the built libraries; nothing falls back to the CPU."""
 import argparse
@@ -178,15 +182,61 @@ def stores(args):
             "outputs_identical": bool(np.array_equal(outs[0], outs[1]))}
 
 
+# configuration codes of the tiled GEMM kernel, tnn_rocm_debug_set_gemm_config
+TILE_CODES = {"half": (9111141, 9121141, 3112221, 3112222, 3212221, 4221141, 2112211, 2222221, 3332221, 3331182),
+              "fp32": (9111141, 9121141, 9111181, 9221141, 9321140, 3231142, 2331142, 3222121, 2222221)}
+
+
+def tiles(args):
+    from . import capi
+    lib = capi.load()
+    cfg = (EncoderConfig.bert_large if args.large else EncoderConfig.bert_base)(args.layers or (4 if args.large else 12))
+    B, S = args.batch or 8, args.seq or 384
+    w = make_weights(cfg, seed=20240601)
+    if args.precision == "int8":
+        scales = {n: 0.05 for n in quant.calibration_outputs(cfg)}
+        inst = host.RocmInstance.from_graph(quant.int8_encoder_graph(cfg, w, scales, B, S), "fp16")
+    else:
+        inst = host.RocmInstance.from_graph(tnnmodel.encoder_graph(cfg, w, B, S), args.precision)
+    ids, seg, lens, mask = make_inputs(cfg, B, S, max(1, S // 2), S, seed=20240602)
+    for name, value in (("input_ids", ids), ("token_type_ids", seg), ("attention_bias", mask.reshape(B, 1, 1, S))):
+        inst.set_input(name, value)
+    H, F = cfg.hidden, cfg.ffn
+    size = {"fp32": 4, "int8": 1}.get(args.precision, 2)
+    found = {"config": "tiles", "workload": "%d-layer encoder %s, hidden %d, B%d S%d" % (cfg.layers, args.precision, H, B, S)}
+    rounds = 7
+    _time_forward(inst, args.steps)
+    for proj, n, k in (("qkv", 3 * H, H), ("out", H, H), ("ffn1", F, H), ("ffn2", H, F)):
+        codes = [c for c in TILE_CODES["fp32" if args.precision == "fp32" else "half"] if k * size % (64 << c % 10) == 0]
+        diff = {c: [] for c in codes}
+        try:
+            for _ in range(rounds):
+                for c in codes:
+                    ms = []
+                    for spec in (b"", b"%d:%d:%d" % (n, k, c)):
+                        inst.sync()
+                        lib.tnn_rocm_debug_set_gemm_tune(spec)
+                        ms.append(_time_forward(inst, args.steps, warmup=3))
+                    diff[c].append((ms[1] - ms[0]) * 1e6 / cfg.layers)
+        finally:
+            lib.tnn_rocm_debug_set_gemm_tune(b"")
+        found[proj] = {str(c): round(sorted(d)[rounds // 2], 2) for c, d in sorted(diff.items(), key=lambda e: sorted(e[1])[rounds // 2])}
+        print("%s %dx%dx%d: %s" % (proj, B * S, n, k, found[proj]), flush=True)
+    inst.close()
+    return found
+
+
 def main():
     ap = argparse.ArgumentParser(description=__doc__, formatter_class=argparse.RawDescriptionHelpFormatter)
-    ap.add_argument("--config", choices=["c1", "c3", "c4", "c5", "stores"], required=True)
+    ap.add_argument("--config", choices=["c1", "c3", "c4", "c5", "stores", "tiles"], required=True)
     ap.add_argument("--steps", type=int, default=20)
     ap.add_argument("--layers", type=int, default=0, help="fewer layers than the configuration names (c4, c5)")
-    ap.add_argument("--batch", type=int, default=0, help="c3: batch instead of 32")
-    ap.add_argument("--seq", type=int, default=0, help="c3: sequence length instead of 512")
+    ap.add_argument("--batch", type=int, default=0, help="c3: batch instead of 32; tiles: instead of 8")
+    ap.add_argument("--seq", type=int, default=0, help="c3: sequence length instead of 512; tiles: instead of 384")
+    ap.add_argument("--precision", choices=["fp16", "bf16", "fp32", "int8"], default="fp16", help="tiles")
+    ap.add_argument("--large", action="store_true", help="tiles: BERT-large, four layers")
     args = ap.parse_args()
-    print(json.dumps({"c1": c1, "c3": c3, "c4": c4, "c5": c5, "stores": stores}[args.config](args)))
+    print(json.dumps({"c1": c1, "c3": c3, "c4": c4, "c5": c5, "stores": stores, "tiles": tiles}[args.config](args)))
 
 
 if __name__ == "__main__":

@@ -185,11 +185,92 @@ def mall_probe(launches=20):
     return rows
 
 
+# (code, rows, columns, tiles a CU holds at once) of the shapes the launcher chooses from, see TileCost in csrc/gemm_kernels.h
+TILE_SHAPES = {
+    "half": ((9111141, 32, 32, 2), (9121141, 32, 64, 1), (3112221, 64, 64, 3), (3112222, 64, 64, 1), (3212221, 128, 64, 2),
+             (4221141, 64, 64, 2), (2112211, 64, 64, 4), (2222221, 128, 128, 2), (3332221, 192, 192, 1), (3331182, 96, 96, 1)),
+    "f32": ((9111141, 32, 32, 2), (9121141, 32, 64, 1), (9111181, 32, 32, 1), (9221141, 64, 64, 1), (9321140, 96, 64, 1),
+            (3231142, 64, 96, 1), (2331142, 96, 96, 1), (3222121, 128, 64, 2), (2222221, 128, 128, 1))}
+
+
+def tile_sweep(dtype, report):
+    """Every tile shape of the GEMM kernel over the launches of an encoder: the four projections with their fused epilogues,
+    M from 16 tokens on, twelve weight sets in turn (inside a network a layer's weights come from the memory-side cache).
+    Reports per launch how far the shape the library picks is behind the best one, and per shape the least-squares fit of the
+    cost model TileCost to its launches, as a row of its table."""
+    import numpy as np
+    lib = capi.load()
+    shapes = TILE_SHAPES["f32" if dtype == "f32" else "half"]
+    td, size = {"f16": (torch.float16, 2), "i8": (torch.int8, 1), "f32": (torch.float32, 4)}[dtype]
+    ms = (16, 32, 64, 100, 128, 197, 256, 384, 512, 700, 1000, 1536, 2000, 3072) + (() if dtype == "f32" else (4096, 8192))
+    seen, behind = {s[0]: [] for s in shapes}, []
+
+    def launches(M, N, K, proj):
+        a = _randi8((M, K)) if dtype == "i8" else _randn((M, K), td)
+        ws = [_randi8((N, K)) if dtype == "i8" else _randn((N, K), td) * 0.02 for _ in range(12)]
+        bias, col = torch.zeros(N, device="cuda"), torch.ones(N, device="cuda")
+        B, heads = 1, N // 192
+        if dtype == "i8":
+            ib, sc, res = torch.zeros(N, dtype=torch.int32, device="cuda"), torch.full((N,), 1e-3, device="cuda"), _randn((M, N), torch.float16)
+            lut = _randi8((256,))
+            if proj == "qkv" and M % 8 == 0:
+                return lambda w: ops.gemm_i8_qkv_split(a, w, ib, sc, col, B, M, heads, dtype=torch.float16), ws
+            if proj == "ffn1":
+                return lambda w: ops.gemm_i8_lut(a, w, ib, sc, lut), ws
+            return lambda w: ops.gemm_i8_dequant_residual(a, w, ib, sc, 0.03, residual=res, dtype=torch.float16), ws
+        res = _randn((M, N), td) if proj in ("out", "ffn2") else None
+        if dtype == "f32" or proj == "qkv" and M % 8:
+            return lambda w: ops.gemm(a, w, True, bias=bias, gelu=proj == "ffn1", residual=res), ws
+        if proj == "qkv":
+            return lambda w: ops.qkv_split_ln(a, w, bias, col, 1e-5, B, M, heads, want_stats=True), ws
+        if proj == "ffn1":
+            return lambda w: ops.gemm_ln(a, w, bias, col, 1e-5, gelu=True, want_stats=True), ws
+        stats = torch.ones(M, 2, device="cuda")
+        sums = torch.zeros(ops.MAX_ROW_SUM_BLOCKS, M, 2, device="cuda")
+        return lambda w: ops.gemm_residual_ln(a, w, res, stats, col, bias, bias=bias, want_row_sums=True, row_sums_out=sums), ws
+
+    for H in (768,) if dtype == "f32" else (768, 1024):
+        for proj, N, K in (("qkv", 3 * H, H), ("out", H, H), ("ffn1", 4 * H, H), ("ffn2", H, 4 * H)):
+            for M in ms:
+                fn, ws = launches(M, N, K, proj)
+                codes = [s[0] for s in shapes if K * size % (64 << s[0] % 10) == 0]
+                us = {}
+                for code in [0] + codes:
+                    lib.tnn_rocm_debug_set_gemm_config(code)
+                    try:
+                        us[code] = _time_us(lambda: [fn(w) for w in ws], 2) / len(ws)
+                    finally:
+                        lib.tnn_rocm_debug_set_gemm_config(0)
+                for code in codes:
+                    seen[code].append((M, N, K * size / 128.0, us[code]))
+                best = min(codes, key=lambda c: us[c])
+                behind.append(us[0] / us[best] - 1)
+                report("%-4s %5d x %4d x %4d  picked %6.2f us, best %6.2f (%d)  %s" % (
+                    proj, M, N, K, us[0], us[best], best, " ".join("%d:%.2f" % (c, us[c]) for c in codes)))
+    report("the pick is %.1f %% behind the best shape on average, %.1f %% at worst" % (100 * np.mean(behind), 100 * np.max(behind)))
+    for code, bm, bn, slots in shapes:
+        rows, want = [], []
+        for M, N, slabs, us in seen[code]:
+            n = -(-(-(-M // bm) * -(-N // bn)) // 256)
+            sets, rest = n // slots, n % slots
+            row = [1.0, float(sets + (rest > 0) - 1)] + [0.0] * slots
+            row[1 + slots] += slabs * sets
+            if rest:
+                row[1 + rest] += slabs
+            rows.append([v / us for v in row])  # relative errors count
+            want.append(1.0)
+        fit, left = np.linalg.lstsq(np.array(rows), np.array(want), rcond=None)[:2]
+        err = np.abs(np.array(rows) @ fit - 1).mean()
+        report("    {%d, %d, %d, %d, %.2ff, %.2ff, {%s}},  // %.1f %% off on average" % (
+            code, bm, bn, slots, fit[0], fit[1], ", ".join("%.3ff" % v for v in fit[2:]), 100 * err))
+
+
 def main():
     ap = argparse.ArgumentParser()
     ap.add_argument("--mall-probe", action="store_true", help="projection GEMMs with resident / evicted operands")
     ap.add_argument("--simd-probe", action="store_true",
                     help="build (if missing) and run the stand-alone SIMD micro-benchmark csrc/probe_simd.hip")
+    ap.add_argument("--tile-sweep", choices=["f16", "i8", "f32"], help="GEMM tile shapes over the launches of an encoder")
     ap.add_argument("--build-only", action="store_true", help="with --simd-probe: compile it, do not run it")
     ap.add_argument("--launches", type=int, default=20)
     ap.add_argument("--only", default="")
@@ -204,6 +285,9 @@ def main():
             build.build_simd_probe()
         if not a.build_only:
             sys.exit(subprocess.call([exe]))
+        return
+    if a.tile_sweep:
+        tile_sweep(a.tile_sweep, lambda text: print(text, flush=True))
         return
     if a.mall_probe:
         for r in mall_probe(a.launches):

@@ -2073,11 +2073,13 @@ constexpr int kNumCU = 256;
 // What a launch takes on this chip with each tile shape.  The busiest CU works through n = ceil(tiles / 256) tiles, up to
 // `slots` of them side by side (what its LDS and registers hold): full sets of `slots`, then the rest.  A set costs its
 // number of 128-byte k-slabs times slab[its tiles - 1], every set after the first also `round` (ramp and epilogue that
-// nothing covers), and the launch `fixed`; microseconds.  The figures are a least-squares fit to 800 launches (fp16 and int8:
-// M from 16 to 8192, the four projections of hidden sizes 768 and 1024 with their fused epilogues; fp32: M from 16 to
-// 3072), taken over twelve weight sets in turn so that weights come from the memory-side cache as they do inside a
-// network.  The shape it picks is on average 1.4 % (fp16), 0.6 % (int8), 2.7 % (fp32) behind the best of the shapes for the
-// same launch; the rules it replaced, made for M >= 1024, were 51 %, 34 % and 77 % behind over that range:
+// nothing covers), and the launch `fixed`; microseconds.  The figures are a least-squares fit to some 800 launches (fp16 and
+// int8: M from 16 to 8192, the four projections of hidden sizes 768 and 1024 with their fused epilogues; fp32: M from 16 to
+// 3072), taken over twelve weight sets in turn so that weights come from the memory-side cache as they do inside a network:
+// python -m tnn_amd.bench_ops --tile-sweep measures them and fits the rows.  A single launch is 4 .. 10 % off its prediction,
+// so picks closer than that are as good as drawn; taken together the picks are 1.5 % (fp16), 1.1 % (int8), 2.9 % (fp32) behind
+// the best shape of each launch back to back, and 0.31, 0.21 and 0.60 us inside the network (bench_configs --config tiles;
+// profiles/gemm_tile_choice.txt).  The rules this replaced, made for M >= 1024, were 51 %, 34 % and 77 % behind over that range:
 //   M=  32 N= 768 K=3072 fp16  23.1 -> 7.3 us   (64x64 tiles: 12 CUs, one two-stage slab after another)
 //   M= 256 N= 768 K=3072 fp16  23.7 -> 7.2      M= 256 N=2304 K=768 fp16  8.7 -> 6.2
 //   M=1000 N= 768 K=3072 fp16  24.3 -> 12.4     M=1000 N= 768 K=768 fp16  8.7 -> 5.5
@@ -2097,6 +2099,8 @@ constexpr TileCost kTilesHalf[] = {
     {3332221, 192, 192, 1, 10.15f, 13.25f, {0.767f}},
     {3331182, 96, 96, 1, 6.94f, 7.10f, {0.264f}},
 };
+// (int8, 64x64 tiles: the slab of four tiles was fitted to 0.944; 4096 x 2304 x 768 then took 128x128 tiles, 1.4 % ahead by the
+// fit and 0 .. 1 us a launch behind in the network)
 constexpr TileCost kTilesI8[] = {
     {9111141, 32, 32, 2, 2.98f, 1.93f, {0.078f, 0.151f}},
     {9121141, 32, 64, 1, 3.25f, 2.21f, {0.130f}},
@@ -2104,16 +2108,16 @@ constexpr TileCost kTilesI8[] = {
     {3112222, 64, 64, 1, 3.09f, 2.21f, {0.196f}},
     {3212221, 128, 64, 2, 4.05f, 3.04f, {0.313f, 0.644f}},
     {4221141, 64, 64, 2, 4.06f, 2.67f, {0.174f, 0.389f}},
-    {2112211, 64, 64, 4, 3.00f, 1.56f, {0.424f, 0.558f, 0.687f, 0.944f}},
+    {2112211, 64, 64, 4, 3.00f, 1.56f, {0.424f, 0.558f, 0.687f, 0.916f}},
     {2222221, 128, 128, 2, 5.15f, 3.79f, {0.640f, 1.156f}},
     {3332221, 192, 192, 1, 9.89f, 9.10f, {0.860f}},
     {3331182, 96, 96, 1, 6.72f, 5.80f, {0.314f}},
 };
 // fp32 on three bf16 planes: six matrix instructions per operand pair and the conversion between them, so a step costs five
 // times a half one.  Large wave tiles convert less per product, K is split over the waves of a CU wherever tiles are few.
-// Fit and sweep as above (M from 16 to 3072, hidden size 768; the pick is 0.2 % behind the best shape on average).
-// us, v_mfma_f32 kernels before -> now:  M=1536: N=768 K=768 27 -> 18, N=3072 K=768 74 -> 52, N=768 K=3072 83 -> 55
-//   M=128: N=768 K=768 7.6 -> 7.0, N=3072 K=768 15.2 -> 10.0, N=768 K=3072 17.6 -> 15.5   (3072 x 768 x 3072: 168 TFLOP/s)
+// Fit and sweep as above (M from 16 to 3072, hidden size 768), made before the planes were scaled, which costs 1 .. 4 %.
+// us, v_mfma_f32 kernels before -> now:  M=1536: N=768 K=768 27 -> 18.4, N=3072 K=768 74 -> 52, N=768 K=3072 83 -> 53.5
+//   M=128: N=768 K=768 7.6 -> 7.0, N=3072 K=768 15.2 -> 10.1, N=768 K=3072 17.6 -> 15.1   (3072 x 768 x 3072: 153 TFLOP/s)
 // Error against float64 (2-norm over 2-norm; 300 x 760 x 768 / 129 x 264 x 3072): 1.5e-7 .. 3e-7 / 3e-7 .. 6e-7 by shape,
 // v_mfma_f32_32x32x2_f32: 5.0e-7 / 9.9e-7.
 constexpr TileCost kTilesF32[] = {
