@@ -1308,22 +1308,17 @@ template <int DT, bool VT> __global__ void __launch_bounds__(256, 2) attention_s
 }
 
 // The kernel for few query blocks is the faster one as long as its blocks of 32 queries are about as many as the chip has CUs
-// (V^T layout: the LDS-staged kernel reads every K and V tile once per 64 or 128 queries and wins from there on), three times
-// as many where V comes row-major (its transposition through LDS is what the other kernel waits for; a CU holds three of these
-// workgroups), there longer still for sequences of more than 256 keys, and always where one block holds the whole sequence
-// (the other kernels' 64 queries are then half empty).  Time against the other kernel's, fp16, 12 and 16 heads, all keys valid
-// (profiles/attention_kernel_choice.txt):
-//   V^T        192 and 240 blocks -8 .. -22 %, 288 to 432 blocks +13 .. +18 %
-//   row-major  36 to 161 keys: up to 768 blocks -3 .. -32 %, 800 to 1600 blocks -9 .. +35 %, mostly +10 .. +20 %
-//              197 to 256 keys: up to 768 blocks -15 .. -39 %, beyond -17 .. +14 %
-//              260 to 500 keys: up to 1200 blocks -47 .. +7 %, beyond -13 .. +11 %
-constexpr long kShortBlocksVT = 256, kShortBlocksRows = 768, kShortBlocksLongRows = 1200;
-constexpr int kLongRows = 256;
+// (V^T layout: the LDS-staged kernel reads every K and V tile once per 64 or 128 queries and wins from there on), several times
+// as many where V comes row-major (its transposition through LDS is what the other kernel waits for), and always where one
+// block holds the whole sequence (the other kernels' 64 queries are then half empty).  us, fp16, 12 heads, before -> now:
+//   V^T        B1 S32 5.0 -> 4.0   B1 S128 6.0 -> 4.8   B1 S256 6.8 -> 5.5   B1 S512 9.1 -> 6.9   B2 S512 9.7 (this one: 10.3)
+//   row-major  B1 S197 8.2 -> 5.5   B5 S197 9.7 -> 7.1   B8 S384 18.3 -> 17.2   B16 S256 14.3 (this one: 15.9)
+constexpr long kShortBlocksVT = 256, kShortBlocksRows = 1200;
 
 template <bool VT> int launch_attention(hipStream_t s, int dtype, AttnParams p, int B, int heads, int S, bool by_size = true) {
     const long blocks128 = (long)((S + 127) / 128) * heads * B, blocks32 = (long)((S + 31) / 32) * heads * B;
     const int mode = g_attention_dma;
-    const bool few = by_size && (S <= 32 || blocks32 <= (VT ? kShortBlocksVT : S > kLongRows ? kShortBlocksLongRows : kShortBlocksRows));
+    const bool few = by_size && (S <= 32 || blocks32 <= (VT ? kShortBlocksVT : kShortBlocksRows));
     p.by_heads     = FixedDivisor::of((uint32_t)heads);
     // grid of the launch with BQ queries per block
     auto blocks_of = [&](int bq) {
