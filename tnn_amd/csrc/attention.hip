@@ -1310,7 +1310,10 @@ template <int DT, bool VT> __global__ void __launch_bounds__(256, 2) attention_s
 // The kernel for few query blocks is the faster one as long as its blocks of 32 queries are about as many as the chip has CUs
 // (V^T layout: the LDS-staged kernel reads every K and V tile once per 64 or 128 queries and wins from there on), several times
 // as many where V comes row-major (its transposition through LDS is what the other kernel waits for), and always where one
-// block holds the whole sequence (the other kernels' 64 queries are then half empty).  us, fp16, 12 heads, before -> now:
+// block holds the whole sequence (the other kernels' 64 queries are then half empty).  Measured around both lines
+// (profiles/attention_kernel_choice.txt): V^T -8 .. -28 % at 144 to 240 blocks, +13 .. +18 % at 288 to 432; row-major, inside the
+// network, -5 .. -0.2 us a layer up to 768 blocks, from there to 1200 -3.4 .. +1.8 us with -0.8 on average, beyond -3.6 .. +3.3.
+// us, fp16, 12 heads, before -> now:
 //   V^T        B1 S32 5.0 -> 4.0   B1 S128 6.0 -> 4.8   B1 S256 6.8 -> 5.5   B1 S512 9.1 -> 6.9   B2 S512 9.7 (this one: 10.3)
 //   row-major  B1 S197 8.2 -> 5.5   B5 S197 9.7 -> 7.1   B8 S384 18.3 -> 17.2   B16 S256 14.3 (this one: 15.9)
 constexpr long kShortBlocksVT = 256, kShortBlocksRows = 1200;

@@ -2398,9 +2398,9 @@ template <int DT>
 int GemmTyped<DT>::residual_ln(hipStream_t s, const void *x, const void *w, const float *bias, void *C, const void *t,
                                const float *row_stats, const float *gamma, const float *beta, int M, int N, int K, int flags,
                                float *row_sums, int *row_sum_blocks) {
-    // With the row sums first.  Half-precision tiles are at least 64 columns wide, so N <= 64 * kMaxRowSumBlocks keeps
-    // the tile columns within what a reader adds up (and within the caller's buffer of kMaxRowSumBlocks * M pairs); a
-    // tile shape that leaves no LDS for the sums runs the plain form and reports zero blocks.
+    // With the row sums first.  A tile shape whose tile columns are more than a reader adds up (and the caller's buffer of
+    // kMaxRowSumBlocks * M pairs holds: 32 columns wide, from N = 769 on), or that leaves no LDS for the sums, declines in
+    // launch_tiled; the plain form runs then and reports zero blocks.
     if (row_sums && N <= 64 * kMaxRowSumBlocks) {
         const int rc = launch_residual_ln<DT, true>(s, x, w, bias, C, t, row_stats, gamma, beta, M, N, K, flags, row_sums);
         if (rc == 0)
