@@ -1211,6 +1211,21 @@ def test_mask_prepare_any_float_type():
         assert list(got & ~(1 << 30)) == [150, 31, 100, 120, 200, 199, 1, 200, 200]
 
 
+def test_store_through_switch_waits_for_the_device():
+    from tnn_amd import capi
+    lib = capi.load()
+    say("store-through switch: waits")
+    big = torch.randn(8192, 8192, device="cuda")
+    try:
+        for on in (0, 1):
+            for _ in range(4):
+                big = torch.tanh(big @ big)
+            assert lib.tnn_rocm_debug_set_store_through(on) == 0 and lib.tnn_rocm_debug_store_through() == on
+            assert torch.cuda.current_stream().query()
+    finally:
+        lib.tnn_rocm_debug_set_store_through(1)
+
+
 def test_store_through_switch_changes_no_result():
     """GEMM, attention and LayerNorm results leave the kernels through device-scope stores by default and through
     ordinary write-back stores with the switch off: the same bits either way, in every epilogue form."""
@@ -1254,11 +1269,7 @@ def test_store_through_switch_changes_no_result():
         return out
 
     try:
-        big = torch.randn(8192, 8192, device="cuda")
-        for _ in range(4):
-            big = torch.tanh(big @ big)
-        assert lib.tnn_rocm_debug_set_store_through(0) == 0 and lib.tnn_rocm_debug_store_through() == 0
-        assert torch.cuda.current_stream().query()  # the call has waited for what was running
+        assert lib.tnn_rocm_debug_set_store_through(0) == 0
         back = run()
     finally:
         assert lib.tnn_rocm_debug_set_store_through(1) == 0

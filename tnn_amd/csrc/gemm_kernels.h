@@ -1077,9 +1077,9 @@ struct TileOrder {
 };
 
 // An infinity, a NaN or a finite value from 2^104 on has no planes (split_f32.h), and turns every sum it enters into something
-// that is not finite, as a sum beyond 2^80 becomes by itself.  A wave that finds such a sum in one of its 32 x 32 blocks multiplies that block
-// again, its own part of K, with the fp32 matrix instruction and operands straight from memory, and takes those sums in the
-// place of the ones that are not finite.  pa, pb = this lane's row of A and of B, eight values into the step for the upper
+// that is not finite, as a sum beyond 2^80 becomes by itself.  A wave that finds such a sum in one of its 32 x 32 blocks
+// multiplies that block again, its own part of K, with the fp32 matrix instruction and operands straight from memory, and
+// takes those sums in the place of the ones that are not finite.  pa, pb = this lane's row of A and of B, eight values into the step for the upper
 // lanes; steps of 16 k from `first` to `end`, `stride` apart.
 // Nothing overlaps here, so a block costs several times what it did: [384,3072] x [3072,768] takes 28 us, with two rows that
 // are not finite 74, with every value NaN 91 (one thread per sum: 1.6 ms and 1.9 ms; 96 x 96 tiles 78 -> 350, were 13 ms).
