@@ -155,8 +155,8 @@ __device__ __forceinline__ float gelu_erf(float x) {
 // ulp (2.8 % for the rational form).  fp32 products take gelu_erf_wide below, the fp32 layer gelu_erf above.
 // max(x, 0) is formed as x/2 + |x/2|: exact for every finite x above twice the smallest normal value (halving and the sum of
 // equal or opposite halves do not round there), and unlike the maximum instruction, which returns its other operand for a
-// NaN, it hands a NaN through, as the reference's GELU does (and gives NaN for -inf, where the reference's 0.5 x (erf + 1) is -inf times 0).  An overflow
-// upstream therefore stays visible in the output instead of turning into zeros.
+// NaN, it hands a NaN through, as the reference's GELU does (and gives NaN for -inf, where the reference's 0.5 x (erf + 1) is
+// -inf times 0).  An overflow upstream therefore stays visible in the output instead of turning into zeros.
 __device__ __forceinline__ float max_with_zero(float x) {
     const float h = __fmul_rn(0.5f, x);
     return __fadd_rn(h, fabsf(h));
