@@ -662,6 +662,28 @@ def test_gemm_fp32_split_shapes(code, M, N, K):
     assert (np.abs(got[fine] - exact[fine]) <= 2.0 ** -24 * 4 * np.sqrt(K) * size[fine]).all()
 
 
+@pytest.mark.parametrize("code", [9111141, 9111181, 9221141, 2321142, 2231142, 2331142, 2222121, 2222221, 2332121])
+@pytest.mark.parametrize("slabs", [1, 2, 3, 4, 5, 6, 9])
+def test_gemm_fp32_split_slab_counts(code, slabs):
+    """Loops of every length, whole tiles and a last one of one row and eight columns: the slab whose loads are not requested
+    any more, the odd slab at the end, and waves that walk K by themselves with one slab more or less than the others, or none."""
+    from tnn_amd import capi
+    lib = capi.load()
+    say("gemm fp32 code %d, %d slabs" % (code, slabs))
+    M, N, K = 193, 200, slabs * (64 << (code % 10)) // 4
+    rng = np.random.default_rng(code % 1000 + slabs)
+    a, w = rng.standard_normal((M, K)).astype(np.float32), rng.standard_normal((N, K)).astype(np.float32)
+    lib.tnn_rocm_debug_set_gemm_config(code)
+    try:
+        got = host(ops().gemm(dev(a), dev(w), True)).astype(np.float64)
+    finally:
+        lib.tnn_rocm_debug_set_gemm_config(0)
+    exact = a.astype(np.float64) @ w.astype(np.float64).T
+    size = np.abs(a.astype(np.float64)) @ np.abs(w.astype(np.float64)).T
+    # as in test_gemm_fp32_split_shapes: K roundings of half a unit of the sum's magnitude at most
+    assert (np.abs(got - exact) <= 2.0 ** -24 * 4 * np.sqrt(K) * size).all()
+
+
 @pytest.mark.parametrize("code", [9111141, 9121141, 9111181, 9221141, 9321140, 3231142, 2331142, 3222121, 2222221])
 @pytest.mark.parametrize("ea,ew", [(-118, 0), (-126, 30), (-140, 60), (0, -118), (-100, -20), (110, -60), (60, 25)])
 def test_gemm_fp32_split_small_and_large(code, ea, ew):

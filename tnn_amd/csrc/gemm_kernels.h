@@ -98,12 +98,14 @@ template <> struct GemmTraits<TNN_ROCM_F32> {
 // slab's planes while it makes the next one's from their LDS reads: a matrix instruction leaves the vector ALU free for 7 of
 // its 8 issue slots, and the conversion (36 vector instructions per operand and step) goes into them a piece at a time.
 // The order is pinned: left to itself the compiler issues the two kinds one after the other, with the wait states that a
-// dot product's result needs standing empty (64x64 tile, K=3072: 43 us; pinned: 41 us).
+// dot product's result needs standing empty.  With every CU at work the matrix pipe's power holds the clock near 1.6 GHz, which
+// is then the bound; on few CUs the vector instructions are.
 template <int TM, int TN, int STEPS> struct SplitSlab {
     static constexpr int OPS    = TM + TN;
     static constexpr int MFMAS  = STEPS * kSplitProducts * TM * TN;
-    static constexpr int PIECES = STEPS * OPS * 6;  // per operand and step two groups of four values, three pieces each
-    Split3 op[STEPS][OPS];                          // A's operands, then B's
+    static constexpr int UNITS  = STEPS * OPS * 20;  // of a conversion: per operand and step five levels of four pairs of values
+    enum { kEarly, kSpread, kAfterReads };  // kAfterReads: the loads go where the reads come from
+    Split3 op[STEPS][OPS];                           // A's operands, then B's
     struct Reads {
         uint4 f[STEPS][OPS][2];
     };
@@ -125,25 +127,31 @@ template <int TM, int TN, int STEPS> struct SplitSlab {
         for (int q = 0; q < MFMAS; ++q)
             mfma(q, acc);
     }
-    // piece k of a conversion: for group k % 2 of operand k / 6, one plane and what is left of the values
-    static __device__ __forceinline__ void piece(int k, SplitSlab &next, float (&rest)[STEPS][OPS][8], const SplitConst &sc) {
-        const int ks = k / (OPS * 6), o = k / 6 % OPS, plane = k % 6 / 2, g = k % 2;
-        float *x = rest[ks][o] + g * 4;
-        uint32_t *p = next.op[ks][o].p[plane] + g * 2;
-        if (plane == 0)
-            x[0] *= kSplitScale, x[1] *= kSplitScale, x[2] *= kSplitScale, x[3] *= kSplitScale;
-        p[0] = split_pack(x[0], x[1]);
-        p[1] = split_pack(x[2], x[3]);
-        if (plane < 2) {
-            x[0] = split_rest(p[0], sc.lo, x[0]);
-            x[1] = split_rest(p[0], sc.hi, x[1]);
-            x[2] = split_rest(p[1], sc.lo, x[2]);
-            x[3] = split_rest(p[1], sc.hi, x[3]);
+    // Unit k of a conversion: one pair of values of operand k / 20, one level (scale and first plane, rest, second plane, rest,
+    // third plane).  The four pairs take turns, so that nothing waits for the unit before it.
+    static __device__ __forceinline__ void unit(int k, SplitSlab &next, float (&rest)[STEPS][OPS][8], const SplitConst &sc) {
+        const int ks = k / (OPS * 20), o = k / 20 % OPS, level = k % 20 / 4, g = k % 4;
+        float &x = rest[ks][o][2 * g], &y = rest[ks][o][2 * g + 1];
+        if (level == 0)
+            x *= kSplitScale, y *= kSplitScale;
+        uint32_t &pair = next.op[ks][o].p[level / 2][g];
+        if (level % 2 == 0) {
+            pair = split_pack(x, y);
+        } else {
+            x = split_rest(pair, sc.lo, x);
+            y = split_rest(pair, sc.hi, y);
         }
     }
-    __device__ __forceinline__ void turn(const Reads &rd, SplitSlab &next, f32x16 (&acc)[TM][TN], const SplitConst &sc) const {
-        // the first matrix instructions alone: the LDS reads arrive meanwhile
-        constexpr int LEAD = MFMAS >= 24 ? 4 : 2, SLOTS = MFMAS - LEAD;
+    // Multiplies this slab's planes while it makes the next one's, whose LDS reads are under way; load(k) requests the k-th of
+    // LOADS loads of the slab after (PLACE: when).
+    // One or two small pieces of that go behind every matrix instruction: a slot holds about seven vector instructions, and a
+    // piece that is longer (a whole plane of four values took twelve) leaves the matrix pipe empty for the rest of it.
+    template <int LOADS, int PLACE, typename Load>
+    __device__ __forceinline__ void turn(const Reads &rd, SplitSlab &next, f32x16 (&acc)[TM][TN], const SplitConst &sc, Load load) const {
+        constexpr int LEAD = MFMAS >= 24 ? 4 : 2;  // the first matrix instructions alone: the LDS reads arrive meanwhile
+        // loads as early as their place is free, one a slot, where the next turn waits for them; else spread over the turn
+        constexpr int L0     = PLACE != kAfterReads ? 0 : LEAD;
+        constexpr int LSLOTS = PLACE != kSpread && LOADS > 0 && LOADS < MFMAS - L0 ? LOADS : MFMAS - L0;
         float rest[STEPS][OPS][8];
 #pragma unroll
         for (int q = 0; q < MFMAS; ++q) {
@@ -163,12 +171,19 @@ template <int TM, int TN, int STEPS> struct SplitSlab {
                         }
             }
             if (q >= LEAD) {
-                const int upto = PIECES * (q - LEAD + 1) / SLOTS;
+                constexpr int SLOTS = MFMAS - LEAD;
 #pragma unroll
-                for (int k = PIECES * (q - LEAD) / SLOTS; k < upto; ++k)
-                    piece(k, next, rest, sc);
-                __builtin_amdgcn_sched_barrier(0);
+                for (int k = UNITS * (q - LEAD) / SLOTS; k < UNITS * (q - LEAD + 1) / SLOTS; ++k)
+                    unit(k, next, rest, sc);
             }
+            if (LOADS > 0 && q >= L0 && q < L0 + LSLOTS) {
+                if (PLACE == kAfterReads && q == L0)
+                    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+                for (int k = LOADS * (q - L0) / LSLOTS; k < LOADS * (q - L0 + 1) / LSLOTS; ++k)
+                    load(k);
+            }
+            __builtin_amdgcn_sched_barrier(0);
         }
     }
 };
@@ -1261,15 +1276,18 @@ __global__ void __launch_bounds__(CFG::NT)
                          : "v"(byte_off), "s"(base), "s"(lds_addr)
                          : "memory", "m0");
         };
-        auto issue = [&](int slab, int stage) __attribute__((always_inline)) {
+        // load k of a slab; the weights first: they come from further away
+        auto issue_one = [&](int k, int slab, int stage) __attribute__((always_inline)) {
             const uint32_t dst = ring_dst + (uint32_t)(stage * STAGE);
-            const T *ga = A + (size_t)slab * KB, *gb = B + (size_t)slab * KB;
+            if (k >= B_LD)
+                load16(A + (size_t)slab * KB, a_off[k >= B_LD ? k - B_LD : 0], dst + (k - B_LD) * 1024);
+            else
+                load16(B + (size_t)slab * KB, b_off[k < B_LD ? k : 0], dst + BM * SLAB + k * 1024);
+        };
+        auto issue = [&](int slab, int stage) __attribute__((always_inline)) {
 #pragma unroll
-            for (int i = 0; i < B_LD; ++i)  // the weights first: they come from further away
-                load16(gb, b_off[i], dst + BM * SLAB + i * 1024);
-#pragma unroll
-            for (int i = 0; i < A_LD; ++i)
-                load16(ga, a_off[i], dst + i * 1024);
+            for (int k = 0; k < LPW; ++k)
+                issue_one(k, slab, stage);
         };
         const int fswz = (frag_row / R256) % VPR;
         const int frow = frag_row * SLAB;
@@ -1279,8 +1297,7 @@ __global__ void __launch_bounds__(CFG::NT)
             if (k_lo + p < k_hi)
                 issue(k_lo + p, p);
         int stage = 0;
-        // this wave's fragments of slab kt, and the request for the slab that takes its place
-        auto fetch = [&](int kt, uint4 (&f)[SLAB / KSTEP][TM + TN][FRAGS]) __attribute__((always_inline)) {
+        auto wait_for = [&](int kt) __attribute__((always_inline)) {
             // slab kt is complete once at most the loads of the slabs requested after it are outstanding
             const int behind = k_hi - 1 - kt;
             if (NS > 3 && behind >= 3)
@@ -1292,6 +1309,8 @@ __global__ void __launch_bounds__(CFG::NT)
             else
                 TR_WAIT_VMCNT(0);
             asm volatile("" ::: "memory");
+        };
+        auto read_fragments = [&](uint4 (&f)[SLAB / KSTEP][TM + TN][FRAGS]) __attribute__((always_inline)) {
             const unsigned char *sa = ring + stage * STAGE, *sb = sa + BM * SLAB;
 #pragma unroll
             for (int kf = 0; kf < SLAB / 32; ++kf) {
@@ -1303,33 +1322,49 @@ __global__ void __launch_bounds__(CFG::NT)
                 for (int j = 0; j < TN; ++j)
                     f[kf / FRAGS][TM + j][kf % FRAGS] = *reinterpret_cast<const uint4 *>(sb + j * 32 * SLAB + frow + chunk);
             }
-            // the fragments are in registers before the slab's place is given to the next load
-            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-            if (kt + NS < k_hi)
-                issue(kt + NS, stage);
-            stage = stage + 1 == NS ? 0 : stage + 1;
         };
         if constexpr (DT == TNN_ROCM_F32) {
             if (k_lo < k_hi) {
                 typedef SplitSlab<TM, TN, SLAB / KSTEP> Planes;
                 Planes p, q;
-                auto half = [&](int kt, const Planes &now, Planes &next) __attribute__((always_inline)) {
+                auto half = [&](int kt, const Planes &now, Planes &next, auto loads) __attribute__((always_inline)) {
                     typename Planes::Reads rd;
-                    fetch(kt, rd.f);
-                    now.turn(rd, next, acc, split_const);
+                    wait_for(kt);
+                    read_fragments(rd.f);
+                    const int here = stage;
+                    stage = stage + 1 == NS ? 0 : stage + 1;
+                    now.template turn<decltype(loads)::value, Planes::kAfterReads>(
+                        rd, next, acc, split_const, [&](int k) __attribute__((always_inline)) { issue_one(k, kt + NS, here); });
                 };
+                typedef std::integral_constant<int, LPW> WithLoads;
+                typedef std::integral_constant<int, 0> NoLoads;
                 {
                     typename Planes::Reads rd;
-                    fetch(k_lo, rd.f);
+                    wait_for(k_lo);
+                    read_fragments(rd.f);
+                    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+                    if (k_lo + NS < k_hi)
+                        issue(k_lo + NS, 0);
+                    stage = 1;
                     p.convert(rd, split_const);
                 }
                 int kt = k_lo + 1;
+                for (; kt + 1 + NS < k_hi; kt += 2) {
+                    half(kt, p, q, WithLoads());
+                    half(kt + 1, q, p, WithLoads());
+                }
+                // the last slabs: one more to request at most
+                if (kt + NS < k_hi) {
+                    half(kt, p, q, WithLoads());
+                    p = q;
+                    ++kt;
+                }
                 for (; kt + 1 < k_hi; kt += 2) {
-                    half(kt, p, q);
-                    half(kt + 1, q, p);
+                    half(kt, p, q, NoLoads());
+                    half(kt + 1, q, p, NoLoads());
                 }
                 if (kt < k_hi) {
-                    half(kt, p, q);
+                    half(kt, p, q, NoLoads());
                     q.multiply(acc);
                 } else {
                     p.multiply(acc);
@@ -1338,7 +1373,13 @@ __global__ void __launch_bounds__(CFG::NT)
         } else {
             for (int kt = k_lo; kt < k_hi; ++kt) {
                 uint4 f[SLAB / KSTEP][TM + TN][FRAGS];
-                fetch(kt, f);
+                wait_for(kt);
+                read_fragments(f);
+                // the fragments are in registers before the slab's place is given to the next load
+                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+                if (kt + NS < k_hi)
+                    issue(kt + NS, stage);
+                stage = stage + 1 == NS ? 0 : stage + 1;
 #pragma unroll
                 for (int kk = 0; kk < SLAB / KSTEP; ++kk) {
                     if constexpr (Epi::kRowStats) {
@@ -1397,15 +1438,18 @@ __global__ void __launch_bounds__(CFG::NT)
                          : "v"(byte_off), "s"(base), "s"(lds_addr)
                          : "memory", "m0");
         };
-        auto issue = [&](int slab, int stage) {
+        auto issue_one = [&](int k, int slab, int stage) __attribute__((always_inline)) {  // load k of a slab
             const uint32_t dst = wave_dst + (uint32_t)(stage * STAGE);
-            const T *ga = A + (size_t)slab * KB, *gb = B + (size_t)slab * KB;
+            if (k < A_LD)
+                load16(A + (size_t)slab * KB, a_off[k < A_LD ? k : 0] * (uint32_t)sizeof(T), dst + k * CFG::NW * 1024);
+            else
+                load16(B + (size_t)slab * KB, b_off[k >= A_LD ? k - A_LD : 0] * (uint32_t)sizeof(T),
+                       dst + BM * SLAB + (k - A_LD) * CFG::NW * 1024);
+        };
+        auto issue = [&](int slab, int stage) __attribute__((always_inline)) {
 #pragma unroll
-            for (int i = 0; i < A_LD; ++i)
-                load16(ga, a_off[i] * (uint32_t)sizeof(T), dst + i * CFG::NW * 1024);
-#pragma unroll
-            for (int i = 0; i < B_LD; ++i)
-                load16(gb, b_off[i] * (uint32_t)sizeof(T), dst + BM * SLAB + i * CFG::NW * 1024);
+            for (int k = 0; k < A_LD + B_LD; ++k)
+                issue_one(k, slab, stage);
         };
         // byte offset of this lane's fragment chunk inside a slab row, per k-step of the slab
         const int fswz = (frag_row / R256) % VPR;
@@ -1587,7 +1631,9 @@ __global__ void __launch_bounds__(CFG::NT)
         } else if constexpr (DT == TNN_ROCM_F32) {
             typedef SplitSlab<TM, TN, KSTEPS> Planes;
             Planes p, q;
-            auto fetch = [&](int kt, uint4 (&f)[KSTEPS][TM + TN][FRAGS]) __attribute__((always_inline)) {
+            static_assert(NS <= 3, "waits written for up to three stages");
+            // slab kt in LDS, and every wave done with slab kt - 1; its fragments
+            auto fetch = [&](int kt, typename Planes::Reads &rd) __attribute__((always_inline)) {
                 // slab kt - 1 is in this wave's registers, see the barrier below
                 asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
                 const int behind = nk - 1 - kt;
@@ -1605,34 +1651,51 @@ __global__ void __launch_bounds__(CFG::NT)
                         const int chunk = ((((wk + ks * WGK) * FRAGS + h) * 2 + (lane >> 5)) ^ fswz) * 16;
 #pragma unroll
                         for (int i = 0; i < TM; ++i)
-                            f[ks][i][h] = *reinterpret_cast<const uint4 *>(sa + (wm * TM + i) * 32 * SLAB + frow + chunk);
+                            rd.f[ks][i][h] = *reinterpret_cast<const uint4 *>(sa + (wm * TM + i) * 32 * SLAB + frow + chunk);
 #pragma unroll
                         for (int j = 0; j < TN; ++j)
-                            f[ks][TM + j][h] = *reinterpret_cast<const uint4 *>(sb + (wn * TN + j) * 32 * SLAB + frow + chunk);
+                            rd.f[ks][TM + j][h] = *reinterpret_cast<const uint4 *>(sb + (wn * TN + j) * 32 * SLAB + frow + chunk);
                     }
-                if (kt + NS - 1 < nk)
-                    issue(kt + NS - 1, fill);
+            };
+            auto advance = [&]() __attribute__((always_inline)) {
                 stage = stage + 1 == NS ? 0 : stage + 1;
                 fill  = fill + 1 == NS ? 0 : fill + 1;
             };
-            static_assert(NS <= 3, "waits written for up to three stages");
-            auto half = [&](int kt, const Planes &now, Planes &next) __attribute__((always_inline)) {
+            auto half = [&](int kt, const Planes &now, Planes &next, auto loads) __attribute__((always_inline)) {
                 typename Planes::Reads rd;
-                fetch(kt, rd.f);
-                now.turn(rd, next, acc, split_const);
+                fetch(kt, rd);
+                const int there = fill;
+                advance();
+                now.template turn<decltype(loads)::value, (NS > 2 ? Planes::kSpread : Planes::kEarly)>(
+                    rd, next, acc, split_const, [&](int k) __attribute__((always_inline)) { issue_one(k, kt + NS - 1, there); });
             };
+            typedef std::integral_constant<int, LPW> WithLoads;
+            typedef std::integral_constant<int, 0> NoLoads;
             {
                 typename Planes::Reads rd;
-                fetch(0, rd.f);
+                fetch(0, rd);
+                if (NS - 1 < nk)
+                    issue(NS - 1, fill);
+                advance();
                 p.convert(rd, split_const);
             }
             int kt = 1;
+            for (; kt + NS < nk; kt += 2) {
+                half(kt, p, q, WithLoads());
+                half(kt + 1, q, p, WithLoads());
+            }
+            // the last slabs: one more to request at most
+            if (kt + NS - 1 < nk) {
+                half(kt, p, q, WithLoads());
+                p = q;
+                ++kt;
+            }
             for (; kt + 1 < nk; kt += 2) {
-                half(kt, p, q);
-                half(kt + 1, q, p);
+                half(kt, p, q, NoLoads());
+                half(kt + 1, q, p, NoLoads());
             }
             if (kt < nk) {
-                half(kt, p, q);
+                half(kt, p, q, NoLoads());
                 q.multiply(acc);
             } else {
                 p.multiply(acc);
@@ -2061,8 +2124,8 @@ int launch_tiled(hipStream_t s, const void *A, const void *B, int M, int N, int 
 //   3112221   64 x  64, 8 waves (two k-waves), 3 stages       3112222   64 x  64, 8 waves, 256-byte slabs
 //   4221141   64 x  64, 4 k-waves, 4 stages                   3212221  128 x  64, 8 waves
 //   2112211   64 x  64, 4 waves, 2 stages                     2222221  128 x 128, 8 waves (two k-waves)
-//   fp32 only: 9111181 32 x 32, 8 k-waves; 9221141, 9321140 64 x 64 and 96 x 64, 4 k-waves with rings of their own;
-//   3231142, 2331142 64 x 96 and 96 x 96, 4 k-waves; 3222121 128 x 64, 4 waves (two k-waves)
+//   fp32 only: 9111181 32 x 32, 8 k-waves; 9221141 64 x 64, 4 k-waves with rings of their own;
+//   2321142, 2231142, 2331142 96 x 64, 64 x 96 and 96 x 96, 4 k-waves; 2222121, 2332121 128 x 64 and 192 x 96, 4 waves (two k-waves)
 //   3332221  192 x 192, 8 waves (two k-waves)                 3331182   96 x  96, 8 k-waves, 256-byte slabs
 //   112210    64 x  64 and 222210 128 x 128, 4 waves: rows that are no multiple of 128 bytes
 // Eight-wave workgroups put two waves on every SIMD inside one tile: while one waits for its LDS fragments the
@@ -2114,22 +2177,25 @@ constexpr TileCost kTilesI8[] = {
     {3331182, 96, 96, 1, 6.72f, 5.80f, {0.314f}},
 };
 // fp32 on three bf16 planes: six matrix instructions per operand pair and the conversion between them, so a step costs five
-// times a half one.  Large wave tiles convert less per product, K is split over the waves of a CU wherever tiles are few.
-// Fit and sweep as above (M from 16 to 3072, hidden size 768), made before the planes were scaled, which costs 1 .. 4 %.
-// us, v_mfma_f32 kernels before -> now:  M=1536: N=768 K=768 27 -> 18.4, N=3072 K=768 74 -> 52, N=768 K=3072 83 -> 53.5
-//   M=128: N=768 K=768 7.6 -> 7.0, N=3072 K=768 15.2 -> 10.1, N=768 K=3072 17.6 -> 15.1   (3072 x 768 x 3072: 153 TFLOP/s)
+// times a half one.  Large wave tiles convert less per product, K is split over the waves of a CU wherever tiles are few, and
+// two stages are enough where the next slab's loads are the first thing that follows a slab's barrier (turn() in SplitSlab).
+// Fit and sweep as above (M from 16 to 3072, hidden size 768).
+// us, v_mfma_f32 kernels -> planes, a whole plane of four values behind a matrix instruction -> a pair of values:
+//   M=1536: N=768 K=768 27 -> 20.2 -> 17.3, N=3072 K=768 74 -> 61 -> 55, N=768 K=3072 83 -> 60 -> 51
+//   M=128: N=768 K=768 7.6 -> 7.1 -> 6.8, N=3072 K=768 15.2 -> 11.4 -> 10.7, N=768 K=3072 17.6 -> 16.2 -> 15.3
 // Error against float64 (2-norm over 2-norm; 300 x 760 x 768 / 129 x 264 x 3072): 1.5e-7 .. 3e-7 / 3e-7 .. 6e-7 by shape,
 // v_mfma_f32_32x32x2_f32: 5.0e-7 / 9.9e-7.
 constexpr TileCost kTilesF32[] = {
-    {9111141, 32, 32, 2, 3.63f, 1.18f, {0.135f, 0.276f}},
-    {9121141, 32, 64, 1, 4.33f, 3.30f, {0.214f}},
-    {9111181, 32, 32, 1, 3.96f, 2.69f, {0.125f}},
-    {9221141, 64, 64, 1, 5.66f, 5.47f, {0.319f}},
-    {9321140, 96, 64, 1, 6.16f, 7.00f, {0.483f}},
-    {3231142, 64, 96, 1, 6.12f, 5.36f, {0.546f}},
-    {2331142, 96, 96, 1, 7.61f, 7.87f, {0.725f}},
-    {3222121, 128, 64, 2, 5.62f, 5.02f, {0.723f, 1.280f}},
-    {2222221, 128, 128, 1, 6.89f, 10.92f, {1.175f}},
+    {9111141, 32, 32, 2, 4.03f, 1.54f, {0.116f, 0.263f}},
+    {9121141, 32, 64, 1, 5.00f, 4.51f, {0.194f}},
+    {9111181, 32, 32, 1, 4.39f, 3.30f, {0.118f}},
+    {9221141, 64, 64, 1, 6.18f, 7.25f, {0.308f}},
+    {2321142, 96, 64, 1, 5.78f, 9.00f, {0.442f}},
+    {2231142, 64, 96, 1, 6.67f, 10.25f, {0.439f}},
+    {2331142, 96, 96, 1, 8.11f, 15.21f, {0.616f}},
+    {2222121, 128, 64, 2, 5.82f, 10.41f, {0.591f, 1.363f}},
+    {2222221, 128, 128, 1, 7.62f, 19.83f, {1.060f}},
+    {2332121, 192, 96, 1, 9.09f, 24.17f, {1.170f}},
 };
 
 template <int COUNT> inline int pick_tile_config(const TileCost (&shapes)[COUNT], long M, long N, size_t kbytes) {
@@ -2176,6 +2242,13 @@ int launch_gemm_fast(hipStream_t s, const void *A, const void *B, int M, int N, 
         case 331182: cfg = 3331182; break;
         default: break;
     }
+    if (DT == TNN_ROCM_F32)
+        switch (cfg) {  // three stages, or rings of the waves' own: two stages took their place
+            case 9321140: cfg = 2321142; break;
+            case 3231142: cfg = 2231142; break;
+            case 3222121: cfg = 2222121; break;
+            default: break;
+        }
     if (kbytes % (64u << (cfg % 10)) != 0) {
         set_error("gemm: K=%d is not a whole number of slabs for tuning configuration %d", K, cfg);
         return TNN_ROCM_ESHAPE;
@@ -2200,10 +2273,11 @@ int launch_gemm_fast(hipStream_t s, const void *A, const void *B, int M, int N, 
         switch (cfg) {
             case 9111181: TR_FAST_OWN(1, 1, 8, 128, 2);
             case 9221141: TR_FAST_OWN(2, 2, 4, 128, 2);
-            case 9321140: TR_FAST_OWN(3, 2, 4, 64, 3);
-            case 3231142: TR_FAST_DL(2, 3, 1, 1, 4, 256, 3);
+            case 2321142: TR_FAST_DL(3, 2, 1, 1, 4, 256, 2);
+            case 2231142: TR_FAST_DL(2, 3, 1, 1, 4, 256, 2);
             case 2331142: TR_FAST_DL(3, 3, 1, 1, 4, 256, 2);
-            case 3222121: TR_FAST_DL(2, 2, 2, 1, 2, 128, 3);
+            case 2222121: TR_FAST_DL(2, 2, 2, 1, 2, 128, 2);
+            case 2332121: TR_FAST_DL(3, 3, 2, 1, 2, 128, 2);
             case 2222221: TR_FAST_DL(2, 2, 2, 2, 2, 128, 2);
             default: break;
         }
