@@ -210,6 +210,28 @@ def test_layernorm_fp16():
     assert abs(got.mean(-1)).max() < 2e-3 and abs(got.var(-1) - 1).max() < 5e-3
 
 
+@pytest.mark.parametrize("dtype", ["float32", "float16", "bfloat16"])
+@pytest.mark.parametrize("vecs", [1, 33, 64, 65, 96, 97, 128, 129, 192, 193, 256, 257, 512])
+def test_layernorm_row_count_changes_nothing(dtype, vecs):
+    """Launches of up to 6144 rows request everything ahead, larger ones do not: the same bits, at every width a lane count or
+    a number of vectors per lane ends at; a few rows against the checker."""
+    say("layernorm %s, rows of %d 16-byte vectors" % (dtype, vecs))
+    td = getattr(torch, dtype)
+    cols, rows = vecs * (4 if dtype == "float32" else 8), 6145
+    gen = torch.Generator(device="cuda").manual_seed(vecs)
+    x, r = (torch.randn(rows, cols, device="cuda", generator=gen).to(td) for _ in range(2))
+    g, b = (torch.randn(cols, device="cuda", generator=gen) for _ in range(2))
+    for res in (None, r):
+        y, q = ops().layernorm(x, g, b, 1e-5, residual=res, q_inv_scale=20.0)
+        for lo, hi in ((0, 6144), (6140, 6145), (0, 1)):
+            ys, qs = ops().layernorm(x[lo:hi].contiguous(), g, b, 1e-5, residual=None if res is None else res[lo:hi].contiguous(),
+                                     q_inv_scale=20.0)
+            assert torch.equal(ys, y[lo:hi]) and torch.equal(qs, q[lo:hi])
+        some = x[:3].float() if res is None else x[:3].float() + res[:3].float()
+        ref = orc.layernorm(host(some), host(g), host(b), 1e-5)
+        assert rel_err(host(y[:3].float()), ref) <= {"float32": 2e-6, "float16": 2e-3, "bfloat16": 1.6e-2}[dtype]
+
+
 def test_layernorm_rejects_empty():
     from tnn_amd import capi
     o = ops()

@@ -11,6 +11,7 @@ namespace {
 
 constexpr int kBlock       = 256;
 constexpr int kRowsPerBlk  = kBlock / kWave;
+constexpr int kLnAheadRows = 6144;  // LayerNorm launches of more rows request scale and shift behind the reduction
 constexpr int kMaxVecPerLn = 8;  // row cached in registers when cols <= 64 * VEC * 8
 
 __device__ __forceinline__ double wave_sum_f64(double v) {
@@ -20,13 +21,32 @@ __device__ __forceinline__ double wave_sum_f64(double v) {
     return v;
 }
 
+// v plus the v of lane ^ O, for O = 32, 16, 8, 4, 2, 1 in turn (from 4 on down the lanes of a row that differ in higher bits
+// hold the same value already, so that a rotation serves): register moves between lanes, where a shuffle goes through LDS at
+// some hundred clocks, ten or twelve of them one after the other in front of the second half of a LayerNorm
+template <int O> __device__ __forceinline__ double add_lane_xor(double v) {
+    typedef uint32_t pair __attribute__((ext_vector_type(2)));
+    const pair u = __builtin_bit_cast(pair, v);
+    if constexpr (O >= 16) {
+        const auto lo = O == 32 ? __builtin_amdgcn_permlane32_swap(u.x, u.x, false, false) : __builtin_amdgcn_permlane16_swap(u.x, u.x, false, false);
+        const auto hi = O == 32 ? __builtin_amdgcn_permlane32_swap(u.y, u.y, false, false) : __builtin_amdgcn_permlane16_swap(u.y, u.y, false, false);
+        return __builtin_bit_cast(double, pair{lo[0], hi[0]}) + __builtin_bit_cast(double, pair{lo[1], hi[1]});
+    } else {
+        constexpr int CTRL = O == 8 ? 0x128 : O == 4 ? 0x124 : O == 2 ? 0x4E : 0xB1;  // row_ror:8, row_ror:4, quad_perm
+        const pair w = {(uint32_t)__builtin_amdgcn_update_dpp(0, (int)u.x, CTRL, 0xf, 0xf, false),
+                        (uint32_t)__builtin_amdgcn_update_dpp(0, (int)u.y, CTRL, 0xf, 0xf, false)};
+        return v + __builtin_bit_cast(double, w);
+    }
+}
 // sum over each aligned group of LPR lanes (32: the two halves of a wave hold different rows)
-template <int LPR>
-__device__ __forceinline__ double lanes_sum_f64(double v) {
-#pragma unroll
-    for (int o = LPR / 2; o > 0; o >>= 1)
-        v += __shfl_xor(v, o, 64);
-    return v;
+template <int LPR> __device__ __forceinline__ double lanes_sum_f64(double v) {
+    if constexpr (LPR == 64)
+        v = add_lane_xor<32>(v);
+    v = add_lane_xor<16>(v);
+    v = add_lane_xor<8>(v);
+    v = add_lane_xor<4>(v);
+    v = add_lane_xor<2>(v);
+    return add_lane_xor<1>(v);
 }
 
 // ---- LayerNorm ----------------------------------------------------------------------------------
@@ -49,7 +69,9 @@ struct EmbedRows {
 
 // LPR lanes own one row (64: a wave per row; 32: a wave holds two rows, which keeps every lane busy and twice the
 // bytes in flight for rows of at most 128 vectors); NV = 16-byte vectors a lane can hold.
-template <int DT, bool VECTOR, int LPR, int NV>
+// AHEAD: everything the row needs is requested at once, scale and shift among it.  Requested where they are used they are a
+// second latency behind the reduction; the registers they take meanwhile cost resident waves.
+template <int DT, bool VECTOR, int LPR, int NV, bool AHEAD>
 __global__ void __launch_bounds__(kBlock) layernorm_kernel(const typename Elem<DT>::type *__restrict__ x,
                                                            const typename Elem<DT>::type *__restrict__ res,
                                                            const float *__restrict__ gamma,
@@ -58,6 +80,7 @@ __global__ void __launch_bounds__(kBlock) layernorm_kernel(const typename Elem<D
                                                            float eps, int8_t *__restrict__ out_q, float q_inv,
                                                            EmbedRows emb, StoreThrough mode) {
     typedef typename Elem<DT>::type T;
+    touch_kernel_args<7 * 8 + 3 * 8 + sizeof(EmbedRows)>();
     constexpr int VEC = VECTOR ? (int)(16 / sizeof(T)) : 1;
     const int lane    = threadIdx.x & (LPR - 1);
     const int row     = (blockIdx.x * kRowsPerBlk + (threadIdx.x >> 6)) * (kWave / LPR) + ((threadIdx.x & (kWave - 1)) / LPR);
@@ -93,19 +116,37 @@ __global__ void __launch_bounds__(kBlock) layernorm_kernel(const typename Elem<D
 
     float v[NV][VEC];
     double s1 = 0.0, s2 = 0.0;
+    uint4 raw[NV], rraw[NV], rraw2[NV];
+    float gam[NV][VEC], bet[NV][VEC];
+    auto request = [&](int j, int vi) __attribute__((always_inline)) {
+        raw[j] = reinterpret_cast<const uint4 *>(px)[vi];
+        if (pr)
+            rraw[j] = reinterpret_cast<const uint4 *>(pr)[vi];
+        if (pr2)
+            rraw2[j] = reinterpret_cast<const uint4 *>(pr2)[vi];
+    };
+    auto request_affine = [&](int j, int vi) __attribute__((always_inline)) {
+#pragma unroll
+        for (int t = 0; t < VEC; ++t)
+            gam[j][t] = gamma[vi * VEC + t], bet[j][t] = beta[vi * VEC + t];
+    };
+    if constexpr (AHEAD) {  // what lies behind the row is clamped and not used
+#pragma unroll
+        for (int j = 0; j < NV; ++j)
+            request(j, lane + j * LPR < nv ? lane + j * LPR : nv - 1);
+#pragma unroll
+        for (int j = 0; j < NV; ++j)
+            request_affine(j, lane + j * LPR < nv ? lane + j * LPR : nv - 1);
+    }
 #pragma unroll
     for (int j = 0; j < NV; ++j) {
         int vi = lane + j * LPR;
         if (vi < nv) {
             if (VECTOR) {
-                uint4 raw = reinterpret_cast<const uint4 *>(px)[vi];
-                const T *e = reinterpret_cast<const T *>(&raw);
-                uint4 rraw, rraw2;
-                const T *re = reinterpret_cast<const T *>(&rraw), *re2 = reinterpret_cast<const T *>(&rraw2);
-                if (pr)
-                    rraw = reinterpret_cast<const uint4 *>(pr)[vi];
-                if (pr2)
-                    rraw2 = reinterpret_cast<const uint4 *>(pr2)[vi];
+                if constexpr (!AHEAD)
+                    request(j, vi);
+                const T *e = reinterpret_cast<const T *>(&raw[j]);
+                const T *re = reinterpret_cast<const T *>(&rraw[j]), *re2 = reinterpret_cast<const T *>(&rraw2[j]);
 #pragma unroll
                 for (int t = 0; t < VEC; ++t) {
                     float f = Elem<DT>::ld(&e[t]);
@@ -149,28 +190,29 @@ __global__ void __launch_bounds__(kBlock) layernorm_kernel(const typename Elem<D
     for (int j = 0; j < NV; ++j) {
         int vi = lane + j * LPR;
         if (vi < nv) {
+            if constexpr (!AHEAD)
+                request_affine(j, vi);
             float o[VEC];
 #pragma unroll
             for (int t = 0; t < VEC; ++t) {
-                int c   = vi * VEC + t;
-                float k = gamma[c];
+                float k = gam[j][t];
                 if (DT == TNN_ROCM_F32) {
                     // the reference's operand order and widths (cpu_layer_norm_layer_acc.cc:126-131): the shifted
                     // bias is formed in double and rounded to float, the affine combination is evaluated in double
-                    float b = (float)((double)beta[c] - mean * rstdd * (double)k);
+                    float b = (float)((double)bet[j][t] - mean * rstdd * (double)k);
                     o[t]    = (float)((double)v[j][t] * rstdd * (double)k + (double)b);
                 } else {
-                    float b = beta[c] - mrs * k;
+                    float b = bet[j][t] - mrs * k;
                     o[t]    = v[j][t] * rstd * k + b;
                 }
             }
             if (VECTOR) {
-                uint4 raw;
-                T *e = reinterpret_cast<T *>(&raw);
+                uint4 out;
+                T *e = reinterpret_cast<T *>(&out);
 #pragma unroll
                 for (int t = 0; t < VEC; ++t)
                     Elem<DT>::st(&e[t], o[t]);
-                store_out16(mode.through, reinterpret_cast<uint4 *>(py) + vi, store_u32x4{raw.x, raw.y, raw.z, raw.w});
+                store_out16(mode.through, reinterpret_cast<uint4 *>(py) + vi, store_u32x4{out.x, out.y, out.z, out.w});
                 if (pq) {  // the VEC (4 or 8) quantised values of this lane leave as one 4- or 8-byte store
                     uint32_t w[2] = {0u, 0u};
 #pragma unroll
@@ -262,22 +304,38 @@ int launch_layernorm(hipStream_t s, const void *x, const void *res, const float 
         return TNN_ROCM_ESHAPE;
     }
     if (al && cols <= kWave * VEC * kMaxVecPerLn) {
-#define TR_LN(LPR, NV)                                                                                                \
-    hipLaunchKernelGGL((layernorm_kernel<DT, true, LPR, NV>),                                                         \
+        // All rows resident at once (768 columns fp16: 3 workgroups of 8 rows a CU with everything requested ahead): the launch
+        // is as long as one row's chain.  More rows, and other waves cover it: 196608 rows of 1024 with a residual 158 us, 222
+        // requested ahead.
+        const bool ahead = rows <= kLnAheadRows;
+#define TR_LN_LAUNCH(LPR, NV, AHEAD)                                                                                  \
+    hipLaunchKernelGGL((layernorm_kernel<DT, true, LPR, NV, AHEAD>),                                                  \
                        dim3((rows + kRowsPerBlk * (kWave / LPR) - 1) / (kRowsPerBlk * (kWave / LPR))), block, 0, s,   \
                        (const T *)x, (const T *)res, gamma, beta, (T *)y, rows, cols, eps, out_q, q_inv, emb,     \
                        StoreThrough())
+#define TR_LN(LPR, NV)                                                                                                \
+    do {                                                                                                              \
+        if (ahead)                                                                                                    \
+            TR_LN_LAUNCH(LPR, NV, true);                                                                              \
+        else                                                                                                          \
+            TR_LN_LAUNCH(LPR, NV, false);                                                                             \
+    } while (0)
         if (nv <= 64)
             TR_LN(32, 2);
+        else if (nv <= 96)
+            TR_LN(32, 3);
         else if (nv <= 128)
             TR_LN(32, 4);
+        else if (nv <= 192)
+            TR_LN(64, 3);
         else if (nv <= 256)
             TR_LN(64, 4);
         else
             TR_LN(64, 8);
 #undef TR_LN
+#undef TR_LN_LAUNCH
     } else if (cols <= kWave * kMaxVecPerLn) {
-        hipLaunchKernelGGL((layernorm_kernel<DT, false, kWave, kMaxVecPerLn>), grid, block, 0, s, (const T *)x,
+        hipLaunchKernelGGL((layernorm_kernel<DT, false, kWave, kMaxVecPerLn, false>), grid, block, 0, s, (const T *)x,
                            (const T *)res, gamma, beta, (T *)y, rows, cols, eps, out_q, q_inv, emb, StoreThrough());
     } else {
         hipLaunchKernelGGL((layernorm_long_kernel<DT>), grid, block, 0, s, (const T *)x, (const T *)res, gamma, beta,
