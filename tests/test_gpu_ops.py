@@ -684,6 +684,25 @@ def test_gemm_fp32_split_shapes(code, M, N, K):
     assert (np.abs(got[fine] - exact[fine]) <= 2.0 ** -24 * 4 * np.sqrt(K) * size[fine]).all()
 
 
+@pytest.mark.parametrize("code", [6111141, 6211141, 6121141])
+@pytest.mark.parametrize("M,N,K", [(1, 8, 256), (17, 24, 256), (33, 776, 768), (130, 136, 3072)])
+def test_gemm_16x16_blocks(code, M, N, K):
+    """The tiles of 16 x 16 blocks at one row, a row and eight columns behind whole tiles, few slabs and many: every epilogue."""
+    test_gemm_small_product_shapes(code, M, N, K)
+
+
+@pytest.mark.parametrize("code", [6111141, 6211141, 6121141, 6111181, 6211181])
+@pytest.mark.parametrize("M,N,K", [(1, 8, 128), (17, 24, 192), (97, 104, 192), (130, 136, 3072)])
+def test_gemm_fp32_16x16_blocks(code, M, N, K):
+    """... and fp32 on them: precision, values next to the ends of the range, infinities and NaN, which are formed again"""
+    test_gemm_fp32_split_shapes(code, M, N, K)
+    if K == 192:
+        for ea, ew in ((-140, 60), (0, -118), (110, -60), (60, 25)):
+            test_gemm_fp32_split_small_and_large(code, ea, ew)
+        for slabs in (1, 2, 3, 4, 5, 6, 9, 16, 17, 25):
+            test_gemm_fp32_split_slab_counts(code, slabs)
+
+
 @pytest.mark.parametrize("code", [9111141, 9111181, 9221141, 2321142, 2231142, 2331142, 2222121, 2222221, 2332121])
 @pytest.mark.parametrize("slabs", [1, 2, 3, 4, 5, 6, 9])
 def test_gemm_fp32_split_slab_counts(code, slabs):

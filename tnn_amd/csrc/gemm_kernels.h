@@ -39,6 +39,7 @@ namespace {
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef int i32x16 __attribute__((ext_vector_type(16)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef int i32x4 __attribute__((ext_vector_type(4)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -53,32 +54,45 @@ template <> struct GemmTraits<TNN_ROCM_F16> {
     static constexpr int FRAGS = 1;
     typedef half_t elem;
     typedef f32x16 acc;
+    typedef f32x4 acc_small;  // of a 16 x 16 block
     static __device__ __forceinline__ void mma(const uint4 &a, const uint4 &b, acc &c) {
         c = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0,
                                                    0);
+    }
+    static __device__ __forceinline__ void mma(const uint4 &a, const uint4 &b, acc_small &c) {
+        c = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
     }
 };
 template <> struct GemmTraits<TNN_ROCM_BF16> {
     static constexpr int FRAGS = 1;
     typedef bf16_bits elem;
     typedef f32x16 acc;
+    typedef f32x4 acc_small;
     static __device__ __forceinline__ void mma(const uint4 &a, const uint4 &b, acc &c) {
         c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0,
                                                     0, 0);
+    }
+    static __device__ __forceinline__ void mma(const uint4 &a, const uint4 &b, acc_small &c) {
+        c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
     }
 };
 template <> struct GemmTraits<TNN_ROCM_I8> {
     static constexpr int FRAGS = 1;
     typedef int8_t elem;
     typedef i32x16 acc;
+    typedef i32x4 acc_small;
     static __device__ __forceinline__ void mma(const uint4 &a, const uint4 &b, acc &c) {
         c = __builtin_amdgcn_mfma_i32_32x32x32_i8(__builtin_bit_cast(i32x4, a), __builtin_bit_cast(i32x4, b), c, 0, 0,
                                                   0);
+    }
+    static __device__ __forceinline__ void mma(const uint4 &a, const uint4 &b, acc_small &c) {
+        c = __builtin_amdgcn_mfma_i32_16x16x64_i8(__builtin_bit_cast(i32x4, a), __builtin_bit_cast(i32x4, b), c, 0, 0, 0);
     }
 };
 template <> struct GemmTraits<TNN_ROCM_F32> {
     typedef float elem;
     typedef f32x16 acc;
+    typedef f32x4 acc_small;
     // the tiled kernel: two reads make one 16-wide step of three bf16 planes (split_f32.h)
     static constexpr int FRAGS = 2;
     static __device__ __forceinline__ Split3 prepare(const uint4 (&f)[2], const SplitConst &c) {
@@ -92,6 +106,12 @@ template <> struct GemmTraits<TNN_ROCM_F32> {
         c = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(a.y), __uint_as_float(b.y), c, 0, 0, 0);
         c = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(a.z), __uint_as_float(b.z), c, 0, 0, 0);
         c = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(a.w), __uint_as_float(b.w), c, 0, 0, 0);
+    }
+    static __device__ __forceinline__ void mma(const uint4 &a, const uint4 &b, acc_small &c) {
+        c = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(a.x), __uint_as_float(b.x), c, 0, 0, 0);
+        c = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(a.y), __uint_as_float(b.y), c, 0, 0, 0);
+        c = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(a.z), __uint_as_float(b.z), c, 0, 0, 0);
+        c = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(a.w), __uint_as_float(b.w), c, 0, 0, 0);
     }
 };
 // fp32, pipelined: the planes of the operands of the STEPS steps that a wave takes from one slab.  turn() multiplies one
@@ -117,12 +137,12 @@ template <int TM, int TN, int STEPS> struct SplitSlab {
             for (int o = 0; o < OPS; ++o)
                 op[ks][o] = GemmTraits<TNN_ROCM_F32>::prepare(rd.f[ks][o], sc);
     }
-    __device__ __forceinline__ void mfma(int q, f32x16 (&acc)[TM][TN]) const {
+    template <typename Acc> __device__ __forceinline__ void mfma(int q, Acc (&acc)[TM][TN]) const {
         const int ks = q / (kSplitProducts * TM * TN), r = q % (kSplitProducts * TM * TN);
         const int product = r / (TM * TN), i = r % (TM * TN) / TN, j = r % TN;
         split_mma(op[ks][TM + j], op[ks][i], product, acc[i][j]);
     }
-    __device__ __forceinline__ void multiply(f32x16 (&acc)[TM][TN]) const {
+    template <typename Acc> __device__ __forceinline__ void multiply(Acc (&acc)[TM][TN]) const {
 #pragma unroll
         for (int q = 0; q < MFMAS; ++q)
             mfma(q, acc);
@@ -146,8 +166,8 @@ template <int TM, int TN, int STEPS> struct SplitSlab {
     // LOADS loads of the slab after (PLACE: when).
     // One or two small pieces of that go behind every matrix instruction: a slot holds about seven vector instructions, and a
     // piece that is longer (a whole plane of four values took twelve) leaves the matrix pipe empty for the rest of it.
-    template <int LOADS, int PLACE, typename Load>
-    __device__ __forceinline__ void turn(const Reads &rd, SplitSlab &next, f32x16 (&acc)[TM][TN], const SplitConst &sc, Load load) const {
+    template <int LOADS, int PLACE, typename Acc, typename Load>
+    __device__ __forceinline__ void turn(const Reads &rd, SplitSlab &next, Acc (&acc)[TM][TN], const SplitConst &sc, Load load) const {
         constexpr int LEAD = MFMAS >= 24 ? 4 : 2;  // the first matrix instructions alone: the LDS reads arrive meanwhile
         // loads as early as their place is free, one a slot, where the next turn waits for them; else spread over the turn
         constexpr int L0     = PLACE != kAfterReads ? 0 : LEAD;
@@ -1037,14 +1057,19 @@ __global__ void __launch_bounds__(WM *WN * 64)
 // OWN (with WGM = WGN = 1): every k-wave has a ring of NSTAGE slabs of its own and walks a contiguous part of K by itself.
 //     A slab is then SLAB bytes of k of ALL rows of the tile for ONE wave, and nothing in the main loop concerns another
 //     wave: no barrier, each wave waits for its own loads only.
-template <int TM_, int TN_, int WGM_, int WGN_, int WGK_, int SLAB_, int NSTAGE_ = 0, bool OWN_ = false> struct TileCfg {
+// BLK = 16 (with OWN): the waves' blocks are 16 x 16 instead of 32 x 32 (v_mfma_*_16x16x32, 64 bytes of k a step), TM and TN
+//     count those, and the whole tile is staged for the epilogue at once.
+template <int TM_, int TN_, int WGM_, int WGN_, int WGK_, int SLAB_, int NSTAGE_ = 0, bool OWN_ = false, int BLK_ = 32> struct TileCfg {
+    static constexpr int BLK = BLK_;
+    static constexpr int GROUPS = BLK_ == 32 ? TM_ : 1, GROWS = BLK_ == 32 ? 32 : BLK_ * TM_;  // staged together: rows of a wave position
+    static_assert(BLK_ == 32 || (BLK_ == 16 && OWN_ && BLK_ * TM_ <= 32), "16 x 16 blocks: small tiles with rings of the waves' own");
     static constexpr int TM = TM_, TN = TN_, WGM = WGM_, WGN = WGN_, WGK = WGK_, SLAB = SLAB_, NSTAGE = NSTAGE_;
     static constexpr bool OWN = OWN_;
-    static constexpr int BM = 32 * TM * WGM, BN = 32 * TN * WGN;
+    static constexpr int BM = BLK * TM * WGM, BN = BLK * TN * WGN;
     static constexpr int STRIDE = NSTAGE_ ? SLAB : SLAB + 16;
-    static constexpr int SSTR   = 32 * TN + 4;  // staged row stride in 32-bit words
+    static constexpr int SSTR   = BLK * TN + 4;  // staged row stride in 32-bit words
     static constexpr size_t slab_bytes  = (size_t)(NSTAGE_ ? NSTAGE_ : 2) * (BM + BN) * STRIDE * (OWN_ ? WGK_ : 1);
-    static constexpr size_t stage_bytes = (size_t)WGM_ * WGN_ * WGK_ * 32 * SSTR * 4;
+    static constexpr size_t stage_bytes = (size_t)WGM_ * WGN_ * WGK_ * GROWS * SSTR * 4;
     static constexpr size_t lds_bytes   = slab_bytes > stage_bytes ? slab_bytes : stage_bytes;
     // where an epilogue that leaves row sums keeps its BM x BN / 8 pairs: in the part of the slab area the staging does
     // not reach when that is large enough (dead by then), else behind everything
@@ -1098,19 +1123,22 @@ struct TileOrder {
 // lanes; steps of 16 k from `first` to `end`, `stride` apart.
 // Nothing overlaps here, so a block costs several times what it did: [384,3072] x [3072,768] takes 28 us, with two rows that
 // are not finite 74, with every value NaN 91 (one thread per sum: 1.6 ms and 1.9 ms; 96 x 96 tiles 78 -> 350, were 13 ms).
-__device__ __forceinline__ void multiply_again(const float *pa, const float *pb, int first, int end, int stride, f32x16 &acc) {
-    f32x16 sum;
+template <typename Acc>
+__device__ __forceinline__ void multiply_again(const float *pa, const float *pb, int first, int end, int stride, Acc &acc) {
+    constexpr int REGS = sizeof(Acc) / 4;  // 16: a 32 x 32 block, a lane holds 8 of a step's values; 4: 16 x 16, it holds 4
+    Acc sum;
 #pragma unroll
-    for (int r = 0; r < 16; ++r)
+    for (int r = 0; r < REGS; ++r)
         sum[r] = 0.f;
 #pragma unroll 1
     for (int t = first; t < end; t += stride) {
         const uint4 *a = reinterpret_cast<const uint4 *>(pa + (size_t)t * 16), *b = reinterpret_cast<const uint4 *>(pb + (size_t)t * 16);
-        GemmTraits<TNN_ROCM_F32>::mma(b[0], a[0], sum);
-        GemmTraits<TNN_ROCM_F32>::mma(b[1], a[1], sum);
+#pragma unroll
+        for (int h = 0; h < REGS / 8 + (REGS < 8); ++h)
+            GemmTraits<TNN_ROCM_F32>::mma(b[h], a[h], sum);
     }
 #pragma unroll
-    for (int r = 0; r < 16; ++r)
+    for (int r = 0; r < REGS; ++r)
         acc[r] = split_finite(__builtin_fabsf(acc[r])) ? acc[r] : sum[r];
 }
 
@@ -1120,7 +1148,8 @@ __global__ void __launch_bounds__(CFG::NT)
                          const typename GemmTraits<DT>::elem *__restrict__ B, int M, int N, int K, long lda, long ldb,
                          int tiles_m, int tiles_n, TileOrder order, Epi epi) {
     typedef typename GemmTraits<DT>::elem T;
-    typedef typename GemmTraits<DT>::acc Acc;
+    constexpr int BLK = CFG::BLK, GROUPS = CFG::GROUPS, GROWS = CFG::GROWS;
+    typedef typename std::conditional<BLK == 32, typename GemmTraits<DT>::acc, typename GemmTraits<DT>::acc_small>::type Acc;
     constexpr int TM = CFG::TM, TN = CFG::TN, WGN = CFG::WGN, WGK = CFG::WGK, SLAB = CFG::SLAB;
     constexpr int BM = CFG::BM, BN = CFG::BN, STRIDE = CFG::STRIDE;
     constexpr int NT     = CFG::NT;
@@ -1163,18 +1192,18 @@ __global__ void __launch_bounds__(CFG::NT)
     // ---- what the epilogue reads, requested before the first slab where a thread has one item and registers to spare: behind
     // the main loop the same loads are two latencies one after the other (columns and row pairs, then the residual), 0.4 us
     // of a launch of 4
-    constexpr int CW    = TN * 32;       // columns per wave
+    constexpr int CW    = TN * BLK;      // columns per wave
     constexpr int CPR   = CW / 8;        // 8-column pieces per staged row
     constexpr int POS   = CFG::NW / WGK;  // wave positions (wm, wn) in the tile
-    constexpr int ITEMS = POS * 32 * CPR;
-    constexpr bool EARLY = TM == 1 && ITEMS <= NT && CFG::NSTAGE > 0;
+    constexpr int ITEMS = POS * GROWS * CPR;
+    constexpr bool EARLY = GROUPS == 1 && ITEMS <= NT && CFG::NSTAGE > 0;
     const bool by_rows   = epi.direct(n0);
-    // row and first column (inside the tile) of an item of the first 32-row group of every wave position
+    // row and first column (inside the tile) of an item of the first group of rows of every wave position
     auto item_at = [&](int item, int *row, int *col) __attribute__((always_inline)) {
-        const int c8  = by_rows ? ((item >> 5) % CPR) * 8 : (item % CPR) * 8;
-        const int r   = by_rows ? (item & 31) : (item / CPR) % 32;
-        const int pos = item / (CPR * 32);
-        *row          = (pos / WGN) * TM * 32 + r;
+        const int c8  = by_rows ? ((item / GROWS) % CPR) * 8 : (item % CPR) * 8;
+        const int r   = by_rows ? (item % GROWS) : (item / CPR) % GROWS;
+        const int pos = item / (CPR * GROWS);
+        *row          = (pos / WGN) * GROUPS * GROWS + r;
         *col          = (pos % WGN) * CW + c8;
     };
     constexpr int COLQ = (ColArrays<Epi>::value * BN + NT - 1) / NT;
@@ -1217,13 +1246,13 @@ __global__ void __launch_bounds__(CFG::NT)
 #pragma unroll
         for (int j = 0; j < TN; ++j)
 #pragma unroll
-            for (int r = 0; r < 16; ++r)
+            for (int r = 0; r < BLK * BLK / 64; ++r)
                 acc[i][j][r] = 0;
 
-    const int frag_row = lane & 31;
+    const int frag_row = lane % BLK;
     const int frag_off = (lane >> 5) * 16;
     const int nk       = K / KB;
-    constexpr int FRAGS = GemmTraits<DT>::FRAGS, KSTEP = 32 * FRAGS;  // bytes of k per row that one step multiplies
+    constexpr int FRAGS = GemmTraits<DT>::FRAGS, KSTEP = (1024 / BLK) * FRAGS;  // bytes of k per row that one step multiplies
     const SplitConst split_const;
 
     // LayerNorm-folding epilogues: this lane's share of sum / sum of squares of A row (wm * TM + i) * 32 + frag_row.  The
@@ -1313,14 +1342,14 @@ __global__ void __launch_bounds__(CFG::NT)
         auto read_fragments = [&](uint4 (&f)[SLAB / KSTEP][TM + TN][FRAGS]) __attribute__((always_inline)) {
             const unsigned char *sa = ring + stage * STAGE, *sb = sa + BM * SLAB;
 #pragma unroll
-            for (int kf = 0; kf < SLAB / 32; ++kf) {
-                const int chunk = ((kf * 2 + (lane >> 5)) ^ fswz) * 16;
+            for (int kf = 0; kf < SLAB * BLK / 1024; ++kf) {
+                const int chunk = ((kf * (64 / BLK) + lane / BLK) ^ fswz) * 16;
 #pragma unroll
                 for (int i = 0; i < TM; ++i)
-                    f[kf / FRAGS][i][kf % FRAGS] = *reinterpret_cast<const uint4 *>(sa + i * 32 * SLAB + frow + chunk);
+                    f[kf / FRAGS][i][kf % FRAGS] = *reinterpret_cast<const uint4 *>(sa + i * BLK * SLAB + frow + chunk);
 #pragma unroll
                 for (int j = 0; j < TN; ++j)
-                    f[kf / FRAGS][TM + j][kf % FRAGS] = *reinterpret_cast<const uint4 *>(sb + j * 32 * SLAB + frow + chunk);
+                    f[kf / FRAGS][TM + j][kf % FRAGS] = *reinterpret_cast<const uint4 *>(sb + j * BLK * SLAB + frow + chunk);
             }
         };
         if constexpr (DT == TNN_ROCM_F32) {
@@ -1788,24 +1817,24 @@ __global__ void __launch_bounds__(CFG::NT)
     }
 
     if constexpr (DT == TNN_ROCM_F32 && CFG::NSTAGE > 0) {
-        constexpr int STEPS = SLAB / KSTEP;  // 16-wide steps per slab
+        constexpr int STEPS = SLAB / 64, REGS = BLK * BLK / 64;  // steps of 16 values of k per slab
 #pragma unroll
         for (int i = 0; i < TM; ++i)
 #pragma unroll
             for (int j = 0; j < TN; ++j) {
                 float size = 0.f;
 #pragma unroll
-                for (int r = 0; r < 16; ++r)
+                for (int r = 0; r < REGS; ++r)
                     size += __builtin_fabsf(acc[i][j][r]);
 #pragma unroll
-                for (int r = 0; r < 16; ++r)
+                for (int r = 0; r < REGS; ++r)
                     acc[i][j][r] *= kSplitUnscale;
                 if (__all(split_finite(size)))
                     continue;
                 // clamped as the slabs' rows are
-                const int ra = m0 + (wm * TM + i) * 32 + frag_row, rb = n0 + (wn * TN + j) * 32 + frag_row;
-                const T *pa = A + (size_t)(ra < M ? ra : M - 1) * lda + 8 * (lane >> 5);
-                const T *pb = B + (size_t)(rb < N ? rb : N - 1) * ldb + 8 * (lane >> 5);
+                const int ra = m0 + (wm * TM + i) * BLK + frag_row, rb = n0 + (wn * TN + j) * BLK + frag_row;
+                const T *pa = A + (size_t)(ra < M ? ra : M - 1) * lda + BLK / 4 * (lane / BLK);
+                const T *pb = B + (size_t)(rb < N ? rb : N - 1) * ldb + BLK / 4 * (lane / BLK);
                 if constexpr (CFG::OWN)
                     multiply_again(pa, pb, nk * wk / WGK * STEPS, nk * (wk + 1) / WGK * STEPS, 1, acc[i][j]);
                 else
@@ -1823,7 +1852,7 @@ __global__ void __launch_bounds__(CFG::NT)
     constexpr int SSTR = CFG::SSTR;     // staged row stride in 32-bit words (16-byte pad spreads the b128 banks)
     typedef AccT acc4 __attribute__((ext_vector_type(4)));
     AccT *const stage_all = reinterpret_cast<AccT *>(lds_dyn);
-    AccT *const stage_me  = stage_all + wave * (32 * SSTR);  // wave = (wm*WGN + wn)*WGK + wk
+    AccT *const stage_me  = stage_all + wave * (GROWS * SSTR);  // wave = (wm*WGN + wn)*WGK + wk
     const int tid_piece = tid % CPR, tid_rowpos = tid / CPR;
     __syncthreads();  // every wave is done reading the slabs
     TR_TL(2);         // main loop done
@@ -1861,9 +1890,13 @@ __global__ void __launch_bounds__(CFG::NT)
         static_assert(CFG::NSTAGE > 0, "LayerNorm-folding epilogues run on the direct-to-LDS pipeline");
 #pragma unroll
         for (int i = 0; i < TM; ++i) {
-            const double s1 = ln_s1[i] + __shfl_xor(ln_s1[i], 32, 64), s2 = ln_s2[i] + __shfl_xor(ln_s2[i], 32, 64);
-            if (lane < 32)
-                row_part[(wk * WGN + wn) * BM + (wm * TM + i) * 32 + frag_row] = make_double2(s1, s2);
+            double s1 = ln_s1[i] + __shfl_xor(ln_s1[i], 32, 64), s2 = ln_s2[i] + __shfl_xor(ln_s2[i], 32, 64);
+            if constexpr (BLK == 16) {
+                s1 += __shfl_xor(s1, 16, 64);
+                s2 += __shfl_xor(s2, 16, 64);
+            }
+            if (lane < BLK)
+                row_part[(wk * WGN + wn) * BM + (wm * TM + i) * BLK + frag_row] = make_double2(s1, s2);
         }
         __syncthreads();
         if (tid < BM) {
@@ -1897,15 +1930,23 @@ __global__ void __launch_bounds__(CFG::NT)
         }
     }
 #pragma unroll
-    for (int i = 0; i < TM; ++i) {
+    for (int i = 0; i < GROUPS; ++i) {
+        if constexpr (BLK == 32) {
 #pragma unroll
-        for (int j = 0; j < TN; ++j)
+            for (int j = 0; j < TN; ++j)
 #pragma unroll
-            for (int r4 = 0; r4 < 4; ++r4)
-                *reinterpret_cast<acc4 *>(stage_me + (lane & 31) * SSTR + j * 32 + 8 * r4 + 4 * (lane >> 5)) =
-                    acc4{acc[i][j][r4 * 4 + 0], acc[i][j][r4 * 4 + 1], acc[i][j][r4 * 4 + 2], acc[i][j][r4 * 4 + 3]};
+                for (int r4 = 0; r4 < 4; ++r4)
+                    *reinterpret_cast<acc4 *>(stage_me + (lane & 31) * SSTR + j * 32 + 8 * r4 + 4 * (lane >> 5)) =
+                        acc4{acc[i][j][r4 * 4 + 0], acc[i][j][r4 * 4 + 1], acc[i][j][r4 * 4 + 2], acc[i][j][r4 * 4 + 3]};
+        } else {
+#pragma unroll
+            for (int b = 0; b < TM; ++b)
+#pragma unroll
+                for (int j = 0; j < TN; ++j)
+                    *reinterpret_cast<acc4 *>(stage_me + (b * 16 + (lane & 15)) * SSTR + j * 16 + 4 * (lane >> 4)) = acc[b][j];
+        }
         if constexpr (Epi::kRowStats) {
-            if (i == TM - 1) {
+            if (i == GROUPS - 1) {
 #pragma unroll
                 for (int q = 0; q < YPRE; ++q) {
                     const int item = tid + q * NT;
@@ -1937,18 +1978,18 @@ __global__ void __launch_bounds__(CFG::NT)
                 piece  = item % CPR;
                 rowpos = item / CPR;
             }
-            const int c8  = by_rows ? ((item >> 5) % CPR) * 8 : piece * 8;
-            const int row = by_rows ? (item & 31) : rowpos % 32;
-            const int pos = rowpos / 32;  // = item / (CPR * 32) = pm * WGN + pn
-            const AccT *src = stage_all + (pos * WGK) * (32 * SSTR) + row * SSTR + c8;
+            const int c8  = by_rows ? ((item / GROWS) % CPR) * 8 : piece * 8;
+            const int row = by_rows ? (item % GROWS) : rowpos % GROWS;
+            const int pos = rowpos / GROWS;  // = item / (CPR * GROWS) = pm * WGN + pn
+            const AccT *src = stage_all + (pos * WGK) * (GROWS * SSTR) + row * SSTR + c8;
             acc4 lo = *reinterpret_cast<const acc4 *>(src);
             acc4 hi = *reinterpret_cast<const acc4 *>(src + 4);
 #pragma unroll
             for (int q = 1; q < WGK; ++q) {
-                lo += *reinterpret_cast<const acc4 *>(src + q * (32 * SSTR));
-                hi += *reinterpret_cast<const acc4 *>(src + q * (32 * SSTR) + 4);
+                lo += *reinterpret_cast<const acc4 *>(src + q * (GROWS * SSTR));
+                hi += *reinterpret_cast<const acc4 *>(src + q * (GROWS * SSTR) + 4);
             }
-            const int m = m0 + ((pos / WGN) * TM + i) * 32 + row;
+            const int m = m0 + ((pos / WGN) * GROUPS + i) * GROWS + row;
             const int n = n0 + (pos % WGN) * CW + c8;
             const int nl = (pos % WGN) * CW + c8;  // column inside the tile
             const u32x4 *const ahead = AHEAD > 0 ? ahead_vec : nullptr;
@@ -1975,7 +2016,7 @@ __global__ void __launch_bounds__(CFG::NT)
                     if (piece == 0 && m < M && n < N)
                         store_out8(epi.through, &epi.row_sums[(size_t)(n / CFG::sum_cols) * M + m], sm);
                 } else {
-                    reinterpret_cast<float2 *>(lds_dyn + CFG::sums_offset)[(((pos / WGN) * TM + i) * 32 + row) * (BN / 8) +
+                    reinterpret_cast<float2 *>(lds_dyn + CFG::sums_offset)[(((pos / WGN) * GROUPS + i) * GROWS + row) * (BN / 8) +
                                                                          ((pos % WGN) * CW + c8) / 8] = sm;
                 }
             } else if (m < M) {
@@ -1997,13 +2038,13 @@ __global__ void __launch_bounds__(CFG::NT)
                             AccT x = src[t];
 #pragma unroll
                             for (int q = 1; q < WGK; ++q)
-                                x += src[q * (32 * SSTR) + t];
+                                x += src[q * (GROWS * SSTR) + t];
                             epi.store(m, n + t, x, epi.col_const(n + t));
                         }
                 }
             }
         }
-        if (i + 1 < TM)
+        if (i + 1 < GROUPS)
             __syncthreads();
     }
     TR_TL(3);  // C stored
@@ -2123,8 +2164,9 @@ int launch_tiled(hipStream_t s, const void *A, const void *B, int M, int N, int 
 //   9111141   32 x  32, 4 k-waves with rings of their own     9121141   32 x  64, likewise
 //   3112221   64 x  64, 8 waves (two k-waves), 3 stages       3112222   64 x  64, 8 waves, 256-byte slabs
 //   4221141   64 x  64, 4 k-waves, 4 stages                   3212221  128 x  64, 8 waves
+//   6111141   16 x  16, 6211141 32 x 16, 6121141 16 x 32: 16 x 16 blocks, 4 k-waves with rings of their own (three slabs)
 //   2112211   64 x  64, 4 waves, 2 stages                     2222221  128 x 128, 8 waves (two k-waves)
-//   fp32 only: 9111181 32 x 32, 8 k-waves; 9221141 64 x 64, 4 k-waves with rings of their own;
+//   fp32 only: 6111181, 6211181 16 x 16 and 32 x 16, 8 k-waves; 9111181 32 x 32, 8 k-waves; 9221141 64 x 64, 4 k-waves with rings of their own;
 //   2321142, 2231142, 2331142 96 x 64, 64 x 96 and 96 x 96, 4 k-waves; 2222121, 2332121 128 x 64 and 192 x 96, 4 waves (two k-waves)
 //   3332221  192 x 192, 8 waves (two k-waves)                 3331182   96 x  96, 8 k-waves, 256-byte slabs
 //   112210    64 x  64 and 222210 128 x 128, 4 waves: rows that are no multiple of 128 bytes
@@ -2151,6 +2193,9 @@ struct TileCost {
     float fixed, round, slab[4];
 };
 constexpr TileCost kTilesHalf[] = {
+    {6111141, 16, 16, 3, 3.51f, 1.75f, {0.027f, 0.068f, 0.093f}},
+    {6211141, 32, 16, 2, 3.56f, 2.22f, {0.042f, 0.088f}},
+    {6121141, 16, 32, 2, 3.68f, 1.95f, {0.046f, 0.093f}},
     {9111141, 32, 32, 2, 3.47f, 2.09f, {0.067f, 0.147f}},
     {9121141, 32, 64, 1, 3.46f, 2.56f, {0.121f}},
     {3112221, 64, 64, 3, 3.72f, 3.06f, {0.205f, 0.377f, 0.654f}},
@@ -2162,9 +2207,20 @@ constexpr TileCost kTilesHalf[] = {
     {3332221, 192, 192, 1, 10.15f, 13.25f, {0.767f}},
     {3331182, 96, 96, 1, 6.94f, 7.10f, {0.264f}},
 };
+// Tiles of 16 x 16 blocks are for the products whose 32x32 tiles are too few for the chip: a CU's panels come through its L1 at
+// 64 bytes a clock at best, so 24 tiles of (32 + 32) rows of K=3072 take 4 us for that alone, and 96 of (16 + 16) rows half.
+// us a launch, best shape before -> now (fp32: 8 waves where K is long):
+//   M= 32 N= 768 K=3072 fp16  7.4 -> 5.0   int8 5.0 -> 4.1   fp32 14.9 -> 8.8     M= 32 N=768 K=768 fp16 3.9 -> 3.2, fp32 6.4 -> 4.6
+//   M=128 N= 768 K=3072 fp16  7.5 -> 6.0   int8 5.4 -> 4.7   fp32 14.9 -> 12.1    M=128 N=768 K=768 fp16 4.3 -> 3.5, fp32 6.7 -> 5.8
+//   M= 32 N=2304 K=768  fp16  4.7 -> 4.5 (folded LayerNorm)  fp32  6.7 -> 5.9
+// (Measured and not taken: eight waves for fp16 and int8, 0.1 .. 0.4 us behind; rings of four slabs, 0.1 behind.  The int8 rows'
+// fixed part is 0.2 us below its fit: the other int8 rows were fitted on a faster machine.)
 // (int8, 64x64 tiles: the slab of four tiles was fitted to 0.944; 4096 x 2304 x 768 then took 128x128 tiles, 1.4 % ahead by the
 // fit and 0 .. 1 us a launch behind in the network)
 constexpr TileCost kTilesI8[] = {
+    {6111141, 16, 16, 3, 3.10f, 1.66f, {0.036f, 0.078f, 0.087f}},
+    {6211141, 32, 16, 2, 3.10f, 1.71f, {0.052f, 0.097f}},
+    {6121141, 16, 32, 2, 3.10f, 1.69f, {0.053f, 0.095f}},
     {9111141, 32, 32, 2, 2.98f, 1.93f, {0.078f, 0.151f}},
     {9121141, 32, 64, 1, 3.25f, 2.21f, {0.130f}},
     {3112221, 64, 64, 3, 3.40f, 2.05f, {0.218f, 0.398f, 0.701f}},
@@ -2186,19 +2242,26 @@ constexpr TileCost kTilesI8[] = {
 // Error against float64 (2-norm over 2-norm; 300 x 760 x 768 / 129 x 264 x 3072): 1.5e-7 .. 3e-7 / 3e-7 .. 6e-7 by shape,
 // v_mfma_f32_32x32x2_f32: 5.0e-7 / 9.9e-7.
 constexpr TileCost kTilesF32[] = {
-    {9111141, 32, 32, 2, 4.03f, 1.54f, {0.116f, 0.263f}},
-    {9121141, 32, 64, 1, 5.00f, 4.51f, {0.194f}},
-    {9111181, 32, 32, 1, 4.39f, 3.30f, {0.118f}},
-    {9221141, 64, 64, 1, 6.18f, 7.25f, {0.308f}},
-    {2321142, 96, 64, 1, 5.78f, 9.00f, {0.442f}},
-    {2231142, 64, 96, 1, 6.67f, 10.25f, {0.439f}},
-    {2331142, 96, 96, 1, 8.11f, 15.21f, {0.616f}},
-    {2222121, 128, 64, 2, 5.82f, 10.41f, {0.591f, 1.363f}},
-    {2222221, 128, 128, 1, 7.62f, 19.83f, {1.060f}},
-    {2332121, 192, 96, 1, 9.09f, 24.17f, {1.170f}},
+    {6111141, 16, 16, 3, 3.80f, 1.14f, {0.054f, 0.107f, 0.164f}},
+    {6211141, 32, 16, 2, 3.83f, 1.35f, {0.089f, 0.184f}},
+    {6121141, 16, 32, 2, 4.03f, 1.50f, {0.086f, 0.178f}},
+    {6111181, 16, 16, 1, 3.71f, 2.33f, {0.053f}},
+    {6211181, 32, 16, 1, 3.97f, 2.67f, {0.086f}},
+    {9111141, 32, 32, 2, 3.92f, 1.81f, {0.115f, 0.253f}},
+    {9121141, 32, 64, 1, 4.69f, 4.59f, {0.199f}},
+    {9111181, 32, 32, 1, 4.27f, 3.31f, {0.120f}},
+    {9221141, 64, 64, 1, 6.03f, 7.55f, {0.312f}},
+    {2321142, 96, 64, 1, 5.69f, 9.55f, {0.445f}},
+    {2231142, 64, 96, 1, 6.64f, 10.54f, {0.442f}},
+    {2331142, 96, 96, 1, 8.12f, 15.53f, {0.619f}},
+    {2222121, 128, 64, 2, 5.87f, 11.44f, {0.593f, 1.378f}},
+    {2222221, 128, 128, 1, 7.53f, 20.38f, {1.065f}},
+    {2332121, 192, 96, 1, 9.10f, 25.11f, {1.177f}},
 };
 
-template <int COUNT> inline int pick_tile_config(const TileCost (&shapes)[COUNT], long M, long N, size_t kbytes) {
+// row_stats: the shape takes the rows' statistics from its own A fragments, which 32 rows of 16 x 16 blocks pay for with twice the
+// sums a wave (M=32 N=2304 K=768: 4.8 us, with 16 x 32 tiles 4.5)
+template <int COUNT> inline int pick_tile_config(const TileCost (&shapes)[COUNT], long M, long N, size_t kbytes, bool row_stats) {
     int best        = 0;
     float best_cost = 0.f;
     const float slabs = (float)(kbytes / 128);
@@ -2208,7 +2271,7 @@ template <int COUNT> inline int pick_tile_config(const TileCost (&shapes)[COUNT]
         const long tiles = ((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn), n = (tiles + kNumCU - 1) / kNumCU;
         const long sets = n / t.slots, rest = n % t.slots;
         float cost = t.fixed + slabs * ((float)sets * t.slab[t.slots - 1] + (rest ? t.slab[rest - 1] : 0.f)) +
-                     t.round * (float)(sets + (rest ? 1 : 0) - 1);
+                     t.round * (float)(sets + (rest ? 1 : 0) - 1) + (row_stats && t.code / 100000 == 62 ? 0.4f : 0.f);
         if (best == 0 || cost < best_cost)
             best = t.code, best_cost = cost;
     }
@@ -2228,11 +2291,11 @@ int launch_gemm_fast(hipStream_t s, const void *A, const void *B, int M, int N, 
         if (kbytes % 128 != 0 || wide)
             cfg = (((long)M + 127) / 128) * (((long)N + 127) / 128) > kNumCU ? 222210 : 112210;
         else if (DT == TNN_ROCM_F32)
-            cfg = pick_tile_config(kTilesF32, M, N, kbytes);
+            cfg = pick_tile_config(kTilesF32, M, N, kbytes, Epi::kRowStats);
         else if (DT == TNN_ROCM_I8)
-            cfg = pick_tile_config(kTilesI8, M, N, kbytes);
+            cfg = pick_tile_config(kTilesI8, M, N, kbytes, Epi::kRowStats);
         else
-            cfg = pick_tile_config(kTilesHalf, M, N, kbytes);
+            cfg = pick_tile_config(kTilesHalf, M, N, kbytes, Epi::kRowStats);
     }
     switch (cfg) {  // a code of 128-byte or larger slabs without its stage digit
         case 112211: cfg = 2112211; break;
@@ -2257,16 +2320,31 @@ int launch_gemm_fast(hipStream_t s, const void *A, const void *B, int M, int N, 
     return launch_tiled<DT, TileCfg<TMv, TNv, WGMv, WGNv, WGKv, SLABv>, Epi>(s, A, B, M, N, K, lda, ldb, epi)
 #define TR_FAST_DL(TMv, TNv, WGMv, WGNv, WGKv, SLABv, NSv)                                                            \
     return launch_tiled<DT, TileCfg<TMv, TNv, WGMv, WGNv, WGKv, SLABv, NSv>, Epi>(s, A, B, M, N, K, lda, ldb, epi)
+#define TR_FAST_SMALL(TMv, TNv, WGKv, SLABv, NSv)                                                                     \
+    return launch_tiled<DT, TileCfg<TMv, TNv, 1, 1, WGKv, SLABv, NSv, true, 16>, Epi>(s, A, B, M, N, K, lda, ldb, epi)
 #define TR_FAST_OWN(TMv, TNv, WGKv, SLABv, NSv)                                                                       \
     return launch_tiled<DT, TileCfg<TMv, TNv, 1, 1, WGKv, SLABv, NSv, true>, Epi>(s, A, B, M, N, K, lda, ldb, epi)
     if constexpr (TakesRowSums<Epi>::value) {
-        if (cfg >= 9000000)
+        if (cfg >= 6000000)
             return kNotWithRowSums;
     } else {
         switch (cfg) {
             case 9111141: TR_FAST_OWN(1, 1, 4, 128, 2);
             case 9121141: TR_FAST_OWN(1, 2, 4, 128, 2);
             default: break;
+        }
+        switch (cfg) {
+            case 6111141: TR_FAST_SMALL(1, 1, 4, 128, 3);
+            case 6211141: TR_FAST_SMALL(2, 1, 4, 128, 3);
+            case 6121141: TR_FAST_SMALL(1, 2, 4, 128, 3);
+            default: break;
+        }
+        if constexpr (DT == TNN_ROCM_F32) {
+            switch (cfg) {
+                case 6111181: TR_FAST_SMALL(1, 1, 8, 128, 3);
+                case 6211181: TR_FAST_SMALL(2, 1, 8, 128, 3);
+                default: break;
+            }
         }
     }
     if constexpr (DT == TNN_ROCM_F32) {
@@ -2302,6 +2380,7 @@ int launch_gemm_fast(hipStream_t s, const void *A, const void *B, int M, int N, 
         }
     }
 #undef TR_FAST_OWN
+#undef TR_FAST_SMALL
 #undef TR_FAST
 #undef TR_FAST_DL
     set_error("gemm: unknown tuning configuration %d", cfg);

@@ -28,6 +28,7 @@ namespace tnn_rocm {
 typedef __bf16 split_bf16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 split_bf16x8 __attribute__((ext_vector_type(8)));
 typedef float split_f32x2 __attribute__((ext_vector_type(2)));
+typedef float split_f32x4 __attribute__((ext_vector_type(4)));
 typedef float split_f32x16 __attribute__((ext_vector_type(16)));
 
 constexpr float kSplitScale   = 16777216.0f;                 // 2^24, of every operand
@@ -80,6 +81,12 @@ __device__ __forceinline__ void split_mma(const Split3 &a, const Split3 &b, int 
     const u32x4 va = {a.p[pa][0], a.p[pa][1], a.p[pa][2], a.p[pa][3]}, vb = {b.p[pb][0], b.p[pb][1], b.p[pb][2], b.p[pb][3]};
     c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(split_bf16x8, va), __builtin_bit_cast(split_bf16x8, vb), c,
                                                 0, 0, 0);
+}
+__device__ __forceinline__ void split_mma(const Split3 &a, const Split3 &b, int product, split_f32x4 &c) {  // of 16 x 16 blocks
+    const int pa = kSplitOrder[product][0], pb = kSplitOrder[product][1];
+    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+    const u32x4 va = {a.p[pa][0], a.p[pa][1], a.p[pa][2], a.p[pa][3]}, vb = {b.p[pb][0], b.p[pb][1], b.p[pb][2], b.p[pb][3]};
+    c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(split_bf16x8, va), __builtin_bit_cast(split_bf16x8, vb), c, 0, 0, 0);
 }
 
 // is x, a value without sign, neither infinite nor a NaN?  On the bits: of a sum of magnitudes "< INFINITY" the compiler makes
