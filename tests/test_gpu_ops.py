@@ -684,6 +684,42 @@ def test_gemm_fp32_split_shapes(code, M, N, K):
     assert (np.abs(got[fine] - exact[fine]) <= 2.0 ** -24 * 4 * np.sqrt(K) * size[fine]).all()
 
 
+@pytest.mark.parametrize("code", [2222221, 3212221, 3332221, 2244211])
+@pytest.mark.parametrize("slabs", [1, 2, 3, 4, 5, 8])
+def test_gemm_fragments_read_ahead(code, slabs):
+    """Shapes that read a slab's first fragments under the slab before: loops of every length (fewer slabs than stages, the last
+    ones whose successors are not requested any more), whole tiles and remainders, every epilogue; handed-over row sums against
+    sums in double."""
+    from tnn_amd import capi
+    lib = capi.load()
+    K = 64 * slabs
+    rng = np.random.default_rng(code % 1000 + slabs)
+    say("tile configuration %d, %d slabs" % (code, slabs))
+    if slabs % 4 == 0:
+        test_gemm_small_product_shapes(code, 257, 264, K)
+    o = ops()
+    for td in (torch.float16, torch.bfloat16):
+        M, N = 300, 264
+        a, w = (torch.from_numpy(rng.standard_normal(n).astype(np.float32)).to(td) for n in ((M, K), (N, K)))
+        lib.tnn_rocm_debug_set_gemm_config(code)
+        try:
+            got = host(o.gemm(a.cuda(), w.cuda(), True).float()).astype(np.float64)
+            if slabs % 2 == 0:
+                for blocks in (2, 12, 24):  # few enough for the shape to ask for them late, and more
+                    part = torch.zeros(blocks, M, 2)
+                    part[blocks - 1, :, 0], part[blocks - 1, :, 1] = a.double().sum(1), (a.double() ** 2).sum(1)
+                    cs, zero = w.double().sum(1).float(), torch.zeros(N)
+                    fed = o.gemm_ln(a.cuda(), w.cuda(), zero.cuda(), cs.cuda(), 1e-5, row_sums=(part.cuda(), blocks))
+                    norm = ((a.double() - a.double().mean(1, keepdim=True)) / (a.double().var(1, unbiased=False, keepdim=True) + 1e-5).sqrt())
+                    ref = host(norm @ w.double().T)
+                    assert rel_err(host(fed.float()), ref) <= (FP16_TOL if td is torch.float16 else 2e-2), blocks
+        finally:
+            lib.tnn_rocm_debug_set_gemm_config(0)
+        exact = a.double().numpy() @ w.double().numpy().T
+        # one rounding of the result (11 or 8 bits) and fp32 sums
+        assert np.abs(got - exact).max() <= (2.0 ** -11 if td is torch.float16 else 2.0 ** -8) * np.abs(exact).max() + 1e-4 * np.sqrt(K)
+
+
 @pytest.mark.parametrize("code", [6111141, 6211141, 6121141])
 @pytest.mark.parametrize("M,N,K", [(1, 8, 256), (17, 24, 256), (33, 776, 768), (130, 136, 3072)])
 def test_gemm_16x16_blocks(code, M, N, K):

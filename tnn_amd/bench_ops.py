@@ -189,7 +189,7 @@ def mall_probe(launches=20):
 TILE_SHAPES = {
     "half": ((6111141, 16, 16, 3), (6211141, 32, 16, 2), (6121141, 16, 32, 2), (9111141, 32, 32, 2), (9121141, 32, 64, 1),
              (3112221, 64, 64, 3), (3112222, 64, 64, 1), (3212221, 128, 64, 2), (4221141, 64, 64, 2), (2112211, 64, 64, 4),
-             (2222221, 128, 128, 2), (3332221, 192, 192, 1), (3331182, 96, 96, 1)),
+             (2222221, 128, 128, 2), (3332221, 192, 192, 1), (3331182, 96, 96, 1), (2244211, 256, 256, 1)),
     "f32": ((6111141, 16, 16, 3), (6211141, 32, 16, 2), (6121141, 16, 32, 2), (6111181, 16, 16, 1), (6211181, 32, 16, 1),
             (9111141, 32, 32, 2), (9121141, 32, 64, 1), (9111181, 32, 32, 1), (9221141, 64, 64, 1), (2321142, 96, 64, 1),
             (2231142, 64, 96, 1), (2331142, 96, 96, 1), (2222121, 128, 64, 2), (2222221, 128, 128, 1), (2332121, 192, 96, 1))}

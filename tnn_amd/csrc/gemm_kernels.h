@@ -1609,11 +1609,20 @@ __global__ void __launch_bounds__(CFG::NT)
                 }
             }
         };
+        // Waves with more than one block and more than one step a slab: step s + 1's fragments are read between the MFMAs of step s,
+        // and so are the first ones of the next slab, whose barrier stands in front of the last step.  Read behind the barrier,
+        // they are a burst of all waves' reads that no MFMA covers (256 x 256: 48 KB, 380 of 2400 clocks a slab).  fp16, us,
+        // burst -> this: 192 x 192 tiles 3072 x 3072 x 768 23.0 -> 22.6, 3072 x 768 x 3072 45.9 -> 39.2; 128 x 128 tiles
+        // 3072 x 2304 x 768 18.9 -> 18.1, 8192 x 1024 x 4096 72.3 -> 70.8; 128 x 64 tiles 256 x 768 x 768 7.2 -> 6.5; 256 x 256
+        // tiles 8192 x 4096 x 4096 239 -> 228.  (Waves with one block have nothing to hide them behind: 64 x 64 tiles
+        // 256 x 3072 x 768 6.3 -> 6.6 and 6.7 -> 6.9, four waves 985 x 2304 x 768 9.7 -> 10.1.)
+        constexpr bool PIPE = DT != TNN_ROCM_F32 && CFG::NW == 8 && KSTEPS >= 2 && TM * TN > 1;
+        static_assert(!PIPE || KSTEPS % 2 == 0, "two sets of fragments, every slab begins with the first");
         if constexpr (TakesRowSums<Epi>::value && !kLateSums)
             request_sums();
         int issued = 0;
 #pragma unroll
-        for (int p = 0; p < NS - 1; ++p)
+        for (int p = 0; p < (PIPE ? NS : NS - 1); ++p)
             if (p < nk)
                 issue(p, p), ++issued;
         TR_TL(5);  // first slabs requested
@@ -1650,7 +1659,92 @@ __global__ void __launch_bounds__(CFG::NT)
             stage = stage + 1 == NS ? 0 : stage + 1;
             fill  = fill + 1 == NS ? 0 : fill + 1;
         };
-        if constexpr (kLateSums) {
+        if constexpr (PIPE) {
+            constexpr int READS = TM + TN, MFMAS = TM * TN;
+            uint4 fa[2][TM][1], fb[2][TN][1];
+            int chunk[KSTEPS];
+#pragma unroll
+            for (int ks = 0; ks < KSTEPS; ++ks)
+                chunk[ks] = frow + (((wk + ks * WGK) * 2 + (lane >> 5)) ^ fswz) * 16;
+            auto read_one = [&](int k, int ks, int from) __attribute__((always_inline)) {  // fragment k of step ks
+                const unsigned char *at = lds_dyn + from * STAGE + chunk[ks];
+                if (k < TM)
+                    fa[ks & 1][k < TM ? k : 0][0] = *reinterpret_cast<const uint4 *>(at + (wm * TM + k) * 32 * SLAB);
+                else
+                    fb[ks & 1][k >= TM ? k - TM : 0][0] = *reinterpret_cast<const uint4 *>(at + BM * SLAB + (wn * TN + k - TM) * 32 * SLAB);
+            };
+            // slab kt, the first of whose fragments have been read; MORE: another one follows, LOADS: and one is requested
+            auto slab = [&](int kt, auto more, auto loads) __attribute__((always_inline)) {
+                constexpr bool MORE = decltype(more)::value, LOADS = decltype(loads)::value;
+                const int here = stage, next = stage + 1 == NS ? 0 : stage + 1;
+#pragma unroll
+                for (int ks = 0; ks < KSTEPS; ++ks) {
+                    const bool last = ks == KSTEPS - 1;
+                    if (last && MORE) {
+                        // this wave's fragments of slab kt are in registers; slab kt + 1 has landed once at most the loads of
+                        // the slabs requested after it are outstanding
+                        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+                        if (NS > 2 && kt + 2 < nk)
+                            TR_WAIT_VMCNT(NS > 2 ? LPW : 0);
+                        else
+                            TR_WAIT_VMCNT(0);
+                        __builtin_amdgcn_s_barrier();
+                        asm volatile("" ::: "memory");
+                    }
+                    if (last && !MORE && kLateSums)
+                        request_sums();
+                    if constexpr (Epi::kRowStats && !TakesRowSums<Epi>::value) {
+#pragma unroll
+                        for (int i = 0; i < TM; ++i)
+                            if ((i + ks) % WGN == wn)
+                                ln_take(fa[ks & 1][i][0], i);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int q = 0; q < MFMAS; ++q) {
+                        GemmTraits<DT>::mma(fb[ks & 1][q % TN][0], fa[ks & 1][q / TN][0], acc[q / TN][q % TN]);
+                        __builtin_amdgcn_sched_barrier(0);
+                        if (!last || MORE) {
+#pragma unroll
+                            for (int k = READS * q / MFMAS; k < READS * (q + 1) / MFMAS; ++k)
+                                read_one(k, last ? 0 : ks + 1, last ? next : here);
+                        }
+                        if (last && LOADS) {
+#pragma unroll
+                            for (int k = LPW * q / MFMAS; k < LPW * (q + 1) / MFMAS; ++k)
+                                issue_one(k, kt + NS, here);
+                        }
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                }
+                stage = next;
+            };
+            {
+                const int behind = nk - 1 < NS - 1 ? nk - 1 : NS - 1;  // slabs requested after the first
+                if (behind >= 2)
+                    TR_WAIT_VMCNT(2 * LPW);
+                else if (behind == 1)
+                    TR_WAIT_VMCNT(LPW);
+                else
+                    TR_WAIT_VMCNT(0);
+                __builtin_amdgcn_s_barrier();
+                TR_TL(1);  // first slab landed
+                asm volatile("" ::: "memory");
+#pragma unroll
+                for (int k = 0; k < READS; ++k)
+                    read_one(k, 0, 0);
+            }
+            int kt = 0;
+            for (; kt + NS < nk; ++kt)
+                slab(kt, std::true_type(), std::true_type());
+            for (; kt + 1 < nk; ++kt)
+                slab(kt, std::true_type(), std::false_type());
+            slab(kt, std::false_type(), std::false_type());
+            if constexpr (kLateSums) {
+                finish_sums(0);
+                TR_TL(6);  // handed-over row sums added up
+            }
+        } else if constexpr (kLateSums) {
             // the last slab apart, so that the requested sums cross no loop edge on their way to the wait
             for (int kt = 0; kt + 1 < nk; ++kt)
                 step(kt, std::false_type());
@@ -2168,6 +2262,7 @@ int launch_tiled(hipStream_t s, const void *A, const void *B, int M, int N, int 
 //   2112211   64 x  64, 4 waves, 2 stages                     2222221  128 x 128, 8 waves (two k-waves)
 //   fp32 only: 6111181, 6211181 16 x 16 and 32 x 16, 8 k-waves; 9111181 32 x 32, 8 k-waves; 9221141 64 x 64, 4 k-waves with rings of their own;
 //   2321142, 2231142, 2331142 96 x 64, 64 x 96 and 96 x 96, 4 k-waves; 2222121, 2332121 128 x 64 and 192 x 96, 4 waves (two k-waves)
+//   2244211  256 x 256, 8 waves
 //   3332221  192 x 192, 8 waves (two k-waves)                 3331182   96 x  96, 8 k-waves, 256-byte slabs
 //   112210    64 x  64 and 222210 128 x 128, 4 waves: rows that are no multiple of 128 bytes
 // Eight-wave workgroups put two waves on every SIMD inside one tile: while one waits for its LDS fragments the
@@ -2206,7 +2301,12 @@ constexpr TileCost kTilesHalf[] = {
     {2222221, 128, 128, 2, 4.84f, 5.77f, {0.561f, 1.044f}},
     {3332221, 192, 192, 1, 10.15f, 13.25f, {0.767f}},
     {3331182, 96, 96, 1, 6.94f, 7.10f, {0.264f}},
+    {2244211, 256, 256, 1, 10.0f, 8.0f, {1.6f}},
 };
+// 256 x 256 tiles are for products that fill the chip with them: half the bytes a flop of 128 x 128 tiles.  Their row is set by
+// hand between the full and the half-empty rounds (a round of 192 tiles is 13 % shorter than one of 256, which a linear model
+// does not know).  us, 128 x 128 -> 256 x 256, GELU and folded LayerNorm: fp16 8192 x 4096 x 1024 97 -> 83, 4096 x 4096 x 1024 55
+// -> 46, 3072 x 4096 x 1024 43.4 -> 42.0; int8 8192 x 4096 x 1024 57.8 -> 52.4, 4096 x 4096 x 1024 28.4 -> 27.4.
 // Tiles of 16 x 16 blocks are for the products whose 32x32 tiles are too few for the chip: a CU's panels come through its L1 at
 // 64 bytes a clock at best, so 24 tiles of (32 + 32) rows of K=3072 take 4 us for that alone, and 96 of (16 + 16) rows half.
 // us a launch, best shape before -> now (fp32: 8 waves where K is long):
@@ -2231,6 +2331,7 @@ constexpr TileCost kTilesI8[] = {
     {2222221, 128, 128, 2, 5.15f, 3.79f, {0.640f, 1.156f}},
     {3332221, 192, 192, 1, 9.89f, 9.10f, {0.860f}},
     {3331182, 96, 96, 1, 6.72f, 5.80f, {0.314f}},
+    {2244211, 256, 256, 1, 10.6f, 8.2f, {2.1f}},
 };
 // fp32 on three bf16 planes: six matrix instructions per operand pair and the conversion between them, so a step costs five
 // times a half one.  Large wave tiles convert less per product, K is split over the waves of a CU wherever tiles are few, and
@@ -2369,6 +2470,7 @@ int launch_gemm_fast(hipStream_t s, const void *A, const void *B, int M, int N, 
             case 2222221: TR_FAST_DL(2, 2, 2, 2, 2, 128, 2);
             case 3332221: TR_FAST_DL(3, 3, 2, 2, 2, 128, 3);
             case 3331182: TR_FAST_DL(3, 3, 1, 1, 8, 256, 3);
+            case 2244211: TR_FAST_DL(2, 4, 4, 2, 1, 128, 2);
             default: break;
         }
     }
