@@ -229,6 +229,24 @@ __device__ __forceinline__ float wave_max(float v) {
     return v;
 }
 
+// v plus the v of lane ^ O, for O = 32, 16, 8, 4, 2, 1 in turn (from 4 on down the lanes of a row that differ in higher bits
+// hold the same value already, so that a rotation serves): register moves between lanes, where a shuffle goes through LDS at
+// some hundred clocks
+template <int O> __device__ __forceinline__ double add_lane_xor(double v) {
+    typedef uint32_t pair __attribute__((ext_vector_type(2)));
+    const pair u = __builtin_bit_cast(pair, v);
+    if constexpr (O >= 16) {
+        const auto lo = O == 32 ? __builtin_amdgcn_permlane32_swap(u.x, u.x, false, false) : __builtin_amdgcn_permlane16_swap(u.x, u.x, false, false);
+        const auto hi = O == 32 ? __builtin_amdgcn_permlane32_swap(u.y, u.y, false, false) : __builtin_amdgcn_permlane16_swap(u.y, u.y, false, false);
+        return __builtin_bit_cast(double, pair{lo[0], hi[0]}) + __builtin_bit_cast(double, pair{lo[1], hi[1]});
+    } else {
+        constexpr int CTRL = O == 8 ? 0x128 : O == 4 ? 0x124 : O == 2 ? 0x4E : 0xB1;  // row_ror:8, row_ror:4, quad_perm
+        const pair w = {(uint32_t)__builtin_amdgcn_update_dpp(0, (int)u.x, CTRL, 0xf, 0xf, false),
+                        (uint32_t)__builtin_amdgcn_update_dpp(0, (int)u.y, CTRL, 0xf, 0xf, false)};
+        return v + __builtin_bit_cast(double, w);
+    }
+}
+
 // A kernel's arguments lie in cache lines that nothing on the chip has read yet.  The compiler loads them as it comes to them,
 // one miss after the other (1700 clocks to a GEMM's first slab request, with five lines); touched together they cost one.
 template <size_t BYTES> __device__ __forceinline__ void touch_kernel_args() {

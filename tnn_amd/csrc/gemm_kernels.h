@@ -1530,9 +1530,8 @@ __global__ void __launch_bounds__(CFG::NT)
             }
         };
         constexpr int LPW = A_LD + B_LD;
-        // A folding epilogue that is handed the row sums of A: the first BM threads request their row's sums (one
-        // 8-byte load per tile column of the kernel that wrote A), add them up and park {rstd, mean} behind everything
-        // else in LDS, where the epilogue finds them.  In the early form the loads are spelled as assembly like the
+        // A folding epilogue that is handed the row sums of A: the rows' sums (8 bytes per tile column of the kernel that wrote
+        // A) are requested, added up, and {rstd, mean} parked behind everything else in LDS, where the epilogue finds them.  In the early form the loads are spelled as assembly like the
         // slab loads and the wait is placed by hand: the compiler knows nothing of the slabs in flight, and the wait it
         // would place itself (everything outstanding) would also wait for the slabs requested after the sums.  In the
         // late form they are ordinary loads.  When:
@@ -1544,30 +1543,42 @@ __global__ void __launch_bounds__(CFG::NT)
         //   early (shapes that share a CU, with up to 24 blocks: the 48 registers the sums would occupy through the last
         //         slab would cost a resident workgroup): before the first slabs, added up while those are on their way.  Older than
         //         every slab load, they are complete once at most the slab loads are outstanding.
+        // Every wave adds up the sums of BM / NW rows, 64 / that many lanes a row, each with its share of the blocks (where the
+        // rows of a tile do not divide so, the first BM threads a row each): one wave with 24 loads and 48 additions in double
+        // while the others wait for it took 0.5 us of a launch of 6.5 (256 x 2304 x 768).
         typedef float f32x2 __attribute__((ext_vector_type(2)));
-        constexpr int NSUM      = SumBlocks<Epi>::value;
-        constexpr bool kLateSums = TakesRowSums<Epi>::value && (EpiLds<CFG, Epi>::total > 80 * 1024 || NSUM <= 12);
+        constexpr bool kLateSums = TakesRowSums<Epi>::value && (EpiLds<CFG, Epi>::total > 80 * 1024 || SumBlocks<Epi>::value <= 12);
+        constexpr int ROWS_WAVE = BM / CFG::NW;
+        constexpr bool SHARED   = ROWS_WAVE == 8 || ROWS_WAVE == 16 || ROWS_WAVE == 32;
+        constexpr int LANES_ROW = SHARED ? 64 / ROWS_WAVE : 1;
+        constexpr int NSUM      = (SumBlocks<Epi>::value + LANES_ROW - 1) / LANES_ROW;  // blocks of a lane
+        const int sum_row  = SHARED ? wave * ROWS_WAVE + lane % ROWS_WAVE : tid;         // row of the tile
+        const int sum_part = SHARED ? lane / ROWS_WAVE : 0;
         f32x2 early[NSUM];
         auto request_sums = [&]() __attribute__((always_inline)) {
             if constexpr (TakesRowSums<Epi>::value) {
-                if (tid < BM) {
-                    const int m = m0 + tid < M ? m0 + tid : M - 1;
+                if (SHARED || tid < BM) {
+                    const int m = m0 + sum_row < M ? m0 + sum_row : M - 1;
 #pragma unroll
-                    for (int q = 0; q < NSUM; ++q) {
-                        early[q] = f32x2{0.f, 0.f};
-                        if (q < epi.ln.sum_blocks) {
-                            if constexpr (kLateSums)
-                                // ordinary loads: they are the youngest of the kernel, so the wait the compiler puts in
-                                // front of their first use (everything outstanding) is the wait that is wanted, and
-                                // the compiler knows the registers are not valid before it
-                                early[q] = *reinterpret_cast<const f32x2 *>(
-                                    reinterpret_cast<const char *>(epi.ln.row_sums) + ((size_t)q * M + m) * sizeof(float2));
-                            else
-                                asm volatile("global_load_dwordx2 %0, %1, %2"
-                                             : "=v"(early[q])
-                                             : "v"((uint32_t)(((size_t)q * M + m) * sizeof(float2))), "s"(epi.ln.row_sums)
-                                             : "memory");
-                        }
+                    for (int i = 0; i < NSUM; ++i) {
+                        // lanes that differ in their block: clamped, and what lies beyond the blocks is not added (a branch by
+                        // lane could copy a register before its load has arrived)
+                        const int k = i * LANES_ROW + sum_part, q = k < epi.ln.sum_blocks ? k : epi.ln.sum_blocks - 1;
+                        if (!SHARED)
+                            early[i] = f32x2{0.f, 0.f};
+                        if (!SHARED && k >= epi.ln.sum_blocks)
+                            continue;
+                        if constexpr (kLateSums)
+                            // ordinary loads: they are the youngest of the kernel, so the wait the compiler puts in
+                            // front of their first use (everything outstanding) is the wait that is wanted, and
+                            // the compiler knows the registers are not valid before it
+                            early[i] = *reinterpret_cast<const f32x2 *>(
+                                reinterpret_cast<const char *>(epi.ln.row_sums) + ((size_t)q * M + m) * sizeof(float2));
+                        else
+                            asm volatile("global_load_dwordx2 %0, %1, %2"
+                                         : "=v"(early[i])
+                                         : "v"((uint32_t)(((size_t)q * M + m) * sizeof(float2))), "s"(epi.ln.row_sums)
+                                         : "memory");
                     }
                 }
             }
@@ -1575,7 +1586,7 @@ __global__ void __launch_bounds__(CFG::NT)
         // slab_loads_behind: slab loads requested after the sums that may still be outstanding when the sums are read
         auto finish_sums = [&](int slab_loads_behind) __attribute__((always_inline)) {
             if constexpr (TakesRowSums<Epi>::value) {
-                if (tid < BM) {
+                if (SHARED || tid < BM) {
                     if constexpr (!kLateSums) {
                         if (slab_loads_behind >= 2)
                             TR_WAIT_VMCNT(2 * LPW);
@@ -1590,14 +1601,20 @@ __global__ void __launch_bounds__(CFG::NT)
                     // and its reciprocal root is taken in single precision with one Newton step.
                     double f1 = 0.0, f2 = 0.0;
 #pragma unroll
-                    for (int q = 0; q < NSUM; ++q) {
+                    for (int i = 0; i < NSUM; ++i) {
                         if constexpr (!kLateSums)
-                            asm volatile("" : "+v"(early[q]));  // not to be read before the wait above
-                        if (q < epi.ln.sum_blocks) {
-                            f1 += (double)early[q].x;
-                            f2 += (double)early[q].y;
+                            asm volatile("" : "+v"(early[i]));  // not to be read before the wait above
+                        if (i * LANES_ROW + sum_part < epi.ln.sum_blocks) {
+                            f1 += (double)early[i].x;
+                            f2 += (double)early[i].y;
                         }
                     }
+                    if constexpr (LANES_ROW >= 8)
+                        f1 = add_lane_xor<8>(f1), f2 = add_lane_xor<8>(f2);
+                    if constexpr (LANES_ROW >= 4)
+                        f1 = add_lane_xor<16>(f1), f2 = add_lane_xor<16>(f2);
+                    if constexpr (LANES_ROW >= 2)
+                        f1 = add_lane_xor<32>(f1), f2 = add_lane_xor<32>(f2);
                     const double mean = f1 * (double)epi.ln.inv_cols;
                     // fp32 block sums can leave E[x^2] - mean^2 a hair below zero for rows whose spread is tiny next to
                     // their mean; the variance is clamped there (with eps = 1e-12 the root would otherwise be NaN)
@@ -1605,7 +1622,8 @@ __global__ void __launch_bounds__(CFG::NT)
                     const float ve    = (float)((var > 0.0 ? var : 0.0) + (double)epi.ln.eps);
                     float r           = __builtin_amdgcn_rsqf(ve);
                     r                 = r * (1.5f - 0.5f * ve * r * r);
-                    reinterpret_cast<float2 *>(lds_dyn + CFG::lds_bytes)[tid] = make_float2(r, (float)mean);
+                    if (sum_part == 0)
+                        reinterpret_cast<float2 *>(lds_dyn + CFG::lds_bytes)[sum_row] = make_float2(r, (float)mean);
                 }
             }
         };
@@ -1984,11 +2002,9 @@ __global__ void __launch_bounds__(CFG::NT)
         static_assert(CFG::NSTAGE > 0, "LayerNorm-folding epilogues run on the direct-to-LDS pipeline");
 #pragma unroll
         for (int i = 0; i < TM; ++i) {
-            double s1 = ln_s1[i] + __shfl_xor(ln_s1[i], 32, 64), s2 = ln_s2[i] + __shfl_xor(ln_s2[i], 32, 64);
-            if constexpr (BLK == 16) {
-                s1 += __shfl_xor(s1, 16, 64);
-                s2 += __shfl_xor(s2, 16, 64);
-            }
+            double s1 = add_lane_xor<32>(ln_s1[i]), s2 = add_lane_xor<32>(ln_s2[i]);
+            if constexpr (BLK == 16)
+                s1 = add_lane_xor<16>(s1), s2 = add_lane_xor<16>(s2);
             if (lane < BLK)
                 row_part[(wk * WGN + wn) * BM + (wm * TM + i) * BLK + frag_row] = make_double2(s1, s2);
         }
@@ -2001,8 +2017,11 @@ __global__ void __launch_bounds__(CFG::NT)
                 s2 += v.y;
             }
             const double mean = s1 * (double)epi.ln.inv_cols;
-            const double var  = s2 * (double)epi.ln.inv_cols - mean * mean;
-            const float2 st   = make_float2((float)(1.0 / sqrt(var + (double)epi.ln.eps)), (float)mean);
+            const double var  = s2 * (double)epi.ln.inv_cols - mean * mean + (double)epi.ln.eps;
+            // the root's estimate (2^-26) after one Newton step is a few double ulps off, which its rounding does not see
+            const double r    = __builtin_amdgcn_rsq(var);
+            const double root = r > 1e-150 ? r + r * (0.5 - 0.5 * var * r * r) : r;  // (an infinite variance)
+            const float2 st   = make_float2((float)root, (float)mean);
             row_st[tid]       = st;
             if (epi.ln.stats && n0 == 0 && m0 + tid < M)  // every tile column holds them; the first one hands them on
                 store_out8(epi.through, &epi.ln.stats[m0 + tid], st);
