@@ -1627,20 +1627,21 @@ __global__ void __launch_bounds__(CFG::NT)
                 }
             }
         };
-        // Waves with more than one block and more than one step a slab: step s + 1's fragments are read between the MFMAs of step s,
-        // and so are the first ones of the next slab, whose barrier stands in front of the last step.  Read behind the barrier,
-        // they are a burst of all waves' reads that no MFMA covers (256 x 256: 48 KB, 380 of 2400 clocks a slab).  fp16, us,
-        // burst -> this: 192 x 192 tiles 3072 x 3072 x 768 23.0 -> 22.6, 3072 x 768 x 3072 45.9 -> 39.2; 128 x 128 tiles
-        // 3072 x 2304 x 768 18.9 -> 18.1, 8192 x 1024 x 4096 72.3 -> 70.8; 128 x 64 tiles 256 x 768 x 768 7.2 -> 6.5; 256 x 256
-        // tiles 8192 x 4096 x 4096 239 -> 228.  (Waves with one block have nothing to hide them behind: 64 x 64 tiles
-        // 256 x 3072 x 768 6.3 -> 6.6 and 6.7 -> 6.9, four waves 985 x 2304 x 768 9.7 -> 10.1.)
-        constexpr bool PIPE = DT != TNN_ROCM_F32 && CFG::NW == 8 && KSTEPS >= 2 && TM * TN > 1;
+        // Large wave tiles with more than one step a slab: step s + 1's fragments are read between the MFMAs of step s, and so are
+        // the first ones of the next slab, whose barrier stands in front of the last step.  Read behind the barrier, they are a
+        // burst of all waves' reads that no MFMA covers (256 x 256: 48 KB, 380 of 2400 clocks a slab).  fp16, us, burst -> this:
+        // 192 x 192 tiles 3072 x 3072 x 768 23.0 -> 22.6, 3072 x 768 x 3072 45.9 -> 39.2; 256 x 256 tiles 8192 x 4096 x 4096
+        // 239 -> 228.  Not where two workgroups share a CU and cover each other: 128 x 128 tiles gain back to back
+        // (3072 x 2304 x 768 18.9 -> 18.1), but with operands that come from the memory-side cache, as in a network, they lose
+        // (17.5 -> 17.7; twelve layers of 8 x 384 tokens 1134 -> 1145 us over eight instances).  Waves with one block have
+        // nothing to hide the reads behind: 64 x 64 tiles 256 x 3072 x 768 6.3 -> 6.6, four waves 985 x 2304 x 768 9.7 -> 10.1.
+        constexpr bool PIPE = DT != TNN_ROCM_F32 && CFG::NW == 8 && KSTEPS >= 2 && TM * TN > 4;
         static_assert(!PIPE || KSTEPS % 2 == 0, "two sets of fragments, every slab begins with the first");
         if constexpr (TakesRowSums<Epi>::value && !kLateSums)
             request_sums();
         int issued = 0;
 #pragma unroll
-        for (int p = 0; p < (PIPE ? NS : NS - 1); ++p)
+        for (int p = 0; p < NS - 1; ++p)
             if (p < nk)
                 issue(p, p), ++issued;
         TR_TL(5);  // first slabs requested
@@ -1738,11 +1739,9 @@ __global__ void __launch_bounds__(CFG::NT)
                 stage = next;
             };
             {
-                const int behind = nk - 1 < NS - 1 ? nk - 1 : NS - 1;  // slabs requested after the first
-                if (behind >= 2)
-                    TR_WAIT_VMCNT(2 * LPW);
-                else if (behind == 1)
-                    TR_WAIT_VMCNT(LPW);
+                static_assert(NS <= 3, "waits written for up to three stages");
+                if (NS > 2 && nk > 1)
+                    TR_WAIT_VMCNT(NS > 2 ? LPW : 0);
                 else
                     TR_WAIT_VMCNT(0);
                 __builtin_amdgcn_s_barrier();
@@ -1751,6 +1750,10 @@ __global__ void __launch_bounds__(CFG::NT)
 #pragma unroll
                 for (int k = 0; k < READS; ++k)
                     read_one(k, 0, 0);
+                // the last stage's slab only now: all workgroups start together, and what they request ahead stands in the way
+                // of one another's first slabs
+                if (NS - 1 < nk)
+                    issue(NS - 1, NS - 1);
             }
             int kt = 0;
             for (; kt + NS < nk; ++kt)
