@@ -1088,6 +1088,21 @@ def test_attention_fp32(B, h, S, masked):
     assert got.dtype == np.float32 and rel_err(got, ref) <= 3e-6
 
 
+@pytest.mark.parametrize("S", [1, 31, 32, 33, 63, 64, 65, 129, 160, 289])
+def test_attention_fp32_rows_inside_a_matrix(S):
+    """Rows of Q, K and V as column blocks of one matrix, whole and cut-off blocks of keys, lengths that leave key waves without a
+    block (0 included): bit for bit what contiguous heads give, whose answers are checked above"""
+    say("attention fp32 packed S=%d" % S)
+    B, h = 3, 2
+    rng = np.random.default_rng(S)
+    qkv = dev(rng.standard_normal((B * S, 3 * h * 64)).astype(np.float32))
+    q, k, v = (t.contiguous() for t in qkv.view(B, S, 3, h, 64).permute(2, 0, 3, 1, 4))
+    for lens in (None, [S, 0, 1], [min(S, 32), min(S, 33), max(S - 1, 0)]):
+        kv = None if lens is None else dev(np.array(lens, np.int32))
+        want = ops().attention(q, k, v, 0.125, kv_len=kv).permute(0, 2, 1, 3).reshape(B * S, h * 64)
+        assert torch.equal(ops().attention_packed(qkv, B, S, h, 0.125, kv_len=kv), want)
+
+
 def _attention_layers(q, k, v, scale, mask):
     """the decomposed layers in float64, scores and probabilities as they are: infinities and NaN take their course"""
     q, k, v = (t.astype(np.float64) for t in (q, k, v))

@@ -19,9 +19,13 @@
 // with the fp32 matrix instruction, operands straight from memory (`exact` below): the answer is then that of the layers in
 // fp32 arithmetic.  The check is 33 instructions a wave.
 //
-// What bounds it: the vector ALU (conversion of K, V and P: 36 instructions per operand and 16-wide step, and the
-// exponentials) and the matrix pipe, about equal.  us, the decomposed launches -> this kernel, 12 heads:
-//   1 x 128 tokens 45 -> 7.6, 4 x 384 136 -> 29 (K and V read once per block of 32 queries: 113 MB from L2), 8 x 128 11, 1 x 512 16
+// What bounds it: the vector ALU (4.5 instructions for each of the 80 values of K, P and V that a lane converts for a block, 7 for
+// each of its 17 exponentials; 57 % of all clocks at 16 x 384 tokens, the matrix pipe 25 %) once a SIMD has three waves, and the
+// latency of a block's chain below that.  So: three waves a SIMD (the planes of Q are made once per workgroup and lie in LDS, a
+// block's rows are requested when the registers of the rows before are free), no work for the mask in blocks that are whole, and
+// requests that every path to their waits makes alike, or the compiler waits for V where K is meant.
+// us, 12 heads, in a row: the decomposed launches -> Q's planes in registers, two waves a SIMD -> this form
+//   1 x 128 tokens 45 -> 6.9 -> 6.4, 4 x 384 136 -> 29.1 -> 26.2 (with an additive mask 38 -> 28), 16 x 384 79 -> 73, 1 x 16 6.1 -> 5.8
 #include "common.h"
 #include "split_f32.h"
 
@@ -56,8 +60,25 @@ __device__ __forceinline__ float other_half(float v) {
     return (threadIdx.x & 32) ? __uint_as_float(r[0]) : __uint_as_float(r[1]);
 }
 
-template <int NW> __global__ void __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) attention_f32_kernel(AttnF32Params p) {
-    __shared__ __attribute__((aligned(16))) float stage[NW][kBlockQ * kStageRow];
+// exp(x) for x <= 0 (a NaN stays one): the product with log2 e in two parts, the first to the exponential instruction (1 ulp), the
+// second as a factor 1 + d.  Seven instructions where expf takes fourteen; results below the smallest normal value are zero, next
+// to a sum that holds a 1.
+__device__ __forceinline__ float exp_not_positive(float x) {
+    const float y  = __fmul_rn(x, 1.44269502f);
+    const float lo = fmaf(x, 1.92596299e-8f, fmaf(x, 1.44269502f, -y));
+    const float e  = __builtin_amdgcn_exp2f(y);
+    // where x or y is infinite the second part is no number, and the first is zero
+    return fmaf(e, __fmul_rn(__builtin_amdgcn_fmed3f(lo, -1.f, 1.f), 0.693147182f), e);
+}
+
+// At least three waves a SIMD (168 registers): 4 x 384 tokens are 576 workgroups, two and a quarter for each CU, and with two a CU
+// the last 64 were a round of their own.  Four (128 registers) spill.
+template <int NW> __global__ void __launch_bounds__(NW * 64, NW == 4 ? 3 : 1) attention_f32_kernel(AttnF32Params p) {
+    // the planes of Q (a step's three, a lane's 16 bytes each), then every wave's sums
+    constexpr int kQBytes = 4 * 3 * 64 * 16, kStageBytes = NW * kBlockQ * kStageRow * 4;
+    __shared__ __attribute__((aligned(16))) unsigned char shared[kQBytes > kStageBytes ? kQBytes : kStageBytes];
+    uint4 *const q_planes = reinterpret_cast<uint4 *>(shared);
+    float(*const stage)[kBlockQ * kStageRow] = reinterpret_cast<float(*)[kBlockQ * kStageRow]>(shared);
     __shared__ float stat_m[NW][kBlockQ], stat_l[NW][kBlockQ];
     __shared__ int again[NW];
 
@@ -106,13 +127,10 @@ template <int NW> __global__ void __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) at
             raw[2 * kk + 1] = *reinterpret_cast<const f32x4 *>(src + kk * 16 + 4);
         }
     };
-    auto load_q = [&](f32x4 (&raw)[8]) __attribute__((always_inline)) {
-        const int row = q0 + lq < S ? q0 + lq : S - 1;
-        load_row(qb + (size_t)row * p.q_ss + 8 * g, raw);
-    };
+    // blocks inside the sequence have a uniform base and one offset per lane; the last one clamps its rows
     auto load_k = [&](int t, f32x4 (&raw)[8]) __attribute__((always_inline)) {
-        const int row = t * kBlockK + lq < S ? t * kBlockK + lq : S - 1;
-        load_row(kb + ((uint32_t)row * ss + 8u * g), raw);
+        const int row = t * kBlockK + lq < S ? lq : S - 1 - t * kBlockK;
+        load_row(kb + (size_t)(uint32_t)(t * kBlockK) * ss + ((uint32_t)row * ss + 8u * g), raw);
     };
     auto begin = [&]() __attribute__((always_inline)) {
 #pragma unroll
@@ -124,40 +142,64 @@ template <int NW> __global__ void __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) at
     };
     // V of block t: slot e of step st and lane half g is key 16*st + 4*g + e (e < 4), 16*st + 8 + 4*g + e-4
     auto load_v = [&](int t, f32x2 (&vraw)[16]) __attribute__((always_inline)) {
+        const float *const block = vb + (size_t)(uint32_t)(t * kBlockK) * ss;
+        uint32_t mine            = (uint32_t)(4 * g) * ss + 2u * lq;
+        asm volatile("" : "+v"(mine));  // or every row's address is kept from block to block, in 32 registers
+        if (t * kBlockK + kBlockK <= S) {
+            typedef const __attribute__((address_space(1))) f32x2 *GlobalPair;
+            uint64_t row = reinterpret_cast<uint64_t>(block + mine);
 #pragma unroll
-        for (int st = 0; st < 2; ++st)
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                int row = t * kBlockK + 16 * st + 4 * g + (e & 3) + (e & 4) * 2;
-                row     = row < S ? row : S - 1;
-                vraw[st * 8 + e] = *reinterpret_cast<const f32x2 *>(vb + ((uint32_t)row * ss + 2u * lq));
+            for (int i = 0; i < 16; ++i) {
+                asm("" : "+v"(row));  // one addition a row, not a product and a sum in scalar registers
+                vraw[i] = *reinterpret_cast<GlobalPair>(row);
+                row += 4 * ((i & 3) == 3 ? 5 * (uint64_t)ss : ss);
             }
+        } else {
+            const uint32_t last_row = (uint32_t)(S - 1 - t * kBlockK);
+#pragma unroll
+            for (int i = 0; i < 16; ++i)
+                vraw[i] = *reinterpret_cast<const f32x2 *>(block + (min(16u * (i >> 3) + (i & 3) + (i & 4) * 2 + 4u * g, last_row) * ss + 2u * lq));
+        }
     };
     // softmax over block t's keys: scores * scale + mask, as the decomposed layers form them
-    auto softmax = [&](int t, float scale, f32x16 &s) __attribute__((always_inline)) {
+    auto softmax = [&](int t, float scale, auto exp_of, f32x16 &s) __attribute__((always_inline)) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            low  = fminf(low, s[r]);
+            s[r] = __fmul_rn(s[r], scale);
+        }
+        if (mb) {
+            int first_key = t * kBlockK + 4 * g;
+            asm volatile("" : "+v"(first_key));  // or the keys are counted outside, for every block
+            float m[16];
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int key = first_key + (r >> 2) * 8 + (r & 3);
+                m[r]          = mb[key < S ? key : S - 1];
+            }
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+                s[r] = __fadd_rn(s[r], m[r]);
+        }
+        if (t * kBlockK + kBlockK > kv_end) {
+            int left = kv_end - t * kBlockK - 4 * g;
+            asm volatile("" : "+v"(left));
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+                s[r] = (r >> 2) * 8 + (r & 3) < left ? s[r] : -INFINITY;
+        }
         float mx = -INFINITY;
 #pragma unroll
-        for (int r4 = 0; r4 < 4; ++r4) {
-            const int key0 = t * kBlockK + 8 * r4 + 4 * g;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                low     = fminf(low, s[r4 * 4 + e]);
-                float v = __fmul_rn(s[r4 * 4 + e], scale);
-                if (mb)
-                    v = __fadd_rn(v, mb[key0 + e < S ? key0 + e : S - 1]);
-                v             = key0 + e < kv_end ? v : -INFINITY;
-                s[r4 * 4 + e] = v;
-                mx            = fmaxf(mx, v);
-            }
-        }
+        for (int r = 0; r < 16; ++r)
+            mx = fmaxf(mx, s[r]);
         mx                = fmaxf(mx, other_half(mx));
         const float m_new = fmaxf(m_i, mx);
         const float m_use = m_new == -INFINITY ? 0.f : m_new;
-        const float alpha = expf(m_i - m_use);
+        const float alpha = exp_of(m_i - m_use);
         float sum         = 0.f;
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-            s[r] = expf(s[r] - m_use);
+            s[r] = exp_of(s[r] - m_use);
             sum += s[r];
         }
         l_i = fmaf(l_i, alpha, sum + other_half(sum));
@@ -187,59 +229,97 @@ template <int NW> __global__ void __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) at
 
     {
         const SplitConst sc;
-        Split3 qf[4];
         f32x4 kraw[8];
-        load_q(kraw);
-#pragma unroll
-        for (int kk = 0; kk < 4; ++kk) {
-            const f32x4 lo = kraw[2 * kk], hi = kraw[2 * kk + 1];
-            const float x[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-            qf[kk]           = split3(x, sc);
-        }
+        f32x2 vraw[16];
         begin();
-        if (wave < n_tiles)
-            load_k(wave, kraw);
-        for (int t = wave; t < n_tiles; t += NW) {
-            f32x2 vraw[16];
-            load_v(t, vraw);
-            // ---- S^T = K Q^T
-            f32x16 s;
+        // the waves share the queries: each makes its share of the steps' planes for all
+        const float *const q_row = qb + (size_t)(q0 + lq < S ? q0 + lq : S - 1) * p.q_ss + 8 * g;
+        f32x4 qraw[8 / NW];
+        Split3 own[4 / NW];  // read with one wave only: nothing to share
+#pragma unroll
+        for (int i = 0; i < 4 / NW; ++i) {
+            qraw[2 * i]     = *reinterpret_cast<const f32x4 *>(q_row + (wave + i * NW) * 16);
+            qraw[2 * i + 1] = *reinterpret_cast<const f32x4 *>(q_row + (wave + i * NW) * 16 + 4);
+        }
+        const int first = wave < n_tiles ? wave : 0;  // a wave without a block requests the first one all the same
+        load_k(first, kraw);
+        if (NW == 1)
+            load_v(0, vraw);
+#pragma unroll
+        for (int i = 0; i < 4 / NW; ++i) {
+            const f32x4 lo = qraw[2 * i], hi = qraw[2 * i + 1];
+            const float x[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+            const Split3 qf  = split3(x, sc);
+            if (NW == 1) {
+                own[i] = qf;
+                continue;
+            }
+#pragma unroll
+            for (int w = 0; w < 3; ++w)
+                q_planes[((wave + i * NW) * 3 + w) * 64 + lane] = make_uint4(qf.p[w][0], qf.p[w][1], qf.p[w][2], qf.p[w][3]);
+        }
+        if (NW > 1)
+            __syncthreads();
+        // scores of block t, from the rows in kraw
+        auto scores = [&](f32x16 &s) __attribute__((always_inline)) {
 #pragma unroll
             for (int r = 0; r < 16; ++r)
                 s[r] = 0.f;
+            int mine = lane;
+            asm volatile("" : "+v"(mine));  // or the compiler reads Q's planes once, into 48 registers
 #pragma unroll
             for (int kk = 0; kk < 4; ++kk) {
                 const f32x4 lo = kraw[2 * kk], hi = kraw[2 * kk + 1];
                 const float x[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-                const Split3 kf  = split3(x, sc);
+                Split3 qf = own[kk % (4 / NW)];
+#pragma unroll
+                for (int w = 0; NW > 1 && w < 3; ++w)
+                    *reinterpret_cast<uint4 *>(qf.p[w]) = q_planes[(kk * 3 + w) * 64 + mine];
+                const Split3 kf = split3(x, sc);
 #pragma unroll
                 for (int pr = 0; pr < kSplitProducts; ++pr)
-                    split_mma(kf, qf[kk], pr, s);
+                    split_mma(kf, qf, pr, s);
             }
+        };
+        // O^T += V^T P^T over half st of the block
+        auto weigh = [&](int st, const f32x16 &s, const f32x2 (&vraw)[16]) __attribute__((always_inline)) {
+            const float x[8] = {s[8 * st + 0], s[8 * st + 1], s[8 * st + 2], s[8 * st + 3],
+                                s[8 * st + 4], s[8 * st + 5], s[8 * st + 6], s[8 * st + 7]};
+            const Split3 pf  = split3(x, sc);
+#pragma unroll
+            for (int dt = 0; dt < 2; ++dt) {
+                const f32x2 *vr  = vraw + st * 8;
+                const float y[8] = {vr[0][dt], vr[1][dt], vr[2][dt], vr[3][dt], vr[4][dt], vr[5][dt], vr[6][dt], vr[7][dt]};
+                const Split3 vf  = split3(y, sc);
+#pragma unroll
+                for (int pr = 0; pr < kSplitProducts; ++pr)
+                    split_mma(vf, pf, pr, oacc[dt]);
+            }
+        };
+        // V is requested with the block's begin, the next block's K when half of V is done with
+        for (int t = wave; t < n_tiles; t += NW) {
+            f32x16 s;
+            if (NW > 1)
+                load_v(t, vraw);
+            asm volatile("" ::: "memory");
+            scores(s);
+            softmax(t, p.split_scale, [](float x) __attribute__((always_inline)) { return exp_not_positive(x); }, s);
+            weigh(0, s, vraw);
+#pragma unroll
+            for (int i = 8; i < 16; ++i)
+                asm volatile("" : "+v"(vraw[i]));  // all of V is here: weigh(1) does not wait for K
+            asm volatile("" ::: "memory");
             if (t + NW < n_tiles)
                 load_k(t + NW, kraw);
-            softmax(t, p.split_scale, s);
-            // ---- O^T += V^T P^T
+            else
 #pragma unroll
-            for (int st = 0; st < 2; ++st) {
-                const float x[8] = {s[8 * st + 0], s[8 * st + 1], s[8 * st + 2], s[8 * st + 3],
-                                    s[8 * st + 4], s[8 * st + 5], s[8 * st + 6], s[8 * st + 7]};
-                const Split3 pf  = split3(x, sc);
-                Split3 vf[2];
-#pragma unroll
-                for (int dt = 0; dt < 2; ++dt) {
-                    const f32x2 *vr  = vraw + st * 8;
-                    const float y[8] = {vr[0][dt], vr[1][dt], vr[2][dt], vr[3][dt], vr[4][dt], vr[5][dt], vr[6][dt], vr[7][dt]};
-                    vf[dt]           = split3(y, sc);
-                }
-#pragma unroll
-                for (int pr = 0; pr < kSplitProducts; ++pr)
-#pragma unroll
-                    for (int dt = 0; dt < 2; ++dt)
-                        split_mma(vf[dt], pf, pr, oacc[dt]);
-            }
+                for (int i = 0; i < 8; ++i)
+                    asm volatile("" : "=v"(kraw[i]));  // no registers for the values of before
+            asm volatile("" ::: "memory");
+            weigh(1, s, vraw);
         }
     }
+    __syncthreads();  // every wave is done with Q's planes
     leave();
     {
         // a score of -inf may be one that has no planes, or one that is; anything else that is not finite is in the sums
@@ -272,15 +352,20 @@ template <int NW> __global__ void __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) at
 #pragma unroll
             for (int r = 0; r < 16; ++r)
                 s[r] = 0.f;
-            f32x4 kraw[8], qraw[8];
-            load_k(t, kraw);
-            load_q(qraw);
+            const float *k_row = kb + (size_t)(uint32_t)(t * kBlockK) * ss +
+                                 ((uint32_t)(t * kBlockK + lq < S ? lq : S - 1 - t * kBlockK) * ss + 8u * g);
+            const float *q_row = qb + (size_t)(q0 + lq < S ? q0 + lq : S - 1) * p.q_ss + 8 * g;
+#pragma unroll 1
+            for (int kk = 0; kk < 4; ++kk)
 #pragma unroll
-            for (int kk = 0; kk < 8; ++kk)
+                for (int h = 0; h < 2; ++h) {
+                    const f32x4 kr = *reinterpret_cast<const f32x4 *>(k_row + kk * 16 + h * 4);
+                    const f32x4 qr = *reinterpret_cast<const f32x4 *>(q_row + kk * 16 + h * 4);
 #pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    s = __builtin_amdgcn_mfma_f32_32x32x2f32(kraw[kk][e], qraw[kk][e], s, 0, 0, 0);
-            softmax(t, p.scale, s);
+                    for (int e = 0; e < 4; ++e)
+                        s = __builtin_amdgcn_mfma_f32_32x32x2f32(kr[e], qr[e], s, 0, 0, 0);
+                }
+            softmax(t, p.scale, [](float x) __attribute__((always_inline)) { return expf(x); }, s);
             f32x2 vraw[16];
             load_v(t, vraw);
 #pragma unroll
