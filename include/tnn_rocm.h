@@ -282,6 +282,19 @@ TNN_ROCM_API int tnn_rocm_mask_prepare(void *stream, int dtype, const void *mask
  * whatever the source type; it is required unless the source is dense fp32. */
 TNN_ROCM_API int tnn_rocm_mask_prepare_strided(void *stream, int dtype, const void *mask, long mask_batch_stride,
                                                float *mask_f32, int32_t *kv_len, int B, int S, float threshold);
+/* The same for a mask [B,S] of integers (1 = token, 0 = padding, as a tokenizer hands it over) and the layers that make the
+ * additive mask of it: Cast to dtype (fp32, fp16 or bf16), then n_steps element-wise steps by one constant each (ops on the
+ * host, constants on the device, of type dtype), every result rounded to dtype as the layers' own tensors are
+ * (cpu_cast_layer_acc.cc:41-53, cpu_binary_op_layer_acc.cc).  mask [B,S] of dtype receives the last layer's result; mask_f32
+ * [B,S] is required unless dtype is fp32, whose mask is used where it lies. */
+#define TNN_ROCM_MAX_MASK_STEPS 4
+#define TNN_ROCM_MASK_ADD 0      /* x + c */
+#define TNN_ROCM_MASK_SUB 1      /* x - c */
+#define TNN_ROCM_MASK_SUB_FROM 2 /* c - x */
+#define TNN_ROCM_MASK_MUL 3      /* x * c */
+TNN_ROCM_API int tnn_rocm_mask_prepare_i32(void *stream, int dtype, const int32_t *ints, int n_steps, const int *ops,
+                                           const void *constants, void *mask, float *mask_f32, int32_t *kv_len, int B, int S,
+                                           float threshold);
 
 /* ---- row-wise ops ---------------------------------------------------------------------------
  * Softmax over `channel` of x viewed as [outer][channel][inner]

@@ -872,6 +872,44 @@ def test_encoder_int32_mask_input_builds_the_additive_mask_in_the_graph(precisio
     assert err <= (FP16_TOL if precision == "fp16" else FP32_ASSERT)
 
 
+@pytest.mark.parametrize("precision", ["fp32", "fp16", "bf16"])
+def test_mask_made_of_integers_in_one_launch(precision):
+    """The layers that make the additive mask out of integers run as one launch in a plain forward and one by one under
+    ForwardWithCallback, or where a blob between them is a model output: the answer and the mask are bit for bit the same, for
+    every mask that an instance is given in turn and after a reshape."""
+    host, tnnmodel, EncoderConfig, make_weights, make_inputs = _mods()
+    say("host: mask of integers as a group, " + precision)
+    cfg = EncoderConfig(2, 256, 4, 512)
+    w = make_weights(cfg, seed=53, bias_std=0.05)
+    B, S = 3, 40
+    graphs = [tnnmodel.encoder_graph(cfg, w, B, S, int_mask=True, dynamic=True, position_ids=True, extra_outputs=extra)
+              for extra in (("attention_bias",), ("attention_bias", "mask_pad"))]
+    group, single = (host.RocmInstance.from_graph(g, precision) for g in graphs)
+    rng = np.random.default_rng(54)
+    for b, n in ((B, S), (1, 56), (2, 33)):
+        ids, seg, lens, _ = make_inputs(cfg, b, n, 1, n, seed=b)
+        masks = [np.ones((b, n)), np.arange(n)[None, :] < lens[:, None], rng.integers(0, 2, (b, n)), np.zeros((b, n))]
+        shapes = {k: [b, n] for k in ("input_ids", "token_type_ids", "input_mask", "position_ids")}
+        for inst in (group, single):
+            inst.reshape(shapes)
+            for name, value in (("input_ids", ids), ("token_type_ids", seg), ("position_ids", np.tile(np.arange(n), (b, 1)))):
+                inst.set_input(name, value.astype(np.int32))
+        for m in masks:
+            got = []
+            for inst, run in ((group, "forward"), (group, "callback"), (single, "forward")):
+                inst.set_input("input_mask", m.astype(np.int32))
+                inst.forward() if run == "forward" else inst.forward_with_callback()
+                got.append((inst.output("last_hidden"), inst.output("attention_bias")))
+            assert np.isfinite(got[0][0]).all()
+            assert np.array_equal(got[0][1].reshape(b, n) == 0, m.astype(bool))
+            if precision != "fp32":  # with a callback an fp32 net runs the attention's layers one by one as well
+                assert np.array_equal(got[0][0], got[1][0])
+            assert np.array_equal(got[0][0], got[2][0])
+            assert np.array_equal(got[0][1], got[1][1]) and np.array_equal(got[0][1], got[2][1])
+    group.close()
+    single.close()
+
+
 @pytest.mark.parametrize("precision", ["fp32", "fp16"])
 def test_reading_comprehension_demo_shape(precision):
     """The shape the reference's BERT demo feeds (examples/linux/src/BertReadingComprehension/BertReadingComprehension.cc:

@@ -1325,6 +1325,35 @@ def test_mask_prepare_any_float_type():
         assert list(got & ~(1 << 30)) == [150, 31, 100, 120, 200, 199, 1, 200, 200]
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("S", [1, 63, 64, 65, 200])
+def test_mask_prepare_ints(S, dtype):
+    """Integers -> additive mask -> key counts in one launch: bit for bit the cast and element-wise launches and the launch that
+    takes the counts from their result, also for values and constants that the type rounds or cannot hold."""
+    say("mask_prepare_ints S=%d %s" % (S, dtype))
+    o = ops()
+    rng = np.random.default_rng(S)
+    B = 6
+    m = (np.arange(S)[None, :] < np.array([S, 1, max(1, S // 2), S, S, S])[:, None]).astype(np.int32)
+    m[3] = rng.integers(0, 2, S)
+    m[4] = rng.integers(-3000, 3000, S)      # half and bfloat16 round these
+    m[5, S // 2] = 2 ** 31 - 1               # infinite in half
+    ints = dev(m)
+    chains = [[], [(2, 1.0), (3, -10000.0)], [(1, 1.0), (3, 10000.0)], [(2, 1.0), (3, -1e9)], [(0, 0.3), (3, -7.7), (1, 2.1), (2, 3e38)]]
+    for steps in chains:
+        t = o.cast(ints, dtype)
+        for code, c in steps:
+            const = o.cast(dev(np.array([c], np.float32)), dtype)
+            t = {0: lambda: o.binary("add", t, const), 1: lambda: o.binary("sub", t, const), 2: lambda: o.binary("sub", const, t),
+                 3: lambda: o.binary("mul", t, const)}[code]()
+        want_kv, want_f32 = o.mask_prepare(t)
+        made, kv, f32 = o.mask_prepare_ints(ints, steps, dtype)
+        same = (made == t) | (torch.isnan(made) & torch.isnan(t))
+        assert bool(same.all()), (steps, dtype)
+        assert torch.equal(kv, want_kv), (steps, host(kv), host(want_kv))
+        assert torch.equal(torch.nan_to_num(f32), torch.nan_to_num(want_f32)) and torch.equal(torch.isnan(f32), torch.isnan(want_f32))
+
+
 def test_store_through_switch_waits_for_the_device():
     from tnn_amd import capi
     lib = capi.load()

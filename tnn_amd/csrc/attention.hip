@@ -1019,16 +1019,41 @@ __global__ void __launch_bounds__(NW * 64, (NW == 4 && DT == TNN_ROCM_F16) ? 3 :
 // large negative number) below the best key's contributes exp(threshold + score difference) = 0 in fp32, whatever
 // constant the whole row carries.  Row b is read at mask + b * src_stride (0: one row serves every sequence); with
 // mask_f32 given, the row is also written there in fp32, densely (what the attention kernels read).
-template <int DT>
-__global__ void mask_to_kv_len_kernel(const typename Elem<DT>::type *__restrict__ mask, long src_stride,
-                                      float *__restrict__ mask_f32, int32_t *__restrict__ kv_len, int S, float threshold,
-                                      int flag_zero_rows) {
+// SRC = int32_t: the values are integers, and the additive mask is what the layers cast -> steps (each by one constant)
+// make of them in type DT, rounded to it after every one as those layers' tensors are; it is written to `made`.
+struct MaskSteps {
+    int n = 0;
+    int op[TNN_ROCM_MAX_MASK_STEPS] = {};
+};
+template <int DT, typename SRC>
+__global__ void mask_to_kv_len_kernel(const SRC *__restrict__ mask, long src_stride, MaskSteps steps,
+                                      const typename Elem<DT>::type *__restrict__ constants,
+                                      typename Elem<DT>::type *__restrict__ made, float *__restrict__ mask_f32,
+                                      int32_t *__restrict__ kv_len, int S, float threshold, int flag_zero_rows) {
     const int b    = blockIdx.x;
     const int lane = threadIdx.x;
-    const typename Elem<DT>::type *row = mask + (size_t)b * src_stride;
+    const SRC *row = mask + (size_t)b * src_stride;
+    auto value     = [&](int j) -> float {
+        if constexpr (std::is_same<SRC, int32_t>::value) {
+            typename Elem<DT>::type t;
+            Elem<DT>::st(&t, (float)row[j]);
+            for (int i = 0; i < steps.n; ++i) {
+                const float x = Elem<DT>::ld(&t), c = Elem<DT>::ld(&constants[i]);
+                Elem<DT>::st(&t, steps.op[i] == TNN_ROCM_MASK_ADD        ? __fadd_rn(x, c)
+                                 : steps.op[i] == TNN_ROCM_MASK_SUB      ? __fsub_rn(x, c)
+                                 : steps.op[i] == TNN_ROCM_MASK_SUB_FROM ? __fsub_rn(c, x)
+                                                                         : __fmul_rn(x, c));
+            }
+            return Elem<DT>::ld(&t);
+        } else {
+            return Elem<DT>::ld(&row[j]);
+        }
+    };
     float top = -INFINITY;
     for (int j = lane; j < S; j += 64) {
-        const float v = Elem<DT>::ld(&row[j]);
+        const float v = value(j);
+        if (made)
+            Elem<DT>::st(&made[(size_t)b * S + j], v);
         if (mask_f32)
             mask_f32[(size_t)b * S + j] = v;
         top = v > top ? v : top;
@@ -1041,7 +1066,7 @@ __global__ void mask_to_kv_len_kernel(const typename Elem<DT>::type *__restrict_
     const float cut = top + threshold;
     int last = -1, first_nonzero = S;
     for (int j = lane; j < S; j += 64) {
-        const float v = Elem<DT>::ld(&row[j]);
+        const float v = value(j);
         if (v > cut)
             last = j;
         if (v != 0.0f && j < first_nonzero)
@@ -1507,8 +1532,8 @@ int tnn_rocm_mask_to_kv_len(void *stream, const float *mask, int32_t *kv_len, in
     if (B == 0)
         return 0;
     TR_REQUIRE(mask && kv_len, TNN_ROCM_EINVAL, "mask_to_kv_len: null pointer");
-    hipLaunchKernelGGL(mask_to_kv_len_kernel<TNN_ROCM_F32>, dim3(B), dim3(64), 0, (hipStream_t)stream, mask, (long)S, nullptr,
-                       kv_len, S, threshold, 0);
+    hipLaunchKernelGGL((mask_to_kv_len_kernel<TNN_ROCM_F32, float>), dim3(B), dim3(64), 0, (hipStream_t)stream, mask, (long)S,
+                       MaskSteps{}, (const float *)nullptr, (float *)nullptr, (float *)nullptr, kv_len, S, threshold, 0);
     TR_CHECK_LAUNCH();
     return 0;
 }
@@ -1530,20 +1555,50 @@ int tnn_rocm_mask_prepare_strided(void *stream, int dtype, const void *mask, lon
     hipStream_t s = (hipStream_t)stream;
     switch (dtype) {
         case TNN_ROCM_F32:
-            hipLaunchKernelGGL(mask_to_kv_len_kernel<TNN_ROCM_F32>, dim3(B), dim3(64), 0, s, (const float *)mask,
-                               mask_batch_stride, mask_f32, kv_len, S, threshold, 1);
+            hipLaunchKernelGGL((mask_to_kv_len_kernel<TNN_ROCM_F32, float>), dim3(B), dim3(64), 0, s, (const float *)mask,
+                               mask_batch_stride, MaskSteps{}, (const float *)nullptr, (float *)nullptr, mask_f32, kv_len, S, threshold, 1);
             break;
         case TNN_ROCM_F16:
-            hipLaunchKernelGGL(mask_to_kv_len_kernel<TNN_ROCM_F16>, dim3(B), dim3(64), 0, s, (const half_t *)mask,
-                               mask_batch_stride, mask_f32, kv_len, S, threshold, 1);
+            hipLaunchKernelGGL((mask_to_kv_len_kernel<TNN_ROCM_F16, half_t>), dim3(B), dim3(64), 0, s, (const half_t *)mask,
+                               mask_batch_stride, MaskSteps{}, (const half_t *)nullptr, (half_t *)nullptr, mask_f32, kv_len, S, threshold, 1);
             break;
         case TNN_ROCM_BF16:
-            hipLaunchKernelGGL(mask_to_kv_len_kernel<TNN_ROCM_BF16>, dim3(B), dim3(64), 0, s, (const bf16_bits *)mask,
-                               mask_batch_stride, mask_f32, kv_len, S, threshold, 1);
+            hipLaunchKernelGGL((mask_to_kv_len_kernel<TNN_ROCM_BF16, bf16_bits>), dim3(B), dim3(64), 0, s, (const bf16_bits *)mask,
+                               mask_batch_stride, MaskSteps{}, (const bf16_bits *)nullptr, (bf16_bits *)nullptr, mask_f32, kv_len, S, threshold, 1);
             break;
         default:
             TR_REQUIRE(false, TNN_ROCM_EDTYPE, "mask_prepare: dtype %d unsupported", dtype);
     }
+    TR_CHECK_LAUNCH();
+    return 0;
+}
+
+int tnn_rocm_mask_prepare_i32(void *stream, int dtype, const int32_t *ints, int n_steps, const int *ops, const void *constants,
+                              void *mask, float *mask_f32, int32_t *kv_len, int B, int S, float threshold) {
+    TR_REQUIRE(B >= 0 && S >= 0 && S < kKvLenMaskZero, TNN_ROCM_ESHAPE, "mask_prepare_i32: bad size");
+    TR_REQUIRE(n_steps >= 0 && n_steps <= TNN_ROCM_MAX_MASK_STEPS && (n_steps == 0 || (ops && constants)), TNN_ROCM_EINVAL,
+               "mask_prepare_i32: %d steps", n_steps);
+    MaskSteps steps;
+    steps.n = n_steps;
+    for (int i = 0; i < n_steps; ++i) {
+        TR_REQUIRE(ops[i] >= TNN_ROCM_MASK_ADD && ops[i] <= TNN_ROCM_MASK_MUL, TNN_ROCM_EINVAL, "mask_prepare_i32: unknown step %d",
+                   ops[i]);
+        steps.op[i] = ops[i];
+    }
+    if (B == 0)
+        return 0;
+    TR_REQUIRE(ints && mask && kv_len && (mask_f32 || dtype == TNN_ROCM_F32), TNN_ROCM_EINVAL, "mask_prepare_i32: null pointer");
+    hipStream_t s = (hipStream_t)stream;
+#define TR_MASK(DT)                                                                                                     \
+    hipLaunchKernelGGL((mask_to_kv_len_kernel<DT, int32_t>), dim3(B), dim3(64), 0, s, ints, (long)S, steps,             \
+                       (const Elem<DT>::type *)constants, (Elem<DT>::type *)mask, mask_f32, kv_len, S, threshold, 1)
+    switch (dtype) {
+        case TNN_ROCM_F32: TR_MASK(TNN_ROCM_F32); break;
+        case TNN_ROCM_F16: TR_MASK(TNN_ROCM_F16); break;
+        case TNN_ROCM_BF16: TR_MASK(TNN_ROCM_BF16); break;
+        default: TR_REQUIRE(false, TNN_ROCM_EDTYPE, "mask_prepare_i32: dtype %d unsupported", dtype);
+    }
+#undef TR_MASK
     TR_CHECK_LAUNCH();
     return 0;
 }

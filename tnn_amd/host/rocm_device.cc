@@ -78,8 +78,7 @@ Status RocmContext::OnInstanceForwardBegin() {
     return TNN_OK;
 }
 
-Status RocmContext::AttentionMask(const std::string &name, const void *mask_blob, int mask_dtype, int B, int S, bool one_row,
-                                  const float **mask_f32, const int32_t **kv_len) {
+Status RocmContext::MaskRoom(int B, int S, bool one_row) {
     auto &c = mask_cache_;
     if ((size_t)B * S > c.cap_mask || (size_t)B > c.cap_len || !c.kv_len) {
         ROCM_CALL(tnn_rocm_stream_sync(stream_));
@@ -95,6 +94,24 @@ Status RocmContext::AttentionMask(const std::string &name, const void *mask_blob
     }
     if (c.B != B || c.S != S || c.one_row != one_row)
         c.B = B, c.S = S, c.one_row = one_row, c.src = nullptr;
+    return TNN_OK;
+}
+
+Status RocmContext::MakeAttentionMask(const std::string &name, void *mask_blob, int mask_dtype, int B, int S, const int32_t *ints,
+                                      const std::vector<int> &ops, const void *constants) {
+    auto &c = mask_cache_;
+    RETURN_ON_NEQ(MaskRoom(B, S, false), TNN_OK);
+    ROCM_CALL(tnn_rocm_mask_prepare_i32(stream_, mask_dtype, ints, (int)ops.size(), ops.data(), constants, mask_blob,
+                                        mask_dtype == TNN_ROCM_F32 ? nullptr : (float *)c.mask_f32, (int32_t *)c.kv_len, B, S,
+                                        -1000.0f));
+    c.src = mask_blob, c.name = name, c.epoch = forward_epoch_;
+    return TNN_OK;
+}
+
+Status RocmContext::AttentionMask(const std::string &name, const void *mask_blob, int mask_dtype, int B, int S, bool one_row,
+                                  const float **mask_f32, const int32_t **kv_len) {
+    auto &c = mask_cache_;
+    RETURN_ON_NEQ(MaskRoom(B, S, one_row), TNN_OK);
     // a dense fp32 mask is read where it lies; any other (half precision, or one row for all sequences) from the copy
     const bool in_place = mask_dtype == TNN_ROCM_F32 && !one_row;
     const float *m      = in_place ? (const float *)mask_blob : (const float *)c.mask_f32;

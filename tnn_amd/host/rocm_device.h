@@ -80,8 +80,14 @@ public:
     // (an additive mask [1,1,1,S])
     Status AttentionMask(const std::string &name, const void *mask_blob, int mask_dtype, int B, int S, bool one_row,
                          const float **mask_f32, const int32_t **kv_len);
+    // The blob mask_blob [B,S] itself is made out of integers (ops on the host, constants on the device, see
+    // tnn_rocm_mask_prepare_i32), and what AttentionMask would derive from it in the same launch.
+    Status MakeAttentionMask(const std::string &name, void *mask_blob, int mask_dtype, int B, int S, const int32_t *ints,
+                             const std::vector<int> &ops, const void *constants);
 
 private:
+    // room for B masks of S values and their key counts; a mask held for another shape is forgotten
+    Status MaskRoom(int B, int S, bool one_row);
     int device_id_       = 0;
     void *stream_        = nullptr;
     bool own_stream_     = true;

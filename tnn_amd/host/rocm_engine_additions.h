@@ -27,6 +27,8 @@ constexpr LayerType LAYER_ROCM_FUSED_EMBEDDING   = static_cast<LayerType>(905);
 constexpr LayerType LAYER_ROCM_QUANT_LINEAR_GELU = static_cast<LayerType>(906);
 // LayerNorm (LayerNormLayerParam, inputs x, scale, bias) with a second, int8 output: the quantised copy of the first
 constexpr LayerType LAYER_ROCM_LAYER_NORM_QUANT  = static_cast<LayerType>(907);
+// names the acc of a group of layers only (RocmFindMaskGroups): no layer of a graph has this type
+constexpr LayerType LAYER_ROCM_MASK_FROM_INT     = static_cast<LayerType>(908);
 
 struct RocmFusedLinearResource : public LayerResource {
     RawBuffer weight_nk;  // [N, K] fp32
@@ -81,6 +83,11 @@ struct RocmFusedAttentionParam : public LayerParam {
     std::string ln_stats_key, ln_sums_key;
     // the last output blob is int8: the context quantised as the Reformat layer that followed would (ROCm int8 pass)
     int out_quant = 0;
+};
+// Cast of an int32 mask to the network's float type, then element-wise steps (TNN_ROCM_MASK_*) by one constant each
+struct RocmMaskFromIntParam : public LayerParam {
+    std::vector<int> ops;
+    std::vector<float> constants;
 };
 // Gather(word ids) + Add(position constant) + Gather(type ids) + Add + LayerNorm of a BERT-style front end.
 // Inputs: word ids, type ids (int32), gamma, beta (constant blobs); resource: RocmFusedEmbeddingResource.

@@ -1511,6 +1511,77 @@ std::vector<RocmLayerGroup> RocmFindAttentionGroups(NetStructure *structure, Net
     return RocmFusionPass().FindAttention(structure, resource);
 }
 
+// An attention core's additive mask that is made out of integers,
+//   int32 blob -> Cast(float) -> [Unsqueeze] [Add / Sub / Mul by one constant] ... -> mask of a fused attention,
+// by layers that follow each other and whose blobs on the way have no other reader and are no model outputs: one launch instead
+// of three or four, and it derives the key counts as well.
+std::vector<RocmLayerGroup> RocmFindMaskGroups(NetStructure *s, NetResource *r, const std::vector<RocmLayerGroup> &attention) {
+    auto &L = s->layers;
+    std::set<std::string> masks;
+    auto take = [&](const std::shared_ptr<LayerInfo> &l) {
+        auto p = l ? dynamic_cast<RocmFusedAttentionParam *>(l->param.get()) : nullptr;
+        if (p && p->has_mask && l->inputs.size() > 1)
+            masks.insert(l->inputs[1]);
+    };
+    for (auto &l : L)
+        take(l);
+    for (auto &g : attention)
+        take(g.layer);
+    std::vector<RocmLayerGroup> found;
+    GraphIndex g(L);
+    for (auto &mask : masks) {
+        auto param      = std::make_shared<RocmMaskFromIntParam>();
+        auto &ops       = param->ops;
+        auto &constants = param->constants;
+        std::set<int> chain;
+        std::string cur = mask;
+        bool plain = true, whole = false;
+        while (plain && !whole) {
+            const int p = g.producer_of(cur);
+            if (p < 0 || !L[p] || L[p]->inputs.size() != 1 || L[p]->outputs.size() != 1 || L[p]->param->quantized ||
+                (cur != mask && (g.sole_consumer(cur) < 0 || s->outputs.count(cur))))
+                break;
+            auto l = L[p];
+            chain.insert(p);
+            cur = l->inputs[0];
+            if (l->type == LAYER_CAST) {
+                auto cp = dynamic_cast<CastLayerParam *>(l->param.get());
+                whole = plain = cp && cp->to == DATA_TYPE_FLOAT && r->constant_map.count(cur) == 0;
+            } else if (l->type == LAYER_ADD || l->type == LAYER_SUB || l->type == LAYER_MUL) {
+                auto it = r->resource_map.find(l->name);
+                auto er = it == r->resource_map.end() ? nullptr : dynamic_cast<EltwiseLayerResource *>(it->second.get());
+                auto bp = dynamic_cast<MultidirBroadcastLayerParam *>(l->param.get());
+                plain   = er && bp && er->element_handle.GetDataCount() == 1 &&
+                        er->element_handle.GetDataType() == DATA_TYPE_FLOAT && (int)ops.size() < TNN_ROCM_MAX_MASK_STEPS;
+                if (!plain)
+                    break;
+                ops.insert(ops.begin(), l->type == LAYER_ADD          ? TNN_ROCM_MASK_ADD
+                                        : l->type == LAYER_MUL        ? TNN_ROCM_MASK_MUL
+                                        : bp->weight_input_index == 0 ? TNN_ROCM_MASK_SUB_FROM
+                                                                      : TNN_ROCM_MASK_SUB);
+                constants.insert(constants.begin(), er->element_handle.force_to<float *>()[0]);
+            } else {
+                plain = l->type == LAYER_UNSQUEEZE;
+            }
+        }
+        if (!whole || *chain.rbegin() - *chain.begin() + 1 != (int)chain.size())
+            continue;
+        RocmLayerGroup group;
+        group.first = *chain.begin(), group.last = *chain.rbegin();
+        group.layer           = std::make_shared<LayerInfo>();
+        group.layer->type     = LAYER_ROCM_MASK_FROM_INT;
+        group.layer->type_str = "RocmMaskFromInt";
+        group.layer->name     = L[group.last]->name + "_from_int";
+        group.layer->inputs   = {cur};
+        group.layer->outputs  = {mask};
+        param->type           = group.layer->type_str;
+        param->name           = group.layer->name;
+        group.layer->param    = param;
+        found.push_back(group);
+    }
+    return found;
+}
+
 // ---- LayerNorm folded into a projection: weight preparation ---------------------------------------------------
 // value of f after rounding to the activation type (round to nearest even, as the device conversion does)
 static float RoundToActivationType(float f, DataType dt) {
@@ -1899,6 +1970,39 @@ Status RocmShareProjections(AbstractLayerAcc *attention, AbstractLayerAcc *const
     }
     return att->TakeProjections(from);
 }
+
+// ---- RocmMaskFromInt ----------------------------------------------------------------------------------------------
+// Stands for the layers of a mask group, see RocmFindMaskGroups.
+class RocmMaskFromIntLayerAcc : public RocmLayerAcc {
+public:
+    Status Reshape(const std::vector<Blob *> &inputs, const std::vector<Blob *> &outputs) override {
+        auto p = dynamic_cast<RocmMaskFromIntParam *>(param_);
+        CHECK_PARAM_NULL(p);
+        auto &in = inputs[0]->GetBlobDesc(), &out = outputs[0]->GetBlobDesc();
+        const DataType dt = out.data_type;
+        if (in.data_type != DATA_TYPE_INT32 || (dt != DATA_TYPE_FLOAT && dt != DATA_TYPE_HALF && dt != DATA_TYPE_BFP16) || out.dims.empty() ||
+            DimsVectorUtils::Count(in.dims) != DimsVectorUtils::Count(out.dims))
+            return Status(TNNERR_PARAM_ERR, "mask from integers: an int32 and a float blob of one size are required");
+        S_ = out.dims.back();
+        B_ = S_ > 0 ? DimsVectorUtils::Count(out.dims) / S_ : 0;
+        if (B_ <= 0)
+            return Status(TNNERR_PARAM_ERR, "mask from integers: no elements");
+        if (!constants_)
+            return UploadConverted(p->constants.data(), p->constants.size(), DATA_TYPE_FLOAT, dt, &constants_);
+        return TNN_OK;
+    }
+    Status Forward(const std::vector<Blob *> &inputs, const std::vector<Blob *> &outputs) override {
+        auto p    = dynamic_cast<RocmMaskFromIntParam *>(param_);
+        auto &out = outputs[0]->GetBlobDesc();
+        return context_->MakeAttentionMask(out.name, Ptr(outputs[0]), (int)out.data_type, B_, S_, (const int32_t *)Ptr(inputs[0]),
+                                           p->ops, constants_);
+    }
+
+private:
+    void *constants_ = nullptr;
+    int B_ = 0, S_ = 0;
+};
+REGISTER_ROCM_ACC(RocmMaskFromIntLayerAcc, LAYER_ROCM_MASK_FROM_INT);
 
 // ---- RocmFusedEmbedding ----------------------------------------------------------------------------------------
 class RocmFusedEmbeddingLayerAcc : public RocmLayerAcc {

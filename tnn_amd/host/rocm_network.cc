@@ -1,5 +1,6 @@
 #include "rocm_network.h"
 
+#include <algorithm>
 #include <cstdio>
 #include <cstdlib>
 
@@ -63,9 +64,14 @@ void RocmNetwork::Signature(std::vector<uint64_t> *sig) {
 #ifndef TNN_ROCM_ENGINE_TREE
 Status RocmNetwork::Init(NetworkConfig &net_config, ModelInterpreter *interpreter, const InputShapesMap &max_inputs_shape) {
     RETURN_ON_NEQ(DefaultNetwork::Init(net_config, interpreter, max_inputs_shape), TNN_OK);
-    if (config_.precision != PRECISION_HIGH)
-        return TNN_OK;
-    for (auto &found : RocmFindAttentionGroups(&structure_, &resource_)) {
+    std::vector<RocmLayerGroup> all;
+    if (config_.precision == PRECISION_HIGH)
+        all = RocmFindAttentionGroups(&structure_, &resource_);
+    for (auto &mask : RocmFindMaskGroups(&structure_, &resource_, all))
+        all.push_back(mask);
+    std::sort(all.begin(), all.end(), [](const RocmLayerGroup &a, const RocmLayerGroup &b) { return a.first < b.first; });
+    for (auto &found : all) {
+        const bool attention = found.layer->type == LAYER_ROCM_FUSED_ATTENTION;
         Group g;
         g.first = found.first, g.last = found.last;
         g.layer = found.layer, g.resource = found.resource;
@@ -76,7 +82,8 @@ Status RocmNetwork::Init(NetworkConfig &net_config, ModelInterpreter *interprete
         bool known = true;
         for (auto blobs : {&g.inputs, &g.outputs})
             for (Blob *b : *blobs)
-                known &= b != nullptr && b->GetBlobDesc().data_type == DATA_TYPE_FLOAT;
+                known &= b != nullptr && (!attention || b->GetBlobDesc().data_type == DATA_TYPE_FLOAT);
+        known = known && (attention || g.inputs[0]->GetBlobDesc().data_type == DATA_TYPE_INT32);
         if (!known)
             continue;
         g.acc.reset(device_->CreateLayerAcc(g.layer->type));
@@ -84,10 +91,12 @@ Status RocmNetwork::Init(NetworkConfig &net_config, ModelInterpreter *interprete
             continue;
         g.acc->SetConstantResource(&resource_.constant_map);
         RETURN_ON_NEQ(g.acc->Init(context_, g.layer->param.get(), g.resource.get(), g.inputs, g.outputs), TNN_OK);
-        AbstractLayerAcc *projections[3];
-        for (int t = 0; t < 3; ++t)
-            projections[t] = layers_[found.projections[t]]->layer_acc_;
-        RETURN_ON_NEQ(RocmShareProjections(g.acc.get(), projections), TNN_OK);
+        if (attention) {
+            AbstractLayerAcc *projections[3];
+            for (int t = 0; t < 3; ++t)
+                projections[t] = layers_[found.projections[t]]->layer_acc_;
+            RETURN_ON_NEQ(RocmShareProjections(g.acc.get(), projections), TNN_OK);
+        }
         groups_.push_back(std::move(g));
     }
     return ReshapeGroups();
@@ -101,13 +110,14 @@ Status RocmNetwork::Reshape(const InputShapesMap &inputs) {
 Status RocmNetwork::ReshapeGroups() {
     auto range = [](Blob *b) {
         const char *at = (const char *)b->GetHandle().base + b->GetHandle().bytes_offset;
-        return std::make_pair(at, at + (size_t)DimsVectorUtils::Count(b->GetBlobDesc().dims) * sizeof(float));
+        return std::make_pair(at, at + (size_t)DimsVectorUtils::Count(b->GetBlobDesc().dims) * sizeof(float));  // half: more than it is
     };
     for (auto &g : groups_) {
-        // the projections read all of the input before the attention kernel writes, but the mask is read while it does
+        // the projections read all of the input before the attention kernel writes, but the mask is read while it does; the
+        // integers of a mask are read twice
         g.active       = true;
         const auto out = range(g.outputs[0]);
-        for (size_t i = 1; i < g.inputs.size(); ++i) {
+        for (size_t i = g.layer->type == LAYER_ROCM_FUSED_ATTENTION ? 1 : 0; i < g.inputs.size(); ++i) {
             const auto in = range(g.inputs[i]);
             g.active &= g.inputs[i]->IsConstant() || in.second <= out.first || out.second <= in.first;
         }

@@ -23,12 +23,15 @@ namespace TNN_NS {
 // the single layers; what lies between the group's inputs and its output is simply not written.
 struct RocmLayerGroup {
     int first = 0, last = 0;
-    int projections[3] = {0, 0, 0};    // the layers that make Q, K and V
+    int projections[3] = {0, 0, 0};    // the layers that make Q, K and V (of an attention core)
     std::shared_ptr<LayerInfo> layer;  // type, inputs, output and parameters of the acc that stands for the group
     std::shared_ptr<LayerResource> resource;
 };
 // the attention cores (projections included) that an fp32 net keeps as layers
 std::vector<RocmLayerGroup> RocmFindAttentionGroups(NetStructure *structure, NetResource *resource);
+// the layers that make the masks of a net's attention cores out of integers
+std::vector<RocmLayerGroup> RocmFindMaskGroups(NetStructure *structure, NetResource *resource,
+                                               const std::vector<RocmLayerGroup> &attention);
 // One set of weights for a group and its layers: the attention acc packs the device weights of the three projections, and
 // the projections' accs go on with the packed ones.  The attention acc must outlive any Forward of theirs.
 Status RocmShareProjections(AbstractLayerAcc *attention, AbstractLayerAcc *const projections[3]);
@@ -48,7 +51,9 @@ protected:
     // The layer loop of a plain forward.  An fp32 net keeps its attention as layers (every intermediate blob is there for
     // ForwardWithCallback, profiling and whoever names one as a model output), and those ways of running it take them one
     // by one; a plain forward runs each core as a group: one projection for Q, K and V and one attention kernel instead of
-    // sixteen launches that pass the [B*h, S, S] scores through memory six times.
+    // sixteen launches that pass the [B*h, S, S] scores through memory six times.  In a net of any precision the layers that make
+    // the additive mask out of integers are such a group: one launch instead of four (three layers', and the one that takes the
+    // key counts from the mask), 12 layers fp16 of 1 x 32 tokens 367 -> 356 us, 1 x 256 481 -> 467, fp32 of 1 x 128 771 -> 753.
     Status RunLayers(void *prof_stream) override;
 #endif
 #ifdef TNN_ROCM_ENGINE_TREE

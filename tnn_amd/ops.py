@@ -3,6 +3,8 @@
 torch is used only as plumbing: it owns device memory and the stream.  Every function passes raw
 device pointers into libtnn_rocm.so; there is no torch implementation behind any of them.
 """
+import ctypes
+
 import torch
 
 from . import capi
@@ -234,6 +236,20 @@ def mask_prepare(mask, threshold=-1000.0):
     capi.call("tnn_rocm_mask_prepare", _stream(), dt(mask), _p(mask), None if mask.dtype == torch.float32 else _p(f32), _p(out),
               B, S, float(threshold))
     return out, f32
+
+
+def mask_prepare_ints(mask, steps, dtype, threshold=-1000.0):
+    """int32 mask [B,S] -> cast to dtype -> steps ((code, constant), ...): (mask of dtype [B,S], flagged kv_len [B], fp32 mask)"""
+    _chk(mask)
+    B, S = mask.shape
+    out = torch.empty(B, dtype=torch.int32, device=mask.device)
+    made = torch.empty(B, S, dtype=dtype, device=mask.device)
+    f32 = made if dtype == torch.float32 else torch.empty(B, S, dtype=torch.float32, device=mask.device)
+    codes = (ctypes.c_int * max(1, len(steps)))(*[s[0] for s in steps])
+    const = torch.tensor([s[1] for s in steps] or [0.0], dtype=torch.float32, device=mask.device).to(dtype)
+    capi.call("tnn_rocm_mask_prepare_i32", _stream(), dt(const), _p(mask), len(steps), ctypes.cast(codes, ctypes.c_void_p),
+              _p(const), _p(made), None if f32 is made else _p(f32), _p(out), B, S, float(threshold))
+    return made, out, f32
 
 
 def mask_prepare_broadcast(mask_row, B, threshold=-1000.0):
