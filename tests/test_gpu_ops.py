@@ -1088,6 +1088,30 @@ def test_attention_fp32(B, h, S, masked):
     assert got.dtype == np.float32 and rel_err(got, ref) <= 3e-6
 
 
+@pytest.mark.parametrize("B,h,S", [(1, 65, 256), (3, 29, 200), (5, 13, 264), (7, 12, 384), (2, 43, 512)])
+def test_attention_order_of_the_pairs(B, h, S):
+    """Launches around and above one workgroup a CU, where the kernels take the (sequence, head) pairs head by head: every sequence
+    is the checker's in fp16 (V transposed), and in fp32 has the bits that it has alone"""
+    say("attention order of pairs B=%d h=%d S=%d" % (B, h, S))
+    rng = np.random.default_rng(B * S + h)
+    o, H = ops(), h * 64
+    lens = rng.integers(1, S + 1, B).astype(np.int32)
+    lens[0] = S
+    qk = dev(rng.standard_normal((B * S, 2 * H)).astype(np.float32)).half()
+    vt = dev(rng.standard_normal((B, h, 64, S)).astype(np.float32)).half()
+    qkv = dev(rng.standard_normal((B * S, 3 * H)).astype(np.float32))
+    order = 1 if S % 16 == 0 else 0
+    got = o.attention_qk_vt(qk, o.permute_keys(vt) if order else vt, B, S, h, 0.125, kv_len=dev(lens), vt_key_order=order)
+    got32 = o.attention_packed(qkv, B, S, h, 0.125, kv_len=dev(lens))
+    for b in range(B):
+        rows, kv = slice(b * S, (b + 1) * S), dev(lens[b:b + 1])
+        assert torch.equal(got32[rows], o.attention_packed(qkv[rows].contiguous(), 1, S, h, 0.125, kv_len=kv))
+        ref = orc.attention_core(*(host(t).astype(np.float32)[None] for t in (
+            qk[rows, :H].reshape(S, h, 64).transpose(0, 1), qk[rows, H:].reshape(S, h, 64).transpose(0, 1), vt[b].transpose(1, 2))), 0.125,
+            np.where(np.arange(S)[None, :] < lens[b], 0.0, -10000.0).astype(np.float32))
+        assert rel_err(host(got[rows]).reshape(S, h, 64).transpose(1, 0, 2)[None], ref) <= FP16_TOL
+
+
 @pytest.mark.parametrize("S", [1, 31, 32, 33, 63, 64, 65, 129, 160, 289])
 def test_attention_fp32_rows_inside_a_matrix(S):
     """Rows of Q, K and V as column blocks of one matrix, whole and cut-off blocks of keys, lengths that leave key waves without a

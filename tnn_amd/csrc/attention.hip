@@ -122,6 +122,8 @@ struct AttnParams : StoreThrough {
     long vt_sb, vt_sh, vt_sd;  // V^T layout (VT kernels): element (b, head, d, s) at v[b*vt_sb + head*vt_sh + d*vt_sd + s]
     int S, B, heads;
     FixedDivisor by_blocks, by_heads;  // query blocks of a head (set by the launch, which knows the block size); heads
+    int sequences_inside;              // attention_dma_kernel's order of (sequence, head) pairs, see launch_attention
+    FixedDivisor by_batch;
     float scale_log2e;  // scale * log2(e)
     const float *mask;  // [B,S] additive or null
     const int32_t *kv_len;
@@ -506,8 +508,9 @@ __global__ void __launch_bounds__(NW * 64, (NW == 4 && DT == TNN_ROCM_F16) ? 3 :
     if (vid >= total)
         return;
     const int bh   = p.by_blocks.quotient(vid);
-    const int b    = p.by_heads.quotient(bh);
-    const int head = bh - b * p.heads;
+    const int outer = (p.sequences_inside ? p.by_batch : p.by_heads).quotient(bh);
+    const int inner = bh - outer * (p.sequences_inside ? p.B : p.heads);
+    const int b = p.sequences_inside ? inner : outer, head = p.sequences_inside ? outer : inner;
     const int q0   = (vid - bh * n_q) * BQ + wave * 32;
 
     int kv_end = S;
@@ -1343,11 +1346,24 @@ template <int DT, bool VT> __global__ void __launch_bounds__(256, 2) attention_s
 //   row-major  B1 S197 8.2 -> 5.5   B5 S197 9.7 -> 7.1   B8 S384 18.3 -> 17.2   B16 S256 14.3 (this one: 15.9)
 constexpr long kShortBlocksVT = 256, kShortBlocksRows = 1200;
 
+// Every XCD takes a contiguous run of (sequence, head) pairs.  Sequence by sequence, each gets the heads of one or few sequences,
+// and the one with the longest of them ends last.  Where the workgroups are on the chip at once (two waves each, below 1024 of
+// them, three a CU) and more than one a CU, the pairs go head by head instead, so that every XCD has heads of nearly all
+// sequences; us, 12 heads, lengths S / S/2 .. S / 16 .. S:
+//   B4 S384 10.0 10.9 11.1 -> 10.1 10.2 10.6   B8 S384 11.6 12.6 11.3 -> 11.7 11.8 10.5   B16 S256 10.2 11.2 11.1 -> 10.3 11.0 11.1
+// Larger launches run in several rounds, and there it is no better (B16 S512 21.9 21.8 18.7, head by head 22.2 21.8 19.2; B32 S512
+// 42.7 39.8 32.0, 43.7 39.5 33.1).  The longest sequence first, found from the lengths in the kernel, ends earlier still (B8 S384
+// 16 .. S 9.9, B16 S512 17.3), but every workgroup then waits for the lengths before its first address: +0.3 .. +1.0 us where
+// they are equal.
+constexpr unsigned kCusOfTheChip = 256;
+
 template <bool VT> int launch_attention(hipStream_t s, int dtype, AttnParams p, int B, int heads, int S, bool by_size = true) {
     const long blocks128 = (long)((S + 127) / 128) * heads * B, blocks32 = (long)((S + 31) / 32) * heads * B;
     const int mode = g_attention_dma;
     const bool few = by_size && (S <= 32 || blocks32 <= (VT ? kShortBlocksVT : kShortBlocksRows));
     p.by_heads     = FixedDivisor::of((uint32_t)heads);
+    p.by_batch     = FixedDivisor::of((uint32_t)B);
+    p.sequences_inside = 0;
     // grid of the launch with BQ queries per block
     auto blocks_of = [&](int bq) {
         const long n_q = (S + bq - 1) / bq;
@@ -1377,7 +1393,8 @@ template <bool VT> int launch_attention(hipStream_t s, int dtype, AttnParams p, 
             const dim3 grid = blocks_of(128);
             TR_LAUNCH_DMA(4, 256);
         } else {
-            const dim3 grid = blocks_of(64);
+            const dim3 grid    = blocks_of(64);
+            p.sequences_inside = p.kv_len && grid.x > kCusOfTheChip;
             TR_LAUNCH_DMA(2, 128);
         }
 #undef TR_LAUNCH_DMA
