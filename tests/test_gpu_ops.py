@@ -1350,7 +1350,7 @@ def test_mask_prepare_any_float_type():
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
-@pytest.mark.parametrize("S", [1, 63, 64, 65, 200])
+@pytest.mark.parametrize("S", [1, 63, 64, 65, 200, 256, 1023, 1025, 2300])
 def test_mask_prepare_ints(S, dtype):
     """Integers -> additive mask -> key counts in one launch: bit for bit the cast and element-wise launches and the launch that
     takes the counts from their result, also for values and constants that the type rounds or cannot hold."""

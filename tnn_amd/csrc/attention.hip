@@ -1016,9 +1016,11 @@ __global__ void __launch_bounds__(NW * 64, (NW == 4 && DT == TNN_ROCM_F16) ? 3 :
     }
 }
 
-// One wave per batch row, two passes over it (the second finds the row in cache): the row's largest value, then the
-// largest index whose mask value is above (largest value + threshold) and the smallest index whose value is not
-// exactly zero.  The cut is relative to the row's maximum because softmax is: a key whose bias lies `threshold` (a
+// One workgroup per batch row: the row's largest value, then the largest index whose mask value is above (largest value +
+// threshold) and the smallest index whose value is not exactly zero.  A thread holds its first four values (rows of up to 1024
+// keys are requested at once and read once); one wave a row with two passes was a chain of loads.  us, fp16 back to back:
+// B8 S384 3.4 -> 2.9, 4 x 1024 5.5 -> 3.0, 2 x 4096 16.3 -> 5.6; rows of one wave 2.1 -> 2.3.
+// The cut is relative to the row's maximum because softmax is: a key whose bias lies `threshold` (a
 // large negative number) below the best key's contributes exp(threshold + score difference) = 0 in fp32, whatever
 // constant the whole row carries.  Row b is read at mask + b * src_stride (0: one row serves every sequence); with
 // mask_f32 given, the row is also written there in fp32, densely (what the attention kernels read).
@@ -1028,37 +1030,64 @@ struct MaskSteps {
     int n = 0;
     int op[TNN_ROCM_MAX_MASK_STEPS] = {};
 };
+constexpr int kMaskThreads = 256;
 template <int DT, typename SRC>
-__global__ void mask_to_kv_len_kernel(const SRC *__restrict__ mask, long src_stride, MaskSteps steps,
-                                      const typename Elem<DT>::type *__restrict__ constants,
-                                      typename Elem<DT>::type *__restrict__ made, float *__restrict__ mask_f32,
-                                      int32_t *__restrict__ kv_len, int S, float threshold, int flag_zero_rows) {
-    const int b    = blockIdx.x;
-    const int lane = threadIdx.x;
+__global__ void __launch_bounds__(kMaskThreads)
+mask_to_kv_len_kernel(const SRC *__restrict__ mask, long src_stride, MaskSteps steps,
+                      const typename Elem<DT>::type *__restrict__ constants, typename Elem<DT>::type *__restrict__ made,
+                      float *__restrict__ mask_f32, int32_t *__restrict__ kv_len, int S, float threshold, int flag_zero_rows) {
+    constexpr int HELD = 4;
+    __shared__ float tops[kMaskThreads / 64];
+    __shared__ int lasts[kMaskThreads / 64], firsts[kMaskThreads / 64];
+    const int b = blockIdx.x, tid = threadIdx.x, step = blockDim.x, waves = step >> 6;
     const SRC *row = mask + (size_t)b * src_stride;
-    auto value     = [&](int j) -> float {
+    float c[TNN_ROCM_MAX_MASK_STEPS];  // requested together with the row
+#pragma unroll
+    for (int i = 0; i < TNN_ROCM_MAX_MASK_STEPS; ++i)
+        c[i] = std::is_same<SRC, int32_t>::value && i < steps.n ? Elem<DT>::ld(&constants[i]) : 0.f;
+    auto value = [&](SRC x) -> float {
         if constexpr (std::is_same<SRC, int32_t>::value) {
             typename Elem<DT>::type t;
-            Elem<DT>::st(&t, (float)row[j]);
-            for (int i = 0; i < steps.n; ++i) {
-                const float x = Elem<DT>::ld(&t), c = Elem<DT>::ld(&constants[i]);
-                Elem<DT>::st(&t, steps.op[i] == TNN_ROCM_MASK_ADD        ? __fadd_rn(x, c)
-                                 : steps.op[i] == TNN_ROCM_MASK_SUB      ? __fsub_rn(x, c)
-                                 : steps.op[i] == TNN_ROCM_MASK_SUB_FROM ? __fsub_rn(c, x)
-                                                                         : __fmul_rn(x, c));
+            Elem<DT>::st(&t, (float)x);
+#pragma unroll
+            for (int i = 0; i < TNN_ROCM_MAX_MASK_STEPS; ++i) {
+                if (i >= steps.n)
+                    break;
+                const float y = Elem<DT>::ld(&t);
+                Elem<DT>::st(&t, steps.op[i] == TNN_ROCM_MASK_ADD        ? __fadd_rn(y, c[i])
+                                 : steps.op[i] == TNN_ROCM_MASK_SUB      ? __fsub_rn(y, c[i])
+                                 : steps.op[i] == TNN_ROCM_MASK_SUB_FROM ? __fsub_rn(c[i], y)
+                                                                         : __fmul_rn(y, c[i]));
             }
             return Elem<DT>::ld(&t);
         } else {
-            return Elem<DT>::ld(&row[j]);
+            return Elem<DT>::ld(&x);
         }
     };
-    float top = -INFINITY;
-    for (int j = lane; j < S; j += 64) {
-        const float v = value(j);
+    auto write = [&](int j, float v) {
         if (made)
             Elem<DT>::st(&made[(size_t)b * S + j], v);
         if (mask_f32)
             mask_f32[(size_t)b * S + j] = v;
+    };
+    SRC raw[HELD];
+#pragma unroll
+    for (int i = 0; i < HELD; ++i) {
+        const int j = tid + i * step;
+        raw[i]      = S > 0 ? row[j < S ? j : S - 1] : SRC();
+    }
+    float held[HELD], top = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < HELD; ++i) {
+        held[i] = value(raw[i]);
+        if (tid + i * step < S) {
+            write(tid + i * step, held[i]);
+            top = held[i] > top ? held[i] : top;
+        }
+    }
+    for (int j = tid + HELD * step; j < S; j += step) {
+        const float v = value(row[j]);
+        write(j, v);
         top = v > top ? v : top;
     }
 #pragma unroll
@@ -1066,20 +1095,37 @@ __global__ void mask_to_kv_len_kernel(const SRC *__restrict__ mask, long src_str
         const float other = __shfl_xor(top, o, 64);
         top               = other > top ? other : top;
     }
+    if ((tid & 63) == 0)
+        tops[tid >> 6] = top;
+    __syncthreads();
+    for (int w = 0; w < waves; ++w)
+        top = tops[w] > top ? tops[w] : top;
     const float cut = top + threshold;
     int last = -1, first_nonzero = S;
-    for (int j = lane; j < S; j += 64) {
-        const float v = value(j);
+    auto look = [&](int j, float v) {
         if (v > cut)
-            last = j;
+            last = j;  // j grows
         if (v != 0.0f && j < first_nonzero)
             first_nonzero = j;
-    }
+    };
+#pragma unroll
+    for (int i = 0; i < HELD; ++i)
+        if (tid + i * step < S)
+            look(tid + i * step, held[i]);
+    for (int j = tid + HELD * step; j < S; j += step)
+        look(j, value(row[j]));
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) {
         const int other = __shfl_xor(last, o, 64), other_nz = __shfl_xor(first_nonzero, o, 64);
         last            = other > last ? other : last;
         first_nonzero   = other_nz < first_nonzero ? other_nz : first_nonzero;
+    }
+    if ((tid & 63) == 0)
+        lasts[tid >> 6] = last, firsts[tid >> 6] = first_nonzero;
+    __syncthreads();
+    for (int w = 0; w < waves; ++w) {
+        last          = lasts[w] > last ? lasts[w] : last;
+        first_nonzero = firsts[w] < first_nonzero ? firsts[w] : first_nonzero;
     }
     // No key above the cut (a row of -inf or NaN only): the reference still runs softmax(scores + mask) over all S
     // keys, so every key stays in, with its bias.  A row that masks every key with the same finite value keeps all
@@ -1088,7 +1134,7 @@ __global__ void mask_to_kv_len_kernel(const SRC *__restrict__ mask, long src_str
     // a plain padding mask is exactly 0 on every visible key: the attention kernel then needs the length only
     if (flag_zero_rows && first_nonzero >= len)
         len |= kKvLenMaskZero;
-    if (lane == 0)
+    if (tid == 0)
         kv_len[b] = len;
 }
 
@@ -1418,6 +1464,8 @@ template <bool VT> int launch_attention(hipStream_t s, int dtype, AttnParams p, 
 
 }  // namespace
 
+static dim3 mask_threads(int S) { return dim3(S >= kMaskThreads ? kMaskThreads : S <= 64 ? 64 : (S + 63) / 64 * 64); }
+
 extern "C" {
 
 int tnn_rocm_attention(void *stream, int dtype, const void *q, const void *k, const void *v, void *out, int B,
@@ -1549,7 +1597,7 @@ int tnn_rocm_mask_to_kv_len(void *stream, const float *mask, int32_t *kv_len, in
     if (B == 0)
         return 0;
     TR_REQUIRE(mask && kv_len, TNN_ROCM_EINVAL, "mask_to_kv_len: null pointer");
-    hipLaunchKernelGGL((mask_to_kv_len_kernel<TNN_ROCM_F32, float>), dim3(B), dim3(64), 0, (hipStream_t)stream, mask, (long)S,
+    hipLaunchKernelGGL((mask_to_kv_len_kernel<TNN_ROCM_F32, float>), dim3(B), mask_threads(S), 0, (hipStream_t)stream, mask, (long)S,
                        MaskSteps{}, (const float *)nullptr, (float *)nullptr, (float *)nullptr, kv_len, S, threshold, 0);
     TR_CHECK_LAUNCH();
     return 0;
@@ -1572,15 +1620,15 @@ int tnn_rocm_mask_prepare_strided(void *stream, int dtype, const void *mask, lon
     hipStream_t s = (hipStream_t)stream;
     switch (dtype) {
         case TNN_ROCM_F32:
-            hipLaunchKernelGGL((mask_to_kv_len_kernel<TNN_ROCM_F32, float>), dim3(B), dim3(64), 0, s, (const float *)mask,
+            hipLaunchKernelGGL((mask_to_kv_len_kernel<TNN_ROCM_F32, float>), dim3(B), mask_threads(S), 0, s, (const float *)mask,
                                mask_batch_stride, MaskSteps{}, (const float *)nullptr, (float *)nullptr, mask_f32, kv_len, S, threshold, 1);
             break;
         case TNN_ROCM_F16:
-            hipLaunchKernelGGL((mask_to_kv_len_kernel<TNN_ROCM_F16, half_t>), dim3(B), dim3(64), 0, s, (const half_t *)mask,
+            hipLaunchKernelGGL((mask_to_kv_len_kernel<TNN_ROCM_F16, half_t>), dim3(B), mask_threads(S), 0, s, (const half_t *)mask,
                                mask_batch_stride, MaskSteps{}, (const half_t *)nullptr, (half_t *)nullptr, mask_f32, kv_len, S, threshold, 1);
             break;
         case TNN_ROCM_BF16:
-            hipLaunchKernelGGL((mask_to_kv_len_kernel<TNN_ROCM_BF16, bf16_bits>), dim3(B), dim3(64), 0, s, (const bf16_bits *)mask,
+            hipLaunchKernelGGL((mask_to_kv_len_kernel<TNN_ROCM_BF16, bf16_bits>), dim3(B), mask_threads(S), 0, s, (const bf16_bits *)mask,
                                mask_batch_stride, MaskSteps{}, (const bf16_bits *)nullptr, (bf16_bits *)nullptr, mask_f32, kv_len, S, threshold, 1);
             break;
         default:
@@ -1607,7 +1655,7 @@ int tnn_rocm_mask_prepare_i32(void *stream, int dtype, const int32_t *ints, int 
     TR_REQUIRE(ints && mask && kv_len && (mask_f32 || dtype == TNN_ROCM_F32), TNN_ROCM_EINVAL, "mask_prepare_i32: null pointer");
     hipStream_t s = (hipStream_t)stream;
 #define TR_MASK(DT)                                                                                                     \
-    hipLaunchKernelGGL((mask_to_kv_len_kernel<DT, int32_t>), dim3(B), dim3(64), 0, s, ints, (long)S, steps,             \
+    hipLaunchKernelGGL((mask_to_kv_len_kernel<DT, int32_t>), dim3(B), mask_threads(S), 0, s, ints, (long)S, steps,             \
                        (const Elem<DT>::type *)constants, (Elem<DT>::type *)mask, mask_f32, kv_len, S, threshold, 1)
     switch (dtype) {
         case TNN_ROCM_F32: TR_MASK(TNN_ROCM_F32); break;
