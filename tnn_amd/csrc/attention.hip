@@ -1079,8 +1079,8 @@ mask_to_kv_len_kernel(const SRC *__restrict__ mask, long src_stride, MaskSteps s
     float held[HELD], top = -INFINITY;
 #pragma unroll
     for (int i = 0; i < HELD; ++i) {
-        held[i] = value(raw[i]);
-        if (tid + i * step < S) {
+        if (tid + i * step < S) {  // waves beyond the row's end make nothing
+            held[i] = value(raw[i]);
             write(tid + i * step, held[i]);
             top = held[i] > top ? held[i] : top;
         }
