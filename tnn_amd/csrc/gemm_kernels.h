@@ -2299,8 +2299,8 @@ constexpr int kNumCU = 256;
 // int8: M from 16 to 8192, the four projections of hidden sizes 768 and 1024 with their fused epilogues; fp32: M from 16 to
 // 3072), taken over twelve weight sets in turn so that weights come from the memory-side cache as they do inside a network:
 // python -m tnn_amd.bench_ops --tile-sweep measures them and fits the rows.  A single launch is 4 .. 10 % off its prediction,
-// so picks closer than that are as good as drawn; taken together the picks are 1.5 % (fp16), 1.1 % (int8), 2.9 % (fp32) behind
-// the best shape of each launch back to back, and 0.31, 0.21 and 0.60 us inside the network (bench_configs --config tiles;
+// so picks closer than that are as good as drawn; taken together the picks are 2.4 % (fp16), 1.9 % (int8), 5.2 % (fp32) behind
+// the best shape of each launch back to back, and 0.29, 0.37 and 0.45 us inside the network (bench_configs --config tiles;
 // profiles/gemm_tile_choice.txt).  The rules this replaced, made for M >= 1024, were 51 %, 34 % and 77 % behind over that range:
 //   M=  32 N= 768 K=3072 fp16  23.1 -> 7.3 us   (64x64 tiles: 12 CUs, one two-stage slab after another)
 //   M= 256 N= 768 K=3072 fp16  23.7 -> 7.2      M= 256 N=2304 K=768 fp16  8.7 -> 6.2
