@@ -508,9 +508,10 @@ __global__ void __launch_bounds__(NW * 64, (NW == 4 && DT == TNN_ROCM_F16) ? 3 :
     if (vid >= total)
         return;
     const int bh   = p.by_blocks.quotient(vid);
-    const int outer = (p.sequences_inside ? p.by_batch : p.by_heads).quotient(bh);
-    const int inner = bh - outer * (p.sequences_inside ? p.B : p.heads);
-    const int b = p.sequences_inside ? inner : outer, head = p.sequences_inside ? outer : inner;
+    const bool inside = NW == 2 && p.sequences_inside;
+    const int outer   = (inside ? p.by_batch : p.by_heads).quotient(bh);
+    const int inner   = bh - outer * (inside ? p.B : p.heads);
+    const int b = inside ? inner : outer, head = inside ? outer : inner;
     const int q0   = (vid - bh * n_q) * BQ + wave * 32;
 
     int kv_end = S;
