@@ -1199,6 +1199,32 @@ def test_attention_fp32_small_and_large(S, eq, ek, ev, scale):
     assert np.abs(got - ref).max() <= 3e-6 * np.abs(ref).max() + 2.0 ** -149
 
 
+@pytest.mark.parametrize("what,S", [("probability", 20), ("probability", 160), ("rescaling factor", 160)])
+def test_attention_fp32_exponentials(what, S):
+    """Two keys count, one with score 0 and one with score x < -17.4, so that the sum rounds to 1, and V is 1 at the second key: the
+    answer is the kernel's exp(x) itself, as a probability or as the factor that a block's sums get from a later, larger maximum.  It
+    keeps expf's errors (0.857 ulp at most and 2.63e-8 root mean square, over every float), and the bits there are below the
+    smallest normal value: half of the smallest step for the exponential's own and half for its scaling."""
+    say("attention fp32 exponential S=%d, %s" % (S, what))
+    rng = np.random.default_rng(S)
+    B, h = 24, 16
+    q, k, v = (np.zeros((B, h, S, 64), np.float32) for _ in range(3))
+    x = -rng.uniform(17.5, 104, (B, h, S)).astype(np.float32)
+    small, top = (1, 0) if what == "probability" else (0, 128)  # the keys with score x and with score 0
+    q[..., 0], k[:, :, small, 0], v[:, :, small, :] = x, 1, 1
+    mask = np.full((B, S), -np.inf, np.float32)
+    mask[:, [small, top]] = 0
+    got = host(ops().attention(dev(q), dev(k), dev(v), 1.0, mask=dev(mask)))
+    assert (got == got[..., :1]).all()
+    e, want = got[..., 0].astype(np.float64), np.exp(x.astype(np.float64))
+    normal = want >= 2.0 ** -126
+    ulps = np.abs(e - want) / np.spacing(want.astype(np.float32)).astype(np.float64)
+    assert ulps[normal].max() <= 0.87, ulps[normal].max()
+    rel = ((e - want) / want)[normal]
+    assert np.sqrt((rel ** 2).mean()) <= 2.75e-8, np.sqrt((rel ** 2).mean())
+    assert (~normal).any() and ulps[~normal].max() <= 1.0, ulps[~normal].max()
+
+
 def test_attention_packed_qkv_layout():
     say("attention packed [T,3H]")
     B, S, h = 2, 96, 12

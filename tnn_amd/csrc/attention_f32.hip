@@ -19,13 +19,15 @@
 // with the fp32 matrix instruction, operands straight from memory (`exact` below): the answer is then that of the layers in
 // fp32 arithmetic.  The check is 33 instructions a wave.
 //
-// What bounds it: the vector ALU (4.5 instructions for each of the 80 values of K, P and V that a lane converts for a block, 7 for
-// each of its 17 exponentials; 57 % of all clocks at 16 x 384 tokens, the matrix pipe 25 %) once a SIMD has three waves, and the
+// What bounds it: the vector ALU (4.5 instructions for each of the 80 values of K, P and V that a lane converts for a block, 10 for
+// each of its 17 exponentials; 57 % of all clocks at 16 x 384 tokens, the matrix pipe 25 %, when it was 7) once a SIMD has three waves, and the
 // latency of a block's chain below that.  So: three waves a SIMD (the planes of Q are made once per workgroup and lie in LDS, a
 // block's rows are requested when the registers of the rows before are free), no work for the mask in blocks that are whole, and
 // requests that every path to their waits makes alike, or the compiler waits for V where K is meant.
 // us, 12 heads, in a row: the decomposed launches -> Q's planes in registers, two waves a SIMD -> this form
 //   1 x 128 tokens 45 -> 6.9 -> 6.4, 4 x 384 136 -> 29.1 -> 26.2 (with an additive mask 38 -> 28), 16 x 384 79 -> 73, 1 x 16 6.1 -> 5.8
+// and with exponentials as accurate as expf's (another machine) 1 x 128 6.68 -> 6.77, 4 x 384 27.1 -> 27.4, 16 x 384 73.9 -> 75.9,
+// 1 x 16 6.07 -> 6.13; expf itself: see exp_not_positive
 #include "common.h"
 #include "split_f32.h"
 
@@ -60,15 +62,19 @@ __device__ __forceinline__ float other_half(float v) {
     return (threadIdx.x & 32) ? __uint_as_float(r[0]) : __uint_as_float(r[1]);
 }
 
-// exp(x) for x <= 0 (a NaN stays one): the product with log2 e in two parts, the first to the exponential instruction (1 ulp), the
-// second as a factor 1 + d.  Seven instructions where expf takes fourteen; results below the smallest normal value are zero, next
-// to a sum that holds a 1.
+// exp(x) for x <= 0 as 2^n 2^f, n the whole number nearest to x log2 e.  The product with log2 e is formed in two parts and the
+// second joins f behind the subtraction of n, which is exact, so that the argument of the exponential instruction is rounded once
+// and its result never again.  Below -200 the result is zero without a product that overflows; a NaN stays one; results below the
+// smallest normal value keep the bits there are.  Ten instructions where expf takes fourteen, for any sign.  Errors over every
+// float of [-87.3, -2^-20]: at most 0.857 ulp, 2.63e-8 root mean square from -1 down, both as expf's (0.857, 2.63e-8).  The second part as
+// a factor behind the exponential is seven instructions, but rounds the result again and loses what is not normal: 1.262 ulp,
+// 3.63e-8.
 __device__ __forceinline__ float exp_not_positive(float x) {
+    x              = __builtin_elementwise_maximum(x, -200.f);
     const float y  = __fmul_rn(x, 1.44269502f);
     const float lo = fmaf(x, 1.92596299e-8f, fmaf(x, 1.44269502f, -y));
-    const float e  = __builtin_amdgcn_exp2f(y);
-    // where x or y is infinite the second part is no number, and the first is zero
-    return fmaf(e, __fmul_rn(__builtin_amdgcn_fmed3f(lo, -1.f, 1.f), 0.693147182f), e);
+    const float n  = rintf(y);
+    return __builtin_ldexpf(__builtin_amdgcn_exp2f(__fadd_rn(__fsub_rn(y, n), lo)), (int)n);
 }
 
 // At least three waves a SIMD (168 registers): 4 x 384 tokens are 576 workgroups, two and a quarter for each CU, and with two a CU
