@@ -1827,6 +1827,45 @@ def test_folded_layernorm_statistics_at_the_ends(dtype, code):
         lib.tnn_rocm_debug_set_gemm_config(0)
 
 
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
+@pytest.mark.parametrize("K", [384, 768, 1536])
+@pytest.mark.parametrize("code", [0, 6111141, 9111141, 3112221, 2222221, 3332221])
+def test_folded_layernorm_statistics_of_rows_with_little_spread(dtype, K, code):
+    """Widths that are no power of two and rows that hardly vary: {rstd, mean} as far as the row's fp32 sums know the variance
+    (which is all the way where these are exact: constant rows, and one value of a row a step off)"""
+    say("folded LayerNorm, little spread %s, K=%d, shape %d" % (dtype, K, code))
+    from tnn_amd import capi
+    o, lib, td = ops(), capi.load(), getattr(torch, dtype)
+    gen = torch.Generator().manual_seed(K + code)
+    M, N = 66, 136
+    t = torch.randn(M, K, generator=gen).to(td)
+    for row, c in enumerate((0, 1, -2.5, 100, -0.0078125, 768)):
+        t[row] = c
+    t[6], t[6, 7], t[7], t[7, K - 1] = 1, 1.0078125, -3, -3.015625
+    exact = 8
+    for row, c in enumerate((1, 3.3, 20, 300)):
+        t[exact + row] = (c * (1 + 0.01 * torch.randn(K, generator=gen))).to(td)
+    w = (torch.randn(N, K, generator=gen) * 0.05).to(td)
+    zero, col = torch.zeros(N, device="cuda"), w.float().sum(1).cuda()
+    sums = _row_sums(t, 8)
+    d = t.double()
+    lib.tnn_rocm_debug_set_gemm_config(code)
+    try:
+        for eps in (1e-12, 1e-5):
+            var = d.var(1, unbiased=False) + float(np.float32(eps))
+            # each sum of squares is up to 2^-24 off, and so is the sum whose square is taken off; the root halves the error
+            allowed = 3e-7 + 2.0 ** -24 * 1.5 * (d ** 2).mean(1) / var
+            allowed[:exact] = 3e-7
+            for row_sums in (None, (sums, 8)):
+                h, st = o.gemm_ln(t.cuda(), w.cuda(), zero, col, eps, want_stats=True, row_sums=row_sums)
+                st = st.cpu().double()
+                assert ((st[:, 0] * var.sqrt() - 1).abs() <= allowed).all()
+                assert ((st[:, 1] - d.mean(1)).abs() <= 2e-7 * d.abs().mean(1)).all()
+                assert torch.isfinite(h).all()
+    finally:
+        lib.tnn_rocm_debug_set_gemm_config(0)
+
+
 @pytest.mark.parametrize("dtype", ["f16", "bf16"])
 def test_attention_quantised_second_output_bit_exact(dtype):
     """The int8 tensor the attention kernel can write next to its output equals the checker's x86 quantiser applied to

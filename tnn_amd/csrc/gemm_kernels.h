@@ -385,7 +385,8 @@ template <int DT> struct QkvSplitEpilogue : StoreThrough {
 // Other readers of y (the residual additions) still need the tensor: the workgroup of tile column j writes
 // y for the j-th share of the columns of its rows, so the LayerNorm launch disappears without y disappearing.
 struct LnFold {
-    float inv_cols, eps;
+    double cols, inv_cols;      // K and 1 / K: rounded to fp32, 1 / 768 took 3e-8 of the squared mean off the variance
+    float eps;
     const float *colsum;        // [N]
     const float *gamma, *beta;  // [K], for the y side output
     void *y;                    // [M, K] in the compute type, or nullptr
@@ -394,6 +395,17 @@ struct LnFold {
     const float2 *row_sums;     // kTakesRowSums: [sum_blocks][M] {sum, sum of squares} over a block of columns of t
     int sum_blocks;
 };
+
+// Mean, and variance + eps, of a row from its sums.  K s2 - s1^2 is formed exactly before it is rounded, so that rows of little
+// spread far from zero keep what the sums themselves know of their variance: with E[x^2] - mean^2 in double a row at 100 is off by
+// 2e-12, twice the eps of the models.  The sums are made of fp32 parts and can leave it a hair below zero, where it is cut
+// off.  A NaN stays one.
+__device__ __forceinline__ double row_moments(const LnFold &ln, double s1, double s2, double *mean) {
+    const double square = s1 * s1;
+    const double spread = fma(ln.cols, s2, -square) - fma(s1, s1, -square);
+    *mean = s1 * ln.inv_cols;
+    return (spread < 0.0 ? 0.0 : spread * (ln.inv_cols * ln.inv_cols)) + (double)ln.eps;
+}
 
 // row sum and sum of squares of the eight values of an A fragment register quad
 template <int DT> __device__ __forceinline__ void ln_accumulate(const uint4 &frag, float &s1, float &s2) {
@@ -1597,8 +1609,8 @@ __global__ void __launch_bounds__(CFG::NT)
                     }
                     // The other waves wait at a barrier while these do this, so it is kept short: the block sums (fp32)
                     // are added up in double in a fixed order (the sum of squares of a row that sits far from zero
-                    // would lose the variance's digits in fp32), the variance is formed as a difference of doubles,
-                    // and its reciprocal root is taken in single precision with one Newton step.
+                    // would lose the variance's digits in fp32), and the reciprocal root of the variance is taken in
+                    // single precision with one Newton step.
                     double f1 = 0.0, f2 = 0.0;
 #pragma unroll
                     for (int i = 0; i < NSUM; ++i) {
@@ -1615,14 +1627,11 @@ __global__ void __launch_bounds__(CFG::NT)
                         f1 = add_lane_xor<16>(f1), f2 = add_lane_xor<16>(f2);
                     if constexpr (LANES_ROW >= 2)
                         f1 = add_lane_xor<32>(f1), f2 = add_lane_xor<32>(f2);
-                    const double mean = f1 * (double)epi.ln.inv_cols;
-                    // fp32 block sums can leave E[x^2] - mean^2 a hair below zero for rows whose spread is tiny next to
-                    // their mean; the variance is clamped there (with eps = 1e-12 the root would otherwise be NaN)
-                    const double var  = f2 * (double)epi.ln.inv_cols - mean * mean;
-                    const float ve    = (float)((var > 0.0 ? var : 0.0) + (double)epi.ln.eps);
-                    const float e     = __builtin_amdgcn_rsqf(ve);
+                    double mean;
+                    const float ve = (float)row_moments(epi.ln, f1, f2, &mean);
+                    const float e  = __builtin_amdgcn_rsqf(ve);
                     // an infinite variance has the root 0, and none at all without eps an infinite one
-                    const float r     = e > 0.f && e < INFINITY ? e * (1.5f - 0.5f * ve * e * e) : e;
+                    const float r  = e > 0.f && e < INFINITY ? e * (1.5f - 0.5f * ve * e * e) : e;
                     if (sum_part == 0)
                         reinterpret_cast<float2 *>(lds_dyn + CFG::lds_bytes)[sum_row] = make_float2(r, (float)mean);
                 }
@@ -2020,10 +2029,10 @@ __global__ void __launch_bounds__(CFG::NT)
                 s1 += v.x;
                 s2 += v.y;
             }
-            const double mean = s1 * (double)epi.ln.inv_cols;
-            const double var  = s2 * (double)epi.ln.inv_cols - mean * mean + (double)epi.ln.eps;
-            const float2 st   = make_float2((float)reciprocal_root(var), (float)mean);
-            row_st[tid]       = st;
+            double mean;
+            const double var = row_moments(epi.ln, s1, s2, &mean);
+            const float2 st  = make_float2((float)reciprocal_root(var), (float)mean);
+            row_st[tid]      = st;
             if (epi.ln.stats && n0 == 0 && m0 + tid < M)  // every tile column holds them; the first one hands them on
                 store_out8(epi.through, &epi.ln.stats[m0 + tid], st);
         }
@@ -2609,7 +2618,7 @@ template <int DT>
 int GemmTyped<DT>::ln(hipStream_t s, const void *t, const void *w_folded, const float *bias_folded, const float *colsum,
                       const float *gamma, const float *beta, float eps, void *C, void *y, float *row_stats,
                       const float *row_sums, int row_sum_blocks, int M, int N, int K, int flags, const void *residual) {
-    const LnFold ln{1.0f / (float)K, eps, colsum, gamma, beta, y, g_ln_y_ahead.load(), (float2 *)row_stats,
+    const LnFold ln{(double)K, 1.0 / (double)K, eps, colsum, gamma, beta, y, g_ln_y_ahead.load(), (float2 *)row_stats,
                     (const float2 *)row_sums, row_sum_blocks};
     int rc = kNotWithRowSums;  // a tile shape that takes the statistics from its own tiles declines handed-over sums
     if (row_sums && row_sum_blocks <= 12)
@@ -2640,7 +2649,7 @@ int GemmTyped<DT>::qkv_split_ln(hipStream_t s, const void *t, const void *wqkv_f
                                 const float *colsum, const float *gamma, const float *beta, float eps, void *qk, void *vt,
                                 void *y, float *row_stats, const float *row_sums, int row_sum_blocks, int B, int S, int heads,
                                 int K, int vt_key_order) {
-    const LnFold ln{1.0f / (float)K, eps, colsum, gamma, beta, y, g_ln_y_ahead.load(), (float2 *)row_stats,
+    const LnFold ln{(double)K, 1.0 / (double)K, eps, colsum, gamma, beta, y, g_ln_y_ahead.load(), (float2 *)row_stats,
                     (const float2 *)row_sums, row_sum_blocks};
     int rc = kNotWithRowSums;
     if (row_sums && row_sum_blocks <= 12)
