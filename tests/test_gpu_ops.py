@@ -211,25 +211,60 @@ def test_layernorm_fp16():
 
 
 @pytest.mark.parametrize("dtype", ["float32", "float16", "bfloat16"])
-@pytest.mark.parametrize("vecs", [1, 33, 64, 65, 96, 97, 128, 129, 192, 193, 256, 257, 512])
+@pytest.mark.parametrize("vecs", [1, 32, 33, 64, 65, 96, 97, 128, 129, 192, 193, 256, 257, 512])
 def test_layernorm_row_count_changes_nothing(dtype, vecs):
-    """Launches of up to 6144 rows request everything ahead, larger ones do not: the same bits, at every width a lane count or
-    a number of vectors per lane ends at; a few rows against the checker."""
+    """Launches of up to 1024 (rows of more than 256 half vectors) .. 16384 rows (up to 64 fp32 vectors) request everything ahead, larger
+    ones do not: the same bits, at every width a lane count or a number of vectors per lane ends at; a few rows against the checker."""
     say("layernorm %s, rows of %d 16-byte vectors" % (dtype, vecs))
     td = getattr(torch, dtype)
-    cols, rows = vecs * (4 if dtype == "float32" else 8), 6145
+    cols, rows = vecs * (4 if dtype == "float32" else 8), 6145 if vecs > 128 else 16392
     gen = torch.Generator(device="cuda").manual_seed(vecs)
     x, r = (torch.randn(rows, cols, device="cuda", generator=gen).to(td) for _ in range(2))
     g, b = (torch.randn(cols, device="cuda", generator=gen) for _ in range(2))
     for res in (None, r):
         y, q = ops().layernorm(x, g, b, 1e-5, residual=res, q_inv_scale=20.0)
-        for lo, hi in ((0, 6144), (6140, 6145), (0, 1)):
+        for lo, hi in ((0, 6144), (6140, 6145), (0, 1), (0, 1024), (1000, 3049), (2000, 5072)):
             ys, qs = ops().layernorm(x[lo:hi].contiguous(), g, b, 1e-5, residual=None if res is None else res[lo:hi].contiguous(),
                                      q_inv_scale=20.0)
             assert torch.equal(ys, y[lo:hi]) and torch.equal(qs, q[lo:hi])
         some = x[:3].float() if res is None else x[:3].float() + res[:3].float()
         ref = orc.layernorm(host(some), host(g), host(b), 1e-5)
         assert rel_err(host(y[:3].float()), ref) <= {"float32": 2e-6, "float16": 2e-3, "bfloat16": 1.6e-2}[dtype]
+
+
+def _device_us(fns, launches=10, replays=5):
+    """us a launch of each function, in graphs of `launches` that take turns: the best replay of each"""
+    graphs = []
+    for fn in fns:
+        fn()
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            for _ in range(launches):
+                fn()
+        graphs.append(graph)
+    best = [float("inf")] * len(fns)
+    for _ in range(replays):
+        for i, graph in enumerate(graphs):
+            e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            graph.replay()
+            e0.record()
+            graph.replay()
+            e1.record()
+            torch.cuda.synchronize()
+            best[i] = min(best[i], e0.elapsed_time(e1) * 1e3 / launches)
+    return best
+
+
+@pytest.mark.parametrize("cols", [2304, 4096])
+def test_layernorm_wide_rows_keep_their_waves(cols):
+    """Half the rows take half the time (0.51 of it, measured with 2304 columns).  With everything requested ahead beyond the rows that
+    are resident then, a quarter of the waves are, and they took as long as all of them (1.14)."""
+    say("layernorm fp16, time of 4096 and 8192 rows of %d" % cols)
+    x, r = (torch.randn(8192, cols, device="cuda").half() for _ in range(2))
+    g, b = torch.ones(cols, device="cuda"), torch.zeros(cols, device="cuda")
+    half, whole = _device_us([lambda n=n: ops().layernorm(x[:n], g, b, 1e-5, residual=r[:n]) for n in (4096, 8192)])
+    assert half < 0.75 * whole, (half, whole)
 
 
 def test_layernorm_rejects_empty():

@@ -11,7 +11,6 @@ namespace {
 
 constexpr int kBlock       = 256;
 constexpr int kRowsPerBlk  = kBlock / kWave;
-constexpr int kLnAheadRows = 6144;  // LayerNorm launches of more rows request scale and shift behind the reduction
 constexpr int kMaxVecPerLn = 8;  // row cached in registers when cols <= 64 * VEC * 8
 
 __device__ __forceinline__ double wave_sum_f64(double v) {
@@ -287,34 +286,41 @@ int launch_layernorm(hipStream_t s, const void *x, const void *res, const float 
         return TNN_ROCM_ESHAPE;
     }
     if (al && cols <= kWave * VEC * kMaxVecPerLn) {
-        // All rows resident at once (768 columns fp16: 3 workgroups of 8 rows a CU with everything requested ahead): the launch
-        // is as long as one row's chain.  More rows, and other waves cover it: 196608 rows of 1024 with a residual 158 us, 222
-        // requested ahead.
-        const bool ahead = rows <= kLnAheadRows;
+        // Everything requested ahead where all rows are resident at once: the launch is as long as one row's chain.  More rows, and
+        // other waves cover it, of which the registers taken leave fewer: 196608 rows of 1024 with a residual 158 us, 222 requested
+        // ahead.  How many rows that is follows from the registers of the form: HALF / F32 workgroups a CU (of eight rows, or of
+        // four where a wave owns one).  us with a residual, requested where used -> ahead, at the last rows that are resident and
+        // at more of them:
+        //   fp16  768 columns 6144 rows 6.1 -> 6.0, 12288 9.9 -> 11.5     1536 4096 7.2 -> 7.1, 6144 9.6 -> 11.0
+        //        2048 3072 7.2 -> 7.1, 4096 8.7 -> 10.0                   2304 1024 5.9 -> 6.0, 2048 7.4 -> 11.2, 4096 10.6 -> 23.5
+        //   fp32 1024 4096 7.2 -> 6.6, 5120 10.8 -> 11.5                  2048 2048 10.0 -> 7.2, 4096 16.4 -> 18.0
 #define TR_LN_LAUNCH(LPR, NV, AHEAD)                                                                                  \
     hipLaunchKernelGGL((layernorm_kernel<DT, true, LPR, NV, AHEAD>),                                                  \
                        dim3((rows + kRowsPerBlk * (kWave / LPR) - 1) / (kRowsPerBlk * (kWave / LPR))), block, 0, s,   \
                        (const T *)x, (const T *)res, gamma, beta, (T *)y, rows, cols, eps, out_q, q_inv, emb,     \
                        StoreThrough())
-#define TR_LN(LPR, NV)                                                                                                \
+#define TR_LN(LPR, NV, HALF, F32)                                                                                     \
     do {                                                                                                              \
-        if (ahead)                                                                                                    \
+        constexpr int resident = 256 * kRowsPerBlk * (kWave / LPR) * (DT == TNN_ROCM_F32 ? F32 : HALF);               \
+        if (rows <= resident)                                                                                         \
             TR_LN_LAUNCH(LPR, NV, true);                                                                              \
         else                                                                                                          \
             TR_LN_LAUNCH(LPR, NV, false);                                                                             \
     } while (0)
-        if (nv <= 64)
-            TR_LN(32, 2);
+        if (nv <= 32)  // a second vector of a lane would be requested twice: 8192 embedded rows of 256 halves 6.6 us with it
+            TR_LN(32, 1, 8, 8);
+        else if (nv <= 64)
+            TR_LN(32, 2, 5, 8);
         else if (nv <= 96)
-            TR_LN(32, 3);
+            TR_LN(32, 3, 4, 6);
         else if (nv <= 128)
-            TR_LN(32, 4);
+            TR_LN(32, 4, 3, 4);
         else if (nv <= 192)
-            TR_LN(64, 3);
+            TR_LN(64, 3, 4, 6);
         else if (nv <= 256)
-            TR_LN(64, 4);
+            TR_LN(64, 4, 3, 4);
         else
-            TR_LN(64, 8);
+            TR_LN(64, 8, 1, 2);
 #undef TR_LN
 #undef TR_LN_LAUNCH
     } else if (cols <= kWave * kMaxVecPerLn) {
