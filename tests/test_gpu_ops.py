@@ -1411,7 +1411,7 @@ def test_mask_prepare_any_float_type():
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
-@pytest.mark.parametrize("S", [1, 63, 64, 65, 200, 256, 1023, 1025, 2300])
+@pytest.mark.parametrize("S", [1, 63, 64, 65, 200, 256, 257, 1023, 1025, 2300])
 def test_mask_prepare_ints(S, dtype):
     """Integers -> additive mask -> key counts in one launch: bit for bit the cast and element-wise launches and the launch that
     takes the counts from their result, also for values and constants that the type rounds or cannot hold."""
@@ -1643,6 +1643,32 @@ def test_mask_to_kv_len():
     a1 = ops().attention_qk_vt(qk, vt, B, S8, h, 0.125, mask=dev(mm))
     a2 = ops().attention_qk_vt(qk, vt, B, S8, h, 0.125, mask=dev(mm), kv_len=ops().mask_to_kv_len(dev(mm), flagged=True))
     assert rel_err(host(a2), host(a1)) <= 1e-3
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("S", [1, 2, 63, 64, 65, 128, 191, 255, 256, 257, 511, 512, 513, 1024, 1025])
+def test_mask_key_counts_at_the_edges(S, dtype):
+    """Rows that one wave holds, rows that four hold and longer ones, whose last visible key is the first, the last or one where a
+    lane's next value or another wave's begins: the counts and flags by their definition, and the row's copy."""
+    say("mask key counts S=%d %s" % (S, dtype))
+    lens = [n for n in sorted({1, 2, S // 2, S - 1, S} | {e + d for e in (64, 128, 192, 256, 512, 768, 1024) for d in (0, 1)}) if 0 < n <= S]
+    m = np.full((2 * len(lens) + 2, S), -10000.0, np.float32)
+    for i, n in enumerate(lens):
+        m[2 * i:2 * i + 2, :n] = 0
+        m[2 * i + 1, n - 1] = -0.5              # the last visible key has a bias
+    m[-2], m[-1] = -np.inf, np.nan              # no key above the cut: all stay
+    md = dev(m).to(dtype)
+    wide = host(md.float())
+    kv, f32 = ops().mask_prepare(md)
+    with np.errstate(invalid="ignore"):
+        top = np.where(np.isnan(wide), -np.inf, wide).max(1)
+        seen = wide > (top - np.float32(1000))[:, None]
+    want = [int(np.nonzero(r)[0].max()) + 1 if r.any() else S for r in seen]
+    plain = [not (w[:n] != 0).any() for w, n in zip(wide, want)]
+    got = host(kv)
+    assert [int(v) & ~(1 << 30) for v in got] == want
+    assert [bool(int(v) >> 30 & 1) for v in got] == plain
+    assert np.array_equal(host(f32), wide, equal_nan=True)
 
 
 def test_mask_cut_is_relative_to_the_row_maximum():

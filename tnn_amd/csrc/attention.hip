@@ -1019,8 +1019,8 @@ __global__ void __launch_bounds__(NW * 64, (NW == 4 && DT == TNN_ROCM_F16) ? 3 :
 
 // One workgroup per batch row: the row's largest value, then the largest index whose mask value is above (largest value +
 // threshold) and the smallest index whose value is not exactly zero.  A thread holds its first four values (rows of up to 1024
-// keys are requested at once and read once); one wave a row with two passes was a chain of loads.  us, fp16 back to back:
-// B8 S384 3.4 -> 2.9, 4 x 1024 5.5 -> 3.0, 2 x 4096 16.3 -> 5.6; rows of one wave 2.1 -> 2.3.
+// keys are requested at once and read once); one wave a row with two passes was a chain of loads.  us, fp16 back to back, eight
+// rows: 64 keys 2.3 as before, 256 2.9 -> 2.5, 384 3.3 -> 2.7, 1024 5.5 -> 2.8, 4096 16.3 -> 5.6.
 // The cut is relative to the row's maximum because softmax is: a key whose bias lies `threshold` (a
 // large negative number) below the best key's contributes exp(threshold + score difference) = 0 in fp32, whatever
 // constant the whole row carries.  Row b is read at mask + b * src_stride (0: one row serves every sequence); with
@@ -1032,15 +1032,19 @@ struct MaskSteps {
     int op[TNN_ROCM_MAX_MASK_STEPS] = {};
 };
 constexpr int kMaskThreads = 256;
-template <int DT, typename SRC>
-__global__ void __launch_bounds__(kMaskThreads)
+// ONE_WAVE: rows of up to 256 values, which one wave holds: nothing goes through LDS and no wave waits for another (four waves for
+// these too: 64 keys 2.6, 128 2.7, 256 2.9 us).
+template <int DT, typename SRC, bool ONE_WAVE>
+__global__ void __launch_bounds__(ONE_WAVE ? 64 : kMaskThreads)
 mask_to_kv_len_kernel(const SRC *__restrict__ mask, long src_stride, MaskSteps steps,
                       const typename Elem<DT>::type *__restrict__ constants, typename Elem<DT>::type *__restrict__ made,
                       float *__restrict__ mask_f32, int32_t *__restrict__ kv_len, int S, float threshold, int flag_zero_rows) {
     constexpr int HELD = 4;
     __shared__ float tops[kMaskThreads / 64];
     __shared__ int lasts[kMaskThreads / 64], firsts[kMaskThreads / 64];
-    const int b = blockIdx.x, tid = threadIdx.x, step = blockDim.x, waves = step >> 6;
+    constexpr int step = ONE_WAVE ? 64 : kMaskThreads, waves = step / 64;
+    const int b = blockIdx.x, tid = threadIdx.x;
+    touch_kernel_args<128>();
     const SRC *row = mask + (size_t)b * src_stride;
     float c[TNN_ROCM_MAX_MASK_STEPS];  // requested together with the row
 #pragma unroll
@@ -1075,7 +1079,7 @@ mask_to_kv_len_kernel(const SRC *__restrict__ mask, long src_stride, MaskSteps s
 #pragma unroll
     for (int i = 0; i < HELD; ++i) {
         const int j = tid + i * step;
-        raw[i]      = S > 0 ? row[j < S ? j : S - 1] : SRC();
+        raw[i]      = i * step < S ? row[j < S ? j : S - 1] : SRC();
     }
     float held[HELD], top = -INFINITY;
 #pragma unroll
@@ -1086,7 +1090,7 @@ mask_to_kv_len_kernel(const SRC *__restrict__ mask, long src_stride, MaskSteps s
             top = held[i] > top ? held[i] : top;
         }
     }
-    for (int j = tid + HELD * step; j < S; j += step) {
+    for (int j = tid + HELD * step; !ONE_WAVE && j < S; j += step) {
         const float v = value(row[j]);
         write(j, v);
         top = v > top ? v : top;
@@ -1096,11 +1100,13 @@ mask_to_kv_len_kernel(const SRC *__restrict__ mask, long src_stride, MaskSteps s
         const float other = __shfl_xor(top, o, 64);
         top               = other > top ? other : top;
     }
-    if ((tid & 63) == 0)
-        tops[tid >> 6] = top;
-    __syncthreads();
-    for (int w = 0; w < waves; ++w)
-        top = tops[w] > top ? tops[w] : top;
+    if constexpr (!ONE_WAVE) {
+        if ((tid & 63) == 0)
+            tops[tid >> 6] = top;
+        __syncthreads();
+        for (int w = 0; w < waves; ++w)
+            top = tops[w] > top ? tops[w] : top;
+    }
     const float cut = top + threshold;
     int last = -1, first_nonzero = S;
     auto look = [&](int j, float v) {
@@ -1113,7 +1119,7 @@ mask_to_kv_len_kernel(const SRC *__restrict__ mask, long src_stride, MaskSteps s
     for (int i = 0; i < HELD; ++i)
         if (tid + i * step < S)
             look(tid + i * step, held[i]);
-    for (int j = tid + HELD * step; j < S; j += step)
+    for (int j = tid + HELD * step; !ONE_WAVE && j < S; j += step)
         look(j, value(row[j]));
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) {
@@ -1121,12 +1127,14 @@ mask_to_kv_len_kernel(const SRC *__restrict__ mask, long src_stride, MaskSteps s
         last            = other > last ? other : last;
         first_nonzero   = other_nz < first_nonzero ? other_nz : first_nonzero;
     }
-    if ((tid & 63) == 0)
-        lasts[tid >> 6] = last, firsts[tid >> 6] = first_nonzero;
-    __syncthreads();
-    for (int w = 0; w < waves; ++w) {
-        last          = lasts[w] > last ? lasts[w] : last;
-        first_nonzero = firsts[w] < first_nonzero ? firsts[w] : first_nonzero;
+    if constexpr (!ONE_WAVE) {
+        if ((tid & 63) == 0)
+            lasts[tid >> 6] = last, firsts[tid >> 6] = first_nonzero;
+        __syncthreads();
+        for (int w = 0; w < waves; ++w) {
+            last          = lasts[w] > last ? lasts[w] : last;
+            first_nonzero = firsts[w] < first_nonzero ? firsts[w] : first_nonzero;
+        }
     }
     // No key above the cut (a row of -inf or NaN only): the reference still runs softmax(scores + mask) over all S
     // keys, so every key stays in, with its bias.  A row that masks every key with the same finite value keeps all
@@ -1465,7 +1473,19 @@ template <bool VT> int launch_attention(hipStream_t s, int dtype, AttnParams p, 
 
 }  // namespace
 
-static dim3 mask_threads(int S) { return dim3(S >= kMaskThreads ? kMaskThreads : S <= 64 ? 64 : (S + 63) / 64 * 64); }
+template <int DT, typename SRC>
+static void launch_mask(hipStream_t s, const SRC *mask, long src_stride, const MaskSteps &steps, const void *constants, void *made,
+                        float *mask_f32, int32_t *kv_len, int B, int S, float threshold, int flag_zero_rows) {
+    typedef typename Elem<DT>::type T;
+#define TR_MASK(ONE_WAVE)                                                                                             \
+    hipLaunchKernelGGL((mask_to_kv_len_kernel<DT, SRC, ONE_WAVE>), dim3(B), dim3(ONE_WAVE ? 64 : kMaskThreads), 0, s, mask, src_stride, \
+                       steps, (const T *)constants, (T *)made, mask_f32, kv_len, S, threshold, flag_zero_rows)
+    if (S <= kMaskThreads)
+        TR_MASK(true);
+    else
+        TR_MASK(false);
+#undef TR_MASK
+}
 
 extern "C" {
 
@@ -1598,8 +1618,7 @@ int tnn_rocm_mask_to_kv_len(void *stream, const float *mask, int32_t *kv_len, in
     if (B == 0)
         return 0;
     TR_REQUIRE(mask && kv_len, TNN_ROCM_EINVAL, "mask_to_kv_len: null pointer");
-    hipLaunchKernelGGL((mask_to_kv_len_kernel<TNN_ROCM_F32, float>), dim3(B), mask_threads(S), 0, (hipStream_t)stream, mask, (long)S,
-                       MaskSteps{}, (const float *)nullptr, (float *)nullptr, (float *)nullptr, kv_len, S, threshold, 0);
+    launch_mask<TNN_ROCM_F32>((hipStream_t)stream, mask, (long)S, MaskSteps{}, nullptr, nullptr, nullptr, kv_len, B, S, threshold, 0);
     TR_CHECK_LAUNCH();
     return 0;
 }
@@ -1621,16 +1640,16 @@ int tnn_rocm_mask_prepare_strided(void *stream, int dtype, const void *mask, lon
     hipStream_t s = (hipStream_t)stream;
     switch (dtype) {
         case TNN_ROCM_F32:
-            hipLaunchKernelGGL((mask_to_kv_len_kernel<TNN_ROCM_F32, float>), dim3(B), mask_threads(S), 0, s, (const float *)mask,
-                               mask_batch_stride, MaskSteps{}, (const float *)nullptr, (float *)nullptr, mask_f32, kv_len, S, threshold, 1);
+            launch_mask<TNN_ROCM_F32>(s, (const float *)mask, mask_batch_stride, MaskSteps{}, nullptr, nullptr, mask_f32, kv_len, B, S,
+                                      threshold, 1);
             break;
         case TNN_ROCM_F16:
-            hipLaunchKernelGGL((mask_to_kv_len_kernel<TNN_ROCM_F16, half_t>), dim3(B), mask_threads(S), 0, s, (const half_t *)mask,
-                               mask_batch_stride, MaskSteps{}, (const half_t *)nullptr, (half_t *)nullptr, mask_f32, kv_len, S, threshold, 1);
+            launch_mask<TNN_ROCM_F16>(s, (const half_t *)mask, mask_batch_stride, MaskSteps{}, nullptr, nullptr, mask_f32, kv_len, B, S,
+                                      threshold, 1);
             break;
         case TNN_ROCM_BF16:
-            hipLaunchKernelGGL((mask_to_kv_len_kernel<TNN_ROCM_BF16, bf16_bits>), dim3(B), mask_threads(S), 0, s, (const bf16_bits *)mask,
-                               mask_batch_stride, MaskSteps{}, (const bf16_bits *)nullptr, (bf16_bits *)nullptr, mask_f32, kv_len, S, threshold, 1);
+            launch_mask<TNN_ROCM_BF16>(s, (const bf16_bits *)mask, mask_batch_stride, MaskSteps{}, nullptr, nullptr, mask_f32, kv_len, B, S,
+                                       threshold, 1);
             break;
         default:
             TR_REQUIRE(false, TNN_ROCM_EDTYPE, "mask_prepare: dtype %d unsupported", dtype);
@@ -1655,9 +1674,7 @@ int tnn_rocm_mask_prepare_i32(void *stream, int dtype, const int32_t *ints, int 
         return 0;
     TR_REQUIRE(ints && mask && kv_len && (mask_f32 || dtype == TNN_ROCM_F32), TNN_ROCM_EINVAL, "mask_prepare_i32: null pointer");
     hipStream_t s = (hipStream_t)stream;
-#define TR_MASK(DT)                                                                                                     \
-    hipLaunchKernelGGL((mask_to_kv_len_kernel<DT, int32_t>), dim3(B), mask_threads(S), 0, s, ints, (long)S, steps,             \
-                       (const Elem<DT>::type *)constants, (Elem<DT>::type *)mask, mask_f32, kv_len, S, threshold, 1)
+#define TR_MASK(DT) launch_mask<DT>(s, ints, (long)S, steps, constants, mask, mask_f32, kv_len, B, S, threshold, 1)
     switch (dtype) {
         case TNN_ROCM_F32: TR_MASK(TNN_ROCM_F32); break;
         case TNN_ROCM_F16: TR_MASK(TNN_ROCM_F16); break;
