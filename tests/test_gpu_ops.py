@@ -1123,10 +1123,11 @@ def test_attention_fp32(B, h, S, masked):
     assert got.dtype == np.float32 and rel_err(got, ref) <= 3e-6
 
 
-@pytest.mark.parametrize("B,h,S", [(1, 65, 256), (3, 29, 200), (5, 13, 264), (7, 12, 384), (2, 43, 512)])
+@pytest.mark.parametrize("B,h,S", [(1, 65, 256), (3, 29, 200), (5, 13, 264), (7, 12, 384), (2, 43, 512), (7, 32, 256), (29, 8, 256)])
 def test_attention_order_of_the_pairs(B, h, S):
-    """Launches around and above one workgroup a CU, where the kernels take the (sequence, head) pairs head by head: every sequence
-    is the checker's in fp16 (V transposed), and in fp32 has the bits that it has alone"""
+    """Launches around one workgroup a CU and around three and a half, between which the fp16 kernel takes the (sequence, head) pairs
+    head by head (the fp32 kernel always does): every sequence is the checker's in fp16 (V transposed), and in fp32 has the bits
+    that it has alone"""
     say("attention order of pairs B=%d h=%d S=%d" % (B, h, S))
     rng = np.random.default_rng(B * S + h)
     o, H = ops(), h * 64

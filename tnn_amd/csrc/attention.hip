@@ -1402,15 +1402,20 @@ template <int DT, bool VT> __global__ void __launch_bounds__(256, 2) attention_s
 constexpr long kShortBlocksVT = 256, kShortBlocksRows = 1200;
 
 // Every XCD takes a contiguous run of (sequence, head) pairs.  Sequence by sequence, each gets the heads of one or few sequences,
-// and the one with the longest of them ends last.  Where the workgroups are on the chip at once (two waves each, below 1024 of
-// them, three a CU) and more than one a CU, the pairs go head by head instead, so that every XCD has heads of nearly all
-// sequences; us, 12 heads, lengths S / S/2 .. S / 16 .. S:
-//   B4 S384 10.0 10.9 11.1 -> 10.1 10.2 10.6   B8 S384 11.6 12.6 11.3 -> 11.7 11.8 10.5   B16 S256 10.2 11.2 11.1 -> 10.3 11.0 11.1
-// Larger launches run in several rounds, and there it is no better (B16 S512 21.9 21.8 18.7, head by head 22.2 21.8 19.2; B32 S512
-// 42.7 39.8 32.0, 43.7 39.5 33.1).  The longest sequence first, found from the lengths in the kernel, ends earlier still (B8 S384
-// 16 .. S 9.9, B16 S512 17.3), but every workgroup then waits for the lengths before its first address: +0.3 .. +1.0 us where
-// they are equal.
-constexpr unsigned kCusOfTheChip = 256;
+// and the one with the longest of them ends last.  In launches of the two-wave kernel (three workgroups a CU at once) of one to
+// three and a half workgroups a CU the pairs go head by head instead, so that every XCD has heads of nearly all sequences; us,
+// 12 heads, means of eight draws of lengths S/2 .. S / 16 .. S:
+//    768 workgroups  8 x 512 13.7 13.3 -> 13.4 12.7    16 x 256  9.8  9.7 ->  9.9  9.5
+//    792            11 x 384 17.0 15.8 -> 15.8 13.1    33 x 128 11.3 10.7 -> 11.3 10.2
+//    864            12 x 384 17.2 16.6 -> 16.4 15.1    18 x 256 14.1 13.6 -> 14.0 12.6    36 x 128 11.5 11.5 -> 11.7 11.2
+//    912            19 x 256 14.5 14.1 -> 14.7 13.7
+//    960            20 x 256 14.7 13.5 -> 15.4 14.0    10 x 512 20.5 18.6 -> 20.9 17.2
+//   1008            14 x 384 18.6 17.1 -> 19.3 16.1    21 x 256 15.3 14.7 -> 16.0 14.9    42 x 128 12.3 12.1 -> 12.5 12.5
+// Nor is it better in larger launches, which run in several rounds (B16 S512 21.9 21.8 18.7, head by head 22.2 21.8 19.2; B32 S512
+// 42.7 39.8 32.0, 43.7 39.5 33.1: lengths S / S/2 .. S / 16 .. S).  The longest sequence first, found from the lengths in the kernel,
+// ends earlier still (B8 S384 16 .. S 9.9, B16 S512 17.3), but every workgroup then waits for the lengths before its first address:
+// +0.3 .. +1.0 us where they are equal.
+constexpr unsigned kPairsByHeadFrom = kNumCU, kPairsByHeadTo = kNumCU * 7 / 2;
 
 template <bool VT> int launch_attention(hipStream_t s, int dtype, AttnParams p, int B, int heads, int S, bool by_size = true) {
     const long blocks128 = (long)((S + 127) / 128) * heads * B, blocks32 = (long)((S + 31) / 32) * heads * B;
@@ -1449,7 +1454,7 @@ template <bool VT> int launch_attention(hipStream_t s, int dtype, AttnParams p, 
             TR_LAUNCH_DMA(4, 256);
         } else {
             const dim3 grid    = blocks_of(64);
-            p.sequences_inside = p.kv_len && grid.x > kCusOfTheChip;
+            p.sequences_inside = p.kv_len && grid.x > kPairsByHeadFrom && grid.x <= kPairsByHeadTo;
             TR_LAUNCH_DMA(2, 128);
         }
 #undef TR_LAUNCH_DMA

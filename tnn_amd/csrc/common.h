@@ -258,6 +258,8 @@ __device__ __forceinline__ double reciprocal_root(double v) {
     return e > 0.0 && e < (double)INFINITY ? root : e;
 }
 
+constexpr int kNumCU = 256;  // compute units of the chip, in eight XCDs
+
 // A kernel's arguments lie in cache lines that nothing on the chip has read yet.  The compiler loads them as it comes to them,
 // one miss after the other (1700 clocks to a GEMM's first slab request, with five lines); touched together they cost one.
 template <size_t BYTES> __device__ __forceinline__ void touch_kernel_args() {

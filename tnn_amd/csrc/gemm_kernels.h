@@ -2297,7 +2297,6 @@ int launch_tiled(hipStream_t s, const void *A, const void *B, int M, int N, int 
 // Eight-wave workgroups put two waves on every SIMD inside one tile: while one waits for its LDS fragments the
 // other issues MFMAs, and a larger tile per CU moves fewer bytes through LDS and L2 per flop.  Four-wave tiles
 // larger than 128 x 128 (one wave per SIMD) were measured and never won with compiler-scheduled code.
-constexpr int kNumCU = 256;
 
 // What a launch takes on this chip with each tile shape.  The busiest CU works through n = ceil(tiles / 256) tiles, up to
 // `slots` of them side by side (what its LDS and registers hold): full sets of `slots`, then the rest.  A set costs its

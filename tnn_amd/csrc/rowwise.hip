@@ -301,7 +301,7 @@ int launch_layernorm(hipStream_t s, const void *x, const void *res, const float 
                        StoreThrough())
 #define TR_LN(LPR, NV, HALF, F32)                                                                                     \
     do {                                                                                                              \
-        constexpr int resident = 256 * kRowsPerBlk * (kWave / LPR) * (DT == TNN_ROCM_F32 ? F32 : HALF);               \
+        constexpr int resident = kNumCU * kRowsPerBlk * (kWave / LPR) * (DT == TNN_ROCM_F32 ? F32 : HALF);            \
         if (rows <= resident)                                                                                         \
             TR_LN_LAUNCH(LPR, NV, true);                                                                              \
         else                                                                                                          \
