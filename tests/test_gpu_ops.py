@@ -755,6 +755,26 @@ def test_gemm_fragments_read_ahead(code, slabs):
         assert np.abs(got - exact).max() <= (2.0 ** -11 if td is torch.float16 else 2.0 ** -8) * np.abs(exact).max() + 1e-4 * np.sqrt(K)
 
 
+@pytest.mark.parametrize("M,N,K,gelu,most", [(24576, 1536, 384, True, 1.1), (12288, 1024, 256, True, 1.07), (4096, 4096, 1024, False, 0.93)])
+def test_gemm_shape_picked_for_large_products(M, N, K, gelu, most):
+    """256 x 256 tiles where they are the faster ones: with GELU and a short K they took 1.21, 1.12 times what 128 x 128 tiles take, and
+    0.83 of it where the chip is full and the epilogue light."""
+    from tnn_amd import capi
+    say("gemm bf16 %d x %d x %d, gelu %d, time of the shape picked" % (M, N, K, gelu))
+    lib, o = capi.load(), ops()
+    a, w = torch.randn(M, K, device="cuda").bfloat16(), torch.randn(N, K, device="cuda").bfloat16()
+    bias, out = torch.zeros(N, device="cuda"), torch.empty(M, N, device="cuda", dtype=torch.bfloat16)
+
+    def run(code):
+        lib.tnn_rocm_debug_set_gemm_config(code)
+        try:
+            o.gemm(a, w, True, bias=bias, gelu=gelu, out=out)
+        finally:
+            lib.tnn_rocm_debug_set_gemm_config(0)
+    picked, other = _device_us([lambda: run(0), lambda: run(2222221)])
+    assert picked <= most * other, (picked, other)
+
+
 @pytest.mark.parametrize("code", [6111141, 6211141, 6121141])
 @pytest.mark.parametrize("M,N,K", [(1, 8, 256), (17, 24, 256), (33, 776, 768), (130, 136, 3072)])
 def test_gemm_16x16_blocks(code, M, N, K):

@@ -23,6 +23,7 @@
 #define TNN_ROCM_CSRC_GEMM_KERNELS_H_
 
 #include <type_traits>
+#include <utility>
 
 #include "gemm_typed.h"
 #include "split_f32.h"
@@ -231,6 +232,14 @@ template <typename E> struct RowIn<E, typename std::enable_if<E::kRowIn>::type> 
 //                  where they are, or null.  A shape whose threads have one item each requests them before its first slab
 template <typename E, typename = void> struct AheadVecs : std::integral_constant<int, 0> {};
 template <typename E> struct AheadVecs<E, typename std::enable_if<(E::kAheadVecs > 0)>::type> : std::integral_constant<int, E::kAheadVecs> {};
+//   wide_us()      what the epilogue adds to every round of 256 x 256 tiles, in the cost model's microseconds: its 128 values a thread
+//                  stand behind the last product of a CU's only tile, and nothing covers them
+template <typename E, typename = void> struct WideEpilogue {
+    static float us(const E &) { return 0.f; }
+};
+template <typename E> struct WideEpilogue<E, std::void_t<decltype(std::declval<const E &>().wide_us())>> {
+    static float us(const E &e) { return e.wide_us(); }
+};
 template <typename E, typename = void> struct SumBlocks : std::integral_constant<int, 1> {};
 template <typename E> struct SumBlocks<E, typename std::enable_if<E::kTakesRowSums>::type> : std::integral_constant<int, E::kSumBlocks> {};  // tile columns of a producer a consumer can add up (768 columns of 32)
 
@@ -251,6 +260,7 @@ template <int DT> struct FloatEpilogue : StoreThrough {
     long ldc;
     long batch_stride_c;
     long batch_stride_r;
+    float wide_us() const { return (flags & TNN_ROCM_EPI_GELU) ? 1.75f : 0.f; }
     __device__ __forceinline__ void set_batch(int b) {
         C += (size_t)b * batch_stride_c;
         if (residual)
@@ -329,6 +339,7 @@ template <int DT> struct QkvSplitEpilogue : StoreThrough {
     T *vt;
     int H, S, heads;
     int vt_sh;  // 0: V^T keys in natural order; 1: bits 2 and 3 of the key index change places (see key_slot)
+    float wide_us() const { return 1.5f; }  // V^T
     __device__ __forceinline__ void set_batch(int) {}
     __device__ __forceinline__ float col_const(int n) const { return bias ? bias[n] : 0.f; }
     __device__ __forceinline__ void store(int m, int n, float acc, float bias_n) const {
@@ -449,6 +460,7 @@ template <int DT, int SUMS = 0> struct LnFloatEpilogue : StoreThrough {
     T *C;
     long ldc;
     LnFold ln;
+    float wide_us() const { return (flags & TNN_ROCM_EPI_GELU) ? 1.75f : 0.f; }
     __device__ __forceinline__ void set_batch(int) {}
     __device__ __forceinline__ float col_const(int) const { return 0.f; }
     __device__ __forceinline__ void store(int, int, float, float) const {}  // N % 8 == 0 is required at launch
@@ -520,6 +532,7 @@ template <int DT, int SUMS = 0> struct LnQkvSplitEpilogue : StoreThrough {
     int H, S, heads;
     int vt_sh;  // 0: V^T keys in natural order; 1: bits 2 and 3 of the key index change places (see key_slot)
     LnFold ln;
+    float wide_us() const { return 1.5f; }  // V^T
     __device__ __forceinline__ void set_batch(int) {}
     __device__ __forceinline__ float col_const(int) const { return 0.f; }
     __device__ __forceinline__ void store(int, int, float, float) const {}
@@ -574,6 +587,7 @@ template <int DT, bool SUMS = false> struct LnResidualEpilogue : StoreThrough {
     const float *gamma, *beta;  // [N]
     T *C;
     long ldc;
+    float wide_us() const { return (flags & TNN_ROCM_EPI_GELU) ? 1.75f : 0.f; }
     __device__ __forceinline__ void set_batch(int) {}
     __device__ __forceinline__ float col_const(int n) const { return (flags & TNN_ROCM_EPI_BIAS) ? bias[n] : 0.f; }
     __device__ __forceinline__ void store(int m, int n, float acc, float bias_n) const {
@@ -2329,12 +2343,15 @@ constexpr TileCost kTilesHalf[] = {
     {2222221, 128, 128, 2, 4.84f, 5.77f, {0.561f, 1.044f}},
     {3332221, 192, 192, 1, 10.15f, 13.25f, {0.767f}},
     {3331182, 96, 96, 1, 6.94f, 7.10f, {0.264f}},
-    {2244211, 256, 256, 1, 10.0f, 8.0f, {1.6f}},
+    {2244211, 256, 256, 1, 10.5f, 12.0f, {1.5f}},
 };
-// 256 x 256 tiles are for products that fill the chip with them: half the bytes a flop of 128 x 128 tiles.  Their row is set by
-// hand between the full and the half-empty rounds (a round of 192 tiles is 13 % shorter than one of 256, which a linear model
-// does not know).  us, 128 x 128 -> 256 x 256, GELU and folded LayerNorm: fp16 8192 x 4096 x 1024 97 -> 83, 4096 x 4096 x 1024 55
-// -> 46, 3072 x 4096 x 1024 43.4 -> 42.0; int8 8192 x 4096 x 1024 57.8 -> 52.4, 4096 x 4096 x 1024 28.4 -> 27.4.
+// 256 x 256 tiles are for products that fill the chip with them: half the bytes a flop of 128 x 128 tiles.  A linear model knows
+// neither that a round of 192 tiles is 13 % shorter than one of 256 nor what the epilogue leaves uncovered, so their row and the
+// epilogues' wide_us() are fitted to the comparison with the other shapes' picks: 1155 launches of 185 products (1024 to 24576 rows,
+// hidden sizes 256 to 4096).  With {10.0, 8.0, 1.6} for every epilogue 91 of the 839 that took 256 x 256 tiles were more than 3 %
+// slower for it, by up to 21 %; now 15 of 888, by up to 9 %.  us, 128 x 128 -> 256 x 256, folded LayerNorm and GELU: 8192 x 4096 x 1024
+// 89 -> 81, 4096 x 4096 x 1024 47 -> 42, 3072 x 4096 x 1024 37.3 -> 35.7 (with a bias only 34.8 -> 31.1); not picked 12288 x 3072 x 768
+// 82 -> 92, 4096 x 3072 x 768 29.6 -> 31.1, 8192 x 1536 x 384 21.1 -> 22.7.
 // Tiles of 16 x 16 blocks are for the products whose 32x32 tiles are too few for the chip: a CU's panels come through its L1 at
 // 64 bytes a clock at best, so 24 tiles of (32 + 32) rows of K=3072 take 4 us for that alone, and 96 of (16 + 16) rows half.
 // us a launch, best shape before -> now (fp32: 8 waves where K is long):
@@ -2390,7 +2407,8 @@ constexpr TileCost kTilesF32[] = {
 
 // row_stats: the shape takes the rows' statistics from its own A fragments, which 32 rows of 16 x 16 blocks pay for with twice the
 // sums a wave (M=32 N=2304 K=768: 4.8 us, with 16 x 32 tiles 4.5)
-template <int COUNT> inline int pick_tile_config(const TileCost (&shapes)[COUNT], long M, long N, size_t kbytes, bool row_stats) {
+template <int COUNT>
+inline int pick_tile_config(const TileCost (&shapes)[COUNT], long M, long N, size_t kbytes, bool row_stats, float wide_us) {
     int best        = 0;
     float best_cost = 0.f;
     const float slabs = (float)(kbytes / 128);
@@ -2400,7 +2418,8 @@ template <int COUNT> inline int pick_tile_config(const TileCost (&shapes)[COUNT]
         const long tiles = ((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn), n = (tiles + kNumCU - 1) / kNumCU;
         const long sets = n / t.slots, rest = n % t.slots;
         float cost = t.fixed + slabs * ((float)sets * t.slab[t.slots - 1] + (rest ? t.slab[rest - 1] : 0.f)) +
-                     t.round * (float)(sets + (rest ? 1 : 0) - 1) + (row_stats && t.code / 100000 == 62 ? 0.4f : 0.f);
+                     t.round * (float)(sets + (rest ? 1 : 0) - 1) + (row_stats && t.code / 100000 == 62 ? 0.4f : 0.f) +
+                     (t.bm == 256 ? wide_us * (float)n : 0.f);
         if (best == 0 || cost < best_cost)
             best = t.code, best_cost = cost;
     }
@@ -2420,11 +2439,11 @@ int launch_gemm_fast(hipStream_t s, const void *A, const void *B, int M, int N, 
         if (kbytes % 128 != 0 || wide)
             cfg = (((long)M + 127) / 128) * (((long)N + 127) / 128) > kNumCU ? 222210 : 112210;
         else if (DT == TNN_ROCM_F32)
-            cfg = pick_tile_config(kTilesF32, M, N, kbytes, Epi::kRowStats);
+            cfg = pick_tile_config(kTilesF32, M, N, kbytes, Epi::kRowStats, WideEpilogue<Epi>::us(epi));
         else if (DT == TNN_ROCM_I8)
-            cfg = pick_tile_config(kTilesI8, M, N, kbytes, Epi::kRowStats);
+            cfg = pick_tile_config(kTilesI8, M, N, kbytes, Epi::kRowStats, WideEpilogue<Epi>::us(epi));
         else
-            cfg = pick_tile_config(kTilesHalf, M, N, kbytes, Epi::kRowStats);
+            cfg = pick_tile_config(kTilesHalf, M, N, kbytes, Epi::kRowStats, WideEpilogue<Epi>::us(epi));
     }
     switch (cfg) {  // a code of 128-byte or larger slabs without its stage digit
         case 112211: cfg = 2112211; break;
