@@ -97,7 +97,7 @@ def test_gelu_of_fp32_products():
     eye = np.eye(K, dtype=np.float32)
     o = ops()
     got = host(o.gemm(dev(x), dev(eye), True, gelu=True))
-    for code in (-1, 9111141, 9111181, 3222121, 2222221):
+    for code in (-1, 9111141, 9111181, 2222121, 2332121, 2222221):
         lib.tnn_rocm_debug_set_gemm_config(code)
         try:
             assert np.array_equal(host(o.gemm(dev(x), dev(eye), True, gelu=True)), got), code
@@ -690,7 +690,7 @@ def test_gemm_small_product_shapes(code, M, N, K):
         lib.tnn_rocm_debug_set_gemm_config(0)
 
 
-@pytest.mark.parametrize("code", [9111141, 9121141, 9111181, 9221141, 9321140, 3231142, 2331142, 3222121, 2222221])
+@pytest.mark.parametrize("code", [9111141, 9121141, 9111181, 9221141, 2321142, 2231142, 2331142, 2222121, 2222221, 2332121])
 @pytest.mark.parametrize("M,N,K", [(1, 8, 128), (97, 104, 192), (130, 136, 3072)])
 def test_gemm_fp32_split_shapes(code, M, N, K):
     """fp32 products on three bf16 planes, every tile shape: no further from float64 than an fp32 sum is, over magnitudes
@@ -719,12 +719,13 @@ def test_gemm_fp32_split_shapes(code, M, N, K):
     assert (np.abs(got[fine] - exact[fine]) <= 2.0 ** -24 * 4 * np.sqrt(K) * size[fine]).all()
 
 
-@pytest.mark.parametrize("code", [2222221, 3212221, 3332221, 2244211])
+@pytest.mark.parametrize("code", [2222221, 3212221, 3332221, 2244211, 3112221])
 @pytest.mark.parametrize("slabs", [1, 2, 3, 4, 5, 8])
 def test_gemm_fragments_read_ahead(code, slabs):
-    """Shapes that read a slab's first fragments under the slab before: loops of every length (fewer slabs than stages, the last
-    ones whose successors are not requested any more), whole tiles and remainders, every epilogue; handed-over row sums against
-    sums in double."""
+    """Shapes that read a slab's first fragments under the slab before (192 x 192 and 256 x 256 tiles) and, by the same measure, three that
+    read them where they are used: loops of every length (fewer slabs than stages, the last ones whose successors are not requested
+    any more), whole tiles and remainders, every epilogue; handed-over row sums against sums in double, at numbers of blocks that
+    the lanes of a row (two, four or eight of them) share evenly or not, or that are fewer than these, every block's sums others."""
     from tnn_amd import capi
     lib = capi.load()
     K = 64 * slabs
@@ -740,11 +741,9 @@ def test_gemm_fragments_read_ahead(code, slabs):
         try:
             got = host(o.gemm(a.cuda(), w.cuda(), True).float()).astype(np.float64)
             if slabs % 2 == 0:
-                for blocks in (2, 12, 24):  # few enough for the shape to ask for them late, and more
-                    part = torch.zeros(blocks, M, 2)
-                    part[blocks - 1, :, 0], part[blocks - 1, :, 1] = a.double().sum(1), (a.double() ** 2).sum(1)
+                for blocks in (1, 2, 5, 11, 12, 13, 23, 24):  # few enough for the shape to ask for them late, and more
                     cs, zero = w.double().sum(1).float(), torch.zeros(N)
-                    fed = o.gemm_ln(a.cuda(), w.cuda(), zero.cuda(), cs.cuda(), 1e-5, row_sums=(part.cuda(), blocks))
+                    fed = o.gemm_ln(a.cuda(), w.cuda(), zero.cuda(), cs.cuda(), 1e-5, row_sums=(_row_sums(a, blocks), blocks))
                     norm = ((a.double() - a.double().mean(1, keepdim=True)) / (a.double().var(1, unbiased=False, keepdim=True) + 1e-5).sqrt())
                     ref = host(norm @ w.double().T)
                     assert rel_err(host(fed.float()), ref) <= (FP16_TOL if td is torch.float16 else 2e-2), blocks
@@ -787,11 +786,39 @@ def test_gemm_16x16_blocks(code, M, N, K):
 def test_gemm_fp32_16x16_blocks(code, M, N, K):
     """... and fp32 on them: precision, values next to the ends of the range, infinities and NaN, which are formed again"""
     test_gemm_fp32_split_shapes(code, M, N, K)
-    if K == 192:
+    if (M, K) == (97, 192):
         for ea, ew in ((-140, 60), (0, -118), (110, -60), (60, 25)):
             test_gemm_fp32_split_small_and_large(code, ea, ew)
         for slabs in (1, 2, 3, 4, 5, 6, 9, 16, 17, 25):
             test_gemm_fp32_split_slab_counts(code, slabs)
+
+
+@pytest.mark.parametrize("code", [6111181, 6211181, 9111141, 9121141, 9111181, 9221141, 2321142, 2231142, 2331142, 2222121, 2222221, 2332121])
+def test_gemm_fp32_split_epilogues(code):
+    """Bias, GELU and residual of every fp32 tile shape, whole tiles and a last one of one row and eight columns, against float64: the
+    sum's K roundings of half a unit at most, as in test_gemm_fp32_split_shapes, one more for each of the epilogue's steps, and the
+    GELU's slope (1.13 at most) and its own ulp"""
+    from tnn_amd import capi
+    lib, o = capi.load(), ops()
+    say("gemm fp32 epilogues, code %d" % code)
+    M, N, K = 193, 200, 512
+    rng = np.random.default_rng(code % 1000)
+    a, w, res = (rng.standard_normal(n).astype(np.float32) for n in ((M, K), (N, K), (M, N)))
+    w *= np.float32(0.1)
+    bias = rng.standard_normal(N).astype(np.float32)
+    sums = a.astype(np.float64) @ w.astype(np.float64).T + bias
+    size = np.abs(a.astype(np.float64)) @ np.abs(w.astype(np.float64)).T + np.abs(bias)
+    gelu = 0.5 * sums * torch.special.erfc(torch.from_numpy(-sums / np.sqrt(2.0))).numpy()
+    u = 2.0 ** -24
+    lib.tnn_rocm_debug_set_gemm_config(code)
+    try:
+        for gl, r in ((False, None), (True, None), (False, res), (True, res)):
+            got = host(o.gemm(dev(a), dev(w), True, bias=dev(bias), gelu=gl, residual=None if r is None else dev(r))).astype(np.float64)
+            want = (gelu if gl else sums) + (0 if r is None else r)
+            allowed = 1.13 * u * (4 * np.sqrt(K) + 1) * size + 2 * u * np.abs(gelu) * gl + u * np.abs(want)
+            assert (np.abs(got - want) <= allowed).all(), (gl, r is None)
+    finally:
+        lib.tnn_rocm_debug_set_gemm_config(0)
 
 
 @pytest.mark.parametrize("code", [9111141, 9111181, 9221141, 2321142, 2231142, 2331142, 2222121, 2222221, 2332121])
@@ -816,7 +843,7 @@ def test_gemm_fp32_split_slab_counts(code, slabs):
     assert (np.abs(got - exact) <= 2.0 ** -24 * 4 * np.sqrt(K) * size).all()
 
 
-@pytest.mark.parametrize("code", [9111141, 9121141, 9111181, 9221141, 9321140, 3231142, 2331142, 3222121, 2222221])
+@pytest.mark.parametrize("code", [9111141, 9121141, 9111181, 9221141, 2321142, 2231142, 2331142, 2222121, 2222221, 2332121])
 @pytest.mark.parametrize("ea,ew", [(-118, 0), (-126, 30), (-140, 60), (0, -118), (-100, -20), (110, -60), (60, 25)])
 def test_gemm_fp32_split_small_and_large(code, ea, ew):
     """Operands at the ends of the fp32 range (values below the normal ones among them) keep their 24 bits through the three
@@ -840,7 +867,7 @@ def test_gemm_fp32_split_small_and_large(code, ea, ew):
     assert (np.abs(got - exact) <= 2.0 ** -24 * 4 * size + 2.0 ** -149).all()
 
 
-@pytest.mark.parametrize("code", [0, 9111181, 9321140, 2331142, 2222221])
+@pytest.mark.parametrize("code", [0, 9111181, 2321142, 2331142, 2222221, 2332121])
 def test_gemm_fp32_not_finite_costs_a_few_launches(code):
     """An overflow upstream makes whole rows, or all, of an activation NaN: the product says so, and does not take orders of
     magnitude longer for it (three to five times as long; the bound leaves room for a busy device)."""
@@ -1869,10 +1896,11 @@ def test_folding_gemm_fed_row_sums_against_own_statistics(blocks, offset_rows):
 
 
 def _row_sums(t, blocks):
-    """the sums that a producer hands over, made on the host: [MAX_ROW_SUM_BLOCKS, M, 2] {sum, sum of squares} per block of columns"""
-    per = t.double().reshape(t.shape[0], blocks, -1)
-    sums = torch.zeros(ops().MAX_ROW_SUM_BLOCKS, t.shape[0], 2)
-    sums[:blocks, :, 0], sums[:blocks, :, 1] = per.sum(2).T.float(), (per ** 2).sum(2).T.float()
+    """the sums that a producer hands over, made on the host: [MAX_ROW_SUM_BLOCKS, M, 2] {sum, sum of squares} per block of columns;
+    what lies behind them is not to be added"""
+    sums = torch.full((ops().MAX_ROW_SUM_BLOCKS, t.shape[0], 2), 1e6)
+    for i, part in enumerate(t.double().tensor_split(blocks, 1)):
+        sums[i, :, 0], sums[i, :, 1] = part.sum(1), (part ** 2).sum(1)
     return sums.cuda()
 
 

@@ -125,7 +125,6 @@ template <int TM, int TN, int STEPS> struct SplitSlab {
     static constexpr int OPS    = TM + TN;
     static constexpr int MFMAS  = STEPS * kSplitProducts * TM * TN;
     static constexpr int UNITS  = STEPS * OPS * 20;  // of a conversion: per operand and step five levels of four pairs of values
-    enum { kEarly, kSpread, kAfterReads };  // kAfterReads: the loads go where the reads come from
     Split3 op[STEPS][OPS];                           // A's operands, then B's
     struct Reads {
         uint4 f[STEPS][OPS][2];
@@ -164,15 +163,15 @@ template <int TM, int TN, int STEPS> struct SplitSlab {
         }
     }
     // Multiplies this slab's planes while it makes the next one's, whose LDS reads are under way; load(k) requests the k-th of
-    // LOADS loads of the slab after (PLACE: when).
+    // LOADS loads of the slab after, as early as their place is free, one a slot: the next turn waits for them.
+    // AFTER_READS: they go where the reads come from.
     // One or two small pieces of that go behind every matrix instruction: a slot holds about seven vector instructions, and a
     // piece that is longer (a whole plane of four values took twelve) leaves the matrix pipe empty for the rest of it.
-    template <int LOADS, int PLACE, typename Acc, typename Load>
+    template <int LOADS, bool AFTER_READS, typename Acc, typename Load>
     __device__ __forceinline__ void turn(const Reads &rd, SplitSlab &next, Acc (&acc)[TM][TN], const SplitConst &sc, Load load) const {
         constexpr int LEAD = MFMAS >= 24 ? 4 : 2;  // the first matrix instructions alone: the LDS reads arrive meanwhile
-        // loads as early as their place is free, one a slot, where the next turn waits for them; else spread over the turn
-        constexpr int L0     = PLACE != kAfterReads ? 0 : LEAD;
-        constexpr int LSLOTS = PLACE != kSpread && LOADS > 0 && LOADS < MFMAS - L0 ? LOADS : MFMAS - L0;
+        constexpr int L0     = AFTER_READS ? LEAD : 0;
+        constexpr int LSLOTS = LOADS > 0 && LOADS < MFMAS - L0 ? LOADS : MFMAS - L0;
         float rest[STEPS][OPS][8];
 #pragma unroll
         for (int q = 0; q < MFMAS; ++q) {
@@ -198,7 +197,7 @@ template <int TM, int TN, int STEPS> struct SplitSlab {
                     unit(k, next, rest, sc);
             }
             if (LOADS > 0 && q >= L0 && q < L0 + LSLOTS) {
-                if (PLACE == kAfterReads && q == L0)
+                if (AFTER_READS && q == L0)
                     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
 #pragma unroll
                 for (int k = LOADS * (q - L0) / LSLOTS; k < LOADS * (q - L0 + 1) / LSLOTS; ++k)
@@ -1388,7 +1387,7 @@ __global__ void __launch_bounds__(CFG::NT)
                     read_fragments(rd.f);
                     const int here = stage;
                     stage = stage + 1 == NS ? 0 : stage + 1;
-                    now.template turn<decltype(loads)::value, Planes::kAfterReads>(
+                    now.template turn<decltype(loads)::value, true>(
                         rd, next, acc, split_const, [&](int k) __attribute__((always_inline)) { issue_one(k, kt + NS, here); });
                 };
                 typedef std::integral_constant<int, LPW> WithLoads;
@@ -1799,16 +1798,12 @@ __global__ void __launch_bounds__(CFG::NT)
         } else if constexpr (DT == TNN_ROCM_F32) {
             typedef SplitSlab<TM, TN, KSTEPS> Planes;
             Planes p, q;
-            static_assert(NS <= 3, "waits written for up to three stages");
+            static_assert(DT != TNN_ROCM_F32 || NS == 2, "one slab is requested while the one before is multiplied");
             // slab kt in LDS, and every wave done with slab kt - 1; its fragments
             auto fetch = [&](int kt, typename Planes::Reads &rd) __attribute__((always_inline)) {
                 // slab kt - 1 is in this wave's registers, see the barrier below
                 asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-                const int behind = nk - 1 - kt;
-                if (NS > 2 && behind >= 1)
-                    TR_WAIT_VMCNT(NS > 2 ? LPW : 0);
-                else
-                    TR_WAIT_VMCNT(0);
+                TR_WAIT_VMCNT(0);
                 __builtin_amdgcn_s_barrier();
                 asm volatile("" ::: "memory");
                 const unsigned char *sa = lds_dyn + stage * STAGE, *sb = sa + BM * SLAB;
@@ -1834,7 +1829,7 @@ __global__ void __launch_bounds__(CFG::NT)
                 fetch(kt, rd);
                 const int there = fill;
                 advance();
-                now.template turn<decltype(loads)::value, (NS > 2 ? Planes::kSpread : Planes::kEarly)>(
+                now.template turn<decltype(loads)::value, false>(
                     rd, next, acc, split_const, [&](int k) __attribute__((always_inline)) { issue_one(k, kt + NS - 1, there); });
             };
             typedef std::integral_constant<int, LPW> WithLoads;
@@ -2453,13 +2448,6 @@ int launch_gemm_fast(hipStream_t s, const void *A, const void *B, int M, int N, 
         case 331182: cfg = 3331182; break;
         default: break;
     }
-    if (DT == TNN_ROCM_F32)
-        switch (cfg) {  // three stages, or rings of the waves' own: two stages took their place
-            case 9321140: cfg = 2321142; break;
-            case 3231142: cfg = 2231142; break;
-            case 3222121: cfg = 2222121; break;
-            default: break;
-        }
     if (kbytes % (64u << (cfg % 10)) != 0) {
         set_error("gemm: K=%d is not a whole number of slabs for tuning configuration %d", K, cfg);
         return TNN_ROCM_ESHAPE;
