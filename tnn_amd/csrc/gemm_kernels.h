@@ -240,7 +240,7 @@ template <typename E> struct WideEpilogue<E, std::void_t<decltype(std::declval<c
     static float us(const E &e) { return e.wide_us(); }
 };
 template <typename E, typename = void> struct SumBlocks : std::integral_constant<int, 1> {};
-template <typename E> struct SumBlocks<E, typename std::enable_if<E::kTakesRowSums>::type> : std::integral_constant<int, E::kSumBlocks> {};  // tile columns of a producer a consumer can add up (768 columns of 32)
+template <typename E> struct SumBlocks<E, typename std::enable_if<E::kTakesRowSums>::type> : std::integral_constant<int, E::kSumBlocks> {};  // tile columns of a producer a consumer can add up (at most 24: 768 columns of 32, 384 of 16)
 
 
 // GELU of a product, in every kernel and at every column the same function of the sum
@@ -1295,7 +1295,7 @@ __global__ void __launch_bounds__(CFG::NT)
     };
 
     if constexpr (CFG::OWN) {
-        // Every wave streams its own part of K: both panels' rows of one 64-byte k-slab per stage, through a ring that
+        // Every wave streams its own part of K: both panels' rows of one k-slab of SLAB bytes per stage, through a ring that
         // only this wave fills and reads.  Row swizzle as in the shared pipeline below.
         static_assert(!TakesRowSums<Epi>::value, "own-ring shapes take the row statistics from their A fragments");
         constexpr int NS   = CFG::NSTAGE;
@@ -2313,10 +2313,12 @@ int launch_tiled(hipStream_t s, const void *A, const void *B, int M, int N, int 
 // nothing covers), and the launch `fixed`; microseconds.  The figures are a least-squares fit to some 800 launches (fp16 and
 // int8: M from 16 to 8192, the four projections of hidden sizes 768 and 1024 with their fused epilogues; fp32: M from 16 to
 // 3072), taken over twelve weight sets in turn so that weights come from the memory-side cache as they do inside a network:
-// python -m tnn_amd.bench_ops --tile-sweep measures them and fits the rows.  A single launch is 4 .. 10 % off its prediction,
-// so picks closer than that are as good as drawn; taken together the picks are 2.4 % (fp16), 1.9 % (int8), 5.2 % (fp32) behind
-// the best shape of each launch back to back, and 0.29, 0.37 and 0.45 us inside the network (bench_configs --config tiles;
-// profiles/gemm_tile_choice.txt).  The rules this replaced, made for M >= 1024, were 51 %, 34 % and 77 % behind over that range:
+// python -m tnn_amd.bench_ops --tile-sweep measures them and fits the rows.  A launch is 3 .. 20 % off its prediction on average,
+// by shape (the large ones most), so picks closer than that are as good as drawn.  Taken together the picks are 1.1 % (fp16), 1.0 %
+// (int8), 1.0 % (fp32) behind the best shape of each launch back to back, at worst 15 % (M=4096 N=768 K=3072, where 2112211 leads),
+// 11 % and 6 %, and 0.29, 0.37 and 0.45 us inside the network (bench_configs --config tiles; profiles/gemm_tile_choice.txt).  Not
+// as the sweep fits them: the 256 x 256 rows (below), the 192 x 192 row of the half table, which is of before its loop read ahead,
+// and in the int8 table what the comment above it says.  The rules this replaced, made for M >= 1024, were 51 %, 34 % and 77 % behind:
 //   M=  32 N= 768 K=3072 fp16  23.1 -> 7.3 us   (64x64 tiles: 12 CUs, one two-stage slab after another)
 //   M= 256 N= 768 K=3072 fp16  23.7 -> 7.2      M= 256 N=2304 K=768 fp16  8.7 -> 6.2
 //   M=1000 N= 768 K=3072 fp16  24.3 -> 12.4     M=1000 N= 768 K=768 fp16  8.7 -> 5.5
@@ -2346,7 +2348,10 @@ constexpr TileCost kTilesHalf[] = {
 // hidden sizes 256 to 4096).  With {10.0, 8.0, 1.6} for every epilogue 91 of the 839 that took 256 x 256 tiles were more than 3 %
 // slower for it, by up to 21 %; now 15 of 888, by up to 9 %.  us, 128 x 128 -> 256 x 256, folded LayerNorm and GELU: 8192 x 4096 x 1024
 // 89 -> 81, 4096 x 4096 x 1024 47 -> 42, 3072 x 4096 x 1024 37.3 -> 35.7 (with a bias only 34.8 -> 31.1); not picked 12288 x 3072 x 768
-// 82 -> 92, 4096 x 3072 x 768 29.6 -> 31.1, 8192 x 1536 x 384 21.1 -> 22.7.
+// 82 -> 92, 4096 x 3072 x 768 29.6 -> 31.1, 8192 x 1536 x 384 21.1 -> 22.7.  With twelve weight sets in turn, over 260 launches, the
+// picks that are slower cost 25 % together (187 % with the old row), the shape where it is left out and faster 88 % (99 %).  The int8
+// row is set by hand: of its picks three of 60 are slower, 24576 x 1920 x 640 into Q, K and V^T by 6 % and [16384, 1024] x 1024 and
+// 24576 x 1280 x 1280 with a residual by 3 %.
 // Tiles of 16 x 16 blocks are for the products whose 32x32 tiles are too few for the chip: a CU's panels come through its L1 at
 // 64 bytes a clock at best, so 24 tiles of (32 + 32) rows of K=3072 take 4 us for that alone, and 96 of (16 + 16) rows half.
 // us a launch, best shape before -> now (fp32: 8 waves where K is long):
@@ -2380,6 +2385,7 @@ constexpr TileCost kTilesI8[] = {
 // us, v_mfma_f32 kernels -> planes, a whole plane of four values behind a matrix instruction -> a pair of values:
 //   M=1536: N=768 K=768 27 -> 20.2 -> 17.3, N=3072 K=768 74 -> 61 -> 55, N=768 K=3072 83 -> 60 -> 51
 //   M=128: N=768 K=768 7.6 -> 7.1 -> 6.8, N=3072 K=768 15.2 -> 11.4 -> 10.7, N=768 K=3072 17.6 -> 16.2 -> 15.3
+// (the 16 x 16 blocks, which came after that, see above, not counted)
 // Error against float64 (2-norm over 2-norm; 300 x 760 x 768 / 129 x 264 x 3072): 1.5e-7 .. 3e-7 / 3e-7 .. 6e-7 by shape,
 // v_mfma_f32_32x32x2_f32: 5.0e-7 / 9.9e-7.
 constexpr TileCost kTilesF32[] = {
@@ -2401,7 +2407,7 @@ constexpr TileCost kTilesF32[] = {
 };
 
 // row_stats: the shape takes the rows' statistics from its own A fragments, which 32 rows of 16 x 16 blocks pay for with twice the
-// sums a wave (M=32 N=2304 K=768: 4.8 us, with 16 x 32 tiles 4.5)
+// sums a wave (32 rows, hidden sizes 768 and 1024: QKV 4.7 and 5.0 us, FFN1 4.9 and 5.3; with 16 x 32 tiles 4.4, 4.7, 4.6 and 4.9)
 template <int COUNT>
 inline int pick_tile_config(const TileCost (&shapes)[COUNT], long M, long N, size_t kbytes, bool row_stats, float wide_us) {
     int best        = 0;
@@ -2689,8 +2695,8 @@ int GemmTyped<DT>::residual_ln(hipStream_t s, const void *x, const void *w, cons
                                const float *row_stats, const float *gamma, const float *beta, int M, int N, int K, int flags,
                                float *row_sums, int *row_sum_blocks) {
     // With the row sums first.  A tile shape whose tile columns are more than a reader adds up (and the caller's buffer of
-    // kMaxRowSumBlocks * M pairs holds: 32 columns wide, from N = 769 on), or that leaves no LDS for the sums, declines in
-    // launch_tiled; the plain form runs then and reports zero blocks.
+    // kMaxRowSumBlocks * M pairs holds: 16 columns wide from N = 385 on, 32 columns wide from N = 769 on), or that leaves no LDS for
+    // the sums, declines in launch_tiled; the plain form runs then and reports zero blocks.
     if (row_sums && N <= 64 * kMaxRowSumBlocks) {
         const int rc = launch_residual_ln<DT, true>(s, x, w, bias, C, t, row_stats, gamma, beta, M, N, K, flags, row_sums);
         if (rc == 0)
