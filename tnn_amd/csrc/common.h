@@ -7,6 +7,7 @@
 #include <stdio.h>
 
 #include <atomic>
+#include <type_traits>
 
 #include "tnn_rocm.h"
 
@@ -247,6 +248,19 @@ template <int O> __device__ __forceinline__ double add_lane_xor(double v) {
     }
 }
 
+// the sum over N = 2, 4 or 8 neighbouring lanes, in every one of them
+template <int N> __device__ __forceinline__ float add_neighbours(float v) {
+    auto add = [](float x, auto ctrl) {
+        return x + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), decltype(ctrl)::value, 0xf, 0xf, false));
+    };
+    v = add(v, std::integral_constant<int, 0xB1>());  // quad_perm: lane ^ 1
+    if constexpr (N >= 4)
+        v = add(v, std::integral_constant<int, 0x4E>());  // quad_perm: lane ^ 2
+    if constexpr (N >= 8)
+        v = add(v, std::integral_constant<int, 0x141>());  // row_half_mirror: the other four of eight
+    return v;
+}
+
 // 1 / sqrt(v), of zero, infinities and NaN too: the instruction's estimate (2^-26) and two Newton steps, the second with the exact
 // rest of v r, so that the result is the rounded root nearly everywhere (over 4 million values from 1e-12 to 1e8 0.5005 ulp at most;
 // 1.0 / sqrt(v) 1.48, one step 19.9) in nine double instructions.
@@ -262,14 +276,18 @@ constexpr int kNumCU = 256;  // compute units of the chip, in eight XCDs
 
 // A kernel's arguments lie in cache lines that nothing on the chip has read yet.  The compiler loads them as it comes to them,
 // one miss after the other (1700 clocks to a GEMM's first slab request, with five lines); touched together they cost one.
-template <size_t BYTES> __device__ __forceinline__ void touch_kernel_args() {
+// request_kernel_args only asks for them: the wait is where the caller uses the result.
+template <size_t BYTES> __device__ __forceinline__ uint32_t request_kernel_args() {
     typedef const __attribute__((address_space(4))) uint32_t *KernArg;
     const KernArg args = (KernArg)__builtin_amdgcn_kernarg_segment_ptr();
     uint32_t touched   = 0;
 #pragma unroll
     for (int w = 0; w < (int)(BYTES / 4); w += 16)
         touched |= args[w];
-    asm volatile("" ::"s"(touched));
+    return touched;
+}
+template <size_t BYTES> __device__ __forceinline__ void touch_kernel_args() {
+    asm volatile("" ::"s"(request_kernel_args<BYTES>()));
 }
 
 // Division by a number the host knows, as a product: three scalar instructions where the compiler's sequence for an unknown

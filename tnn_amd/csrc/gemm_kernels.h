@@ -1102,8 +1102,10 @@ template <int TM_, int TN_, int WGM_, int WGN_, int WGK_, int SLAB_, int NSTAGE_
     static constexpr size_t sums_offset = (slab_bytes >= stage_bytes + sums_bytes) ? stage_bytes : lds_bytes;
     // ... unless there is no such part and a row of a wave's columns lies in eight neighbouring lanes: the lanes then add up
     // the sums of each wave's columns among themselves (128 x 128: 16 KB of LDS would cost the CU's second workgroup)
-    static constexpr bool sums_by_lanes = TN_ == 2 && !(slab_bytes >= stage_bytes + sums_bytes);
-    static constexpr int sum_cols       = sums_by_lanes ? 32 * TN_ : BN;  // columns behind one pair of row sums
+    // or where all columns are one wave's anyway (32 x 32 tiles with rings of their own, 256 x 768 x 768: 4.60 -> 4.40 us against
+    // sums through LDS, a barrier and a loop over them)
+    static constexpr bool sums_by_lanes = OWN_ || (TN_ == 2 && !(slab_bytes >= stage_bytes + sums_bytes));
+    static constexpr int sum_cols       = sums_by_lanes ? BLK_ * TN_ : BN;  // columns behind one pair of row sums
     static constexpr int NW = WGM * WGN * WGK, NT = 64 * NW;  // waves and threads per workgroup
     static_assert(NW == 4 || NW == 8, "four or eight waves per workgroup");
     static_assert(OWN_ || ((BM * (SLAB / 16)) % NT == 0 && (BN * (SLAB / 16)) % NT == 0), "slab must divide over the workgroup");
@@ -1136,9 +1138,20 @@ template <typename CFG, typename Epi> struct EpiLds {
 // 15:14, expcnt 6:4 and lgkmcnt 11:8 left at their maxima)
 #define TR_WAIT_VMCNT(n) __builtin_amdgcn_s_waitcnt((((n)&0xF) | ((((n) >> 4) & 3) << 14) | (0x7 << 4) | (0xF << 8)))
 
+// Divisors of the tile order: tiles of a group, tile rows of a group, tile rows of the last, smaller group; and the tile rows of a
+// group.  With the panels and the sizes in front of them they are 13 words, which is what the dispatcher has registers for
+// (-amdgpu-kernarg-preload-count): a workgroup requests its first slab without a look at the argument memory, which
+// nothing on the chip has read yet.  us a launch, all arguments loaded -> these in registers, fp16, twelve weight sets in turn:
+//   32 x 768 x 3072 5.41 -> 5.13, 32 x 2304 x 768 4.84 -> 4.65, 985 x 2304 x 768 10.0 -> 9.7
 struct TileOrder {
-    int group_m;
-    FixedDivisor group, rows, last_rows;  // tiles of a group; tile rows of a group; tile rows of the last, smaller group
+    uint32_t group, rows, last_rows;  // FixedDivisor::magic
+    uint32_t packed;                  // their shifts, six bits each, and the tile rows of a group from bit 18 on
+    static constexpr int kMaxRows = (1 << 14) - 1;
+    static TileOrder of(int tiles_m, int tiles_n, int group_m) {
+        const FixedDivisor g = FixedDivisor::of((uint32_t)group_m * (uint32_t)tiles_n), r = FixedDivisor::of((uint32_t)group_m),
+                           l = FixedDivisor::of((uint32_t)(tiles_m % group_m));
+        return {g.magic, r.magic, l.magic, g.shift | r.shift << 6 | l.shift << 12 | (uint32_t)group_m << 18};
+    }
 };
 
 // An infinity, a NaN or a finite value from 2^104 on has no planes (split_f32.h), and turns every sum it enters into something
@@ -1170,8 +1183,8 @@ __device__ __forceinline__ void multiply_again(const float *pa, const float *pb,
 template <int DT, typename CFG, typename Epi>
 __global__ void __launch_bounds__(CFG::NT)
     gemm_nk_tiled_kernel(const typename GemmTraits<DT>::elem *__restrict__ A,
-                         const typename GemmTraits<DT>::elem *__restrict__ B, int M, int N, int K, long lda, long ldb,
-                         int tiles_m, int tiles_n, TileOrder order, Epi epi) {
+                         const typename GemmTraits<DT>::elem *__restrict__ B, int M, int N, int K, int lda, int ldb,
+                         uint32_t group_magic, uint32_t rows_magic, uint32_t last_magic, uint32_t order_packed, Epi epi) {
     typedef typename GemmTraits<DT>::elem T;
     constexpr int BLK = CFG::BLK, GROUPS = CFG::GROUPS, GROWS = CFG::GROWS;
     typedef typename std::conditional<BLK == 32, typename GemmTraits<DT>::acc, typename GemmTraits<DT>::acc_small>::type Acc;
@@ -1199,22 +1212,25 @@ __global__ void __launch_bounds__(CFG::NT)
     // compact block of the tile grid: their A and W panels fit that L2 and are fetched from HBM once, instead of
     // the whole W panel streaming through every L2 once per tile row.
     TR_TL(0);  // entry
-    touch_kernel_args<64 + sizeof(TileOrder) + sizeof(Epi)>();
+    // the epilogue's arguments, needed behind the first slab requests only
+    const uint32_t epi_args = request_kernel_args<56 + sizeof(Epi)>();
+    const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
     const int n_tiles = tiles_m * tiles_n;
     const int per_xcd = (n_tiles + 7) >> 3;
     const int vid     = (int)(blockIdx.x & 7) * per_xcd + (int)(blockIdx.x >> 3);
-    const int grp      = order.group.quotient(vid);
-    const int first_m  = grp * order.group_m;
-    const bool last_g  = tiles_m - first_m < order.group_m;
-    const int rows_g   = last_g ? tiles_m - first_m : order.group_m;
-    const int in_grp   = vid - grp * order.group_m * tiles_n;
-    const int col_g    = last_g ? order.last_rows.quotient(in_grp) : order.rows.quotient(in_grp);
+    const int group_m  = (int)(order_packed >> 18);
+    const int grp      = FixedDivisor{group_magic, order_packed & 63}.quotient(vid);
+    const int first_m  = grp * group_m;
+    const bool last_g  = tiles_m - first_m < group_m;
+    const int rows_g   = last_g ? tiles_m - first_m : group_m;
+    const int in_grp   = vid - grp * group_m * tiles_n;
+    const int col_g    = FixedDivisor{last_g ? last_magic : rows_magic, (order_packed >> (last_g ? 12 : 6)) & 63}.quotient(in_grp);
     const int m0       = (first_m + in_grp - col_g * rows_g) * BM;
     const int n0       = col_g * BN;
     if (vid >= n_tiles)
         return;  // the grid is padded to a multiple of 8; whole workgroups leave before any barrier
 
-    // ---- what the epilogue reads, requested before the first slab where a thread has one item and registers to spare: behind
+    // ---- what the epilogue reads, requested with the first slabs where a thread has one item and registers to spare: behind
     // the main loop the same loads are two latencies one after the other (columns and row pairs, then the residual), 0.4 us
     // of a launch of 4
     constexpr int CW    = TN * BLK;      // columns per wave
@@ -1247,23 +1263,27 @@ __global__ void __launch_bounds__(CFG::NT)
         if constexpr (RowIn<Epi>::value)
             early_row = epi.row_src(m0 + tid % BM < M ? m0 + tid % BM : M - 1);
     };
-    if constexpr (EARLY) {
-        if constexpr (ColArrays<Epi>::value > 0)
-            request_columns();
-        if constexpr (AHEAD > 0) {
-            int row = 0, col = 0;
-            item_at(tid % ITEMS, &row, &col);
-            const int m = m0 + row < M ? m0 + row : M - 1, n = n0 + col + 8 <= N ? n0 + col : N - 8;
-            if (N >= 8) {
-                const u32x4 *src = reinterpret_cast<const u32x4 *>(epi.ahead_src(m, n));
-                if (src) {
+    // Behind the first slabs: their place in memory is not in a register.  What waits for the first slabs waits for these as well.
+    auto request_ahead = [&]() __attribute__((always_inline)) {
+        asm volatile("" ::"s"(epi_args));
+        if constexpr (EARLY) {
+            if constexpr (ColArrays<Epi>::value > 0)
+                request_columns();
+            if constexpr (AHEAD > 0) {
+                int row = 0, col = 0;
+                item_at(tid % ITEMS, &row, &col);
+                const int m = m0 + row < M ? m0 + row : M - 1, n = n0 + col + 8 <= N ? n0 + col : N - 8;
+                if (N >= 8) {
+                    const u32x4 *src = reinterpret_cast<const u32x4 *>(epi.ahead_src(m, n));
+                    if (src) {
 #pragma unroll
-                    for (int q = 0; q < AHEAD; ++q)
-                        ahead_vec[q] = src[q];
+                        for (int q = 0; q < AHEAD; ++q)
+                            ahead_vec[q] = src[q];
+                    }
                 }
             }
         }
-    }
+    };
 
     Acc acc[TM][TN];
 #pragma unroll
@@ -1350,6 +1370,8 @@ __global__ void __launch_bounds__(CFG::NT)
         for (int p = 0; p < NS; ++p)
             if (k_lo + p < k_hi)
                 issue(k_lo + p, p);
+        TR_TL(5);  // first slabs requested
+        request_ahead();
         int stage = 0;
         auto wait_for = [&](int kt) __attribute__((always_inline)) {
             // slab kt is complete once at most the loads of the slabs requested after it are outstanding
@@ -1672,6 +1694,7 @@ __global__ void __launch_bounds__(CFG::NT)
             finish_sums(issued);
             TR_TL(6);  // handed-over row sums added up
         }
+        request_ahead();
         int stage = 0, fill = NS - 1;  // stage of slab kt; stage that slab kt + NS - 1 goes to
         // one slab; with_sums (the last slab in the late form) also requests the row sums
         auto step = [&](int kt, auto with_sums) __attribute__((always_inline)) {
@@ -1930,6 +1953,7 @@ __global__ void __launch_bounds__(CFG::NT)
 #define TR_CLAMPK(SLABIDX) (((SLABIDX)*KB) < last ? ((SLABIDX)*KB) : last)
     TR_LOAD_GLOBAL(ra0, rb0, 0);
     TR_LOAD_GLOBAL(ra1, rb1, TR_CLAMPK(1));
+    request_ahead();
     TR_STORE_LDS(0, ra0, rb0);
     __syncthreads();
     for (int kt = 0; kt + 2 <= nk; kt += 2) {
@@ -2091,6 +2115,11 @@ __global__ void __launch_bounds__(CFG::NT)
             }
         }
         __syncthreads();
+        // Waited for on every path: where a path passes their use by, the compiler waits where the paths meet, and there it waits for
+        // the result's store too, 960 clocks in front of the row sums.
+#pragma unroll
+        for (int q = 0; q < AHEAD; ++q)
+            asm volatile("" : "+v"(ahead_vec[q]));
 #pragma unroll
         for (int it = 0; it < (ITEMS + NT - 1) / NT; ++it) {
             const int item = it * NT + tid;
@@ -2139,12 +2168,10 @@ __global__ void __launch_bounds__(CFG::NT)
                     sm = epi.store8(m, n, v, col_lds + nl, BN, row_lds[m - m0], ahead);
                 }
                 if constexpr (CFG::sums_by_lanes) {
-                    static_assert(CPR == 8 && ITEMS % NT == 0, "eight lanes hold a row, and every lane has an item");
-#pragma unroll
-                    for (int o = 1; o < 8; o <<= 1) {
-                        sm.x += __shfl_xor(sm.x, o, 64);
-                        sm.y += __shfl_xor(sm.y, o, 64);
-                    }
+                    static_assert((CPR == 2 || CPR == 4 || CPR == 8) && (ITEMS % NT == 0 || ITEMS <= NT),
+                                  "so many neighbouring lanes hold a row, and all of them have an item or none");
+                    sm.x = add_neighbours<CPR>(sm.x);
+                    sm.y = add_neighbours<CPR>(sm.y);
                     if (piece == 0 && m < M && n < N)
                         store_out8(epi.through, &epi.row_sums[(size_t)(n / CFG::sum_cols) * M + m], sm);
                 } else {
@@ -2278,15 +2305,12 @@ int launch_tiled(hipStream_t s, const void *A, const void *B, int M, int N, int 
         while ((long)(group_m + 1) * (group_m + 1) <= resident)
             ++group_m;
     group_m = group_m > tiles_m ? tiles_m : group_m;
-    TileOrder order;
-    order.group_m   = group_m;
-    order.group     = FixedDivisor::of((uint32_t)(group_m * tiles_n));
-    order.rows      = FixedDivisor::of((uint32_t)group_m);
-    order.last_rows = FixedDivisor::of((uint32_t)(tiles_m % group_m));
+    group_m = group_m > TileOrder::kMaxRows ? TileOrder::kMaxRows : group_m;
+    const TileOrder order = TileOrder::of(tiles_m, tiles_n, group_m);
     unsigned grid = (unsigned)(((tiles_m * tiles_n + 7) / 8) * 8);
     t_last_sum_blocks = sum_blocks;
-    hipLaunchKernelGGL(kern, dim3(grid), dim3(CFG::NT), lds, s, (const T *)A, (const T *)B, M, N, K, lda, ldb, tiles_m, tiles_n,
-                       order, epi);
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(CFG::NT), lds, s, (const T *)A, (const T *)B, M, N, K, (int)lda, (int)ldb,
+                       order.group, order.rows, order.last_rows, order.packed, epi);
     TR_CHECK_LAUNCH();
     return 0;
 }
