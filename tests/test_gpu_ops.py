@@ -754,6 +754,41 @@ def test_gemm_fragments_read_ahead(code, slabs):
         assert np.abs(got - exact).max() <= (2.0 ** -11 if td is torch.float16 else 2.0 ** -8) * np.abs(exact).max() + 1e-4 * np.sqrt(K)
 
 
+@pytest.mark.parametrize("code", [8222222, 8322222, 8332222, 8422222])
+@pytest.mark.parametrize("slabs", [1, 2, 3, 4, 6, 24])
+def test_gemm_16x16_blocks_of_a_shared_slab(code, slabs):
+    """Tiles of 16 x 16 blocks whose slabs all waves share: fewer slabs than stages and more, one row or eight columns behind
+    whole tiles, less than a tile, every epilogue with its row sums; Q, K and V^T with tiles across their borders and
+    sequences that end inside a tile."""
+    from tnn_amd import capi
+    lib, o = capi.load(), ops()
+    K = 128 * slabs
+    say("tile configuration %d, %d slabs" % (code, slabs))
+    if slabs % 2 == 0:  # int8 rows of whole slabs
+        test_gemm_small_product_shapes(code, 1, 8, K)
+        test_gemm_small_product_shapes(code, 193, 200, K)
+    rng = np.random.default_rng(code % 1000 + slabs)
+    B, S, heads = 5, 72, 2
+    for td, unit in ((torch.float16, 2.0 ** -11), (torch.bfloat16, 2.0 ** -8)):
+        t, w = (torch.from_numpy(rng.standard_normal(n).astype(np.float32)).to(td) for n in ((B * S, K), (3 * heads * 64, K)))
+        bias = torch.from_numpy(rng.standard_normal(3 * heads * 64).astype(np.float32))
+        lib.tnn_rocm_debug_set_gemm_config(code)
+        try:
+            plain = host(o.gemm(t.cuda(), w.cuda(), True, bias=bias.cuda()).float()).astype(np.float64)
+            qk, vt = (host(x.float()).astype(np.float64) for x in o.qkv_split(t.cuda(), w.cuda(), bias.cuda(), B, S, heads))
+            fed = host(o.gemm_ln(t.cuda(), w.cuda(), bias.cuda(), w.double().sum(1).float().cuda(), 1e-5, row_sums=(_row_sums(t, 8), 8)).float())
+        finally:
+            lib.tnn_rocm_debug_set_gemm_config(0)
+        exact = t.double().numpy() @ w.double().numpy().T + bias.double().numpy()
+        # one rounding of the result and sums in fp32
+        allowed = unit * np.abs(exact).max() + 2.0 ** -22 * np.sqrt(K) * np.abs(exact).max()
+        assert np.abs(plain - exact).max() <= allowed and np.abs(qk - exact[:, :256]).max() <= allowed
+        assert np.abs(vt - exact[:, 256:].reshape(B, S, heads, 64).transpose(0, 2, 3, 1)).max() <= allowed
+        norm = (t.double() - t.double().mean(1, keepdim=True)) / (t.double().var(1, unbiased=False, keepdim=True) + 1e-5).sqrt()
+        ref = (norm @ w.double().T).numpy() + bias.double().numpy()
+        assert rel_err(fed, ref) <= (FP16_TOL if td is torch.float16 else 2e-2)
+
+
 @pytest.mark.parametrize("M,N,K,gelu,most", [(24576, 1536, 384, True, 1.1), (12288, 1024, 256, True, 1.07), (4096, 4096, 1024, False, 0.93)])
 def test_gemm_shape_picked_for_large_products(M, N, K, gelu, most):
     """256 x 256 tiles where they are the faster ones: with GELU and a short K they took 1.21, 1.12 times what 128 x 128 tiles take, and

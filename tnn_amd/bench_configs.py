@@ -183,8 +183,8 @@ def stores(args):
 
 
 # configuration codes of the tiled GEMM kernel, tnn_rocm_debug_set_gemm_config
-TILE_CODES = {"half": (6111141, 6211141, 6121141, 9111141, 9121141, 3112221, 3112222, 3212221, 4221141, 2112211, 2222221, 3332221,
-                       3331182, 2244211),
+TILE_CODES = {"half": (6111141, 6211141, 6121141, 9111141, 9121141, 3112221, 3212221, 2112211, 8222222, 8322222, 8332222, 8422222,
+                       2222221, 3332221, 2244211),
               "fp32": (6111141, 6211141, 6121141, 6111181, 6211181, 9111141, 9121141, 9111181, 9221141, 2321142, 2231142,
                        2331142, 2222121, 2222221, 2332121)}
 

@@ -188,14 +188,14 @@ def mall_probe(launches=20):
 # (code, rows, columns, tiles a CU holds at once) of the shapes the launcher chooses from, see TileCost in csrc/gemm_kernels.h
 TILE_SHAPES = {
     "half": ((6111141, 16, 16, 3), (6211141, 32, 16, 2), (6121141, 16, 32, 2), (9111141, 32, 32, 2), (9121141, 32, 64, 1),
-             (3112221, 64, 64, 3), (3112222, 64, 64, 1), (3212221, 128, 64, 2), (4221141, 64, 64, 2), (2112211, 64, 64, 4),
-             (2222221, 128, 128, 2), (3332221, 192, 192, 1), (3331182, 96, 96, 1), (2244211, 256, 256, 1)),
+             (3112221, 64, 64, 3), (3212221, 128, 64, 2), (2112211, 64, 64, 4), (8222222, 64, 64, 1), (8322222, 96, 64, 1),
+             (8332222, 96, 96, 1), (8422222, 128, 64, 1), (2222221, 128, 128, 2), (3332221, 192, 192, 1), (2244211, 256, 256, 1)),
     "f32": ((6111141, 16, 16, 3), (6211141, 32, 16, 2), (6121141, 16, 32, 2), (6111181, 16, 16, 1), (6211181, 32, 16, 1),
             (9111141, 32, 32, 2), (9121141, 32, 64, 1), (9111181, 32, 32, 1), (9221141, 64, 64, 1), (2321142, 96, 64, 1),
             (2231142, 64, 96, 1), (2331142, 96, 96, 1), (2222121, 128, 64, 2), (2222221, 128, 128, 1), (2332121, 192, 96, 1))}
 
 
-def tile_sweep(dtype, report):
+def tile_sweep(dtype, report, rows=()):
     """Every tile shape of the GEMM kernel over the launches of an encoder: the four projections with their fused epilogues,
     M from 16 tokens on, twelve weight sets in turn (inside a network a layer's weights come from the memory-side cache).
     Reports per launch how far the shape the library picks is behind the best one, and per shape the least-squares fit of the
@@ -204,7 +204,7 @@ def tile_sweep(dtype, report):
     lib = capi.load()
     shapes = TILE_SHAPES["f32" if dtype == "f32" else "half"]
     td, size = {"f16": (torch.float16, 2), "i8": (torch.int8, 1), "f32": (torch.float32, 4)}[dtype]
-    ms = (16, 32, 64, 100, 128, 197, 256, 384, 512, 700, 1000, 1536, 2000, 3072) + (() if dtype == "f32" else (4096, 8192))
+    ms = tuple(rows) or (16, 32, 64, 100, 128, 197, 256, 384, 512, 700, 1000, 1536, 2000, 3072) + (() if dtype == "f32" else (4096, 8192))
     seen, behind = {s[0]: [] for s in shapes}, []
 
     def launches(M, N, K, proj):
@@ -223,12 +223,14 @@ def tile_sweep(dtype, report):
         res = _randn((M, N), td) if proj in ("out", "ffn2") else None
         if dtype == "f32" or proj == "qkv" and M % 8:
             return lambda w: ops.gemm(a, w, True, bias=bias, gelu=proj == "ffn1", residual=res), ws
-        if proj == "qkv":
-            return lambda w: ops.qkv_split_ln(a, w, bias, col, 1e-5, B, M, heads, want_stats=True), ws
-        if proj == "ffn1":
-            return lambda w: ops.gemm_ln(a, w, bias, col, 1e-5, gelu=True, want_stats=True), ws
         stats = torch.ones(M, 2, device="cuda")
-        sums = torch.zeros(ops.MAX_ROW_SUM_BLOCKS, M, 2, device="cuda")
+        sums = torch.ones(ops.MAX_ROW_SUM_BLOCKS, M, 2, device="cuda")
+        # the projections that write a narrower tensor leave the rows' sums from about 190 rows on
+        fed = (sums, 12) if M >= 190 else None
+        if proj == "qkv":
+            return lambda w: ops.qkv_split_ln(a, w, bias, col, 1e-5, B, M, heads, want_stats=True, row_sums=fed), ws
+        if proj == "ffn1":
+            return lambda w: ops.gemm_ln(a, w, bias, col, 1e-5, gelu=True, want_stats=True, row_sums=fed), ws
         return lambda w: ops.gemm_residual_ln(a, w, res, stats, col, bias, bias=bias, want_row_sums=True, row_sums_out=sums), ws
 
     for H in (768,) if dtype == "f32" else (768, 1024):
@@ -274,6 +276,7 @@ def main():
     ap.add_argument("--simd-probe", action="store_true",
                     help="build (if missing) and run the stand-alone SIMD micro-benchmark csrc/probe_simd.hip")
     ap.add_argument("--tile-sweep", choices=["f16", "i8", "f32"], help="GEMM tile shapes over the launches of an encoder")
+    ap.add_argument("--rows", default="", help="with --tile-sweep: rows of the left operand, with commas")
     ap.add_argument("--build-only", action="store_true", help="with --simd-probe: compile it, do not run it")
     ap.add_argument("--launches", type=int, default=20)
     ap.add_argument("--only", default="")
@@ -290,7 +293,7 @@ def main():
             sys.exit(subprocess.call([exe]))
         return
     if a.tile_sweep:
-        tile_sweep(a.tile_sweep, lambda text: print(text, flush=True))
+        tile_sweep(a.tile_sweep, lambda text: print(text, flush=True), [int(m) for m in a.rows.split(",") if m])
         return
     if a.mall_probe:
         for r in mall_probe(a.launches):

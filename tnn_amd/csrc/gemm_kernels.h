@@ -1082,12 +1082,12 @@ __global__ void __launch_bounds__(WM *WN * 64)
 // OWN (with WGM = WGN = 1): every k-wave has a ring of NSTAGE slabs of its own and walks a contiguous part of K by itself.
 //     A slab is then SLAB bytes of k of ALL rows of the tile for ONE wave, and nothing in the main loop concerns another
 //     wave: no barrier, each wave waits for its own loads only.
-// BLK = 16 (with OWN): the waves' blocks are 16 x 16 instead of 32 x 32 (v_mfma_*_16x16x32, 64 bytes of k a step), TM and TN
-//     count those, and the whole tile is staged for the epilogue at once.
+// BLK = 16 (slabs direct to LDS): the waves' blocks are 16 x 16 instead of 32 x 32 (v_mfma_*_16x16x32, 64 bytes of k a step), TM
+//     and TN count those, and the whole tile is staged for the epilogue at once.
 template <int TM_, int TN_, int WGM_, int WGN_, int WGK_, int SLAB_, int NSTAGE_ = 0, bool OWN_ = false, int BLK_ = 32> struct TileCfg {
     static constexpr int BLK = BLK_;
     static constexpr int GROUPS = BLK_ == 32 ? TM_ : 1, GROWS = BLK_ == 32 ? 32 : BLK_ * TM_;  // staged together: rows of a wave position
-    static_assert(BLK_ == 32 || (BLK_ == 16 && OWN_ && BLK_ * TM_ <= 32), "16 x 16 blocks: small tiles with rings of the waves' own");
+    static_assert(BLK_ == 32 || (BLK_ == 16 && NSTAGE_ > 0 && (!OWN_ || BLK_ * TM_ <= 32)), "16 x 16 blocks: direct-to-LDS slabs only");
     static constexpr int TM = TM_, TN = TN_, WGM = WGM_, WGN = WGN_, WGK = WGK_, SLAB = SLAB_, NSTAGE = NSTAGE_;
     static constexpr bool OWN = OWN_;
     static constexpr int BM = BLK * TM * WGM, BN = BLK * TN * WGN;
@@ -1098,19 +1098,21 @@ template <int TM_, int TN_, int WGM_, int WGN_, int WGK_, int SLAB_, int NSTAGE_
     static constexpr size_t lds_bytes   = slab_bytes > stage_bytes ? slab_bytes : stage_bytes;
     // where an epilogue that leaves row sums keeps its BM x BN / 8 pairs: in the part of the slab area the staging does
     // not reach when that is large enough (dead by then), else behind everything
-    static constexpr size_t sums_bytes  = (size_t)BM * BN;
+    // Where the whole tile is staged at once, an item's pair goes into the place of its own staged values.
+    static constexpr bool sums_in_place = GROUPS == 1 && !OWN_;
+    static constexpr size_t sums_bytes  = sums_in_place ? 0 : (size_t)BM * BN;
     static constexpr size_t sums_offset = (slab_bytes >= stage_bytes + sums_bytes) ? stage_bytes : lds_bytes;
     // ... unless there is no such part and a row of a wave's columns lies in eight neighbouring lanes: the lanes then add up
     // the sums of each wave's columns among themselves (128 x 128: 16 KB of LDS would cost the CU's second workgroup)
     // or where all columns are one wave's anyway (32 x 32 tiles with rings of their own, 256 x 768 x 768: 4.60 -> 4.40 us against
     // sums through LDS, a barrier and a loop over them)
-    static constexpr bool sums_by_lanes = OWN_ || (TN_ == 2 && !(slab_bytes >= stage_bytes + sums_bytes));
+    static constexpr bool sums_by_lanes = OWN_ || (BLK_ == 32 && TN_ == 2 && !(slab_bytes >= stage_bytes + sums_bytes));
     static constexpr int sum_cols       = sums_by_lanes ? BLK_ * TN_ : BN;  // columns behind one pair of row sums
     static constexpr int NW = WGM * WGN * WGK, NT = 64 * NW;  // waves and threads per workgroup
     static_assert(NW == 4 || NW == 8, "four or eight waves per workgroup");
     static_assert(OWN_ || ((BM * (SLAB / 16)) % NT == 0 && (BN * (SLAB / 16)) % NT == 0), "slab must divide over the workgroup");
-    static_assert(!OWN_ || (WGM_ == 1 && WGN_ == 1 && NSTAGE_ >= 2 && NSTAGE_ <= 4), "rings of two to four slabs, k-waves only");
-    static_assert(OWN_ || NSTAGE_ == 0 || (NSTAGE_ >= 2 && NSTAGE_ <= 5), "register-staged, or two to five direct-to-LDS stages");
+    static_assert(!OWN_ || (WGM_ == 1 && WGN_ == 1 && NSTAGE_ >= 2 && NSTAGE_ <= 3), "rings of two or three slabs, k-waves only");
+    static_assert(OWN_ || NSTAGE_ == 0 || (NSTAGE_ >= 2 && NSTAGE_ <= 3), "register-staged, or two or three direct-to-LDS stages");
 };
 
 // Dynamic LDS of one (tile shape, epilogue) pair, for the kernel and its launcher alike: the slab / staging area, what
@@ -1230,14 +1232,15 @@ __global__ void __launch_bounds__(CFG::NT)
     if (vid >= n_tiles)
         return;  // the grid is padded to a multiple of 8; whole workgroups leave before any barrier
 
-    // ---- what the epilogue reads, requested with the first slabs where a thread has one item and registers to spare: behind
+    // ---- what the epilogue reads, requested with the first slabs where a thread has few items and registers to spare: behind
     // the main loop the same loads are two latencies one after the other (columns and row pairs, then the residual), 0.4 us
     // of a launch of 4
     constexpr int CW    = TN * BLK;      // columns per wave
     constexpr int CPR   = CW / 8;        // 8-column pieces per staged row
     constexpr int POS   = CFG::NW / WGK;  // wave positions (wm, wn) in the tile
     constexpr int ITEMS = POS * GROWS * CPR;
-    constexpr bool EARLY = GROUPS == 1 && ITEMS <= NT && CFG::NSTAGE > 0;
+    constexpr int MY_ITEMS = (ITEMS + NT - 1) / NT;  // of a thread
+    constexpr bool EARLY = GROUPS == 1 && MY_ITEMS <= 3 && CFG::NSTAGE > 0;
     const bool by_rows   = epi.direct(n0);
     // row and first column (inside the tile) of an item of the first group of rows of every wave position
     auto item_at = [&](int item, int *row, int *col) __attribute__((always_inline)) {
@@ -1251,7 +1254,7 @@ __global__ void __launch_bounds__(CFG::NT)
     float early_col[COLQ > 0 ? COLQ : 1];
     float2 early_row = make_float2(0.f, 0.f);
     constexpr int AHEAD = EARLY ? AheadVecs<Epi>::value : 0;
-    u32x4 ahead_vec[AHEAD > 0 ? AHEAD : 1];
+    u32x4 ahead_vec[MY_ITEMS][AHEAD > 0 ? AHEAD : 1];
     auto request_columns = [&]() __attribute__((always_inline)) {
 #pragma unroll
         for (int q = 0; q < COLQ; ++q) {
@@ -1270,15 +1273,18 @@ __global__ void __launch_bounds__(CFG::NT)
             if constexpr (ColArrays<Epi>::value > 0)
                 request_columns();
             if constexpr (AHEAD > 0) {
-                int row = 0, col = 0;
-                item_at(tid % ITEMS, &row, &col);
-                const int m = m0 + row < M ? m0 + row : M - 1, n = n0 + col + 8 <= N ? n0 + col : N - 8;
-                if (N >= 8) {
-                    const u32x4 *src = reinterpret_cast<const u32x4 *>(epi.ahead_src(m, n));
-                    if (src) {
 #pragma unroll
-                        for (int q = 0; q < AHEAD; ++q)
-                            ahead_vec[q] = src[q];
+                for (int it = 0; it < MY_ITEMS; ++it) {
+                    int row = 0, col = 0;
+                    item_at((it * NT + tid) % ITEMS, &row, &col);
+                    const int m = m0 + row < M ? m0 + row : M - 1, n = n0 + col + 8 <= N ? n0 + col : N - 8;
+                    if (N >= 8) {
+                        const u32x4 *src = reinterpret_cast<const u32x4 *>(epi.ahead_src(m, n));
+                        if (src) {
+#pragma unroll
+                            for (int q = 0; q < AHEAD; ++q)
+                                ahead_vec[it][q] = src[q];
+                        }
                     }
                 }
             }
@@ -1295,7 +1301,7 @@ __global__ void __launch_bounds__(CFG::NT)
                 acc[i][j][r] = 0;
 
     const int frag_row = lane % BLK;
-    const int frag_off = (lane >> 5) * 16;
+    const int frag_off = (lane >> 5) * 16;  // slabs staged through registers: blocks of 32 x 32
     const int nk       = K / KB;
     constexpr int FRAGS = GemmTraits<DT>::FRAGS, KSTEP = (1024 / BLK) * FRAGS;  // bytes of k per row that one step multiplies
     const SplitConst split_const;
@@ -1376,9 +1382,7 @@ __global__ void __launch_bounds__(CFG::NT)
         auto wait_for = [&](int kt) __attribute__((always_inline)) {
             // slab kt is complete once at most the loads of the slabs requested after it are outstanding
             const int behind = k_hi - 1 - kt;
-            if (NS > 3 && behind >= 3)
-                TR_WAIT_VMCNT(NS > 3 ? 3 * LPW : 0);
-            else if (NS > 2 && behind >= 2)
+            if (NS > 2 && behind >= 2)
                 TR_WAIT_VMCNT(NS > 2 ? 2 * LPW : 0);
             else if (behind >= 1)
                 TR_WAIT_VMCNT(LPW);
@@ -1530,50 +1534,35 @@ __global__ void __launch_bounds__(CFG::NT)
         // byte offset of this lane's fragment chunk inside a slab row, per k-step of the slab
         const int fswz = (frag_row / R256) % VPR;
         const int frow = frag_row * SLAB;
-        // One slab: this wave's fragments of it, then `between` (the requests for the slab that goes into the stage freed
-        // last), then the MFMAs.  READ_AHEAD reads all of the slab's fragments before the requests, so that the LDS
-        // latency runs while the requests are issued; it needs the registers for them.
+        // One slab: `between` (the requests for the slab that goes into the stage freed last), then step by step this wave's
+        // fragments and their MFMAs
         constexpr int KSTEPS      = SLAB / KSTEP / WGK;
         static_assert((SLAB / KSTEP) % WGK == 0, "k-steps of a slab must split evenly over the k-waves");
-        constexpr bool READ_AHEAD = NS >= 4 && (TM + TN) * KSTEPS <= 8;
         auto compute = [&](int stage, auto between) __attribute__((always_inline)) {
             const unsigned char *sa = lds_dyn + stage * STAGE, *sb = sa + BM * SLAB;
-            uint4 fa[READ_AHEAD ? KSTEPS : 1][TM][FRAGS], fb[READ_AHEAD ? KSTEPS : 1][TN][FRAGS];
-            auto read = [&](int ks, int slot) __attribute__((always_inline)) {
-#pragma unroll
-                for (int f = 0; f < FRAGS; ++f) {
-                    const int chunk = ((((wk + ks * WGK) * FRAGS + f) * 2 + (lane >> 5)) ^ fswz) * 16;
-#pragma unroll
-                    for (int i = 0; i < TM; ++i)
-                        fa[slot][i][f] = *reinterpret_cast<const uint4 *>(sa + (wm * TM + i) * 32 * SLAB + frow + chunk);
-#pragma unroll
-                    for (int j = 0; j < TN; ++j)
-                        fb[slot][j][f] = *reinterpret_cast<const uint4 *>(sb + (wn * TN + j) * 32 * SLAB + frow + chunk);
-                }
-            };
-            if constexpr (READ_AHEAD) {
-#pragma unroll
-                for (int ks = 0; ks < KSTEPS; ++ks)
-                    read(ks, ks);
-            }
             between();
 #pragma unroll
             for (int ks = 0; ks < KSTEPS; ++ks) {
-                const int slot = READ_AHEAD ? ks : 0;
-                if constexpr (!READ_AHEAD)
-                    read(ks, 0);
+                uint4 fa[TM], fb[TN];
+                const int chunk = (((wk + ks * WGK) * (64 / BLK) + lane / BLK) ^ fswz) * 16;
+#pragma unroll
+                for (int i = 0; i < TM; ++i)
+                    fa[i] = *reinterpret_cast<const uint4 *>(sa + (wm * TM + i) * BLK * SLAB + frow + chunk);
+#pragma unroll
+                for (int j = 0; j < TN; ++j)
+                    fb[j] = *reinterpret_cast<const uint4 *>(sb + (wn * TN + j) * BLK * SLAB + frow + chunk);
                 if constexpr (Epi::kRowStats && !TakesRowSums<Epi>::value) {
                     // the WGN waves that hold the same A rows take turns over the row groups and k-steps
 #pragma unroll
                     for (int i = 0; i < TM; ++i)
                         if ((i + ks) % WGN == wn)
-                            ln_take(fa[slot][i][0], i);
+                            ln_take(fa[i], i);
                 }
 #pragma unroll
                 for (int i = 0; i < TM; ++i)
 #pragma unroll
                     for (int j = 0; j < TN; ++j)
-                        GemmTraits<DT>::mma(fb[slot][j][0], fa[slot][i][0], acc[i][j]);
+                        GemmTraits<DT>::mma(fb[j], fa[i], acc[i][j]);
             }
         };
         constexpr int LPW = A_LD + B_LD;
@@ -1680,7 +1669,7 @@ __global__ void __launch_bounds__(CFG::NT)
         // (3072 x 2304 x 768 18.9 -> 18.1), but with operands that come from the memory-side cache, as in a network, they lose
         // (17.5 -> 17.7; twelve layers of 8 x 384 tokens 1134 -> 1145 us over eight instances).  Waves with one block have
         // nothing to hide the reads behind: 64 x 64 tiles 256 x 3072 x 768 6.3 -> 6.6, four waves 985 x 2304 x 768 9.7 -> 10.1.
-        constexpr bool PIPE = DT != TNN_ROCM_F32 && CFG::NW == 8 && KSTEPS >= 2 && TM * TN > 4;
+        constexpr bool PIPE = DT != TNN_ROCM_F32 && CFG::NW == 8 && KSTEPS >= 2 && (TM * TN > 4 || BLK == 16);
         static_assert(!PIPE || KSTEPS % 2 == 0, "two sets of fragments, every slab begins with the first");
         if constexpr (TakesRowSums<Epi>::value && !kLateSums)
             request_sums();
@@ -1700,11 +1689,7 @@ __global__ void __launch_bounds__(CFG::NT)
         auto step = [&](int kt, auto with_sums) __attribute__((always_inline)) {
             // slab kt has landed once at most the loads of the slabs issued after it are outstanding
             const int behind = nk - 1 - kt;
-            if (NS > 4 && behind >= 3)
-                TR_WAIT_VMCNT(NS > 4 ? 3 * LPW : 0);
-            else if (NS > 3 && behind >= 2)
-                TR_WAIT_VMCNT(NS > 3 ? 2 * LPW : 0);
-            else if (NS > 2 && behind >= 1)
+            if (NS > 2 && behind >= 1)
                 TR_WAIT_VMCNT(NS > 2 ? LPW : 0);
             else
                 TR_WAIT_VMCNT(0);
@@ -1730,13 +1715,13 @@ __global__ void __launch_bounds__(CFG::NT)
             int chunk[KSTEPS];
 #pragma unroll
             for (int ks = 0; ks < KSTEPS; ++ks)
-                chunk[ks] = frow + (((wk + ks * WGK) * 2 + (lane >> 5)) ^ fswz) * 16;
+                chunk[ks] = frow + (((wk + ks * WGK) * (64 / BLK) + lane / BLK) ^ fswz) * 16;
             auto read_one = [&](int k, int ks, int from) __attribute__((always_inline)) {  // fragment k of step ks
                 const unsigned char *at = lds_dyn + from * STAGE + chunk[ks];
                 if (k < TM)
-                    fa[ks & 1][k < TM ? k : 0][0] = *reinterpret_cast<const uint4 *>(at + (wm * TM + k) * 32 * SLAB);
+                    fa[ks & 1][k < TM ? k : 0][0] = *reinterpret_cast<const uint4 *>(at + (wm * TM + k) * BLK * SLAB);
                 else
-                    fb[ks & 1][k >= TM ? k - TM : 0][0] = *reinterpret_cast<const uint4 *>(at + BM * SLAB + (wn * TN + k - TM) * 32 * SLAB);
+                    fb[ks & 1][k >= TM ? k - TM : 0][0] = *reinterpret_cast<const uint4 *>(at + BM * SLAB + (wn * TN + k - TM) * BLK * SLAB);
             };
             // slab kt, the first of whose fragments have been read; MORE: another one follows, LOADS: and one is requested
             auto slab = [&](int kt, auto more, auto loads) __attribute__((always_inline)) {
@@ -2118,10 +2103,10 @@ __global__ void __launch_bounds__(CFG::NT)
         // Waited for on every path: where a path passes their use by, the compiler waits where the paths meet, and there it waits for
         // the result's store too, 960 clocks in front of the row sums.
 #pragma unroll
-        for (int q = 0; q < AHEAD; ++q)
-            asm volatile("" : "+v"(ahead_vec[q]));
+        for (int q = 0; q < MY_ITEMS * AHEAD; ++q)
+            asm volatile("" : "+v"(ahead_vec[q / (AHEAD > 0 ? AHEAD : 1)][q % (AHEAD > 0 ? AHEAD : 1)]));
 #pragma unroll
-        for (int it = 0; it < (ITEMS + NT - 1) / NT; ++it) {
+        for (int it = 0; it < MY_ITEMS; ++it) {
             const int item = it * NT + tid;
             if (ITEMS % NT != 0 && item >= ITEMS)
                 break;
@@ -2153,7 +2138,7 @@ __global__ void __launch_bounds__(CFG::NT)
             const int m = m0 + ((pos / WGN) * GROUPS + i) * GROWS + row;
             const int n = n0 + (pos % WGN) * CW + c8;
             const int nl = (pos % WGN) * CW + c8;  // column inside the tile
-            const u32x4 *const ahead = AHEAD > 0 ? ahead_vec : nullptr;
+            const u32x4 *const ahead = AHEAD > 0 ? ahead_vec[it] : nullptr;
             if constexpr (Epi::kRowStats) {
                 if (m < M && n + 7 < N) {  // N is a multiple of 8 for these epilogues (checked at launch)
                     AccT v[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
@@ -2174,6 +2159,8 @@ __global__ void __launch_bounds__(CFG::NT)
                     sm.y = add_neighbours<CPR>(sm.y);
                     if (piece == 0 && m < M && n < N)
                         store_out8(epi.through, &epi.row_sums[(size_t)(n / CFG::sum_cols) * M + m], sm);
+                } else if constexpr (CFG::sums_in_place) {
+                    *reinterpret_cast<float2 *>(const_cast<AccT *>(src)) = sm;
                 } else {
                     reinterpret_cast<float2 *>(lds_dyn + CFG::sums_offset)[(((pos / WGN) * GROUPS + i) * GROWS + row) * (BN / 8) +
                                                                          ((pos % WGN) * CW + c8) / 8] = sm;
@@ -2212,11 +2199,18 @@ __global__ void __launch_bounds__(CFG::NT)
         // that reads C next
         __syncthreads();
         if (tid < BM && m0 + tid < M) {
-            const float2 *part = reinterpret_cast<const float2 *>(lds_dyn + CFG::sums_offset) + tid * (BN / 8);
             float s1 = 0.f, s2 = 0.f;
 #pragma unroll
-            for (int q = 0; q < BN / 8; ++q)
-                s1 += part[q].x, s2 += part[q].y;
+            for (int q = 0; q < BN / 8; ++q) {
+                float2 part;
+                if constexpr (CFG::sums_in_place) {
+                    const int pos = tid / GROWS * WGN + q / CPR;
+                    part = *reinterpret_cast<const float2 *>(stage_all + (pos * WGK) * (GROWS * SSTR) + tid % GROWS * SSTR + q % CPR * 8);
+                } else {
+                    part = reinterpret_cast<const float2 *>(lds_dyn + CFG::sums_offset)[tid * (BN / 8) + q];
+                }
+                s1 += part.x, s2 += part.y;
+            }
             store_out8(epi.through, &epi.row_sums[(size_t)(n0 / BN) * M + m0 + tid], make_float2(s1, s2));
         }
     }
@@ -2318,14 +2312,14 @@ int launch_tiled(hipStream_t s, const void *A, const void *B, int M, int N, int 
 // Configuration codes: [P] TM TN WGM WGN WGK S (one decimal digit each; slab bytes = 64 << S; P = number of
 // direct-to-LDS stages, 9 = rings of the waves' own, absent = slabs staged through registers).
 //   9111141   32 x  32, 4 k-waves with rings of their own     9121141   32 x  64, likewise
-//   3112221   64 x  64, 8 waves (two k-waves), 3 stages       3112222   64 x  64, 8 waves, 256-byte slabs
-//   4221141   64 x  64, 4 k-waves, 4 stages                   3212221  128 x  64, 8 waves
+//   3112221   64 x  64, 8 waves (two k-waves), 3 stages       3212221  128 x  64, 8 waves
 //   6111141   16 x  16, 6211141 32 x 16, 6121141 16 x 32: 16 x 16 blocks, 4 k-waves with rings of their own (three slabs)
+//   8222222   64 x  64, 8322222 96 x 64, 8332222 96 x 96, 8422222 128 x 64: 16 x 16 blocks, 8 waves (two k-waves), 3 stages of 256 bytes
 //   2112211   64 x  64, 4 waves, 2 stages                     2222221  128 x 128, 8 waves (two k-waves)
 //   fp32 only: 6111181, 6211181 16 x 16 and 32 x 16, 8 k-waves; 9111181 32 x 32, 8 k-waves; 9221141 64 x 64, 4 k-waves with rings of their own;
 //   2321142, 2231142, 2331142 96 x 64, 64 x 96 and 96 x 96, 4 k-waves; 2222121, 2332121 128 x 64 and 192 x 96, 4 waves (two k-waves)
 //   2244211  256 x 256, 8 waves
-//   3332221  192 x 192, 8 waves (two k-waves)                 3331182   96 x  96, 8 k-waves, 256-byte slabs
+//   3332221  192 x 192, 8 waves (two k-waves)
 //   112210    64 x  64 and 222210 128 x 128, 4 waves: rows that are no multiple of 128 bytes
 // Eight-wave workgroups put two waves on every SIMD inside one tile: while one waits for its LDS fragments the
 // other issues MFMAs, and a larger tile per CU moves fewer bytes through LDS and L2 per flop.  Four-wave tiles
@@ -2338,11 +2332,11 @@ int launch_tiled(hipStream_t s, const void *A, const void *B, int M, int N, int 
 // int8: M from 16 to 8192, the four projections of hidden sizes 768 and 1024 with their fused epilogues; fp32: M from 16 to
 // 3072), taken over twelve weight sets in turn so that weights come from the memory-side cache as they do inside a network:
 // python -m tnn_amd.bench_ops --tile-sweep measures them and fits the rows.  A launch is 3 .. 20 % off its prediction on average,
-// by shape (the large ones most), so picks closer than that are as good as drawn.  Taken together the picks are 1.1 % (fp16), 1.0 %
-// (int8), 1.0 % (fp32) behind the best shape of each launch back to back, at worst 15 % (M=4096 N=768 K=3072, where 2112211 leads),
-// 11 % and 6 %, and 0.29, 0.37 and 0.45 us inside the network (bench_configs --config tiles; profiles/gemm_tile_choice.txt).  Not
-// as the sweep fits them: the 256 x 256 rows (below), the 192 x 192 row of the half table, which is of before its loop read ahead,
-// and in the int8 table what the comment above it says.  The rules this replaced, made for M >= 1024, were 51 %, 34 % and 77 % behind:
+// by shape (the large ones most), so picks closer than that are as good as drawn.  Taken together the picks are 0.6 % (fp16), 0.9 %
+// (int8), 1.0 % (fp32) behind the best shape of each launch back to back (256 launches each of fp16 and int8, of which half had no
+// part in the fit).  Not as the sweep fits them: the 256 x 256 rows (below), the 192 x 192 row of the half table, which is of
+// before its loop read ahead, the rows of 16 x 16 blocks of a shared slab (below), and in the int8 table what the comment above
+// it says.  The rules this replaced, made for M >= 1024, were 51 %, 34 % and 77 % behind:
 //   M=  32 N= 768 K=3072 fp16  23.1 -> 7.3 us   (64x64 tiles: 12 CUs, one two-stage slab after another)
 //   M= 256 N= 768 K=3072 fp16  23.7 -> 7.2      M= 256 N=2304 K=768 fp16  8.7 -> 6.2
 //   M=1000 N= 768 K=3072 fp16  24.3 -> 12.4     M=1000 N= 768 K=768 fp16  8.7 -> 5.5
@@ -2357,13 +2351,14 @@ constexpr TileCost kTilesHalf[] = {
     {9111141, 32, 32, 2, 3.47f, 2.09f, {0.067f, 0.147f}},
     {9121141, 32, 64, 1, 3.46f, 2.56f, {0.121f}},
     {3112221, 64, 64, 3, 3.72f, 3.06f, {0.205f, 0.377f, 0.654f}},
-    {3112222, 64, 64, 1, 3.45f, 3.09f, {0.179f}},
     {3212221, 128, 64, 2, 4.60f, 5.12f, {0.287f, 0.607f}},
-    {4221141, 64, 64, 2, 4.34f, 3.22f, {0.158f, 0.351f}},
     {2112211, 64, 64, 4, 2.96f, 1.83f, {0.411f, 0.493f, 0.607f, 0.877f}},
     {2222221, 128, 128, 2, 4.84f, 5.77f, {0.561f, 1.044f}},
     {3332221, 192, 192, 1, 10.15f, 13.25f, {0.767f}},
-    {3331182, 96, 96, 1, 6.94f, 7.10f, {0.264f}},
+    {8222222, 64, 64, 1, 3.70f, 2.89f, {0.145f}},
+    {8322222, 96, 64, 1, 4.32f, 3.75f, {0.205f}},
+    {8332222, 96, 96, 1, 5.06f, 5.33f, {0.242f}},
+    {8422222, 128, 64, 1, 4.45f, 4.28f, {0.243f}},
     {2244211, 256, 256, 1, 10.5f, 12.0f, {1.5f}},
 };
 // 256 x 256 tiles are for products that fill the chip with them: half the bytes a flop of 128 x 128 tiles.  A linear model knows
@@ -2376,7 +2371,16 @@ constexpr TileCost kTilesHalf[] = {
 // picks that are slower cost 25 % together (187 % with the old row), the shape where it is left out and faster 88 % (99 %).  The int8
 // row is set by hand: of its picks three of 60 are slower, 24576 x 1920 x 640 into Q, K and V^T by 6 % and [16384, 1024] x 1024 and
 // 24576 x 1280 x 1280 with a residual by 3 %.
-// Tiles of 16 x 16 blocks are for the products whose 32x32 tiles are too few for the chip: a CU's panels come through its L1 at
+// 16 x 16 blocks of a shared slab, 64 x 64 to 128 x 64: eight waves as 2 x 2 positions and two k-waves, so that a tile of any number of
+// 32 rows and columns is dealt out evenly.  96 x 96 as eight k-waves of 3 x 3 blocks of 32 x 32 passed 295 KB of partial sums
+// through LDS behind its loop (half of the 11 us of 3072 x 768 x 768), now 74; 96 x 64 is one round of the chip where 64 x 64 are
+// two.  Their rows are the fit's, moved until no launch of the sweep that changed its shape for them is slower (of 512 two are, by
+// 3 %).  fp16 launches are 2.9 % faster on average and by up to 24 %, int8 1.4 % and 21 %.  us, the picks before -> these:
+//   fp16 3072 x 768 x 768 10.9 -> 8.8, 3072 x 768 x 3072 22.9 -> 20.1, 1536 x 768 x 3072 18.8 -> 14.5, 984 x 768 x 3072 13.0 -> 11.8,
+//   700 x 3072 x 768 10.9 -> 8.3, 1536 x 1024 x 4096 23.1 -> 18.1; int8 1536 x 768 x 3072 11.8 -> 9.3, 3072 x 768 x 3072 15.5 -> 13.2
+// (Not taken: 64 x 96, 32 x 64, 64 x 32, 32 x 96, 64 x 128, within 0.1 % of the sweep together; two stages instead of three, 96 x 96 8.9 ->
+// 9.9; four k-waves, 96 x 96 9.1 -> 9.4.)
+// Tiles of 16 x 16 blocks with rings of the waves' own are for the products whose 32x32 tiles are too few for the chip: a CU's panels come through its L1 at
 // 64 bytes a clock at best, so 24 tiles of (32 + 32) rows of K=3072 take 4 us for that alone, and 96 of (16 + 16) rows half.
 // us a launch, best shape before -> now (fp32: 8 waves where K is long):
 //   M= 32 N= 768 K=3072 fp16  7.4 -> 5.0   int8 5.0 -> 4.1   fp32 14.9 -> 8.8     M= 32 N=768 K=768 fp16 3.9 -> 3.2, fp32 6.4 -> 4.6
@@ -2393,13 +2397,14 @@ constexpr TileCost kTilesI8[] = {
     {9111141, 32, 32, 2, 2.98f, 1.93f, {0.078f, 0.151f}},
     {9121141, 32, 64, 1, 3.25f, 2.21f, {0.130f}},
     {3112221, 64, 64, 3, 3.40f, 2.05f, {0.218f, 0.398f, 0.701f}},
-    {3112222, 64, 64, 1, 3.09f, 2.21f, {0.196f}},
     {3212221, 128, 64, 2, 4.05f, 3.04f, {0.313f, 0.644f}},
-    {4221141, 64, 64, 2, 4.06f, 2.67f, {0.174f, 0.389f}},
     {2112211, 64, 64, 4, 3.00f, 1.56f, {0.424f, 0.558f, 0.687f, 0.916f}},
     {2222221, 128, 128, 2, 5.15f, 3.79f, {0.640f, 1.156f}},
     {3332221, 192, 192, 1, 9.89f, 9.10f, {0.860f}},
-    {3331182, 96, 96, 1, 6.72f, 5.80f, {0.314f}},
+    {8222222, 64, 64, 1, 3.23f, 2.32f, {0.162f}},
+    {8322222, 96, 64, 1, 4.20f, 5.50f, {0.212f}},
+    {8332222, 96, 96, 1, 5.62f, 4.51f, {0.276f}},
+    {8422222, 128, 64, 1, 4.46f, 4.15f, {0.261f}},
     {2244211, 256, 256, 1, 10.6f, 8.2f, {2.1f}},
 };
 // fp32 on three bf16 planes: six matrix instructions per operand pair and the conversion between them, so a step costs five
@@ -2475,7 +2480,10 @@ int launch_gemm_fast(hipStream_t s, const void *A, const void *B, int M, int N, 
         case 222221:
         case 224211: cfg = 2222221; break;
         case 332221: cfg = 3332221; break;
-        case 331182: cfg = 3331182; break;
+        case 331182:
+        case 3331182: cfg = 8332222; break;  // the shapes that these blocks took the place of
+        case 4221141:
+        case 3112222: cfg = 8222222; break;
         default: break;
     }
     if (kbytes % (64u << (cfg % 10)) != 0) {
@@ -2486,12 +2494,14 @@ int launch_gemm_fast(hipStream_t s, const void *A, const void *B, int M, int N, 
     return launch_tiled<DT, TileCfg<TMv, TNv, WGMv, WGNv, WGKv, SLABv>, Epi>(s, A, B, M, N, K, lda, ldb, epi)
 #define TR_FAST_DL(TMv, TNv, WGMv, WGNv, WGKv, SLABv, NSv)                                                            \
     return launch_tiled<DT, TileCfg<TMv, TNv, WGMv, WGNv, WGKv, SLABv, NSv>, Epi>(s, A, B, M, N, K, lda, ldb, epi)
+#define TR_FAST_DL16(TMv, TNv, WGMv, WGNv, WGKv, SLABv, NSv)                                                          \
+    return launch_tiled<DT, TileCfg<TMv, TNv, WGMv, WGNv, WGKv, SLABv, NSv, false, 16>, Epi>(s, A, B, M, N, K, lda, ldb, epi)
 #define TR_FAST_SMALL(TMv, TNv, WGKv, SLABv, NSv)                                                                     \
     return launch_tiled<DT, TileCfg<TMv, TNv, 1, 1, WGKv, SLABv, NSv, true, 16>, Epi>(s, A, B, M, N, K, lda, ldb, epi)
 #define TR_FAST_OWN(TMv, TNv, WGKv, SLABv, NSv)                                                                       \
     return launch_tiled<DT, TileCfg<TMv, TNv, 1, 1, WGKv, SLABv, NSv, true>, Epi>(s, A, B, M, N, K, lda, ldb, epi)
     if constexpr (TakesRowSums<Epi>::value) {
-        if (cfg >= 6000000)
+        if (cfg >= 9000000 || (cfg >= 6000000 && cfg < 7000000))
             return kNotWithRowSums;
     } else {
         switch (cfg) {
@@ -2528,14 +2538,15 @@ int launch_gemm_fast(hipStream_t s, const void *A, const void *B, int M, int N, 
     } else {
         switch (cfg) {
             case 2112211: TR_FAST_DL(1, 1, 2, 2, 1, 128, 2);
-            case 4221141: TR_FAST_DL(2, 2, 1, 1, 4, 128, 4);
             case 3112221: TR_FAST_DL(1, 1, 2, 2, 2, 128, 3);
-            case 3112222: TR_FAST_DL(1, 1, 2, 2, 2, 256, 3);
             case 3212221: TR_FAST_DL(2, 1, 2, 2, 2, 128, 3);
             case 2222221: TR_FAST_DL(2, 2, 2, 2, 2, 128, 2);
             case 3332221: TR_FAST_DL(3, 3, 2, 2, 2, 128, 3);
-            case 3331182: TR_FAST_DL(3, 3, 1, 1, 8, 256, 3);
             case 2244211: TR_FAST_DL(2, 4, 4, 2, 1, 128, 2);
+            case 8222222: TR_FAST_DL16(2, 2, 2, 2, 2, 256, 3);
+            case 8322222: TR_FAST_DL16(3, 2, 2, 2, 2, 256, 3);
+            case 8332222: TR_FAST_DL16(3, 3, 2, 2, 2, 256, 3);
+            case 8422222: TR_FAST_DL16(4, 2, 2, 2, 2, 256, 3);
             default: break;
         }
     }
@@ -2548,6 +2559,7 @@ int launch_gemm_fast(hipStream_t s, const void *A, const void *B, int M, int N, 
     }
 #undef TR_FAST_OWN
 #undef TR_FAST_SMALL
+#undef TR_FAST_DL16
 #undef TR_FAST
 #undef TR_FAST_DL
     set_error("gemm: unknown tuning configuration %d", cfg);
