@@ -754,7 +754,7 @@ def test_gemm_fragments_read_ahead(code, slabs):
         assert np.abs(got - exact).max() <= (2.0 ** -11 if td is torch.float16 else 2.0 ** -8) * np.abs(exact).max() + 1e-4 * np.sqrt(K)
 
 
-@pytest.mark.parametrize("code", [8222222, 8322222, 8332222, 8422222])
+@pytest.mark.parametrize("code", [8222222, 8322222, 8332222, 8422222, 7244211, 8244211, 8264211, 8344211, 8364211, 8444211])
 @pytest.mark.parametrize("slabs", [1, 2, 3, 4, 6, 24])
 def test_gemm_16x16_blocks_of_a_shared_slab(code, slabs):
     """Tiles of 16 x 16 blocks whose slabs all waves share: fewer slabs than stages and more, one row or eight columns behind
@@ -762,9 +762,9 @@ def test_gemm_16x16_blocks_of_a_shared_slab(code, slabs):
     sequences that end inside a tile."""
     from tnn_amd import capi
     lib, o = capi.load(), ops()
-    K = 128 * slabs
+    K = 64 * slabs << code % 10 - 1
     say("tile configuration %d, %d slabs" % (code, slabs))
-    if slabs % 2 == 0:  # int8 rows of whole slabs
+    if slabs % 2 == 0 and code not in (8264211, 8444211):  # int8 rows of whole slabs, in the shapes that int8 has
         test_gemm_small_product_shapes(code, 1, 8, K)
         test_gemm_small_product_shapes(code, 193, 200, K)
     rng = np.random.default_rng(code % 1000 + slabs)
@@ -776,7 +776,14 @@ def test_gemm_16x16_blocks_of_a_shared_slab(code, slabs):
         try:
             plain = host(o.gemm(t.cuda(), w.cuda(), True, bias=bias.cuda()).float()).astype(np.float64)
             qk, vt = (host(x.float()).astype(np.float64) for x in o.qkv_split(t.cuda(), w.cuda(), bias.cuda(), B, S, heads))
-            fed = host(o.gemm_ln(t.cuda(), w.cuda(), bias.cuda(), w.double().sum(1).float().cuda(), 1e-5, row_sums=(_row_sums(t, 8), 8)).float())
+            cs = w.double().sum(1).float().cuda()
+            fed = [host(o.gemm_ln(t.cuda(), w.cuda(), bias.cuda(), cs, 1e-5, row_sums=r).float())
+                   for r in (None, (_row_sums(t, 8), 8), (_row_sums(t, 24), 24)) if K % 128 == 0]
+            st = torch.stack([1 / (x.var(1, unbiased=False) + 1e-5).sqrt() for x in (t.double(),)] + [t.double().mean(1)], 1).float().cuda()
+            one, x = torch.ones(K, device="cuda"), t[:, :64].contiguous()
+            wx = torch.from_numpy(rng.standard_normal((K, 64)).astype(np.float32)).to(td)
+            left, (sums, blocks) = o.gemm_residual_ln(x.cuda(), wx.cuda(), t.cuda(), st, one, one, want_row_sums=True) \
+                if code % 10 == 1 else (None, (None, 0))
         finally:
             lib.tnn_rocm_debug_set_gemm_config(0)
         exact = t.double().numpy() @ w.double().numpy().T + bias.double().numpy()
@@ -786,7 +793,15 @@ def test_gemm_16x16_blocks_of_a_shared_slab(code, slabs):
         assert np.abs(vt - exact[:, 256:].reshape(B, S, heads, 64).transpose(0, 2, 3, 1)).max() <= allowed
         norm = (t.double() - t.double().mean(1, keepdim=True)) / (t.double().var(1, unbiased=False, keepdim=True) + 1e-5).sqrt()
         ref = (norm @ w.double().T).numpy() + bias.double().numpy()
-        assert rel_err(fed, ref) <= (FP16_TOL if td is torch.float16 else 2e-2)
+        for f in fed:
+            assert rel_err(f, ref) <= (FP16_TOL if td is torch.float16 else 2e-2)
+        if left is not None:
+            want = x.double() @ wx.double().T + (t.double() - t.double().mean(1, keepdim=True)) * st[:, :1].double().cpu() + 1
+            assert rel_err(host(left.float()), want.numpy()) <= (FP16_TOL if td is torch.float16 else 2e-2)
+            stored, got = left.double().cpu(), sums.double().cpu()[:blocks].sum(0)
+            assert blocks == -(-K // (int(str(code)[2]) * 16 * int(str(code)[4])))
+            assert (got[:, 0] - stored.sum(1)).abs().max() <= 1e-5 * stored.abs().sum(1).max()
+            assert (got[:, 1] / (stored ** 2).sum(1) - 1).abs().max() <= 1e-5
 
 
 @pytest.mark.parametrize("M,N,K,gelu,most", [(24576, 1536, 384, True, 1.1), (12288, 1024, 256, True, 1.07), (4096, 4096, 1024, False, 0.93)])

@@ -183,8 +183,8 @@ def stores(args):
 
 
 # configuration codes of the tiled GEMM kernel, tnn_rocm_debug_set_gemm_config
-TILE_CODES = {"half": (6111141, 6211141, 6121141, 9111141, 9121141, 3112221, 3212221, 2112211, 8222222, 8322222, 8332222, 8422222,
-                       2222221, 3332221, 2244211),
+TILE_CODES = {"half": (6111141, 6211141, 6121141, 9111141, 9121141, 3112221, 2112211, 8222222, 8322222, 8332222, 8422222,
+                       7244211, 8244211, 8264211, 8344211, 8364211, 8444211, 2244211),
               "fp32": (6111141, 6211141, 6121141, 6111181, 6211181, 9111141, 9121141, 9111181, 9221141, 2321142, 2231142,
                        2331142, 2222121, 2222221, 2332121)}
 
@@ -210,6 +210,8 @@ def tiles(args):
     _time_forward(inst, args.steps)
     for proj, n, k in (("qkv", 3 * H, H), ("out", H, H), ("ffn1", F, H), ("ffn2", H, F)):
         codes = [c for c in TILE_CODES["fp32" if args.precision == "fp32" else "half"] if k * size % (64 << c % 10) == 0]
+        if args.precision == "int8":
+            codes = [c for c in codes if c not in (8264211, 8444211)]
         diff = {c: [] for c in codes}
         try:
             for _ in range(rounds):

@@ -188,8 +188,9 @@ def mall_probe(launches=20):
 # (code, rows, columns, tiles a CU holds at once) of the shapes the launcher chooses from, see TileCost in csrc/gemm_kernels.h
 TILE_SHAPES = {
     "half": ((6111141, 16, 16, 3), (6211141, 32, 16, 2), (6121141, 16, 32, 2), (9111141, 32, 32, 2), (9121141, 32, 64, 1),
-             (3112221, 64, 64, 3), (3212221, 128, 64, 2), (2112211, 64, 64, 4), (8222222, 64, 64, 1), (8322222, 96, 64, 1),
-             (8332222, 96, 96, 1), (8422222, 128, 64, 1), (2222221, 128, 128, 2), (3332221, 192, 192, 1), (2244211, 256, 256, 1)),
+             (3112221, 64, 64, 3), (2112211, 64, 64, 4), (8222222, 64, 64, 1), (8322222, 96, 64, 1), (8332222, 96, 96, 1),
+             (8422222, 128, 64, 1), (7244211, 128, 128, 2), (8244211, 128, 128, 1), (8264211, 128, 192, 1), (8344211, 192, 128, 1),
+             (8364211, 192, 192, 1), (8444211, 256, 128, 1), (2244211, 256, 256, 1)),
     "f32": ((6111141, 16, 16, 3), (6211141, 32, 16, 2), (6121141, 16, 32, 2), (6111181, 16, 16, 1), (6211181, 32, 16, 1),
             (9111141, 32, 32, 2), (9121141, 32, 64, 1), (9111181, 32, 32, 1), (9221141, 64, 64, 1), (2321142, 96, 64, 1),
             (2231142, 64, 96, 1), (2331142, 96, 96, 1), (2222121, 128, 64, 2), (2222221, 128, 128, 1), (2332121, 192, 96, 1))}
@@ -203,6 +204,8 @@ def tile_sweep(dtype, report, rows=()):
     import numpy as np
     lib = capi.load()
     shapes = TILE_SHAPES["f32" if dtype == "f32" else "half"]
+    if dtype == "i8":
+        shapes = tuple(s for s in shapes if s[0] not in (8264211, 8444211))
     td, size = {"f16": (torch.float16, 2), "i8": (torch.int8, 1), "f32": (torch.float32, 4)}[dtype]
     ms = tuple(rows) or (16, 32, 64, 100, 128, 197, 256, 384, 512, 700, 1000, 1536, 2000, 3072) + (() if dtype == "f32" else (4096, 8192))
     seen, behind = {s[0]: [] for s in shapes}, []

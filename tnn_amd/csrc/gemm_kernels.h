@@ -1096,18 +1096,11 @@ template <int TM_, int TN_, int WGM_, int WGN_, int WGK_, int SLAB_, int NSTAGE_
     static constexpr size_t slab_bytes  = (size_t)(NSTAGE_ ? NSTAGE_ : 2) * (BM + BN) * STRIDE * (OWN_ ? WGK_ : 1);
     static constexpr size_t stage_bytes = (size_t)WGM_ * WGN_ * WGK_ * GROWS * SSTR * 4;
     static constexpr size_t lds_bytes   = slab_bytes > stage_bytes ? slab_bytes : stage_bytes;
-    // where an epilogue that leaves row sums keeps its BM x BN / 8 pairs: in the part of the slab area the staging does
-    // not reach when that is large enough (dead by then), else behind everything
-    // Where the whole tile is staged at once, an item's pair goes into the place of its own staged values.
-    static constexpr bool sums_in_place = GROUPS == 1 && !OWN_;
-    static constexpr size_t sums_bytes  = sums_in_place ? 0 : (size_t)BM * BN;
-    static constexpr size_t sums_offset = (slab_bytes >= stage_bytes + sums_bytes) ? stage_bytes : lds_bytes;
-    // ... unless there is no such part and a row of a wave's columns lies in eight neighbouring lanes: the lanes then add up
-    // the sums of each wave's columns among themselves (128 x 128: 16 KB of LDS would cost the CU's second workgroup)
-    // or where all columns are one wave's anyway (32 x 32 tiles with rings of their own, 256 x 768 x 768: 4.60 -> 4.40 us against
-    // sums through LDS, a barrier and a loop over them)
-    static constexpr bool sums_by_lanes = OWN_ || (BLK_ == 32 && TN_ == 2 && !(slab_bytes >= stage_bytes + sums_bytes));
-    static constexpr int sum_cols       = sums_by_lanes ? BLK_ * TN_ : BN;  // columns behind one pair of row sums
+    // Row sums of what an epilogue stored.  Where all columns are one wave's they are added up over the two to eight lanes that hold a
+    // row (32 x 32 tiles, 256 x 768 x 768: 4.60 -> 4.40 us against sums through LDS); elsewhere an item's pair goes into the place of its
+    // own staged values, which takes the whole tile staged at once.
+    static constexpr bool sums_by_lanes = OWN_;
+    static constexpr bool leaves_sums   = OWN_ || GROUPS == 1;
     static constexpr int NW = WGM * WGN * WGK, NT = 64 * NW;  // waves and threads per workgroup
     static_assert(NW == 4 || NW == 8, "four or eight waves per workgroup");
     static_assert(OWN_ || ((BM * (SLAB / 16)) % NT == 0 && (BN * (SLAB / 16)) % NT == 0), "slab must divide over the workgroup");
@@ -1126,11 +1119,7 @@ template <typename CFG, typename Epi> struct EpiLds {
     // behind the slabs before the main loop
     static constexpr size_t base1 = TakesRowSums<Epi>::value ? CFG::lds_bytes + (size_t)CFG::BM * 8
                                     : (Epi::kRowStats && stats_need > base0) ? stats_need : base0;
-    // without / with the row-sum side output (eight bytes per eight columns and row)
-    static constexpr size_t plain     = base1;
-    static constexpr size_t with_sums = CFG::sums_offset + CFG::sums_bytes > base1 ? CFG::sums_offset + CFG::sums_bytes : base1;
-    static constexpr size_t front      = EmitsRowSums<Epi>::value && !CFG::sums_by_lanes ? with_sums : plain;
-    static constexpr size_t col_offset = (front + 15) & ~(size_t)15;
+    static constexpr size_t col_offset = (base1 + 15) & ~(size_t)15;
     static constexpr size_t row_offset = col_offset + (size_t)ColArrays<Epi>::value * CFG::BN * 4;
     static constexpr size_t side_bytes = (size_t)ColArrays<Epi>::value * CFG::BN * 4 + (RowIn<Epi>::value ? (size_t)CFG::BM * 8 : 0);
     static constexpr size_t total      = col_offset + side_bytes;
@@ -1664,11 +1653,8 @@ __global__ void __launch_bounds__(CFG::NT)
         // Large wave tiles with more than one step a slab: step s + 1's fragments are read between the MFMAs of step s, and so are
         // the first ones of the next slab, whose barrier stands in front of the last step.  Read behind the barrier, they are a
         // burst of all waves' reads that no MFMA covers (256 x 256: 48 KB, 380 of 2400 clocks a slab).  fp16, us, burst -> this:
-        // 192 x 192 tiles 3072 x 3072 x 768 23.0 -> 22.6, 3072 x 768 x 3072 45.9 -> 39.2; 256 x 256 tiles 8192 x 4096 x 4096
-        // 239 -> 228.  Not where two workgroups share a CU and cover each other: 128 x 128 tiles gain back to back
-        // (3072 x 2304 x 768 18.9 -> 18.1), but with operands that come from the memory-side cache, as in a network, they lose
-        // (17.5 -> 17.7; twelve layers of 8 x 384 tokens 1134 -> 1145 us over eight instances).  Waves with one block have
-        // nothing to hide the reads behind: 64 x 64 tiles 256 x 3072 x 768 6.3 -> 6.6, four waves 985 x 2304 x 768 9.7 -> 10.1.
+        // 256 x 256 tiles 8192 x 4096 x 4096 239 -> 228.  Waves with one block of 32 x 32 have nothing to hide the reads behind: 64 x 64
+        // tiles 256 x 3072 x 768 6.3 -> 6.6, four waves 985 x 2304 x 768 9.7 -> 10.1.
         constexpr bool PIPE = DT != TNN_ROCM_F32 && CFG::NW == 8 && KSTEPS >= 2 && (TM * TN > 4 || BLK == 16);
         static_assert(!PIPE || KSTEPS % 2 == 0, "two sets of fragments, every slab begins with the first");
         if constexpr (TakesRowSums<Epi>::value && !kLateSums)
@@ -2158,12 +2144,9 @@ __global__ void __launch_bounds__(CFG::NT)
                     sm.x = add_neighbours<CPR>(sm.x);
                     sm.y = add_neighbours<CPR>(sm.y);
                     if (piece == 0 && m < M && n < N)
-                        store_out8(epi.through, &epi.row_sums[(size_t)(n / CFG::sum_cols) * M + m], sm);
-                } else if constexpr (CFG::sums_in_place) {
-                    *reinterpret_cast<float2 *>(const_cast<AccT *>(src)) = sm;
+                        store_out8(epi.through, &epi.row_sums[(size_t)(n / BN) * M + m], sm);
                 } else {
-                    reinterpret_cast<float2 *>(lds_dyn + CFG::sums_offset)[(((pos / WGN) * GROUPS + i) * GROWS + row) * (BN / 8) +
-                                                                         ((pos % WGN) * CW + c8) / 8] = sm;
+                    *reinterpret_cast<float2 *>(const_cast<AccT *>(src)) = sm;
                 }
             } else if (m < M) {
                 AccT v[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
@@ -2202,13 +2185,8 @@ __global__ void __launch_bounds__(CFG::NT)
             float s1 = 0.f, s2 = 0.f;
 #pragma unroll
             for (int q = 0; q < BN / 8; ++q) {
-                float2 part;
-                if constexpr (CFG::sums_in_place) {
-                    const int pos = tid / GROWS * WGN + q / CPR;
-                    part = *reinterpret_cast<const float2 *>(stage_all + (pos * WGK) * (GROWS * SSTR) + tid % GROWS * SSTR + q % CPR * 8);
-                } else {
-                    part = reinterpret_cast<const float2 *>(lds_dyn + CFG::sums_offset)[tid * (BN / 8) + q];
-                }
+                const int pos = tid / GROWS * WGN + q / CPR;
+                const float2 part = *reinterpret_cast<const float2 *>(stage_all + (pos * WGK) * (GROWS * SSTR) + tid % GROWS * SSTR + q % CPR * 8);
                 s1 += part.x, s2 += part.y;
             }
             store_out8(epi.through, &epi.row_sums[(size_t)(n0 / BN) * M + m0 + tid], make_float2(s1, s2));
@@ -2258,21 +2236,14 @@ constexpr int kNotWithRowSums = -12345;
 thread_local int t_last_sum_blocks = 0;  // row-sum blocks of this thread's last tiled launch
 
 template <int DT, typename CFG, typename Epi>
-int launch_tiled(hipStream_t s, const void *A, const void *B, int M, int N, int K, long lda, long ldb, const Epi &epi) {
+int launch_shape(hipStream_t s, const void *A, const void *B, int M, int N, int K, long lda, long ldb, const Epi &epi) {
     typedef typename GemmTraits<DT>::elem T;
     int tiles_m = (M + CFG::BM - 1) / CFG::BM, tiles_n = (N + CFG::BN - 1) / CFG::BN;
     typedef EpiLds<CFG, Epi> L;
     const size_t lds = L::total;
-    const int sum_blocks = (N + CFG::sum_cols - 1) / CFG::sum_cols;
+    const int sum_blocks = tiles_n;
     if (EmitsRowSums<Epi>::value && sum_blocks > kMaxRowSumBlocks)
         return kNotWithRowSums;
-    if (EmitsRowSums<Epi>::value && !CFG::sums_by_lanes) {
-        // the row sums are not taken at the price of a workgroup per CU (the plain form runs instead)
-        const size_t without = L::plain + L::side_bytes + 16;
-        const long cu = 160 * 1024;
-        if (lds > (size_t)cu || cu / (long)(lds + 1024) < (cu / (long)(without + 1024) > 4 ? 4 : cu / (long)(without + 1024)))
-            return kNotWithRowSums;
-    }
     auto kern   = gemm_nk_tiled_kernel<DT, CFG, Epi>;
     if (lds > 64 * 1024) {
         // the attribute belongs to the (kernel, device) pair: one bit per device, per instantiation
@@ -2309,17 +2280,26 @@ int launch_tiled(hipStream_t s, const void *A, const void *B, int M, int N, int 
     return 0;
 }
 
+template <int DT, typename CFG, typename Epi>
+int launch_tiled(hipStream_t s, const void *A, const void *B, int M, int N, int K, long lda, long ldb, const Epi &epi) {
+    if constexpr (EmitsRowSums<Epi>::value && !CFG::leaves_sums)
+        return kNotWithRowSums;
+    else
+        return launch_shape<DT, CFG, Epi>(s, A, B, M, N, K, lda, ldb, epi);
+}
+
 // Configuration codes: [P] TM TN WGM WGN WGK S (one decimal digit each; slab bytes = 64 << S; P = number of
 // direct-to-LDS stages, 9 = rings of the waves' own, absent = slabs staged through registers).
 //   9111141   32 x  32, 4 k-waves with rings of their own     9121141   32 x  64, likewise
-//   3112221   64 x  64, 8 waves (two k-waves), 3 stages       3212221  128 x  64, 8 waves
 //   6111141   16 x  16, 6211141 32 x 16, 6121141 16 x 32: 16 x 16 blocks, 4 k-waves with rings of their own (three slabs)
-//   8222222   64 x  64, 8322222 96 x 64, 8332222 96 x 96, 8422222 128 x 64: 16 x 16 blocks, 8 waves (two k-waves), 3 stages of 256 bytes
-//   2112211   64 x  64, 4 waves, 2 stages                     2222221  128 x 128, 8 waves (two k-waves)
-//   fp32 only: 6111181, 6211181 16 x 16 and 32 x 16, 8 k-waves; 9111181 32 x 32, 8 k-waves; 9221141 64 x 64, 4 k-waves with rings of their own;
-//   2321142, 2231142, 2331142 96 x 64, 64 x 96 and 96 x 96, 4 k-waves; 2222121, 2332121 128 x 64 and 192 x 96, 4 waves (two k-waves)
+//   3112221   64 x  64, 8 waves (two k-waves), 3 stages       2112211   64 x  64, 4 waves, 2 stages
+//   7 and 8 (two and three stages): 16 x 16 blocks, 8 waves that share the slabs
+//   8222222   64 x  64, 8322222 96 x 64, 8332222 96 x 96, 8422222 128 x 64: 2 x 2 positions and two k-waves, 256-byte slabs
+//   7244211  128 x 128, 8244211 128 x 128, 8344211 192 x 128, 8364211 192 x 192: 4 x 2 positions; not int8: 8264211 128 x 192, 8444211 256 x 128
 //   2244211  256 x 256, 8 waves
-//   3332221  192 x 192, 8 waves (two k-waves)
+//   fp32 only: 6111181, 6211181 16 x 16 and 32 x 16, 8 k-waves; 9111181 32 x 32, 8 k-waves; 9221141 64 x 64, 4 k-waves with rings of their own;
+//   2321142, 2231142, 2331142 96 x 64, 64 x 96 and 96 x 96, 4 k-waves; 2222121, 2332121 128 x 64 and 192 x 96, 4 waves (two k-waves);
+//   2222221 128 x 128, 8 waves (two k-waves)
 //   112210    64 x  64 and 222210 128 x 128, 4 waves: rows that are no multiple of 128 bytes
 // Eight-wave workgroups put two waves on every SIMD inside one tile: while one waits for its LDS fragments the
 // other issues MFMAs, and a larger tile per CU moves fewer bytes through LDS and L2 per flop.  Four-wave tiles
@@ -2332,11 +2312,11 @@ int launch_tiled(hipStream_t s, const void *A, const void *B, int M, int N, int 
 // int8: M from 16 to 8192, the four projections of hidden sizes 768 and 1024 with their fused epilogues; fp32: M from 16 to
 // 3072), taken over twelve weight sets in turn so that weights come from the memory-side cache as they do inside a network:
 // python -m tnn_amd.bench_ops --tile-sweep measures them and fits the rows.  A launch is 3 .. 20 % off its prediction on average,
-// by shape (the large ones most), so picks closer than that are as good as drawn.  Taken together the picks are 0.6 % (fp16), 0.9 %
-// (int8), 1.0 % (fp32) behind the best shape of each launch back to back (256 launches each of fp16 and int8, of which half had no
-// part in the fit).  Not as the sweep fits them: the 256 x 256 rows (below), the 192 x 192 row of the half table, which is of
-// before its loop read ahead, the rows of 16 x 16 blocks of a shared slab (below), and in the int8 table what the comment above
-// it says.  The rules this replaced, made for M >= 1024, were 51 %, 34 % and 77 % behind:
+// by shape (the large ones most), so picks closer than that are as good as drawn.  The half and int8 rows were then moved as little
+// as it took for few launches to be slower than with the tables and shapes before them: over 584 launches of each type (hidden sizes
+// 256 to 2048, M from 16 to 12288) the picks are 0.4 % (fp16) and 0.5 % (int8) behind the best shape of each, and 7 % and 8 % faster than
+// before; of the 392 compared 11 and 16 are more than 2 % slower, one and three more than 5 (8192 x 2048 x 8192 by 10).  fp32: 1.0 % behind.
+// The rules this replaced, made for M >= 1024, were 51 %, 34 % and 77 % behind:
 //   M=  32 N= 768 K=3072 fp16  23.1 -> 7.3 us   (64x64 tiles: 12 CUs, one two-stage slab after another)
 //   M= 256 N= 768 K=3072 fp16  23.7 -> 7.2      M= 256 N=2304 K=768 fp16  8.7 -> 6.2
 //   M=1000 N= 768 K=3072 fp16  24.3 -> 12.4     M=1000 N= 768 K=768 fp16  8.7 -> 5.5
@@ -2345,21 +2325,24 @@ struct TileCost {
     float fixed, round, slab[4];
 };
 constexpr TileCost kTilesHalf[] = {
-    {6111141, 16, 16, 3, 3.51f, 1.75f, {0.027f, 0.068f, 0.093f}},
-    {6211141, 32, 16, 2, 3.56f, 2.22f, {0.042f, 0.088f}},
-    {6121141, 16, 32, 2, 3.68f, 1.95f, {0.046f, 0.093f}},
-    {9111141, 32, 32, 2, 3.47f, 2.09f, {0.067f, 0.147f}},
-    {9121141, 32, 64, 1, 3.46f, 2.56f, {0.121f}},
-    {3112221, 64, 64, 3, 3.72f, 3.06f, {0.205f, 0.377f, 0.654f}},
-    {3212221, 128, 64, 2, 4.60f, 5.12f, {0.287f, 0.607f}},
-    {2112211, 64, 64, 4, 2.96f, 1.83f, {0.411f, 0.493f, 0.607f, 0.877f}},
-    {2222221, 128, 128, 2, 4.84f, 5.77f, {0.561f, 1.044f}},
-    {3332221, 192, 192, 1, 10.15f, 13.25f, {0.767f}},
-    {8222222, 64, 64, 1, 3.70f, 2.89f, {0.145f}},
-    {8322222, 96, 64, 1, 4.32f, 3.75f, {0.205f}},
-    {8332222, 96, 96, 1, 5.06f, 5.33f, {0.242f}},
-    {8422222, 128, 64, 1, 4.45f, 4.28f, {0.243f}},
-    {2244211, 256, 256, 1, 10.5f, 12.0f, {1.5f}},
+    {6111141, 16, 16, 3, 3.45f, 1.51f, {0.027f, 0.067f, 0.092f}},
+    {6211141, 32, 16, 2, 3.43f, 2.01f, {0.040f, 0.089f}},
+    {6121141, 16, 32, 2, 3.37f, 1.74f, {0.046f, 0.095f}},
+    {9111141, 32, 32, 2, 3.39f, 1.89f, {0.064f, 0.139f}},
+    {9121141, 32, 64, 1, 3.54f, 2.58f, {0.113f}},
+    {3112221, 64, 64, 3, 3.86f, 2.73f, {0.207f, 0.344f, 0.616f}},
+    {2112211, 64, 64, 4, 3.04f, 1.86f, {0.411f, 0.480f, 0.573f, 0.855f}},
+    {8222222, 64, 64, 1, 3.69f, 2.83f, {0.154f}},
+    {8322222, 96, 64, 1, 4.38f, 3.65f, {0.192f}},
+    {8332222, 96, 96, 1, 5.21f, 5.31f, {0.242f}},
+    {8422222, 128, 64, 1, 4.48f, 4.16f, {0.239f}},
+    {7244211, 128, 128, 2, 3.87f, 6.00f, {0.594f, 0.920f}},
+    {8244211, 128, 128, 1, 4.81f, 6.73f, {0.358f}},
+    {8264211, 128, 192, 1, 7.38f, 10.11f, {0.482f}},
+    {8344211, 192, 128, 1, 6.59f, 8.74f, {0.465f}},
+    {8364211, 192, 192, 1, 8.80f, 12.52f, {0.666f}},
+    {8444211, 256, 128, 1, 7.77f, 11.65f, {0.596f}},
+    {2244211, 256, 256, 1, 10.50f, 12.00f, {1.255f}},
 };
 // 256 x 256 tiles are for products that fill the chip with them: half the bytes a flop of 128 x 128 tiles.  A linear model knows
 // neither that a round of 192 tiles is 13 % shorter than one of 256 nor what the epilogue leaves uncovered, so their row and the
@@ -2371,41 +2354,42 @@ constexpr TileCost kTilesHalf[] = {
 // picks that are slower cost 25 % together (187 % with the old row), the shape where it is left out and faster 88 % (99 %).  The int8
 // row is set by hand: of its picks three of 60 are slower, 24576 x 1920 x 640 into Q, K and V^T by 6 % and [16384, 1024] x 1024 and
 // 24576 x 1280 x 1280 with a residual by 3 %.
-// 16 x 16 blocks of a shared slab, 64 x 64 to 128 x 64: eight waves as 2 x 2 positions and two k-waves, so that a tile of any number of
-// 32 rows and columns is dealt out evenly.  96 x 96 as eight k-waves of 3 x 3 blocks of 32 x 32 passed 295 KB of partial sums
-// through LDS behind its loop (half of the 11 us of 3072 x 768 x 768), now 74; 96 x 64 is one round of the chip where 64 x 64 are
-// two.  Their rows are the fit's, moved until no launch of the sweep that changed its shape for them is slower (of 512 two are, by
-// 3 %).  fp16 launches are 2.9 % faster on average and by up to 24 %, int8 1.4 % and 21 %.  us, the picks before -> these:
+// 16 x 16 blocks of a shared slab.  Up to 128 x 64: eight waves as 2 x 2 positions and two k-waves, so that a tile of any number of 32
+// rows and columns is dealt out evenly.  96 x 96 as eight k-waves of 3 x 3 blocks of 32 x 32 passed 295 KB of partial sums through
+// LDS behind its loop (half of the 11 us of 3072 x 768 x 768), now 74; 96 x 64 is one round of the chip where 64 x 64 are two.
+// From 128 x 128 on: 4 x 2 positions and no k-waves.  The waves' blocks are longer than high, which costs a third more LDS reads than
+// square ones, but the sums pass through LDS once instead of twice, the fragments of a step are read under the products of
+// the step before, across the slab's barrier too, and 128 x 128 take 36 registers for sums instead of 64.  us, the picks before -> these:
 //   fp16 3072 x 768 x 768 10.9 -> 8.8, 3072 x 768 x 3072 22.9 -> 20.1, 1536 x 768 x 3072 18.8 -> 14.5, 984 x 768 x 3072 13.0 -> 11.8,
-//   700 x 3072 x 768 10.9 -> 8.3, 1536 x 1024 x 4096 23.1 -> 18.1; int8 1536 x 768 x 3072 11.8 -> 9.3, 3072 x 768 x 3072 15.5 -> 13.2
-// (Not taken: 64 x 96, 32 x 64, 64 x 32, 32 x 96, 64 x 128, within 0.1 % of the sweep together; two stages instead of three, 96 x 96 8.9 ->
-// 9.9; four k-waves, 96 x 96 9.1 -> 9.4.)
+//   700 x 3072 x 768 10.9 -> 8.3, 3072 x 3072 x 768 22.9 -> 21.1, 2048 x 2304 x 768 16.9 -> 14.4, 8192 x 3072 x 1024 77.2 -> 70.8,
+//   8192 x 1024 x 4096 79.7 -> 70.7; int8 1536 x 768 x 3072 11.8 -> 9.3, 3072 x 768 x 3072 15.5 -> 13.2
+// Over the sweeps fp16 launches take 0.944, int8 ones 0.970 of what they did with 32 x 32 blocks.  (Not taken: 64 x 96, 32 x 64, 64 x 32,
+// 32 x 96, 64 x 128 with two k-waves, 0.1 % of the sweep together; 96 x 96 with two stages 8.9 -> 9.9 or four k-waves 9.1 -> 9.4;
+// 128 x 64 and 192 x 96 with 4 x 2 positions, 0.1 % together; 128 x 256, the same as 256 x 128.)
 // Tiles of 16 x 16 blocks with rings of the waves' own are for the products whose 32x32 tiles are too few for the chip: a CU's panels come through its L1 at
 // 64 bytes a clock at best, so 24 tiles of (32 + 32) rows of K=3072 take 4 us for that alone, and 96 of (16 + 16) rows half.
 // us a launch, best shape before -> now (fp32: 8 waves where K is long):
 //   M= 32 N= 768 K=3072 fp16  7.4 -> 5.0   int8 5.0 -> 4.1   fp32 14.9 -> 8.8     M= 32 N=768 K=768 fp16 3.9 -> 3.2, fp32 6.4 -> 4.6
 //   M=128 N= 768 K=3072 fp16  7.5 -> 6.0   int8 5.4 -> 4.7   fp32 14.9 -> 12.1    M=128 N=768 K=768 fp16 4.3 -> 3.5, fp32 6.7 -> 5.8
 //   M= 32 N=2304 K=768  fp16  4.7 -> 4.5 (folded LayerNorm)  fp32  6.7 -> 5.9
-// (Measured and not taken: eight waves for fp16 and int8, 0.1 .. 0.4 us behind; rings of four slabs, 0.1 behind.  The int8 rows'
-// fixed part is 0.2 us below its fit: the other int8 rows were fitted on a faster machine.)
-// (int8, 64x64 tiles: the slab of four tiles was fitted to 0.944; 4096 x 2304 x 768 then took 128x128 tiles, 1.4 % ahead by the
-// fit and 0 .. 1 us a launch behind in the network)
+// (Measured and not taken: eight waves for fp16 and int8, 0.1 .. 0.4 us behind; rings of four slabs, 0.1 behind.)
 constexpr TileCost kTilesI8[] = {
-    {6111141, 16, 16, 3, 3.10f, 1.66f, {0.036f, 0.078f, 0.087f}},
-    {6211141, 32, 16, 2, 3.10f, 1.71f, {0.052f, 0.097f}},
-    {6121141, 16, 32, 2, 3.10f, 1.69f, {0.053f, 0.095f}},
-    {9111141, 32, 32, 2, 2.98f, 1.93f, {0.078f, 0.151f}},
-    {9121141, 32, 64, 1, 3.25f, 2.21f, {0.130f}},
-    {3112221, 64, 64, 3, 3.40f, 2.05f, {0.218f, 0.398f, 0.701f}},
-    {3212221, 128, 64, 2, 4.05f, 3.04f, {0.313f, 0.644f}},
-    {2112211, 64, 64, 4, 3.00f, 1.56f, {0.424f, 0.558f, 0.687f, 0.916f}},
-    {2222221, 128, 128, 2, 5.15f, 3.79f, {0.640f, 1.156f}},
-    {3332221, 192, 192, 1, 9.89f, 9.10f, {0.860f}},
-    {8222222, 64, 64, 1, 3.23f, 2.32f, {0.162f}},
-    {8322222, 96, 64, 1, 4.20f, 5.50f, {0.212f}},
-    {8332222, 96, 96, 1, 5.62f, 4.51f, {0.276f}},
-    {8422222, 128, 64, 1, 4.46f, 4.15f, {0.261f}},
-    {2244211, 256, 256, 1, 10.6f, 8.2f, {2.1f}},
+    {6111141, 16, 16, 3, 3.21f, 1.59f, {0.031f, 0.071f, 0.084f}},
+    {6211141, 32, 16, 2, 3.17f, 1.60f, {0.047f, 0.093f}},
+    {6121141, 16, 32, 2, 3.13f, 1.58f, {0.051f, 0.092f}},
+    {9111141, 32, 32, 2, 3.17f, 1.63f, {0.070f, 0.139f}},
+    {9121141, 32, 64, 1, 3.29f, 2.09f, {0.123f}},
+    {3112221, 64, 64, 3, 3.25f, 1.79f, {0.210f, 0.375f, 0.655f}},
+    {2112211, 64, 64, 4, 2.68f, 1.77f, {0.426f, 0.565f, 0.562f, 0.874f}},
+    {8222222, 64, 64, 1, 3.20f, 2.27f, {0.165f}},
+    {8322222, 96, 64, 1, 3.92f, 3.17f, {0.206f}},
+    {8332222, 96, 96, 1, 4.96f, 4.41f, {0.271f}},
+    {8422222, 128, 64, 1, 3.66f, 3.60f, {0.271f}},
+    {7244211, 128, 128, 2, 3.92f, 3.61f, {0.632f, 1.148f}},
+    {8244211, 128, 128, 1, 4.99f, 12.00f, {0.418f}},
+    {8344211, 192, 128, 1, 6.60f, 9.50f, {0.543f}},
+    {8364211, 192, 192, 1, 8.95f, 12.02f, {0.850f}},
+    {2244211, 256, 256, 1, 10.50f, 8.20f, {2.049f}},
 };
 // fp32 on three bf16 planes: six matrix instructions per operand pair and the conversion between them, so a step costs five
 // times a half one.  Large wave tiles convert less per product, K is split over the waves of a CU wherever tiles are few, and
@@ -2449,7 +2433,7 @@ inline int pick_tile_config(const TileCost (&shapes)[COUNT], long M, long N, siz
         const long sets = n / t.slots, rest = n % t.slots;
         float cost = t.fixed + slabs * ((float)sets * t.slab[t.slots - 1] + (rest ? t.slab[rest - 1] : 0.f)) +
                      t.round * (float)(sets + (rest ? 1 : 0) - 1) + (row_stats && t.code / 100000 == 62 ? 0.4f : 0.f) +
-                     (t.bm == 256 ? wide_us * (float)n : 0.f);
+                     (t.bm == 256 && t.bn == 256 ? wide_us * (float)n : 0.f);
         if (best == 0 || cost < best_cost)
             best = t.code, best_cost = cost;
     }
@@ -2480,11 +2464,19 @@ int launch_gemm_fast(hipStream_t s, const void *A, const void *B, int M, int N, 
         case 222221:
         case 224211: cfg = 2222221; break;
         case 332221: cfg = 3332221; break;
-        case 331182:
-        case 3331182: cfg = 8332222; break;  // the shapes that these blocks took the place of
-        case 4221141:
-        case 3112222: cfg = 8222222; break;
+        case 331182: cfg = 3331182; break;
         default: break;
+    }
+    if constexpr (DT != TNN_ROCM_F32) {
+        switch (cfg) {  // the code of a shape whose tile is made of 16 x 16 blocks now
+            case 3212221:
+            case 2222221: cfg = 7244211; break;
+            case 3332221: cfg = 8364211; break;
+            case 3331182: cfg = 8332222; break;
+            case 4221141:
+            case 3112222: cfg = 8222222; break;
+            default: break;
+        }
     }
     if (kbytes % (64u << (cfg % 10)) != 0) {
         set_error("gemm: K=%d is not a whole number of slabs for tuning configuration %d", K, cfg);
@@ -2539,15 +2531,23 @@ int launch_gemm_fast(hipStream_t s, const void *A, const void *B, int M, int N, 
         switch (cfg) {
             case 2112211: TR_FAST_DL(1, 1, 2, 2, 1, 128, 2);
             case 3112221: TR_FAST_DL(1, 1, 2, 2, 2, 128, 3);
-            case 3212221: TR_FAST_DL(2, 1, 2, 2, 2, 128, 3);
-            case 2222221: TR_FAST_DL(2, 2, 2, 2, 2, 128, 2);
-            case 3332221: TR_FAST_DL(3, 3, 2, 2, 2, 128, 3);
+            case 7244211: TR_FAST_DL16(2, 4, 4, 2, 1, 128, 2);
+            case 8244211: TR_FAST_DL16(2, 4, 4, 2, 1, 128, 3);
+            case 8344211: TR_FAST_DL16(3, 4, 4, 2, 1, 128, 3);
+            case 8364211: TR_FAST_DL16(3, 6, 4, 2, 1, 128, 3);
             case 2244211: TR_FAST_DL(2, 4, 4, 2, 1, 128, 2);
             case 8222222: TR_FAST_DL16(2, 2, 2, 2, 2, 256, 3);
             case 8322222: TR_FAST_DL16(3, 2, 2, 2, 2, 256, 3);
             case 8332222: TR_FAST_DL16(3, 3, 2, 2, 2, 256, 3);
             case 8422222: TR_FAST_DL16(4, 2, 2, 2, 2, 256, 3);
             default: break;
+        }
+        if constexpr (DT != TNN_ROCM_I8) {
+            switch (cfg) {
+                case 8264211: TR_FAST_DL16(2, 6, 4, 2, 1, 128, 3);
+                case 8444211: TR_FAST_DL16(4, 4, 4, 2, 1, 128, 3);
+                default: break;
+            }
         }
     }
     if constexpr (!Epi::kRowStats) {  // the LayerNorm-folding epilogues exist for the direct-to-LDS pipelines only
