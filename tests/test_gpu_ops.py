@@ -232,6 +232,31 @@ def test_layernorm_row_count_changes_nothing(dtype, vecs):
         assert rel_err(host(y[:3].float()), ref) <= {"float32": 2e-6, "float16": 2e-3, "bfloat16": 1.6e-2}[dtype]
 
 
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
+@pytest.mark.parametrize("cols", [256, 264, 504, 512, 520, 760, 768, 776, 1016, 1024, 1032])
+def test_embed_layernorm_row_count_changes_nothing(dtype, cols):
+    """Up to 3072 half rows of 257 to 1024 columns a wave owns a row in vectors of 8 bytes, beyond half a wave in vectors of 16: the same
+    bits on both sides of the line, for looked-up rows and for stored ones, and the formula in float64 to a rounding of the type."""
+    say("embed_layernorm %s, rows of %d" % (dtype, cols))
+    td, rows, vocab = getattr(torch, dtype), 3073, 700
+    gen = torch.Generator(device="cuda").manual_seed(cols)
+    word, types, pos = (torch.randn(n, cols, device="cuda", generator=gen).to(td) for n in (vocab, 2, 512))
+    g, b = (torch.randn(cols, device="cuda", generator=gen) for _ in range(2))
+    ids = torch.randint(0, vocab, (1, rows), device="cuda", generator=gen, dtype=torch.int32)
+    seg, at = ids % 2, torch.arange(rows, device="cuda", dtype=torch.int32).view(1, -1) % 512
+    y, flag = ops().embed_layernorm(ids, seg, word, types, pos, g, b, 1e-5, pos_ids=at)
+    assert int(flag.item()) == 0
+    t = (word[ids[0].long()].float() + pos[at[0].long()].float()) + types[seg[0].long()].float()
+    for lo, hi in ((0, 3072), (1, 3073), (0, 1), (3070, 3073), (5, 518)):
+        part, flag = ops().embed_layernorm(*(i[:, lo:hi].contiguous() for i in (ids, seg)), word, types, pos, g, b, 1e-5,
+                                           pos_ids=at[:, lo:hi].contiguous())
+        assert int(flag.item()) == 0 and torch.equal(part, y[lo:hi]), (lo, hi)
+    ref = torch.nn.functional.layer_norm(t.double(), (cols,), g.double(), b.double(), 1e-5)
+    # the affine combination in fp32 (a few ulp of the terms), then one rounding to the type
+    ulp = 2.0 ** -11 if dtype == "float16" else 2.0 ** -8
+    assert ((y.double() - ref).abs() <= ulp * ref.abs() + 1e-5).all()
+
+
 def _device_us(fns, launches=10, replays=5):
     """us a launch of each function, in graphs of `launches` that take turns: the best replay of each"""
     graphs = []

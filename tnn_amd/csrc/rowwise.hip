@@ -53,7 +53,8 @@ struct EmbedRows {
 // bytes in flight for rows of at most 128 vectors); NV = 16-byte vectors a lane can hold.
 // AHEAD: everything the row needs is requested at once, scale and shift among it.  Requested where they are used they are a
 // second latency behind the reduction; the registers they take meanwhile cost resident waves.
-template <int DT, bool VECTOR, int LPR, int NV, bool AHEAD>
+// VB: bytes of a vector, 16 or, for half types, 8.
+template <int DT, bool VECTOR, int LPR, int NV, bool AHEAD, int VB = 16>
 __global__ void __launch_bounds__(kBlock) layernorm_kernel(const typename Elem<DT>::type *__restrict__ x,
                                                            const typename Elem<DT>::type *__restrict__ res,
                                                            const float *__restrict__ gamma,
@@ -63,7 +64,8 @@ __global__ void __launch_bounds__(kBlock) layernorm_kernel(const typename Elem<D
                                                            EmbedRows emb, StoreThrough mode) {
     typedef typename Elem<DT>::type T;
     touch_kernel_args<7 * 8 + 3 * 8 + sizeof(EmbedRows)>();
-    constexpr int VEC = VECTOR ? (int)(16 / sizeof(T)) : 1;
+    typedef typename std::conditional<VB == 16, uint4, uint2>::type Raw;
+    constexpr int VEC = VECTOR ? (int)(VB / sizeof(T)) : 1;
     const int lane    = threadIdx.x & (LPR - 1);
     const int row     = (blockIdx.x * kRowsPerBlk + (threadIdx.x >> 6)) * (kWave / LPR) + ((threadIdx.x & (kWave - 1)) / LPR);
     if (row >= rows)
@@ -98,14 +100,14 @@ __global__ void __launch_bounds__(kBlock) layernorm_kernel(const typename Elem<D
 
     float v[NV][VEC];
     double s1 = 0.0, s2 = 0.0;
-    uint4 raw[NV], rraw[NV], rraw2[NV];
+    Raw raw[NV], rraw[NV], rraw2[NV];
     float gam[NV][VEC], bet[NV][VEC];
     auto request = [&](int j, int vi) __attribute__((always_inline)) {
-        raw[j] = reinterpret_cast<const uint4 *>(px)[vi];
+        raw[j] = reinterpret_cast<const Raw *>(px)[vi];
         if (pr)
-            rraw[j] = reinterpret_cast<const uint4 *>(pr)[vi];
+            rraw[j] = reinterpret_cast<const Raw *>(pr)[vi];
         if (pr2)
-            rraw2[j] = reinterpret_cast<const uint4 *>(pr2)[vi];
+            rraw2[j] = reinterpret_cast<const Raw *>(pr2)[vi];
     };
     auto request_affine = [&](int j, int vi) __attribute__((always_inline)) {
 #pragma unroll
@@ -189,12 +191,15 @@ __global__ void __launch_bounds__(kBlock) layernorm_kernel(const typename Elem<D
                 }
             }
             if (VECTOR) {
-                uint4 out;
+                Raw out;
                 T *e = reinterpret_cast<T *>(&out);
 #pragma unroll
                 for (int t = 0; t < VEC; ++t)
                     Elem<DT>::st(&e[t], o[t]);
-                store_out16(mode.through, reinterpret_cast<uint4 *>(py) + vi, store_u32x4{out.x, out.y, out.z, out.w});
+                if constexpr (VB == 16)
+                    store_out16(mode.through, reinterpret_cast<uint4 *>(py) + vi, store_u32x4{out.x, out.y, out.z, out.w});
+                else
+                    store_out8(mode.through, reinterpret_cast<uint2 *>(py) + vi, store_u32x2{out.x, out.y});
                 if (pq) {  // the VEC (4 or 8) quantised values of this lane leave as one 4- or 8-byte store
                     uint32_t w[2] = {0u, 0u};
 #pragma unroll
@@ -307,6 +312,29 @@ int launch_layernorm(hipStream_t s, const void *x, const void *res, const float 
         else                                                                                                          \
             TR_LN_LAUNCH(LPR, NV, false);                                                                             \
     } while (0)
+        // Few half rows of 257 to 1024 columns: a wave a row and vectors of eight bytes, so that a lane adds up 8 to 16 values in
+        // double, not 16 to 32; that chain is most of such a launch.  Up to three workgroups a CU; from there on the waves, twice
+        // as many, cost more than the shorter chain gives.  Sums in double round the order of their terms away: the results are
+        // those of the form below.  us with a residual and an int8 copy, half a wave a row -> this:
+        //   768 columns  128 rows 4.68 -> 4.06, 1024 4.98 -> 4.10, 3072 5.88 -> 5.43, 4096 6.09 -> 6.31
+        //   1024         128      5.51 -> 4.49, 3072 7.04 -> 6.40, 4096 7.48 -> 7.35 (without the copy 6.35 -> 6.56)
+        //   256          1024     3.10 -> 3.00, 2048 3.37 -> 3.51          embedding, 768, 128 rows 6.61 -> 6.09, 4096 7.67 -> 8.07
+        if constexpr (DT != TNN_ROCM_F32) {
+            if (cols > 256 && cols <= 1024 && rows <= 3 * kNumCU * kRowsPerBlk) {
+#define TR_LN_FEW(NV)                                                                                                 \
+    hipLaunchKernelGGL((layernorm_kernel<DT, true, 64, NV, true, 8>), grid, block, 0, s, (const T *)x, (const T *)res, gamma, \
+                       beta, (T *)y, rows, cols, eps, out_q, q_inv, emb, StoreThrough())
+                if (cols <= 512)
+                    TR_LN_FEW(2);
+                else if (cols <= 768)
+                    TR_LN_FEW(3);
+                else
+                    TR_LN_FEW(4);
+#undef TR_LN_FEW
+                TR_CHECK_LAUNCH();
+                return 0;
+            }
+        }
         if (nv <= 32)  // a second vector of a lane would be requested twice: 8192 embedded rows of 256 halves 6.6 us with it
             TR_LN(32, 1, 8, 8);
         else if (nv <= 64)
