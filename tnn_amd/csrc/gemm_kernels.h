@@ -116,15 +116,21 @@ template <> struct GemmTraits<TNN_ROCM_F32> {
     }
 };
 // fp32, pipelined: the planes of the operands of the STEPS steps that a wave takes from one slab.  turn() multiplies one
-// slab's planes while it makes the next one's from their LDS reads: a matrix instruction leaves the vector ALU free for 7 of
-// its 8 issue slots, and the conversion (36 vector instructions per operand and step) goes into them a piece at a time.
+// slab's planes while it makes the next one's from their LDS reads.  Of the conversion's 36 vector instructions per operand and step
+// the 20 that scale and round go behind the matrix instructions, which leave the vector ALU free for about 28 of their 33 clocks (five
+// of them fit).  The 16 dot products do not: one waits until the matrix instruction in front of it is done (33 clocks -> 52, every
+// further one 5; a wave alone on its SIMD), so they stand together, twice in a turn, where only the first of each pays that.
+// Spread over all slots with the others (as they were) a turn took the sum of both kinds: K slabs of 96 x 64 tiles 0.61 us (of 256
+// bytes a row, 96 of them 49.7 us), now 0.55 (45.4), of 128 x 128 1.09 -> 0.96, of 192 x 96 1.21 -> 1.09.  A subtraction of the
+// widened plane in place of a dot product would hide, but takes two instructions: 2 .. 3 % less for tiles of 3 x 3 blocks on few CUs,
+// nothing with all of them at work, 5 .. 10 % more for smaller tiles.  Reading the next slab's values from LDS a turn ahead gave nothing.
 // The order is pinned: left to itself the compiler issues the two kinds one after the other, with the wait states that a
 // dot product's result needs standing empty.  With every CU at work the matrix pipe's power holds the clock near 1.6 GHz, which
 // is then the bound; on few CUs the vector instructions are.
 template <int TM, int TN, int STEPS> struct SplitSlab {
     static constexpr int OPS    = TM + TN;
     static constexpr int MFMAS  = STEPS * kSplitProducts * TM * TN;
-    static constexpr int UNITS  = STEPS * OPS * 20;  // of a conversion: per operand and step five levels of four pairs of values
+    static constexpr int PAIRS  = STEPS * OPS * 4;  // of values
     Split3 op[STEPS][OPS];                           // A's operands, then B's
     struct Reads {
         uint4 f[STEPS][OPS][2];
@@ -147,15 +153,14 @@ template <int TM, int TN, int STEPS> struct SplitSlab {
         for (int q = 0; q < MFMAS; ++q)
             mfma(q, acc);
     }
-    // Unit k of a conversion: one pair of values of operand k / 20, one level (scale and first plane, rest, second plane, rest,
-    // third plane).  The four pairs take turns, so that nothing waits for the unit before it.
-    static __device__ __forceinline__ void unit(int k, SplitSlab &next, float (&rest)[STEPS][OPS][8], const SplitConst &sc) {
-        const int ks = k / (OPS * 20), o = k / 20 % OPS, level = k % 20 / 4, g = k % 4;
+    // One level of a pair of values: scale and first plane, rest, second plane, rest, third plane
+    static __device__ __forceinline__ void level(int pair_index, int l, SplitSlab &next, float (&rest)[STEPS][OPS][8], const SplitConst &sc) {
+        const int ks = pair_index / (OPS * 4), o = pair_index / 4 % OPS, g = pair_index % 4;
         float &x = rest[ks][o][2 * g], &y = rest[ks][o][2 * g + 1];
-        if (level == 0)
+        if (l == 0)
             x *= kSplitScale, y *= kSplitScale;
-        uint32_t &pair = next.op[ks][o].p[level / 2][g];
-        if (level % 2 == 0) {
+        uint32_t &pair = next.op[ks][o].p[l / 2][g];
+        if (l % 2 == 0) {
             pair = split_pack(x, y);
         } else {
             x = split_rest(pair, sc.lo, x);
@@ -165,19 +170,20 @@ template <int TM, int TN, int STEPS> struct SplitSlab {
     // Multiplies this slab's planes while it makes the next one's, whose LDS reads are under way; load(k) requests the k-th of
     // LOADS loads of the slab after, as early as their place is free, one a slot: the next turn waits for them.
     // AFTER_READS: they go where the reads come from.
-    // One or two small pieces of that go behind every matrix instruction: a slot holds about seven vector instructions, and a
-    // piece that is longer (a whole plane of four values took twelve) leaves the matrix pipe empty for the rest of it.
+    // Levels 0, 2 and 4 go behind the matrix instructions, in proportion to their instructions (three, one and one a pair), levels 1
+    // and 3 in one piece each behind the last slot of the level in front.
     template <int LOADS, bool AFTER_READS, typename Acc, typename Load>
     __device__ __forceinline__ void turn(const Reads &rd, SplitSlab &next, Acc (&acc)[TM][TN], const SplitConst &sc, Load load) const {
-        constexpr int LEAD = MFMAS >= 24 ? 4 : 2;  // the first matrix instructions alone: the LDS reads arrive meanwhile
+        constexpr int LEAD   = MFMAS >= 24 ? 4 : 2;  // the first matrix instructions alone: the LDS reads arrive meanwhile
+        constexpr int SLOTS  = MFMAS - LEAD, SECOND = SLOTS >= 5 ? SLOTS / 5 : 1, FIRST = SLOTS - 2 * SECOND;
         constexpr int L0     = AFTER_READS ? LEAD : 0;
         constexpr int LSLOTS = LOADS > 0 && LOADS < MFMAS - L0 ? LOADS : MFMAS - L0;
         float rest[STEPS][OPS][8];
-#pragma unroll
-        for (int q = 0; q < MFMAS; ++q) {
+        each(std::make_integer_sequence<int, MFMAS>(), [&](auto slot) __attribute__((always_inline)) {
+            constexpr int q = decltype(slot)::value, i = q - LEAD;
             mfma(q, acc);
             __builtin_amdgcn_sched_barrier(0);
-            if (q == LEAD - 1) {
+            if constexpr (i == -1) {
 #pragma unroll
                 for (int ks = 0; ks < STEPS; ++ks)
 #pragma unroll
@@ -190,13 +196,19 @@ template <int TM, int TN, int STEPS> struct SplitSlab {
                             rest[ks][o][h * 4 + 3] = __uint_as_float(rd.f[ks][o][h].w);
                         }
             }
-            if (q >= LEAD) {
-                constexpr int SLOTS = MFMAS - LEAD;
+            if constexpr (i >= 0) {  // this slot's level, and its share of the level's slots
+                constexpr int l  = i < FIRST ? 0 : i < FIRST + SECOND ? 2 : 4;
+                constexpr int at = i - (l == 0 ? 0 : l == 2 ? FIRST : FIRST + SECOND), of = l == 0 ? FIRST : SECOND;
 #pragma unroll
-                for (int k = UNITS * (q - LEAD) / SLOTS; k < UNITS * (q - LEAD + 1) / SLOTS; ++k)
-                    unit(k, next, rest, sc);
+                for (int k = PAIRS * at / of; k < PAIRS * (at + 1) / of; ++k)
+                    level(k, l, next, rest, sc);
+                if constexpr (l < 4 && at == of - 1) {
+#pragma unroll
+                    for (int k = 0; k < PAIRS; ++k)
+                        level(k, l + 1, next, rest, sc);
+                }
             }
-            if (LOADS > 0 && q >= L0 && q < L0 + LSLOTS) {
+            if constexpr (LOADS > 0 && q >= L0 && q < L0 + LSLOTS) {
                 if (AFTER_READS && q == L0)
                     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
 #pragma unroll
@@ -204,7 +216,11 @@ template <int TM, int TN, int STEPS> struct SplitSlab {
                     load(k);
             }
             __builtin_amdgcn_sched_barrier(0);
-        }
+        });
+    }
+    // (the slots one by one as constants: the unroller gives up on a loop of this size)
+    template <int... Q, typename F> static __device__ __forceinline__ void each(std::integer_sequence<int, Q...>, F f) {
+        (f(std::integral_constant<int, Q>()), ...);
     }
 };
 
@@ -2398,7 +2414,10 @@ constexpr TileCost kTilesI8[] = {
 // us, v_mfma_f32 kernels -> planes, a whole plane of four values behind a matrix instruction -> a pair of values:
 //   M=1536: N=768 K=768 27 -> 20.2 -> 17.3, N=3072 K=768 74 -> 61 -> 55, N=768 K=3072 83 -> 60 -> 51
 //   M=128: N=768 K=768 7.6 -> 7.1 -> 6.8, N=3072 K=768 15.2 -> 11.4 -> 10.7, N=768 K=3072 17.6 -> 16.2 -> 15.3
-// (the 16 x 16 blocks, which came after that, see above, not counted)
+// (the 16 x 16 blocks, which came after that, see above, not counted).  Since the dot products stand together (SplitSlab; six sets
+// of weights in turn): M=1536 20.3 -> 19.2, 56.2 -> 52, 58.1 -> 54; M=128 6.8 -> 6.6, 12.1 -> 11.7, 13.5 -> 13.2.  The figures
+// below are from before; with them the choice is 0.45 % from the best shape in the mean (192 launches, 16 to 3072 rows, hidden sizes
+// 512 to 1024; fitted again 0.32 %).
 // Error against float64 (2-norm over 2-norm; 300 x 760 x 768 / 129 x 264 x 3072): 1.5e-7 .. 3e-7 / 3e-7 .. 6e-7 by shape,
 // v_mfma_f32_32x32x2_f32: 5.0e-7 / 9.9e-7.
 constexpr TileCost kTilesF32[] = {
