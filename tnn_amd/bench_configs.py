@@ -184,7 +184,7 @@ def stores(args):
 
 # configuration codes of the tiled GEMM kernel, tnn_rocm_debug_set_gemm_config
 TILE_CODES = {"half": (6111141, 6211141, 6121141, 9111141, 9121141, 3112221, 2112211, 8222222, 8322222, 8332222, 8422222,
-                       7244211, 8244211, 8264211, 8344211, 8364211, 8444211, 2244211),
+                       7244211, 8244211, 8264211, 8344211, 8364211, 8444211, 7484211),
               "fp32": (6111141, 6211141, 6121141, 6111181, 6211181, 9111141, 9121141, 9111181, 9221141, 2321142, 2231142,
                        2331142, 2222121, 2222221, 2332121)}
 

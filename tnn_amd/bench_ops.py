@@ -190,7 +190,7 @@ TILE_SHAPES = {
     "half": ((6111141, 16, 16, 3), (6211141, 32, 16, 2), (6121141, 16, 32, 2), (9111141, 32, 32, 2), (9121141, 32, 64, 1),
              (3112221, 64, 64, 3), (2112211, 64, 64, 4), (8222222, 64, 64, 1), (8322222, 96, 64, 1), (8332222, 96, 96, 1),
              (8422222, 128, 64, 1), (7244211, 128, 128, 2), (8244211, 128, 128, 1), (8264211, 128, 192, 1), (8344211, 192, 128, 1),
-             (8364211, 192, 192, 1), (8444211, 256, 128, 1), (2244211, 256, 256, 1)),
+             (8364211, 192, 192, 1), (8444211, 256, 128, 1), (7484211, 256, 256, 1)),
     "f32": ((6111141, 16, 16, 3), (6211141, 32, 16, 2), (6121141, 16, 32, 2), (6111181, 16, 16, 1), (6211181, 32, 16, 1),
             (9111141, 32, 32, 2), (9121141, 32, 64, 1), (9111181, 32, 32, 1), (9221141, 64, 64, 1), (2321142, 96, 64, 1),
             (2231142, 64, 96, 1), (2331142, 96, 96, 1), (2222121, 128, 64, 2), (2222221, 128, 128, 1), (2332121, 192, 96, 1))}

@@ -1099,10 +1099,12 @@ __global__ void __launch_bounds__(WM *WN * 64)
 //     A slab is then SLAB bytes of k of ALL rows of the tile for ONE wave, and nothing in the main loop concerns another
 //     wave: no barrier, each wave waits for its own loads only.
 // BLK = 16 (slabs direct to LDS): the waves' blocks are 16 x 16 instead of 32 x 32 (v_mfma_*_16x16x32, 64 bytes of k a step), TM
-//     and TN count those, and the whole tile is staged for the epilogue at once.
+//     and TN count those.
 template <int TM_, int TN_, int WGM_, int WGN_, int WGK_, int SLAB_, int NSTAGE_ = 0, bool OWN_ = false, int BLK_ = 32> struct TileCfg {
     static constexpr int BLK = BLK_;
-    static constexpr int GROUPS = BLK_ == 32 ? TM_ : 1, GROWS = BLK_ == 32 ? 32 : BLK_ * TM_;  // staged together: rows of a wave position
+    // groups of rows that are staged one after the other, and the rows of a wave position in one: blocks of 32 rows, or the whole tile
+    // where it is one of 16 x 16 blocks and fits into LDS at once (256 x 256 tiles do not: halves)
+    static constexpr int GROUPS = BLK_ == 32 ? TM_ : WGM_ * WGN_ * WGK_ * TM_ * (4 * TN_ + 1) > 640 ? 2 : 1, GROWS = BLK_ * TM_ / GROUPS;
     static_assert(BLK_ == 32 || (BLK_ == 16 && NSTAGE_ > 0 && (!OWN_ || BLK_ * TM_ <= 32)), "16 x 16 blocks: direct-to-LDS slabs only");
     static constexpr int TM = TM_, TN = TN_, WGM = WGM_, WGN = WGN_, WGK = WGK_, SLAB = SLAB_, NSTAGE = NSTAGE_;
     static constexpr bool OWN = OWN_;
@@ -2083,10 +2085,11 @@ __global__ void __launch_bounds__(CFG::NT)
                         acc4{acc[i][j][r4 * 4 + 0], acc[i][j][r4 * 4 + 1], acc[i][j][r4 * 4 + 2], acc[i][j][r4 * 4 + 3]};
         } else {
 #pragma unroll
-            for (int b = 0; b < TM; ++b)
+            for (int b = 0; b < TM / GROUPS; ++b)
 #pragma unroll
                 for (int j = 0; j < TN; ++j)
-                    *reinterpret_cast<acc4 *>(stage_me + (b * 16 + (lane & 15)) * SSTR + j * 16 + 4 * (lane >> 4)) = acc[b][j];
+                    *reinterpret_cast<acc4 *>(stage_me + (b * 16 + (lane & 15)) * SSTR + j * 16 + 4 * (lane >> 4)) =
+                        acc[i * (TM / GROUPS) + b][j];
         }
         if constexpr (Epi::kRowStats) {
             if (i == GROUPS - 1) {
@@ -2312,7 +2315,7 @@ int launch_tiled(hipStream_t s, const void *A, const void *B, int M, int N, int 
 //   7 and 8 (two and three stages): 16 x 16 blocks, 8 waves that share the slabs
 //   8222222   64 x  64, 8322222 96 x 64, 8332222 96 x 96, 8422222 128 x 64: 2 x 2 positions and two k-waves, 256-byte slabs
 //   7244211  128 x 128, 8244211 128 x 128, 8344211 192 x 128, 8364211 192 x 192: 4 x 2 positions; not int8: 8264211 128 x 192, 8444211 256 x 128
-//   2244211  256 x 256, 8 waves
+//   7484211  256 x 256: 4 x 2 positions
 //   fp32 only: 6111181, 6211181 16 x 16 and 32 x 16, 8 k-waves; 9111181 32 x 32, 8 k-waves; 9221141 64 x 64, 4 k-waves with rings of their own;
 //   2321142, 2231142, 2331142 96 x 64, 64 x 96 and 96 x 96, 4 k-waves; 2222121, 2332121 128 x 64 and 192 x 96, 4 waves (two k-waves);
 //   2222221 128 x 128, 8 waves (two k-waves)
@@ -2331,7 +2334,8 @@ int launch_tiled(hipStream_t s, const void *A, const void *B, int M, int N, int 
 // by shape (the large ones most), so picks closer than that are as good as drawn.  The half and int8 rows were then moved as little
 // as it took for few launches to be slower than with the tables and shapes before them: over 584 launches of each type (hidden sizes
 // 256 to 2048, M from 16 to 12288) the picks are 0.4 % (fp16) and 0.5 % (int8) behind the best shape of each, and 7 % and 8 % faster than
-// before; of the 392 compared 11 and 16 are more than 2 % slower, one and three more than 5 (8192 x 2048 x 8192 by 10).  fp32: 1.0 % behind.
+// before; of the 392 compared 11 and 16 are more than 2 % slower, one and three more than 5 (8192 x 2048 x 8192 by 10, which 256 x 256
+// tiles of 16 x 16 blocks have turned into 14 % faster).  fp32: 1.0 % behind.
 // The rules this replaced, made for M >= 1024, were 51 %, 34 % and 77 % behind:
 //   M=  32 N= 768 K=3072 fp16  23.1 -> 7.3 us   (64x64 tiles: 12 CUs, one two-stage slab after another)
 //   M= 256 N= 768 K=3072 fp16  23.7 -> 7.2      M= 256 N=2304 K=768 fp16  8.7 -> 6.2
@@ -2358,7 +2362,7 @@ constexpr TileCost kTilesHalf[] = {
     {8344211, 192, 128, 1, 6.59f, 8.74f, {0.465f}},
     {8364211, 192, 192, 1, 8.80f, 12.52f, {0.666f}},
     {8444211, 256, 128, 1, 7.77f, 11.65f, {0.596f}},
-    {2244211, 256, 256, 1, 10.50f, 12.00f, {1.255f}},
+    {7484211, 256, 256, 1, 11.80f, 13.30f, {1.145f}},
 };
 // 256 x 256 tiles are for products that fill the chip with them: half the bytes a flop of 128 x 128 tiles.  A linear model knows
 // neither that a round of 192 tiles is 13 % shorter than one of 256 nor what the epilogue leaves uncovered, so their row and the
@@ -2369,7 +2373,13 @@ constexpr TileCost kTilesHalf[] = {
 // 82 -> 92, 4096 x 3072 x 768 29.6 -> 31.1, 8192 x 1536 x 384 21.1 -> 22.7.  With twelve weight sets in turn, over 260 launches, the
 // picks that are slower cost 25 % together (187 % with the old row), the shape where it is left out and faster 88 % (99 %).  The int8
 // row is set by hand: of its picks three of 60 are slower, 24576 x 1920 x 640 into Q, K and V^T by 6 % and [16384, 1024] x 1024 and
-// 24576 x 1280 x 1280 with a residual by 3 %.
+// 24576 x 1280 x 1280 with a residual by 3 %.  That was with 32 x 32 blocks, whose row was {10.5, 12.0, 1.255} (int8 {10.5, 8.2, 2.049}).
+// As 16 x 16 blocks a step's products are twice as many of half the length, between which the next step's reads spread finer, and
+// the loop is 4 .. 10 % faster; the tile is staged in two halves instead of two blocks' rows.  us: 16384 x 4096 x 1024 with GELU
+// 167 -> 152, 16384 x 1024 x 4096 124 -> 115, 8192 x 8192 x 8192 936 -> 861, bf16 873 -> 839, int8 16384 x 1024 x 4096 68.6 -> 62.0,
+// 16384 x 4096 x 1024 105 -> 100, 8192 x 4096 x 4096 136 -> 125.  The row's slab is smaller by that and its other two figures larger
+// by twelve slabs of it, so that the line stays where it is at K = 768 (with 1.165 alone K = 512 lost 10 %) and moves with K: of the
+// seven products of hidden sizes 512 to 4096 that changed for it five are 3 .. 21 % faster, two 1 % slower.
 // 16 x 16 blocks of a shared slab.  Up to 128 x 64: eight waves as 2 x 2 positions and two k-waves, so that a tile of any number of 32
 // rows and columns is dealt out evenly.  96 x 96 as eight k-waves of 3 x 3 blocks of 32 x 32 passed 295 KB of partial sums through
 // LDS behind its loop (half of the 11 us of 3072 x 768 x 768), now 74; 96 x 64 is one round of the chip where 64 x 64 are two.
@@ -2405,7 +2415,7 @@ constexpr TileCost kTilesI8[] = {
     {8244211, 128, 128, 1, 4.99f, 12.00f, {0.418f}},
     {8344211, 192, 128, 1, 6.60f, 9.50f, {0.543f}},
     {8364211, 192, 192, 1, 8.95f, 12.02f, {0.850f}},
-    {2244211, 256, 256, 1, 10.50f, 8.20f, {2.049f}},
+    {7484211, 256, 256, 1, 11.80f, 9.50f, {1.920f}},
 };
 // fp32 on three bf16 planes: six matrix instructions per operand pair and the conversion between them, so a step costs five
 // times a half one.  Large wave tiles convert less per product, K is split over the waves of a CU wherever tiles are few, and
@@ -2491,6 +2501,7 @@ int launch_gemm_fast(hipStream_t s, const void *A, const void *B, int M, int N, 
             case 3212221:
             case 2222221: cfg = 7244211; break;
             case 3332221: cfg = 8364211; break;
+            case 2244211: cfg = 7484211; break;
             case 3331182: cfg = 8332222; break;
             case 4221141:
             case 3112222: cfg = 8222222; break;
@@ -2554,7 +2565,7 @@ int launch_gemm_fast(hipStream_t s, const void *A, const void *B, int M, int N, 
             case 8244211: TR_FAST_DL16(2, 4, 4, 2, 1, 128, 3);
             case 8344211: TR_FAST_DL16(3, 4, 4, 2, 1, 128, 3);
             case 8364211: TR_FAST_DL16(3, 6, 4, 2, 1, 128, 3);
-            case 2244211: TR_FAST_DL(2, 4, 4, 2, 1, 128, 2);
+            case 7484211: TR_FAST_DL16(4, 8, 4, 2, 1, 128, 2);
             case 8222222: TR_FAST_DL16(2, 2, 2, 2, 2, 256, 3);
             case 8322222: TR_FAST_DL16(3, 2, 2, 2, 2, 256, 3);
             case 8332222: TR_FAST_DL16(3, 3, 2, 2, 2, 256, 3);
