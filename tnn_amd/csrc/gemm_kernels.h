@@ -2377,9 +2377,12 @@ constexpr TileCost kTilesHalf[] = {
 // As 16 x 16 blocks a step's products are twice as many of half the length, between which the next step's reads spread finer, and
 // the loop is 4 .. 10 % faster; the tile is staged in two halves instead of two blocks' rows.  us: 16384 x 4096 x 1024 with GELU
 // 167 -> 152, 16384 x 1024 x 4096 124 -> 115, 8192 x 8192 x 8192 936 -> 861, bf16 873 -> 839, int8 16384 x 1024 x 4096 68.6 -> 62.0,
-// 16384 x 4096 x 1024 105 -> 100, 8192 x 4096 x 4096 136 -> 125.  The row's slab is smaller by that and its other two figures larger
+// 16384 x 4096 x 1024 105 -> 100, 8192 x 4096 x 4096 136 -> 125.  The half row's slab is smaller by that and its other two figures larger
 // by twelve slabs of it, so that the line stays where it is at K = 768 (with 1.165 alone K = 512 lost 10 %) and moves with K: of the
-// seven products of hidden sizes 512 to 4096 that changed for it five are 3 .. 21 % faster, two 1 % slower.
+// seven products of hidden sizes 512 to 4096 that changed for it five are 3 .. 21 % faster, two 1 % slower.  The int8 row, and with it
+// the second slab of two 128 x 128 tiles a CU (1.148, 10 % above what it measures at K of 3072 and up), are set to order the shapes
+// from 128 x 128 on as they measure: 49 products change (hidden sizes 256 to 4096, 512 to 24576 rows), 11 % faster in the mean, the
+// slowest 4 % slower; us: 8192 x 768 x 3072 32.0 -> 27.5, 4096 x 4096 x 4096 77.6 -> 63.0, 12288 x 1280 x 5120 91.7 -> 72.3.
 // 16 x 16 blocks of a shared slab.  Up to 128 x 64: eight waves as 2 x 2 positions and two k-waves, so that a tile of any number of 32
 // rows and columns is dealt out evenly.  96 x 96 as eight k-waves of 3 x 3 blocks of 32 x 32 passed 295 KB of partial sums through
 // LDS behind its loop (half of the 11 us of 3072 x 768 x 768), now 74; 96 x 64 is one round of the chip where 64 x 64 are two.
@@ -2411,11 +2414,11 @@ constexpr TileCost kTilesI8[] = {
     {8322222, 96, 64, 1, 3.92f, 3.17f, {0.206f}},
     {8332222, 96, 96, 1, 4.96f, 4.41f, {0.271f}},
     {8422222, 128, 64, 1, 3.66f, 3.60f, {0.271f}},
-    {7244211, 128, 128, 2, 3.92f, 3.61f, {0.632f, 1.148f}},
+    {7244211, 128, 128, 2, 3.92f, 3.61f, {0.632f, 1.040f}},
     {8244211, 128, 128, 1, 4.99f, 12.00f, {0.418f}},
     {8344211, 192, 128, 1, 6.60f, 9.50f, {0.543f}},
     {8364211, 192, 192, 1, 8.95f, 12.02f, {0.850f}},
-    {7484211, 256, 256, 1, 11.80f, 9.50f, {1.920f}},
+    {7484211, 256, 256, 1, 13.00f, 10.70f, {1.700f}},
 };
 // fp32 on three bf16 planes: six matrix instructions per operand pair and the conversion between them, so a step costs five
 // times a half one.  Large wave tiles convert less per product, K is split over the waves of a CU wherever tiles are few, and
