@@ -2051,6 +2051,72 @@ def test_folded_layernorm_statistics_of_rows_with_little_spread(dtype, K, code):
         lib.tnn_rocm_debug_set_gemm_config(0)
 
 
+def _residual_row_sums(code, t, N, K=512):
+    """what gemm_residual_ln leaves of t itself (a product of zeros, statistics {1, 0}): (the row sums' blocks, their width)"""
+    from tnn_amd import capi
+    lib, M = capi.load(), t.shape[0]
+    x, w = (torch.zeros(n, K, dtype=t.dtype, device="cuda") for n in (M, N))
+    st = torch.tensor([[1.0, 0.0]], device="cuda").repeat(M, 1)
+    one, zero = torch.ones(N, device="cuda"), torch.zeros(N, device="cuda")
+    lib.tnn_rocm_debug_set_gemm_config(code)
+    try:
+        left, (sums, blocks) = ops().gemm_residual_ln(x, w, t.cuda(), st, one, zero, want_row_sums=True)
+    finally:
+        lib.tnn_rocm_debug_set_gemm_config(0)
+    assert torch.equal(left.cpu(), t) and blocks > 0
+    return sums[:blocks].cpu()
+
+
+# shapes whose row sums pass through LDS, and their columns
+ROW_SUM_SHAPES = {2112211: 64, 3112221: 64, 112210: 64, 8222222: 64, 8322222: 64, 8332222: 96, 8422222: 64, 7244211: 128, 8244211: 128,
+                  8264211: 192, 8344211: 128, 8364211: 192, 8444211: 128}
+
+
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
+@pytest.mark.parametrize("code", sorted(ROW_SUM_SHAPES))
+def test_row_sums_of_a_tile_are_rounded_once(dtype, code):
+    """Values whose sums over eight columns are exact in fp32 and over a tile's are not: every pair that a tile leaves is the exact sum,
+    rounded once.  One row behind whole tiles, a part of a tile column, columns of zeros."""
+    say("row sums %s, shape %d" % (dtype, code))
+    gen = torch.Generator().manual_seed(code)
+    M, N, wide = 257, 776, ROW_SUM_SHAPES[code]
+    if dtype == "float16":  # ten bits: eight squares in 23, a tile's in 26 or 27
+        t = torch.randint(512, 1024, (M, N), generator=gen) * 2.0 ** -9
+    else:  # eight bits, with the squares of neighbouring items 2^8 apart
+        t = torch.randint(128, 256, (M, N), generator=gen) * 2.0 ** -7 * (16.0 ** (torch.arange(N) // 8 % 4))
+    t[:, 400:408] = 0
+    got = _residual_row_sums(code, t.to(getattr(torch, dtype)), N).double()
+    for k, part in enumerate(t.double().split(wide, 1)):
+        assert torch.equal(got[k, :, 0], part.sum(1).float().double()) and torch.equal(got[k, :, 1], (part ** 2).sum(1).float().double()), k
+    assert got.shape[0] == -(-N // wide)
+
+
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
+@pytest.mark.parametrize("sigmas", [0, 5, 20, 50])
+@pytest.mark.parametrize("code", [0, 6111141, 9111141] + sorted(ROW_SUM_SHAPES))
+def test_row_sums_left_by_a_shape_give_the_variance(dtype, sigmas, code):
+    """{rstd, mean} from the sums that a shape itself left, of rows up to 50 standard deviations from zero: what fp32 sums of eight
+    values know of the variance"""
+    say("variance from the row sums of shape %d, %s, %d sigma" % (code, dtype, sigmas))
+    gen = torch.Generator().manual_seed(code + sigmas)
+    M, N = 130, 384
+    t = (sigmas + torch.randn(M, N, generator=gen)).to(getattr(torch, dtype))
+    sums = _residual_row_sums(code, t, N)
+    handed = torch.zeros(ops().MAX_ROW_SUM_BLOCKS, M, 2)
+    handed[:len(sums)] = sums
+    w = torch.zeros(8, N, dtype=t.dtype, device="cuda")
+    zero = torch.zeros(8, device="cuda")
+    st = ops().gemm_ln(t.cuda(), w, zero, zero, 1e-5, want_stats=True, row_sums=(handed.cuda(), len(sums)))[1].cpu().double()
+    d = t.double()
+    var = d.var(1, unbiased=False) + float(np.float32(1e-5))
+    # A row's sums are those of its items of eight values, which carry some roundings of half a unit each (a unit and a half at most, once they
+    # are averaged over the row's items, for the squares and as much for the square of the sum), and of the pairs made of them, one more;
+    # the root halves that.  Its own roundings as in the tests of sums made on the host.
+    allowed = 3e-7 + 0.5 * 2.0 ** -24 * 3 * (d ** 2).mean(1) / var
+    assert ((st[:, 0] * var.sqrt() - 1).abs() <= allowed).all(), float(((st[:, 0] * var.sqrt() - 1).abs() / allowed).max())
+    assert ((st[:, 1] - d.mean(1)).abs() <= 2e-7 * d.abs().mean(1)).all()
+
+
 @pytest.mark.parametrize("dtype", ["f16", "bf16"])
 def test_attention_quantised_second_output_bit_exact(dtype):
     """The int8 tensor the attention kernel can write next to its output equals the checker's x86 quantiser applied to

@@ -248,16 +248,23 @@ template <int O> __device__ __forceinline__ double add_lane_xor(double v) {
     }
 }
 
+// the v of another lane of the same eight, by a DPP control word
+template <int CTRL> __device__ __forceinline__ float lane_of_eight(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, false));
+}
+template <int CTRL> __device__ __forceinline__ double lane_of_eight(double v) {
+    typedef float pair __attribute__((ext_vector_type(2)));
+    const pair u = __builtin_bit_cast(pair, v);
+    return __builtin_bit_cast(double, pair{lane_of_eight<CTRL>(u.x), lane_of_eight<CTRL>(u.y)});
+}
+
 // the sum over N = 2, 4 or 8 neighbouring lanes, in every one of them
-template <int N> __device__ __forceinline__ float add_neighbours(float v) {
-    auto add = [](float x, auto ctrl) {
-        return x + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), decltype(ctrl)::value, 0xf, 0xf, false));
-    };
-    v = add(v, std::integral_constant<int, 0xB1>());  // quad_perm: lane ^ 1
+template <int N, typename V> __device__ __forceinline__ V add_neighbours(V v) {
+    v = v + lane_of_eight<0xB1>(v);  // quad_perm: lane ^ 1
     if constexpr (N >= 4)
-        v = add(v, std::integral_constant<int, 0x4E>());  // quad_perm: lane ^ 2
+        v = v + lane_of_eight<0x4E>(v);  // quad_perm: lane ^ 2
     if constexpr (N >= 8)
-        v = add(v, std::integral_constant<int, 0x141>());  // row_half_mirror: the other four of eight
+        v = v + lane_of_eight<0x141>(v);  // row_half_mirror: the other four of eight
     return v;
 }
 

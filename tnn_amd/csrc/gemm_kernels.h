@@ -2197,18 +2197,25 @@ __global__ void __launch_bounds__(CFG::NT)
     }
     TR_TL(3);  // C stored
     if constexpr (EmitsRowSums<Epi>::value && !CFG::sums_by_lanes) {
-        // this tile's share of every row's sum and sum of squares, added up in a fixed order, for the folding GEMM
-        // that reads C next
+        // This tile's share of every row's sum and sum of squares, added up in a fixed order, for the folding GEMM that reads C next.
+        // LANES neighbouring lanes share a row and add in double, as the reader does with the tiles' pairs: a pair is rounded once,
+        // whatever the tile's width (16 of them one after the other in fp32 took 2 .. 3 times the variance's error of rows far from zero).
+        constexpr int SPLIT = NT / BM, LANES = SPLIT >= 8 ? 8 : SPLIT >= 4 ? 4 : 2;
+        static_assert(SPLIT >= 2 && BM * LANES % 64 == 0 && BN / 8 % LANES == 0, "whole waves, every lane with as many pairs");
         __syncthreads();
-        if (tid < BM && m0 + tid < M) {
-            float s1 = 0.f, s2 = 0.f;
+        if (tid < BM * LANES) {
+            const int row   = tid / LANES;
+            const AccT *src = stage_all + (row / GROWS * WGN * WGK) * (GROWS * SSTR) + row % GROWS * SSTR;
+            double s1 = 0.0, s2 = 0.0;
 #pragma unroll
-            for (int q = 0; q < BN / 8; ++q) {
-                const int pos = tid / GROWS * WGN + q / CPR;
-                const float2 part = *reinterpret_cast<const float2 *>(stage_all + (pos * WGK) * (GROWS * SSTR) + tid % GROWS * SSTR + q % CPR * 8);
-                s1 += part.x, s2 += part.y;
+            for (int q = 0; q < BN / 8; q += LANES) {
+                const int piece   = q + tid % LANES;
+                const float2 part = *reinterpret_cast<const float2 *>(src + (piece / CPR * WGK) * (GROWS * SSTR) + piece % CPR * 8);
+                s1 += (double)part.x, s2 += (double)part.y;
             }
-            store_out8(epi.through, &epi.row_sums[(size_t)(n0 / BN) * M + m0 + tid], make_float2(s1, s2));
+            s1 = add_neighbours<LANES>(s1), s2 = add_neighbours<LANES>(s2);
+            if (tid % LANES == 0 && m0 + row < M)
+                store_out8(epi.through, &epi.row_sums[(size_t)(n0 / BN) * M + m0 + row], make_float2((float)s1, (float)s2));
         }
     }
     if constexpr (Epi::kRowStats) {
