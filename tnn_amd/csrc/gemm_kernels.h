@@ -2198,20 +2198,22 @@ __global__ void __launch_bounds__(CFG::NT)
     TR_TL(3);  // C stored
     if constexpr (EmitsRowSums<Epi>::value && !CFG::sums_by_lanes) {
         // This tile's share of every row's sum and sum of squares, added up in a fixed order, for the folding GEMM that reads C next.
-        // LANES neighbouring lanes share a row and add in double, as the reader does with the tiles' pairs: a pair is rounded once,
-        // whatever the tile's width (16 of them one after the other in fp32 took 2 .. 3 times the variance's error of rows far from zero).
+        // LANES neighbouring lanes share a row.  Tiles of 128 columns and more add in double, so that their pairs are rounded once and the
+        // variance is as exact as from pairs of 64 columns (in fp32 rows far from zero had up to twice the error); narrower ones need not,
+        // and it would cost 0.3 us of the 8 to 23 of theirs.
+        typedef typename std::conditional<(BN > 96), double, float>::type Sum;
         constexpr int SPLIT = NT / BM, LANES = SPLIT >= 8 ? 8 : SPLIT >= 4 ? 4 : 2;
         static_assert(SPLIT >= 2 && BM * LANES % 64 == 0 && BN / 8 % LANES == 0, "whole waves, every lane with as many pairs");
         __syncthreads();
         if (tid < BM * LANES) {
             const int row   = tid / LANES;
             const AccT *src = stage_all + (row / GROWS * WGN * WGK) * (GROWS * SSTR) + row % GROWS * SSTR;
-            double s1 = 0.0, s2 = 0.0;
+            Sum s1 = 0, s2 = 0;
 #pragma unroll
             for (int q = 0; q < BN / 8; q += LANES) {
                 const int piece   = q + tid % LANES;
                 const float2 part = *reinterpret_cast<const float2 *>(src + (piece / CPR * WGK) * (GROWS * SSTR) + piece % CPR * 8);
-                s1 += (double)part.x, s2 += (double)part.y;
+                s1 += (Sum)part.x, s2 += (Sum)part.y;
             }
             s1 = add_neighbours<LANES>(s1), s2 = add_neighbours<LANES>(s2);
             if (tid % LANES == 0 && m0 + row < M)
