@@ -829,7 +829,43 @@ def test_gemm_16x16_blocks_of_a_shared_slab(code, slabs):
             assert (got[:, 1] / (stored ** 2).sum(1) - 1).abs().max() <= 1e-5
 
 
-@pytest.mark.parametrize("M,N,K,gelu,most", [(24576, 1536, 384, True, 1.1), (12288, 1024, 256, True, 1.07), (4096, 4096, 1024, False, 0.93)])
+# parts that a shape adds a long product up in, each in a set of sums of its own
+SUM_PARTS = {2112211: 1, 3112221: 2, 8222222: 4, 8322222: 4, 8422222: 4, 8332222: 8, 7244211: 2, 8244211: 4, 8264211: 2, 8344211: 8,
+             8364211: 2, 8444211: 2, 7484211: 1, 6111141: 4, 9111141: 4}
+
+
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
+def test_gemm_error_of_the_sums_falls_with_the_parts(dtype):
+    """Sums in fp32 against float64, without the result's rounding: the bias takes the exact product off, so that what is stored is the
+    sum's error.  An error that every addition grows by a share of the sum so far goes with the root of the additions in a row: of
+    n parts, one n-th of the error's square, and the additions of the parts, log2(n) of the sum's own size and rounded by half a unit at
+    most each, evenly spread.  A tenth more for the sample."""
+    from tnn_amd import capi
+    lib, o, td = capi.load(), ops(), getattr(torch, dtype)
+    M, N = 40, 2048
+    for K in (768, 3072, 4096):
+        gen = torch.Generator().manual_seed(K)
+        x, w = (16 * torch.randn(1, K, generator=gen)).to(td), (16 * torch.randn(N, K, generator=gen)).to(td)
+        exact = (x.double() @ w.double().T)[0]
+        bias = -exact.float()
+        error = {}
+        for code, parts in SUM_PARTS.items():
+            say("error of the sums %s, K=%d, shape %d" % (dtype, K, code))
+            lib.tnn_rocm_debug_set_gemm_config(code)
+            try:
+                got = host(o.gemm(x.expand(M, K).contiguous().cuda(), w.cuda(), True, bias=bias.cuda()).double())
+            finally:
+                lib.tnn_rocm_debug_set_gemm_config(0)
+            assert (got == got[0]).all()
+            error[code] = np.linalg.norm(got[0] - host(exact + bias.double())) / np.linalg.norm(host(exact))
+            if code == 8344211 and K < 1536:  # the further parts are of 768 products each
+                parts = 2
+            assert error[code] <= 1.1 * np.sqrt(error[2112211] ** 2 / parts + np.log2(parts) * 2.0 ** -48 / 3), (K, code, error)
+        assert error[2112211] <= 2.0 ** -24 * (K / 16) ** 0.5  # a rounding of half a unit at most every sixteen products
+
+
+@pytest.mark.parametrize("M,N,K,gelu,most", [(24576, 1536, 384, True, 1.1), (12288, 1024, 256, True, 1.07), (4096, 4096, 1024, False, 0.93),
+                                             (4096, 3072, 768, True, 1.02)])
 def test_gemm_shape_picked_for_large_products(M, N, K, gelu, most):
     """256 x 256 tiles where they are the faster ones: with GELU and a short K they took 1.21, 1.12 times what 128 x 128 tiles take, and
     0.83 of it where the chip is full and the epilogue light."""

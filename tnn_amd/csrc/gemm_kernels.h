@@ -275,7 +275,7 @@ template <int DT> struct FloatEpilogue : StoreThrough {
     long ldc;
     long batch_stride_c;
     long batch_stride_r;
-    float wide_us() const { return (flags & TNN_ROCM_EPI_GELU) ? 1.75f : 0.f; }
+    float wide_us() const { return (flags & TNN_ROCM_EPI_GELU) ? 2.5f : 0.f; }
     __device__ __forceinline__ void set_batch(int b) {
         C += (size_t)b * batch_stride_c;
         if (residual)
@@ -475,7 +475,7 @@ template <int DT, int SUMS = 0> struct LnFloatEpilogue : StoreThrough {
     T *C;
     long ldc;
     LnFold ln;
-    float wide_us() const { return (flags & TNN_ROCM_EPI_GELU) ? 1.75f : 0.f; }
+    float wide_us() const { return (flags & TNN_ROCM_EPI_GELU) ? 2.5f : 0.f; }
     __device__ __forceinline__ void set_batch(int) {}
     __device__ __forceinline__ float col_const(int) const { return 0.f; }
     __device__ __forceinline__ void store(int, int, float, float) const {}  // N % 8 == 0 is required at launch
@@ -602,7 +602,7 @@ template <int DT, bool SUMS = false> struct LnResidualEpilogue : StoreThrough {
     const float *gamma, *beta;  // [N]
     T *C;
     long ldc;
-    float wide_us() const { return (flags & TNN_ROCM_EPI_GELU) ? 1.75f : 0.f; }
+    float wide_us() const { return (flags & TNN_ROCM_EPI_GELU) ? 2.5f : 0.f; }
     __device__ __forceinline__ void set_batch(int) {}
     __device__ __forceinline__ float col_const(int n) const { return (flags & TNN_ROCM_EPI_BIAS) ? bias[n] : 0.f; }
     __device__ __forceinline__ void store(int m, int n, float acc, float bias_n) const {
@@ -1100,14 +1100,27 @@ __global__ void __launch_bounds__(WM *WN * 64)
 //     wave: no barrier, each wave waits for its own loads only.
 // BLK = 16 (slabs direct to LDS): the waves' blocks are 16 x 16 instead of 32 x 32 (v_mfma_*_16x16x32, 64 bytes of k a step), TM
 //     and TN count those.
-template <int TM_, int TN_, int WGM_, int WGN_, int WGK_, int SLAB_, int NSTAGE_ = 0, bool OWN_ = false, int BLK_ = 32> struct TileCfg {
+// SETS (shared slabs of two steps a wave): sets of sums that a wave's steps take turns on, added up at the end.  A sum in fp32 grows its
+//     error with the root of the products that follow one another in it, and the shapes of 32 x 32 blocks that these took the place of
+//     had K in two, four or eight parts.  K is in WGK * SETS parts here, as many as those had: 96 x 96 tiles eight, 64 x 64 four, 128 x 128
+//     and larger two (three stages deep four: they took the place of some 64 x 64 ones, too).  256 x 256 tiles have no registers for a second
+//     set and one part, as they had.  FOLDS (192 x 128): the sets go to totals every 768 products, eight parts of K = 3072, where such
+//     tiles took the place of 96 x 96 ones.  Error of the sums (2-norm over 2-norm), fp16, K = 768 / 3072 / 4096:
+//       shapes before: 96 x 96 0.85 / 1.41 / 1.54e-7, 64 x 64 1.00 / 1.82 / 2.03, 128 x 128 1.29 / 2.45 / 2.97
+//       one set:       96 x 96 1.28 / 2.56 / 2.91e-7, 64 x 64 1.28 / 2.56 / 2.91, 128 x 128 1.73 / 3.53 / 4.06
+//       these:         96 x 96 0.81 / 1.35 / 1.51e-7, 64 x 64 0.99 / 1.83 / 2.10, 128 x 128 1.28 / 2.56 / 2.91
+//     The kernels of a forward of 8 x 384 tokens 1032 us with one set, 1032 with these, 16 x 512 1065 and 1060, bf16 5 x 197 612 and 613.
+template <int TM_, int TN_, int WGM_, int WGN_, int WGK_, int SLAB_, int NSTAGE_ = 0, bool OWN_ = false, int BLK_ = 32,
+          int SETS_ = 1, bool FOLDS_ = false>
+struct TileCfg {
     static constexpr int BLK = BLK_;
     // groups of rows that are staged one after the other, and the rows of a wave position in one: blocks of 32 rows, or the whole tile
     // where it is one of 16 x 16 blocks and fits into LDS at once (256 x 256 tiles do not: halves)
     static constexpr int GROUPS = BLK_ == 32 ? TM_ : WGM_ * WGN_ * WGK_ * TM_ * (4 * TN_ + 1) > 640 ? 2 : 1, GROWS = BLK_ * TM_ / GROUPS;
     static_assert(BLK_ == 32 || (BLK_ == 16 && NSTAGE_ > 0 && (!OWN_ || BLK_ * TM_ <= 32)), "16 x 16 blocks: direct-to-LDS slabs only");
     static constexpr int TM = TM_, TN = TN_, WGM = WGM_, WGN = WGN_, WGK = WGK_, SLAB = SLAB_, NSTAGE = NSTAGE_;
-    static constexpr bool OWN = OWN_;
+    static constexpr bool OWN = OWN_, FOLDS = FOLDS_;
+    static constexpr int SETS = SETS_;
     static constexpr int BM = BLK * TM * WGM, BN = BLK * TN * WGN;
     static constexpr int STRIDE = NSTAGE_ ? SLAB : SLAB + 16;
     static constexpr int SSTR   = BLK * TN + 4;  // staged row stride in 32-bit words
@@ -1298,14 +1311,27 @@ __global__ void __launch_bounds__(CFG::NT)
         }
     };
 
-    Acc acc[TM][TN];
+    constexpr int SETS = DT == TNN_ROCM_I8 ? 1 : CFG::SETS;  // sums of whole numbers are exact
+    Acc parts[SETS][TM][TN];
+    Acc(&acc)[TM][TN] = parts[0];
+    auto clear = [](Acc(&sums)[TM][TN]) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < TM; ++i)
+        for (int i = 0; i < TM; ++i)
 #pragma unroll
-        for (int j = 0; j < TN; ++j)
+            for (int j = 0; j < TN; ++j)
 #pragma unroll
-            for (int r = 0; r < BLK * BLK / 64; ++r)
-                acc[i][j][r] = 0;
+                for (int r = 0; r < BLK * BLK / 64; ++r)
+                    sums[i][j][r] = 0;
+    };
+    auto add_to = [](Acc(&sums)[TM][TN], const Acc(&more)[TM][TN]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+                sums[i][j] += more[i][j];
+    };
+    if constexpr (SETS == 1)
+        clear(parts[0]);
 
     const int frag_row = lane % BLK;
     const int frag_off = (lane >> 5) * 16;  // slabs staged through registers: blocks of 32 x 32
@@ -1590,7 +1616,9 @@ __global__ void __launch_bounds__(CFG::NT)
         // rows of a tile do not divide so, the first BM threads a row each): one wave with 24 loads and 48 additions in double
         // while the others wait for it took 0.5 us of a launch of 6.5 (256 x 2304 x 768).
         typedef float f32x2 __attribute__((ext_vector_type(2)));
-        constexpr bool kLateSums = TakesRowSums<Epi>::value && (EpiLds<CFG, Epi>::total > 80 * 1024 || SumBlocks<Epi>::value <= 12);
+        // Two sets of sums of 3 x 6 blocks leave no 24 registers either (eight of them would go to scratch memory).
+        constexpr bool kLateSums = TakesRowSums<Epi>::value &&
+                                   ((EpiLds<CFG, Epi>::total > 80 * 1024 && !(SETS > 1 && TM * TN >= 18)) || SumBlocks<Epi>::value <= 12);
         constexpr int ROWS_WAVE = BM / CFG::NW;
         constexpr bool SHARED   = ROWS_WAVE == 8 || ROWS_WAVE == 16 || ROWS_WAVE == 32;
         constexpr int LANES_ROW = SHARED ? 64 / ROWS_WAVE : 1;
@@ -1727,9 +1755,16 @@ __global__ void __launch_bounds__(CFG::NT)
                 else
                     fb[ks & 1][k >= TM ? k - TM : 0][0] = *reinterpret_cast<const uint4 *>(at + BM * SLAB + (wn * TN + k - TM) * BLK * SLAB);
             };
-            // slab kt, the first of whose fragments have been read; MORE: another one follows, LOADS: and one is requested
-            auto slab = [&](int kt, auto more, auto loads) __attribute__((always_inline)) {
+            // slab kt, the first of whose fragments have been read; MORE: another one follows, LOADS: and one is requested; PAIR: the pair
+            // of sets that its steps take turns on
+            // The sets but the first two, and the totals, are added up behind the last slab's matrix instructions, the two that are left where
+            // the epilogue stages them: together behind the loop they took 0.3 us of the 8.8 of 3072 x 768 x 768.
+            static_assert(SETS == 1 || KSTEPS == 2, "two steps a slab");
+            constexpr bool FOLDS = CFG::FOLDS && SETS == 2;
+            Acc total[FOLDS ? TM : 1][FOLDS ? TN : 1];
+            auto slab = [&](int kt, auto more, auto loads, auto pair) __attribute__((always_inline)) {
                 constexpr bool MORE = decltype(more)::value, LOADS = decltype(loads)::value;
+                constexpr int PAIR  = SETS == 4 ? decltype(pair)::value : 0;
                 const int here = stage, next = stage + 1 == NS ? 0 : stage + 1;
 #pragma unroll
                 for (int ks = 0; ks < KSTEPS; ++ks) {
@@ -1756,8 +1791,13 @@ __global__ void __launch_bounds__(CFG::NT)
                     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
                     for (int q = 0; q < MFMAS; ++q) {
-                        GemmTraits<DT>::mma(fb[ks & 1][q % TN][0], fa[ks & 1][q / TN][0], acc[q / TN][q % TN]);
+                        GemmTraits<DT>::mma(fb[ks & 1][q % TN][0], fa[ks & 1][q / TN][0], parts[SETS > 1 ? 2 * PAIR + ks : 0][q / TN][q % TN]);
                         __builtin_amdgcn_sched_barrier(0);
+                        if constexpr (!MORE && SETS == 4)
+                            parts[2 - 2 * ks][q / TN][q % TN] += parts[3 - ks][q / TN][q % TN];
+                        if constexpr (!MORE && FOLDS)
+                            if (last)
+                                parts[0][q / TN][q % TN] += total[q / TN][q % TN];
                         if (!last || MORE) {
 #pragma unroll
                             for (int k = READS * q / MFMAS; k < READS * (q + 1) / MFMAS; ++k)
@@ -1773,6 +1813,15 @@ __global__ void __launch_bounds__(CFG::NT)
                 }
                 stage = next;
             };
+            if constexpr (SETS > 1) {  // while the first slab is on its way
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int p = 0; p < SETS; ++p)
+                    clear(parts[p]);
+                if constexpr (FOLDS)
+                    clear(total);
+                __builtin_amdgcn_sched_barrier(0);
+            }
             {
                 static_assert(NS <= 3, "waits written for up to three stages");
                 if (NS > 2 && nk > 1)
@@ -1790,12 +1839,25 @@ __global__ void __launch_bounds__(CFG::NT)
                 if (NS - 1 < nk)
                     issue(NS - 1, NS - 1);
             }
+            typedef std::integral_constant<int, 0> First;
+            typedef std::integral_constant<int, 1> Second;
             int kt = 0;
-            for (; kt + NS < nk; ++kt)
-                slab(kt, std::true_type(), std::true_type());
+            if constexpr (SETS == 4)
+                for (; kt + 1 + NS < nk; kt += 2) {
+                    slab(kt, std::true_type(), std::true_type(), First());
+                    slab(kt + 1, std::true_type(), std::true_type(), Second());
+                }
+            for (; kt + NS < nk; ++kt) {
+                slab(kt, std::true_type(), std::true_type(), First());
+                if constexpr (FOLDS)
+                    if ((kt + 1) % (768 / KB) == 0) {
+                        add_to(total, parts[0]), add_to(total, parts[1]);
+                        clear(parts[0]), clear(parts[1]);
+                    }
+            }
             for (; kt + 1 < nk; ++kt)
-                slab(kt, std::true_type(), std::false_type());
-            slab(kt, std::false_type(), std::false_type());
+                slab(kt, std::true_type(), std::false_type(), Second());
+            slab(kt, std::false_type(), std::false_type(), First());
             if constexpr (kLateSums) {
                 finish_sums(0);
                 TR_TL(6);  // handed-over row sums added up
@@ -2087,9 +2149,12 @@ __global__ void __launch_bounds__(CFG::NT)
 #pragma unroll
             for (int b = 0; b < TM / GROUPS; ++b)
 #pragma unroll
-                for (int j = 0; j < TN; ++j)
-                    *reinterpret_cast<acc4 *>(stage_me + (b * 16 + (lane & 15)) * SSTR + j * 16 + 4 * (lane >> 4)) =
-                        acc[i * (TM / GROUPS) + b][j];
+                for (int j = 0; j < TN; ++j) {
+                    acc4 sums = acc[i * (TM / GROUPS) + b][j];
+                    if constexpr (SETS > 1)
+                        sums += parts[1][i * (TM / GROUPS) + b][j];
+                    *reinterpret_cast<acc4 *>(stage_me + (b * 16 + (lane & 15)) * SSTR + j * 16 + 4 * (lane >> 4)) = sums;
+                }
         }
         if constexpr (Epi::kRowStats) {
             if (i == GROUPS - 1) {
@@ -2392,6 +2457,9 @@ constexpr TileCost kTilesHalf[] = {
 // the second slab of two 128 x 128 tiles a CU (1.148, 10 % above what it measures at K of 3072 and up), are set to order the shapes
 // from 128 x 128 on as they measure: 49 products change (hidden sizes 256 to 4096, 512 to 24576 rows), 11 % faster in the mean, the
 // slowest 4 % slower; us: 8192 x 768 x 3072 32.0 -> 27.5, 4096 x 4096 x 4096 77.6 -> 63.0, 12288 x 1280 x 5120 91.7 -> 72.3.
+// GELU adds 2.5 us a round of 256 x 256 tiles in this model, 1.75 before 128 x 128 tiles were of 16 x 16 blocks: with that,
+// products moved to them whose sums the tiles before had in two parts (TileCfg), and that are no faster for it: 4096 x 3072 x 768
+// 28.4 us, with 128 x 128 tiles 26.8, 6400 x 4096 x 1024 66.3 and 67.3.
 // 16 x 16 blocks of a shared slab.  Up to 128 x 64: eight waves as 2 x 2 positions and two k-waves, so that a tile of any number of 32
 // rows and columns is dealt out evenly.  96 x 96 as eight k-waves of 3 x 3 blocks of 32 x 32 passed 295 KB of partial sums through
 // LDS behind its loop (half of the 11 us of 3072 x 768 x 768), now 74; 96 x 64 is one round of the chip where 64 x 64 are two.
@@ -2528,8 +2596,8 @@ int launch_gemm_fast(hipStream_t s, const void *A, const void *B, int M, int N, 
     return launch_tiled<DT, TileCfg<TMv, TNv, WGMv, WGNv, WGKv, SLABv>, Epi>(s, A, B, M, N, K, lda, ldb, epi)
 #define TR_FAST_DL(TMv, TNv, WGMv, WGNv, WGKv, SLABv, NSv)                                                            \
     return launch_tiled<DT, TileCfg<TMv, TNv, WGMv, WGNv, WGKv, SLABv, NSv>, Epi>(s, A, B, M, N, K, lda, ldb, epi)
-#define TR_FAST_DL16(TMv, TNv, WGMv, WGNv, WGKv, SLABv, NSv)                                                          \
-    return launch_tiled<DT, TileCfg<TMv, TNv, WGMv, WGNv, WGKv, SLABv, NSv, false, 16>, Epi>(s, A, B, M, N, K, lda, ldb, epi)
+#define TR_FAST_DL16(TMv, TNv, WGMv, WGNv, WGKv, SLABv, NSv, ...)                                                     \
+    return launch_tiled<DT, TileCfg<TMv, TNv, WGMv, WGNv, WGKv, SLABv, NSv, false, 16, __VA_ARGS__>, Epi>(s, A, B, M, N, K, lda, ldb, epi)
 #define TR_FAST_SMALL(TMv, TNv, WGKv, SLABv, NSv)                                                                     \
     return launch_tiled<DT, TileCfg<TMv, TNv, 1, 1, WGKv, SLABv, NSv, true, 16>, Epi>(s, A, B, M, N, K, lda, ldb, epi)
 #define TR_FAST_OWN(TMv, TNv, WGKv, SLABv, NSv)                                                                       \
@@ -2573,21 +2641,21 @@ int launch_gemm_fast(hipStream_t s, const void *A, const void *B, int M, int N, 
         switch (cfg) {
             case 2112211: TR_FAST_DL(1, 1, 2, 2, 1, 128, 2);
             case 3112221: TR_FAST_DL(1, 1, 2, 2, 2, 128, 3);
-            case 7244211: TR_FAST_DL16(2, 4, 4, 2, 1, 128, 2);
-            case 8244211: TR_FAST_DL16(2, 4, 4, 2, 1, 128, 3);
-            case 8344211: TR_FAST_DL16(3, 4, 4, 2, 1, 128, 3);
-            case 8364211: TR_FAST_DL16(3, 6, 4, 2, 1, 128, 3);
-            case 7484211: TR_FAST_DL16(4, 8, 4, 2, 1, 128, 2);
-            case 8222222: TR_FAST_DL16(2, 2, 2, 2, 2, 256, 3);
-            case 8322222: TR_FAST_DL16(3, 2, 2, 2, 2, 256, 3);
-            case 8332222: TR_FAST_DL16(3, 3, 2, 2, 2, 256, 3);
-            case 8422222: TR_FAST_DL16(4, 2, 2, 2, 2, 256, 3);
+            case 7244211: TR_FAST_DL16(2, 4, 4, 2, 1, 128, 2, 2);
+            case 8244211: TR_FAST_DL16(2, 4, 4, 2, 1, 128, 3, 4);
+            case 8344211: TR_FAST_DL16(3, 4, 4, 2, 1, 128, 3, 2, true);
+            case 8364211: TR_FAST_DL16(3, 6, 4, 2, 1, 128, 3, 2);
+            case 7484211: TR_FAST_DL16(4, 8, 4, 2, 1, 128, 2, 1);
+            case 8222222: TR_FAST_DL16(2, 2, 2, 2, 2, 256, 3, 2);
+            case 8322222: TR_FAST_DL16(3, 2, 2, 2, 2, 256, 3, 2);
+            case 8332222: TR_FAST_DL16(3, 3, 2, 2, 2, 256, 3, 4);
+            case 8422222: TR_FAST_DL16(4, 2, 2, 2, 2, 256, 3, 2);
             default: break;
         }
         if constexpr (DT != TNN_ROCM_I8) {
             switch (cfg) {
-                case 8264211: TR_FAST_DL16(2, 6, 4, 2, 1, 128, 3);
-                case 8444211: TR_FAST_DL16(4, 4, 4, 2, 1, 128, 3);
+                case 8264211: TR_FAST_DL16(2, 6, 4, 2, 1, 128, 3, 2);
+                case 8444211: TR_FAST_DL16(4, 4, 4, 2, 1, 128, 3, 2);
                 default: break;
             }
         }
