@@ -393,7 +393,7 @@ TNN_ROCM_API int tnn_rocm_gelu_i8(void *stream, const int8_t *q_in, float in_sca
  * No counterpart in the reference.  Process-wide switches for experiments and for the tests that force each kernel
  * variant; plain words read by later launches, so set them while no other thread is launching.  All return 0.
  *   gemm_config   : 0 = shape heuristic, -1 = the baseline kernel, else a tile-configuration code of the tiled kernel
- *   gemm_tune     : "MxNxK:code,..." overrides of the heuristic for single shapes (also TNN_ROCM_GEMM_TUNE at first use)
+ *   gemm_tune     : "N:K:code[:group],..." overrides of the heuristic for single (N, K) (also TNN_ROCM_GEMM_TUNE at first use)
  *   gemm_group_m  : tiles per group of the XCD-aware tile order (0 = default)
  *   ln_y_ahead    : 1 (default) = the LayerNorm-folding GEMMs request the source vectors of their y output early
  *   attention_dma : 1 (default) = by size: the kernel for few query blocks, or K / V^T tiles staged global -> LDS directly

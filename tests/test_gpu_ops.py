@@ -661,6 +661,41 @@ def test_gemm_every_tile_configuration(code):
         lib.tnn_rocm_debug_set_gemm_config(0)
 
 
+@pytest.mark.parametrize("code,slab,columns", [(2222221, 128, 128), (3332221, 128, 192), (2244211, 128, 0), (3331182, 256, 96), (3112222, 256, 64),
+                                               (4221141, 128, 64), (3212221, 128, 64)])
+def test_codes_of_retired_tile_shapes(code, slab, columns):
+    """A code that a user's tuning table may hold, of a shape that there is no more: it runs for every K that it ran for, whole slabs of
+    its own, on a tile of the same columns (row sums' blocks; 0: it left none), half and int8."""
+    from tnn_amd import capi
+    lib, o = capi.load(), ops()
+    rng = np.random.default_rng(code)
+    M, N = 150, 384
+    for slabs in (1, 2, 3, 5):
+        say("retired code %d, %d slabs of %d bytes" % (code, slabs, slab))
+        K = slabs * slab // 2
+        a, w = (torch.from_numpy(rng.standard_normal(n).astype(np.float32)).half() for n in ((M, K), (N, K)))
+        a8, w8 = rng.integers(-128, 128, (M, 2 * K), dtype=np.int8), rng.integers(-127, 128, (N, 2 * K), dtype=np.int8)
+        zero, scale = np.zeros(N, np.int32), np.full(N, 1e-3, np.float32)
+        one, st = torch.ones(N, device="cuda"), torch.tensor([[1.0, 0.0]], device="cuda").repeat(M, 1)
+        lib.tnn_rocm_debug_set_gemm_config(code)
+        try:
+            got = host(o.gemm(a.cuda(), w.cuda(), True).double())
+            left, (sums, blocks) = o.gemm_residual_ln(a.cuda(), w.cuda(), a.new_zeros(M, N).cuda(), st, one, 0 * one, want_row_sums=True)
+            q, acc, _ = o.gemm_i8(dev(a8), dev(w8), dev(zero), dev(scale), want_acc=True)
+        finally:
+            lib.tnn_rocm_debug_set_gemm_config(0)
+        exact = host(a.double() @ w.double().T)
+        # one rounding of the result to 11 bits, and fp32 sums
+        assert np.abs(got - exact).max() <= 2.0 ** -11 * np.abs(exact).max() + 2.0 ** -22 * np.sqrt(K) * np.abs(exact).max()
+        assert np.array_equal(host(left.double()), got)
+        assert np.array_equal(host(acc), a8.astype(np.int32) @ w8.astype(np.int32).T)
+        if columns == 0 or (code == 3212221 and slabs % 2):  # 128 x 64 tiles have 256-byte slabs: such a K goes on 128 x 128 ones
+            columns_now = columns and 128
+        else:
+            columns_now = columns
+        assert blocks == (-(-N // columns_now) if columns_now else 0)
+
+
 @pytest.mark.parametrize("code", [9111141, 9121141, 3112221, 3112222, 3212221, 4221141])
 @pytest.mark.parametrize("M,N,K", [(1, 8, 256), (33, 776, 256), (130, 136, 3072)])
 def test_gemm_small_product_shapes(code, M, N, K):

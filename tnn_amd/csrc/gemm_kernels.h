@@ -2577,14 +2577,14 @@ int launch_gemm_fast(hipStream_t s, const void *A, const void *B, int M, int N, 
         default: break;
     }
     if constexpr (DT != TNN_ROCM_F32) {
-        switch (cfg) {  // the code of a shape whose tile is made of 16 x 16 blocks now
-            case 3212221:
+        switch (cfg) {  // codes of shapes that are no more: the same tile in slabs that every K of theirs is a whole number of
             case 2222221: cfg = 7244211; break;
             case 3332221: cfg = 8364211; break;
             case 2244211: cfg = 7484211; break;
             case 3331182: cfg = 8332222; break;
-            case 4221141:
             case 3112222: cfg = 8222222; break;
+            case 4221141: cfg = kbytes % 256 == 0 ? 8222222 : 3112221; break;
+            case 3212221: cfg = kbytes % 256 == 0 ? 8422222 : 7244211; break;  // (128 x 64 has 256-byte slabs only)
             default: break;
         }
     }
