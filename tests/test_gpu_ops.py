@@ -2163,6 +2163,31 @@ def test_row_sums_of_a_wide_tile_are_rounded_once(dtype, code):
 
 
 @pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
+def test_row_sums_of_a_tile_staged_in_groups(dtype):
+    """The 128 x 128 tiles of panels of 4 GiB and more, forced: they are staged in groups of rows and leave their sums all the same, a pair
+    of 64 columns each"""
+    from tnn_amd import capi
+    M, N, K = 300, 1032, 128
+    say("row sums %s, shape 222210" % dtype)
+    gen, td = torch.Generator().manual_seed(K), getattr(torch, dtype)
+    x, w, t = (torch.randn(*n, generator=gen).to(td).cuda() for n in ((M, K), (N, K), (M, N)))
+    st = torch.tensor([[1.0, 0.0]], device="cuda").repeat(M, 1)
+    one = torch.ones(N, device="cuda")
+    capi.load().tnn_rocm_debug_set_gemm_config(222210)
+    try:
+        plain = ops().gemm_residual_ln(x, w, t, st, one, 0 * one)
+        left, (sums, blocks) = ops().gemm_residual_ln(x, w, t, st, one, 0 * one, want_row_sums=True)
+    finally:
+        capi.load().tnn_rocm_debug_set_gemm_config(0)
+    assert blocks == -(-N // 64) and torch.equal(left, plain)
+    for k, part in enumerate(left.cpu().double().split(64, 1)):
+        got = sums[k].cpu().double()
+        # a tree over eight items of eight values each: seven additions in a row, and their own three, of half a unit each at most
+        assert ((got[:, 0] - part.sum(1)).abs() <= 10 * 2.0 ** -24 * part.abs().sum(1)).all()
+        assert ((got[:, 1] - (part ** 2).sum(1)).abs() <= 10 * 2.0 ** -24 * (part ** 2).sum(1)).all()
+
+
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
 @pytest.mark.parametrize("sigmas", [0, 5, 20, 50])
 @pytest.mark.parametrize("code", [0, 6111141, 9111141] + sorted(ROW_SUM_SHAPES))
 def test_row_sums_left_by_a_shape_give_the_variance(dtype, sigmas, code):

@@ -1128,10 +1128,12 @@ struct TileCfg {
     static constexpr size_t stage_bytes = (size_t)WGM_ * WGN_ * WGK_ * GROWS * SSTR * 4;
     static constexpr size_t lds_bytes   = slab_bytes > stage_bytes ? slab_bytes : stage_bytes;
     // Row sums of what an epilogue stored.  Where all columns are one wave's they are added up over the two to eight lanes that hold a
-    // row (32 x 32 tiles, 256 x 768 x 768: 4.60 -> 4.40 us against sums through LDS); elsewhere an item's pair goes into the place of its
-    // own staged values, which takes the whole tile staged at once.
-    static constexpr bool sums_by_lanes = OWN_;
-    static constexpr bool leaves_sums   = OWN_ || GROUPS == 1;
+    // row (32 x 32 tiles, 256 x 768 x 768: 4.60 -> 4.40 us against sums through LDS), and so are those of each wave's 64 columns where the
+    // tile is staged in groups; elsewhere an item's pair goes into the place of its own staged values, which takes the whole tile
+    // staged at once.
+    static constexpr bool sums_by_lanes = OWN_ || (GROUPS > 1 && BLK_ * TN_ == 64);
+    static constexpr bool leaves_sums   = sums_by_lanes || GROUPS == 1;
+    static constexpr int sum_cols       = sums_by_lanes ? BLK_ * TN_ : BN;  // columns of a pair of row sums
     static constexpr int NW = WGM * WGN * WGK, NT = 64 * NW;  // waves and threads per workgroup
     static_assert(NW == 4 || NW == 8, "four or eight waves per workgroup");
     static_assert(OWN_ || ((BM * (SLAB / 16)) % NT == 0 && (BN * (SLAB / 16)) % NT == 0), "slab must divide over the workgroup");
@@ -2228,7 +2230,7 @@ __global__ void __launch_bounds__(CFG::NT)
                     sm.x = add_neighbours<CPR>(sm.x);
                     sm.y = add_neighbours<CPR>(sm.y);
                     if (piece == 0 && m < M && n < N)
-                        store_out8(epi.through, &epi.row_sums[(size_t)(n / BN) * M + m], sm);
+                        store_out8(epi.through, &epi.row_sums[(size_t)(n / CFG::sum_cols) * M + m], sm);
                 } else {
                     *reinterpret_cast<float2 *>(const_cast<AccT *>(src)) = sm;
                 }
@@ -2323,8 +2325,8 @@ __global__ void __launch_bounds__(CFG::NT)
     TR_TL(4);  // kernel end
 }
 
-// internal: the chosen tile shape does not leave row sums (no LDS, too many tile columns) or does not take them; the
-// caller launches the form without
+// internal: the chosen tile shape does not leave row sums (256 x 256 tiles, staged in halves; more blocks of columns than a reader adds
+// up) or does not take them; the caller launches the form without
 constexpr int kNotWithRowSums = -12345;
 thread_local int t_last_sum_blocks = 0;  // row-sum blocks of this thread's last tiled launch
 
@@ -2334,7 +2336,7 @@ int launch_shape(hipStream_t s, const void *A, const void *B, int M, int N, int 
     int tiles_m = (M + CFG::BM - 1) / CFG::BM, tiles_n = (N + CFG::BN - 1) / CFG::BN;
     typedef EpiLds<CFG, Epi> L;
     const size_t lds = L::total;
-    const int sum_blocks = tiles_n;
+    const int sum_blocks = (N + CFG::sum_cols - 1) / CFG::sum_cols;
     if (EmitsRowSums<Epi>::value && sum_blocks > kMaxRowSumBlocks)
         return kNotWithRowSums;
     auto kern   = gemm_nk_tiled_kernel<DT, CFG, Epi>;
@@ -2840,9 +2842,9 @@ template <int DT>
 int GemmTyped<DT>::residual_ln(hipStream_t s, const void *x, const void *w, const float *bias, void *C, const void *t,
                                const float *row_stats, const float *gamma, const float *beta, int M, int N, int K, int flags,
                                float *row_sums, int *row_sum_blocks) {
-    // With the row sums first.  A tile shape whose tile columns are more than a reader adds up (and the caller's buffer of
-    // kMaxRowSumBlocks * M pairs holds: 16 columns wide from N = 385 on, 32 columns wide from N = 769 on), or that leaves no LDS for
-    // the sums, declines in launch_tiled; the plain form runs then and reports zero blocks.
+    // With the row sums first.  A tile shape whose blocks of columns are more than a reader adds up (and the caller's buffer of
+    // kMaxRowSumBlocks * M pairs holds: 16 columns wide from N = 385 on, 32 columns wide from N = 769 on) declines in launch_shape, one
+    // that leaves no sums (256 x 256) in launch_tiled; the plain form runs then and reports zero blocks.
     if (row_sums && N <= 64 * kMaxRowSumBlocks) {
         const int rc = launch_residual_ln<DT, true>(s, x, w, bias, C, t, row_stats, gamma, beta, M, N, K, flags, row_sums);
         if (rc == 0)
