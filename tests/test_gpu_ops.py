@@ -236,7 +236,8 @@ def test_layernorm_row_count_changes_nothing(dtype, vecs):
 @pytest.mark.parametrize("cols", [256, 264, 504, 512, 520, 760, 768, 776, 1016, 1024, 1032])
 def test_embed_layernorm_row_count_changes_nothing(dtype, cols):
     """Up to 3072 half rows of 257 to 1024 columns a wave owns a row in vectors of 8 bytes, beyond half a wave in vectors of 16: the same
-    bits on both sides of the line, for looked-up rows and for stored ones, and the formula in float64 to a rounding of the type."""
+    bits on both sides of the line, and the formula in float64 to a rounding of the type.  (Stored rows, with a residual and an int8
+    copy: test_layernorm_row_count_changes_nothing.)"""
     say("embed_layernorm %s, rows of %d" % (dtype, cols))
     td, rows, vocab = getattr(torch, dtype), 3073, 700
     gen = torch.Generator(device="cuda").manual_seed(cols)
@@ -625,8 +626,8 @@ def test_gemm_half_epilogues(M, N, K, dtype):
     assert rel_err(got, orc.inner_product(af, wf, bias) + rf) <= tol
 
 
-TILE_CODES = [112211, 222221, 224211, 332221, 331182,   # slabs staged through registers
-              2112211, 2222221, 3332221, 3331182]       # slabs loaded global -> LDS directly (2 / 3 stages)
+TILE_CODES = [112210, 222210,                            # slabs staged through registers
+              2112211, 3112221, 8222222, 8322222, 8332222, 8422222, 7244211, 8244211, 8344211, 8364211, 7484211]  # global -> LDS directly
 
 
 @pytest.mark.parametrize("code", TILE_CODES)
@@ -661,10 +662,20 @@ def test_gemm_every_tile_configuration(code):
         lib.tnn_rocm_debug_set_gemm_config(0)
 
 
+HALF_ONLY = (8264211, 8444211)  # tile shapes that int8 has not
+
+
+def _tile_columns(code):
+    """columns of a tile by its code: blocks of 32, or of 16 where the first digit is 6, 7 or 8, times their number and the waves across"""
+    p, _, tn, _, wn = (int(d) for d in str(code)[:5])
+    return (16 if p in (6, 7, 8) else 32) * tn * wn
+
+
 @pytest.mark.parametrize("code,slab,columns", [(2222221, 128, 128), (3332221, 128, 192), (2244211, 128, 0), (3331182, 256, 96), (3112222, 256, 64),
-                                               (4221141, 128, 64), (3212221, 128, 64)])
+                                               (4221141, 128, 64), (3212221, 128, 64), (112211, 128, 64), (222221, 128, 128),
+                                               (224211, 128, 128), (332221, 128, 192), (331182, 256, 96)])
 def test_codes_of_retired_tile_shapes(code, slab, columns):
-    """A code that a user's tuning table may hold, of a shape that there is no more: it runs for every K that it ran for, whole slabs of
+    """A code that a user's tuning table may hold, of a shape that there is no more or without its stages: it runs for every K that it ran for, whole slabs of
     its own, on a tile of the same columns (row sums' blocks; 0: it left none), half and int8."""
     from tnn_amd import capi
     lib, o = capi.load(), ops()
@@ -696,13 +707,13 @@ def test_codes_of_retired_tile_shapes(code, slab, columns):
         assert blocks == (-(-N // columns_now) if columns_now else 0)
 
 
-@pytest.mark.parametrize("code", [9111141, 9121141, 3112221, 3112222, 3212221, 4221141])
+@pytest.mark.parametrize("code", [9111141, 9121141, 3112221, 8222222, 8422222])
 @pytest.mark.parametrize("M,N,K", [(1, 8, 256), (33, 776, 256), (130, 136, 3072)])
 def test_gemm_small_product_shapes(code, M, N, K):
     """The tile shapes of the small products, forced where they can go wrong: one row, a remainder of one row or of eight
     columns behind whole tiles, fewer slabs than a ring or a wave count has places, many slabs.  fp16 epilogues (the
     folded LayerNorm with its statistics and the row sums handed on among them), fp32 where the shape serves it, int8
-    bit-exact."""
+    bit-exact where there is such a shape."""
     from tnn_amd import capi
     lib = capi.load()
     say("tile configuration %d, M=%d N=%d K=%d" % (code, M, N, K))
@@ -734,15 +745,17 @@ def test_gemm_small_product_shapes(code, M, N, K):
         plain = o.gemm_residual_ln(ah.cuda(), wh.cuda(), rh.cuda(), out_st, go, beo, bias=dev(bias))
         assert rel_err(host(plain), orc.inner_product(af, wf, bias) + orc.layernorm(rf, host(go), host(beo), 1e-5)) <= FP16_TOL
         c, (sums, blocks) = o.gemm_residual_ln(ah.cuda(), wh.cuda(), rh.cuda(), out_st, go, beo, bias=dev(bias), want_row_sums=True)
-        assert torch.equal(c, plain) and blocks <= o.MAX_ROW_SUM_BLOCKS
+        columns = _tile_columns(code)
+        assert torch.equal(c, plain) and blocks == (-(-N // columns) if -(-N // columns) <= o.MAX_ROW_SUM_BLOCKS and code != 7484211 else 0)
         if blocks:
             cf = host(c).astype(np.float64)
             got_s = host(sums)[:blocks].astype(np.float64).sum(0)
             assert np.abs(got_s[:, 0] - cf.sum(1)).max() <= 1e-5 * np.abs(cf).sum(1).max()
             assert np.abs(got_s[:, 1] / (cf ** 2).sum(1) - 1).max() <= 1e-5
-        q, acc, _ = o.gemm_i8(dev(a8), dev(w8), dev(b8), dev(scale), want_acc=True)
-        assert np.array_equal(host(acc), ref_acc)
-        assert np.array_equal(host(q), ref_q)
+        if code not in HALF_ONLY and K % (64 << code % 10) == 0:
+            q, acc, _ = o.gemm_i8(dev(a8), dev(w8), dev(b8), dev(scale), want_acc=True)
+            assert np.array_equal(host(acc), ref_acc)
+            assert np.array_equal(host(q), ref_q)
         if code in (9111141, 9121141):
             got = host(o.gemm(a.cuda(), w.cuda(), True, bias=dev(bias), residual=res.cuda()))
             assert rel_err(got, orc.inner_product(a.numpy(), w.numpy(), bias) + res.numpy()) <= 1e-5
@@ -779,11 +792,11 @@ def test_gemm_fp32_split_shapes(code, M, N, K):
     assert (np.abs(got[fine] - exact[fine]) <= 2.0 ** -24 * 4 * np.sqrt(K) * size[fine]).all()
 
 
-@pytest.mark.parametrize("code", [2222221, 3212221, 3332221, 2244211, 3112221])
-@pytest.mark.parametrize("slabs", [1, 2, 3, 4, 5, 8])
+@pytest.mark.parametrize("code", [7244211, 8244211, 8344211, 8364211, 8444211, 7484211, 3112221])
+@pytest.mark.parametrize("slabs", [1, 2, 3, 4, 5, 8, 27, 28])
 def test_gemm_fragments_read_ahead(code, slabs):
-    """Shapes that read a slab's first fragments under the slab before (192 x 192 and 256 x 256 tiles) and, by the same measure, three that
-    read them where they are used: loops of every length (fewer slabs than stages, the last ones whose successors are not requested
+    """Shapes of 128-byte slabs that read a slab's first fragments under the slab before (16 x 16 blocks) and, by the same measure, one that
+    reads them where they are used: loops of every length (fewer slabs than stages, the last ones whose successors are not requested
     any more), whole tiles and remainders, every epilogue; handed-over row sums against sums in double, at numbers of blocks that
     the lanes of a row (two, four or eight of them) share evenly or not, or that are fewer than these, every block's sums others."""
     from tnn_amd import capi
@@ -791,7 +804,7 @@ def test_gemm_fragments_read_ahead(code, slabs):
     K = 64 * slabs
     rng = np.random.default_rng(code % 1000 + slabs)
     say("tile configuration %d, %d slabs" % (code, slabs))
-    if slabs % 4 == 0:
+    if slabs in (4, 8, 28):
         test_gemm_small_product_shapes(code, 257, 264, K)
     o = ops()
     for td in (torch.float16, torch.bfloat16):
@@ -800,7 +813,7 @@ def test_gemm_fragments_read_ahead(code, slabs):
         lib.tnn_rocm_debug_set_gemm_config(code)
         try:
             got = host(o.gemm(a.cuda(), w.cuda(), True).float()).astype(np.float64)
-            if slabs % 2 == 0:
+            if slabs in (2, 4, 8):
                 for blocks in (1, 2, 5, 11, 12, 13, 23, 24):  # few enough for the shape to ask for them late, and more
                     cs, zero = w.double().sum(1).float(), torch.zeros(N)
                     fed = o.gemm_ln(a.cuda(), w.cuda(), zero.cuda(), cs.cuda(), 1e-5, row_sums=(_row_sums(a, blocks), blocks))
@@ -814,54 +827,95 @@ def test_gemm_fragments_read_ahead(code, slabs):
         assert np.abs(got - exact).max() <= (2.0 ** -11 if td is torch.float16 else 2.0 ** -8) * np.abs(exact).max() + 1e-4 * np.sqrt(K)
 
 
-@pytest.mark.parametrize("code", [8222222, 8322222, 8332222, 8422222, 7244211, 8244211, 8264211, 8344211, 8364211, 8444211])
+SHARED_SLABS = [8222222, 8322222, 8332222, 8422222, 7244211, 8244211, 8264211, 8344211, 8364211, 8444211, 7484211]
+
+
+@pytest.mark.parametrize("code", SHARED_SLABS)
 @pytest.mark.parametrize("slabs", [1, 2, 3, 4, 6, 24])
 def test_gemm_16x16_blocks_of_a_shared_slab(code, slabs):
     """Tiles of 16 x 16 blocks whose slabs all waves share: fewer slabs than stages and more, one row or eight columns behind
-    whole tiles, less than a tile, every epilogue with its row sums; Q, K and V^T with tiles across their borders and
-    sequences that end inside a tile."""
+    whole tiles, less than a tile, every epilogue with its row sums; Q, K and V^T with tiles across their borders (two heads and 192
+    columns) and with a part of a tile behind the last whole one (three, and 128 or 256), sequences that end inside a tile."""
     from tnn_amd import capi
     lib, o = capi.load(), ops()
     K = 64 * slabs << code % 10 - 1
     say("tile configuration %d, %d slabs" % (code, slabs))
-    if slabs % 2 == 0 and code not in (8264211, 8444211):  # int8 rows of whole slabs, in the shapes that int8 has
+    if slabs % 2 == 0:
         test_gemm_small_product_shapes(code, 1, 8, K)
         test_gemm_small_product_shapes(code, 193, 200, K)
     rng = np.random.default_rng(code % 1000 + slabs)
-    B, S, heads = 5, 72, 2
-    for td, unit in ((torch.float16, 2.0 ** -11), (torch.bfloat16, 2.0 ** -8)):
-        t, w = (torch.from_numpy(rng.standard_normal(n).astype(np.float32)).to(td) for n in ((B * S, K), (3 * heads * 64, K)))
-        bias = torch.from_numpy(rng.standard_normal(3 * heads * 64).astype(np.float32))
+    B, S = 5, 72
+    for td, unit, heads in ((torch.float16, 2.0 ** -11, 2), (torch.float16, 2.0 ** -11, 3), (torch.bfloat16, 2.0 ** -8, 2)):
+        H = heads * 64
+        t, w = (torch.from_numpy(rng.standard_normal(n).astype(np.float32)).to(td) for n in ((B * S, K), (3 * H, K)))
+        bias = torch.from_numpy(rng.standard_normal(3 * H).astype(np.float32))
+        handed = [(None, 0)] + [(_row_sums(t, n), n) for n in (8, 24) if K % 128 == 0]
         lib.tnn_rocm_debug_set_gemm_config(code)
         try:
             plain = host(o.gemm(t.cuda(), w.cuda(), True, bias=bias.cuda()).float()).astype(np.float64)
-            qk, vt = (host(x.float()).astype(np.float64) for x in o.qkv_split(t.cuda(), w.cuda(), bias.cuda(), B, S, heads))
+            split = [o.qkv_split(t.cuda(), w.cuda(), bias.cuda(), B, S, heads)]
             cs = w.double().sum(1).float().cuda()
-            fed = [host(o.gemm_ln(t.cuda(), w.cuda(), bias.cuda(), cs, 1e-5, row_sums=r).float())
-                   for r in (None, (_row_sums(t, 8), 8), (_row_sums(t, 24), 24)) if K % 128 == 0]
+            fed = [host(o.gemm_ln(t.cuda(), w.cuda(), bias.cuda(), cs, 1e-5, row_sums=h if h[1] else None).float())
+                   for h in handed] if K % 128 == 0 else []
+            normed = [o.qkv_split_ln(t.cuda(), w.cuda(), bias.cuda(), cs, 1e-5, B, S, heads, row_sums=h if h[1] else None)
+                      for h in handed] if K % 128 == 0 else []
             st = torch.stack([1 / (x.var(1, unbiased=False) + 1e-5).sqrt() for x in (t.double(),)] + [t.double().mean(1)], 1).float().cuda()
-            one, x = torch.ones(K, device="cuda"), t[:, :64].contiguous()
-            wx = torch.from_numpy(rng.standard_normal((K, 64)).astype(np.float32)).to(td)
-            left, (sums, blocks) = o.gemm_residual_ln(x.cuda(), wx.cuda(), t.cuda(), st, one, one, want_row_sums=True) \
-                if code % 10 == 1 else (None, (None, 0))
+            one, x = torch.ones(K, device="cuda"), t[:, :64 << code % 10 - 1].contiguous()
+            wx = torch.from_numpy(rng.standard_normal((K, x.shape[1])).astype(np.float32)).to(td)
+            left, (sums, blocks) = o.gemm_residual_ln(x.cuda(), wx.cuda(), t.cuda(), st, one, one, want_row_sums=True)
         finally:
             lib.tnn_rocm_debug_set_gemm_config(0)
         exact = t.double().numpy() @ w.double().numpy().T + bias.double().numpy()
-        # one rounding of the result and sums in fp32
-        allowed = unit * np.abs(exact).max() + 2.0 ** -22 * np.sqrt(K) * np.abs(exact).max()
-        assert np.abs(plain - exact).max() <= allowed and np.abs(qk - exact[:, :256]).max() <= allowed
-        assert np.abs(vt - exact[:, 256:].reshape(B, S, heads, 64).transpose(0, 2, 3, 1)).max() <= allowed
         norm = (t.double() - t.double().mean(1, keepdim=True)) / (t.double().var(1, unbiased=False, keepdim=True) + 1e-5).sqrt()
         ref = (norm @ w.double().T).numpy() + bias.double().numpy()
+        tol = FP16_TOL if td is torch.float16 else 2e-2
+
+        def v_of(y):
+            return y[:, 2 * H:].reshape(B, S, heads, 64).transpose(0, 2, 3, 1)
+        # one rounding of the result and sums in fp32
+        allowed = unit * np.abs(exact).max() + 2.0 ** -22 * np.sqrt(K) * np.abs(exact).max()
+        assert np.abs(plain - exact).max() <= allowed
+        for qk, vt in split:
+            assert np.abs(host(qk.float()) - exact[:, :2 * H]).max() <= allowed and np.abs(host(vt.float()) - v_of(exact)).max() <= allowed
+        for qk, vt in normed:
+            assert rel_err(host(qk.float()), ref[:, :2 * H]) <= tol and rel_err(host(vt.float()), v_of(ref)) <= tol
         for f in fed:
-            assert rel_err(f, ref) <= (FP16_TOL if td is torch.float16 else 2e-2)
-        if left is not None:
-            want = x.double() @ wx.double().T + (t.double() - t.double().mean(1, keepdim=True)) * st[:, :1].double().cpu() + 1
-            assert rel_err(host(left.float()), want.numpy()) <= (FP16_TOL if td is torch.float16 else 2e-2)
+            assert rel_err(f, ref) <= tol
+        want = x.double() @ wx.double().T + (t.double() - t.double().mean(1, keepdim=True)) * st[:, :1].double().cpu() + 1
+        assert rel_err(host(left.float()), want.numpy()) <= tol
+        columns = _tile_columns(code)
+        assert blocks == (-(-K // columns) if -(-K // columns) <= o.MAX_ROW_SUM_BLOCKS and code != 7484211 else 0)
+        if blocks:
             stored, got = left.double().cpu(), sums.double().cpu()[:blocks].sum(0)
-            assert blocks == -(-K // (int(str(code)[2]) * 16 * int(str(code)[4])))
-            assert (got[:, 0] - stored.sum(1)).abs().max() <= 1e-5 * stored.abs().sum(1).max()
-            assert (got[:, 1] / (stored ** 2).sum(1) - 1).abs().max() <= 1e-5
+            # per value ten roundings of half a unit at most, in front of the sum in double
+            assert ((got[:, 0] - stored.sum(1)).abs() <= 10 * 2.0 ** -24 * stored.abs().sum(1)).all()
+            assert ((got[:, 1] / (stored ** 2).sum(1) - 1).abs() <= 10 * 2.0 ** -24).all()
+
+
+@pytest.mark.parametrize("code", [2112211, 3112221] + [c for c in SHARED_SLABS if c not in HALF_ONLY])
+@pytest.mark.parametrize("heads", [2, 3])
+def test_gemm_i8_qkv_split_of_every_shape(code, heads):
+    """int8 Q, K and V^T on every shape, tiles across the border of V^T and a part of a tile behind the last whole one, in rows and columns:
+    whole numbers, so the same bits as of the smallest tiles, whose are the checker's (test_gemm_i8_qkv_split_bit_exact)"""
+    from tnn_amd import capi
+    lib, o = capi.load(), ops()
+    say("gemm_i8_qkv_split, tile configuration %d, %d heads" % (code, heads))
+    B, S, K, H = 5, 72, 768, heads * 64
+    gen = torch.Generator().manual_seed(code + heads)
+    x, w = (torch.randint(-127, 128, n, generator=gen, dtype=torch.int8).cuda() for n in ((B * S, K), (3 * H, K)))
+    bias = torch.randint(-2000, 2000, (3 * H,), generator=gen, dtype=torch.int32).cuda()
+    scale, dequant = (torch.rand(3 * H, generator=gen) * 1e-3 + 1e-5).cuda(), (torch.rand(3 * H, generator=gen) + 0.5).cuda()
+    got = []
+    for c in (6111141, code):
+        lib.tnn_rocm_debug_set_gemm_config(c)
+        try:
+            got.append([o.gemm_i8_qkv_split(x, w, bias, scale, dequant, B, S, heads, vt_key_order=0),
+                        o.gemm_i8_qkv_split(x[:64].contiguous(), w, bias, scale, dequant, 4, 16, heads, vt_key_order=1)])
+        finally:
+            lib.tnn_rocm_debug_set_gemm_config(0)
+    for (qk0, vt0), (qk1, vt1) in zip(*got):
+        assert torch.equal(qk0, qk1) and torch.equal(vt0, vt1)
+        assert len(torch.unique(vt0)) > 100
 
 
 # parts that a shape adds a long product up in, each in a set of sums of its own
@@ -902,8 +956,8 @@ def test_gemm_error_of_the_sums_falls_with_the_parts(dtype):
 @pytest.mark.parametrize("M,N,K,gelu,most", [(24576, 1536, 384, True, 1.1), (12288, 1024, 256, True, 1.07), (4096, 4096, 1024, False, 0.93),
                                              (4096, 3072, 768, True, 1.02)])
 def test_gemm_shape_picked_for_large_products(M, N, K, gelu, most):
-    """256 x 256 tiles where they are the faster ones: with GELU and a short K they took 1.21, 1.12 times what 128 x 128 tiles take, and
-    0.83 of it where the chip is full and the epilogue light."""
+    """256 x 256 tiles where they are the faster ones: with GELU and a short K they take 1.38, 1.28 and 1.09 times what 128 x 128 tiles take,
+    and 0.87 of it where the chip is full and the epilogue light."""
     from tnn_amd import capi
     say("gemm bf16 %d x %d x %d, gelu %d, time of the shape picked" % (M, N, K, gelu))
     lib, o = capi.load(), ops()
@@ -916,7 +970,7 @@ def test_gemm_shape_picked_for_large_products(M, N, K, gelu, most):
             o.gemm(a, w, True, bias=bias, gelu=gelu, out=out)
         finally:
             lib.tnn_rocm_debug_set_gemm_config(0)
-    picked, other = _device_us([lambda: run(0), lambda: run(2222221)])
+    picked, other = _device_us([lambda: run(0), lambda: run(7244211)])
     assert picked <= most * other, (picked, other)
 
 
@@ -2051,7 +2105,7 @@ def _row_sums(t, blocks):
 
 
 @pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
-@pytest.mark.parametrize("code", [0, 6111141, 6211141, 9111141, 3112221, 4221141, 2222221, 3332221, 2244211])
+@pytest.mark.parametrize("code", [0, 6111141, 6211141, 9111141, 2112211, 3112221] + SHARED_SLABS)
 def test_folded_layernorm_statistics_at_the_ends(dtype, code):
     """{rstd, mean} that a folding GEMM leaves, own and from handed-over sums: what 1 / sqrt(variance + eps) is in float64 to the
     last bits of fp32, infinite where a constant row meets eps 0, 0 where the squares run over in fp32 (bf16)"""
@@ -2085,7 +2139,7 @@ def test_folded_layernorm_statistics_at_the_ends(dtype, code):
 
 @pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
 @pytest.mark.parametrize("K", [384, 768, 1536])
-@pytest.mark.parametrize("code", [0, 6111141, 9111141, 3112221, 2222221, 3332221])
+@pytest.mark.parametrize("code", [0, 6111141, 9111141, 3112221] + SHARED_SLABS)
 def test_folded_layernorm_statistics_of_rows_with_little_spread(dtype, K, code):
     """Widths that are no power of two and rows that hardly vary: {rstd, mean} as far as the row's fp32 sums know the variance
     (which is all the way where these are exact: constant rows, and one value of a row a step off)"""

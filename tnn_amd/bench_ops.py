@@ -196,7 +196,7 @@ TILE_SHAPES = {
             (2231142, 64, 96, 1), (2331142, 96, 96, 1), (2222121, 128, 64, 2), (2222221, 128, 128, 1), (2332121, 192, 96, 1))}
 
 
-def tile_sweep(dtype, report, rows=()):
+def tile_sweep(dtype, report, rows=(), hidden=()):
     """Every tile shape of the GEMM kernel over the launches of an encoder: the four projections with their fused epilogues,
     M from 16 tokens on, twelve weight sets in turn (inside a network a layer's weights come from the memory-side cache).
     Reports per launch how far the shape the library picks is behind the best one, and per shape the least-squares fit of the
@@ -236,7 +236,7 @@ def tile_sweep(dtype, report, rows=()):
             return lambda w: ops.gemm_ln(a, w, bias, col, 1e-5, gelu=True, want_stats=True, row_sums=fed), ws
         return lambda w: ops.gemm_residual_ln(a, w, res, stats, col, bias, bias=bias, want_row_sums=True, row_sums_out=sums), ws
 
-    for H in (768,) if dtype == "f32" else (768, 1024):
+    for H in tuple(hidden) or ((768,) if dtype == "f32" else (768, 1024)):
         for proj, N, K in (("qkv", 3 * H, H), ("out", H, H), ("ffn1", 4 * H, H), ("ffn2", H, 4 * H)):
             for M in ms:
                 fn, ws = launches(M, N, K, proj)
@@ -280,6 +280,7 @@ def main():
                     help="build (if missing) and run the stand-alone SIMD micro-benchmark csrc/probe_simd.hip")
     ap.add_argument("--tile-sweep", choices=["f16", "i8", "f32"], help="GEMM tile shapes over the launches of an encoder")
     ap.add_argument("--rows", default="", help="with --tile-sweep: rows of the left operand, with commas")
+    ap.add_argument("--hidden", default="", help="with --tile-sweep: hidden sizes, with commas")
     ap.add_argument("--build-only", action="store_true", help="with --simd-probe: compile it, do not run it")
     ap.add_argument("--launches", type=int, default=20)
     ap.add_argument("--only", default="")
@@ -296,7 +297,7 @@ def main():
             sys.exit(subprocess.call([exe]))
         return
     if a.tile_sweep:
-        tile_sweep(a.tile_sweep, lambda text: print(text, flush=True), [int(m) for m in a.rows.split(",") if m])
+        tile_sweep(a.tile_sweep, lambda text: print(text, flush=True), *([int(n) for n in v.split(",") if n] for v in (a.rows, a.hidden)))
         return
     if a.mall_probe:
         for r in mall_probe(a.launches):
