@@ -793,7 +793,7 @@ def test_gemm_fp32_split_shapes(code, M, N, K):
 
 
 @pytest.mark.parametrize("code", [7244211, 8244211, 8344211, 8364211, 8444211, 7484211, 3112221])
-@pytest.mark.parametrize("slabs", [1, 2, 3, 4, 5, 8, 27, 28])
+@pytest.mark.parametrize("slabs", [1, 2, 3, 4, 5, 8, 15, 16, 31, 32, 33, 36])
 def test_gemm_fragments_read_ahead(code, slabs):
     """Shapes of 128-byte slabs that read a slab's first fragments under the slab before (16 x 16 blocks) and, by the same measure, one that
     reads them where they are used: loops of every length (fewer slabs than stages, the last ones whose successors are not requested
@@ -804,7 +804,7 @@ def test_gemm_fragments_read_ahead(code, slabs):
     K = 64 * slabs
     rng = np.random.default_rng(code % 1000 + slabs)
     say("tile configuration %d, %d slabs" % (code, slabs))
-    if slabs in (4, 8, 28):
+    if slabs in (4, 8, 32):
         test_gemm_small_product_shapes(code, 257, 264, K)
     o = ops()
     for td in (torch.float16, torch.bfloat16):
@@ -947,7 +947,7 @@ def test_gemm_error_of_the_sums_falls_with_the_parts(dtype):
                 lib.tnn_rocm_debug_set_gemm_config(0)
             assert (got == got[0]).all()
             error[code] = np.linalg.norm(got[0] - host(exact + bias.double())) / np.linalg.norm(host(exact))
-            if code == 8344211 and K < 1536:  # the further parts are of 768 products each
+            if code == 8344211 and K < 2048:  # the further parts are of 768 products each, in long sums
                 parts = 2
             assert error[code] <= 1.1 * np.sqrt(error[2112211] ** 2 / parts + np.log2(parts) * 2.0 ** -48 / 3), (K, code, error)
         assert error[2112211] <= 2.0 ** -24 * (K / 16) ** 0.5  # a rounding of half a unit at most every sixteen products

@@ -594,7 +594,7 @@ template <int DT, bool SUMS = false> struct LnResidualEpilogue : StoreThrough {
     typedef typename Elem<DT>::type T;
     static constexpr bool kRowStats = false;
     static constexpr bool kEmitsRowSums = SUMS;
-    float2 *row_sums;  // kEmitsRowSums: [tile columns][M] {sum, sum of squares} of the stored values of C
+    float2 *row_sums;  // kEmitsRowSums: [blocks of columns][M] {sum, sum of squares} of the stored values of C
     int flags;  // TNN_ROCM_EPI_BIAS, TNN_ROCM_EPI_GELU
     const float *bias;
     const T *t;                 // [M, N]
@@ -1104,12 +1104,14 @@ __global__ void __launch_bounds__(WM *WN * 64)
 //     error with the root of the products that follow one another in it, and the shapes of 32 x 32 blocks that these took the place of
 //     had K in two, four or eight parts.  K is in WGK * SETS parts here, as many as those had: 96 x 96 tiles eight, 64 x 64 four, 128 x 128
 //     and larger two (three stages deep four: they took the place of some 64 x 64 ones, too).  256 x 256 tiles have no registers for a second
-//     set and one part, as they had.  FOLDS (192 x 128): the sets go to totals every 768 products, eight parts of K = 3072, where such
-//     tiles took the place of 96 x 96 ones.  Error of the sums (2-norm over 2-norm), fp16, K = 768 / 3072 / 4096:
+//     set and one part, as they had.  FOLDS (192 x 128 from K = 2048 on): the sets go to totals every 768 products, eight parts of
+//     K = 3072, where such tiles took the place of 96 x 96 ones.  (As a kernel of its own: with the totals in one, launches of K = 768
+//     and 1024 took 2 .. 5 % more.)  Error of the sums (2-norm over 2-norm), fp16, K = 768 / 3072 / 4096:
 //       shapes before: 96 x 96 0.85 / 1.41 / 1.54e-7, 64 x 64 1.00 / 1.82 / 2.03, 128 x 128 1.29 / 2.45 / 2.97
 //       one set:       96 x 96 1.28 / 2.56 / 2.91e-7, 64 x 64 1.28 / 2.56 / 2.91, 128 x 128 1.73 / 3.53 / 4.06
 //       these:         96 x 96 0.81 / 1.35 / 1.51e-7, 64 x 64 0.99 / 1.83 / 2.10, 128 x 128 1.28 / 2.56 / 2.91
-//     The kernels of a forward of 8 x 384 tokens 1032 us with one set, 1032 with these, 16 x 512 1065 and 1060, bf16 5 x 197 612 and 613.
+//     A launch takes 0.992 of what it did with one set in the mean (96 of hidden sizes 768 and 1024, 64 to 8192 rows), at most 1.007, with folds
+//     1.03 (5600 x 768 x 3072 31.9 -> 32.7).
 template <int TM_, int TN_, int WGM_, int WGN_, int WGK_, int SLAB_, int NSTAGE_ = 0, bool OWN_ = false, int BLK_ = 32,
           int SETS_ = 1, bool FOLDS_ = false>
 struct TileCfg {
@@ -1335,7 +1337,7 @@ __global__ void __launch_bounds__(CFG::NT)
     if constexpr (SETS == 1)
         clear(parts[0]);
 
-    const int frag_row = lane % BLK;
+    const int frag_row = lane & (BLK - 1);
     const int frag_off = (lane >> 5) * 16;  // slabs staged through registers: blocks of 32 x 32
     const int nk       = K / KB;
     constexpr int FRAGS = GemmTraits<DT>::FRAGS, KSTEP = (1024 / BLK) * FRAGS;  // bytes of k per row that one step multiplies
@@ -1404,7 +1406,7 @@ __global__ void __launch_bounds__(CFG::NT)
             for (int k = 0; k < LPW; ++k)
                 issue_one(k, slab, stage);
         };
-        const int fswz = (frag_row / R256) % VPR;
+        const int fswz = (frag_row / R256) & (VPR - 1);
         const int frow = frag_row * SLAB;
         const int k_lo = nk * uwave / CFG::WGK, k_hi = nk * (uwave + 1) / CFG::WGK;
 #pragma unroll
@@ -1542,9 +1544,12 @@ __global__ void __launch_bounds__(CFG::NT)
         }
         // The load is spelled as inline assembly on purpose: for the compiler's own global_load_lds builtin the
         // wait-count pass puts vmcnt(0) in front of every later LDS read (it cannot tell the stages apart), which
-        // serialises the pipeline.  Here the waits are placed by hand (TR_WAIT_VMCNT below); the kernel issues no
-        // other vector-memory operation until the loop has drained.  m0 carries the wave-uniform LDS address and
-        // needs one wait state before the load.
+        // serialises the pipeline.  Here the waits are placed by hand (TR_WAIT_VMCNT below): a slab has landed once no more operations
+        // are outstanding than the slab loads requested after it.  Any other vector-memory operation behind a slab (the epilogue's
+        // early reads between the first slabs and the next, the late row sums behind the last) is one more that is
+        // younger, so that a wait lets it stand in a slab load's place and waits longer, never shorter; one in front of a slab
+        // (the early row sums) is older and done before it.  m0 carries the wave-uniform LDS address and needs one wait state
+        // before the load.
         const uint32_t lds_base = (uint32_t)(uintptr_t)lds_dyn;  // generic -> LDS offset (low 32 bits of the aperture address)
         const uint32_t wave_dst = (uint32_t)__builtin_amdgcn_readfirstlane((int)(lds_base + (uint32_t)wave * 1024u));
         auto load16 = [](const T *base, uint32_t byte_off, uint32_t lds_addr) {
@@ -1567,7 +1572,7 @@ __global__ void __launch_bounds__(CFG::NT)
                 issue_one(k, slab, stage);
         };
         // byte offset of this lane's fragment chunk inside a slab row, per k-step of the slab
-        const int fswz = (frag_row / R256) % VPR;
+        const int fswz = (frag_row / R256) & (VPR - 1);
         const int frow = frag_row * SLAB;
         // One slab: `between` (the requests for the slab that goes into the stage freed last), then step by step this wave's
         // fragments and their MFMAs
@@ -1758,15 +1763,17 @@ __global__ void __launch_bounds__(CFG::NT)
                     fb[ks & 1][k >= TM ? k - TM : 0][0] = *reinterpret_cast<const uint4 *>(at + BM * SLAB + (wn * TN + k - TM) * BLK * SLAB);
             };
             // slab kt, the first of whose fragments have been read; MORE: another one follows, LOADS: and one is requested; PAIR: the pair
-            // of sets that its steps take turns on
-            // The sets but the first two, and the totals, are added up behind the last slab's matrix instructions, the two that are left where
-            // the epilogue stages them: together behind the loop they took 0.3 us of the 8.8 of 3072 x 768 x 768.
+            // of sets that its steps take turns on; FRESH: it begins their sums, with zeros that stand in the matrix instruction (zeroed
+            // registers cost 0.35 us of the 8.7 of 3072 x 768 x 768, with four sets of nine blocks)
+            // The sets but the first two are added up behind the last slab's matrix instructions, the two that are left where the epilogue
+            // stages them.
             static_assert(SETS == 1 || KSTEPS == 2, "two steps a slab");
             constexpr bool FOLDS = CFG::FOLDS && SETS == 2;
             Acc total[FOLDS ? TM : 1][FOLDS ? TN : 1];
-            auto slab = [&](int kt, auto more, auto loads, auto pair) __attribute__((always_inline)) {
+            auto slab = [&](int kt, auto more, auto loads, auto pair, auto fresh) __attribute__((always_inline)) {
                 constexpr bool MORE = decltype(more)::value, LOADS = decltype(loads)::value;
-                constexpr int PAIR  = SETS == 4 ? decltype(pair)::value : 0;
+                constexpr bool FRESH = decltype(fresh)::value;
+                constexpr int PAIR   = SETS == 4 ? decltype(pair)::value : 0;
                 const int here = stage, next = stage + 1 == NS ? 0 : stage + 1;
 #pragma unroll
                 for (int ks = 0; ks < KSTEPS; ++ks) {
@@ -1793,13 +1800,13 @@ __global__ void __launch_bounds__(CFG::NT)
                     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
                     for (int q = 0; q < MFMAS; ++q) {
-                        GemmTraits<DT>::mma(fb[ks & 1][q % TN][0], fa[ks & 1][q / TN][0], parts[SETS > 1 ? 2 * PAIR + ks : 0][q / TN][q % TN]);
+                        Acc &sum = parts[SETS > 1 ? 2 * PAIR + ks : 0][q / TN][q % TN];
+                        if constexpr (FRESH)
+                            sum = Acc{};
+                        GemmTraits<DT>::mma(fb[ks & 1][q % TN][0], fa[ks & 1][q / TN][0], sum);
                         __builtin_amdgcn_sched_barrier(0);
                         if constexpr (!MORE && SETS == 4)
                             parts[2 - 2 * ks][q / TN][q % TN] += parts[3 - ks][q / TN][q % TN];
-                        if constexpr (!MORE && FOLDS)
-                            if (last)
-                                parts[0][q / TN][q % TN] += total[q / TN][q % TN];
                         if (!last || MORE) {
 #pragma unroll
                             for (int k = READS * q / MFMAS; k < READS * (q + 1) / MFMAS; ++k)
@@ -1815,15 +1822,6 @@ __global__ void __launch_bounds__(CFG::NT)
                 }
                 stage = next;
             };
-            if constexpr (SETS > 1) {  // while the first slab is on its way
-                __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                for (int p = 0; p < SETS; ++p)
-                    clear(parts[p]);
-                if constexpr (FOLDS)
-                    clear(total);
-                __builtin_amdgcn_sched_barrier(0);
-            }
             {
                 static_assert(NS <= 3, "waits written for up to three stages");
                 if (NS > 2 && nk > 1)
@@ -1843,23 +1841,48 @@ __global__ void __launch_bounds__(CFG::NT)
             }
             typedef std::integral_constant<int, 0> First;
             typedef std::integral_constant<int, 1> Second;
+            typedef std::true_type Yes;
+            typedef std::false_type No;
             int kt = 0;
+            constexpr int PER_FOLD = 768 / KB;
+            const bool folds = FOLDS && nk >= PER_FOLD + NS;  // the loop that requests others has slab PER_FOLD - 1
+            if constexpr (SETS > 1) {
+                constexpr int LEAD = SETS / 2;  // slabs that begin the sets
+                if (LEAD - 1 + NS < nk) {
+                    slab(0, Yes(), Yes(), First(), Yes());
+                    if constexpr (SETS == 4)
+                        slab(1, Yes(), Yes(), Second(), Yes());
+                    kt = LEAD;
+                } else {
+#pragma unroll
+                    for (int p = 0; p < SETS; ++p)
+                        clear(parts[p]);
+                }
+                if constexpr (FOLDS)
+                    if (folds)
+                        clear(total);
+            }
             if constexpr (SETS == 4)
                 for (; kt + 1 + NS < nk; kt += 2) {
-                    slab(kt, std::true_type(), std::true_type(), First());
-                    slab(kt + 1, std::true_type(), std::true_type(), Second());
+                    slab(kt, Yes(), Yes(), First(), No());
+                    slab(kt + 1, Yes(), Yes(), Second(), No());
                 }
+            int to_fold = folds ? PER_FOLD - kt : nk;
             for (; kt + NS < nk; ++kt) {
-                slab(kt, std::true_type(), std::true_type(), First());
+                slab(kt, Yes(), Yes(), First(), No());
                 if constexpr (FOLDS)
-                    if ((kt + 1) % (768 / KB) == 0) {
+                    if (--to_fold == 0) {
+                        to_fold = PER_FOLD;
                         add_to(total, parts[0]), add_to(total, parts[1]);
                         clear(parts[0]), clear(parts[1]);
                     }
             }
             for (; kt + 1 < nk; ++kt)
-                slab(kt, std::true_type(), std::false_type(), Second());
-            slab(kt, std::false_type(), std::false_type(), First());
+                slab(kt, Yes(), No(), Second(), No());
+            slab(kt, No(), No(), First(), No());
+            if constexpr (FOLDS)
+                if (folds)
+                    add_to(parts[0], total);
             if constexpr (kLateSums) {
                 finish_sums(0);
                 TR_TL(6);  // handed-over row sums added up
@@ -2407,11 +2430,13 @@ int launch_tiled(hipStream_t s, const void *A, const void *B, int M, int N, int 
 // int8: M from 16 to 8192, the four projections of hidden sizes 768 and 1024 with their fused epilogues; fp32: M from 16 to
 // 3072), taken over twelve weight sets in turn so that weights come from the memory-side cache as they do inside a network:
 // python -m tnn_amd.bench_ops --tile-sweep measures them and fits the rows.  A launch is 3 .. 20 % off its prediction on average,
-// by shape (the large ones most), so picks closer than that are as good as drawn.  The half and int8 rows were then moved as little
-// as it took for few launches to be slower than with the tables and shapes before them: over 584 launches of each type (hidden sizes
-// 256 to 2048, M from 16 to 12288) the picks are 0.4 % (fp16) and 0.5 % (int8) behind the best shape of each, and 7 % and 8 % faster than
-// before; of the 392 compared 11 and 16 are more than 2 % slower, one and three more than 5 (8192 x 2048 x 8192 by 10, which 256 x 256
-// tiles of 16 x 16 blocks have turned into 14 % faster).  fp32: 1.0 % behind.
+// by shape (the large ones most), so picks closer than that are as good as drawn.  The half and int8 rows were then moved by hand as
+// little as it took for few launches to be slower than with the tables and shapes before them; by hand altogether: 256 x 256 in both, and in
+// the int8 table 128 x 128 (the second tile's slab of two stages, the round of three), 192 x 128 and 192 x 192.  The picks are 0.4 %
+// (fp16, int8) behind the best shape of each launch at hidden sizes 768 and 1024, at worst 9 %; at 256 to 2048 (int8: 4096) 0.9 and 1.1 %, at
+// worst 32 % (QKV of 12288 x 1536 x 512).  Against the tables and shapes of 32 x 32 blocks, over 448 launches of each type (hidden sizes
+// 256 to 2048, M from 16 to 12288), they take 0.939 (fp16) and 0.948 (int8) of the time in the mean, six and four of them 5 .. 10 % more.
+// fp32: 1.0 % behind.  profiles/gemm_tile_choice.txt has them one by one, and inside the network.
 // The rules this replaced, made for M >= 1024, were 51 %, 34 % and 77 % behind:
 //   M=  32 N= 768 K=3072 fp16  23.1 -> 7.3 us   (64x64 tiles: 12 CUs, one two-stage slab after another)
 //   M= 256 N= 768 K=3072 fp16  23.7 -> 7.2      M= 256 N=2304 K=768 fp16  8.7 -> 6.2
@@ -2451,27 +2476,26 @@ constexpr TileCost kTilesHalf[] = {
 // row is set by hand: of its picks three of 60 are slower, 24576 x 1920 x 640 into Q, K and V^T by 6 % and [16384, 1024] x 1024 and
 // 24576 x 1280 x 1280 with a residual by 3 %.  That was with 32 x 32 blocks, whose row was {10.5, 12.0, 1.255} (int8 {10.5, 8.2, 2.049}).
 // As 16 x 16 blocks a step's products are twice as many of half the length, between which the next step's reads spread finer, and
-// the loop is 4 .. 10 % faster; the tile is staged in two halves instead of two blocks' rows.  us: 16384 x 4096 x 1024 with GELU
-// 167 -> 152, 16384 x 1024 x 4096 124 -> 115, 8192 x 8192 x 8192 936 -> 861, bf16 873 -> 839, int8 16384 x 1024 x 4096 68.6 -> 62.0,
-// 16384 x 4096 x 1024 105 -> 100, 8192 x 4096 x 4096 136 -> 125.  The half row's slab is smaller by that and its other two figures larger
-// by twelve slabs of it, so that the line stays where it is at K = 768 (with 1.165 alone K = 512 lost 10 %) and moves with K: of the
-// seven products of hidden sizes 512 to 4096 that changed for it five are 3 .. 21 % faster, two 1 % slower.  The int8 row, and with it
+// the loop is 4 .. 11 % faster; the tile is staged in two halves instead of two blocks' rows.  us: 16384 x 4096 x 1024 with GELU
+// 145.5 -> 138.6, 16384 x 1024 x 4096 115 -> 102, 8192 x 8192 x 8192 890 -> 838, bf16 839 -> 795, int8 16384 x 1024 x 4096 72.1 -> 66.6,
+// 16384 x 4096 x 1024 103.0 -> 96.6, 8192 x 4096 x 4096 144.6 -> 136.6.  The half row's slab is smaller by that and its other two figures larger
+// by twelve slabs of it, so that the line stays where it is at K = 768 (with 1.165 alone K = 512 lost 10 %) and moves with K.  The int8 row, and with it
 // the second slab of two 128 x 128 tiles a CU (1.148, 10 % above what it measures at K of 3072 and up), are set to order the shapes
-// from 128 x 128 on as they measure: 49 products change (hidden sizes 256 to 4096, 512 to 24576 rows), 11 % faster in the mean, the
-// slowest 4 % slower; us: 8192 x 768 x 3072 32.0 -> 27.5, 4096 x 4096 x 4096 77.6 -> 63.0, 12288 x 1280 x 5120 91.7 -> 72.3.
+// from 128 x 128 on as they measure; us, the picks before and these, each with its own shapes: 8192 x 768 x 3072 31.0 -> 27.0,
+// 4096 x 4096 x 4096 83.1 -> 65.8, 12288 x 1280 x 5120 96.9 -> 76.7.
 // GELU adds 2.5 us a round of 256 x 256 tiles in this model, 1.75 before 128 x 128 tiles were of 16 x 16 blocks: with that,
 // products moved to them whose sums the tiles before had in two parts (TileCfg), and that are no faster for it: 4096 x 3072 x 768
 // 28.4 us, with 128 x 128 tiles 26.8, 6400 x 4096 x 1024 66.3 and 67.3.
 // 16 x 16 blocks of a shared slab.  Up to 128 x 64: eight waves as 2 x 2 positions and two k-waves, so that a tile of any number of 32
 // rows and columns is dealt out evenly.  96 x 96 as eight k-waves of 3 x 3 blocks of 32 x 32 passed 295 KB of partial sums through
 // LDS behind its loop (half of the 11 us of 3072 x 768 x 768), now 74; 96 x 64 is one round of the chip where 64 x 64 are two.
-// From 128 x 128 on: 4 x 2 positions and no k-waves.  The waves' blocks are longer than high, which costs a third more LDS reads than
-// square ones, but the sums pass through LDS once instead of twice, the fragments of a step are read under the products of
-// the step before, across the slab's barrier too, and 128 x 128 take 36 registers for sums instead of 64.  us, the picks before -> these:
+// From 128 x 128 on: 4 x 2 positions and no k-waves.  The waves' blocks are longer than high, which costs half more LDS reads than square
+// ones (12 KB a wave and slab of 128 x 128, not 8), but the sums pass through LDS once instead of twice and the fragments of a step are
+// read under the products of the step before, across the slab's barrier too.  us, the picks before -> these:
 //   fp16 3072 x 768 x 768 10.9 -> 8.8, 3072 x 768 x 3072 22.9 -> 20.1, 1536 x 768 x 3072 18.8 -> 14.5, 984 x 768 x 3072 13.0 -> 11.8,
 //   700 x 3072 x 768 10.9 -> 8.3, 3072 x 3072 x 768 22.9 -> 21.1, 2048 x 2304 x 768 16.9 -> 14.4, 8192 x 3072 x 1024 77.2 -> 70.8,
 //   8192 x 1024 x 4096 79.7 -> 70.7; int8 1536 x 768 x 3072 11.8 -> 9.3, 3072 x 768 x 3072 15.5 -> 13.2
-// Over the sweeps fp16 launches take 0.944, int8 ones 0.970 of what they did with 32 x 32 blocks.  (Not taken: 64 x 96, 32 x 64, 64 x 32,
+// (Not taken: 64 x 96, 32 x 64, 64 x 32,
 // 32 x 96, 64 x 128 with two k-waves, 0.1 % of the sweep together; 96 x 96 with two stages 8.9 -> 9.9 or four k-waves 9.1 -> 9.4;
 // 128 x 64 and 192 x 96 with 4 x 2 positions, 0.1 % together; 128 x 256, the same as 256 x 128.)
 // Tiles of 16 x 16 blocks with rings of the waves' own are for the products whose 32x32 tiles are too few for the chip: a CU's panels come through its L1 at
@@ -2645,7 +2669,10 @@ int launch_gemm_fast(hipStream_t s, const void *A, const void *B, int M, int N, 
             case 3112221: TR_FAST_DL(1, 1, 2, 2, 2, 128, 3);
             case 7244211: TR_FAST_DL16(2, 4, 4, 2, 1, 128, 2, 2);
             case 8244211: TR_FAST_DL16(2, 4, 4, 2, 1, 128, 3, 4);
-            case 8344211: TR_FAST_DL16(3, 4, 4, 2, 1, 128, 3, 2, true);
+            case 8344211:
+                if (DT != TNN_ROCM_I8 && kbytes >= 4096)
+                    TR_FAST_DL16(3, 4, 4, 2, 1, 128, 3, 2, DT != TNN_ROCM_I8);
+                TR_FAST_DL16(3, 4, 4, 2, 1, 128, 3, 2);
             case 8364211: TR_FAST_DL16(3, 6, 4, 2, 1, 128, 3, 2);
             case 7484211: TR_FAST_DL16(4, 8, 4, 2, 1, 128, 2, 1);
             case 8222222: TR_FAST_DL16(2, 2, 2, 2, 2, 256, 3, 2);

@@ -314,8 +314,8 @@ int launch_layernorm(hipStream_t s, const void *x, const void *res, const float 
     } while (0)
         // Few half rows of 257 to 1024 columns: a wave a row and vectors of eight bytes, so that a lane adds up 8 to 16 values in
         // double, not 16 to 32; that chain is most of such a launch.  Up to three workgroups a CU; from there on the waves, twice
-        // as many, cost more than the shorter chain gives.  Sums in double round the order of their terms away: the results are
-        // those of the form below.  us with a residual and an int8 copy, half a wave a row -> this:
+        // as many, cost more than the shorter chain gives.  The sums in double differ from those of the form below by their order alone, some 2^-50
+        // of a sum, which the roundings to fp32 behind them leave nothing of but in a rare tie.  us with a residual and an int8 copy, half a wave a row -> this:
         //   768 columns  128 rows 4.68 -> 4.06, 1024 4.98 -> 4.10, 3072 5.88 -> 5.43, 4096 6.09 -> 6.31
         //   1024         128      5.51 -> 4.49, 3072 7.04 -> 6.40, 4096 7.48 -> 7.35 (without the copy 6.35 -> 6.56)
         //   256          1024     3.10 -> 3.00, 2048 3.37 -> 3.51          embedding, 768, 128 rows 6.61 -> 6.09, 4096 7.67 -> 8.07
