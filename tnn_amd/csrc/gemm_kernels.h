@@ -2432,11 +2432,12 @@ int launch_tiled(hipStream_t s, const void *A, const void *B, int M, int N, int 
 // python -m tnn_amd.bench_ops --tile-sweep measures them and fits the rows.  A launch is 3 .. 20 % off its prediction on average,
 // by shape (the large ones most), so picks closer than that are as good as drawn.  The half and int8 rows were then moved by hand as
 // little as it took for few launches to be slower than with the tables and shapes before them; by hand altogether: 256 x 256 in both, and in
-// the int8 table 128 x 128 (the second tile's slab of two stages, the round of three), 192 x 128 and 192 x 192.  The picks are 0.4 %
-// (fp16, int8) behind the best shape of each launch at hidden sizes 768 and 1024, at worst 9 %; at 256 to 2048 (int8: 4096) 0.9 and 1.1 %, at
-// worst 32 % (QKV of 12288 x 1536 x 512).  Against the tables and shapes of 32 x 32 blocks, over 448 launches of each type (hidden sizes
-// 256 to 2048, M from 16 to 12288), they take 0.939 (fp16) and 0.948 (int8) of the time in the mean, six and four of them 5 .. 10 % more.
-// fp32: 1.0 % behind.  profiles/gemm_tile_choice.txt has them one by one, and inside the network.
+// the int8 table 128 x 128 (the second tile's slab of two stages, the round of three), 192 x 128 and 192 x 192.  The picks are 0.5 %
+// (fp16, int8) and 0.9 .. 1.6 % (fp32, two sweeps) behind the best shape of each launch at hidden sizes 768 and 1024, at worst 5, 6 and 8 %; at 256
+// to 2048 0.6 (fp16) and 0.8 % (int8), at worst 32 % (QKV of 12288 x 1536 x 512) and 13 %: profiles/gemm_tile_choice.txt, with the launches
+// that are furthest behind, and inside the network.  Against the tables and shapes of 32 x 32 blocks, over 448 launches of each type
+// (hidden sizes 256 to 2048, M from 16 to 12288), they take 0.939 (fp16) and 0.948 (int8) of the time
+// in the mean, six and four of them 5 .. 10 % more.
 // The rules this replaced, made for M >= 1024, were 51 %, 34 % and 77 % behind:
 //   M=  32 N= 768 K=3072 fp16  23.1 -> 7.3 us   (64x64 tiles: 12 CUs, one two-stage slab after another)
 //   M= 256 N= 768 K=3072 fp16  23.7 -> 7.2      M= 256 N=2304 K=768 fp16  8.7 -> 6.2
